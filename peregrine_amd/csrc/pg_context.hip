@@ -69,6 +69,91 @@ pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out) {
     return PG_OK;
 }
 
+void pg_dev_pool::drain(bool close) {
+    std::vector<std::pair<size_t, void *>> take;
+    {
+        std::lock_guard<std::mutex> g(mu);
+        take.swap(blocks);
+        bytes = 0;
+        if (close) open = false;
+    }
+    for (auto &b : take) (void)hipFree(b.second);
+}
+
+pg_status pg_dev_block::alloc(pg_ctx *ctx, size_t want) {
+    release();
+    // to the next sixteenth of a power of two, so that objects of nearly one size can take each other's blocks
+    size_t unit = 4096;
+    while (unit * 16 < want) unit *= 2;
+    want = pg_round_up(want ? want : 1, unit);
+    pool = ctx->pool;
+    {
+        std::lock_guard<std::mutex> g(pool->mu);
+        size_t best = pool->blocks.size();
+        for (size_t i = 0; i < pool->blocks.size(); ++i) {
+            const size_t c = pool->blocks[i].first;
+            if (c >= want && c <= want + want / 4 && (best == pool->blocks.size() || c < pool->blocks[best].first)) best = i;
+        }
+        if (best < pool->blocks.size()) {
+            cap = pool->blocks[best].first;
+            p = pool->blocks[best].second;
+            pool->bytes -= cap;
+            pool->blocks[best] = pool->blocks.back();
+            pool->blocks.pop_back();
+            return PG_OK;
+        }
+    }
+    hipError_t e = hipMalloc(&p, want);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        pool->drain(false);
+        e = hipMalloc(&p, want);
+    }
+    if (e != hipSuccess) {
+        p = nullptr;
+        pool.reset();
+        return pg_fail(PG_ENOMEM, "hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
+    }
+    cap = want;
+    return PG_OK;
+}
+
+void pg_dev_block::touch(const pg_ctx *ctx) {
+    if (p && pool && pool != ctx->pool) foreign = true;
+}
+
+void pg_dev_block::release() {
+    if (!p) return;
+    bool kept = false;
+    if (!foreign) {
+        std::lock_guard<std::mutex> g(pool->mu);
+        if (pool->open && pool->bytes + cap <= PG_POOL_BYTES) {
+            pool->blocks.emplace_back(cap, p);
+            pool->bytes += cap;
+            kept = true;
+        }
+    }
+    if (!kept) (void)hipFree(p);  // (waits for the device)
+    p = nullptr;
+    cap = 0;
+    foreign = false;
+    pool.reset();
+}
+
+pg_status pg_pinned(pg_ctx *ctx, size_t bytes, void **out) {
+    if (bytes > ctx->pin_bytes) {
+        PG_HIP(hipStreamSynchronize(ctx->stream));
+        if (ctx->pin) PG_HIP(hipHostFree(ctx->pin));
+        ctx->pin = nullptr;
+        ctx->pin_bytes = 0;
+        const size_t want = pg_round_up(bytes + bytes / 4, 1 << 16);
+        PG_HIP(hipHostMalloc(&ctx->pin, want, hipHostMallocDefault));
+        ctx->pin_bytes = want;
+    }
+    *out = ctx->pin;
+    return PG_OK;
+}
+
 PG_API pg_status pg_ctx_create(int device, void *hip_stream, pg_ctx **out) {
     PG_CHECK_ARG(out != nullptr, "pg_ctx_create: out is null");
     *out = nullptr;
@@ -111,6 +196,8 @@ PG_API void pg_ctx_destroy(pg_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->ws) (void)hipFree(ctx->ws);
+    if (ctx->pin) (void)hipHostFree(ctx->pin);
+    ctx->pool->drain(true);
     for (auto &t : ctx->moe_tabs)
         if (t.dev) (void)hipFree(t.dev);
     prof_drop(ctx);

@@ -5,14 +5,20 @@
 //   HuffmanKVCache::compress_chunk / decompress_chunk                             reference: src/huffman.rs:612-680
 //   HuffmanKVCache::len / get_kv                                                  reference: src/huffman.rs:683-724
 //
-// Everything but the 256-entry code table is device work here: the hot window is the device
-// StandardKVCache, a chunk's per-head absolute maximum, its int8 values and their histogram come
-// from two kernels, the host builds the table from the histogram (2 KB down, 1 KB up), and the
-// encoder is a prefix sum over the code lengths followed by one pass in which every thread packs
-// 16 consecutive codes into the words of the MSB-first stream.  Coded chunks stay in device
-// memory, each with its 8 KB decode table beside it; decoding is the self-synchronising decoder of
-// the Huffman-coded weights over all chunks of a cache at once (every stream under its own table),
-// followed by one scaling kernel that writes straight into the caller's [heads, tokens, head_dim] layout.
+// Everything is device work here, and all the chunks that one append cuts (both sides) are one batch of four
+// launches: the heads' absolute maxima; the int8 values with a histogram per 4096 of them; the code table, one
+// workgroup a chunk, which also turns the small histograms into the bit at which each 4096 values start; and the
+// encoder.  The host takes part once per batch: it learns the coded sizes (words that the table kernel stores in
+// pinned memory), allocates exactly that much and launches the encoder.  A batch was 10 launches, 12 copies and 8
+// waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
+// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.38.
+//
+// The encoder knows where every code starts, so it leaves an index beside the stream (a 16-bit offset per 64 values,
+// 0.25 bit a value): the decoder of such a chunk is one launch that starts a thread per 64 values, with no search for
+// code boundaries, and writes the scaled f32 values into the caller's layout.  A chunk made from stored parts has no
+// index and goes through the self-synchronising decoder of the Huffman-coded weights and a scaling launch.
+#include <chrono>
+#include <memory>
 #include <new>
 #include <vector>
 #include "pg_internal.h"
@@ -21,149 +27,591 @@
 namespace {
 
 constexpr int NUM_SYMBOLS = 256;
+constexpr int KV_MAX_BITS = 12;                // longest code (src/huffman.rs:30)
+constexpr int KV_LUT = 1 << KV_MAX_BITS;
 constexpr int KV_WG = 256;
 constexpr int ENC_SPT = 16;                    // symbols per thread of the encoder
-constexpr int ENC_PER_WG = KV_WG * ENC_SPT;    // symbols per workgroup
-constexpr unsigned KV_MAX_SPLITS = 64;         // workgroups per head of the two quantising kernels
+constexpr int ENC_PER_WG = KV_WG * ENC_SPT;    // symbols per workgroup: one histogram and one start bit each
+constexpr int SUB_SYMS = 64;                   // symbols per entry of the index, and per thread of the decoder
+constexpr int DEC_PER_WG = KV_WG * SUB_SYMS;   // symbols per workgroup of the decoder
+constexpr unsigned KV_MAX_SPLITS = 64;         // workgroups per head of the maximum and scaling kernels
+constexpr size_t KV_BATCH_SYMBOLS = 64u << 20; // symbols of one batch: bounds what a batch takes of the scratch arena
+constexpr unsigned KV_BATCH_CHUNKS = 2048;     // and its chunks
 
-// Largest |v| of every head (NaN ignored, as f32::max does): grid (splits, heads), amax_bits zeroed.
-__global__ __launch_bounds__(KV_WG) void kv_absmax_kernel(const float *__restrict__ data, size_t head_stride, size_t head_elems,
-                                                          unsigned *__restrict__ amax_bits) {
+// Device layout of a coded chunk: [scales][code lengths][decode table]{[start bit per 4096][offset per 64]}[stream, padded].
+struct kv_layout {
+    size_t o_book, o_lut, o_wg, o_sub, o_bits;
+    __host__ __device__ kv_layout(size_t heads, size_t total, bool indexed) {
+        const size_t nwg = (total + ENC_PER_WG - 1) / ENC_PER_WG, nsub = (total + SUB_SYMS - 1) / SUB_SYMS;
+        o_book = (heads * sizeof(float) + 255) / 256 * 256;
+        o_lut = o_book + NUM_SYMBOLS;
+        o_wg = o_lut + KV_LUT * sizeof(uint16_t);
+        o_sub = o_wg + (indexed ? (nwg + 1) * sizeof(unsigned long long) : 0);
+        o_bits = (o_sub + (indexed ? nsub * sizeof(uint16_t) : 0) + 255) / 256 * 256;
+    }
+    // with the stream's last word whole and 16 bytes of zeros behind it
+    __host__ __device__ size_t size(unsigned long long bytes) const { return (o_bits + (bytes + 3) / 4 * 4 + 16 + 255) / 256 * 256; }
+};
+
+// One batch: chunk c of `count` is side c % sides, number c / sides of that side; its head h starts at
+// data[side] + number * chunk_step + h * head_stride, head_elems values.  Scratch is per chunk, back to back.
+struct kv_batch {
+    const float *data[2];
+    size_t chunk_step, head_stride;
+    unsigned sides, count, heads, head_elems, total, nwg, splits;
+    float *amax;                  // [count][heads][splits]
+    float *scales;                // [count][heads]
+    int8_t *q;                    // [count][q_stride]
+    size_t q_stride;
+    uint16_t *hist;               // [count][nwg][256]
+    unsigned long long *wg_bit;   // [count][nwg + 1] start bits, then the total
+    unsigned *codes;              // [count][256] length << 16 | code
+    uint16_t *lut;                // [count][KV_LUT]
+    __device__ const float *head(unsigned c, unsigned h) const { return data[c % sides] + (size_t)(c / sides) * chunk_step + (size_t)h * head_stride; }
+};
+
+// Largest |v| of every head (NaN ignored, as f32::max does), one value per split: grid (splits, heads, chunks).
+__global__ __launch_bounds__(KV_WG) void kv_absmax_kernel(const kv_batch b, int vec) {
     __shared__ float red[4];
-    const float *p = data + (size_t)blockIdx.y * head_stride;
+    const float *p = b.head(blockIdx.z, blockIdx.y);
     float m = 0.0f;
-    for (size_t i = (size_t)blockIdx.x * KV_WG + threadIdx.x; i < head_elems; i += (size_t)gridDim.x * KV_WG)
-        m = fmaxf(m, fabsf(p[i]));
-    m = pg_block_max_256(m, red);
-    if (threadIdx.x == 0) atomicMax(amax_bits + blockIdx.y, __float_as_uint(m));  // m >= 0: the bit patterns order as the values
-}
-
-// q = round(v / scale) clamped to +-127 with scale = amax / 127 (1 for an all-zero head), the
-// histogram of q, and the scales.   src/huffman.rs:624-646
-__global__ __launch_bounds__(KV_WG) void kv_quant_hist_kernel(const float *__restrict__ data, size_t head_stride, size_t head_elems,
-                                                              const unsigned *__restrict__ amax_bits, int8_t *__restrict__ q,
-                                                              float *__restrict__ scales, unsigned long long *__restrict__ hist) {
-    __shared__ unsigned lh[NUM_SYMBOLS];
-    lh[threadIdx.x] = 0;
-    __syncthreads();
-    const float amax = __uint_as_float(amax_bits[blockIdx.y]);
-    const float scale = (amax == 0.0f) ? 1.0f : amax / 127.0f;
-    const float inv_scale = 1.0f / scale;
-    if (blockIdx.x == 0 && threadIdx.x == 0) scales[blockIdx.y] = scale;
-    const float *p = data + (size_t)blockIdx.y * head_stride;
-    int8_t *o = q + (size_t)blockIdx.y * head_elems;
-    for (size_t i = (size_t)blockIdx.x * KV_WG + threadIdx.x; i < head_elems; i += (size_t)gridDim.x * KV_WG) {
-        const int v = pg_quant_to_i8(p[i] * inv_scale);
-        o[i] = (int8_t)v;
-        atomicAdd(&lh[v + 128], 1u);
-    }
-    __syncthreads();
-    if (lh[threadIdx.x]) atomicAdd(hist + threadIdx.x, (unsigned long long)lh[threadIdx.x]);
-}
-
-// The code lengths of a thread's ENC_SPT symbols (codes[s] = length << 16 | code), and the symbols.
-__device__ __forceinline__ unsigned enc_load(const int8_t *__restrict__ q, size_t n, size_t base, const unsigned *lc, int8_t *sym,
-                                             int &count) {
-    count = base >= n ? 0 : (int)(n - base < (size_t)ENC_SPT ? n - base : (size_t)ENC_SPT);
-    if (count == ENC_SPT) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(q + base);  // base is a multiple of 16 and q is 256-byte aligned
-        const unsigned w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < ENC_SPT; ++j) sym[j] = (int8_t)(w[j >> 2] >> (8 * (j & 3)));
-    } else {
-#pragma unroll
-        for (int j = 0; j < ENC_SPT; ++j) sym[j] = j < count ? q[base + j] : (int8_t)0;
-    }
-    unsigned bits = 0;
-#pragma unroll
-    for (int j = 0; j < ENC_SPT; ++j)
-        if (j < count) bits += lc[(int)sym[j] + 128] >> 16;
-    return bits;
-}
-
-// Inclusive sum over the workgroup's 256 threads; `sc` = 256 unsigned of LDS.
-__device__ __forceinline__ unsigned block_inclusive_sum(unsigned v, unsigned *sc) {
-    sc[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < KV_WG; off <<= 1) {
-        const unsigned add = threadIdx.x >= (unsigned)off ? sc[threadIdx.x - off] : 0u;
-        __syncthreads();
-        sc[threadIdx.x] += add;
-        __syncthreads();
-    }
-    return sc[threadIdx.x];
-}
-
-// Bits every workgroup's ENC_PER_WG symbols take.
-__global__ __launch_bounds__(KV_WG) void kv_encode_bits_kernel(const int8_t *__restrict__ q, size_t n,
-                                                               const unsigned *__restrict__ codes,
-                                                               unsigned long long *__restrict__ wg_bits) {
-    __shared__ unsigned lc[NUM_SYMBOLS], sc[KV_WG];
-    lc[threadIdx.x] = codes[threadIdx.x];
-    __syncthreads();
-    int8_t sym[ENC_SPT];
-    int count;
-    const unsigned bits = enc_load(q, n, (size_t)blockIdx.x * ENC_PER_WG + (size_t)threadIdx.x * ENC_SPT, lc, sym, count);
-    const unsigned incl = block_inclusive_sum(bits, sc);
-    if (threadIdx.x == KV_WG - 1) wg_bits[blockIdx.x] = incl;
-}
-
-// One workgroup: wg_bits[0 .. nwg) becomes its exclusive running sum, wg_bits[nwg] the total.
-__global__ __launch_bounds__(KV_WG) void kv_encode_scan_kernel(unsigned long long *__restrict__ wg_bits, size_t nwg) {
-    __shared__ unsigned long long sc[KV_WG];
-    unsigned long long run = 0;
-    for (size_t c = 0; c < nwg; c += KV_WG) {
-        const size_t i = c + threadIdx.x;
-        const unsigned long long v = i < nwg ? wg_bits[i] : 0ull;
-        sc[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < KV_WG; off <<= 1) {
-            const unsigned long long add = threadIdx.x >= (unsigned)off ? sc[threadIdx.x - off] : 0ull;
-            __syncthreads();
-            sc[threadIdx.x] += add;
-            __syncthreads();
+    if (vec) {
+        const unsigned n4 = b.head_elems / 4;
+        for (unsigned i = blockIdx.x * KV_WG + threadIdx.x; i < n4; i += gridDim.x * KV_WG) {
+            const float4 v = reinterpret_cast<const float4 *>(p)[i];
+            m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
         }
-        if (i < nwg) wg_bits[i] = run + sc[threadIdx.x] - v;
-        run += sc[KV_WG - 1];
-        __syncthreads();
+    } else {
+        for (unsigned i = blockIdx.x * KV_WG + threadIdx.x; i < b.head_elems; i += gridDim.x * KV_WG) m = fmaxf(m, fabsf(p[i]));
     }
-    if (threadIdx.x == 0) wg_bits[nwg] = run;
+    m = pg_block_max_256(m, red);
+    if (threadIdx.x == 0) b.amax[((size_t)blockIdx.z * b.heads + blockIdx.y) * b.splits + blockIdx.x] = m;
 }
 
-// HuffmanTable::encode (src/huffman.rs:216-251) in parallel: every thread knows the bit its first
-// code starts at, shifts its codes into a 64-bit window and ORs whole big-endian words into the
-// zeroed stream (only a thread's first and last word are shared with its neighbours).
-__global__ __launch_bounds__(KV_WG) void kv_encode_write_kernel(const int8_t *__restrict__ q, size_t n,
-                                                                const unsigned *__restrict__ codes,
-                                                                const unsigned long long *__restrict__ wg_excl,
-                                                                unsigned *__restrict__ words) {
-    __shared__ unsigned lc[NUM_SYMBOLS], sc[KV_WG];
-    lc[threadIdx.x] = codes[threadIdx.x];
+// q = round(v / scale) clamped to +-127 with scale = amax / 127 (1 for an all-zero head), the scales, and the
+// histogram of each workgroup's ENC_PER_WG values (a table per wavefront: fewer lanes meet on a common value).
+// src/huffman.rs:624-646.  Grid (nwg, chunks).
+__global__ __launch_bounds__(KV_WG) void kv_quant_hist_kernel(const kv_batch b, int vec) {
+    __shared__ unsigned lh[4][NUM_SYMBOLS];
+    __shared__ float sc[ENC_PER_WG];  // scales of the heads the workgroup meets (every value its own head at the most)
+    const unsigned c = blockIdx.y, t = threadIdx.x, base = blockIdx.x * ENC_PER_WG;
+    const unsigned last = min(base + ENC_PER_WG, b.total) - 1;
+    const unsigned h0 = base / b.head_elems, h1 = last / b.head_elems;
+    for (unsigned h = h0 + t; h <= h1; h += KV_WG) {
+        const float *a = b.amax + ((size_t)c * b.heads + h) * b.splits;
+        float m = 0.0f;
+        for (unsigned s = 0; s < b.splits; ++s) m = fmaxf(m, a[s]);
+        const float scale = (m == 0.0f) ? 1.0f : m / 127.0f;
+        sc[h - h0] = scale;
+        if (base <= h * b.head_elems) b.scales[(size_t)c * b.heads + h] = scale;  // the workgroup of the head's first value
+    }
+    for (int i = 0; i < 4; ++i) lh[i][t] = 0;
     __syncthreads();
-    int8_t sym[ENC_SPT];
-    int count;
-    const unsigned bits = enc_load(q, n, (size_t)blockIdx.x * ENC_PER_WG + (size_t)threadIdx.x * ENC_SPT, lc, sym, count);
-    const unsigned incl = block_inclusive_sum(bits, sc);
-    if (bits == 0) return;
-    const unsigned long long p0 = wg_excl[blockIdx.x] + (incl - bits);
-    size_t word = (size_t)(p0 >> 5);
-    unsigned nacc = (unsigned)(p0 & 31);  // bits of the current word that belong to earlier threads (zeros here)
-    unsigned long long acc = 0;
+    unsigned *mine = lh[t >> 6];
+    int8_t *q = b.q + (size_t)c * b.q_stride;
 #pragma unroll
-    for (int j = 0; j < ENC_SPT; ++j) {
-        if (j < count) {
-            const unsigned e = lc[(int)sym[j] + 128], l = e >> 16;
-            acc = (acc << l) | (e & ((1u << l) - 1u));
-            nacc += l;
-            if (nacc >= 32) {
-                atomicOr(words + word, __builtin_bswap32((unsigned)(acc >> (nacc - 32))));
-                ++word;
-                nacc -= 32;
-                acc &= (1ull << nacc) - 1ull;
+    for (int j = 0; j < ENC_SPT / 4; ++j) {
+        const unsigned i = base + (j * KV_WG + t) * 4;
+        if (vec) {  // four values of one head
+            if (i >= b.total) continue;
+            const unsigned h = i / b.head_elems;
+            const float inv = 1.0f / sc[h - h0];
+            const float4 v = *reinterpret_cast<const float4 *>(b.head(c, h) + (i - h * b.head_elems));
+            const int x0 = pg_quant_to_i8(v.x * inv), x1 = pg_quant_to_i8(v.y * inv), x2 = pg_quant_to_i8(v.z * inv), x3 = pg_quant_to_i8(v.w * inv);
+            *reinterpret_cast<unsigned *>(q + i) = (x0 & 255) | (x1 & 255) << 8 | (x2 & 255) << 16 | (unsigned)x3 << 24;
+            atomicAdd(mine + x0 + 128, 1u);
+            atomicAdd(mine + x1 + 128, 1u);
+            atomicAdd(mine + x2 + 128, 1u);
+            atomicAdd(mine + x3 + 128, 1u);
+        } else {
+            for (unsigned k = i; k < i + 4 && k < b.total; ++k) {
+                const unsigned h = k / b.head_elems;
+                const int x = pg_quant_to_i8(b.head(c, h)[k - h * b.head_elems] * (1.0f / sc[h - h0]));
+                q[k] = (int8_t)x;
+                atomicAdd(mine + x + 128, 1u);
             }
         }
     }
-    if (nacc > 0) atomicOr(words + word, __builtin_bswap32((unsigned)(acc << (32 - nacc))));
+    __syncthreads();
+    b.hist[((size_t)c * b.nwg + blockIdx.x) * NUM_SYMBOLS + t] = (uint16_t)(lh[0][t] + lh[1][t] + lh[2][t] + lh[3][t]);
+}
+
+// The chunk's code table and where its 4096-value runs start: one workgroup of 1024 a chunk.
+//
+// Lengths as HuffmanTable::from_frequencies gives them (src/huffman.rs:35-150: two queues over the symbols sorted by
+// frequency, a leaf wins a tie; depths clamped to 12), and where the clamp over-subscribes the code the same repair
+// as table_that_decodes in pg_huffman.hip.
+//
+// The merges are not made one after the other (a chain of up to 255 dependent steps: 80 us on one wavefront) but in
+// rounds: with the trees still apart in queue order, the sum m of the first two is the smallest weight a new tree can
+// have, so all those of weight <= m are taken, two by two, before any tree that the round makes (a tie goes to the one
+// that was there first).  A round pairs them up and merges the sums, ascending as they are, into what is left; some
+// 18 rounds of 0.8 us for a chunk of 262144 normally distributed values, half of the kernel's 28 us.  Each node's parent is kept; depths follow by
+// pointer doubling.
+__global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsigned long long *host_bits) {
+    __shared__ unsigned part[4][NUM_SYMBOLS], rank_up[NUM_SYMBOLS], rank_down[NUM_SYMBOLS];
+    __shared__ __attribute__((aligned(16))) unsigned long long keys[NUM_SYMBOLS];
+    __shared__ unsigned tree_w[2][NUM_SYMBOLS], tree_id[2][NUM_SYMBOLS];
+    __shared__ unsigned parent[2 * NUM_SYMBOLS];  // of the leaves (by ascending frequency), then of the nodes
+    __shared__ unsigned anc[2][NUM_SYMBOLS], dep[2][NUM_SYMBOLS];
+    __shared__ unsigned cnt[16], first_code[16], limit[16], offset[16], lane_cnt[4][16];
+    __shared__ __attribute__((aligned(16))) uint8_t bl[NUM_SYMBOLS];
+    __shared__ uint8_t by_len[NUM_SYMBOLS];
+    __shared__ unsigned over, wsum[16];
+    __shared__ unsigned run_bits[1024];
+    const unsigned c = blockIdx.x, t = threadIdx.x, s = t & 255, p = t >> 8;
+    const uint16_t *hist = b.hist + (size_t)c * b.nwg * NUM_SYMBOLS;
+
+    unsigned sum = 0;
+    for (unsigned i = p; i < b.nwg; i += 4) sum += hist[(size_t)i * NUM_SYMBOLS + s];
+    part[p][s] = sum;
+    if (t < 16) cnt[t] = 0;
+    if (t < NUM_SYMBOLS) rank_up[t] = rank_down[t] = 0;
+    __syncthreads();
+    const unsigned f = part[0][s] + part[1][s] + part[2][s] + part[3][s];
+    // symbols in order of frequency, ties by symbol: one key each, symbols not in use behind all others
+    const unsigned long long key = f ? (unsigned long long)f << 8 | s : ~0ull;
+    if (p == 0) keys[s] = key;
+    const unsigned n = __builtin_amdgcn_readfirstlane(__syncthreads_count(p == 0 && f > 0));  // symbols in use
+    unsigned up = 0;
+#pragma unroll 8
+    for (unsigned o = p * 64; o < p * 64 + 64; ++o) up += keys[o] < key;
+    atomicAdd(&rank_up[s], up);
+    __syncthreads();
+    const unsigned lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    constexpr unsigned NONE = 0xFFFFFFFFu;  // (weights stay below 2^31)
+    if (p == 0 && f > 0) {
+        tree_w[0][rank_up[s]] = f;
+        tree_id[0][rank_up[s]] = rank_up[s];
+    }
+    __syncthreads();
+    unsigned cur = 0, made = 0;
+    for (unsigned alive = n; alive > 1;) {
+        unsigned a[4], b2[2];
+#pragma unroll
+        for (unsigned r = 0; r < 4; ++r) a[r] = lane + 64 * r < alive ? tree_w[cur][lane + 64 * r] : NONE;
+        const unsigned m = __builtin_amdgcn_readlane(a[0], 0) + __builtin_amdgcn_readlane(a[0], 1);
+        unsigned taken = 0;
+#pragma unroll
+        for (unsigned r = 0; r < 4; ++r) taken += __popcll(__ballot(a[r] <= m));
+        taken &= ~1u;
+        const unsigned pairs = taken / 2;
+        if (wave < 6) {
+#pragma unroll
+            for (unsigned h = 0; h < 2; ++h) {
+                const unsigned k = lane + 64 * h;
+                b2[h] = k < pairs ? tree_w[cur][2 * k] + tree_w[cur][2 * k + 1] : NONE;
+            }
+        }
+        if (wave < 4) {  // what is left: 64 trees to a wavefront, each behind the new ones that are lighter
+            const unsigned own = wave == 0 ? a[0] : wave == 1 ? a[1] : wave == 2 ? a[2] : a[3], i = lane + 64 * wave;
+            const unsigned id = tree_id[cur][i];
+            unsigned at = i - taken;
+            for (unsigned k = 0; k < min(pairs, 64u); k += 8)
+#pragma unroll
+                for (unsigned u = 0; u < 8; ++u) at += __builtin_amdgcn_readlane(b2[0], k + u) < own ? 1u : 0u;
+            for (unsigned k = 64; k < pairs; ++k) at += __builtin_amdgcn_readlane(b2[1], k - 64) < own ? 1u : 0u;
+            if (i >= taken && i < alive) {
+                tree_w[cur ^ 1][at] = own;
+                tree_id[cur ^ 1][at] = id;
+            }
+        } else if (wave < 6) {  // the new ones: one to a lane of two wavefronts, each behind what is left of at most its weight
+            const unsigned w = wave == 4 ? b2[0] : b2[1], k = lane + 64 * (wave - 4);
+            unsigned at = taken;
+            for (unsigned step = 128; step > 0; step >>= 1)
+                if (step <= alive - taken) {
+                    const unsigned to = min(at + step, alive);
+                    at = tree_w[cur][to - 1] <= w ? to : at;
+                }
+            if (k < pairs) {
+                at += k - taken;
+                tree_w[cur ^ 1][at] = w;
+                tree_id[cur ^ 1][at] = NUM_SYMBOLS + made + k;
+            }
+        } else if (wave < 8) {
+            const unsigned k = lane + 64 * (wave - 6);
+            if (k < pairs) parent[tree_id[cur][2 * k]] = parent[tree_id[cur][2 * k + 1]] = made + k;
+        }
+        made += pairs;
+        alive -= pairs;
+        cur ^= 1;
+        __syncthreads();
+    }
+    if (t < NUM_SYMBOLS) {
+        const bool root = n < 2 || t >= n - 2;
+        anc[0][t] = root ? t : parent[NUM_SYMBOLS + t];
+        dep[0][t] = root ? 0 : 1;
+    }
+    __syncthreads();
+    for (int r = 0; r < 8; ++r) {
+        if (t < NUM_SYMBOLS) {
+            const unsigned a = anc[r & 1][t];
+            anc[(r + 1) & 1][t] = anc[r & 1][a];
+            dep[(r + 1) & 1][t] = dep[r & 1][t] + dep[r & 1][a];
+        }
+        __syncthreads();
+    }
+    unsigned len = 0;  // of symbol s (threads with p == 0)
+    if (p == 0 && f > 0) {
+        len = n < 2 ? 1u : min(dep[0][parent[rank_up[s]]] + 1u, (unsigned)KV_MAX_BITS);
+        atomicAdd(&cnt[len], 1u);
+    }
+    __syncthreads();
+    if (wave == 0) {  // uniform: the counts of the twelve lengths in registers
+        const unsigned mine = cnt[lane & 15];
+        unsigned cn[KV_MAX_BITS + 1];
+        int excess = -KV_LUT;  // of the Kraft sum, in 1 / 4096
+#pragma unroll
+        for (int l = 1; l <= KV_MAX_BITS; ++l) {
+            cn[l] = __builtin_amdgcn_readlane(mine, l);
+            excess += (int)cn[l] * (KV_LUT >> l);
+        }
+        const bool too_many = excess > 0;
+        // While there is too much, lengthen by a bit the least frequent symbol of the deepest level below the limit:
+        // it stays the deepest until it gets there, so whole symbols go to the limit level by level, as many as the
+        // excess holds, and the last one part of the way.
+        int part_level = KV_MAX_BITS;
+#pragma unroll
+        for (int l = KV_MAX_BITS - 1; l >= 1; --l) {
+            const int gain = (KV_LUT >> l) - 1;
+            if (excess > 0 && part_level == KV_MAX_BITS) {
+                const unsigned x = min(cn[l], (unsigned)excess / (unsigned)gain);
+                cn[l] -= x;
+                cn[KV_MAX_BITS] += x;
+                excess -= (int)x * gain;
+                if (excess > 0 && cn[l] > 0) part_level = l;
+            }
+        }
+#pragma unroll
+        for (int l = 1; l < KV_MAX_BITS; ++l)
+            if (l >= part_level && excess > 0) {
+                cn[l] -= 1;
+                cn[l + 1] += 1;
+                excess -= KV_LUT >> (l + 1);
+            }
+        unsigned slack = too_many ? (unsigned)-excess : 0u;
+        if (slack > 0) {  // and give what is left to the most frequent symbols
+            unsigned had[KV_MAX_BITS + 1];
+#pragma unroll
+            for (int l = 1; l <= KV_MAX_BITS; ++l) { had[l] = cn[l]; cn[l] = 0; }
+#pragma unroll
+            for (int l = 1; l <= KV_MAX_BITS; ++l) {
+                for (; had[l] > 0 && l > 1 && (unsigned)(KV_LUT >> l) <= slack; --had[l]) {
+                    bool going = true;
+#pragma unroll
+                    for (int m = l; m >= 1; --m) {
+                        const bool shorter = going && m > 1 && (unsigned)(KV_LUT >> m) <= slack;
+                        if (shorter) slack -= KV_LUT >> m;
+                        else if (going) cn[m] += 1;
+                        going = shorter;
+                    }
+                }
+                cn[l] += had[l];
+            }
+        }
+        unsigned code = 0, off = 0;
+#pragma unroll
+        for (int l = 1; l <= KV_MAX_BITS; ++l) {  // src/huffman.rs:152-186
+            code <<= 1;
+            if (t == 0) {
+                first_code[l] = code;
+                offset[l] = off;
+                limit[l] = (code + cn[l]) << (KV_MAX_BITS - l);
+            }
+            code += cn[l];
+            off += cn[l];
+        }
+        if (t == 0) {
+            offset[KV_MAX_BITS + 1] = off;
+            over = too_many;
+        }
+    }
+    __syncthreads();
+    if (over) {  // the repaired lengths go out again, shortest to most frequent (ties: lower symbol first)
+        const unsigned long long down_key = f ? (unsigned long long)~f << 8 | s : ~0ull;
+        if (p == 0) keys[s] = down_key;
+        __syncthreads();
+        unsigned down = 0;
+#pragma unroll 8
+        for (unsigned o = p * 64; o < p * 64 + 64; ++o) down += keys[o] < down_key;
+        atomicAdd(&rank_down[s], down);
+        __syncthreads();
+        if (p == 0 && f > 0) {
+            len = 1;
+#pragma unroll
+            for (int l = 2; l <= KV_MAX_BITS; ++l) len += offset[l] <= rank_down[s] ? 1 : 0;
+        }
+    }
+    if (p == 0) bl[s] = (uint8_t)len;
+    // the symbol's place among those of its length
+    unsigned before = 0;
+    if (p == 0) {
+        for (unsigned l = 1; l <= KV_MAX_BITS; ++l) {
+            const unsigned long long m = __ballot(len == l);
+            if (len == l) before = __popcll(m & ((1ull << (t & 63)) - 1));
+            if ((t & 63) == 0) lane_cnt[t >> 6][l] = __popcll(m);
+        }
+    }
+    __syncthreads();
+    if (p == 0) {
+        unsigned e = 0;
+        if (len) {
+            for (unsigned w = 0; w < (t >> 6); ++w) before += lane_cnt[w][len];
+            e = len << 16 | (first_code[len] + before);
+            by_len[offset[len] + before] = (uint8_t)s;
+        }
+        b.codes[(size_t)c * NUM_SYMBOLS + s] = e;
+    }
+    __syncthreads();
+    {   // decode table, four entries a thread: length << 8 | symbol; codes nobody has decode as (length 0, value 0)
+        ushort4 e;
+        uint16_t *ev = reinterpret_cast<uint16_t *>(&e);
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k) {
+            const unsigned x = t * 4 + k;
+            unsigned l = 1;  // (the limits ascend)
+#pragma unroll
+            for (int i = 1; i <= KV_MAX_BITS; ++i) l += x >= limit[i] ? 1 : 0;
+            const unsigned at = l > KV_MAX_BITS ? 0 : offset[l] + (x >> (KV_MAX_BITS - l)) - first_code[l];
+            ev[k] = l > KV_MAX_BITS ? (uint16_t)128 : (uint16_t)(l << 8 | by_len[at]);
+        }
+        reinterpret_cast<ushort4 *>(b.lut + (size_t)c * KV_LUT)[t] = e;
+    }
+    // bits of every run of 4096 values, and their running sum
+    const uchar4 lens = reinterpret_cast<const uchar4 *>(bl)[lane];
+    unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
+    unsigned long long run = 0;
+    for (unsigned at = 0; at < b.nwg; at += 1024) {
+        for (unsigned i = at + wave; i < min(at + 1024u, b.nwg); i += 16) {
+            const ushort4 h = reinterpret_cast<const ushort4 *>(hist + (size_t)i * NUM_SYMBOLS)[lane];
+            const int bits = pg_wave_sum_i32((int)(h.x * lens.x + h.y * lens.y + h.z * lens.z + h.w * lens.w));
+            if (lane == 0) run_bits[i - at] = (unsigned)bits;
+        }
+        __syncthreads();
+        const unsigned v = at + t < b.nwg ? run_bits[t] : 0u;
+        unsigned incl = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned o = __shfl_up(incl, d, 64);
+            incl += lane >= (unsigned)d ? o : 0u;
+        }
+        if (lane == 63) wsum[wave] = incl;
+        __syncthreads();
+        unsigned long long pre = run;
+        for (unsigned w = 0; w < wave; ++w) pre += wsum[w];
+        if (at + t < b.nwg) wg_bit[at + t] = pre + incl - v;
+        for (unsigned w = 0; w < 16; ++w) run += wsum[w];
+        __syncthreads();
+    }
+    if (t == 0) {
+        wg_bit[b.nwg] = run;
+        __hip_atomic_store(host_bits + c, run + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);  // (0 = not there yet)
+    }
+}
+
+// Where up to KV_PLACES chunks of a batch, from number `first` on, are written to.
+constexpr unsigned KV_PLACES = 32;
+struct kv_places {
+    unsigned first;
+    char *at[KV_PLACES];
+    // the window's rows that move to the front in the same launch (workgroups behind the chunks', which read the int8
+    // values only): heads of both sides, `rest` values each, from `from` values on
+    float *hot[2];
+    size_t hot_stride, from, rest;
+};
+
+// Appends the code `e` (length << 16 | code) to a right-aligned window; returns the next whole word if one is full.
+__device__ __forceinline__ bool push_code(unsigned e, unsigned long long &acc, unsigned &nacc, unsigned &word) {
+    const unsigned l = e >> 16;
+    acc = (acc << l) | (e & 0xFFFFu);
+    nacc += l;
+    if (nacc < 32) return false;
+    nacc -= 32;
+    word = (unsigned)(acc >> nacc);
+    acc &= (1ull << nacc) - 1ull;
+    return true;
+}
+
+// HuffmanTable::encode (src/huffman.rs:216-251) in parallel: grid (nwg, chunks).  A workgroup's bit range is
+// known; its threads put their codes together in LDS and the workgroup stores the words that START in its
+// range, whole: the bits that the last of them takes from the next run it encodes itself (up to 31 values), so no word
+// has two writers and nothing is zeroed first.
+__global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, const kv_places places, char **__restrict__ table) {
+    __shared__ unsigned lc[NUM_SYMBOLS], wsum[4];
+    __shared__ unsigned words[ENC_PER_WG * KV_MAX_BITS / 32 + 2];
+    const unsigned c = places.first + blockIdx.y, g = blockIdx.x, t = threadIdx.x, lane = t & 63;
+    if (c >= b.count) {
+        const unsigned row = c - b.count;
+        float *p = places.hot[row / b.heads] + (size_t)(row % b.heads) * places.hot_stride;
+        for (size_t i = (size_t)g * KV_WG + t; i < places.rest; i += (size_t)gridDim.x * KV_WG) p[i] = p[places.from + i];
+        return;
+    }
+    const kv_layout lay(b.heads, b.total, true);
+    char *dst = places.at[blockIdx.y];
+    const unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
+    const unsigned long long first = wg_bit[g], last = wg_bit[g + 1];
+    lc[t] = b.codes[(size_t)c * NUM_SYMBOLS + t];
+    for (unsigned i = t; i < sizeof(words) / 4; i += KV_WG) words[i] = 0;
+    const int8_t *q = b.q + (size_t)c * b.q_stride;
+    const unsigned base = g * ENC_PER_WG + t * ENC_SPT;
+    const unsigned count = base >= b.total ? 0u : min(b.total - base, (unsigned)ENC_SPT);
+    uint4 v = {0, 0, 0, 0};
+    if (count) v = *reinterpret_cast<const uint4 *>(q + base);  // (q is padded to a multiple of 16)
+    __syncthreads();
+    const unsigned sw[4] = {v.x, v.y, v.z, v.w};
+    unsigned bits = 0;
+#pragma unroll
+    for (unsigned j = 0; j < ENC_SPT; ++j)
+        if (j < count) bits += lc[((sw[j >> 2] >> (8 * (j & 3))) & 255u) ^ 128u] >> 16;
+    unsigned incl = bits;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned o = __shfl_up(incl, d, 64);
+        incl += lane >= (unsigned)d ? o : 0u;
+    }
+    if (lane == 63) wsum[t >> 6] = incl;
+    __syncthreads();
+    unsigned start = incl - bits;  // within the run
+    for (unsigned w = 0; w < (t >> 6); ++w) start += wsum[w];
+    if (count && (t & (SUB_SYMS / ENC_SPT - 1)) == 0)
+        reinterpret_cast<uint16_t *>(dst + lay.o_sub)[base / SUB_SYMS] = (uint16_t)start;  // below 4096 * 12
+    const unsigned r = (unsigned)(first & 31);  // bits of the first word that belong to the run before
+    {
+        unsigned k = (r + start) >> 5, nacc = (r + start) & 31, word;
+        unsigned long long acc = 0;
+#pragma unroll
+        for (unsigned j = 0; j < ENC_SPT; ++j)
+            if (j < count && push_code(lc[((sw[j >> 2] >> (8 * (j & 3))) & 255u) ^ 128u], acc, nacc, word)) atomicOr(&words[k++], word);
+        if (nacc && count) atomicOr(&words[k], (unsigned)(acc << (32 - nacc)));
+    }
+    __syncthreads();
+    if (t == 0 && ((unsigned)last & 31)) {  // fill the last word up from the next run
+        unsigned nacc = (unsigned)last & 31, k = (unsigned)((last >> 5) - (first >> 5)), word;
+        unsigned long long acc = words[k] >> (32 - nacc);
+        bool full = false;
+        for (unsigned i = (g + 1) * ENC_PER_WG; !full && i < b.total; ++i) full = push_code(lc[(unsigned)(uint8_t)q[i] ^ 128u], acc, nacc, word);
+        words[k] = full ? word : (unsigned)(acc << (32 - nacc));
+    }
+    __syncthreads();
+    unsigned *out = reinterpret_cast<unsigned *>(dst + lay.o_bits) + (size_t)(first >> 5);
+    const unsigned nwords = (unsigned)(((last + 31) >> 5) - (first >> 5));
+    for (unsigned i = t + (r ? 1 : 0); i < nwords; i += KV_WG) out[i] = __builtin_bswap32(words[i]);
+    if (t == 0) reinterpret_cast<unsigned long long *>(dst + lay.o_wg)[g] = first;
+    if (g == 0) {  // the chunk's head
+        for (unsigned h = t; h < b.heads; h += KV_WG) reinterpret_cast<float *>(dst)[h] = b.scales[(size_t)c * b.heads + h];
+        dst[lay.o_book + t] = (char)(lc[t] >> 16);
+        const uint4 *lut = reinterpret_cast<const uint4 *>(b.lut + (size_t)c * KV_LUT);
+        for (unsigned i = t; i < KV_LUT * 2 / 16; i += KV_WG) reinterpret_cast<uint4 *>(dst + lay.o_lut)[i] = lut[i];
+        if (t == 0) {
+            reinterpret_cast<unsigned long long *>(dst + lay.o_wg)[b.nwg] = wg_bit[b.nwg];
+            if (table) table[c] = dst;
+        }
+        if (t < 4) reinterpret_cast<unsigned *>(dst + lay.o_bits)[(size_t)((wg_bit[b.nwg] + 31) >> 5) + t] = 0;  // the padding
+    }
+}
+
+// Chunks with an index, decoded, scaled and laid out, and the window copied behind them.  Chunk c (address table[c], or
+// `single`) is side c % sides, number c / sides: its head h goes to out[side] + number * chunk_step + h * out_stride.
+struct kv_decode_args {
+    char *const *table;
+    const char *single;
+    float *out[2];
+    size_t chunk_step, out_stride;
+    unsigned sides, count, heads, head_elems, total, wgs;  // wgs = workgroups per chunk
+    const float *hot[2];       // window rows: head h at hot[side] + h * hot_stride, hot_elems values to out[side] + hot_at + h * out_stride
+    size_t hot_stride, hot_at;
+    unsigned hot_elems, hot_wgs;  // hot_wgs = workgroups per (side, head)
+};
+
+// A thread decodes SUB_SYMS values from the bit the index names: table and stream in LDS (the workgroup's part of the
+// stream is contiguous), a 64-bit window in registers with the next word already read; the values go through LDS so
+// that the f32 stores are whole lines.  What it takes is the chain of 64 table look-ups: 20 chunks of 262144 values in
+// 19 us, where the search for code boundaries, the scans, the write pass and the scaling launch took 170.
+template <bool VEC>
+__global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a) {
+    constexpr unsigned MAX_WORDS = DEC_PER_WG * KV_MAX_BITS / 32 + 4;
+    __shared__ __attribute__((aligned(16))) uint16_t lut[KV_LUT];
+    __shared__ unsigned words[MAX_WORDS];
+    __shared__ unsigned sym[KV_WG * (SUB_SYMS / 4 + 1)];  // four values a word; a thread's words start an odd number apart
+    const unsigned t = threadIdx.x, nchunk = a.count * a.wgs;
+    if (blockIdx.x >= nchunk) {  // the window
+        const unsigned g = blockIdx.x - nchunk, row = g / a.hot_wgs, part = g % a.hot_wgs, side = row / a.heads, h = row % a.heads;
+        const float *src = a.hot[side] + (size_t)h * a.hot_stride;
+        float *dst = a.out[side] + a.hot_at + (size_t)h * a.out_stride;
+        const unsigned end = min(a.hot_elems, (part + 1) * DEC_PER_WG);
+        if (VEC)
+            for (unsigned i = part * DEC_PER_WG + t * 4; i < end; i += KV_WG * 4) *reinterpret_cast<float4 *>(dst + i) = *reinterpret_cast<const float4 *>(src + i);
+        else
+            for (unsigned i = part * DEC_PER_WG + t; i < end; i += KV_WG) dst[i] = src[i];
+        return;
+    }
+    const unsigned c = blockIdx.x / a.wgs, g = blockIdx.x % a.wgs;
+    const char *chunk = a.table ? a.table[c] : a.single;
+    const kv_layout lay(a.heads, a.total, true);
+    const uint4 *lut_g = reinterpret_cast<const uint4 *>(chunk + lay.o_lut);
+    for (unsigned i = t; i < KV_LUT * 2 / 16; i += KV_WG) reinterpret_cast<uint4 *>(lut)[i] = lut_g[i];
+    constexpr unsigned RUNS = DEC_PER_WG / ENC_PER_WG;
+    const unsigned long long *wg_bit = reinterpret_cast<const unsigned long long *>(chunk + lay.o_wg);
+    const unsigned nwg = (a.total + ENC_PER_WG - 1) / ENC_PER_WG, r0 = g * RUNS, r1 = min(r0 + RUNS, nwg);
+    const unsigned long long w0 = wg_bit[r0] >> 5, w1 = (wg_bit[r1] + 31) >> 5;
+    const unsigned *stream = reinterpret_cast<const unsigned *>(chunk + lay.o_bits) + w0;
+    const unsigned nwords = min((unsigned)(w1 - w0) + 3, MAX_WORDS);  // (up to 16 bytes of padding follow a stream)
+    for (unsigned i = t; i < nwords; i += KV_WG) words[i] = __builtin_bswap32(stream[i]);
+    const unsigned base = g * DEC_PER_WG, sub = g * KV_WG + t;
+    const unsigned count = base + t * SUB_SYMS >= a.total ? 0u : min(a.total - (base + t * SUB_SYMS), (unsigned)SUB_SYMS);
+    unsigned pos = 0;
+    if (count)
+        pos = (unsigned)(wg_bit[sub / (ENC_PER_WG / SUB_SYMS)] - (w0 << 5)) + reinterpret_cast<const uint16_t *>(chunk + lay.o_sub)[sub];
+    __syncthreads();
+    if (count) {
+        unsigned k = pos >> 5;
+        unsigned long long buf = ((unsigned long long)words[k] << 32 | words[k + 1]) << (pos & 31);
+        unsigned avail = 64 - (pos & 31);
+        k += 2;
+        unsigned next = words[k];
+        unsigned *o = sym + t * (SUB_SYMS / 4 + 1);
+        for (unsigned j = 0; j < count; j += 4) {
+            unsigned four = 0;
+#pragma unroll
+            for (unsigned i = 0; i < 4; ++i) {
+                const unsigned e = lut[buf >> (64 - KV_MAX_BITS)], l = e >> 8;
+                four |= (e & 255u) << (8 * i);
+                buf <<= l;
+                avail -= l;
+                if (avail <= 32) {
+                    buf |= (unsigned long long)next << (32 - avail);
+                    avail += 32;
+                    k = min(k + 1, MAX_WORDS - 1);
+                    next = words[k];
+                }
+            }
+            o[j / 4] = four;
+        }
+    }
+    __syncthreads();
+    const float *scales = reinterpret_cast<const float *>(chunk);
+    float *out = a.out[c % a.sides] + (size_t)(c / a.sides) * a.chunk_step;
+#pragma unroll 4
+    for (unsigned j = 0; j < DEC_PER_WG / (4 * KV_WG); ++j) {
+        const unsigned local = (j * KV_WG + t) * 4, i = base + local;
+        if (i >= a.total) break;
+        const unsigned four = sym[local / SUB_SYMS * (SUB_SYMS / 4 + 1) + local % SUB_SYMS / 4];
+        if (VEC) {
+            const unsigned h = i / a.head_elems;
+            const float scale = scales[h];
+            float4 v;
+            v.x = (float)((int)(four & 255u) - 128) * scale;
+            v.y = (float)((int)(four >> 8 & 255u) - 128) * scale;
+            v.z = (float)((int)(four >> 16 & 255u) - 128) * scale;
+            v.w = (float)((int)(four >> 24) - 128) * scale;
+            *reinterpret_cast<float4 *>(out + (size_t)h * a.out_stride + (i - h * a.head_elems)) = v;
+        } else {
+            for (unsigned k = 0; k < 4 && i + k < a.total; ++k) {
+                const unsigned h = (i + k) / a.head_elems;
+                out[(size_t)h * a.out_stride + (i + k - h * a.head_elems)] = (float)((int)(four >> (8 * k) & 255u) - 128) * scales[h];
+            }
+        }
+    }
 }
 
 // decoded_i8 as f32 * scale[head]   src/huffman.rs:669-677 for several chunks in one launch: grid
@@ -190,21 +638,22 @@ unsigned splits_for(size_t head_elems) {
 
 }  // namespace
 
-// CompressedChunk  src/huffman.rs:500-513 with its bitstream (and a copy of the scales) in device memory.
+// CompressedChunk  src/huffman.rs:500-513 in device memory (kv_layout).
 struct pg_huffman_kv_chunk {
-    uint8_t codebook[NUM_SYMBOLS];
-    std::vector<float> scales;
-    char *dev = nullptr;  // [scales, 256-byte rounded][decode table][bitstream, zero padded to a whole word and 16 bytes on]
-    size_t bytes = 0;     // of the bitstream
+    mutable uint8_t codebook[NUM_SYMBOLS];  // copies of what the device holds, once `on_host`
+    mutable std::vector<float> scales;
+    mutable bool on_host = false;
+    std::shared_ptr<pg_dev_block> block;  // shared by the chunks of a batch
+    char *dev = nullptr;
+    size_t bytes = 0;  // of the bitstream
     size_t num_tokens = 0, num_heads = 0, head_dim = 0;
     bool decodable = false;  // the codebook fits the decode table (always, for chunks made here)
-    size_t scales_bytes() const { return pg_round_up(num_heads * sizeof(float), 256); }
-    size_t head_bytes() const { return scales_bytes() + pg_huffman_lut_entries() * sizeof(uint16_t); }
-    const float *scales_dev() const { return reinterpret_cast<const float *>(dev); }
-    const uint16_t *lut_dev() const { return reinterpret_cast<const uint16_t *>(dev + scales_bytes()); }
-    const uint8_t *bits_dev() const { return reinterpret_cast<const uint8_t *>(dev + head_bytes()); }
+    bool indexed = false;    // made here: with the index the one-launch decoder reads
     size_t symbols() const { return num_heads * num_tokens * head_dim; }
-    ~pg_huffman_kv_chunk() { if (dev) (void)hipFree(dev); }
+    kv_layout layout() const { return kv_layout(num_heads, symbols(), indexed); }
+    const float *scales_dev() const { return reinterpret_cast<const float *>(dev); }
+    const uint16_t *lut_dev() const { return reinterpret_cast<const uint16_t *>(dev + layout().o_lut); }
+    const uint8_t *bits_dev() const { return reinterpret_cast<const uint8_t *>(dev + layout().o_bits); }
 };
 
 // HuffmanKVCache  src/huffman.rs:484-497
@@ -212,6 +661,23 @@ struct pg_huffman_kv_cache {
     pg_kv_cache *hot = nullptr;
     std::vector<pg_huffman_kv_chunk *> k_chunks, v_chunks;
     size_t compressed_len = 0, compress_threshold = 0, chunk_size = 0;
+    // The chunks' addresses on the device, key and value side in turn (written by the encoder).  An outgrown table
+    // may still be read by work in flight and stays until the cache goes.
+    pg_dev_block table_mem;
+    char **table = nullptr;
+    size_t table_cap = 0;
+    std::vector<pg_dev_block> old_tables;
+    bool foreign() const { return hot->k_mem.foreign || table_mem.foreign; }
+    // Before ctx's stream uses any of it.  (Once another context has, the chunks' blocks are marked one by one.)
+    void touch(const pg_ctx *ctx) {
+        const bool was = foreign();
+        hot->touch(ctx);
+        table_mem.touch(ctx);
+        if (!foreign() || was) return;
+        for (auto *v : {&k_chunks, &v_chunks})
+            for (auto *p : *v) p->block->foreign = true;
+        for (auto &t : old_tables) t.foreign = true;
+    }
 };
 
 static pg_status chunk_shape_ok(const char *who, size_t num_tokens, size_t num_heads, size_t head_dim) {
@@ -223,21 +689,127 @@ static pg_status chunk_shape_ok(const char *who, size_t num_tokens, size_t num_h
     return PG_OK;
 }
 
-// Allocates the chunk's device memory, zeroes it (stream ordered) and puts the decode table of c->codebook in place.
+// Allocates the device memory of a chunk without an index, zeroes it (stream ordered) and puts scales and the decode
+// table of c->codebook in place.
 static pg_status chunk_alloc(pg_ctx *ctx, pg_huffman_kv_chunk *c, size_t bytes) {
     c->bytes = bytes;
-    const size_t total = c->head_bytes() + pg_round_up(bytes, 4) + 16;
-    hipError_t e = hipMalloc((void **)&c->dev, total);
-    if (e != hipSuccess) {
-        c->dev = nullptr;
-        return pg_fail(PG_ENOMEM, "hipMalloc(%zu) failed: %s", total, hipGetErrorString(e));
-    }
-    PG_HIP(hipMemsetAsync(c->dev, 0, total, ctx->stream));
-    std::vector<uint16_t> lut(pg_huffman_lut_entries());
+    c->on_host = true;
+    const kv_layout lay = c->layout();
+    c->block = std::make_shared<pg_dev_block>();
+    PG_TRY(c->block->alloc(ctx, lay.size(bytes)));
+    c->dev = static_cast<char *>(c->block->p);
+    PG_HIP(hipMemsetAsync(c->dev, 0, lay.size(bytes), ctx->stream));
+    std::vector<uint16_t> lut(KV_LUT);
     c->decodable = pg_huffman_host_lut(c->codebook, lut.data()) == PG_OK;  // else: reported when the chunk is decoded
-    if (c->decodable) {
-        PG_HIP(hipMemcpyAsync(c->dev + c->scales_bytes(), lut.data(), lut.size() * sizeof(uint16_t), hipMemcpyHostToDevice, ctx->stream));
-        PG_HIP(hipStreamSynchronize(ctx->stream));  // lut is a local
+    if (c->num_heads) PG_HIP(hipMemcpyAsync(c->dev, c->scales.data(), c->num_heads * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    if (c->decodable)
+        PG_HIP(hipMemcpyAsync(c->dev + lay.o_lut, lut.data(), lut.size() * sizeof(uint16_t), hipMemcpyHostToDevice, ctx->stream));
+    PG_HIP(hipStreamSynchronize(ctx->stream));  // lut is a local
+    return PG_OK;
+}
+
+// Waits until the `n` words at `words` (pinned, zeroed before the launch that stores them) are there.  The kernel that
+// stores them is usually a few tens of microseconds away and waking from a stream wait costs ten: so this looks for a
+// while first.
+static pg_status wait_for_words(pg_ctx *ctx, const uint64_t *words, size_t n) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    size_t have = 0;
+    for (;;) {
+        while (have < n && __atomic_load_n(words + have, __ATOMIC_ACQUIRE)) ++have;
+        if (have == n) return PG_OK;
+        if (std::chrono::steady_clock::now() > until) break;
+    }
+    PG_HIP(hipStreamSynchronize(ctx->stream));
+    for (; have < n; ++have)
+        if (!__atomic_load_n(words + have, __ATOMIC_ACQUIRE)) return pg_fail(PG_EDEVICE, "huffman kv: the table kernel left no size");
+    return PG_OK;
+}
+
+// The window's move to the front, for compress_batch to fold into its last launch (done = true) where it can.
+struct kv_shift {
+    float *hot[2];
+    size_t stride, from, rest;
+    bool done = false;
+};
+
+// compress_chunk of `count` chunks of one shape (none of them empty), chunk c being number c / sides of side c % sides:
+// head h of it starts at data[side] + number * chunk_step + h * head_stride.  Their addresses go to table_dev[0 ..) if given.
+static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t sides, size_t count, size_t chunk_step, size_t head_stride,
+                                size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift,
+                                std::vector<std::unique_ptr<pg_huffman_kv_chunk>> &out) {
+    const size_t head_elems = num_tokens * head_dim, total = num_heads * head_elems;
+    const size_t nwg = (total + ENC_PER_WG - 1) / ENC_PER_WG;
+    const size_t most = std::max<size_t>(1, std::min<size_t>(KV_BATCH_SYMBOLS / total, KV_BATCH_CHUNKS) / sides) * sides;
+    for (size_t first = 0; first < count; first += most) {
+        kv_batch b;
+        const size_t n = std::min(most, count - first);
+        bool vec = head_elems % 4 == 0 && head_stride % 4 == 0 && chunk_step % 4 == 0;
+        for (size_t s = 0; s < 2; ++s) {
+            b.data[s] = data[s < sides ? s : 0] + first / sides * chunk_step;
+            vec = vec && (uintptr_t)b.data[s] % 16 == 0;
+        }
+        b.chunk_step = chunk_step; b.head_stride = head_stride;
+        b.sides = (unsigned)sides; b.count = (unsigned)n; b.heads = (unsigned)num_heads; b.head_elems = (unsigned)head_elems;
+        b.total = (unsigned)total; b.nwg = (unsigned)nwg;
+        b.splits = (unsigned)std::min<size_t>(std::max<size_t>((head_elems + ENC_PER_WG - 1) / ENC_PER_WG, 1), KV_MAX_SPLITS);
+        b.q_stride = pg_round_up(total, 16);
+        size_t off = 0;
+        auto take = [&](size_t bytes) { const size_t at = off; off += pg_round_up(bytes, 256); return at; };
+        const size_t o_amax = take(n * num_heads * b.splits * 4), o_scales = take(n * num_heads * 4), o_q = take(n * b.q_stride);
+        const size_t o_hist = take(n * nwg * NUM_SYMBOLS * 2), o_bit = take(n * (nwg + 1) * 8), o_codes = take(n * NUM_SYMBOLS * 4);
+        const size_t o_lut = take(n * KV_LUT * 2);
+        void *ws = nullptr, *pin = nullptr;
+        PG_TRY(pg_workspace(ctx, off, &ws));
+        PG_TRY(pg_pinned(ctx, n * sizeof(uint64_t), &pin));
+        char *base = static_cast<char *>(ws);
+        b.amax = reinterpret_cast<float *>(base + o_amax);
+        b.scales = reinterpret_cast<float *>(base + o_scales);
+        b.q = reinterpret_cast<int8_t *>(base + o_q);
+        b.hist = reinterpret_cast<uint16_t *>(base + o_hist);
+        b.wg_bit = reinterpret_cast<unsigned long long *>(base + o_bit);
+        b.codes = reinterpret_cast<unsigned *>(base + o_codes);
+        b.lut = reinterpret_cast<uint16_t *>(base + o_lut);
+        uint64_t *sizes = static_cast<uint64_t *>(pin);
+        std::fill(sizes, sizes + n, (uint64_t)0);
+        PG_TRY(pg_launch(ctx, "huffman_kv_absmax", kv_absmax_kernel, dim3(b.splits, b.heads, b.count), dim3(KV_WG), 0, b, (int)vec));
+        PG_TRY(pg_launch(ctx, "huffman_kv_quant", kv_quant_hist_kernel, dim3(b.nwg, b.count), dim3(KV_WG), 0, b, (int)vec));
+        PG_TRY(pg_launch(ctx, "huffman_kv_table", kv_table_kernel, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
+        const kv_layout lay(num_heads, total, true);
+        PG_TRY(wait_for_words(ctx, sizes, n));
+        size_t bytes = 0;
+        for (size_t c = 0; c < n; ++c) bytes += lay.size((sizes[c] - 1 + 7) / 8);
+        auto block = std::make_shared<pg_dev_block>();
+        PG_TRY(block->alloc(ctx, bytes));
+        char *at = static_cast<char *>(block->p);
+        for (size_t c0 = 0; c0 < n; c0 += KV_PLACES) {
+            kv_places places;
+            places.first = (unsigned)c0;
+            const size_t here = std::min<size_t>(KV_PLACES, n - c0);
+            for (size_t c = c0; c < c0 + here; ++c) {
+                std::unique_ptr<pg_huffman_kv_chunk> ch(new (std::nothrow) pg_huffman_kv_chunk());
+                if (!ch) return pg_fail(PG_ENOMEM, "host allocation failed");
+                ch->num_tokens = num_tokens; ch->num_heads = num_heads; ch->head_dim = head_dim;
+                ch->block = block;
+                ch->dev = at;
+                ch->bytes = (size_t)((sizes[c] - 1 + 7) / 8);
+                ch->decodable = ch->indexed = true;
+                places.at[c - c0] = at;
+                at += lay.size(ch->bytes);
+                out.push_back(std::move(ch));
+            }
+            size_t rows = 0;
+            if (shift && first + c0 + here == count && shift->rest <= shift->from && here + sides * num_heads <= 65535) {  // (no row reads what it writes)
+                places.hot[0] = shift->hot[0];
+                places.hot[1] = shift->hot[1];
+                places.hot_stride = shift->stride;
+                places.from = shift->from;
+                places.rest = shift->rest;
+                rows = sides * num_heads;
+                shift->done = true;
+            }
+            PG_TRY(pg_launch(ctx, "huffman_kv_encode", kv_encode_kernel, dim3(b.nwg, (unsigned)(here + rows)), dim3(KV_WG), 0, b, places,
+                             table_dev ? table_dev + first : nullptr));
+        }
     }
     return PG_OK;
 }
@@ -247,68 +819,34 @@ static pg_status compress_dev(pg_ctx *ctx, const float *data, size_t head_stride
                               size_t head_dim, pg_huffman_kv_chunk **out) {
     *out = nullptr;
     PG_TRY(chunk_shape_ok("huffman kv compress_chunk", num_tokens, num_heads, head_dim));
-    pg_huffman_kv_chunk *c = new (std::nothrow) pg_huffman_kv_chunk();
-    if (!c) return pg_fail(PG_ENOMEM, "host allocation failed");
-    struct guard { pg_huffman_kv_chunk *c; ~guard() { delete c; } } g{c};
-    c->num_tokens = num_tokens; c->num_heads = num_heads; c->head_dim = head_dim;
-    std::fill(c->codebook, c->codebook + NUM_SYMBOLS, (uint8_t)0);
-    c->scales.assign(num_heads, 1.0f);  // absmax == 0.0 -> 1.0
-    const size_t head_elems = num_tokens * head_dim, total = num_heads * head_elems;
-    if (total == 0) {  // an empty table, an empty stream
-        PG_TRY(chunk_alloc(ctx, c, 0));
-        if (num_heads)
-            PG_HIP(hipMemcpyAsync(c->dev, c->scales.data(), num_heads * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-        PG_HIP(hipStreamSynchronize(ctx->stream));
-        g.c = nullptr;
-        *out = c;
+    if (num_tokens * num_heads * head_dim == 0) {  // an empty table, an empty stream; absmax == 0.0 -> scale 1.0
+        std::unique_ptr<pg_huffman_kv_chunk> c(new (std::nothrow) pg_huffman_kv_chunk());
+        if (!c) return pg_fail(PG_ENOMEM, "host allocation failed");
+        c->num_tokens = num_tokens; c->num_heads = num_heads; c->head_dim = head_dim;
+        std::fill(c->codebook, c->codebook + NUM_SYMBOLS, (uint8_t)0);
+        c->scales.assign(num_heads, 1.0f);
+        PG_TRY(chunk_alloc(ctx, c.get(), 0));
+        *out = c.release();
         return PG_OK;
     }
-    const size_t nwg = (total + ENC_PER_WG - 1) / ENC_PER_WG;
-    // amax | scales | hist | codes | wg bits (+ total) | q
-    const size_t o_scale = pg_round_up(num_heads * 4, 256), o_hist = o_scale + pg_round_up(num_heads * 4, 256);
-    const size_t o_codes = o_hist + NUM_SYMBOLS * 8, o_wg = o_codes + NUM_SYMBOLS * 4;
-    const size_t o_q = o_wg + pg_round_up((nwg + 1) * 8, 256);
-    pg_tmp buf;
-    PG_TRY(buf.alloc(o_q + pg_round_up(total, 16)));
-    char *base = buf.as<char>();
-    auto *d_amax = reinterpret_cast<unsigned *>(base);
-    auto *d_scales = reinterpret_cast<float *>(base + o_scale);
-    auto *d_hist = reinterpret_cast<unsigned long long *>(base + o_hist);
-    auto *d_codes = reinterpret_cast<unsigned *>(base + o_codes);
-    auto *d_wg = reinterpret_cast<unsigned long long *>(base + o_wg);
-    auto *d_q = reinterpret_cast<int8_t *>(base + o_q);
-    PG_HIP(hipMemsetAsync(base, 0, o_codes, ctx->stream));
-    const dim3 grid(splits_for(head_elems), (unsigned)num_heads);
-    PG_TRY(pg_launch(ctx, "huffman_kv_absmax", kv_absmax_kernel, grid, dim3(KV_WG), 0, data, head_stride, head_elems, d_amax));
-    PG_TRY(pg_launch(ctx, "huffman_kv_quant", kv_quant_hist_kernel, grid, dim3(KV_WG), 0, data, head_stride, head_elems,
-                     (const unsigned *)d_amax, d_q, d_scales, d_hist));
-    uint64_t freqs[NUM_SYMBOLS];
-    static_assert(sizeof(uint64_t) == sizeof(unsigned long long), "histogram element size");
-    PG_HIP(hipMemcpyAsync(freqs, d_hist, sizeof freqs, hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipMemcpyAsync(c->scales.data(), d_scales, num_heads * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    uint32_t codes[NUM_SYMBOLS];
-    (void)pg_huffman_host_table(freqs, c->codebook, codes);  // the reference's table wherever that one decodes
-    for (int s = 0; s < NUM_SYMBOLS; ++s) codes[s] = (uint32_t)c->codebook[s] << 16 | (codes[s] & 0xFFFFu);
-    PG_HIP(hipMemcpyAsync(d_codes, codes, sizeof codes, hipMemcpyHostToDevice, ctx->stream));
-    PG_TRY(pg_launch(ctx, "huffman_kv_encode_bits", kv_encode_bits_kernel, dim3((unsigned)nwg), dim3(KV_WG), 0,
-                     (const int8_t *)d_q, total, (const unsigned *)d_codes, d_wg));
-    PG_TRY(pg_launch(ctx, "huffman_kv_encode_scan", kv_encode_scan_kernel, dim3(1), dim3(KV_WG), 0, d_wg, nwg));
-    unsigned long long bits = 0;
-    PG_HIP(hipMemcpyAsync(&bits, d_wg + nwg, sizeof bits, hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    PG_TRY(chunk_alloc(ctx, c, (size_t)((bits + 7) / 8)));
-    PG_HIP(hipMemcpyAsync(c->dev, d_scales, num_heads * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
-    PG_TRY(pg_launch(ctx, "huffman_kv_encode_write", kv_encode_write_kernel, dim3((unsigned)nwg), dim3(KV_WG), 0,
-                     (const int8_t *)d_q, total, (const unsigned *)d_codes, (const unsigned long long *)d_wg,
-                     reinterpret_cast<unsigned *>(c->dev + c->head_bytes())));
-    PG_HIP(hipStreamSynchronize(ctx->stream));  // buf is freed on return
-    g.c = nullptr;
-    *out = c;
+    std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
+    PG_TRY(compress_batch(ctx, &data, 1, 1, 0, head_stride, num_tokens, num_heads, head_dim, nullptr, nullptr, made));
+    *out = made[0].release();
     return PG_OK;
 }
 
-// decompress_chunk for several chunks in one pass: chunk i's head h goes to out[i] + h * out_stride[i].
+// The one-launch decoder over chunks of one shape with an index (args.table or args.single), and the window's rows.
+static pg_status launch_decode(pg_ctx *ctx, kv_decode_args a) {
+    bool vec = a.head_elems % 4 == 0 && a.out_stride % 4 == 0 && a.chunk_step % 4 == 0 && a.hot_elems % 4 == 0 && a.hot_stride % 4 == 0 && a.hot_at % 4 == 0;
+    for (unsigned s = 0; s < a.sides; ++s) vec = vec && (uintptr_t)a.out[s] % 16 == 0 && (uintptr_t)a.hot[s] % 16 == 0;
+    a.wgs = (a.total + DEC_PER_WG - 1) / DEC_PER_WG;
+    a.hot_wgs = (a.hot_elems + DEC_PER_WG - 1) / DEC_PER_WG;
+    const size_t grid = (size_t)a.count * a.wgs + (size_t)a.hot_wgs * a.sides * a.heads;
+    if (grid == 0) return PG_OK;
+    return pg_launch(ctx, "huffman_kv_decode", vec ? kv_decode_kernel<true> : kv_decode_kernel<false>, dim3((unsigned)grid), dim3(KV_WG), 0, a);
+}
+
+// decompress_chunk of chunks made from stored parts, several in one pass: chunk i's head h goes to out[i] + h * out_stride[i].
 static pg_status decompress_many(pg_ctx *ctx, const pg_huffman_kv_chunk *const *chunks, float *const *out, const size_t *out_stride,
                                  size_t count) {
     std::vector<pg_huffman_dev_stream> streams;
@@ -342,7 +880,15 @@ static pg_status decompress_many(pg_ctx *ctx, const pg_huffman_kv_chunk *const *
 }
 
 static pg_status decompress_dev(pg_ctx *ctx, const pg_huffman_kv_chunk *c, float *out, size_t out_stride) {
-    return decompress_many(ctx, &c, &out, &out_stride, 1);
+    c->block->touch(ctx);
+    if (!c->indexed) return decompress_many(ctx, &c, &out, &out_stride, 1);
+    kv_decode_args a = {};
+    a.single = c->dev;
+    a.out[0] = out;
+    a.out_stride = out_stride;
+    a.sides = a.count = 1;
+    a.heads = (unsigned)c->num_heads; a.head_elems = (unsigned)(c->num_tokens * c->head_dim); a.total = (unsigned)c->symbols();
+    return launch_decode(ctx, a);
 }
 
 PG_API pg_status pg_huffman_kv_compress_chunk_dev(pg_ctx *ctx, const float *data_dev, size_t head_stride, size_t num_tokens,
@@ -367,7 +913,12 @@ PG_API pg_status pg_huffman_kv_compress_chunk(pg_ctx *ctx, const float *data, si
     pg_tmp d;
     PG_TRY(d.alloc(total * sizeof(float)));
     if (total) PG_HIP(hipMemcpyAsync(d.p, data, total * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    return compress_dev(ctx, d.as<float>(), num_tokens * head_dim, num_tokens, num_heads, head_dim, out);
+    PG_TRY(compress_dev(ctx, d.as<float>(), num_tokens * head_dim, num_tokens, num_heads, head_dim, out));
+    const hipError_t e = hipStreamSynchronize(ctx->stream);  // d is freed on return
+    if (e == hipSuccess) return PG_OK;
+    delete *out;
+    *out = nullptr;
+    return pg_fail(PG_EDEVICE, "huffman kv compress_chunk: %s", hipGetErrorString(e));
 }
 
 PG_API pg_status pg_huffman_kv_chunk_from_parts(pg_ctx *ctx, const uint8_t *bitstream, size_t bytes, const float *scales,
@@ -378,18 +929,15 @@ PG_API pg_status pg_huffman_kv_chunk_from_parts(pg_ctx *ctx, const uint8_t *bits
     *out = nullptr;
     PG_TRY(chunk_shape_ok("pg_huffman_kv_chunk_from_parts", num_tokens, num_heads, head_dim));
     PG_CHECK_ARG(codebook && (scales || num_heads == 0) && (bitstream || bytes == 0), "pg_huffman_kv_chunk_from_parts: null pointer");
-    pg_huffman_kv_chunk *c = new (std::nothrow) pg_huffman_kv_chunk();
+    std::unique_ptr<pg_huffman_kv_chunk> c(new (std::nothrow) pg_huffman_kv_chunk());
     if (!c) return pg_fail(PG_ENOMEM, "host allocation failed");
-    struct guard { pg_huffman_kv_chunk *c; ~guard() { delete c; } } g{c};
     c->num_tokens = num_tokens; c->num_heads = num_heads; c->head_dim = head_dim;
     std::copy(codebook, codebook + NUM_SYMBOLS, c->codebook);
     c->scales.assign(scales, scales + num_heads);
-    PG_TRY(chunk_alloc(ctx, c, bytes));
-    if (num_heads) PG_HIP(hipMemcpyAsync(c->dev, scales, num_heads * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    if (bytes) PG_HIP(hipMemcpyAsync(c->dev + c->head_bytes(), bitstream, bytes, hipMemcpyHostToDevice, ctx->stream));
+    PG_TRY(chunk_alloc(ctx, c.get(), bytes));
+    if (bytes) PG_HIP(hipMemcpyAsync(c->dev + c->layout().o_bits, bitstream, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_HIP(hipStreamSynchronize(ctx->stream));
-    g.c = nullptr;
-    *out = c;
+    *out = c.release();
     return PG_OK;
 }
 
@@ -397,7 +945,8 @@ PG_API void pg_huffman_kv_chunk_free(pg_ctx *ctx, pg_huffman_kv_chunk *c) {
     if (!c) return;
     if (ctx) {
         (void)pg_use(ctx);
-        (void)hipStreamSynchronize(ctx->stream);
+        if (c->block) c->block->touch(ctx);
+        if (!c->block || c->block->foreign) (void)hipStreamSynchronize(ctx->stream);
     }
     delete c;
 }
@@ -416,6 +965,14 @@ PG_API pg_status pg_huffman_kv_chunk_parts(pg_ctx *ctx, const pg_huffman_kv_chun
                                            uint8_t *codebook) {
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(c != nullptr, "pg_huffman_kv_chunk_parts: null chunk");
+    c->block->touch(ctx);
+    if ((codebook || scales) && !c->on_host) {
+        c->scales.resize(c->num_heads);
+        PG_HIP(hipMemcpyAsync(c->codebook, c->dev + c->layout().o_book, NUM_SYMBOLS, hipMemcpyDeviceToHost, ctx->stream));
+        PG_HIP(hipMemcpyAsync(c->scales.data(), c->dev, c->num_heads * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+        PG_HIP(hipStreamSynchronize(ctx->stream));
+        c->on_host = true;
+    }
     if (codebook) std::copy(c->codebook, c->codebook + NUM_SYMBOLS, codebook);
     if (scales) std::copy(c->scales.begin(), c->scales.end(), scales);
     if (bitstream && c->bytes) {
@@ -471,7 +1028,12 @@ PG_API pg_status pg_huffman_kv_cache_create(pg_ctx *ctx, size_t num_kv_heads, si
 
 PG_API void pg_huffman_kv_cache_free(pg_ctx *ctx, pg_huffman_kv_cache *c) {
     if (!c) return;
-    pg_kv_cache_free(ctx, c->hot);  // waits for the stream
+    if (ctx) {
+        (void)pg_use(ctx);
+        c->touch(ctx);
+        if (c->foreign()) (void)hipStreamSynchronize(ctx->stream);
+    }
+    pg_kv_cache_free(ctx, c->hot);
     for (auto *p : c->k_chunks) delete p;
     for (auto *p : c->v_chunks) delete p;
     delete c;
@@ -496,37 +1058,49 @@ PG_API pg_status pg_huffman_kv_cache_chunk(const pg_huffman_kv_cache *c, int val
     return PG_OK;
 }
 
+// Room for `chunks` addresses in the cache's table.
+static pg_status table_reserve(pg_ctx *ctx, pg_huffman_kv_cache *c, size_t chunks) {
+    if (chunks <= c->table_cap) return PG_OK;
+    const size_t cap = std::max<size_t>(std::max<size_t>(chunks, 2 * c->table_cap), 64);
+    pg_dev_block grown;
+    PG_TRY(grown.alloc(ctx, cap * sizeof(char *)));
+    if (c->table) {
+        PG_HIP(hipMemcpyAsync(grown.p, c->table, c->table_cap * sizeof(char *), hipMemcpyDeviceToDevice, ctx->stream));
+        c->old_tables.push_back(std::move(c->table_mem));
+    }
+    c->table_mem = std::move(grown);
+    c->table = static_cast<char **>(c->table_mem.p);
+    c->table_cap = cap;
+    return PG_OK;
+}
+
 // The reference compresses the oldest chunk_size tokens and shifts the rest to the front, once per
-// chunk; here the chunks are cut at a moving token offset and the window is shifted once.
+// chunk; here every chunk that an append cuts, of both sides, is one batch and the window is shifted once.
 static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c) {
     pg_kv_cache *hot = c->hot;
-    const size_t hd = hot->head_dim, stride = hot->capacity * hd, heads = hot->num_kv_heads;
+    if (hot->len < c->compress_threshold) return PG_OK;
+    const size_t hd = hot->head_dim, stride = hot->capacity * hd, heads = hot->num_kv_heads, tokens = c->chunk_size;
+    const size_t chunks = (hot->len - c->compress_threshold) / tokens + 1;  // compress_threshold >= chunk_size: every chunk is whole
+    PG_TRY(chunk_shape_ok("huffman kv append", tokens, heads, hd));
+    PG_TRY(table_reserve(ctx, c, c->k_chunks.size() * 2 + 2 * chunks));
+    const float *data[2] = {hot->k, hot->v};
+    std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
+    kv_shift shift{{hot->k, hot->v}, stride, chunks * tokens * hd, (hot->len - chunks * tokens) * hd};
+    const pg_status st = compress_batch(ctx, data, 2, 2 * chunks, tokens * hd, stride, tokens, heads, hd, c->table + c->k_chunks.size() * 2, &shift, made);
     size_t done = 0;
-    pg_status st = PG_OK;
-    while (hot->len - done >= c->compress_threshold) {
-        const size_t tokens = std::min(c->chunk_size, hot->len - done);
-        pg_huffman_kv_chunk *kc = nullptr, *vc = nullptr;
-        st = compress_dev(ctx, hot->k + done * hd, stride, tokens, heads, hd, &kc);
-        if (st == PG_OK) st = compress_dev(ctx, hot->v + done * hd, stride, tokens, heads, hd, &vc);
-        if (st != PG_OK) {
-            delete kc;
-            break;
-        }
-        c->k_chunks.push_back(kc);
-        c->v_chunks.push_back(vc);
-        c->compressed_len += tokens;
+    for (size_t i = 0; i + 1 < made.size(); i += 2) {
+        c->k_chunks.push_back(made[i].release());
+        c->v_chunks.push_back(made[i + 1].release());
         done += tokens;
     }
     if (done == 0) return st;
+    c->compressed_len += done;
     const size_t rest = hot->len - done;
-    // The rest moves to the front in slices no longer than the distance it moves, oldest first on
+    // Where the encoder has not done it: the rest moves to the front in slices no longer than the distance it moves, oldest first on
     // the one stream, so that no copy reads what it writes; nothing is allocated and nothing waited for.
-    const size_t pitch = stride * sizeof(float);
-    for (size_t at = 0; at < rest && hd * heads > 0; at += done) {
-        const size_t width = std::min(done, rest - at) * hd * sizeof(float);
-        PG_HIP(hipMemcpy2DAsync(hot->k + at * hd, pitch, hot->k + (done + at) * hd, pitch, width, heads, hipMemcpyDeviceToDevice, ctx->stream));
-        PG_HIP(hipMemcpy2DAsync(hot->v + at * hd, pitch, hot->v + (done + at) * hd, pitch, width, heads, hipMemcpyDeviceToDevice, ctx->stream));
-    }
+    for (size_t at = shift.done ? rest : 0; at < rest; at += done)
+        PG_TRY(pg_launch_kv_rows(ctx, hot->k + at * hd, hot->v + at * hd, stride, hot->k + (done + at) * hd, hot->v + (done + at) * hd, stride,
+                                 std::min(done, rest - at) * hd, heads));
     hot->len = rest;
     return st;
 }
@@ -535,6 +1109,7 @@ PG_API pg_status pg_huffman_kv_cache_append_dev(pg_ctx *ctx, pg_huffman_kv_cache
                                                 const float *new_v_dev, size_t seq_len) {
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(c != nullptr, "pg_huffman_kv_cache_append: null cache");
+    c->touch(ctx);
     PG_TRY(pg_kv_cache_append_dev(ctx, c->hot, new_k_dev, new_v_dev, seq_len));
     return compress_hot(ctx, c);
 }
@@ -543,6 +1118,7 @@ PG_API pg_status pg_huffman_kv_cache_append(pg_ctx *ctx, pg_huffman_kv_cache *c,
                                             size_t seq_len) {
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(c != nullptr, "pg_huffman_kv_cache_append: null cache");
+    c->touch(ctx);
     PG_TRY(pg_kv_cache_append(ctx, c->hot, new_k, new_v, seq_len));
     return compress_hot(ctx, c);
 }
@@ -554,27 +1130,32 @@ PG_API pg_status pg_huffman_kv_cache_get_kv_dev(pg_ctx *ctx, const pg_huffman_kv
     const size_t total_len = c->compressed_len + hot->len, hd = hot->head_dim, heads = hot->num_kv_heads;
     if (total_len * hd * heads == 0) return PG_OK;
     PG_CHECK_ARG(k_dev && v_dev, "pg_huffman_kv_cache_get_kv: null output");
-    size_t off = 0;
-    std::vector<const pg_huffman_kv_chunk *> chunks;
-    std::vector<float *> outs;
-    for (size_t i = 0; i < c->k_chunks.size(); ++i) {  // every chunk of both sides in one decoding pass
-        chunks.push_back(c->k_chunks[i]);
-        outs.push_back(k_dev + off * hd);
-        chunks.push_back(c->v_chunks[i]);
-        outs.push_back(v_dev + off * hd);
-        off += c->k_chunks[i]->num_tokens;
+    const_cast<pg_huffman_kv_cache *>(c)->touch(ctx);
+    kv_decode_args a = {};
+    a.out[0] = k_dev;
+    a.out[1] = v_dev;
+    a.out_stride = total_len * hd;
+    a.chunk_step = c->chunk_size * hd;
+    a.sides = 2;
+    a.heads = (unsigned)heads; a.head_elems = (unsigned)(c->chunk_size * hd); a.total = (unsigned)(heads * c->chunk_size * hd);
+    // every chunk of both sides in one launch, the window's rows with them (a launch takes up to 2^30 workgroups of 16384 values)
+    const size_t chunks = 2 * c->k_chunks.size(), most = std::max<size_t>(1, (1u << 30) / (a.total / DEC_PER_WG + 1)) * 2;
+    for (size_t first = 0; first < chunks; first += most) {
+        a.table = c->table + first;
+        a.count = (unsigned)std::min(most, chunks - first);
+        for (int s = 0; s < 2; ++s) a.out[s] = (s ? v_dev : k_dev) + first / 2 * a.chunk_step;
+        if (first + most >= chunks && hot->len > 0 && hot->len * hd < (1ull << 31)) {
+            a.hot[0] = hot->k;
+            a.hot[1] = hot->v;
+            a.hot_stride = hot->capacity * hd;
+            a.hot_at = c->compressed_len * hd - first / 2 * a.chunk_step;
+            a.hot_elems = (unsigned)(hot->len * hd);
+        }
+        PG_TRY(launch_decode(ctx, a));
     }
-    const std::vector<size_t> strides(chunks.size(), total_len * hd);
-    for (size_t first = 0; first < chunks.size(); first += 16384)  // (a launch takes up to 65535 chunks)
-        PG_TRY(decompress_many(ctx, chunks.data() + first, outs.data() + first, strides.data() + first,
-                               std::min<size_t>(16384, chunks.size() - first)));
-    if (hot->len > 0) {
-        const size_t width = hot->len * hd * sizeof(float);
-        PG_HIP(hipMemcpy2DAsync(k_dev + off * hd, total_len * hd * sizeof(float), hot->k, hot->capacity * hd * sizeof(float), width,
-                                heads, hipMemcpyDeviceToDevice, ctx->stream));
-        PG_HIP(hipMemcpy2DAsync(v_dev + off * hd, total_len * hd * sizeof(float), hot->v, hot->capacity * hd * sizeof(float), width,
-                                heads, hipMemcpyDeviceToDevice, ctx->stream));
-    }
+    if (hot->len > 0 && a.hot_elems == 0)
+        PG_TRY(pg_launch_kv_rows(ctx, k_dev + c->compressed_len * hd, v_dev + c->compressed_len * hd, total_len * hd, hot->k, hot->v,
+                                 hot->capacity * hd, hot->len * hd, heads));
     return PG_OK;
 }
 

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 #include <string.h>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <type_traits>
@@ -26,6 +28,40 @@ struct pg_prof_total {
     std::vector<std::pair<size_t, size_t>> grids;  // distinct launch sizes (work-items) and how many launches had each
 };
 
+// Device blocks that objects of a context gave back and later ones may take (hipMalloc and hipFree cost 6 and 10 us a
+// call and hipFree waits for the device).  A block from the pool is used on the context's stream alone, so whoever
+// takes it next is ordered behind whoever had it; an object that another context has touched gives its memory to
+// hipFree instead.  At most PG_POOL_BYTES lie here; the context's end, or memory running out, empties it.
+constexpr size_t PG_POOL_BYTES = 256u << 20;
+struct pg_dev_pool {
+    std::mutex mu;
+    bool open = true;
+    size_t bytes = 0;
+    std::vector<std::pair<size_t, void *>> blocks;
+    void drain(bool close);
+};
+// One block, and the pool it came from.  `foreign` = another context's stream may have used it.
+struct pg_dev_block {
+    void *p = nullptr;
+    size_t cap = 0;
+    std::shared_ptr<pg_dev_pool> pool;
+    bool foreign = false;
+    pg_status alloc(struct pg_ctx *ctx, size_t bytes);
+    void touch(const struct pg_ctx *ctx);  // the block is about to be used on ctx's stream
+    void release();                        // foreign: the caller has waited for the work that uses it
+    pg_dev_block() = default;
+    pg_dev_block(const pg_dev_block &) = delete;
+    pg_dev_block &operator=(const pg_dev_block &) = delete;
+    pg_dev_block(pg_dev_block &&o) noexcept { *this = std::move(o); }
+    pg_dev_block &operator=(pg_dev_block &&o) noexcept {
+        release();
+        p = o.p; cap = o.cap; pool = std::move(o.pool); foreign = o.foreign;
+        o.p = nullptr; o.cap = 0; o.foreign = false;
+        return *this;
+    }
+    ~pg_dev_block() { release(); }
+};
+
 // One device + one stream + one growable scratch arena.
 struct pg_ctx {
     int device;
@@ -33,6 +69,9 @@ struct pg_ctx {
     bool owns_stream;
     void *ws;        // scratch arena (quantised activations, partial results)
     size_t ws_bytes;
+    void *pin = nullptr;  // pinned host memory for words and arrays that pass between the host and a launch (pg_pinned)
+    size_t pin_bytes = 0;
+    std::shared_ptr<pg_dev_pool> pool = std::make_shared<pg_dev_pool>();
     int num_cu;
     bool profiling;                     // per-kernel HIP events (pg_profile_begin/end)
     std::vector<pg_prof_rec> prof;      // one record per launch while profiling
@@ -87,7 +126,12 @@ struct pg_gguf_tensor {
 struct pg_kv_cache {
     float *k, *v;
     size_t len, capacity, num_kv_heads, head_dim;
+    mutable pg_dev_block k_mem, v_mem;
+    void touch(const pg_ctx *ctx) const { k_mem.touch(ctx); v_mem.touch(ctx); }
 };
+// dst[h * dst_stride + i] = src[h * src_stride + i] for i < width of every head h, key and value side in one launch (no overlap).
+pg_status pg_launch_kv_rows(pg_ctx *ctx, float *dst_k, float *dst_v, size_t dst_stride, const float *src_k, const float *src_v,
+                            size_t src_stride, size_t width, size_t heads);
 constexpr size_t PG_MM_MIN_BLOCKS = 5;
 constexpr int PG_GEMM_MAX_GROUP = 4;  // weights one W8A8 launch can carry (fused q|k|v, gate|up)
 constexpr size_t PG_KPAD = 128;  // device K stride is a multiple of this
@@ -123,6 +167,9 @@ pg_status pg_fail(pg_status st, const char *fmt, ...) __attribute__((format(prin
 pg_status pg_use(pg_ctx *ctx);
 // Scratch arena of at least `bytes` (256-byte aligned); contents undefined.
 pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out);
+// Pinned host memory of at least `bytes` (the context's one block; contents undefined).  The caller has waited for
+// every launch or copy that used it before.
+pg_status pg_pinned(pg_ctx *ctx, size_t bytes, void **out);
 // Check the launch just made.
 pg_status pg_launch_check(const char *what);
 // Let `kernel` use `bytes` of dynamic LDS on this context's device (the attribute is set once

@@ -1511,6 +1511,8 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
                            float logit_cap, float *out, int accumulate, const pg_xdigits *xd = nullptr, int digit_kind = 0,
                            const size_t *global_positions = nullptr, size_t num_global = 0,
                            const attn_args *rope_fusion = nullptr, const pg_mmdigits *md = nullptr, bool *md_written = nullptr) {
+    kc->touch(ctx);
+    vc->touch(ctx);
     // With `md` (digit_kind names the tensor type) a merge of key runs writes the rows as the matrix-core
     // product's digit planes instead of f32 and sets *md_written; a kernel that needs no merge writes `out`.
     // With `xd` (one-token step, accumulate == 0, head_dim % 32 == 0) the rows also, or only,
@@ -1694,39 +1696,35 @@ pg_status check_attention_args(const char *fn, const pg_kv_cache *kc, const pg_k
     return PG_OK;
 }
 
+// Rows of both sides of a cache, copied in one launch (two strided copies of the runtime took two launches of 5 us and
+// twice the host time): grid (parts, heads, sides).
+template <class T>
+__global__ __launch_bounds__(256) void kv_rows_kernel(T *dst_k, T *dst_v, size_t dst_stride, const T *src_k, const T *src_v,
+                                                      size_t src_stride, size_t width) {
+    T *d = (blockIdx.z ? dst_v : dst_k) + (size_t)blockIdx.y * dst_stride;
+    const T *s = (blockIdx.z ? src_v : src_k) + (size_t)blockIdx.y * src_stride;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < width; i += (size_t)gridDim.x * 256) d[i] = s[i];
+}
+
 // Room for `needed` positions per head; grows like the reference (at least double, from 16).
 pg_status cache_reserve(pg_ctx *ctx, pg_kv_cache *c, size_t needed) {
     if (needed <= c->capacity) return PG_OK;
     const size_t grown = (c->capacity > 16 ? c->capacity : 16) * 2;
     const size_t new_cap = needed > grown ? needed : grown;
     const size_t hd = c->head_dim, total = c->num_kv_heads * new_cap * hd * sizeof(float);
-    float *nk = nullptr, *nv = nullptr;
-    PG_HIP(hipMalloc(reinterpret_cast<void **>(&nk), total));
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&nv), total);
-    if (e != hipSuccess) {
-        (void)hipFree(nk);
-        return pg_fail(PG_ENOMEM, "hipMalloc(%zu) failed: %s", total, hipGetErrorString(e));
-    }
-    e = hipMemsetAsync(nk, 0, total, ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(nv, 0, total, ctx->stream);
-    if (e == hipSuccess && c->len > 0) {
-        const size_t width = c->len * hd * sizeof(float);
-        e = hipMemcpy2DAsync(nk, new_cap * hd * sizeof(float), c->k, c->capacity * hd * sizeof(float), width,
-                             c->num_kv_heads, hipMemcpyDeviceToDevice, ctx->stream);
-        if (e == hipSuccess)
-            e = hipMemcpy2DAsync(nv, new_cap * hd * sizeof(float), c->v, c->capacity * hd * sizeof(float), width,
-                                 c->num_kv_heads, hipMemcpyDeviceToDevice, ctx->stream);
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // the old planes are freed next
-    if (e != hipSuccess) {
-        (void)hipFree(nk);
-        (void)hipFree(nv);
-        return pg_fail(PG_EDEVICE, "KV cache growth failed: %s", hipGetErrorString(e));
-    }
-    if (c->k) (void)hipFree(c->k);
-    if (c->v) (void)hipFree(c->v);
-    c->k = nk;
-    c->v = nv;
+    pg_dev_block nk, nv;
+    PG_TRY(nk.alloc(ctx, total));
+    PG_TRY(nv.alloc(ctx, total));
+    hipError_t e = hipMemsetAsync(nk.p, 0, total, ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(nv.p, 0, total, ctx->stream);
+    if (e != hipSuccess) return pg_fail(PG_EDEVICE, "KV cache growth failed: %s", hipGetErrorString(e));
+    PG_TRY(pg_launch_kv_rows(ctx, static_cast<float *>(nk.p), static_cast<float *>(nv.p), new_cap * hd, c->k, c->v, c->capacity * hd, c->len * hd,
+                             c->num_kv_heads));
+    if (c->k_mem.foreign || c->v_mem.foreign) PG_HIP(hipStreamSynchronize(ctx->stream));  // the old planes go to hipFree next, not to the pool
+    c->k_mem = std::move(nk);
+    c->v_mem = std::move(nv);
+    c->k = static_cast<float *>(c->k_mem.p);
+    c->v = static_cast<float *>(c->v_mem.p);
     c->capacity = new_cap;
     return PG_OK;
 }
@@ -1747,6 +1745,16 @@ pg_status launch_rope(pg_ctx *ctx, const rope_args &ra, size_t seq, size_t heads
 }
 
 }  // namespace
+
+pg_status pg_launch_kv_rows(pg_ctx *ctx, float *dst_k, float *dst_v, size_t dst_stride, const float *src_k, const float *src_v,
+                            size_t src_stride, size_t width, size_t heads) {
+    if (width == 0 || heads == 0) return PG_OK;
+    auto grid = [&](size_t items) { return dim3((unsigned)std::min<size_t>((items + 1023) / 1024, 1024), (unsigned)heads, 2); };
+    if (((uintptr_t)dst_k | (uintptr_t)dst_v | (uintptr_t)src_k | (uintptr_t)src_v) % 16 == 0 && dst_stride % 4 == 0 && src_stride % 4 == 0 && width % 4 == 0)
+        return pg_launch(ctx, "kv_rows", kv_rows_kernel<float4>, grid(width / 4), dim3(256), 0, (float4 *)dst_k, (float4 *)dst_v, dst_stride / 4,
+                         (const float4 *)src_k, (const float4 *)src_v, src_stride / 4, width / 4);
+    return pg_launch(ctx, "kv_rows", kv_rows_kernel<float>, grid(width), dim3(256), 0, dst_k, dst_v, dst_stride, src_k, src_v, src_stride, width);
+}
 
 // ---- RMSNorm ----------------------------------------------------------------------------------
 
@@ -1857,7 +1865,7 @@ PG_API pg_status pg_kv_cache_create(pg_ctx *ctx, size_t num_kv_heads, size_t hea
     *out = nullptr;
     PG_CHECK_ARG(num_kv_heads > 0 && head_dim > 0 && head_dim <= 256 && num_kv_heads < 65536,
                  "pg_kv_cache_create: num_kv_heads %zu / head_dim %zu out of range (head_dim <= 256)", num_kv_heads, head_dim);
-    pg_kv_cache *c = new (std::nothrow) pg_kv_cache{nullptr, nullptr, 0, 0, num_kv_heads, head_dim};
+    pg_kv_cache *c = new (std::nothrow) pg_kv_cache{nullptr, nullptr, 0, 0, num_kv_heads, head_dim, {}, {}};
     if (!c) return pg_fail(PG_ENOMEM, "pg_kv_cache_create: out of host memory");
     *out = c;
     return PG_OK;
@@ -1867,10 +1875,9 @@ PG_API void pg_kv_cache_free(pg_ctx *ctx, pg_kv_cache *c) {
     if (!c) return;
     if (ctx) {
         (void)pg_use(ctx);
-        (void)hipStreamSynchronize(ctx->stream);
+        c->touch(ctx);
+        if (c->k_mem.foreign || c->v_mem.foreign) (void)hipStreamSynchronize(ctx->stream);
     }
-    if (c->k) (void)hipFree(c->k);
-    if (c->v) (void)hipFree(c->v);
     delete c;
 }
 
@@ -1891,12 +1898,11 @@ PG_API pg_status pg_kv_cache_append_dev(pg_ctx *ctx, pg_kv_cache *c, const float
     if (seq_len == 0) return PG_OK;
     PG_CHECK_ARG(new_k_dev && new_v_dev, "pg_kv_cache_append: null pointer");
     PG_CHECK_ARG(c->len + seq_len < (1ull << 31), "pg_kv_cache_append: length beyond 2^31");
+    c->touch(ctx);
     PG_TRY(cache_reserve(ctx, c, c->len + seq_len));
-    const size_t hd = c->head_dim, width = seq_len * hd * sizeof(float);
-    PG_HIP(hipMemcpy2DAsync(c->k + c->len * hd, c->capacity * hd * sizeof(float), new_k_dev, width, width,
-                            c->num_kv_heads, hipMemcpyDeviceToDevice, ctx->stream));
-    PG_HIP(hipMemcpy2DAsync(c->v + c->len * hd, c->capacity * hd * sizeof(float), new_v_dev, width, width,
-                            c->num_kv_heads, hipMemcpyDeviceToDevice, ctx->stream));
+    const size_t hd = c->head_dim;
+    PG_TRY(pg_launch_kv_rows(ctx, c->k + c->len * hd, c->v + c->len * hd, c->capacity * hd, new_k_dev, new_v_dev, seq_len * hd, seq_len * hd,
+                             c->num_kv_heads));
     c->len += seq_len;
     return PG_OK;
 }
@@ -1921,6 +1927,7 @@ PG_API pg_status pg_kv_cache_download(pg_ctx *ctx, const pg_kv_cache *c, float *
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(c != nullptr, "pg_kv_cache_download: null cache");
     if (c->len == 0) return PG_OK;
+    c->touch(ctx);
     PG_CHECK_ARG(k && v, "pg_kv_cache_download: null pointer");
     const size_t hd = c->head_dim, width = c->len * hd * sizeof(float);
     PG_HIP(hipMemcpy2DAsync(k, width, c->k, c->capacity * hd * sizeof(float), width, c->num_kv_heads,
@@ -2371,6 +2378,7 @@ PG_API pg_status pg_llama_block_forward_dev(pg_ctx *ctx, pg_llama_block *b, cons
                  "pg_llama_block_forward: cache is %zu heads x %zu, block is %zu x %zu", cache->num_kv_heads,
                  cache->head_dim, b->nkvh, b->hd);
     if (seq == 0) return PG_OK;
+    cache->touch(ctx);
     PG_CHECK_ARG(h_dev && out_dev, "pg_llama_block_forward: null pointer");
     PG_CHECK_ARG(seq < (1ull << 24), "pg_llama_block_forward: seq %zu too large", seq);
     const size_t offset = cache->len;

@@ -207,3 +207,35 @@ def test_cache_on_device_pointers(ctx, orc):
     want_k, want_v = o.get_kv()
     assert (out_k.to_host(np.float32).view(np.uint32) == want_k.view(np.uint32)).all()
     assert (out_v.to_host(np.float32).view(np.uint32) == want_v.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("heads,hd,chunk,chunks", [
+    (1, 1, 4095, 2), (1, 1, 4096, 2), (1, 1, 4097, 2),     # a histogram run of 4096 values, one less, one more
+    (1, 4, 4096, 1), (1, 4, 4097, 1), (3, 1, 5462, 1),     # a decoder workgroup of 16384, and 2 (with a head cut by the runs) past it
+    (1, 64, 1, 45), (5, 3, 2, 40),                         # more chunks in one batch than one encoder launch places
+    (2, 2, 70000, 1),                                      # 69 runs of a head's values, several rounds of the maximum
+])
+@pytest.mark.parametrize("kind", ["normal", "steep", "two"])
+def test_batches_and_run_edges(ctx, orc, heads, hd, chunk, chunks, kind):
+    """One append that cuts `chunks` whole chunks at the edges of the batch's runs, workgroups and launches; `steep` has
+    frequencies that halve from value to value (codes past the limit of 12 bits, repaired), `two` has two values."""
+    from peregrine_amd import huffman
+    say(f"huffman kv batch heads={heads} head_dim={hd} chunk={chunk} x {chunks} {kind}")
+    rng = np.random.default_rng(chunk + heads)
+    n = chunk * chunks
+    if kind == "normal":
+        k, v = (rng.standard_normal((heads, n, hd)).astype(np.float32) for _ in range(2))
+    elif kind == "steep":
+        k, v = (np.minimum(rng.geometric(0.5, (heads, n, hd)), 40).astype(np.float32) for _ in range(2))
+        k[:, 0], v[:, 0] = 40.0, 40.0
+    else:
+        k, v = (rng.integers(0, 2, (heads, n, hd)).astype(np.float32) for _ in range(2))
+    c, o = huffman.HuffmanKVCache(heads, hd, chunk, chunk, ctx), orc.HuffmanKVCache(heads, hd, chunk, chunk)
+    c.append(k, v, n)
+    o.append(k, v, n)
+    assert (c.len(), c.compressed_len, len(c.k_chunks)) == (o.len, o.compressed_len, chunks)
+    for got, want in zip(c.get_kv(), o.get_kv()):
+        assert (got.view(np.uint32) == want.view(np.uint32)).all()
+    for side, made in ((0, c.k_chunks), (1, c.v_chunks)):
+        for i in {0, chunks // 2, chunks - 1}:
+            _same_chunk(made[i], o.chunk(side, i)[:3])
