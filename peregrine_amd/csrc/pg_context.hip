@@ -197,6 +197,7 @@ PG_API void pg_ctx_destroy(pg_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
     ctx->pool->drain(true);
     for (auto &t : ctx->moe_tabs)
         if (t.dev) (void)hipFree(t.dev);

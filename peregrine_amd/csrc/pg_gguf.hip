@@ -1324,12 +1324,9 @@ PG_API pg_status pg_gguf_matmul(pg_ctx *ctx, const float *x, size_t m, const pg_
     PG_CHECK_ARG(w != nullptr, "pg_gguf_matmul: null weights");
     if (m == 0) return PG_OK;
     PG_CHECK_ARG(x && y, "pg_gguf_matmul: null pointer");
-    pg_tmp dx, dy;
-    PG_TRY(dx.alloc(m * w->k_in * sizeof(float)));
-    PG_TRY(dy.alloc(m * w->n_out * sizeof(float)));
-    PG_HIP(hipMemcpyAsync(dx.p, x, m * w->k_in * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    pg_dev_block dx, dy;
+    PG_TRY(dy.alloc(ctx, m * w->n_out * sizeof(float)));
+    PG_TRY(pg_host_in(ctx, x, m * w->k_in * sizeof(float), dx));
     PG_TRY(pg_gguf_matmul_dev(ctx, dx.as<float>(), m, w, dy.as<float>()));
-    PG_HIP(hipMemcpyAsync(y, dy.p, m * w->n_out * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    return pg_host_out(ctx, y, dy.p, m * w->n_out * sizeof(float));
 }

@@ -7,6 +7,7 @@
 #include <string.h>
 #include <memory>
 #include <mutex>
+#include <algorithm>
 #include <string>
 #include <tuple>
 #include <type_traits>
@@ -47,6 +48,7 @@ struct pg_dev_block {
     std::shared_ptr<pg_dev_pool> pool;
     bool foreign = false;
     pg_status alloc(struct pg_ctx *ctx, size_t bytes);
+    template <class T> T *as() const { return static_cast<T *>(p); }
     void touch(const struct pg_ctx *ctx);  // the block is about to be used on ctx's stream
     void release();                        // foreign: the caller has waited for the work that uses it
     pg_dev_block() = default;
@@ -72,6 +74,9 @@ struct pg_ctx {
     void *pin = nullptr;  // pinned host memory for words and arrays that pass between the host and a launch (pg_pinned)
     size_t pin_bytes = 0;
     std::shared_ptr<pg_dev_pool> pool = std::make_shared<pg_dev_pool>();
+    void *stage = nullptr;  // pinned staging of the host-pointer entry points (pg_hostio.hip)
+    size_t stage_bytes = 0, stage_used = 0;
+    unsigned stage_epoch = 0;
     int num_cu;
     bool profiling;                     // per-kernel HIP events (pg_profile_begin/end)
     std::vector<pg_prof_rec> prof;      // one record per launch while profiling
@@ -170,6 +175,12 @@ pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out);
 // Pinned host memory of at least `bytes` (the context's one block; contents undefined).  The caller has waited for
 // every launch or copy that used it before.
 pg_status pg_pinned(pg_ctx *ctx, size_t bytes, void **out);
+// Arrays of the host-pointer entry points (pg_hostio.hip).  pg_host_in: a device copy of a caller's array, stream
+// ordered; the caller's memory is free again on return.  pg_host_pinned: a pinned copy, which a launch that reads it
+// once may read in place.  pg_host_out: device memory to a caller's array (a multiple of 4 bytes), there on return.
+pg_status pg_host_in(pg_ctx *ctx, const void *host, size_t bytes, pg_dev_block &dev);
+pg_status pg_host_pinned(pg_ctx *ctx, const void *host, size_t bytes, void **pinned);
+pg_status pg_host_out(pg_ctx *ctx, void *host, const void *dev, size_t bytes);
 // Check the launch just made.
 pg_status pg_launch_check(const char *what);
 // Let `kernel` use `bytes` of dynamic LDS on this context's device (the attribute is set once

@@ -2442,12 +2442,9 @@ PG_API pg_status pg_llama_block_forward(pg_ctx *ctx, pg_llama_block *b, const fl
     if (seq == 0) return PG_OK;
     PG_CHECK_ARG(h && out, "pg_llama_block_forward: null pointer");
     const size_t bytes = seq * b->d * sizeof(float);
-    pg_tmp dh, dout;
-    PG_TRY(dh.alloc(bytes));
-    PG_TRY(dout.alloc(bytes));
-    PG_HIP(hipMemcpyAsync(dh.p, h, bytes, hipMemcpyHostToDevice, ctx->stream));
+    pg_dev_block dh, dout;
+    PG_TRY(dout.alloc(ctx, bytes));
+    PG_TRY(pg_host_in(ctx, h, bytes, dh));
     PG_TRY(pg_llama_block_forward_dev(ctx, b, dh.as<float>(), seq, cache, dout.as<float>()));
-    PG_HIP(hipMemcpyAsync(out, dout.p, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    return pg_host_out(ctx, out, dout.p, bytes);
 }

@@ -329,21 +329,15 @@ PG_API pg_status pg_moe_ffn_routed(pg_ctx *ctx, const float *x, size_t T, const 
                 PG_CHECK_ARG(expert_idx[t * top_k + j] != e, "pg_moe_ffn_routed: token %zu names expert %d twice", t, (int)e);
         }
     const size_t d = gate[0]->k_in, P = T * top_k;
-    pg_tmp dx, di, dw, dsh, dout;
-    PG_TRY(dx.alloc(T * d * sizeof(float)));
-    PG_TRY(di.alloc(P * sizeof(int32_t)));
-    PG_TRY(dw.alloc(P * sizeof(float)));
-    PG_TRY(dout.alloc(T * d * sizeof(float)));
-    if (shared) PG_TRY(dsh.alloc(T * d * sizeof(float)));
-    PG_HIP(hipMemcpyAsync(dx.p, x, T * d * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    PG_HIP(hipMemcpyAsync(di.p, expert_idx, P * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    PG_HIP(hipMemcpyAsync(dw.p, weight, P * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    if (shared) PG_HIP(hipMemcpyAsync(dsh.p, shared, T * d * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    pg_dev_block dx, di, dw, dsh, dout;
+    PG_TRY(dout.alloc(ctx, T * d * sizeof(float)));
+    PG_TRY(pg_host_in(ctx, x, T * d * sizeof(float), dx));
+    PG_TRY(pg_host_in(ctx, expert_idx, P * sizeof(int32_t), di));
+    PG_TRY(pg_host_in(ctx, weight, P * sizeof(float), dw));
+    if (shared) PG_TRY(pg_host_in(ctx, shared, T * d * sizeof(float), dsh));
     PG_TRY(pg_moe_ffn_routed_dev(ctx, dx.as<float>(), T, di.as<int32_t>(), dw.as<float>(), E, top_k, gate, up, down, act,
                                  shared ? dsh.as<float>() : nullptr, dout.as<float>()));
-    PG_HIP(hipMemcpyAsync(out, dout.p, T * d * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    return pg_host_out(ctx, out, dout.p, T * d * sizeof(float));
 }
 
 PG_API pg_status pg_moe_ffn(pg_ctx *ctx, const float *x, size_t T, const float *router_logits,
@@ -355,14 +349,10 @@ PG_API pg_status pg_moe_ffn(pg_ctx *ctx, const float *x, size_t T, const float *
     if (T == 0) return PG_OK;
     PG_CHECK_ARG(x && router_logits && out, "pg_moe_ffn: null pointer");
     const size_t d = gate[0]->k_in;
-    pg_tmp dx, dl, dout;
-    PG_TRY(dx.alloc(T * d * sizeof(float)));
-    PG_TRY(dl.alloc(T * E * sizeof(float)));
-    PG_TRY(dout.alloc(T * d * sizeof(float)));
-    PG_HIP(hipMemcpyAsync(dx.p, x, T * d * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    PG_HIP(hipMemcpyAsync(dl.p, router_logits, T * E * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    pg_dev_block dx, dl, dout;
+    PG_TRY(dout.alloc(ctx, T * d * sizeof(float)));
+    PG_TRY(pg_host_in(ctx, x, T * d * sizeof(float), dx));
+    PG_TRY(pg_host_in(ctx, router_logits, T * E * sizeof(float), dl));
     PG_TRY(pg_moe_ffn_dev(ctx, dx.as<float>(), T, dl.as<float>(), E, top_k, gate, up, down, act, dout.as<float>()));
-    PG_HIP(hipMemcpyAsync(out, dout.p, T * d * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    return pg_host_out(ctx, out, dout.p, T * d * sizeof(float));
 }

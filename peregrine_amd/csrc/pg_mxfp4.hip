@@ -905,15 +905,12 @@ PG_API pg_status pg_mxfp4_expert_forward(pg_ctx *ctx, const pg_mxfp4_expert *e, 
     PG_CHECK_ARG(e != nullptr, "pg_mxfp4_expert_forward: null expert");
     if (m == 0) return PG_OK;
     PG_CHECK_ARG(x && out, "pg_mxfp4_expert_forward: null pointer");
-    pg_tmp dx, ds, dout;
-    PG_TRY(dx.alloc(m * e->hidden * sizeof(float)));
-    PG_TRY(ds.alloc(m * 3 * e->intermediate * sizeof(float)));
-    PG_TRY(dout.alloc(m * e->hidden * sizeof(float)));
-    PG_HIP(hipMemcpyAsync(dx.p, x, m * e->hidden * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    pg_dev_block dx, ds, dout;
+    PG_TRY(ds.alloc(ctx, m * 3 * e->intermediate * sizeof(float)));
+    PG_TRY(dout.alloc(ctx, m * e->hidden * sizeof(float)));
+    PG_TRY(pg_host_in(ctx, x, m * e->hidden * sizeof(float), dx));
     PG_TRY(pg_mxfp4_expert_forward_dev(ctx, e, dx.as<float>(), m, ds.as<float>(), dout.as<float>()));
-    PG_HIP(hipMemcpyAsync(out, dout.p, m * e->hidden * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    return pg_host_out(ctx, out, dout.p, m * e->hidden * sizeof(float));
 }
 
 
@@ -1086,16 +1083,11 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed(pg_ctx *ctx, const float *x, size_t T, 
                 PG_CHECK_ARG(expert_idx[t * top_k + j] != e, "pg_mxfp4_moe_ffn: token %zu names expert %d twice", t, (int)e);
         }
     const size_t hidden = experts[0]->hidden;
-    pg_tmp dx, di, dw, dout;
-    PG_TRY(dx.alloc(T * hidden * sizeof(float)));
-    PG_TRY(di.alloc(T * top_k * sizeof(int32_t)));
-    PG_TRY(dw.alloc(T * top_k * sizeof(float)));
-    PG_TRY(dout.alloc(T * hidden * sizeof(float)));
-    PG_HIP(hipMemcpyAsync(dx.p, x, T * hidden * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    PG_HIP(hipMemcpyAsync(di.p, expert_idx, T * top_k * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    PG_HIP(hipMemcpyAsync(dw.p, weight, T * top_k * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    pg_dev_block dx, di, dw, dout;
+    PG_TRY(dout.alloc(ctx, T * hidden * sizeof(float)));
+    PG_TRY(pg_host_in(ctx, x, T * hidden * sizeof(float), dx));
+    PG_TRY(pg_host_in(ctx, expert_idx, T * top_k * sizeof(int32_t), di));
+    PG_TRY(pg_host_in(ctx, weight, T * top_k * sizeof(float), dw));
     PG_TRY(pg_mxfp4_moe_ffn_routed_dev(ctx, dx.as<float>(), T, di.as<int32_t>(), dw.as<float>(), top_k, experts, E, dout.as<float>()));
-    PG_HIP(hipMemcpyAsync(out, dout.p, T * hidden * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    return pg_host_out(ctx, out, dout.p, T * hidden * sizeof(float));
 }

@@ -739,14 +739,11 @@ PG_API pg_status pg_matmul_dequant_i8(pg_ctx *ctx, const float *a, size_t m, siz
     PG_CHECK_ARG(w->rows == k, "pg_matmul_dequant_i8: a has k = %zu but w has %zu rows", k, w->rows);
     if (m == 0) return PG_OK;
     PG_CHECK_ARG(a && out, "pg_matmul_dequant_i8: null pointer");
-    pg_tmp da, dout;
-    PG_TRY(da.alloc(m * k * sizeof(float)));
-    PG_TRY(dout.alloc(m * w->cols * sizeof(float)));
-    PG_HIP(hipMemcpyAsync(da.p, a, m * k * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    pg_dev_block da, dout;
+    PG_TRY(pg_host_in(ctx, a, m * k * sizeof(float), da));
+    PG_TRY(dout.alloc(ctx, m * w->cols * sizeof(float)));
     PG_TRY(pg_matmul_dequant_i8_dev(ctx, da.as<float>(), m, k, w, dout.as<float>()));
-    PG_HIP(hipMemcpyAsync(out, dout.p, m * w->cols * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    return pg_host_out(ctx, out, dout.p, m * w->cols * sizeof(float));
 }
 
 PG_API pg_status pg_matmul_quantized(pg_ctx *ctx, const float *a, size_t m, size_t k,
@@ -756,12 +753,18 @@ PG_API pg_status pg_matmul_quantized(pg_ctx *ctx, const float *a, size_t m, size
     PG_CHECK_ARG(w->rows == k, "pg_matmul_quantized: a has k = %zu but w has %zu rows", k, w->rows);
     if (m == 0) return PG_OK;
     PG_CHECK_ARG(a && out, "pg_matmul_quantized: null pointer");
-    pg_tmp da, dout;
-    PG_TRY(da.alloc(m * k * sizeof(float)));
-    PG_TRY(dout.alloc(m * w->cols * sizeof(float)));
-    PG_HIP(hipMemcpyAsync(da.p, a, m * k * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-    PG_TRY(pg_matmul_quantized_dev(ctx, da.as<float>(), m, k, w, dout.as<float>(), nullptr));
-    PG_HIP(hipMemcpyAsync(out, dout.p, m * w->cols * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    PG_HIP(hipStreamSynchronize(ctx->stream));
-    return PG_OK;
+    pg_dev_block da, dout;
+    const size_t a_bytes = m * k * sizeof(float);
+    const float *a_dev = nullptr;
+    if (m > 1 && a_bytes <= (1u << 20)) {  // one piece, read once by the quantisation: in place over PCIe, a launch less
+        void *pin = nullptr;
+        PG_TRY(pg_host_pinned(ctx, a, a_bytes, &pin));
+        a_dev = static_cast<const float *>(pin);
+    } else {
+        PG_TRY(pg_host_in(ctx, a, a_bytes, da));
+        a_dev = da.as<float>();
+    }
+    PG_TRY(dout.alloc(ctx, m * w->cols * sizeof(float)));
+    PG_TRY(pg_matmul_quantized_dev(ctx, a_dev, m, k, w, dout.as<float>(), nullptr));
+    return pg_host_out(ctx, out, dout.p, m * w->cols * sizeof(float));
 }

@@ -531,3 +531,25 @@ def test_matmul_dequant_i8_reference_tolerance_and_closed_form(ctx, orc):
     assert np.isnan(got[5]).all() and np.isfinite(np.delete(got, 5, axis=0)).all()
     with pytest.raises(ValueError):
         quant.matmul_dequant_i8(ai, m, k + 1, qt2, ctx)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (1, 32, 1), (3, 7, 5), (64, 64, 64), (63, 33, 65), (17, 96, 241),   # one word out; 16 KB, 4 bytes less, 4 bytes more
+    (512, 512, 40), (511, 513, 40), (1025, 257, 40),                    # 1 MB in, just below, just above (two pieces)
+    (1024, 64, 1024), (1025, 64, 1023), (1537, 64, 2049), (2050, 1100, 1030),  # one window of 4 MB out, 4 bytes less, several; 9 MB in
+])
+def test_host_arrays_cross_whole(ctx, m, k, n):
+    """The host-array call against the device-pointer call, bit for bit, at the edges of the transfers' pieces; twice,
+    so that the second finds the first one's words in the staging memory."""
+    from peregrine_amd import quant, _ffi
+    say(f"host arrays m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + n)
+    qt = quant.quantize_weights(rng.standard_normal(k * n).astype(np.float32), k, n, ctx).to_gpu(ctx)
+    for _ in range(2):
+        a = rng.standard_normal(m * k).astype(np.float32)
+        da, do = DevBuf(ctx, host=a), DevBuf(ctx, nbytes=4 * m * n)
+        _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, da.ptr, m, k, qt._gpu, do.ptr, None))
+        ctx.sync()
+        want = do.to_host(np.float32)
+        got = quant.matmul_quantized(a, m, k, qt, ctx)
+        assert (got.view(np.uint32) == want.view(np.uint32)).all()
