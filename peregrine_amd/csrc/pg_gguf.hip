@@ -1066,7 +1066,7 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
         PG_TRY(pg_workspace(ctx, pg_mmdigits_bytes(m, w->k_in), &ws));   // (the product is done with the arena)
         const pg_mmdigits md = pg_mmdigits_carve(ws, m, w->k_in);
         PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, m, w->k_in, w->ggml_type, md));
-        return pg_launch_q41_offset(ctx, w, md, m, y_dev);
+        return pg_launch_q41_offset(ctx, w, md, m, nullptr, 1, y_dev);
     }
     const int ks = pg_gguf_mm_splitk(ctx, w->n_out, w->k_in, (m + 31) / 32, m, false, nullptr);
     const size_t sz_d = pg_mmdigits_bytes(m, w->k_in);
@@ -1079,8 +1079,8 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
     PG_TRY(pg_gguf_ensure_tiled(ctx, w));
     grp.tiled = 1;
     // Q4_1: the Q4_0 product on the same nibbles and scales, then the blocks' offsets times the rows' block sums
-    PG_TRY(pg_launch_gguf_mm(ctx, q41 ? PG_GGML_Q4_0 : w->ggml_type, w->n_out, w->k_in, w->qs_tiled, w->d, grp, m, md, y_dev, part));
-    return q41 ? pg_launch_q41_offset(ctx, w, md, m, y_dev) : PG_OK;
+    PG_TRY(pg_launch_gguf_mm(ctx, q41 ? PG_GGML_Q4_0 : w->ggml_type, w->n_out, w->k_in, w->qs_tiled, w->d, grp, m, md, y_dev, part, q41));
+    return q41 ? pg_launch_q41_offset(ctx, w, md, m, part, ks, y_dev) : PG_OK;
 }
 
 // Several products over the same activation rows (q/k/v, gate/up): the rows are rewritten

@@ -71,19 +71,27 @@ __global__ __launch_bounds__(256) void x_to_mm_digits_kernel(const float *__rest
     pg_emit_mm_digits<NIB>(f, row, b, sub, nb, nbp, digits, xs, xsum);
 }
 
-// Q4_1's second term on many rows: y[t][n] += sum_b (8 d[n][b] + m[n][b]) * xsum[t][b] (the first, d sum (q - 8) x,
-// is the Q4_0 product on the same nibbles).  Workgroup = 256 / NQ weight rows x 16 tokens; thread = (row, one of NQ
-// runs of blocks), 16 tokens in registers; the tokens' block sums wait in LDS as [b][16]; the runs are added in
-// ascending order.  NQ = 4 for few tokens (more workgroups, shorter loops), 1 for many (the block sums staged once
-// per 256 rows).
-constexpr int Q41_TT = 16;
-template <int NQ>
+// Q4_1's second term on many rows: y[t][n] = first term + sum_b (8 d[n][b] + m[n][b]) * xsum[t][b]; the first,
+// d sum (q - 8) x, is the Q4_0 product on the same nibbles, in y or (ks > 1) in the planes of its K chunks at part.
+//
+// Up to 64 tokens: workgroup = 16 weight rows x 16 tokens, thread = (row, one of 16 runs of blocks), 16 tokens in
+// registers, eight blocks' scales requested at a time; the tokens' block sums wait in LDS as [b][16]; the runs are added
+// in ascending order, a thread an output.  It is latency: a workgroup per 16 rows gives every CU one from 4096 rows on
+// (64 rows a workgroup, one block's scales at a time and the planes added by a launch of their own took 17 us for
+// 40 x 4096 -> 4096, this 8.7).
+constexpr int Q41_TT = 16, Q41_NQ = 16;
+__device__ __forceinline__ float q41_first_term(const float *part, int ks, size_t stride, const float *y, size_t i) {
+    float v = ks > 1 ? part[i] : y[i];
+    for (int s = 1; s < ks; ++s) v += part[(size_t)s * stride + i];
+    return v;
+}
 __global__ __launch_bounds__(256) void q41_offset_kernel(const uint16_t *__restrict__ d, const uint16_t *__restrict__ m, int n_out,
                                                          int nb, const float *__restrict__ xsum, int nbp, int rows,
-                                                         float *__restrict__ y) {
-    constexpr int RPW = 256 / NQ;
-    extern __shared__ __attribute__((aligned(16))) float s_tile[];  // [nb][Q41_TT], then [NQ - 1][RPW][Q41_TT] partial sums
-    const int t0 = blockIdx.y * Q41_TT, lrow = threadIdx.x % RPW, quarter = threadIdx.x / RPW;
+                                                         const float *__restrict__ part_in, int ks, size_t stride, float *y) {
+    constexpr int RPW = 256 / Q41_NQ, AHEAD = 8;
+    static_assert(RPW * Q41_TT == 256, "a thread adds one output's runs");
+    extern __shared__ __attribute__((aligned(16))) float s_tile[];  // [nb][Q41_TT], then [Q41_NQ][RPW][Q41_TT + 1] partial sums
+    const int t0 = blockIdx.y * Q41_TT, lrow = threadIdx.x % RPW, run = threadIdx.x / RPW;
     const int n = blockIdx.x * RPW + lrow;
     for (int i = threadIdx.x; i < nb * Q41_TT; i += 256) {
         const int t = i / nb, b = i - t * nb;  // (consecutive threads: consecutive blocks of one token)
@@ -95,37 +103,130 @@ __global__ __launch_bounds__(256) void q41_offset_kernel(const uint16_t *__restr
     for (int t = 0; t < Q41_TT; ++t) acc[t] = 0.0f;
     const int nc = n < n_out ? n : n_out - 1;
     const size_t tile = (size_t)(nc >> 3) * nb * 8 + (nc & 7);
-    const int per = (nb + NQ - 1) / NQ, b_lo = quarter * per, b_hi = b_lo + per < nb ? b_lo + per : nb;
-    for (int b = b_lo; b < b_hi; ++b) {
-        _Float16 dh, mh;
-        const uint16_t db = d[tile + (size_t)b * 8], mb = m[tile + (size_t)b * 8];
-        __builtin_memcpy(&dh, &db, 2);
-        __builtin_memcpy(&mh, &mb, 2);
-        const float c = fmaf(8.0f, (float)dh, (float)mh);
+    const int per = (nb + Q41_NQ - 1) / Q41_NQ, b_lo = run * per, b_hi = b_lo + per < nb ? b_lo + per : nb;
+    for (int b0 = b_lo; b0 < b_hi; b0 += AHEAD) {
+        uint16_t db[AHEAD], mb[AHEAD];
 #pragma unroll
-        for (int t4 = 0; t4 < Q41_TT / 4; ++t4) {
-            const float4 sv = *reinterpret_cast<const float4 *>(s_tile + b * Q41_TT + 4 * t4);
-            acc[4 * t4] = fmaf(c, sv.x, acc[4 * t4]); acc[4 * t4 + 1] = fmaf(c, sv.y, acc[4 * t4 + 1]);
-            acc[4 * t4 + 2] = fmaf(c, sv.z, acc[4 * t4 + 2]); acc[4 * t4 + 3] = fmaf(c, sv.w, acc[4 * t4 + 3]);
+        for (int u = 0; u < AHEAD; ++u) {
+            const size_t at = tile + (size_t)(b0 + u < b_hi ? b0 + u : b_hi - 1) * 8;
+            db[u] = d[at];
+            mb[u] = m[at];
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            if (b0 + u >= b_hi) break;
+            _Float16 dh, mh;
+            __builtin_memcpy(&dh, &db[u], 2);
+            __builtin_memcpy(&mh, &mb[u], 2);
+            const float c = fmaf(8.0f, (float)dh, (float)mh);
+#pragma unroll
+            for (int t4 = 0; t4 < Q41_TT / 4; ++t4) {
+                const float4 sv = *reinterpret_cast<const float4 *>(s_tile + (b0 + u) * Q41_TT + 4 * t4);
+                acc[4 * t4] = fmaf(c, sv.x, acc[4 * t4]); acc[4 * t4 + 1] = fmaf(c, sv.y, acc[4 * t4 + 1]);
+                acc[4 * t4 + 2] = fmaf(c, sv.z, acc[4 * t4 + 2]); acc[4 * t4 + 3] = fmaf(c, sv.w, acc[4 * t4 + 3]);
+            }
         }
     }
-    if constexpr (NQ > 1) {
-        float *part = s_tile + nb * Q41_TT;
-        if (quarter > 0) {
+    float *part = s_tile + nb * Q41_TT;
 #pragma unroll
-            for (int t = 0; t < Q41_TT; ++t) part[((quarter - 1) * RPW + lrow) * Q41_TT + t] = acc[t];
+    for (int t = 0; t < Q41_TT; ++t) part[(run * RPW + lrow) * (Q41_TT + 1) + t] = acc[t];
+    __syncthreads();
+    const int t = run;  // (consecutive threads store consecutive rows)
+    float sum = 0.0f;
+#pragma unroll
+    for (int qv = 0; qv < Q41_NQ; ++qv) sum += part[(qv * RPW + lrow) * (Q41_TT + 1) + t];
+    if (n < n_out && t0 + t < rows) {
+        const size_t i = (size_t)(t0 + t) * n_out + n;
+        y[i] = q41_first_term(part_in, ks, stride, y, i) + sum;
+    }
+}
+
+// From 65 tokens on it is a product like any other, over K = the blocks: v_mfma_f32_32x32x2_f32 (the vector form was
+// bound by its own FMAs and LDS reads: 140 of 374 us at 1000 x 4096 -> 14336).  Workgroup = 4 wavefronts of 32 weight rows
+// x 64 tokens.  The order in which blocks meet the instruction's k-slots is free, so lane half h takes blocks
+// 8 i + 4 h .. + 3 for four instructions: one 128-bit load of a token's sums, and of a weight row's scales one 64-byte run
+// per 8 rows.  Result lane = weight row: the read-modify-write of y goes in 128-byte runs.
+typedef float v16f __attribute__((ext_vector_type(16)));
+__global__ __launch_bounds__(256) void q41_offset_mfma_kernel(const uint16_t *__restrict__ d, const uint16_t *__restrict__ m, int n_out,
+                                                              int nb, const float *__restrict__ xsum, int nbp, int rows,
+                                                              const float *__restrict__ part, int ks, size_t stride, float *y) {
+    const int lane = threadIdx.x & 63, l31 = lane & 31, h = lane >> 5;
+    const int n = blockIdx.x * 128 + (threadIdx.x >> 6) * 32 + l31, t0 = blockIdx.y * 64;
+    if (n - l31 >= n_out) return;
+    const int nc = n < n_out ? n : n_out - 1;
+    const size_t tile = (size_t)(nc >> 3) * nb * 8 + (nc & 7);
+    const float *xt[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) xt[j] = xsum + (size_t)(t0 + 32 * j + l31 < rows ? t0 + 32 * j + l31 : rows - 1) * nbp;
+    v16f acc[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+    uint16_t db[2][4], mb[2][4];
+    float4 xv[2][2];
+    auto load = [&](int buf, int i) {  // blocks past the end: the last one, its sum taken as zero
+        const int b = 8 * i + 4 * h;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const size_t at = tile + (size_t)(b + c < nb ? b + c : nb - 1) * 8;
+            db[buf][c] = d[at];
+            mb[buf][c] = m[at];
         }
-        __syncthreads();
-        if (quarter > 0) return;
 #pragma unroll
-        for (int qv = 0; qv < NQ - 1; ++qv)
+        for (int j = 0; j < 2; ++j) {
+            float4 v = *reinterpret_cast<const float4 *>(xt[j] + (b < nbp ? b : 0));
+            if (b + 3 >= nb) {
+                v.x = b < nb ? v.x : 0.0f;
+                v.y = b + 1 < nb ? v.y : 0.0f;
+                v.z = b + 2 < nb ? v.z : 0.0f;
+                v.w = 0.0f;
+            }
+            xv[buf][j] = v;
+        }
+    };
+    auto multiply = [&](int buf) {
 #pragma unroll
-            for (int t = 0; t < Q41_TT; ++t) acc[t] += part[(qv * RPW + lrow) * Q41_TT + t];
+        for (int c = 0; c < 4; ++c) {
+            _Float16 dh, mh;
+            __builtin_memcpy(&dh, &db[buf][c], 2);
+            __builtin_memcpy(&mh, &mb[buf][c], 2);
+            const float w = fmaf(8.0f, (float)dh, (float)mh);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float4 v = xv[buf][j];
+                const float a = c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w;
+                acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, w, acc[j], 0, 0, 0);  // rows = tokens, columns = weight rows
+            }
+        }
+    };
+    const int steps = (nb + 7) / 8;
+    load(0, 0);
+    for (int i = 0; i < steps; i += 2) {
+        if (i + 1 < steps) load(1, i + 1);
+        multiply(0);
+        if (i + 2 < steps) load(0, i + 2);
+        if (i + 1 < steps) multiply(1);
     }
     if (n >= n_out) return;
 #pragma unroll
-    for (int t = 0; t < Q41_TT; ++t)
-        if (t0 + t < rows) y[(size_t)(t0 + t) * n_out + n] += acc[t];
+    for (int j = 0; j < 2; ++j) {
+        float first[16];  // every plane's sixteen loads together, and all of them before the stores
+        auto at = [&](int r) { return 32 * j + 8 * (r >> 2) + 4 * h + (r & 3); };
+#pragma unroll
+        for (int r = 0; r < 16; ++r) first[r] = 0.0f;
+        for (int s = 0; s < (ks > 1 ? ks : 1); ++s) {
+            const float *p = (ks > 1 ? part + (size_t)s * stride : y) + (size_t)t0 * n_out + n;
+            float v[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = t0 + at(r) < rows ? p[(size_t)at(r) * n_out] : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) first[r] += v[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            if (t0 + at(r) < rows) y[(size_t)(t0 + at(r)) * n_out + n] = first[r] + acc[j][r];
+    }
 }
 
 // Two's-complement nibbles (as stored at upload) of one dword -> four signed bytes holding
@@ -545,9 +646,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // half stay free of bank conflicts; no nibbles to unpack.
 // Up to three tensors of equal K in one launch (q|k|v, gate|up of models::llama): tensor g owns the workgroups
 // wg0[g] .. wg0[g + 1] - 1 (unused slots hold INT_MAX).
-template <int QT, int NB, int MT, int NW, int NST>
+// Q41 (with QT = 4): Q4_1, whose value q d + m is (q - 8) d + (8 d + m): besides the Q4_0 product every block adds
+// 8 d + m times the block's plain sum of x, one FMA more per output; a unit holds the blocks' f16 m and the tokens' block sums too.
+template <int QT, int NB, int MT, int NW, int NST, bool Q41 = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <= 8 ? 4 : 2))) void gguf_skinny_kernel(const pg_skinny_group grp, int nb, int nbp, int m,
-                                                                    const int8_t *__restrict__ digits, const float *__restrict__ xs) {
+                                                                    const int8_t *__restrict__ digits, const float *__restrict__ xs,
+                                                                    const float *__restrict__ xsum) {
     int tg = 0;
 #pragma unroll
     for (int i = 1; i < 3; ++i) tg = (int)blockIdx.x >= grp.wg0[i] ? i : tg;
@@ -557,8 +661,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     const float *__restrict__ res = grp.res[tg];
     const int n_out = grp.n[tg];
     constexpr int WF = QT == 8 ? 4 : 2, W_T = WF * 1024, D_T = 256, DIG = MT * 512, XS_B = 512, GQ = MT / 2;  // WF, GQ: weight, digit fills per unit
-    constexpr int OFF_DS = NB * W_T, OFF_DG = OFF_DS + NB * D_T, OFF_X = OFF_DG + DIG, UNIT = OFF_X + XS_B;
-    constexpr int LPS = WF * NB + 1 + GQ + 1;  // fills per unit
+    constexpr int OFF_DS = NB * W_T, OFF_DG = OFF_DS + NB * D_T, OFF_X = OFF_DG + DIG, OFF_MS = OFF_X + XS_B;
+    constexpr int OFF_XSUM = OFF_MS + (Q41 ? NB * D_T : 0), UNIT = OFF_XSUM + (Q41 ? XS_B : 0);
+    constexpr int LPS = WF * NB + 1 + GQ + 1 + (Q41 ? 2 : 0);  // fills per unit
+    static_assert(!Q41 || QT == 4, "Q4_1 is the Q4_0 product and its offsets");
     static_assert((NST - 1) * LPS < 64 && NST <= 6 && NB <= 2, "the wait counter holds 63");
     extern __shared__ __attribute__((aligned(1024))) char lds[];  // NW rings of NST units; afterwards the wavefronts' tiles
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -583,6 +689,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     const int ntile = (n_out + 7) / 8;
     const int dt = pg_gskinny_scale_tile(n0, lane, ntile);
     const char *d_src = reinterpret_cast<const char *>(dsc) + pg_gskinny_scale_offset(dt, nb, 0, lane);
+    const char *ms_src = Q41 ? reinterpret_cast<const char *>(grp.mo[tg]) + pg_gskinny_scale_offset(dt, nb, 0, lane) : nullptr;
     // digits: instruction q covers runs 4 q .. 4 q + 3, run = 2 token + plane; lane -> run 4 q + lane / 16, position lane % 16
     const int8_t *g_src[GQ];
 #pragma unroll
@@ -593,6 +700,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     }
     // token scales: lanes 0 .. 2 MT - 1: token lane / 2, blocks 4 (lane % 2) .. + 3 of the unit
     const float *x_src = xs + (size_t)((lane >> 1) < m ? (lane >> 1) : 0) * nbp + 4 * (lane & 1);
+    const float *sum_src = Q41 ? xsum + (x_src - xs) : nullptr;
 
     const int rot = cnt > 0 ? (int)((blockIdx.x * 5u) % (unsigned)cnt) : 0;
     auto issue = [&](auto slot, int t) {
@@ -608,6 +716,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
         for (int q = 0; q < GQ; ++q)
             __builtin_amdgcn_global_load_lds((gptr_t)(g_src[q] + unit * 256), (lptr_t)(base + OFF_DG + q * 1024), 16, 0, 0);
         if (lane < 2 * MT) __builtin_amdgcn_global_load_lds((gptr_t)(x_src + unit * 8), (lptr_t)(base + OFF_X), 16, 0, 0);
+        if constexpr (Q41) {
+            if (lane < 16 * NB) __builtin_amdgcn_global_load_lds((gptr_t)(ms_src + unit * 128), (lptr_t)(base + OFF_MS), 16, 0, 0);
+            if (lane < 2 * MT) __builtin_amdgcn_global_load_lds((gptr_t)(sum_src + unit * 8), (lptr_t)(base + OFF_XSUM), 16, 0, 0);
+        }
     };
 
     // fragment reads of this lane
@@ -642,7 +754,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
             const int blk = 4 * J + g4;
             // the lane's rows (one a tile) and block: 32 weight bytes each as eight dwords in the order of the digit halves
             int wk[NB][8];
-            float dv[NB];
+            float dv[NB], cv[NB];
 #pragma unroll
             for (int c = 0; c < NB; ++c) {
                 const char *wt = base + c * W_T;
@@ -663,6 +775,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
                     }
                 }
                 dv[c] = half_bits_to_float(*reinterpret_cast<const unsigned short *>(base + ds_rd + c * D_T + blk * 16));
+                if constexpr (Q41) {  // (the sum is divided by 16 at the end)
+                    const float mv = half_bits_to_float(*reinterpret_cast<const unsigned short *>(base + ds_rd + (OFF_MS - OFF_DS) + c * D_T + blk * 16));
+                    cv[c] = fmaf(128.0f, dv[c], 16.0f * mv);
+                }
             }
 #pragma unroll
             for (int s2 = 0; s2 < NQ; ++s2) {
@@ -675,6 +791,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
                 int sx[4];  // the scales of tokens 4 s2 .. + 3 for this lane's block (read as integers: see gguf_mm_kernel)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) sx[i] = *reinterpret_cast<const int *>(base + OFF_X + (4 * s2 + i) * 32 + blk * 4);
+                int sm[4] = {0, 0, 0, 0};  // and their block sums
+                if constexpr (Q41) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sm[i] = *reinterpret_cast<const int *>(base + OFF_XSUM + (4 * s2 + i) * 32 + blk * 4);
+                }
 #pragma unroll
                 for (int c = 0; c < NB; ++c) {
                     v4i ihi = {0, 0, 0, 0}, ilo = {0, 0, 0, 0};
@@ -692,6 +813,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
                     for (int i = 0; i < 4; ++i) {
                         const float fx = (float)(ihi[i] * 256 + ilo[i]) * __int_as_float(sx[i]);
                         acc[c * NQ + s2][i] = fmaf(dv[c], fx, acc[c * NQ + s2][i]);
+                        if constexpr (Q41) acc[c * NQ + s2][i] = fmaf(cv[c], __int_as_float(sm[i]), acc[c * NQ + s2][i]);
                     }
                 }
             }
@@ -717,9 +839,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
         // Software pipeline over the unit's 8 blocks: while block j is scaled and accumulated on the vector ALU,
         // the MFMAs of block j + 1 run and the LDS reads of block j + 2 return (one wavefront a SIMD: nothing else
         // would fill those waits).
+        int sm[Q41 ? 4 : 1][8];  // and their block sums
+        if constexpr (Q41) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const v4i t = *reinterpret_cast<const v4i *>(base + (OFF_XSUM - OFF_X) + x_rd + i * 32 + h * 16);
+                    const int t0 = t[0], t1 = t[1], t2 = t[2], t3 = t[3];
+                    sm[i][4 * h] = t0; sm[i][4 * h + 1] = t1; sm[i][4 * h + 2] = t2; sm[i][4 * h + 3] = t3;
+                }
+        }
         long dh[2], dl[2];
         v2i wraw[2][NB];
-        unsigned db[2][NB];
+        unsigned db[2][NB], mb[2][Q41 ? NB : 1];
         v4i ihi[2][NB], ilo[2][NB];
         auto read = [&](int buf, int j) {
             const int dpos = (((2 * j + (g4 >> 1)) ^ ft) * 16);
@@ -731,6 +864,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
         auto read_d = [&](int buf, int j) {  // the blocks' weight scales of this lane's rows
 #pragma unroll
             for (int c = 0; c < NB; ++c) db[buf][c] = *reinterpret_cast<const unsigned short *>(base + ds_rd + c * D_T + j * 16);
+            if constexpr (Q41) {
+#pragma unroll
+                for (int c = 0; c < NB; ++c) mb[buf][c] = *reinterpret_cast<const unsigned short *>(base + ds_rd + (OFF_MS - OFF_DS) + c * D_T + j * 16);
+            }
         };
         auto mfmas = [&](int buf, int c) {
             const v4i zero = {0, 0, 0, 0};
@@ -752,6 +889,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
                 for (int i = 0; i < 4; ++i) {
                     const float fx = (float)(ihi[buf][c][i] * 256 + ilo[buf][c][i]) * __int_as_float(sx[i][j]);
                     acc[c][i] = fmaf(dv, fx, acc[c][i]);
+                }
+                if constexpr (Q41) {  // (the sum is divided by 16 at the end)
+                    const float cv = fmaf(128.0f, dv, 16.0f * half_bits_to_float(mb[buf][c]));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[c][i] = fmaf(cv, __int_as_float(sm[i][j]), acc[c][i]);
                 }
             }
         };
@@ -886,19 +1028,19 @@ pg_status pg_launch_x_to_mm_digits(pg_ctx *ctx, const float *x_dev, size_t rows,
                      (float *)nullptr);
 }
 
-pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mmdigits &md, size_t rows, float *y) {
+pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mmdigits &md, size_t rows, const float *part, int ks, float *y) {
     const int nb = (int)(w->k_in / 32), nbp = (int)pg_round_up(nb, 4);
-    const bool few = rows <= 64;
-    const size_t lds = ((size_t)nb + (few ? 3 * 64 : 0)) * Q41_TT * sizeof(float);
+    const size_t stride = rows * w->n_out;
+    if (rows > 64) {
+        if ((rows + 63) / 64 > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_matmul: too many activation rows");
+        return pg_launch(ctx, "gguf_q4_1_offsets", q41_offset_mfma_kernel, dim3(grid_for(w->n_out, 128), (unsigned)((rows + 63) / 64)), dim3(256), 0,
+                         (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, (const float *)md.xsum, nbp, (int)rows, part, ks, stride, y);
+    }
+    const size_t lds = ((size_t)nb * Q41_TT + 256 * (Q41_TT + 1)) * sizeof(float);
     if (lds > 128 * 1024) return pg_fail(PG_EUNSUPPORTED, "gguf_matmul: Q4_1 rows of %zu on the matrix-core route", w->k_in);
-    PG_TRY(pg_allow_dynamic_lds(ctx, few ? (const void *)q41_offset_kernel<4> : (const void *)q41_offset_kernel<1>, 128 * 1024));
-    if ((rows + Q41_TT - 1) / Q41_TT > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_matmul: too many activation rows");
-    const dim3 grid(grid_for(w->n_out, few ? 64 : 256), (unsigned)((rows + Q41_TT - 1) / Q41_TT));
-    if (few)
-        return pg_launch(ctx, "gguf_q4_1_offsets", q41_offset_kernel<4>, grid, dim3(256), lds, (const uint16_t *)w->d,
-                         (const uint16_t *)w->m, (int)w->n_out, nb, (const float *)md.xsum, nbp, (int)rows, y);
-    return pg_launch(ctx, "gguf_q4_1_offsets", q41_offset_kernel<1>, grid, dim3(256), lds, (const uint16_t *)w->d,
-                     (const uint16_t *)w->m, (int)w->n_out, nb, (const float *)md.xsum, nbp, (int)rows, y);
+    PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)q41_offset_kernel, 128 * 1024));
+    return pg_launch(ctx, "gguf_q4_1_offsets", q41_offset_kernel, dim3(grid_for(w->n_out, 256 / Q41_NQ), (unsigned)((rows + Q41_TT - 1) / Q41_TT)), dim3(256), lds,
+                     (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, (const float *)md.xsum, nbp, (int)rows, part, ks, stride, y);
 }
 
 // Digits of `act_rows` activation rows that no XCD's L2 (4 MiB) can keep while every workgroup
@@ -948,7 +1090,8 @@ int pg_gguf_mm_splitk(const pg_ctx *ctx, size_t n_out, size_t k_in, size_t group
 // bytes its rings keep in flight: 4 x 4096 -> 14336 takes 9.0 us (with its arithmetic switched off 8.6 - 9.1; in the
 // 16 x 16 x 32 form it took 11.9).
 bool pg_gguf_skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out, size_t k_in) {
-    return (ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0) && m >= 2 && (m <= 8 || (m <= 16 && n_out / 32 < (size_t)ctx->num_cu)) &&
+    // (Q4_1 below eight rows stays with the streaming kernel and its finer fixed point)
+    return (ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0 || (ggml_type == PG_GGML_Q4_1 && m >= 8)) && m >= 2 && (m <= 8 || (m <= 16 && n_out / 32 < (size_t)ctx->num_cu)) &&
            k_in % 256 == 0 && k_in >= 1024 && n_out >= 1 && n_out < (1u << 30) && k_in < (1u << 24);
 }
 
@@ -969,7 +1112,8 @@ pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, c
     // Two weight tiles a workgroup (32 rows) where that still leaves a workgroup for every CU: the digits, which
     // every workgroup fetches for all of K, then cost half as much per weight byte.
     const int tiles = (m <= 8 && n_total / 32 >= (size_t)ctx->num_cu) ? 2 : 1;
-    const size_t unit_bytes = (size_t)tiles * ((q8 ? 4096 : 2048) + 256) + (m <= 4 ? 4 : (m <= 8 ? 8 : 16)) * 512 + 512;
+    const bool q41 = ggml_type == PG_GGML_Q4_1;
+    const size_t unit_bytes = (size_t)tiles * ((q8 ? 4096 : 2048) + (q41 ? 512 : 256)) + (m <= 4 ? 4 : (m <= 8 ? 8 : 16)) * 512 + (q41 ? 1024 : 512);
     const int stages = 2;  // (three stages on fewer wavefronts: 10.7 - 10.9 against 9.0 us on 4 x 4096 -> 14336)
     const size_t lds_cu = 160u << 10;
     pg_skinny_group grp;
@@ -978,6 +1122,7 @@ pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, c
         const bool used = i < count;
         grp.qs[i] = used ? w[i]->qs : nullptr;
         grp.d[i] = used ? w[i]->d : nullptr;
+        grp.mo[i] = used ? w[i]->m : nullptr;
         grp.y[i] = used ? y[i] : nullptr;
         grp.res[i] = i == 0 ? residual : nullptr;
         grp.n[i] = used ? (int)w[i]->n_out : 0;
@@ -988,7 +1133,7 @@ pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, c
     // LDS is handed out per workgroup: nw wavefronts' rings each; up to 16 wavefronts a CU (4 a SIMD)
     const size_t units = (size_t)nb / 8;
     auto fits = [&](int nw_) {
-        if (m > 8) return (size_t)grid.x * nw_ <= (size_t)ctx->num_cu * (q8 ? 6 : 7);
+        if (m > 8) return (size_t)grid.x * nw_ <= (size_t)ctx->num_cu * (q8 || q41 ? 6 : 7);
         const size_t per_cu = std::min<size_t>(lds_cu / ((size_t)nw_ * stages * unit_bytes), 16 / nw_);
         return (size_t)grid.x <= (size_t)ctx->num_cu * per_cu;
     };
@@ -996,11 +1141,11 @@ pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, c
     while (nw > 1 && (!fits(nw) || units / nw < 4)) nw >>= 1;
 #define PG_GSK_LAUNCH(QTT, NBB, MTT, NWW, NSTT)                                                                                \
     do {                                                                                                                       \
-        auto kern = gguf_skinny_kernel<QTT, NBB, MTT, NWW, NSTT>;                                                              \
-        const size_t lds = (size_t)NWW * NSTT * (NBB * ((QTT == 8 ? 4096 : 2048) + 256) + MTT * 512 + 512);                    \
+        auto kern = gguf_skinny_kernel<QTT == 8 ? 8 : 4, NBB, MTT, NWW, NSTT, QTT == 5>;                                       \
+        const size_t lds = (size_t)NWW * NSTT * (NBB * ((QTT == 8 ? 4096 : 2048) + (QTT == 5 ? 512 : 256)) + MTT * 512 + (QTT == 5 ? 1024 : 512)); \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
-        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_few_rows_mm" : "gguf_q4_0_few_rows_mm", kern, grid, dim3(64 * NWW), lds,  \
-                         grp, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs);                               \
+        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_few_rows_mm" : (QTT == 5 ? "gguf_q4_1_few_rows_mm" : "gguf_q4_0_few_rows_mm"), kern, grid, \
+                         dim3(64 * NWW), lds, grp, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs, (const float *)md.xsum); \
     } while (0)
 #define PG_GSK_NW8(QTT, NBB, MTT, NSTT)                     \
     switch (nw) {                                           \
@@ -1019,6 +1164,10 @@ pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, c
         if (m <= 4) { if (tiles == 2) PG_GSK_NW8(8, 2, 4, 2) else PG_GSK_NW8(8, 1, 4, 2) }
         if (m <= 8) { if (tiles == 2) PG_GSK_NW8(8, 2, 8, 2) else PG_GSK_NW8(8, 1, 8, 2) }
         PG_GSK_NW4(8, 16, 2)
+    }
+    if (q41) {  // (5 names Q4_1 here)
+        if (m <= 8) { if (tiles == 2) PG_GSK_NW8(5, 2, 8, 2) else PG_GSK_NW8(5, 1, 8, 2) }
+        PG_GSK_NW4(5, 16, 2)
     }
     if (m <= 4) { if (tiles == 2) PG_GSK_NW8(4, 2, 4, 2) else PG_GSK_NW8(4, 1, 4, 2) }
     if (m <= 8) { if (tiles == 2) PG_GSK_NW8(4, 2, 8, 2) else PG_GSK_NW8(4, 1, 8, 2) }

@@ -363,6 +363,7 @@ bool pg_gguf_skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_o
 struct pg_skinny_group {  // the tensors of one few-rows launch (gguf_skinny_kernel)
     const uint8_t *qs[3];
     const uint16_t *d[3];
+    const uint16_t *mo[3];  // Q4_1 only: the blocks' offsets
     float *y[3];
     const float *res[3];  // where set: y = res + product (same shape as y)
     int n[3];
@@ -375,7 +376,8 @@ pg_status pg_launch_x_to_mm_digits(pg_ctx *ctx, const float *x_dev, size_t rows,
 // Q4_1 on the matrix-core route: the product is the Q4_0 product on the same nibbles and scales plus
 // y[t][n] += sum_b (8 d + m)[n][b] * (sum of x over block b of row t); this adds the second term (md.xsum
 // as pg_launch_x_to_mm_digits leaves it for PG_GGML_Q4_1).  k_in up to 32768.
-pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mmdigits &md, size_t rows, float *y);
+// With ks > 1 the first term is still the ks planes at `part` (rows * n_out floats each), added up on the way.
+pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mmdigits &md, size_t rows, const float *part, int ks, float *y);
 // Which activation rows multiply which weights.  Without `counts`: one weight tensor and pairs
 // 0 .. max_count-1.  With `counts`: expert e owns counts[e] pairs, listed (in ascending order) in
 // lists[e * list_stride ..]; its weights are qs_table[e] / d_table[e].  Pair p reads activation

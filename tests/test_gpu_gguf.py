@@ -377,3 +377,24 @@ def test_gguf_matmul_f16_route_every_quant_value(ctx, orc, typ, bb):
     for r in range(m):
         H.assert_close_rel(got[r], want[r], RTOL_F16_ROUTE, f"row {r}")
     gw.free()
+
+
+@pytest.mark.parametrize("n_out,k_in,m", [
+    (4096, 4096, 8), (1003, 1024, 8), (8200, 1280, 8), (14336, 4096, 8),   # 4 x 4 x 4 products: one and two weight tiles, ragged
+    (4096, 4096, 12), (77, 2304, 9), (4100, 8192, 16), (40, 36864, 11),    # 16 x 16 x 32 products
+    (14336, 4096, 12), (130, 1120, 17), (257, 4096, 64), (515, 2048, 65), (15, 256, 33),  # the offsets by a launch of their own
+])
+def test_gguf_q4_1_few_rows(ctx, orc, n_out, k_in, m):
+    """Q4_1 at 8 .. 16 rows in one launch after the digits (offsets inside), and the offset launch at the edges of its
+    16-row workgroups and 16-token tiles."""
+    from peregrine_amd import gguf
+    say(f"gguf_matmul Q4_1 few rows n_out={n_out} k_in={k_in} m={m}")
+    raw = H.pack_q4_1(orc.rng_normal(31 + n_out, n_out * k_in, 0.0, 0.02) + np.float32(0.03))
+    x = orc.rng_normal(33 + m, m * k_in)
+    x.reshape(m, k_in)[:, :: max(1, k_in // 40)] *= 20
+    gw = gguf.GgufWeight(raw, 3, n_out, k_in, ctx)
+    got, want = gw.matmul(x, m), orc.gguf_matmul(x, m, raw, 3, n_out, k_in)
+    for r in range(m):
+        sl = slice(r * n_out, (r + 1) * n_out)
+        H.assert_close_rel(got[sl], want[sl], RTOL_ACHIEVED_MM, f"row {r}")
+    gw.free()
