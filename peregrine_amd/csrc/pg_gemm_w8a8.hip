@@ -59,14 +59,20 @@ struct gemm_wgroup {
     int panel0[PG_GEMM_MAX_GROUP];
     // The last pass of the W8A32 product (one weight): with `comb` the accumulator is the digit of weight 65536
     // and the output is (65536 acc + 256 comb[comb_plane + i] + comb[i]) * a_scale * w_scale, the integer exact
-    // and the scaling done in f64 (what combine_digits3_kernel computes from three stored planes).
+    // and the scaling done in f64.
     const int32_t *comb;
     long long comb_plane;
+    int a_plane;  // NP planes of activations: bytes from one to the next
 };
 
+// NP = 3: the W8A32 product in one launch.  The activations are three digit planes (weights 1, 256, 65536); a stage holds
+// BM rows of each, every weight fragment meets all three, and the epilogue joins the three accumulators as COMB does.
+// One pass over the weights and no accumulator planes in memory: for tiles up to 128x128, where 3 x TM x TN
+// accumulators fit the registers (197 x 1024 -> 4096: 17.4 us as two launches, 8.2 so).
+//
 // CLK (the clock probe only): thread 0 of every workgroup also stores the shader cycles and the
 // wall-clock ticks its K loop took, clk[2 * blockIdx.x] and clk[2 * blockIdx.x + 1].
-template <int BM, int BN, int BK, int NST, int NWM, int NWN, int OCC, bool CLK = false, bool COMB = false>
+template <int BM, int BN, int BK, int NST, int NWM, int NWN, int OCC, bool CLK = false, bool COMB = false, int NP = 1>
 __global__ __launch_bounds__(64 * NWM * NWN) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup grp, int ldb,
                       const float *__restrict__ a_scales, int32_t *__restrict__ acc_out, int M, int K,
@@ -75,10 +81,11 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     constexpr int WM = BM / NWM, WN = BN / NWN;      // wavefront tile
     constexpr int TM = WM / 32, TN = WN / 32;        // 32x32 MFMA tiles per wavefront
     constexpr int CPR = BK / 16, RPL = 64 / CPR;     // chunks per row, rows per wave-load
-    constexpr int LA = BM / RPL / NW, LB = BN / RPL / NW, LPS = LA + LB;  // wave-loads per wave per stage
-    constexpr int STAGE = (BM + BN) * BK;            // bytes per LDS stage
+    constexpr int LA = NP * BM / RPL / NW, LB = BN / RPL / NW, LPS = LA + LB;  // wave-loads per wave per stage
+    constexpr int STAGE = (NP * BM + BN) * BK;            // bytes per LDS stage
     constexpr int KS = BK / 32;                      // k-steps per stage
-    constexpr int NF = TM + TN, NMFMA = TM * TN;
+    constexpr int TA = NP * TM;                      // activation tiles per wavefront, plane by plane
+    constexpr int NF = TA + TN, NMFMA = TA * TN;
     static_assert(LA >= 1 && LB >= 1 && KS % 2 == 0 && BM <= 64 * NW && BN <= 64 * NW, "unsupported tile configuration");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 
@@ -108,7 +115,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int row = RPL * (wave + NW * i) + lr;
-        a_goff[i] = row * lda + 16 * (pc ^ swz<BK>(row));
+        a_goff[i] = (row % BM) * lda + row / BM * (NP > 1 ? grp.a_plane : 0) + 16 * (pc ^ swz<BK>(row));
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
@@ -129,7 +136,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     for (int ks = 0; ks < KS; ++ks) {
         const int ra = wm * WM + l31, rb = wn * WN + l31;
         a_off[ks] = ra * BK + (((2 * ks + half) ^ swz<BK>(ra)) * 16);
-        b_off[ks] = BM * BK + rb * BK + (((2 * ks + half) ^ swz<BK>(rb)) * 16);
+        b_off[ks] = NP * BM * BK + rb * BK + (((2 * ks + half) ^ swz<BK>(rb)) * 16);
     }
 
     // The scales of this tile's rows and columns go to LDS (behind the stages) now, so that
@@ -141,9 +148,9 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
         if (t < BN) lds_ws[t] = w_scales[n0 + t < N ? n0 + t : N - 1];
     }
 
-    v16i acc[TM][TN];
+    v16i acc[TA][TN];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TA; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -155,19 +162,19 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
         for (int i = 0; i < LA; ++i) load_to_lds_16(a_base + a_goff[i] + k0, base + (wave + NW * i) * 1024);
 #pragma unroll
         for (int i = 0; i < LB; ++i)
-            load_to_lds_16(b_base + b_goff[i] + k0, base + BM * BK + (wave + NW * i) * 1024);
+            load_to_lds_16(b_base + b_goff[i] + k0, base + NP * BM * BK + (wave + NW * i) * 1024);
     };
-    v4i fa[2][TM], fb[2][TN];
+    v4i fa[2][TA], fb[2][TN];
     auto read_frags = [&](int buf, int stage, int ks) {
         const char *base = lds + stage * STAGE;
 #pragma unroll
-        for (int i = 0; i < TM; ++i) fa[buf][i] = *reinterpret_cast<const v4i *>(base + a_off[ks] + i * 32 * BK);
+        for (int i = 0; i < TA; ++i) fa[buf][i] = *reinterpret_cast<const v4i *>(base + a_off[ks] + (i / TM * BM + i % TM * 32) * BK);
 #pragma unroll
         for (int j = 0; j < TN; ++j) fb[buf][j] = *reinterpret_cast<const v4i *>(base + b_off[ks] + j * 32 * BK);
     };
-    auto mfmas = [&](int buf, int lo, int hi) {  // MFMAs lo..hi-1 of the TM x TN set, row-major
+    auto mfmas = [&](int buf, int lo, int hi) {  // MFMAs lo..hi-1 of the TA x TN set, row-major
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TA; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
                 if (i * TN + j >= lo && i * TN + j < hi)
@@ -244,6 +251,27 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     // ---- epilogue.  Accumulator register r of a 32x32 tile holds
     // row 8*(r/4) + 4*(lane/32) + r%4, column lane%32.  (The scales were requested before the
     // K loop: loading them here would put several dependent memory round trips on every tile.)
+    if constexpr (NP == 3) {
+        const bool whole = m0 + BM <= M && n0 + BN <= N;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int n = n0 + wn * WN + 32 * j + l31;
+                const double ws = (double)lds_ws[wn * WN + 32 * j + l31];
+                float *dst = out + (size_t)(m0 + wm * WM + 32 * i + 4 * half) * N + n;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int mr = 8 * (r >> 2) + (r & 3);
+                    const double v = 65536.0 * (double)acc[2 * TM + i][j][r] + 256.0 * (double)acc[TM + i][j][r] + (double)acc[i][j][r];
+                    if (whole || (m0 + wm * WM + 32 * i + 4 * half + mr < M && n < N))
+                        __builtin_nontemporal_store((float)(v * (double)lds_as[wm * WM + 32 * i + 4 * half + mr] * ws), dst + (size_t)mr * N);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        return;
+    }
     if (!COMB && out && !acc_out && m0 + BM <= M && n0 + BN <= N) {
         // A whole tile inside the matrix, f32 output only (every tile of the prefill shapes):
         // straight-line code, the 16 row scales of a 32-row tile as four 128-bit LDS reads.
@@ -350,10 +378,10 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     }
 }
 
-template <int BM, int BN, int BK, int NST, int NWM, int NWN, int OCC, bool COMB = false>
+template <int BM, int BN, int BK, int NST, int NWM, int NWN, int OCC, bool COMB = false, int NP = 1>
 pg_status launch_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                        const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc,
-                       int splits = 1, int kt_per_split = 0, const int32_t *comb = nullptr, size_t comb_plane = 0) {
+                       int splits = 1, int kt_per_split = 0, const int32_t *comb = nullptr, size_t comb_plane = 0, size_t a_plane = 0) {
     const int tiles_m = (int)((m + BM - 1) / BM);
     gemm_wgroup grp;
     int panels = 0;
@@ -368,9 +396,10 @@ pg_status launch_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const f
     }
     grp.comb = comb;
     grp.comb_plane = (long long)comb_plane;
+    grp.a_plane = (int)a_plane;
     const int ntiles = tiles_m * panels;
-    const size_t lds = (size_t)NST * (BM + BN) * BK + (BM + BN) * sizeof(float);
-    auto kern = gemm_w8a8_kernel<BM, BN, BK, NST, NWM, NWN, OCC, false, COMB>;
+    const size_t lds = (size_t)NST * (NP * BM + BN) * BK + (BM + BN) * sizeof(float);
+    auto kern = gemm_w8a8_kernel<BM, BN, BK, NST, NWM, NWN, OCC, false, COMB, NP>;
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
     const unsigned grid = (unsigned)(((ntiles + 7) / 8) * 8);
     const size_t k_pad = w[0]->k_pad;
@@ -378,7 +407,7 @@ pg_status launch_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const f
     ctx->gemm_last_bm = BM;
     ctx->gemm_last_bn = BN;
     ctx->gemm_last_splits = splits;
-    PG_TRY(pg_launch(ctx, "gemm_w8a8", kern, dim3(grid, (unsigned)splits), dim3(64 * NWM * NWN), lds, a_i8, (int)a_stride, grp,
+    PG_TRY(pg_launch(ctx, NP == 3 ? "gemm_w8a32" : "gemm_w8a8", kern, dim3(grid, (unsigned)splits), dim3(64 * NWM * NWN), lds, a_i8, (int)a_stride, grp,
                      (int)k_pad, a_scales, acc, (int)m, (int)k_pad, tiles_m, ntiles, kt_per_split, (long long *)nullptr));
     return pg_launch_check("gemm_w8a8");
 }
@@ -440,10 +469,13 @@ struct skinny_wgroup {
     int wg0[PG_GEMM_MAX_GROUP];
 };
 
-template <int MB, int NB, int NW, int NST>
+// TRI: the W8A32 product.  The activations are three digit planes a_plane bytes apart (weights 1, 256, 65536); tile b is
+// tile b % (MB / 3) of plane b / (MB / 3), and the final pass joins the three sums in f64.
+template <int MB, int NB, int NW, int NST, bool TRI = false>
 __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t *__restrict__ a_i8, const skinny_wgroup grp,
                                                                     int k_pad, int m, const float *__restrict__ a_scales,
-                                                                    int32_t *__restrict__ acc_out) {
+                                                                    int32_t *__restrict__ acc_out, size_t a_plane) {
+    constexpr int MT = TRI ? MB / 3 : MB;  // tiles of activation rows
     int g = 0;
 #pragma unroll
     for (int i = 1; i < PG_GEMM_MAX_GROUP; ++i) g = (int)blockIdx.x >= grp.wg0[i] ? i : g;
@@ -468,7 +500,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
 #pragma unroll
         for (int c = 0; c < NB; ++c) src[c][j] = w_t + pg_skinny_fill_offset(n0 + 16 * c + r, k_pad, 0, ch);  // (weight rows are padded to 256)
 #pragma unroll
-        for (int b = 0; b < MB; ++b) src[NB + b][j] = a_i8 + pg_skinny_fill_offset(16 * b + r, k_pad, 0, ch);
+        for (int b = 0; b < MB; ++b) src[NB + b][j] = a_i8 + (TRI ? b / MT * a_plane : 0) + pg_skinny_fill_offset(16 * (b % MT) + r, k_pad, 0, ch);
     }
     // fragment reads: row lane % 16, chunk 4 s + lane / 16 of k-step s
     const int fr = lane & 15, fsw = (fr >> 1) & 7;
@@ -540,6 +572,22 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
 #pragma unroll
             for (int i = 0; i < 4; ++i) red[((wave * NB * MB + c * MB + b) * 4 + i) * 64 + lane] = acc[c][b][i];
     __syncthreads();
+    if constexpr (TRI) {
+        for (int e = threadIdx.x; e < NB * MT * 4 * 64; e += 64 * NW) {
+            const int l = e & 63, i = (e >> 6) & 3, cb = e >> 8, c = cb / MT, b = cb - c * MT;
+            int sum[3] = {0, 0, 0};
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int w = 0; w < NW; ++w) sum[p] += red[((w * NB * MB + c * MB + p * MT + b) * 4 + i) * 64 + l];
+            const int row = b * 16 + 4 * (l >> 4) + i, col = n0 + 16 * c + (l & 15);
+            if (row < m && col < n) {
+                const double v = 65536.0 * (double)sum[2] + 256.0 * (double)sum[1] + (double)sum[0];
+                out[(size_t)row * n + col] = (float)(v * (double)a_scales[row] * (double)w_scales[col]);
+            }
+        }
+        return;
+    }
     for (int e = threadIdx.x; e < NB * MB * 4 * 64; e += 64 * NW) {
         const int l = e & 63, i = (e >> 6) & 3, cb = e >> 8, c = cb / MB, b = cb - c * MB;
         int sum = 0;
@@ -684,7 +732,7 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         auto kern = gemm_w8a8_skinny_kernel<MBB, NBB, NWW, NSTT>;                                                            \
         const size_t lds = (size_t)NWW * NSTT * (NBB + MBB) * 2048;                                                          \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                          \
-        return pg_launch(ctx, "gemm_w8a8_few_rows", kern, grid, dim3(64 * NWW), lds, a_i8, grp, (int)k_pad, (int)m, a_scales, acc); \
+        return pg_launch(ctx, "gemm_w8a8_few_rows", kern, grid, dim3(64 * NWW), lds, a_i8, grp, (int)k_pad, (int)m, a_scales, acc, (size_t)0); \
     } while (0)
 #define PG_SKINNY_NW8(MBB, NBB, NSTT)                       \
     switch (nw) {                                           \
@@ -737,6 +785,58 @@ pg_status pg_launch_gemm_w8a8(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride,
     return gemm_dispatch(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, acc);
 }
 
+// The W8A32 product over three digit planes in one launch, where it is the better route: up to 32 rows the few-row kernel
+// (three or six tiles of planes), beyond that tiles of 64x64 to 128x128, unless tiles of 256x256 fill the part (then the
+// two low planes stacked and the combining pass below; `takes` says which).  128x128 from one tile a CU on.
+static bool w8a32_large(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+    const size_t cus = (size_t)ctx->num_cu, t256 = ((m + 255) / 256) * ((w->cols + 255) / 256);
+    return t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus);
+}
+bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+    return ctx->gemm_force_tile == 0 && !w8a32_large(ctx, w, m) && w->k_pad < (1ull << 22) && w->cols < (1ull << 30) &&
+           2 * pg_round_up(m, PG_MPAD) * w->k_pad + 128 * w->k_pad < (1ull << 31);
+}
+pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out) {
+    if (!pg_gemm_w8a32_takes(ctx, w, m)) return pg_fail(PG_EINVAL, "gemm_w8a32: m = %zu", m);
+    const size_t k_pad = w->k_pad, n = w->cols;
+    if (m <= 32) {
+        skinny_wgroup grp;
+        for (int i = 0; i < PG_GEMM_MAX_GROUP; ++i) {
+            grp.w[i] = i ? nullptr : w->w_t;
+            grp.ws[i] = i ? nullptr : w->scales;
+            grp.out[i] = i ? nullptr : out;
+            grp.n[i] = i ? 0 : (int)n;
+            grp.wg0[i] = i ? INT_MAX : 0;
+        }
+        // rings of 24 KiB (three tiles of planes, three stages) or 28 (six, two stages): six and five wavefronts a CU
+        const dim3 grid((unsigned)((n + 15) / 16));
+        const size_t slots = (size_t)ctx->num_cu * (m <= 16 ? 6 : 5), units = k_pad / 128;
+        int nw = 4;
+        while (nw > 1 && ((size_t)grid.x * nw > slots || units / nw < 2)) nw >>= 1;
+        auto go = [&](auto kern, size_t lds) -> pg_status {
+            PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
+            return pg_launch(ctx, "gemm_w8a32_few_rows", kern, grid, dim3(64 * nw), lds, planes, grp, (int)k_pad, (int)m, a_scales, (int32_t *)nullptr, plane_bytes);
+        };
+        if (m <= 16) {
+            const size_t lds = (size_t)nw * 3 * 4 * 2048;
+            return nw == 4 ? go(gemm_w8a8_skinny_kernel<3, 1, 4, 3, true>, lds) : nw == 2 ? go(gemm_w8a8_skinny_kernel<3, 1, 2, 3, true>, lds)
+                                                                                            : go(gemm_w8a8_skinny_kernel<3, 1, 1, 3, true>, lds);
+        }
+        const size_t lds = (size_t)nw * 2 * 7 * 2048;
+        return nw == 4 ? go(gemm_w8a8_skinny_kernel<6, 1, 4, 2, true>, lds) : nw == 2 ? go(gemm_w8a8_skinny_kernel<6, 1, 2, 2, true>, lds)
+                                                                                        : go(gemm_w8a8_skinny_kernel<6, 1, 1, 2, true>, lds);
+    }
+    // One workgroup fits a CU whatever the tile: rounds of workgroups times what a round takes (us at K = 4096: 26 for
+    // 64x64, 29 for 64x128, 40 for 128x128; 700 x 1024 -> 4096 19.8 / 17.2 / 15.3, 2048 x 4096 -> 1024 57 / 33 / 44).
+    auto cost = [&](size_t bm, size_t bn, size_t us) { return (((m + bm - 1) / bm) * ((n + bn - 1) / bn) + ctx->num_cu - 1) / ctx->num_cu * us; };
+    const size_t c0 = cost(64, 64, 26), c1 = cost(64, 128, 29), c2 = cost(128, 128, 40);
+    if (c2 < c0 && c2 < c1)
+        return launch_group<128, 128, 128, 2, 2, 4, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes);
+    if (c1 < c0)
+        return launch_group<64, 128, 128, 2, 2, 4, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes);
+    return launch_group<64, 64, 128, 3, 2, 2, 1, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes);
+}
+
 // The W8A32 product's last pass: `a_i8` is the digit plane of weight 65536, `comb` holds the accumulators of
 // the other two ([2][comb_plane], the plane of weight 256 second); writes the finished f32 product.
 pg_status pg_launch_gemm_w8a8_combine(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
@@ -774,6 +874,7 @@ PG_API pg_status pg_probe_gemm_clock(pg_ctx *ctx, size_t m, size_t k, size_t n, 
     }
     grp.comb = nullptr;
     grp.comb_plane = 0;
+    grp.a_plane = 0;
     grp.w[0] = b.as<int8_t>(); grp.ws[0] = sc.as<float>(); grp.out[0] = out.as<float>(); grp.n[0] = (int)n; grp.panel0[0] = 0;
     const size_t lds = (size_t)NST * (BM + BN) * BK + (BM + BN) * sizeof(float);
     auto kern = gemm_w8a8_kernel<BM, BN, BK, NST, 2, 4, 2, true>;

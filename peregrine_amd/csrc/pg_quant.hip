@@ -19,55 +19,118 @@ __device__ __forceinline__ int quant_to_i8(float v) { return pg_quant_to_i8(v); 
 __device__ __forceinline__ float wave_max(float v) { return pg_wave_max_f32(v); }
 __device__ __forceinline__ float block_max_256(float v, float *red) { return pg_block_max_256(v, red); }
 
-// One workgroup per row.  The row is read once into registers (up to
-// 4*256*MAXV floats), reduced to its absmax, then rounded to i8 and written as
-// packed dwords.  Columns [cols, q_stride) of the output row are zero-filled.
-template <int MAXV>
-__global__ __launch_bounds__(QA_THREADS) void quantize_rows_vec4_kernel(
+// ---- f32 rows as three signed byte digits ---------------------------------------------
+// x[k] ~= s * X[k], X = 65536 d2 + 256 d1 + d0 with signed byte digits, |X| <= 8355711, s a power of two:
+// 23 to 24 bits of fixed point per row, exact integer arithmetic on the matrix cores afterwards.
+// planes[p][row][k] (p = 0: d0 .. 2: d2), rows of q_stride bytes, pad columns zero.
+constexpr float DIG3_MAX = 8355711.0f;  // 127 * (65536 + 256 + 1)
+
+// The power-of-two scale of a row of largest magnitude amax (not finite: NaN, which the product hands on) and its inverse.
+// x -> X is exact whenever x has no bits below s (integers stay integers), and s * X is exact again on the way back.
+__device__ __forceinline__ void digits3_scale(float amax, bool finite, float &s, float &inv) {
+    s = 1.0f;
+    inv = 1.0f;
+    if (!finite) {
+        s = __uint_as_float(0x7FC00000u);
+        inv = 0.0f;
+    } else if (amax > 0.0f) {
+        int ex;
+        (void)frexpf(amax, &ex);  // amax = f * 2^ex, f in [0.5, 1)
+        int se = ex - 23;         // |x| / 2^se < 2^23 ...
+        if (se < -126) se = -126;
+        if (rintf(amax * ldexpf(1.0f, -se)) > DIG3_MAX) se += 1;  // ... but three signed bytes stop at 127 * 65793
+        s = ldexpf(1.0f, se);
+        inv = ldexpf(1.0f, -se);
+    }
+}
+// Byte p of the result is digit p: X + 0x808080 has the digits plus 128 as its bytes.
+__device__ __forceinline__ unsigned digits3(float x, float inv, bool finite) {
+    const int X = finite ? (int)fminf(fmaxf(rintf(x * inv), -DIG3_MAX), DIG3_MAX) : 0;
+    return ((unsigned)X + 0x808080u) ^ 0x808080u;
+}
+
+// One workgroup of T threads per row.  The row is read once into registers (up to 4 * T * MAXV floats), reduced to its
+// absmax, then rounded to i8 -- or, DIG3, to three digits -- and written as packed dwords.  Columns [cols, q_stride)
+// of the output row are zero-filled.  A row starts at any float: 128-bit loads need four-byte alignment only, and the
+// up to three columns past the last whole vector go one to a thread (rows of odd length took the two-pass form below:
+// 100 x 7359, 13.9 us against 5.0).
+template <int MAXV, int T, bool DIG3>
+__global__ __launch_bounds__(T) void quantize_rows_vec4_kernel(
     const float *__restrict__ a, size_t cols, int8_t *__restrict__ q, size_t q_stride,
-    float *__restrict__ row_scales) {
-    __shared__ float red[4];
+    float *__restrict__ row_scales, size_t plane_bytes) {
+    __shared__ float red[T / 64];
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
     const size_t row = blockIdx.x;
-    const float4 *ar = reinterpret_cast<const float4 *>(a + row * cols);
-    const int nvec = (int)(cols >> 2);
+    const float *ar = a + row * cols;
+    const int nvec = (int)(cols >> 2), tail = (int)(cols & 3);
     // Every load is issued before anything waits: vectors past the end of the row re-read
     // the last one (no branch between the loads) and are left out of the maximum.
-    float4 v[MAXV];
+    f4u v[MAXV];
 #pragma unroll
     for (int i = 0; i < MAXV; ++i) {
-        const int idx = threadIdx.x + i * QA_THREADS;
-        typedef float f4v __attribute__((ext_vector_type(4)));
+        const int idx = threadIdx.x + i * T;
         // (a plain load: the activations of a layer are read by several products in a row and
         // are usually still in the Infinity Cache; a non-temporal load would fetch them from HBM
         // every time)
-        const f4v t = *(reinterpret_cast<const f4v *>(ar) + (idx < nvec ? idx : nvec - 1));
-        v[i] = make_float4(t.x, t.y, t.z, t.w);
+        v[i] = *reinterpret_cast<const f4u *>(ar + 4 * (idx < nvec ? idx : nvec - 1));
     }
-    float amax = 0.0f;
+    const float tv = ar[(int)threadIdx.x < tail ? 4 * nvec + threadIdx.x : 0];
+    auto mag = [](float x) { return DIG3 && x != x ? __uint_as_float(0x7F800000u) : fabsf(x); };  // (the i8 rows' maximum drops a NaN)
+    float amax = (int)threadIdx.x < tail ? fmaxf(0.0f, mag(tv)) : 0.0f;
 #pragma unroll
     for (int i = 0; i < MAXV; ++i) {
-        const int idx = threadIdx.x + i * QA_THREADS;
-        const float m4 = fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w)));
+        const int idx = threadIdx.x + i * T;
+        const float m4 = fmaxf(fmaxf(mag(v[i].x), mag(v[i].y)), fmaxf(mag(v[i].z), mag(v[i].w)));
         amax = fmaxf(amax, idx < nvec ? m4 : 0.0f);
     }
-    amax = block_max_256(amax, red);
-    const float scale = (amax == 0.0f) ? 1.0f : amax / 127.0f;
-    const float inv_scale = 1.0f / scale;
-    if (threadIdx.x == 0) row_scales[row] = scale;
-    int *qr = reinterpret_cast<int *>(q + row * q_stride);
+    amax = wave_max(amax);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+    __syncthreads();
+    amax = red[0];
 #pragma unroll
-    for (int i = 0; i < MAXV; ++i) {
-        const int idx = threadIdx.x + i * QA_THREADS;
-        if (idx < nvec) {
-            const int b0 = quant_to_i8(v[i].x * inv_scale) & 0xFF;
-            const int b1 = quant_to_i8(v[i].y * inv_scale) & 0xFF;
-            const int b2 = quant_to_i8(v[i].z * inv_scale) & 0xFF;
-            const int b3 = quant_to_i8(v[i].w * inv_scale) & 0xFF;
-            qr[idx] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
-        }
-    }
+    for (int w = 1; w < T / 64; ++w) amax = fmaxf(amax, red[w]);
     const int npad = (int)(q_stride >> 2);
-    for (int idx = nvec + threadIdx.x; idx < npad; idx += QA_THREADS) qr[idx] = 0;
+    int8_t *qr = q + row * q_stride;
+    if constexpr (DIG3) {
+        const bool finite = amax <= 3.4028234663852886e38f;
+        float s, inv;
+        digits3_scale(amax, finite, s, inv);
+        if (threadIdx.x == 0) row_scales[row] = s;
+        auto put = [&](int idx, const unsigned (&d)[4]) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                reinterpret_cast<unsigned *>(qr + p * plane_bytes)[idx] = (d[0] >> (8 * p) & 255u) | (d[1] >> (8 * p) & 255u) << 8 |
+                                                                          (d[2] >> (8 * p) & 255u) << 16 | (d[3] >> (8 * p) & 255u) << 24;
+        };
+#pragma unroll
+        for (int i = 0; i < MAXV; ++i) {
+            const int idx = threadIdx.x + i * T;
+            if (idx < nvec) put(idx, {digits3(v[i].x, inv, finite), digits3(v[i].y, inv, finite), digits3(v[i].z, inv, finite), digits3(v[i].w, inv, finite)});
+        }
+        if (tail && threadIdx.x < 4) {
+            const unsigned d = (int)threadIdx.x < tail ? digits3(tv, inv, finite) : 0u;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) qr[p * plane_bytes + 4 * nvec + threadIdx.x] = (int8_t)(d >> (8 * p));
+        }
+        for (int idx = nvec + (tail != 0) + threadIdx.x; idx < npad; idx += T) put(idx, {0u, 0u, 0u, 0u});
+    } else {
+        const float scale = (amax == 0.0f) ? 1.0f : amax / 127.0f;
+        const float inv_scale = 1.0f / scale;
+        if (threadIdx.x == 0) row_scales[row] = scale;
+#pragma unroll
+        for (int i = 0; i < MAXV; ++i) {
+            const int idx = threadIdx.x + i * T;
+            if (idx < nvec) {
+                const int b0 = quant_to_i8(v[i].x * inv_scale) & 0xFF;
+                const int b1 = quant_to_i8(v[i].y * inv_scale) & 0xFF;
+                const int b2 = quant_to_i8(v[i].z * inv_scale) & 0xFF;
+                const int b3 = quant_to_i8(v[i].w * inv_scale) & 0xFF;
+                reinterpret_cast<int *>(qr)[idx] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
+            }
+        }
+        if (tail && threadIdx.x < 4) qr[4 * nvec + threadIdx.x] = (int8_t)((int)threadIdx.x < tail ? quant_to_i8(tv * inv_scale) : 0);
+        for (int idx = nvec + (tail != 0) + threadIdx.x; idx < npad; idx += T) reinterpret_cast<int *>(qr)[idx] = 0;
+    }
 }
 
 // Any shape: two passes over the row (the second one hits L2), scalar accesses.
@@ -89,11 +152,7 @@ __global__ __launch_bounds__(QA_THREADS) void quantize_rows_generic_kernel(
     for (size_t k = cols + threadIdx.x; k < q_stride; k += QA_THREADS) qr[k] = 0;
 }
 
-// ---- f32 rows as three signed byte digits ---------------------------------------------
-// x[k] ~= s * X[k], X = 65536 d2 + 256 d1 + d0 with signed byte digits, |X| <= 8355711, s a power of two:
-// 23 to 24 bits of fixed point per row, exact integer arithmetic on the matrix cores afterwards.
-// planes[p][row][k] (p = 0: d0 .. 2: d2), rows of q_stride bytes, pad columns zero.
-constexpr float DIG3_MAX = 8355711.0f;  // 127 * (65536 + 256 + 1)
+// Any shape: two passes, scalar accesses.
 __global__ __launch_bounds__(QA_THREADS) void rows_to_digits3_kernel(const float *__restrict__ a, size_t cols,
                                                                      int8_t *__restrict__ planes, size_t q_stride,
                                                                      size_t plane_bytes, float *__restrict__ row_scales) {
@@ -110,47 +169,16 @@ __global__ __launch_bounds__(QA_THREADS) void rows_to_digits3_kernel(const float
     amax = block_max_256(amax, red);
     bad = __syncthreads_or(bad);
     const bool finite = !bad && amax <= 3.4028234663852886e38f;
-    // power-of-two scale, so x -> X is exact whenever x has no bits below s
-    // (integers stay integers), and s * X is exact again on the way back
-    float s = 1.0f, inv = 1.0f;
-    if (!finite) {
-        s = __uint_as_float(0x7FC00000u);
-        inv = 0.0f;
-    } else if (amax > 0.0f) {
-        int ex;
-        (void)frexpf(amax, &ex);  // amax = f * 2^ex, f in [0.5, 1)
-        int se = ex - 23;         // |x| / 2^se < 2^23 ...
-        if (se < -126) se = -126;
-        if (rintf(amax * ldexpf(1.0f, -se)) > DIG3_MAX) se += 1;  // ... but three signed bytes stop at 127 * 65793
-        s = ldexpf(1.0f, se);
-        inv = ldexpf(1.0f, -se);
-    }
+    float s, inv;
+    digits3_scale(amax, finite, s, inv);
     if (threadIdx.x == 0) row_scales[row] = s;
     int8_t *p0 = planes + row * q_stride;
     for (size_t k = threadIdx.x; k < q_stride; k += QA_THREADS) {
-        int X = 0;
-        if (k < cols && finite) {
-            const float t = fminf(fmaxf(rintf(ar[k] * inv), -DIG3_MAX), DIG3_MAX);
-            X = (int)t;
-        }
-        const int d0 = ((X + 128) & 255) - 128;
-        const int X1 = (X - d0) >> 8;
-        const int d1 = ((X1 + 128) & 255) - 128;
-        const int d2 = (X1 - d1) >> 8;
-        p0[k] = (int8_t)d0;
-        p0[plane_bytes + k] = (int8_t)d1;
-        p0[2 * plane_bytes + k] = (int8_t)d2;
+        const unsigned d = k < cols ? digits3(ar[k], inv, finite) : 0u;
+        p0[k] = (int8_t)d;
+        p0[plane_bytes + k] = (int8_t)(d >> 8);
+        p0[2 * plane_bytes + k] = (int8_t)(d >> 16);
     }
-}
-
-// out[m, n] = (65536 I2 + 256 I1 + I0) * s[m] * w_scale[n], the integer exactly in f64.
-__global__ void combine_digits3_kernel(const int32_t *__restrict__ acc, size_t plane_elems, const float *__restrict__ row_scales,
-                                       const float *__restrict__ w_scales, size_t m, size_t n, float *__restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m * n) return;
-    const size_t r = i / n, c = i - r * n;
-    const double v = 65536.0 * (double)acc[2 * plane_elems + i] + 256.0 * (double)acc[plane_elems + i] + (double)acc[i];
-    out[i] = (float)(v * (double)row_scales[r] * (double)w_scales[c]);
 }
 
 // ---- weight quantisation -----------------------------------------------------
@@ -294,25 +322,44 @@ pg_status qtensor_alloc(pg_ctx *ctx, size_t rows, size_t cols, pg_qtensor **out)
 
 }  // namespace
 
+// Rows to i8 or, DIG3, to three digit planes.  A workgroup of 1024 threads for rows past what 256 hold in registers, and
+// where there are at most two rows a CU and a row is longer than 4096: the launch is then the latency of one row, and
+// four threads share what one would do.
+template <bool DIG3>
+static pg_status launch_quantize_rows(pg_ctx *ctx, const char *name, const float *a, size_t rows, size_t cols, int8_t *q, size_t q_stride,
+                                      float *row_scales, size_t plane_bytes) {
+    const size_t nvec = cols / 4;
+    const dim3 grid((unsigned)rows);
+    auto go = [&](auto kern, int threads) {
+        return pg_launch(ctx, name, kern, grid, dim3(threads), 0, a, cols, q, q_stride, row_scales, plane_bytes);
+    };
+    if (nvec >= 1 && q_stride % 4 == 0 && (uintptr_t)q % 4 == 0 && plane_bytes % 4 == 0) {
+        if ((rows <= 2 * (size_t)ctx->num_cu && cols > 4096) || nvec > 16 * 256) {
+            if (nvec <= 1024) return go(quantize_rows_vec4_kernel<1, 1024, DIG3>, 1024);
+            if (nvec <= 2 * 1024) return go(quantize_rows_vec4_kernel<2, 1024, DIG3>, 1024);
+            if (nvec <= 4 * 1024) return go(quantize_rows_vec4_kernel<4, 1024, DIG3>, 1024);
+            if (nvec <= 8 * 1024) return go(quantize_rows_vec4_kernel<8, 1024, DIG3>, 1024);
+        } else {
+            if (nvec <= 1 * 256) return go(quantize_rows_vec4_kernel<1, 256, DIG3>, 256);
+            if (nvec <= 2 * 256) return go(quantize_rows_vec4_kernel<2, 256, DIG3>, 256);
+            if (nvec <= 4 * 256) return go(quantize_rows_vec4_kernel<4, 256, DIG3>, 256);
+            if (nvec <= 6 * 256) return go(quantize_rows_vec4_kernel<6, 256, DIG3>, 256);
+            if (nvec <= 8 * 256) return go(quantize_rows_vec4_kernel<8, 256, DIG3>, 256);
+            if (nvec <= 11 * 256) return go(quantize_rows_vec4_kernel<11, 256, DIG3>, 256);
+            if (nvec <= 14 * 256) return go(quantize_rows_vec4_kernel<14, 256, DIG3>, 256);
+            return go(quantize_rows_vec4_kernel<16, 256, DIG3>, 256);
+        }
+    }
+    if constexpr (DIG3)
+        return pg_launch(ctx, name, rows_to_digits3_kernel, grid, dim3(QA_THREADS), 0, a, cols, q, q_stride, plane_bytes, row_scales);
+    else
+        return pg_launch(ctx, name, quantize_rows_generic_kernel, grid, dim3(QA_THREADS), 0, a, cols, q, q_stride, row_scales);
+}
+
 pg_status pg_launch_quantize_activations(pg_ctx *ctx, const float *a, size_t rows, size_t cols,
                                          int8_t *q, size_t q_stride, float *row_scales) {
     if (rows == 0) return PG_OK;
-    const bool vec_ok = (cols % 4 == 0) && (q_stride % 4 == 0) &&
-                        ((uintptr_t)a % 16 == 0) && ((uintptr_t)q % 4 == 0) && cols > 0;
-    const size_t nvec = cols / 4;
-    const dim3 grid((unsigned)rows);
-#define PG_QROWS(V)                                                                                      \
-    else if (vec_ok && nvec <= (V) * QA_THREADS)                                                         \
-        PG_TRY(pg_launch(ctx, "quantize_rows", quantize_rows_vec4_kernel<V>, grid, dim3(QA_THREADS), 0, a, cols, q, \
-                         q_stride, row_scales));
-    if (cols == 0) PG_TRY(pg_launch(ctx, "quantize_rows", quantize_rows_generic_kernel, grid, dim3(QA_THREADS), 0, a, cols, q,
-                                    q_stride, row_scales));
-    PG_QROWS(2) PG_QROWS(4) PG_QROWS(6) PG_QROWS(8) PG_QROWS(11) PG_QROWS(14) PG_QROWS(16)
-#undef PG_QROWS
-    else
-        PG_TRY(pg_launch(ctx, "quantize_rows", quantize_rows_generic_kernel, grid, dim3(QA_THREADS), 0, a, cols, q,
-                         q_stride, row_scales));
-    return pg_launch_check("quantize_rows");
+    return launch_quantize_rows<false>(ctx, "quantize_rows", a, rows, cols, q, q_stride, row_scales, 0);
 }
 
 PG_API pg_status pg_quantize_activations_dev(pg_ctx *ctx, const float *a_dev, size_t rows,
@@ -703,34 +750,22 @@ PG_API pg_status pg_matmul_dequant_i8_dev(pg_ctx *ctx, const float *a_dev, size_
     // a digit plane holds -128 .. 127 (the carry-free split yields -128), a weight -127 .. 127: 128 * 127 * k < 2^31
     PG_CHECK_ARG(k <= 132104, "pg_matmul_dequant_i8: k = %zu would overflow the i32 digit sums", k);
     const size_t m_pad = pg_round_up(m, PG_MPAD), n = w->cols;
-    // With enough rows the two low digit planes run as ONE product over the planes stacked row-wise (they lie
-    // back to back in the scratch, each m_pad rows; the accumulator planes are then m_pad rows apart) and
-    // the third plane's product finishes the sum in its epilogue.
-    const bool stacked = m >= 192;
-    const size_t plane_bytes = m_pad * w->k_pad, plane_elems = (stacked ? m_pad : m) * n;
+    // One launch over the three digit planes, or, where 256x256 tiles fill the part (and under a tile override): the two
+    // low planes as ONE product over the planes stacked row-wise (they lie back to back in the scratch, each m_pad rows;
+    // the accumulator planes are then m_pad rows apart), and the third plane's product finishes the sum in its epilogue.
+    const bool one = pg_gemm_w8a32_takes(ctx, w, m);
+    const size_t plane_bytes = m_pad * w->k_pad, plane_elems = m_pad * n;
     // (the product's prologue reads a scale per stacked row, whether or not it writes f32: three planes' worth)
     const size_t sz_planes = pg_round_up(3 * plane_bytes, 256), sz_scales = pg_round_up(3 * m_pad * sizeof(float), 256);
     void *ws = nullptr;
-    PG_TRY(pg_workspace(ctx, sz_planes + sz_scales + 3 * plane_elems * sizeof(int32_t), &ws));
+    PG_TRY(pg_workspace(ctx, sz_planes + sz_scales + (one ? 0 : 2 * plane_elems * sizeof(int32_t)), &ws));
     int8_t *planes = static_cast<int8_t *>(ws);
     float *row_scales = reinterpret_cast<float *>(planes + sz_planes);
     int32_t *acc = reinterpret_cast<int32_t *>(planes + sz_planes + sz_scales);
-    PG_TRY(pg_launch(ctx, "rows_to_digits3", rows_to_digits3_kernel, dim3((unsigned)m), dim3(QA_THREADS), 0, a_dev, k, planes,
-                     w->k_pad, plane_bytes, row_scales));
-    if (stacked) {
-        // the two low planes as one product, then the plane of weight 65536, whose epilogue joins the three
-        // accumulators and scales them: no third accumulator plane and no combining launch
-        PG_TRY(pg_launch_gemm_w8a8(ctx, planes, w->k_pad, row_scales, w, m_pad + m, nullptr, acc));
-        return pg_launch_gemm_w8a8_combine(ctx, planes + 2 * plane_bytes, w->k_pad, row_scales, w, m, out_dev, acc, plane_elems);
-    }
-    for (int p = 0; p < 3; ++p) {
-        if (m <= PG_GEMV_MAX_M)
-            PG_TRY(pg_launch_gemv_w8a8(ctx, planes + p * plane_bytes, w->k_pad, row_scales, w, m, nullptr, acc + p * plane_elems));
-        else
-            PG_TRY(pg_launch_gemm_w8a8(ctx, planes + p * plane_bytes, w->k_pad, row_scales, w, m, nullptr, acc + p * plane_elems));
-    }
-    return pg_launch(ctx, "combine_digits3", combine_digits3_kernel, dim3(grid_for(plane_elems, 256)), dim3(256), 0, acc, plane_elems,
-                     row_scales, w->scales, m, n, out_dev);
+    PG_TRY(launch_quantize_rows<true>(ctx, "rows_to_digits3", a_dev, m, k, planes, w->k_pad, row_scales, plane_bytes));
+    if (one) return pg_launch_gemm_w8a32(ctx, planes, plane_bytes, row_scales, w, m, out_dev);
+    PG_TRY(pg_launch_gemm_w8a8(ctx, planes, w->k_pad, row_scales, w, m_pad + m, nullptr, acc));
+    return pg_launch_gemm_w8a8_combine(ctx, planes + 2 * plane_bytes, w->k_pad, row_scales, w, m, out_dev, acc, plane_elems);
 }
 
 PG_API pg_status pg_matmul_dequant_i8(pg_ctx *ctx, const float *a, size_t m, size_t k, const pg_qtensor *w, float *out) {

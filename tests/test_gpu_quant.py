@@ -553,3 +553,55 @@ def test_host_arrays_cross_whole(ctx, m, k, n):
         want = do.to_host(np.float32)
         got = quant.matmul_quantized(a, m, k, qt, ctx)
         assert (got.view(np.uint32) == want.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (2, 128, 16), (16, 4096, 1000), (16, 640, 33), (17, 1000, 250), (32, 4096, 600),     # the few-row kernel: three and six tiles of planes
+    (33, 128, 64), (64, 700, 65), (65, 4000, 300), (197, 1024, 515), (129, 256, 4097),   # 64x64 tiles, ragged
+    (1030, 384, 3600), (1100, 130, 3333),                                                # 128x128 tiles, ragged
+])
+def test_matmul_dequant_i8_one_launch(ctx, orc, m, k, n):
+    """W8A32 over three digit planes in one launch at the edges of its kernels' tiles: exact small integers in, exact
+    integers out, and the float64 product as the bar for random data."""
+    from peregrine_amd import quant
+    say(f"matmul_dequant_i8 one launch m={m} k={k} n={n}")
+    ai = (np.arange(m * k, dtype=np.float32) % 9 - 4).reshape(m, k)
+    qi = (np.arange(k * n).reshape(k, n) % 13 - 6).astype(np.int8)
+    qt = quant.QuantizedTensor(qi.reshape(-1), None, np.ones(n, np.float32), k, n)
+    got = quant.matmul_dequant_i8(ai, m, k, qt, ctx).reshape(m, n)
+    assert (got == ai @ qi.astype(np.float32)).all(), "integer inputs: the product is not exact"
+    qt.free_gpu()
+    a = orc.rng_normal(41 + m, m * k)
+    a.reshape(m, k)[:, :: max(1, k // 37)] *= 20
+    q, q_t, s = orc.quantize_weights(orc.rng_normal(42 + n, k * n, 0.0, 0.02), k, n)
+    qt = quant.QuantizedTensor(q, q_t, s, k, n)
+    got = quant.matmul_dequant_i8(a, m, k, qt, ctx).reshape(m, n)
+    exact = a.reshape(m, k).astype(np.float64) @ orc.dequantize(q, s, k, n).reshape(k, n).astype(np.float64)
+    for r in range(m):
+        H.assert_close_rel(got[r], exact[r], 1e-5, f"row {r} vs exact")
+    qt.free_gpu()
+
+
+@pytest.mark.parametrize("rows,cols", [(3, 4), (2, 5), (5, 1023), (4, 1025), (6, 4098), (2, 4099), (700, 4097),
+                                       (2, 16381), (600, 16389), (1, 32767), (1, 32772), (3, 3)])
+def test_row_kernels_on_rows_of_any_length(ctx, orc, rows, cols):
+    """The row kernels at the edges of their workgroups (256 and 1024 threads) and register counts, with one to three
+    columns past the last whole vector: int8 rows bit for bit through a product (padded rows), and the digit rows of
+    W8A32 through exact integers."""
+    from peregrine_amd import quant
+    say(f"row kernels rows={rows} cols={cols}")
+    n = 3
+    a = orc.rng_normal(51 + cols, rows * cols).reshape(rows, cols)
+    a[-1, -1] = 40.0
+    q, q_t, s = orc.quantize_weights(orc.rng_normal(52 + cols, cols * n, 0.0, 0.02), cols, n)
+    qt = quant.QuantizedTensor(q, q_t, s, cols, n)
+    got = quant.matmul_quantized(a, rows, cols, qt, ctx)
+    want, _ = orc.matmul_quantized(a, rows, cols, q_t, s, n)
+    assert (bits(got) == bits(want)).all()
+    ai = (np.arange(rows * cols, dtype=np.float32) % 9 - 4).reshape(rows, cols)
+    qi = (np.arange(cols * n).reshape(cols, n) % 13 - 6).astype(np.int8)
+    qt_int = quant.QuantizedTensor(qi.reshape(-1), None, np.ones(n, np.float32), cols, n)
+    got = quant.matmul_dequant_i8(ai, rows, cols, qt_int, ctx).reshape(rows, n)
+    assert (got == ai.astype(np.int64) @ qi.astype(np.int64)).all()
+    qt.free_gpu()
+    qt_int.free_gpu()
