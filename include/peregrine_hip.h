@@ -597,7 +597,7 @@ pg_status pg_gemm_w8a8_force_tile(pg_ctx *ctx, int tile);
  * automatic.  Every shape gives the same bits. */
 pg_status pg_gemv_w8a8_force_shape(pg_ctx *ctx, int wavefronts, int rows_per_wavefront);
 /* The many-row Q4_0 / Q8_0 product has two matrix-core routes: the int8 block product with 16-bit fixed-point activations
- * per block, and, from about a hundred rows on where the launch fills the part, f16 tiles with the weights unpacked
+ * per block, and, from 65 rows on where it is estimated to be the faster one, f16 tiles with the weights unpacked
  * in registers and the activations as two f16 planes per row.  mode 0 = the dispatcher chooses, 1 = the f16 route
  * wherever it can run (Q4_0 or Q8_0, K a multiple of 64, at least two rows), 2 = never.  Both keep the weights exact; they
  * round the activations differently (2^-22 of the row's largest value against 2^-16 of the block's). */

@@ -13,18 +13,23 @@
 // FMA per output and block where the int8 block product (pg_gguf_mm.hip) needs four
 // instructions, which is what bounds that kernel at many rows.
 //
-// Workgroup = 8 wavefronts over NWM x NWN tiles of 128 rows x 64 weight rows: 256 x 256
-// (2 x 4) or 128 x 512 (1 x 8).  K runs in stages of two blocks through two LDS stages filled
-// by direct global->LDS loads: the two activation planes [rows][128 B] (16-byte chunks XOR
-// swizzled as in the W8A8 kernel), the weights' packed bytes [weight rows][2 blocks] and their
-// f16 scales.  One barrier per stage.  Inside a stage the wavefront walks 16 steps (2 blocks x
-// 8 row tiles); at every step it issues 8 MFMAs (4 weight tiles x hi, lo) into one of two sets
-// of T registers, and between them the 16 FMAs that fold the previous step's T into the
-// accumulators, so neither unit waits for the other.  The second block's weights are unpacked
-// under the first block's MFMAs.
+// Workgroup = 8 wavefronts side by side over 16 MT rows x 512 weight rows (64 each), MT = 4 .. 8.  K runs in stages of
+// two blocks through two LDS stages filled by direct global->LDS loads: the two activation planes [rows][128 B]
+// (16-byte chunks XOR swizzled as in the W8A8 kernel), the weights' packed bytes [weight rows][2 blocks] and their f16
+// scales.  One barrier per stage.  Inside a stage the wavefront walks 2 MT steps (2 blocks x MT row tiles); at every
+// step it issues one of the next stage's loads, 8 MFMAs (4 weight tiles x hi, lo) into one of two sets of T registers,
+// and between them the 16 FMAs that fold the previous step's T into the accumulators, so neither unit waits for the
+// other.  The second block's weights are unpacked under the first block's MFMAs.
 //
-// A K too short to fill the part with tiles is cut into chunks (blockIdx.y); the chunks' planes
-// are summed in a fixed order by pg_launch_sum_parts.
+// What bounds it: 1024 rows of 4096 -> 28672 (Q8_0) are 481 G f16 operations over the two planes and take 425 to 495 us
+// (short and sustained runs), 0.97 to 1.13 PFLOP/s where a library's dense bf16 product holds 1.34: the chip's power limit
+// first, the instruction mix of the step after it.  The tile's rows follow the launch (hmm_plan_for): 777 rows are 9 tiles
+// of 96 (504 workgroups, two full rounds of the CUs: 366 us) and not 7 of 128 (392: 15 % of the rows padding, the second
+// round half empty: 478 us).  Spreading the loads over the steps instead of issuing them together took 9 % (MT = 8) to
+// 20 % (MT = 4) off a stage, asking for all rows' scales before the first store 8 to 25 us off every launch.
+//
+// A K too short to fill the part with tiles is cut into chunks; the chunks' planes are summed in a fixed order by
+// pg_launch_sum_parts.
 #include <limits.h>
 #include "pg_internal.h"
 #include "pg_f16_planes.h"
@@ -111,29 +116,32 @@ struct hmm_group {
     int panel0[PG_HMM_MAX_GROUP];      // first panel of tensor g (INT_MAX: unused)
 };
 
-constexpr int BKB = 2;  // blocks per stage
+constexpr int BKB = 2;       // blocks per stage
+constexpr int HMM_BN = 512;  // weight rows per tile: 64 per wavefront
 
 // QT = 8 (Q8_0): a weight row is two streams of 16-byte half blocks (elements 0 .. 15 and 16 .. 31 of every block,
 // as the upload splits them); a stage holds 64 bytes a row, chunk 2 block + half at position chunk ^ ((row >> 2) & 3),
 // so that the 64-bit fragment reads of 16 rows spread over all banks.
-template <int QT, int NWM, int NWN>
+template <int QT, int MT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict__ xl, const float *__restrict__ inv,
-                        const hmm_group grp, int M, int nb, int tiles_m, int ntiles, int kt_per_split) {
-    static_assert(NWM * NWN == 8, "eight wavefronts");
-    constexpr int BM = 128 * NWM, BN = 64 * NWN;
+                        const hmm_group grp, int M, int nb, int tiles_m, int ntiles, int ksplit, int kt_per_split) {
+    static_assert(MT >= 4 && MT <= 8, "4 to 8 row tiles a wavefront");
+    constexpr int BM = 16 * MT, BN = HMM_BN;
     constexpr int WROW = QT == 8 ? 64 : 32;                   // bytes of packed weights per row and stage
-    constexpr int LX = BM / 64, LW = (BN * WROW / 1024 + 7) / 8;  // wave-loads per wavefront and stage: one plane, weights
+    constexpr int LX = (BM / 8 + 7) / 8, LW = (BN * WROW / 1024 + 7) / 8;  // most wave-loads of a wavefront and stage: one plane, weights
     constexpr int XP = BM * 128;                              // one activation plane of a stage
     constexpr int OFF_XL = XP, OFF_W = 2 * XP, OFF_D = OFF_W + 8 * LW * 1024, STAGE = OFF_D + 8 * 256;
-    constexpr int LPS = 2 * LX + LW + 1;
+    constexpr int LPS = LW + 1 + 2 * LX, FULL = BM / 8 - 8 * (LX - 1);  // wavefronts from FULL on make one load of a plane less
+    static_assert(LPS <= 2 * MT, "a load a step");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 
-    // Workgroups are dealt round-robin to the 8 XCDs; each XCD gets a contiguous run of tiles
-    // (row tiles fastest), so the tiles that share an L2 share weight panels.
-    const int chunk = (ntiles + 7) / 8;
-    const int t = (blockIdx.x % 8) * chunk + blockIdx.x / 8;
-    if (t >= ntiles) return;
+    // Workgroups are dealt round-robin to the 8 XCDs; each XCD gets a contiguous run of the launch's tiles (row tiles
+    // fastest, K chunks slowest), so the tiles that share an L2 share weight panels; the runs differ by one at most.
+    const int total = ntiles * ksplit, xcd = blockIdx.x % 8;
+    const int tk = (int)((long long)total * xcd / 8) + blockIdx.x / 8;
+    if (tk >= (int)((long long)total * (xcd + 1) / 8)) return;
+    const int split = tk / ntiles, t = tk % ntiles;
     const int np = t / tiles_m;
     int g = 0;
 #pragma unroll
@@ -143,13 +151,12 @@ void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict
     const int N = grp.n[g];
     const int m0 = (t % tiles_m) * BM, n0 = (np - grp.panel0[g]) * BN;
     const int K = nb * 32;
-    const int kt0 = blockIdx.y * kt_per_split;
+    const int kt0 = split * kt_per_split;
     const int KT = nb / BKB - kt0 < kt_per_split ? nb / BKB - kt0 : kt_per_split;
-    float *__restrict__ y = grp.out[g] + (size_t)blockIdx.y * grp.stride[g];
+    float *__restrict__ y = grp.out[g] + (size_t)split * grp.stride[g];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / NWN, wn = wave % NWN;
     const int l15 = lane & 15, q4 = lane >> 4;
 
     // ---- global -> LDS.  Activation planes: wave-load L covers rows 8L .. 8L+7 (lane -> row,
@@ -161,7 +168,7 @@ void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict
         const int lr = lane >> 3, pc = lane & 7;
 #pragma unroll
         for (int i = 0; i < LX; ++i) {
-            const int row = 8 * (wave + 8 * i) + lr;
+            const int row = 8 * (wave + 8 * i) + lr;  // (past the tile: never loaded)
             xsrc[i] = reinterpret_cast<const char *>(xh) + pg_hmm_plane_offset(pg_hmm_clamp_row(m0 + row, M), K, kt0, pc ^ swz128(row));
         }
     }
@@ -183,27 +190,28 @@ void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict
     }
     const char *dsrc;
     {
-        const int row = wn * 64 + 2 * (lane & 31);   // this wavefront's own 64 weight rows, two per lane
+        const int row = wave * 64 + 2 * (lane & 31);   // this wavefront's own 64 weight rows, two per lane
         dsrc = reinterpret_cast<const char *>(d) + pg_hmm_scale_offset(pg_hmm_scale_row(n0 + row, N), nb, kt0, lane >> 5);
     }
-    auto issue = [&](int stage, int kt) {   // kt: stage index within this workgroup's K chunk
+    // Load L of a stage's LPS: the weights, the scales, the high plane, the low plane.  kt: stage index within this workgroup's K chunk.
+    auto issue = [&](int stage, int kt, int L) {
         char *base = lds + stage * STAGE;
-#pragma unroll
-        for (int i = 0; i < LX; ++i)
-            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (size_t)kt * 128), (lptr_t)(base + (wave + 8 * i) * 1024), 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < LX; ++i)
-            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + lo_minus_hi + (size_t)kt * 128), (lptr_t)(base + OFF_XL + (wave + 8 * i) * 1024), 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < LW; ++i)
-            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (size_t)kt * 32), (lptr_t)(base + OFF_W + (wave + 8 * i) * 1024), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((gptr_t)(dsrc + (size_t)kt * 32), (lptr_t)(base + OFF_D + wave * 256), 4, 0, 0);
+        if (L < LW) {
+            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[L] + (size_t)kt * 32), (lptr_t)(base + OFF_W + (wave + 8 * L) * 1024), 16, 0, 0);
+        } else if (L == LW) {
+            __builtin_amdgcn_global_load_lds((gptr_t)(dsrc + (size_t)kt * 32), (lptr_t)(base + OFF_D + wave * 256), 4, 0, 0);
+        } else {
+            const int p = L - LW - 1, i = p % LX;
+            if (i + 1 < LX || FULL == 8 || wave < FULL)
+                __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (p < LX ? 0 : lo_minus_hi) + (size_t)kt * 128),
+                                                 (lptr_t)(base + (p < LX ? 0 : OFF_XL) + (wave + 8 * i) * 1024), 16, 0, 0);
+        }
     };
 
     // ---- fragment offsets: lane = (row l15, k group q4 of 8 elements)
     int a_off[2], w_off[2], d_off[2];
     {
-        const int ra = wm * 128 + l15, rb = wn * 64 + l15;
+        const int ra = l15, rb = wave * 64 + l15;
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             a_off[b] = ra * 128 + (((4 * b + q4) ^ swz128(ra)) * 16);                    // + 16 rows per row tile
@@ -213,19 +221,15 @@ void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict
         }
     }
 
-    v4f acc[8][4];
+    v4f acc[MT][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0, 0, 0, 0};
 
-    issue(0, 0);
-    if (KT > 1) {
-        issue(1, 1);
-        asm volatile("s_waitcnt vmcnt(%0)\n s_barrier" ::"n"(LPS) : "memory");
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)\n s_barrier" ::: "memory");
-    }
+#pragma unroll
+    for (int L = 0; L < LPS; ++L) issue(0, 0, L);
+    asm volatile("s_waitcnt vmcnt(0)\n s_barrier" ::: "memory");
     for (int kt = 0; kt < KT; ++kt) {
         const int s = kt & 1;
         const char *base = lds + s * STAGE;
@@ -258,10 +262,13 @@ void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict
         ah[0] = *reinterpret_cast<const v8h *>(base + a_off[0]);
         al[0] = *reinterpret_cast<const v8h *>(base + OFF_XL + a_off[0]);
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int b = q >> 3, cur = q & 1, nxt = cur ^ 1;
-            if (q + 1 < 16) {
-                const int b1 = (q + 1) >> 3, i1 = (q + 1) & 7;
+        for (int q = 0; q < 2 * MT; ++q) {
+            const int b = q / MT, cur = q & 1, nxt = cur ^ 1;
+            // The next stage's loads, one a step: all at the stage's start, they held back the eight wavefronts' first
+            // steps while the address unit took them in.
+            if (q < LPS && kt + 1 < KT) issue(s ^ 1, kt + 1, q);
+            if (q + 1 < 2 * MT) {
+                const int b1 = (q + 1) / MT, i1 = (q + 1) % MT;
                 ah[nxt] = *reinterpret_cast<const v8h *>(base + a_off[b1] + i1 * 16 * 128);
                 al[nxt] = *reinterpret_cast<const v8h *>(base + OFF_XL + a_off[b1] + i1 * 16 * 128);
             }
@@ -272,17 +279,21 @@ void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict
                     draw[j] = *reinterpret_cast<const _Float16 *>(base + d_off[1] + j * 32);
                 }
             }
-            if (q >= 2 && q < 6) {
-                fb[1][q - 2] = unpack(wraw[q - 2]);
-                df[1][q - 2] = (float)draw[q - 2];
-                asm volatile("" : "+v"(df[1][q - 2]));
+            constexpr int UPS = MT >= 6 ? 1 : 2, UP0 = MT >= 6 ? 2 : 1;  // weight tiles of the second block unpacked a step, from step UP0 on
+            if (q >= UP0 && q < UP0 + 4 / UPS) {
+#pragma unroll
+                for (int u = (q - UP0) * UPS; u < (q - UP0 + 1) * UPS; ++u) {
+                    fb[1][u] = unpack(wraw[u]);
+                    df[1][u] = (float)draw[u];
+                    asm volatile("" : "+v"(df[1][u]));
+                }
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) T[cur][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[cur], fb[b][j], (v4f){0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
             for (int j = 0; j < 4; ++j) T[cur][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[cur], fb[b][j], T[cur][j], 0, 0, 0);
             if (q > 0) {
-                const int bp = (q - 1) >> 3, ip = (q - 1) & 7;
+                const int bp = (q - 1) / MT, ip = (q - 1) % MT;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -300,36 +311,45 @@ void gguf_hmm_kernel(const _Float16 *__restrict__ xh, const _Float16 *__restrict
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[7][j][r] = __builtin_fmaf(T[1][j][r], df[1][j], acc[7][j][r]);
-            asm volatile("" : "+v"(acc[7][j]));
+            for (int r = 0; r < 4; ++r) acc[MT - 1][j][r] = __builtin_fmaf(T[1][j][r], df[1][j], acc[MT - 1][j][r]);
+            asm volatile("" : "+v"(acc[MT - 1][j]));
         }
         if (kt + 1 < KT) {
             // Only the next stage's fills are in flight: wait for mine and meet the others, who have then
             // also read this stage to the end; this stage takes the stage after next.
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n s_barrier" ::: "memory");
-            if (kt + 2 < KT) issue(s, kt + 2);
         }
     }
 
-    // ---- epilogue: register r of tile (i, j) is row 16 i + 4 q4 + r, weight row 16 j + l15
+    // ---- epilogue: register r of tile (i, j) is row 16 i + 4 q4 + r, weight row 16 j + l15.  All rows' scales are
+    // asked for before the first store: one after the other their latencies were 20 to 30 us of every tile.
+    float2 sc[MT][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int m = m0 + wm * 128 + 16 * i + 4 * q4 + r;
+            const int m = m0 + 16 * i + 4 * q4 + r;
+            sc[i][r] = reinterpret_cast<const float2 *>(inv)[m < M ? m : M - 1];
+        }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(sc[i][r].x), "+v"(sc[i][r].y));
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + 16 * i + 4 * q4 + r;
             if (m >= M) continue;
-            const float s1 = inv[2 * m], s2 = inv[2 * m + 1];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int n = n0 + wn * 64 + 16 * j + l15;
-                if (n < N) __builtin_nontemporal_store(acc[i][j][r] * s1 * s2, y + (size_t)m * N + n);
+                const int n = n0 + wave * 64 + 16 * j + l15;
+                if (n < N) __builtin_nontemporal_store(acc[i][j][r] * sc[i][r].x * sc[i][r].y, y + (size_t)m * N + n);
             }
         }
 }
 
-template <int QT, int NWM, int NWN> constexpr size_t hmm_lds_bytes() {
-    return 2 * (size_t)(2 * 128 * NWM * 128 + 8 * ((64 * NWN * (QT == 8 ? 64 : 32) / 1024 + 7) / 8) * 1024 + 8 * 256);
-}
+template <int QT, int MT> constexpr size_t hmm_lds_bytes() { return 2 * (size_t)(2 * 16 * MT * 128 + HMM_BN * (QT == 8 ? 64 : 32) + 8 * 256); }
 
 }  // namespace
 
@@ -357,34 +377,47 @@ pg_status pg_launch_rows_to_f16_planes(pg_ctx *ctx, const float *x_dev, size_t r
                      (_Float16 *)p.hi, (_Float16 *)p.lo, p.inv);
 }
 
-// Which products this kernel takes, and in how many K chunks.  `n_total` = weight rows of all the tensors of the
-// launch.  A tile holds 256 x 256 outputs (128 x 512 up to 128 rows); a workgroup needs the CU to itself, so a
-// launch wants about one workgroup per CU: short of that, K is cut into up to 8 chunks of at least 512.
+// The row tiles of a wavefront (mt) and the K chunks (ks) of a product of m rows with n_total weight rows (all the
+// tensors of the launch), the pair of least estimated time `us`; ks_fixed > 0: the best mt for that many chunks.
+// A launch takes as many rounds of the CUs as its fullest XCD has (one workgroup per CU), each round its stages: 0.86 us
+// and 0.25 us per row tile; 3 us and 0.48 us per row tile go to the first loads and the results.  The conversion of
+// the rows (1.2 us per million values) and the pass over the chunks' planes (1.5 us per million values of each and of
+// their sum) come on top.  Fitted to 13 shapes (1024 to 14336 -> 1000 to 28672) at 48 to 1024 rows and every (mt, ks): 5 %
+// mean error, and the pair it picks takes 1 % longer than the best on average.
+struct hmm_plan { int mt, ks; double us; };
+static hmm_plan hmm_plan_for(const pg_ctx *ctx, size_t m, size_t n_total, size_t k_in, int ks_fixed) {
+    hmm_plan best = {8, 1, 1e300};
+    const size_t stages = k_in / 64, cus_per_xcd = ctx->num_cu >= 8 ? (size_t)ctx->num_cu / 8 : 1;
+    for (size_t ks = ks_fixed > 0 ? (size_t)ks_fixed : 1; ks <= (ks_fixed > 0 ? (size_t)ks_fixed : 8); ++ks) {
+        const size_t per = (stages + ks - 1) / ks;
+        if (ks_fixed <= 0 && ks > 1 && ((stages + per - 1) / per != ks || per < 8)) continue;  // an empty chunk, or one too short
+        for (int mt = 8; mt >= 4; --mt) {
+            const size_t bm = 16 * (size_t)mt, tiles = ((m + bm - 1) / bm) * ((n_total + HMM_BN - 1) / HMM_BN) * ks;
+            const size_t rounds = ((tiles + 7) / 8 + cus_per_xcd - 1) / cus_per_xcd;
+            double us = (double)rounds * ((double)per * (0.86 + 0.25 * mt) + 3.0 + 0.48 * mt) + 4.9 + 1.2e-6 * (double)m * (double)k_in;
+            if (ks > 1) us += 0.8 + 1.5e-6 * (double)(ks + 1) * (double)m * (double)n_total;
+            if (us < best.us) best = {mt, (int)ks, us};
+        }
+    }
+    return best;
+}
+
+// Which products this kernel takes, and in how many K chunks: those it is estimated to do in 0.93 of the int8 block
+// product's time or less (nearer than that the two estimates do not tell them apart).  That one takes about 12 us and 5
+// (short K) to 6.5 (K of 8192 and more) us per G multiply-adds.  f16 route : int8 route, us: 4096 -> 28672 at 97 / 400 / 1024
+// rows 80 : 87 / 194 : 325 / 432 : 698; 4096 -> 4096 at 256 / 400 / 777 43 : 40 / 55 : 57 / 78 : 86; 14336 -> 4096 at
+// 97 / 256 / 777 71 : 57 / 91 : 105 / 211 : 343; 1024 -> 5632 at 400 / 1024 37 : 27 / 44 : 43.  Up to 64 rows are two full
+// row tiles of the int8 product (4096 -> 28672 at 64: 64 : 59).
 bool pg_gguf_hmm_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_total, size_t k_in, int *ks_out) {
     if (ctx->hmm_mode == 2) return false;
     if ((ggml_type != PG_GGML_Q4_0 && ggml_type != PG_GGML_Q8_0) || k_in % 64 != 0 || k_in < 256 || k_in > ((size_t)1 << 24) || n_total < 2 || n_total > ((size_t)1 << 24) ||
         m < 2 || m > ((size_t)1 << 20))
         return false;
-    const bool wide = m <= 128 || ggml_type == PG_GGML_Q8_0;  // (Q8_0: a stage of 256 x 256 does not fit the LDS twice)
-    const size_t bm = wide ? 128 : 256, bn = wide ? 512 : 256;
-    const size_t tiles = ((m + bm - 1) / bm) * ((n_total + bn - 1) / bn);
-    size_t ks = (size_t)ctx->num_cu / tiles;
-    const size_t stages = k_in / 64;
-    while (ks > 1 && stages / ks < 8) --ks;
-    if (ks > 8) ks = 8;
-    if (ks < 1) ks = 1;
-    const size_t per = (stages + ks - 1) / ks;
-    ks = (stages + per - 1) / per;   // chunks of `per` stages: none is empty
-    if (ks_out) *ks_out = (int)ks;
-    if (ctx->hmm_mode == 1) return true;
-    // Measured against the int8 block product (us, f16 route : int8 route, [K] -> [N] at M rows): 4096 -> 14336 at
-    // 256 / 1024 / 4096 rows 97 : 105 / 241 : 329 / 981 : 1290; 14336 -> 4096 at 256 / 384 / 1024 126 : 101 /
-    // 144 : 175 / 268 : 345; 4096 -> 4096 at 512 / 1024 / 4096 74 : 59 / 105 : 106 / 281 : 389; 8192 -> 28672 at
-    // 64 / 96 / 1024 143 : 115 / 149 : 172 / 899 : 1326.  The f16 route wins from about 18 G multiply-adds on:
-    // below that its tiles leave CUs idle or its K chunks cost a pass over their planes.
-    // (Q8_0, always on 128 x 512 tiles: 4096 -> 14336 at 256 / 512 / 1024 rows 109 : 112 / 168 : 180 / 266 : 348, 14336 -> 4096 at
-    // 256 / 512 / 1024 143 : 105 / 166 : 188 / 287 : 351, 4096 -> 4096 at 1024 / 2048 111 : 110 / 186 : 202: from about 24 G.)
-    return m >= 96 && (double)m * (double)n_total * (double)k_in >= (ggml_type == PG_GGML_Q8_0 ? 2.4e10 : 1.8e10);
+    const double int8_us = 12.0 + 1e-9 * (double)m * (double)n_total * (double)k_in * (5.0 + 1.5 * (k_in < 8192 ? (double)k_in : 8192.0) / 8192.0);
+    if (ctx->hmm_mode != 1 && (m <= 64 || int8_us < 30.0)) return false;
+    const hmm_plan plan = hmm_plan_for(ctx, m, n_total, k_in, 0);
+    if (ks_out) *ks_out = plan.ks;
+    return ctx->hmm_mode == 1 || plan.us < 0.93 * int8_us;
 }
 
 size_t pg_gguf_hmm_part_floats(size_t m, size_t n_total, int ks) { return ks > 1 ? (size_t)ks * m * n_total : 0; }
@@ -403,8 +436,11 @@ pg_status pg_launch_gguf_hmm_group(pg_ctx *ctx, size_t k_in, const pg_gguf_tenso
         if (w[i]->k_in != k_in || kind(w[i]->ggml_type) != type) return pg_fail(PG_EINVAL, "gguf (f16 matrix cores): the tensors differ in K or type");
     if (k_in % 64 != 0 || planes.rows < m || planes.k != k_in) return pg_fail(PG_EINVAL, "gguf (f16 matrix cores): K = %zu, planes of %zu x %zu", k_in, planes.rows, planes.k);
     if (ks < 1 || (ks > 1 && !part && !keep_parts)) return pg_fail(PG_EINVAL, "gguf (f16 matrix cores): %d K chunks without a buffer for their planes", ks);
-    const bool q8 = type == PG_GGML_Q8_0, wide = m <= 128 || q8;   // 128 x 512 tiles
-    const size_t bm = wide ? 128 : 256, bn = wide ? 512 : 256;
+    const bool q8 = type == PG_GGML_Q8_0;
+    size_t n_total = 0;
+    for (int i = 0; i < count; ++i) n_total += w[i]->n_out;
+    const hmm_plan plan = hmm_plan_for(ctx, m, n_total, k_in, ks);
+    const size_t bm = 16 * (size_t)plan.mt, bn = HMM_BN;
     hmm_group grp;
     int panels = 0;
     size_t part_off = 0;
@@ -425,19 +461,22 @@ pg_status pg_launch_gguf_hmm_group(pg_ctx *ctx, size_t k_in, const pg_gguf_tenso
     const int stages = (int)(k_in / 64), kt_per = (stages + ks - 1) / ks;
     const int ks_real = (stages + kt_per - 1) / kt_per;
     if (ks_real != ks) return pg_fail(PG_EINVAL, "gguf (f16 matrix cores): %d K chunks of %d stages leave one empty", ks, kt_per);
-    const dim3 grid((unsigned)((ntiles + 7) / 8 * 8), (unsigned)ks_real);
+    const dim3 grid((unsigned)(((size_t)ntiles * ks + 7) / 8 * 8));
     const int nb = (int)(k_in / 32);
-#define PG_HMM_LAUNCH(QTT, NWMM, NWNN)                                                                                          \
-    do {                                                                                                                        \
-        auto kern = gguf_hmm_kernel<QTT, NWMM, NWNN>;                                                                           \
-        const size_t lds = hmm_lds_bytes<QTT, NWMM, NWNN>();                                                                    \
+#define PG_HMM_LAUNCH(QTT, MTT)                                                                                                 \
+    case MTT: {                                                                                                                 \
+        auto kern = gguf_hmm_kernel<QTT, MTT>;                                                                                  \
+        const size_t lds = hmm_lds_bytes<QTT, MTT>();                                                                           \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                             \
         PG_TRY(pg_launch(ctx, QTT == 8 ? "gguf_hmm_q8_0" : "gguf_hmm_q4_0", kern, grid, dim3(512), lds, (const _Float16 *)planes.hi, \
-                         (const _Float16 *)planes.lo, (const float *)planes.inv, grp, (int)m, nb, tiles_m, ntiles, kt_per));    \
-    } while (0)
-    if (q8) PG_HMM_LAUNCH(8, 1, 8);
-    else if (wide) PG_HMM_LAUNCH(4, 1, 8);
-    else PG_HMM_LAUNCH(4, 2, 4);
+                         (const _Float16 *)planes.lo, (const float *)planes.inv, grp, (int)m, nb, tiles_m, ntiles, ks, kt_per)); \
+        break;                                                                                                                  \
+    }
+#define PG_HMM_TILES(QTT)                                                                                                       \
+    switch (plan.mt) { PG_HMM_LAUNCH(QTT, 4) PG_HMM_LAUNCH(QTT, 5) PG_HMM_LAUNCH(QTT, 6) PG_HMM_LAUNCH(QTT, 7) PG_HMM_LAUNCH(QTT, 8) }
+    if (q8) PG_HMM_TILES(8)
+    else PG_HMM_TILES(4)
+#undef PG_HMM_TILES
 #undef PG_HMM_LAUNCH
     if (ks > 1 && !keep_parts) {
         size_t off = 0;

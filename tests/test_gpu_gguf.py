@@ -265,6 +265,29 @@ def test_gguf_matmul_f16_route_vs_oracle(ctx, orc, typ, n_out, k_in, m):
     gw.free()
 
 
+@pytest.mark.parametrize("typ", [2, 8])
+@pytest.mark.parametrize("m,row_tiles", [(441, 4), (513, 5), (561, 6), (673, 7), (785, 8)])
+def test_gguf_matmul_f16_route_every_tile_height(ctx, orc, typ, m, row_tiles):
+    """33 panels of weight rows, the last ragged, and just so many rows that the launch fits one round of the CUs with
+    `row_tiles` row tiles per wavefront and not with fewer: the rows at the edges of its tiles, and the last ones."""
+    from peregrine_amd import gguf, _ffi
+    n_out, k_in = 16461, 256
+    say(f"gguf_matmul f16 route type={typ} m={m} row_tiles={row_tiles}")
+    raw = (H.pack_q4_0 if typ == 2 else H.pack_q8_0)(orc.rng_normal(2900, n_out * k_in, 0.0, 0.02))
+    x = orc.rng_normal(217 + m, m * k_in)
+    gw = gguf.GgufWeight(raw, typ, n_out, k_in, ctx)
+    _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 1))
+    try:
+        got = gw.matmul(x, m).reshape(m, n_out)
+    finally:
+        _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 0))
+    bm = 16 * row_tiles
+    for r in (0, bm - 1, bm, 3 * bm + 17, m // bm * bm - 1, m - 1):
+        want = orc.gguf_matmul(x.reshape(m, k_in)[r], 1, raw, typ, n_out, k_in)
+        H.assert_close_rel(got[r], want, RTOL_F16_ROUTE, f"row {r}")
+    gw.free()
+
+
 def test_gguf_matmul_f16_route_prefill_size_is_the_dispatchers_choice(ctx, orc):
     """1024 rows over [4096] -> [14336] (a prefill's gate projection): the dispatcher takes the f16 route by itself;
     rows spot-checked against the oracle, and the int8 block route on the same input agrees within its own bar."""
