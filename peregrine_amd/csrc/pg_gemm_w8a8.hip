@@ -61,8 +61,7 @@ struct gemm_wgroup {
     // and the output is (65536 acc + 256 comb[comb_plane + i] + comb[i]) * a_scale * w_scale, the integer exact
     // and the scaling done in f64.
     const int32_t *comb;
-    long long comb_plane;
-    int a_plane;  // NP planes of activations: bytes from one to the next
+    long long comb_plane;  // (NP planes of activations: bytes from one of those to the next)
 };
 
 // NP = 3: the W8A32 product in one launch.  The activations are three digit planes (weights 1, 256, 65536); a stage holds
@@ -115,7 +114,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int row = RPL * (wave + NW * i) + lr;
-        a_goff[i] = (row % BM) * lda + row / BM * (NP > 1 ? grp.a_plane : 0) + 16 * (pc ^ swz<BK>(row));
+        a_goff[i] = (NP > 1 ? row % BM * lda + row / BM * (int)grp.comb_plane : row * lda) + 16 * (pc ^ swz<BK>(row));
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
@@ -395,8 +394,7 @@ pg_status launch_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const f
         if (used) panels += (int)((w[i]->cols + BN - 1) / BN);
     }
     grp.comb = comb;
-    grp.comb_plane = (long long)comb_plane;
-    grp.a_plane = (int)a_plane;
+    grp.comb_plane = (long long)(NP > 1 ? a_plane : comb_plane);
     const int ntiles = tiles_m * panels;
     const size_t lds = (size_t)NST * (NP * BM + BN) * BK + (BM + BN) * sizeof(float);
     auto kern = gemm_w8a8_kernel<BM, BN, BK, NST, NWM, NWN, OCC, false, COMB, NP>;
@@ -874,7 +872,6 @@ PG_API pg_status pg_probe_gemm_clock(pg_ctx *ctx, size_t m, size_t k, size_t n, 
     }
     grp.comb = nullptr;
     grp.comb_plane = 0;
-    grp.a_plane = 0;
     grp.w[0] = b.as<int8_t>(); grp.ws[0] = sc.as<float>(); grp.out[0] = out.as<float>(); grp.n[0] = (int)n; grp.panel0[0] = 0;
     const size_t lds = (size_t)NST * (BM + BN) * BK + (BM + BN) * sizeof(float);
     auto kern = gemm_w8a8_kernel<BM, BN, BK, NST, 2, 4, 2, true>;

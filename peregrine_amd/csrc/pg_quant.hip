@@ -53,8 +53,8 @@ __device__ __forceinline__ unsigned digits3(float x, float inv, bool finite) {
 // absmax, then rounded to i8 -- or, DIG3, to three digits -- and written as packed dwords.  Columns [cols, q_stride)
 // of the output row are zero-filled.  A row starts at any float: 128-bit loads need four-byte alignment only, and the
 // up to three columns past the last whole vector go one to a thread (rows of odd length took the two-pass form below:
-// 100 x 7359, 13.9 us against 5.0).
-template <int MAXV, int T, bool DIG3>
+// 100 x 7359, 13.9 us against 5.0; without TAIL the code for them is left out).
+template <int MAXV, int T, bool DIG3, bool TAIL>
 __global__ __launch_bounds__(T) void quantize_rows_vec4_kernel(
     const float *__restrict__ a, size_t cols, int8_t *__restrict__ q, size_t q_stride,
     float *__restrict__ row_scales, size_t plane_bytes) {
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(T) void quantize_rows_vec4_kernel(
     typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
     const size_t row = blockIdx.x;
     const float *ar = a + row * cols;
-    const int nvec = (int)(cols >> 2), tail = (int)(cols & 3);
+    const int nvec = (int)(cols >> 2), tail = TAIL ? (int)(cols & 3) : 0;
     // Every load is issued before anything waits: vectors past the end of the row re-read
     // the last one (no branch between the loads) and are left out of the maximum.
     f4u v[MAXV];
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(T) void quantize_rows_vec4_kernel(
         // every time)
         v[i] = *reinterpret_cast<const f4u *>(ar + 4 * (idx < nvec ? idx : nvec - 1));
     }
-    const float tv = ar[(int)threadIdx.x < tail ? 4 * nvec + threadIdx.x : 0];
+    const float tv = TAIL ? ar[(int)threadIdx.x < tail ? 4 * nvec + threadIdx.x : 0] : 0.0f;
     auto mag = [](float x) { return DIG3 && x != x ? __uint_as_float(0x7F800000u) : fabsf(x); };  // (the i8 rows' maximum drops a NaN)
     float amax = (int)threadIdx.x < tail ? fmaxf(0.0f, mag(tv)) : 0.0f;
 #pragma unroll
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(T) void quantize_rows_vec4_kernel(
             const int idx = threadIdx.x + i * T;
             if (idx < nvec) put(idx, {digits3(v[i].x, inv, finite), digits3(v[i].y, inv, finite), digits3(v[i].z, inv, finite), digits3(v[i].w, inv, finite)});
         }
-        if (tail && threadIdx.x < 4) {
+        if (TAIL && tail && threadIdx.x < 4) {
             const unsigned d = (int)threadIdx.x < tail ? digits3(tv, inv, finite) : 0u;
 #pragma unroll
             for (int p = 0; p < 3; ++p) qr[p * plane_bytes + 4 * nvec + threadIdx.x] = (int8_t)(d >> (8 * p));
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(T) void quantize_rows_vec4_kernel(
                 reinterpret_cast<int *>(qr)[idx] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
             }
         }
-        if (tail && threadIdx.x < 4) qr[4 * nvec + threadIdx.x] = (int8_t)((int)threadIdx.x < tail ? quant_to_i8(tv * inv_scale) : 0);
+        if (TAIL && tail && threadIdx.x < 4) qr[4 * nvec + threadIdx.x] = (int8_t)((int)threadIdx.x < tail ? quant_to_i8(tv * inv_scale) : 0);
         for (int idx = nvec + (tail != 0) + threadIdx.x; idx < npad; idx += T) reinterpret_cast<int *>(qr)[idx] = 0;
     }
 }
@@ -325,31 +325,36 @@ pg_status qtensor_alloc(pg_ctx *ctx, size_t rows, size_t cols, pg_qtensor **out)
 // Rows to i8 or, DIG3, to three digit planes.  A workgroup of 1024 threads for rows past what 256 hold in registers, and
 // where there are at most two rows a CU and a row is longer than 4096: the launch is then the latency of one row, and
 // four threads share what one would do.
+template <bool DIG3, bool TAIL>
+static pg_status launch_quantize_rows_vec4(pg_ctx *ctx, const char *name, const float *a, size_t rows, size_t cols, int8_t *q, size_t q_stride,
+                                           float *row_scales, size_t plane_bytes) {
+    const size_t nvec = cols / 4;
+    auto go = [&](auto kern, int threads) {
+        return pg_launch(ctx, name, kern, dim3((unsigned)rows), dim3(threads), 0, a, cols, q, q_stride, row_scales, plane_bytes);
+    };
+    if ((rows <= 2 * (size_t)ctx->num_cu && cols > 4096) || nvec > 16 * 256) {
+        if (nvec <= 1024) return go(quantize_rows_vec4_kernel<1, 1024, DIG3, TAIL>, 1024);
+        if (nvec <= 2 * 1024) return go(quantize_rows_vec4_kernel<2, 1024, DIG3, TAIL>, 1024);
+        if (nvec <= 4 * 1024) return go(quantize_rows_vec4_kernel<4, 1024, DIG3, TAIL>, 1024);
+        return go(quantize_rows_vec4_kernel<8, 1024, DIG3, TAIL>, 1024);
+    }
+    if (nvec <= 1 * 256) return go(quantize_rows_vec4_kernel<1, 256, DIG3, TAIL>, 256);
+    if (nvec <= 2 * 256) return go(quantize_rows_vec4_kernel<2, 256, DIG3, TAIL>, 256);
+    if (nvec <= 4 * 256) return go(quantize_rows_vec4_kernel<4, 256, DIG3, TAIL>, 256);
+    if (nvec <= 6 * 256) return go(quantize_rows_vec4_kernel<6, 256, DIG3, TAIL>, 256);
+    if (nvec <= 8 * 256) return go(quantize_rows_vec4_kernel<8, 256, DIG3, TAIL>, 256);
+    if (nvec <= 11 * 256) return go(quantize_rows_vec4_kernel<11, 256, DIG3, TAIL>, 256);
+    if (nvec <= 14 * 256) return go(quantize_rows_vec4_kernel<14, 256, DIG3, TAIL>, 256);
+    return go(quantize_rows_vec4_kernel<16, 256, DIG3, TAIL>, 256);
+}
+
 template <bool DIG3>
 static pg_status launch_quantize_rows(pg_ctx *ctx, const char *name, const float *a, size_t rows, size_t cols, int8_t *q, size_t q_stride,
                                       float *row_scales, size_t plane_bytes) {
-    const size_t nvec = cols / 4;
     const dim3 grid((unsigned)rows);
-    auto go = [&](auto kern, int threads) {
-        return pg_launch(ctx, name, kern, grid, dim3(threads), 0, a, cols, q, q_stride, row_scales, plane_bytes);
-    };
-    if (nvec >= 1 && q_stride % 4 == 0 && (uintptr_t)q % 4 == 0 && plane_bytes % 4 == 0) {
-        if ((rows <= 2 * (size_t)ctx->num_cu && cols > 4096) || nvec > 16 * 256) {
-            if (nvec <= 1024) return go(quantize_rows_vec4_kernel<1, 1024, DIG3>, 1024);
-            if (nvec <= 2 * 1024) return go(quantize_rows_vec4_kernel<2, 1024, DIG3>, 1024);
-            if (nvec <= 4 * 1024) return go(quantize_rows_vec4_kernel<4, 1024, DIG3>, 1024);
-            if (nvec <= 8 * 1024) return go(quantize_rows_vec4_kernel<8, 1024, DIG3>, 1024);
-        } else {
-            if (nvec <= 1 * 256) return go(quantize_rows_vec4_kernel<1, 256, DIG3>, 256);
-            if (nvec <= 2 * 256) return go(quantize_rows_vec4_kernel<2, 256, DIG3>, 256);
-            if (nvec <= 4 * 256) return go(quantize_rows_vec4_kernel<4, 256, DIG3>, 256);
-            if (nvec <= 6 * 256) return go(quantize_rows_vec4_kernel<6, 256, DIG3>, 256);
-            if (nvec <= 8 * 256) return go(quantize_rows_vec4_kernel<8, 256, DIG3>, 256);
-            if (nvec <= 11 * 256) return go(quantize_rows_vec4_kernel<11, 256, DIG3>, 256);
-            if (nvec <= 14 * 256) return go(quantize_rows_vec4_kernel<14, 256, DIG3>, 256);
-            return go(quantize_rows_vec4_kernel<16, 256, DIG3>, 256);
-        }
-    }
+    if (cols >= 4 && cols / 4 <= 8 * 1024 && q_stride % 4 == 0 && (uintptr_t)q % 4 == 0 && plane_bytes % 4 == 0)
+        return cols % 4 ? launch_quantize_rows_vec4<DIG3, true>(ctx, name, a, rows, cols, q, q_stride, row_scales, plane_bytes)
+                        : launch_quantize_rows_vec4<DIG3, false>(ctx, name, a, rows, cols, q, q_stride, row_scales, plane_bytes);
     if constexpr (DIG3)
         return pg_launch(ctx, name, rows_to_digits3_kernel, grid, dim3(QA_THREADS), 0, a, cols, q, q_stride, plane_bytes, row_scales);
     else
