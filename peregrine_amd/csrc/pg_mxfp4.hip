@@ -377,9 +377,26 @@ __global__ __launch_bounds__(64) void mxfp4_tile_offsets_kernel(const int *__res
 // their halves, tokens on consecutive lanes: what it writes are whole 256-byte runs of the records, and the
 // 256 bytes it reads of every token row are two full lines.
 // GATHER: the token groups are the experts' slots (mt_gather) instead of the rows in order.
-template <bool GATHER>
+// SWIGLU: x holds mlp1's outputs, [pairs][2 * 32 nb], and the values are their bias and swiglu, made on the way (a launch
+// and a round trip of the pairs' rows less: 11.4 -> 8.1 us for 80 pairs of 2880).
+struct mt_swiglu {
+    const float *const *bias_tab;
+    float alpha, clamp;
+    // biased = h + bias; gate = biased[2i].min(clamp); linear = biased[2i+1].clamp(-clamp, clamp);
+    // out[i] = gate * (1 / (1 + exp(-alpha * gate))) * (linear + 1)   examples/gpt_oss/moe.rs:155-166
+    __device__ __forceinline__ static float of(float g0, float l0, float alpha, float clamp) {
+        const float gate = fminf(g0, clamp);                                     // f32::min: a NaN operand loses
+        const float linear = l0 != l0 ? l0 : fminf(fmaxf(l0, -clamp), clamp);    // f32::clamp keeps NaN
+        const float activated = gate * (1.0f / (1.0f + expf(-alpha * gate)));
+        return activated * (linear + 1.0f);
+    }
+};
+
+template <bool GATHER, bool SWIGLU = false>
 __global__ __launch_bounds__(256) void mxfp4_planes_kernel(const float *__restrict__ x, int m, int nb, int ncp, int token_groups,
-                                                           char *__restrict__ bq, const mt_gather gat) {
+                                                           char *__restrict__ bq, const mt_gather gat, const mt_swiglu act) {
+    static_assert(GATHER || !SWIGLU, "pairs have experts");
+    const float *bias = nullptr;
     const size_t wv = ((size_t)blockIdx.x * 256 + threadIdx.x) >> 6;  // (token group, pair of blocks)
     const int lane = threadIdx.x & 63, col = lane & 15, sub = (lane >> 4) & 1, npair = 2 * ncp;
     const size_t tg = wv / npair;
@@ -394,13 +411,32 @@ __global__ __launch_bounds__(256) void mxfp4_planes_kernel(const float *__restri
         const int slot = ((gt - gat.goff[e]) * gat.tb + (int)(tg % gat.tb)) * 16 + col;
         valid = slot < gat.counts[e] && b < nb;
         t = valid ? (size_t)(gat.lists[(size_t)e * gat.stride + slot] / gat.div) : 0;
+        if (SWIGLU) bias = act.bias_tab[e];
     }
     float f[16];
+    if constexpr (SWIGLU) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (valid) v = reinterpret_cast<const float4 *>(x)[(t * nb + b) * 8 + sub * 4 + e];
-        f[4 * e] = v.x; f[4 * e + 1] = v.y; f[4 * e + 2] = v.z; f[4 * e + 3] = v.w;
+        for (int e = 0; e < 16; ++e) f[e] = 0.0f;
+        if (valid) {
+            const int at = (b * 8 + sub * 4) * 2;  // in float4s: 16 pairs (gate, linear)
+            float4 hv[8], bv[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) hv[e] = reinterpret_cast<const float4 *>(x)[t * nb * 16 + at + e];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bv[e] = reinterpret_cast<const float4 *>(bias)[at + e];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                f[2 * e] = mt_swiglu::of(hv[e].x + bv[e].x, hv[e].y + bv[e].y, act.alpha, act.clamp);
+                f[2 * e + 1] = mt_swiglu::of(hv[e].z + bv[e].z, hv[e].w + bv[e].w, act.alpha, act.clamp);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (valid) v = reinterpret_cast<const float4 *>(x)[(t * nb + b) * 8 + sub * 4 + e];
+            f[4 * e] = v.x; f[4 * e + 1] = v.y; f[4 * e + 2] = v.z; f[4 * e + 3] = v.w;
+        }
     }
     float amax = 0.0f;
     int bad = 0;
@@ -479,8 +515,114 @@ struct mt_experts {
     const uint32_t *const *sc_tab;
 };
 
+// A token tile with at most 16 / NPM slots in use: the spare columns of the B operand take NPM planes of each token (column
+// = token * NPM + plane), so a chunk is 4 / NPM instructions instead of four, and only the operand bytes of those tokens
+// pass through LDS, a batch of four chunks at a time (one barrier a batch).  The planes' sums are joined at the end.
+// Twenty tokens over 32 experts of 2880 x 2880, top 4 (2.7 slots a tile): the two products 71 + 40 -> 51 + 29 us, 250 and
+// 125 MB at 4.9 and 4.3 TB/s; before, the instructions and LDS reads of 16 slots took 40 us beside the stream, and 142
+// registers left one workgroup a CU with 64 KB of weights on their way (now 128 and two).
+template <int RA, int NPM>
+__device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, const uint32_t *__restrict__ sa, const char *__restrict__ bq,
+                                                  int ncp, int turn, v4f (&acc)[RA]) {
+    constexpr int NI = MT_PLANES / NPM, CHUNK = NI * 2048 + 256, STAGE = 4 * CHUNK;
+    const int lane = threadIdx.x & 63, t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const size_t a_stride = (size_t)ncp * 64;
+    // this thread's units of a batch: operand unit (chunk t / 128, half, lane) of every instruction, and a unit of the scales
+    const int oc = t >> 7, ol = t & 63, ocol = ol & 15;
+    const unsigned o_src = (unsigned)oc * MT_RECORD + (ocol % NPM) * MT_FRAG + ((t >> 6) & 1) * 1024 + (ocol / NPM + 16 * (ol >> 4)) * 16;
+    const unsigned o_dst = (unsigned)oc * CHUNK + ((t >> 6) & 1) * 1024 + ol * 16;
+    const unsigned s_src = (unsigned)(lane >> 4) * MT_RECORD + MT_PLANES * MT_FRAG + (lane & 15) * 16;
+    const unsigned s_dst = (unsigned)(lane >> 4) * CHUNK + NI * 2048 + (lane & 15) * 16;
+    v4i so[NI], ss;
+    auto fetch_b = [&](int c) {
+        const char *at = bq + (size_t)c * MT_RECORD;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) so[i] = *reinterpret_cast<const v4i *>(at + o_src + i * NPM * MT_FRAG);
+        ss = *reinterpret_cast<const v4i *>(at + s_src);
+    };
+    auto put_b = [&](int stage) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) *reinterpret_cast<v4i *>(lds + stage * STAGE + o_dst + i * 2048) = so[i];
+        if (wave == 0) *reinterpret_cast<v4i *>(lds + stage * STAGE + s_dst) = ss;
+    };
+    auto chunk_at = [&](int i) { return i + turn < ncp ? i + turn : i + turn - ncp; };
+    v4i a[4][RA], an[4][RA];
+    uint32_t sca[RA], sca_next[RA];
+    auto fetch_a = [&](v4i (&dst)[4][RA], uint32_t (&sc)[RA], int c) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int r = 0; r < RA; ++r) dst[u][r] = __builtin_nontemporal_load(qa + (size_t)r * a_stride + (size_t)(c + u) * 64 + lane);
+#pragma unroll
+        for (int r = 0; r < RA; ++r) sc[r] = sa[((size_t)r * (ncp / 4) + (c >> 2)) * 64 + lane];
+    };
+    const int col = lane & 15;
+    const unsigned sc_at = NI * 2048 + (col / NPM + 16 * (lane >> 4)) * 4, shift = 8 * (col % NPM);
+#pragma unroll
+    for (int r = 0; r < RA; ++r) acc[r] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    fetch_b(chunk_at(0));
+    fetch_a(a, sca, chunk_at(0));
+    put_b(0);
+    if (4 < ncp) fetch_b(chunk_at(4));
+    __syncthreads();
+#pragma unroll 1
+    for (int cb = 0, s = 0; cb < ncp; cb += 4, s ^= 1) {
+        const bool more = cb + 4 < ncp;
+        if (more) fetch_a(an, sca_next, chunk_at(cb + 4));
+        __builtin_amdgcn_sched_barrier(0);
+        const char *st = lds + s * STAGE;
+#define PG_MT_STEP(U, I)                                                                                                   \
+    do {                                                                                                                   \
+        const v4i b0 = *reinterpret_cast<const v4i *>(st + (U) * CHUNK + (I) * 2048 + lane * 16);                          \
+        const v4i b1 = *reinterpret_cast<const v4i *>(st + (U) * CHUNK + (I) * 2048 + 1024 + lane * 16);                   \
+        const int sb = (int)(*reinterpret_cast<const unsigned *>(st + (U) * CHUNK + sc_at) >> shift);                      \
+        const v8i B = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};                                            \
+        _Pragma("unroll") for (int r = 0; r < RA; ++r) {                                                                   \
+            const v4i aw = a[U][r];                                                                                        \
+            const v8i A = {aw[0], aw[1], aw[2], aw[3], 0, 0, 0, 0};                                                        \
+            acc[r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, acc[r], 4, 0, (U), (int)sca[r], NPM * (I), sb); \
+            asm volatile("" : "+v"(acc[r]) : : "memory");  /* (or every chunk's operands are read first: 32 to 64 registers) */ \
+        }                                                                                                                  \
+    } while (0)
+#define PG_MT_STEPS(U)                      \
+    do {                                    \
+        PG_MT_STEP(U, 0);                   \
+        if constexpr (NI == 2) PG_MT_STEP(U, 1); \
+    } while (0)
+        static_assert(NI == 1 || NI == 2, "the instructions of a chunk are written out");
+        PG_MT_STEPS(0);
+        PG_MT_STEPS(1);
+        PG_MT_STEPS(2);
+        PG_MT_STEPS(3);
+#undef PG_MT_STEPS
+#undef PG_MT_STEP
+        if (more) {
+            put_b(s ^ 1);
+            if (cb + 8 < ncp) fetch_b(chunk_at(cb + 8));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");  // (not __syncthreads(): the loads stay in flight)
+        if (more) {
+#pragma unroll
+            for (int r = 0; r < RA; ++r) sca[r] = sca_next[r];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int r = 0; r < RA; ++r) a[u][r] = an[u][r];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < RA; ++r)  // every lane of a token's columns: the sum over the planes
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float v = acc[r][i];
+            v += __shfl_xor(v, 1, 64);
+            if (NPM == 4) v += __shfl_xor(v, 2, 64);
+            acc[r][i] = v;
+        }
+}
+
 template <int RA, int TB, int BD, bool GROUPED>
-__global__ __launch_bounds__(64 * MT_NW) void mxfp4_tiles_kernel(const uint8_t *__restrict__ qs_frag, const uint32_t *__restrict__ sc_frag,
+__global__ __launch_bounds__(64 * MT_NW) __attribute__((amdgpu_waves_per_eu(GROUPED && TB == 1 && RA <= 2 ? 4 : 2))) void mxfp4_tiles_kernel(const uint8_t *__restrict__ qs_frag, const uint32_t *__restrict__ sc_frag,
                                                                  const char *__restrict__ bq, float *__restrict__ y, int n_out,
                                                                  int ncp, int m, int n_tt, int ks, int cps, size_t part_stride,
                                                                  int items, int per_xcd, const mt_gather gat, const mt_experts ex) {
@@ -507,13 +649,47 @@ __global__ __launch_bounds__(64 * MT_NW) void mxfp4_tiles_kernel(const uint8_t *
         const int left = gat.counts[expert] - (tt - gat.goff[expert]) * TB * 16;
         live = __builtin_amdgcn_readfirstlane(left >= TB * 16 ? TB : (left + 15) / 16);
     }
-    const int kc0 = split * cps, kc1 = pg_mt_run_end(split, cps, ncp);  // whole batches of four chunks
+    const int kc0 = split * cps, run = pg_mt_run_end(split, cps, ncp) - kc0;  // whole batches of four chunks
+    // Row groups lie a whole tensor row of chunks apart (24 KB for K = 2880): walked from the same end they would all be at the
+    // same few memory channels at a time, so every row tile begins at a batch of its own and wraps round (71 -> 66 us for
+    // the 250 MB of 30 experts' mlp1, before the narrow tiles).
+    const int turn = 4 * (wt % (run >> 2));
+    auto chunk_at = [&](int i) {  // the i-th chunk of the walk
+        i += turn;
+        return kc0 + (i < run ? i : i - run);
+    };
     const int nrg = (n_out + 15) / 16;                       // >= RA (the launcher's choice of RA)
     const int rg_mine = (wt * MT_NW + wave) * RA;            // the row groups whose tiles this wavefront stores
     const int rg0 = pg_mt_first_row_group(rg_mine, RA, nrg);  // the ones it reads: a spare wavefront repeats the last ones
     const size_t a_stride = (size_t)ncp * 64;                // v4i per row group
     const gv4i_ptr qa = (gv4i_ptr)(uintptr_t)qs_frag + (size_t)rg0 * a_stride;
     const uint32_t *const sa = sc_frag + (size_t)rg0 * (ncp / 4) * 64;
+    if constexpr (GROUPED && TB == 1) {
+        const int first = (tt - gat.goff[expert]) * 16, used = __builtin_amdgcn_readfirstlane(gat.counts[expert] - first);
+        if (used <= 8) {
+            v4f sum[RA];
+            const char *const rec = bq + (size_t)tt * ncp * MT_RECORD;
+            if (used <= 4) mxfp4_narrow_tile<RA, 4>(lds, qa, sa, rec, ncp, turn, sum);
+            else mxfp4_narrow_tile<RA, 2>(lds, qa, sa, rec, ncp, turn, sum);
+            const int npm = used <= 4 ? 4 : 2, slot = (lane & 15) / npm;
+            if ((lane & 15) % npm != 0 || slot >= used || rg_mine >= nrg) return;
+            const size_t token = (size_t)gat.lists[(size_t)expert * gat.stride + first + slot];
+#pragma unroll
+            for (int r = 0; r < RA; ++r) {
+                if (rg0 + r < rg_mine) continue;  // rows a spare wavefront only repeated
+                const size_t row = (size_t)(rg0 + r) * 16 + 4 * (lane >> 4);
+                float *o = y + token * n_out + row;
+                if (row + 3 < (size_t)n_out && (n_out & 3) == 0) {
+                    *reinterpret_cast<v4f *>(o) = sum[r];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (row + i < (size_t)n_out) o[i] = sum[r][i];
+                }
+            }
+            return;
+        }
+    }
     // this thread's share of a chunk's records: 16-byte unit u of the TB records, which lie ncp records apart
     const char *const b_base = bq + (size_t)tt * TB * ncp * MT_RECORD;
     unsigned b_off[ROUNDS];
@@ -544,27 +720,29 @@ __global__ __launch_bounds__(64 * MT_NW) void mxfp4_tiles_kernel(const uint8_t *
 #pragma unroll
         for (int g = 0; g < TB; ++g) acc[r][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-    PG_MT_FETCH_B(0, kc0);
-    if (BD > 1) PG_MT_FETCH_B(BD > 1 ? 1 : 0, kc0 + 1);
+    const int c0 = chunk_at(0);
+    PG_MT_FETCH_B(0, c0);
+    if (BD > 1) PG_MT_FETCH_B(BD > 1 ? 1 : 0, c0 + 1);
     if (BD > 2) {
-        PG_MT_FETCH_B(BD > 2 ? 2 : 0, kc0 + 2);
-        PG_MT_FETCH_B(BD > 2 ? 3 : 0, kc0 + 3);
+        PG_MT_FETCH_B(BD > 2 ? 2 : 0, c0 + 2);
+        PG_MT_FETCH_B(BD > 2 ? 3 : 0, c0 + 3);
     }
 #pragma unroll
-    for (int u = 0; u < (RING ? 2 : 4); ++u) fetch_a(a[u], kc0 + u);
+    for (int u = 0; u < (RING ? 2 : 4); ++u) fetch_a(a[u], c0 + u);
 #pragma unroll
-    for (int r = 0; r < RA; ++r) sca[r] = sa[((size_t)r * (ncp / 4) + (kc0 >> 2)) * 64 + lane];
+    for (int r = 0; r < RA; ++r) sca[r] = sa[((size_t)r * (ncp / 4) + (c0 >> 2)) * 64 + lane];
     PG_MT_PUT_B(0, 0);
-    if (kc0 + BD < kc1) PG_MT_FETCH_B(0, kc0 + BD);
+    if (BD < run) PG_MT_FETCH_B(0, chunk_at(BD));
     __syncthreads();
-    for (int cb = kc0; cb < kc1; cb += 4) {
-        const bool more = cb + 4 < kc1;
+    for (int cb = 0; cb < run; cb += 4) {
+        const bool more = cb + 4 < run;
         if (more) {
+            const int next = chunk_at(cb + 4);
 #pragma unroll
-            for (int r = 0; r < RA; ++r) sca_next[r] = sa[((size_t)r * (ncp / 4) + (cb >> 2) + 1) * 64 + lane];
+            for (int r = 0; r < RA; ++r) sca_next[r] = sa[((size_t)r * (ncp / 4) + (next >> 2)) * 64 + lane];
             if (!RING) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) fetch_a(an[RING ? 0 : u], cb + 4 + u);
+                for (int u = 0; u < 4; ++u) fetch_a(an[RING ? 0 : u], next + u);
             }
         }
     // One plane of one token group: its two operand halves are read while the previous plane's instructions run.
@@ -615,11 +793,11 @@ __global__ __launch_bounds__(64 * MT_NW) void mxfp4_tiles_kernel(const uint8_t *
         PG_MT_GROUP(U, 1);                                                                               \
         PG_MT_GROUP(U, 2);                                                                               \
         PG_MT_GROUP(U, 3);                                                                               \
-        if (c + 1 < kc1) {                                                                               \
+        if (c + 1 < run) {                                                                               \
             PG_MT_PUT_B(((U) + 1) & 1, ((U) + 1) % BD);                                                  \
-            if (c + 1 + BD < kc1) PG_MT_FETCH_B(((U) + 1) % BD, c + 1 + BD);                             \
+            if (c + 1 + BD < run) PG_MT_FETCH_B(((U) + 1) % BD, chunk_at(c + 1 + BD));                   \
         }                                                                                                \
-        if (RING && c + 2 < kc1) fetch_a(a[RING ? (U) & 1 : 0], c + 2);                                  \
+        if (RING && c + 2 < run) fetch_a(a[RING ? (U) & 1 : 0], chunk_at(c + 2));                        \
         __syncthreads();                                                                                 \
     } while (0)
         static_assert(MT_PLANES == 4 && TB <= 4, "the plane steps are written out");
@@ -690,7 +868,7 @@ pg_status launch_tiles(pg_ctx *ctx, const pg_gguf_tensor *w, const char *bq, flo
 template <int RA, int TB, int BD>
 pg_status launch_tiles_grouped(pg_ctx *ctx, size_t n_out, int ncp, const char *bq, float *y, size_t n_wt, size_t max_tiles,
                                const mt_gather &gat, const mt_experts &ex) {
-    const size_t lds = 2 * (size_t)TB * MT_RECORD;
+    const size_t lds = TB == 1 ? std::max<size_t>(2 * MT_RECORD, 2 * 4 * (2 * 2048 + 256)) : 2 * (size_t)TB * MT_RECORD;  // (mxfp4_narrow_tile<RA, 2>)
     auto kern = mxfp4_tiles_kernel<RA, TB, BD, true>;
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
     const size_t per_xcd = (max_tiles + 7) / 8 * n_wt, items = 8 * per_xcd;
@@ -741,7 +919,7 @@ pg_status pg_launch_mxfp4_tiles(pg_ctx *ctx, const float *x_dev, size_t m, const
     const size_t threads = p.groups * 2 * (size_t)ncp * 64;  // a wavefront per token group and pair of blocks
     PG_CHECK_ARG((threads + 255) / 256 < ((size_t)1 << 31), "mxfp4: %zu rows x %zu is too much for one pre-pass", m, w->k_in);
     PG_TRY(pg_launch(ctx, "mxfp4_planes", mxfp4_planes_kernel<false>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, x_dev, (int)m, nb,
-                     ncp, (int)p.groups, bq, mt_gather{}));
+                     ncp, (int)p.groups, bq, mt_gather{}, mt_swiglu{}));
     // the staging depth: the less arithmetic a chunk holds, the more chunks ahead
 #define PG_MT_LAUNCH(RA_, BD1, BD2, BD4) \
     (p.tb == 1 ? launch_tiles<RA_, 1, BD1>(ctx, w, bq, part, m, ncp, p) \
@@ -818,19 +996,14 @@ struct pg_mxfp4_expert {
 };
 
 namespace {
-// biased = h + bias1; gate = biased[2i].min(clamp); linear = biased[2i+1].clamp(-clamp, clamp);
-// out[i] = gate * (1 / (1 + exp(-alpha * gate))) * (linear + 1)
+// biased = h + bias1, then the swiglu (mt_swiglu)
 __global__ __launch_bounds__(256) void mxfp4_bias_swiglu_kernel(const float *__restrict__ h, const float *__restrict__ bias,
                                                                 size_t rows, size_t inter, float alpha, float clamp,
                                                                 float *__restrict__ out) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= rows * inter) return;
     const size_t r = i / inter, c = i - r * inter;
-    const float g0 = h[r * 2 * inter + 2 * c] + bias[2 * c], l0 = h[r * 2 * inter + 2 * c + 1] + bias[2 * c + 1];
-    const float gate = fminf(g0, clamp);                                     // f32::min: a NaN operand loses
-    const float linear = l0 != l0 ? l0 : fminf(fmaxf(l0, -clamp), clamp);    // f32::clamp keeps NaN
-    const float activated = gate * (1.0f / (1.0f + expf(-alpha * gate)));
-    out[i] = activated * (linear + 1.0f);
+    out[i] = mt_swiglu::of(h[r * 2 * inter + 2 * c] + bias[2 * c], h[r * 2 * inter + 2 * c + 1] + bias[2 * c + 1], alpha, clamp);
 }
 
 __global__ __launch_bounds__(256) void bias_add_kernel(const float *__restrict__ a, const float *__restrict__ bias,
@@ -930,11 +1103,7 @@ __global__ __launch_bounds__(256) void mxfp4_moe_swiglu_kernel(const float *__re
     if (i >= pairs * inter) return;
     const size_t p = i / inter, c = i - p * inter;
     const float *bias = bias_tab[topk_idx[p]];
-    const float g0 = h[p * 2 * inter + 2 * c] + bias[2 * c], l0 = h[p * 2 * inter + 2 * c + 1] + bias[2 * c + 1];
-    const float gate = fminf(g0, clamp);                                     // f32::min: a NaN operand loses
-    const float linear = l0 != l0 ? l0 : fminf(fmaxf(l0, -clamp), clamp);    // f32::clamp keeps NaN
-    const float activated = gate * (1.0f / (1.0f + expf(-alpha * gate)));
-    out[i] = activated * (linear + 1.0f);
+    out[i] = mt_swiglu::of(h[p * 2 * inter + 2 * c] + bias[2 * c], h[p * 2 * inter + 2 * c + 1] + bias[2 * c + 1], alpha, clamp);
 }
 
 // output[t] += weight * (out + mlp2_bias) over the token's experts in the order given  (examples/gpt_oss/moe.rs:104-108, 330-334)
@@ -955,14 +1124,16 @@ __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__r
 }
 
 // One grouped product: rows `src` (pair / div) of the experts' slots -> records -> tiles against tensor table `which`.
+// With `act`: the rows are the swiglu of src, mlp1's outputs.
 pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, int tb, size_t max_tiles, mt_gather gat, int div,
-                      const void **tab, size_t experts, int which, char *bq, float *y) {
+                      const void **tab, size_t experts, int which, char *bq, float *y, const mt_swiglu *act = nullptr) {
     const int nb = (int)(k_in / 32), ncp = (int)mx_chunks((size_t)nb);
     gat.div = div;
     const size_t groups = max_tiles * tb, threads = groups * 2 * (size_t)ncp * 64;
     PG_CHECK_ARG((threads + 255) / 256 < ((size_t)1 << 31), "mxfp4 moe: too many pairs x %zu for one pre-pass", k_in);
-    PG_TRY(pg_launch(ctx, "mxfp4_planes_gather", mxfp4_planes_kernel<true>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, src, 0, nb,
-                     ncp, (int)groups, bq, gat));
+    const dim3 grid((unsigned)((threads + 255) / 256));
+    if (act) PG_TRY(pg_launch(ctx, "mxfp4_planes_swiglu", mxfp4_planes_kernel<true, true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, *act));
+    else PG_TRY(pg_launch(ctx, "mxfp4_planes_gather", mxfp4_planes_kernel<true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, mt_swiglu{}));
     const size_t nrg = (n_out + 15) / 16;
     int ra = 4;
     while (ra > 1 && ((size_t)ra > nrg || (nrg + MT_NW * ra - 1) / (MT_NW * ra) * max_tiles < 2 * (size_t)ctx->num_cu)) ra >>= 1;
@@ -974,7 +1145,7 @@ pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, 
     (tb == 1 ? launch_tiles_grouped<RA_, 1, BD1>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex) \
      : tb == 2 ? launch_tiles_grouped<RA_, 2, BD2>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex) \
                : launch_tiles_grouped<RA_, 4, BD4>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex))
-    return ra == 4 ? PG_MTG(4, 4, 2, 1) : (ra == 2 ? PG_MTG(2, 4, 4, 2) : PG_MTG(1, 4, 4, 4));
+    return ra == 4 ? PG_MTG(4, 4, 2, 1) : (ra == 2 ? PG_MTG(2, 2, 4, 2) : PG_MTG(1, 4, 4, 4));
 #undef PG_MTG
 }
 
@@ -1019,10 +1190,13 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     const int tb = P / E <= 16 ? 1 : (P / E <= 32 ? 2 : 4);
     const size_t max_tiles = P / (16 * (size_t)tb) + E;  // sum over experts of ceil(count / (16 tb)) stays below
     const int ncp1 = (int)mx_chunks(hidden / 32), ncp2 = (int)mx_chunks(inter / 32);
+    // With few pairs hardly two of them meet in an expert, and a pair is a one-row product: the decode kernel, one
+    // workgroup column per pair (exact activations; no expert lists).  Otherwise the experts' token tiles on the tile kernel.
+    const bool by_pairs = P <= 2 * E && P <= 64 && pairs_fit(ncp1) && pairs_fit(ncp2);
     const size_t sz_idx = pg_round_up(P * sizeof(int), 256), sz_p = pg_round_up(P * sizeof(float), 256);
     const size_t sz_lists = pg_round_up(E * T * sizeof(int), 256), sz_counts = pg_round_up((2 * E + 1) * sizeof(int), 256);
     const size_t sz_rec = pg_round_up(max_tiles * tb * (size_t)std::max(ncp1, ncp2) * MT_RECORD, 256);
-    const size_t sz_h = pg_round_up(P * 2 * inter * sizeof(float), 256), sz_act = pg_round_up(P * inter * sizeof(float), 256);
+    const size_t sz_h = pg_round_up(P * 2 * inter * sizeof(float), 256), sz_act = by_pairs ? pg_round_up(P * inter * sizeof(float), 256) : 0;
     const size_t sz_y = pg_round_up(P * hidden * sizeof(float), 256);
     void *ws = nullptr;
     PG_TRY(pg_workspace(ctx, sz_idx + sz_p + sz_lists + sz_counts + sz_rec + sz_h + sz_act + sz_y, &ws));
@@ -1044,9 +1218,6 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     }
     const void **tab = nullptr;
     PG_TRY(pg_moe_cached_table(ctx, host_tab, 6 * E, &tab));
-    // With few pairs hardly two of them meet in an expert, and a pair is a one-row product: the decode kernel, one
-    // workgroup column per pair (exact activations; no expert lists).  Otherwise the experts' token tiles on the tile kernel.
-    const bool by_pairs = P <= 2 * E && P <= 64 && pairs_fit(ncp1) && pairs_fit(ncp2);
     PG_TRY(pg_launch_moe_routing(ctx, nullptr, expert_idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, by_pairs ? nullptr : lists, counts));
     if (!by_pairs)
         PG_TRY(pg_launch(ctx, "mxfp4_tile_offsets", mxfp4_tile_offsets_kernel, dim3(1), dim3(64), 0, (const int *)counts, (int)E, tb, goff));
@@ -1055,12 +1226,15 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
         PG_TRY(moe_product_pairs(ctx, x_dev, T, hidden, 2 * inter, P, (int)top_k, tab, E, 0, topk_idx, h));
     else
         PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, tb, max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
-    PG_TRY(pg_launch(ctx, "mxfp4_moe_swiglu", mxfp4_moe_swiglu_kernel, dim3(grid_for(P * inter, 256)), dim3(256), 0, (const float *)h,
-                     reinterpret_cast<const float *const *>(tab + 4 * E), (const int *)topk_idx, P, inter, alpha, clamp, act));
-    if (by_pairs)
+    const float *const *bias1 = reinterpret_cast<const float *const *>(tab + 4 * E);
+    if (by_pairs) {
+        PG_TRY(pg_launch(ctx, "mxfp4_moe_swiglu", mxfp4_moe_swiglu_kernel, dim3(grid_for(P * inter, 256)), dim3(256), 0, (const float *)h,
+                         bias1, (const int *)topk_idx, P, inter, alpha, clamp, act));
         PG_TRY(moe_product_pairs(ctx, act, P, inter, hidden, P, 1, tab, E, 1, topk_idx, yb));
-    else
-        PG_TRY(moe_product(ctx, act, inter, hidden, tb, max_tiles, gat, 1, tab, E, 1, rec, yb));
+    } else {
+        const mt_swiglu sw = {bias1, alpha, clamp};
+        PG_TRY(moe_product(ctx, h, inter, hidden, tb, max_tiles, gat, 1, tab, E, 1, rec, yb, &sw));
+    }
     return pg_launch(ctx, "mxfp4_moe_combine", mxfp4_moe_combine_kernel, dim3(grid_for(T * hidden, 256)), dim3(256), 0, (const float *)yb,
                      reinterpret_cast<const float *const *>(tab + 5 * E), (const int *)topk_idx, (const float *)topk_p, T, hidden,
                      (int)top_k, out_dev);

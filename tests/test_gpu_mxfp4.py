@@ -252,3 +252,36 @@ def test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, 
             mxfp4.moe_forward_routed(x, bad, w, experts, ctx)
     for ex in experts:
         ex.free()
+
+
+@pytest.mark.parametrize("hidden,inter", [(96, 64), (1120, 544), (2880, 288), (544, 2112)])
+def test_mxfp4_moe_tiles_with_few_slots(ctx, orc, hidden, inter):
+    """Experts with 0 to 17 tokens in one launch: up to 4 and up to 8 slots of a token tile go through narrower forms of the
+    product (several digit planes of a token in one operand); 17 is a full tile and one slot.  A token that holds a NaN
+    leaves the others of its tile as they are.  Bound as for the routed test above: 20 bits under a block's largest value."""
+    from peregrine_amd import mxfp4
+    from test_oracle_formats_pins import _mx_expert
+    say(f"mxfp4 moe, few slots, hidden={hidden} inter={inter}")
+    rng = np.random.default_rng(hidden + inter)
+    counts = [0, 1, 3, 4, 5, 8, 9, 15, 16, 17, 2]          # 80 pairs over 11 experts: tiles of 16 slots
+    E, T = len(counts), sum(counts)
+    raw = [_mx_expert(rng, hidden, inter) for _ in range(E)]
+    experts = [mxfp4.Mxfp4Expert(hidden, inter, 1.702, 7.0, *r, ctx=ctx) for r in raw]
+    idx = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(T, 1)
+    w = rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32)
+    x = orc.rng_normal(T + 3, T * hidden).reshape(T, hidden)
+    x[:, ::37] *= 10.0
+    got = mxfp4.moe_forward_routed(x, idx, w, experts, ctx)
+    want = orc.mxfp4_moe_routed(x, T, hidden, inter, 1.702, 7.0, 1, idx, w, raw)
+    for t in range(T):
+        H.assert_close_rel(got[t], want[t], 2e-4, f"token {t}, one of {counts[idx[t, 0]]} of its expert")
+    for n in (3, 8):
+        t = int(np.flatnonzero(idx[:, 0] == counts.index(n))[0])
+        xn = x.copy()
+        xn[t, hidden // 2] = np.nan
+        other = mxfp4.moe_forward_routed(xn, idx, w, experts, ctx)
+        assert not np.isfinite(other[t]).any()
+        keep = np.arange(T) != t
+        assert (other[keep] == got[keep]).all()
+    for ex in experts:
+        ex.free()
