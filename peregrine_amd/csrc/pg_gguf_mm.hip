@@ -294,10 +294,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
     const int count = grp.counts ? grp.counts[e] : grp.max_count;
     if (tt * 32 >= count) return;  // the same for every thread of the workgroup
-    const uint8_t *qs_any = grp.qs_table ? grp.qs_table[e] : qs0;
-    const uint16_t *d_any = grp.d_table ? grp.d_table[e] : d0;
     int n_out = n_out_arg;
     float *__restrict__ out = out_arg;
+    const uint8_t *const *qs_table = grp.qs_table;
+    const uint16_t *const *d_table = grp.d_table;
+    if (grp.qs_table2 && bx >= (n_out_arg + 127) / 128) {  // the expert's second tensor
+        bx -= (n_out_arg + 127) / 128;
+        qs_table = grp.qs_table2;
+        d_table = grp.d_table2;
+        out = grp.out2;
+    }
+    const uint8_t *qs_any = qs_table ? qs_table[e] : qs0;
+    const uint16_t *d_any = d_table ? d_table[e] : d0;
     size_t part_stride = part_stride_arg;
     if (grp.nseg) {  // which tensor of the launch this row group belongs to
         int t = 0;
@@ -1187,12 +1195,14 @@ pg_status pg_launch_gguf_mm(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_i
     const size_t gy = experts * (size_t)grp.tiles_per_expert;
     // token tiles that certainly hold work: all of them without expert lists, one per expert with
     bool by_xcd = false;
-    const int ks = pg_gguf_mm_splitk(ctx, n_out, k_in, grp.counts ? experts : gy, md.rows, grp.counts != nullptr, &chunk, &by_xcd);
+    const bool second = grp.qs_table2 != nullptr;
+    if (second && (!grp.counts || !keep_parts)) return pg_fail(PG_EINVAL, "gguf_mm: a second tensor per expert needs expert lists and leaves its K chunks unsummed");
+    const int ks = pg_gguf_mm_splitk(ctx, second ? pg_mm_pair_rows(n_out) : n_out, k_in, grp.counts ? experts : gy, md.rows, grp.counts != nullptr, &chunk, &by_xcd);
     if (ks > 1 && !part) return pg_fail(PG_EINVAL, "gguf_mm: split-K needs a partial-sum buffer");
     if (grp.nseg && ((ks > 1 && !keep_parts) || grp.counts || !grp.tiled))
         return pg_fail(PG_EINVAL, "gguf_mm: several tensors in one launch leave their K chunks unsummed, take no expert lists and read tile-major copies");
     if (gy > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_mm: too many token tiles");
-    dim3 grid(grid_for(n_out, 128), (unsigned)gy, (unsigned)ks);
+    dim3 grid(grid_for(n_out, 128) * (second ? 2 : 1), (unsigned)gy, (unsigned)ks);
     pg_mm_group g2 = grp;
     g2.remap_rg = g2.remap_tiles = 0;
     if (!grp.counts && ks == 1 && gy >= 16) {  // a plain product over many token tiles: see the kernel

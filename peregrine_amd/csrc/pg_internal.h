@@ -407,7 +407,14 @@ struct pg_mm_group {
     const uint16_t *seg_d[3];
     float *seg_out[3];
     size_t seg_stride[3];
+    // A second tensor per expert of the same shape (gate and up in one launch): its 128-row groups follow the first
+    // ones', its planes go to out2, as far apart as the first ones'.
+    const uint8_t *const *qs_table2;
+    const uint16_t *const *d_table2;
+    float *out2;
 };
+// Rows of a launch over two tensors of n_out rows each (whole 128-row groups).
+inline size_t pg_mm_pair_rows(size_t n_out) { return 2 * pg_round_up(n_out, 128); }
 // Bytes from one 128-row group of a tile-major copy to the next: the group's stages (16 KiB
 // each for Q8_0, 8 KiB for Q4_0) plus 4352 bytes, so that workgroups walking their groups in
 // step do not all address the same memory channels (a bare power-of-two stride would).
@@ -463,7 +470,8 @@ pg_status pg_launch_mxfp4_rows(pg_ctx *ctx, const float *x_dev, size_t m, const 
 constexpr int PG_MOE_MAX_EXPERTS = 256;
 pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n, const void ***dev_tab);
 pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, const int *idx_dev, const float *weight_dev, size_t T,
-                                size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts);
+                                size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts,
+                                int *goff, int tile);
 struct pg_mxfp4_tiles_plan {
     int ra, tb;            // groups of 16 weight rows per wavefront, groups of 16 tokens per workgroup
     int ks, cps;           // runs of K and chunks per run

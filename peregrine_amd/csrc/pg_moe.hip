@@ -8,6 +8,7 @@
 //   5. out[t] = 0 + p_0 * y_0 + p_1 * y_1 ... in k order, multiply then add
 //      (examples/grok1/moe.rs:99-104), raw softmax probabilities.
 #include "pg_internal.h"
+#include "pg_digits.h"
 #include <algorithm>
 
 namespace {
@@ -41,6 +42,101 @@ __global__ void route_topk_kernel(const float *__restrict__ logits, int T, int E
         taken[best >> 5] |= 1u << (best & 31);
         topk_idx[(size_t)t * top_k + k] = best;
         topk_p[(size_t)t * top_k + k] = bp;
+    }
+}
+
+// The same, or a copy of the caller's routing (see below), and the experts' lists and first token tiles, in ONE launch of one
+// workgroup while the routing is small: as launches of their own they are the launch and little else (copy, lists and
+// offsets of 20 tokens over 32 experts 13.8 us, 4.8 here; softmax, top-k and lists of 64 over 8 11.0, 4.8 here).  The logits pass through
+// LDS (a row per thread, an odd number of words apart) and hold the probabilities afterwards, -1 where taken; the chosen
+// experts stay there as bytes for the lists.  Grid 1; MAX_ROUTE_LDS bytes at most.
+constexpr size_t MAX_ROUTE_LDS = 48u << 10;
+__host__ __device__ inline size_t route_row(size_t E) { return E | 1; }
+inline bool route_in_one(size_t T, size_t E, size_t top_k) {
+    // (lists: a wavefront of the 16 takes every 16th expert and looks at 64 pairs at a time: 128 such steps, 4 us, at most)
+    return T * top_k * E <= (1u << 17) && T * route_row(E) * sizeof(float) + T * top_k <= MAX_ROUTE_LDS;
+}
+template <bool LOGITS>
+__global__ __launch_bounds__(1024) void route_lists_kernel(const float *__restrict__ logits, const int *__restrict__ idx_in,
+                                                           const float *__restrict__ w_in, int T, int E, int top_k,
+                                                           int *__restrict__ topk_idx, float *__restrict__ topk_p,
+                                                           int *__restrict__ lists, int *__restrict__ counts, int *__restrict__ goff, int tile) {
+    extern __shared__ __attribute__((aligned(16))) float prob[];  // [T][route_row(E)] (LOGITS), then the pairs' experts as bytes
+    __shared__ int cnt[MAX_EXPERTS];
+    const int row = (int)route_row(E), P = T * top_k;
+    uint8_t *const chosen = reinterpret_cast<uint8_t *>(prob + (LOGITS ? T * row : 0));
+    if (LOGITS) {
+        for (int i = threadIdx.x; i < T * E; i += 1024) prob[i / E * row + i % E] = logits[i];
+        __syncthreads();
+    }
+    for (int t = threadIdx.x; t < T; t += 1024) {
+        uint8_t *mine = chosen + t * top_k;
+        if (LOGITS) {
+            float *x = prob + t * row;
+            float mx = -INFINITY;
+            for (int e = 0; e < E; ++e)
+                if (x[e] > mx) mx = x[e];
+            float sum = 0.0f;
+            for (int e = 0; e < E; ++e) {
+                x[e] = expf(x[e] - mx);
+                sum += x[e];
+            }
+            for (int e = 0; e < E; ++e) x[e] = x[e] / sum;
+            for (int k = 0; k < top_k; ++k) {
+                int best = -1;
+                float bp = 0.0f;
+                for (int e = 0; e < E; ++e) {
+                    const float p = x[e];
+                    if (p == -1.0f) continue;
+                    if (best < 0 || p > bp) { best = e; bp = p; }
+                }
+                x[best] = -1.0f;
+                mine[k] = (uint8_t)best;
+                topk_idx[t * top_k + k] = best;
+                topk_p[t * top_k + k] = bp;
+            }
+        } else {
+            auto taken = [&](int e, int k) {
+                bool is = false;
+                for (int j = 0; j < k; ++j) is |= mine[j] == (uint8_t)e;
+                return is;
+            };
+            for (int k = 0; k < top_k; ++k) {
+                int e = idx_in[t * top_k + k];
+                float w = w_in[t * top_k + k];
+                if (e < 0 || e >= E || taken(e, k)) {
+                    e = 0;
+                    while (taken(e, k)) ++e;  // top_k <= E: a free expert exists
+                    w = 0.0f;
+                }
+                mine[k] = (uint8_t)e;
+                topk_idx[t * top_k + k] = e;
+                topk_p[t * top_k + k] = w;
+            }
+        }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    for (int e = threadIdx.x >> 6; e < E; e += 16) {
+        int base = 0;
+        for (int p0 = 0; p0 < P; p0 += 64) {
+            const int p = p0 + lane;
+            const bool own = p < P && chosen[p] == e;
+            const unsigned long long mask = __ballot(own);
+            if (own) lists[(size_t)e * T + base + __popcll(mask & ((1ull << lane) - 1ull))] = p;
+            base += __popcll(mask);
+        }
+        if (lane == 0) {
+            counts[e] = base;
+            cnt[e] = (base + tile - 1) / tile;
+        }
+    }
+    if (!goff) return;
+    __syncthreads();
+    if ((int)threadIdx.x <= E) {  // first token tile of every expert, and their number
+        int run = 0;
+        for (int e = 0; e < (int)threadIdx.x; ++e) run += cnt[e];
+        goff[threadIdx.x] = run;
     }
 }
 
@@ -85,6 +181,17 @@ __global__ __launch_bounds__(64) void expert_lists_kernel(const int *__restrict_
     if (lane == 0) counts[e] = base;
 }
 
+// First tile of `tile` pairs of every expert: goff[e] = sum over e' < e of ceil(counts[e'] / tile); goff[experts] = all.
+__global__ __launch_bounds__(64) void tile_offsets_kernel(const int *__restrict__ counts, int experts, int tile, int *__restrict__ goff) {
+    if (threadIdx.x != 0) return;
+    int run = 0;
+    for (int e = 0; e < experts; ++e) {
+        goff[e] = run;
+        run += (counts[e] + tile - 1) / tile;
+    }
+    goff[experts] = run;
+}
+
 __device__ __forceinline__ float act_silu(float x) {
     const float sig = 1.0f / (1.0f + expf(-x));
     return x * sig;
@@ -95,6 +202,36 @@ __device__ __forceinline__ float act_gelu_tanh(float x) {
     return 0.5f * x * (1.0f + tanhf(inner));
 }
 
+// act(g) * u of every pair as the digit planes of the matrix-core product; g and u as the sums of `planes` planes, `stride`
+// floats apart, in ascending order.  (As two launches, with the products through memory: 10.5 us for 128 pairs of 8192, 5.6 here.)
+template <bool NIB>
+__global__ __launch_bounds__(256) void act_mm_digits_kernel(const float *__restrict__ g, const float *__restrict__ u, int planes, size_t stride,
+                                                            int act, int nb, int nbp, int8_t *__restrict__ digits, float *__restrict__ xs) {
+    const size_t row = blockIdx.y;
+    const int b = blockIdx.x * 32 + (threadIdx.x >> 3), sub = threadIdx.x & 7;
+    if (b >= nb) return;  // whole 8-thread groups leave together
+    const size_t at = ((row * nb + b) * 8 + sub) * 4;
+    float4 gp[8], up[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+        if (s < planes) {
+            gp[s] = *reinterpret_cast<const float4 *>(g + s * stride + at);
+            up[s] = *reinterpret_cast<const float4 *>(u + s * stride + at);
+        }
+    float4 gv = gp[0], uv = up[0];
+#pragma unroll
+    for (int s = 1; s < 8; ++s)
+        if (s < planes) {
+            gv.x += gp[s].x; gv.y += gp[s].y; gv.z += gp[s].z; gv.w += gp[s].w;
+            uv.x += up[s].x; uv.y += up[s].y; uv.z += up[s].z; uv.w += up[s].w;
+        }
+    const float gf[4] = {gv.x, gv.y, gv.z, gv.w}, uf[4] = {uv.x, uv.y, uv.z, uv.w};
+    float o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (act == PG_ACT_GELU_TANH ? act_gelu_tanh(gf[i]) : act_silu(gf[i])) * uf[i];
+    pg_emit_mm_digits<NIB>(o, row, b, sub, nb, nbp, digits, xs);
+}
+
 __global__ void act_mul_kernel(const float *__restrict__ g, const float *__restrict__ u, size_t n,
                                int act, float *__restrict__ h) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -103,15 +240,19 @@ __global__ void act_mul_kernel(const float *__restrict__ g, const float *__restr
     h[i] = a * u[i];
 }
 
+// yb: the down product's outputs, the sums of `planes` planes (its K chunks) in ascending order.
 // `shared` (optional): the shared experts' output, added last (y.add(&z), examples/deepseek/moe.rs:298-300).
-__global__ void combine_kernel(const float *__restrict__ yb, const float *__restrict__ topk_p, int T,
+__global__ void combine_kernel(const float *__restrict__ yb, int planes, size_t stride, const float *__restrict__ topk_p, int T,
                                int d, int top_k, const float *__restrict__ shared, float *__restrict__ out) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)T * d) return;
     const size_t t = i / d, c = i - t * d;
     float acc = 0.0f;
     for (int k = 0; k < top_k; ++k) {
-        const float prod = topk_p[t * top_k + k] * yb[(t * top_k + k) * d + c];
+        const float *y = yb + (t * top_k + k) * d + c;
+        float v = y[0];
+        for (int s = 1; s < planes; ++s) v += y[s * stride];
+        const float prod = topk_p[t * top_k + k] * v;
         acc = acc + prod;
     }
     out[i] = shared ? acc + shared[i] : acc;
@@ -153,8 +294,15 @@ pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n
 // The routing of T tokens as the expert products want it: topk_idx / topk_p [T * top_k] (from the router's logits,
 // grok1's softmax -> top-k, or a copy of the caller's own choice with out-of-range and repeated experts made
 // harmless), and per expert the (token, k) pairs routed to it in ascending order (lists [E][T], counts [E]).
+// With `goff` also the first of each expert's tiles of `tile` pairs, and their number in goff[E].
 pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, const int *idx_dev, const float *weight_dev, size_t T,
-                                size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts) {
+                                size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts, int *goff, int tile) {
+    if (lists && route_in_one(T, E, top_k)) {
+        const size_t lds = (router_logits_dev ? T * route_row(E) * sizeof(float) : 0) + T * top_k;
+        auto *kern = router_logits_dev ? route_lists_kernel<true> : route_lists_kernel<false>;
+        return pg_launch(ctx, "moe_route_lists", kern, dim3(1), dim3(1024), lds, router_logits_dev, idx_dev, weight_dev, (int)T, (int)E,
+                         (int)top_k, topk_idx, topk_p, lists, counts, goff, tile);
+    }
     if (router_logits_dev)
         PG_TRY(pg_launch(ctx, "moe_route_topk", route_topk_kernel, dim3(grid_for(T, 64)), dim3(64), 0,
                          router_logits_dev, (int)T, (int)E, (int)top_k, topk_idx, topk_p));
@@ -162,8 +310,10 @@ pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, con
         PG_TRY(pg_launch(ctx, "moe_copy_routing", copy_routing_kernel, dim3(grid_for(T, 64)), dim3(64), 0,
                          idx_dev, weight_dev, (int)T, (int)E, (int)top_k, topk_idx, topk_p));
     if (!lists) return PG_OK;  // (a caller that works pair by pair)
-    return pg_launch(ctx, "moe_expert_lists", expert_lists_kernel, dim3((unsigned)E), dim3(64), 0, (const int *)topk_idx,
-                     (int)(T * top_k), (int)T, lists, counts);
+    PG_TRY(pg_launch(ctx, "moe_expert_lists", expert_lists_kernel, dim3((unsigned)E), dim3(64), 0, (const int *)topk_idx,
+                     (int)(T * top_k), (int)T, lists, counts));
+    if (!goff) return PG_OK;
+    return pg_launch(ctx, "moe_tile_offsets", tile_offsets_kernel, dim3(1), dim3(64), 0, (const int *)counts, (int)E, tile, goff);
 }
 
 // The expert FFN behind both entry points: the routing comes from `router_logits_dev` (grok1's softmax -> top-k) or,
@@ -208,33 +358,32 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     //    streaming kernel's case (Grok-1-sized experts, Q8_0, top 2: 315 -> 227 us, the three products at 6.3 TB/s;
     //    from two tokens on pairs share experts and the matrix-core kernel, which reads an expert once, wins)
     const bool one_token = T == 1;
-    const bool up_stream = narrow || one_token || d / 32 < PG_MM_MIN_BLOCKS, down_stream = narrow || one_token || ffn / 32 < PG_MM_MIN_BLOCKS;
+    const bool down_stream = narrow || one_token || ffn / 32 < PG_MM_MIN_BLOCKS, up_stream = down_stream || d / 32 < PG_MM_MIN_BLOCKS;
     PG_CHECK_ARG(!(up_stream || down_stream) || P <= 65535, "pg_moe_ffn: too many pairs for experts this small");
 
     // Arena layout.
-    const int ks_up = up_stream ? 1 : pg_gguf_mm_splitk(ctx, ffn, d, E, T, true, nullptr);
+    // (K chunks' planes stay apart: the launch that reads a product adds them.)
+    const size_t pair_rows = pg_mm_pair_rows(ffn);
+    const int ks_up = up_stream ? 1 : pg_gguf_mm_splitk(ctx, pair_rows, d, E, T, true, nullptr);
     const int ks_down = down_stream ? 1 : pg_gguf_mm_splitk(ctx, d, ffn, E, P, true, nullptr);
-    const size_t part_floats = std::max(ks_up > 1 ? (size_t)ks_up * P * ffn : 0, ks_down > 1 ? (size_t)ks_down * P * d : 0);
     const size_t sz_idx = pg_round_up(P * sizeof(int), 256);
     const size_t sz_p = pg_round_up(P * sizeof(float), 256);
     const size_t sz_lists = pg_round_up(E * T * sizeof(int), 256), sz_counts = pg_round_up(E * sizeof(int), 256);
-    const size_t sz_act = pg_round_up(P * ffn * sizeof(float), 256);
-    const size_t sz_y = pg_round_up(P * d * sizeof(float), 256);
-    const size_t sz_part = pg_round_up(part_floats * sizeof(float), 256);
+    const size_t sz_act = pg_round_up(P * ffn * sizeof(float), 256), sz_gu = pg_round_up((size_t)ks_up * P * ffn * sizeof(float), 256);
+    const size_t sz_h = down_stream ? sz_act : 0, sz_y = pg_round_up((size_t)ks_down * P * d * sizeof(float), 256);
     const size_t sz_xd = up_stream ? pg_xdigits_bytes(T, d) : pg_mmdigits_bytes(T, d);
     const size_t sz_hd = down_stream ? pg_xdigits_bytes(P, ffn) : pg_mmdigits_bytes(P, ffn);
     void *ws = nullptr;
-    PG_TRY(pg_workspace(ctx, sz_idx + sz_p + sz_lists + sz_counts + 3 * sz_act + sz_y + sz_part + sz_xd + sz_hd, &ws));
+    PG_TRY(pg_workspace(ctx, sz_idx + sz_p + sz_lists + sz_counts + 2 * sz_gu + sz_h + sz_y + sz_xd + sz_hd, &ws));
     char *p = static_cast<char *>(ws);
     int *topk_idx = reinterpret_cast<int *>(p); p += sz_idx;
     float *topk_p = reinterpret_cast<float *>(p); p += sz_p;
     int *lists = reinterpret_cast<int *>(p); p += sz_lists;
     int *counts = reinterpret_cast<int *>(p); p += sz_counts;
-    float *g = reinterpret_cast<float *>(p); p += sz_act;
-    float *u = reinterpret_cast<float *>(p); p += sz_act;
-    float *h = reinterpret_cast<float *>(p); p += sz_act;
+    float *g = reinterpret_cast<float *>(p); p += sz_gu;
+    float *u = reinterpret_cast<float *>(p); p += sz_gu;
+    float *h = reinterpret_cast<float *>(p); p += sz_h;
     float *yb = reinterpret_cast<float *>(p); p += sz_y;
-    float *part = sz_part ? reinterpret_cast<float *>(p) : nullptr; p += sz_part;
     char *xd_base = p; p += sz_xd;
     char *hd_base = p;
 
@@ -257,7 +406,7 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     const void **tab = nullptr;
     PG_TRY(pg_moe_cached_table(ctx, host_tab, 6 * E, &tab));
 
-    PG_TRY(pg_launch_moe_routing(ctx, router_logits_dev, idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, lists, counts));
+    PG_TRY(pg_launch_moe_routing(ctx, router_logits_dev, idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, lists, counts, nullptr, 1));
     auto table = [&](int which) { return reinterpret_cast<const uint8_t *const *>(tab + which * E); };
     auto dtable = [&](int which) { return reinterpret_cast<const uint16_t *const *>(tab + which * E); };
     // Each token reaches an expert at most once, so an expert owns at most T pairs.
@@ -272,26 +421,30 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     } else {
         const pg_mmdigits xd = pg_mmdigits_carve(xd_base, T, d);
         PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, T, d, type, xd));
-        const pg_mm_group gg = {(int)E, table(0), dtable(1), lists, counts, (int)T, tiles, (int)T, (int)top_k, 0, 0, 1};
-        PG_TRY(pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xd, g, part));
-        const pg_mm_group gu = {(int)E, table(2), dtable(3), lists, counts, (int)T, tiles, (int)T, (int)top_k, 0, 0, 1};
-        PG_TRY(pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gu, P, xd, u, part));
+        pg_mm_group gg = {(int)E, table(0), dtable(1), lists, counts, (int)T, tiles, (int)T, (int)top_k, 0, 0, 1};
+        gg.qs_table2 = table(2);  // gate and up in one launch
+        gg.d_table2 = dtable(3);
+        gg.out2 = u;
+        PG_TRY(pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xd, g, g, true));
     }
-    PG_TRY(pg_launch(ctx, "moe_act_mul", act_mul_kernel, dim3(grid_for(P * ffn, 256)), dim3(256), 0, g, u, P * ffn,
-                     act, h));
     if (down_stream) {
+        PG_TRY(pg_launch(ctx, "moe_act_mul", act_mul_kernel, dim3(grid_for(P * ffn, 256)), dim3(256), 0, g, u, P * ffn, act, h));
         const pg_xdigits hd = pg_xdigits_carve(hd_base, P, ffn);
         PG_TRY(pg_launch_x_to_digits(ctx, h, P, ffn, type, hd));
         const pg_gemv_batch bd = {(int)P, table(4), dtable(5), topk_idx, 1};
         PG_TRY(pg_launch_gguf_gemv(ctx, type, d, ffn, nullptr, nullptr, bd, hd, yb));
     } else {
         const pg_mmdigits hd = pg_mmdigits_carve(hd_base, P, ffn);
-        PG_TRY(pg_launch_x_to_mm_digits(ctx, h, P, ffn, type, hd));
+        const int nb = (int)(ffn / 32);
+        auto *kern = type == PG_GGML_Q4_0 ? act_mm_digits_kernel<true> : act_mm_digits_kernel<false>;
+        if (P > 65535) return pg_fail(PG_EUNSUPPORTED, "pg_moe_ffn: more than 65535 pairs");
+        PG_TRY(pg_launch(ctx, "moe_act_mm_digits", kern, dim3(grid_for(nb, 32), (unsigned)P), dim3(256), 0, (const float *)g, (const float *)u,
+                         ks_up, P * ffn, act, nb, (int)pg_round_up(nb, 4), hd.digits, hd.xs));
         const pg_mm_group gd = {(int)E, table(4), dtable(5), lists, counts, (int)T, tiles, (int)T, 1, 0, 0, 1};
-        PG_TRY(pg_launch_gguf_mm(ctx, type, d, ffn, nullptr, nullptr, gd, P, hd, yb, part));
+        PG_TRY(pg_launch_gguf_mm(ctx, type, d, ffn, nullptr, nullptr, gd, P, hd, yb, yb, true));
     }
-    return pg_launch(ctx, "moe_combine", combine_kernel, dim3(grid_for(T * d, 256)), dim3(256), 0, yb, topk_p, (int)T,
-                     (int)d, (int)top_k, shared_dev, out_dev);
+    return pg_launch(ctx, "moe_combine", combine_kernel, dim3(grid_for(T * d, 256)), dim3(256), 0, (const float *)yb, ks_down, P * d,
+                     (const float *)topk_p, (int)T, (int)d, (int)top_k, shared_dev, out_dev);
 }
 
 PG_API pg_status pg_moe_ffn_dev(pg_ctx *ctx, const float *x_dev, size_t T,

@@ -362,17 +362,6 @@ __device__ __forceinline__ int mt_expert_of(const mt_gather &g, int gt) {
     return lo;
 }
 
-// First token tile of every expert: goff[e] = sum over e' < e of ceil(counts[e'] / (16 tb)); goff[experts] = all.
-__global__ __launch_bounds__(64) void mxfp4_tile_offsets_kernel(const int *__restrict__ counts, int experts, int tb, int *__restrict__ goff) {
-    if (threadIdx.x != 0) return;
-    int run = 0;
-    for (int e = 0; e < experts; ++e) {
-        goff[e] = run;
-        run += (counts[e] + 16 * tb - 1) / (16 * tb);
-    }
-    goff[experts] = run;
-}
-
 // One thread = 16 consecutive k of one token (half a block).  A wavefront = the 16 tokens of a group x two blocks x
 // their halves, tokens on consecutive lanes: what it writes are whole 256-byte runs of the records, and the
 // 256 bytes it reads of every token row are two full lines.
@@ -1218,9 +1207,8 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     }
     const void **tab = nullptr;
     PG_TRY(pg_moe_cached_table(ctx, host_tab, 6 * E, &tab));
-    PG_TRY(pg_launch_moe_routing(ctx, nullptr, expert_idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, by_pairs ? nullptr : lists, counts));
-    if (!by_pairs)
-        PG_TRY(pg_launch(ctx, "mxfp4_tile_offsets", mxfp4_tile_offsets_kernel, dim3(1), dim3(64), 0, (const int *)counts, (int)E, tb, goff));
+    PG_TRY(pg_launch_moe_routing(ctx, nullptr, expert_idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, by_pairs ? nullptr : lists, counts,
+                                 goff, 16 * tb));
     const mt_gather gat = {lists, counts, goff, (int)T, (int)E, tb, 1};
     if (by_pairs)
         PG_TRY(moe_product_pairs(ctx, x_dev, T, hidden, 2 * inter, P, (int)top_k, tab, E, 0, topk_idx, h));

@@ -309,3 +309,36 @@ def test_moe_routed_argument_errors_and_device_entry_stays_in_bounds(ctx, orc):
     H.assert_close_rel(got[1], one_term[0], MOE_RTOL, "token with a doubled expert keeps the first mention")
     one_term = orc.moe_ffn_routed(x[2:3], 1, d, ffn, E, 1, np.array([[1]], np.int32), wt[2:3, :1], raws[0], raws[1], raws[2], typ, moe.SILU)
     H.assert_close_rel(got[2], one_term[0], MOE_RTOL, "token with an expert out of range keeps its valid term")
+
+
+@pytest.mark.parametrize("T,E,top_k,d,ffn,typ", [
+    (5, 3, 3, 160, 544, 8), (65, 1, 1, 192, 512, 2), (33, 16, 4, 544, 1056, 8),
+    (298, 40, 2, 160, 512, 8), (301, 40, 2, 160, 512, 8),      # the last size whose routing is one launch, and past it
+    (200, 256, 2, 160, 512, 2), (1030, 8, 2, 160, 512, 8),
+])
+def test_moe_routing_in_one_launch_and_split_products(ctx, orc, T, E, top_k, d, ffn, typ):
+    """Softmax, top-k and lists at the edges of the one-launch form; gate and up in one launch and products whose K chunks
+    the next launch adds.  Ties, infinite and NaN logits; the same routing handed in gives the same bits."""
+    from peregrine_amd import gguf, moe
+    say(f"moe routing T={T} E={E} top_k={top_k} typ={typ}")
+    distinct = min(E, 5)                       # (experts repeat: packing 256 of them would take minutes)
+    raws = build(orc, 30 + E, d, ffn, distinct, typ)
+    x = orc.rng_normal(T, T * d).reshape(T, d)
+    logits = orc.rng_normal(T + 1, T * E).reshape(T, E).copy()
+    logits[1] = 0.25                           # a full tie
+    logits[2, E // 2:] = -np.inf if E > 2 * top_k else logits[2, E // 2:]
+    logits[3, E - 1] = np.nan
+    mk = lambda rs, n_out, k_in: (lambda ws: [ws[e % distinct] for e in range(E)])([gguf.GgufWeight(r, typ, n_out, k_in, ctx) for r in rs])
+    ex = moe.MoEExperts(mk(raws[0], ffn, d), mk(raws[1], ffn, d), mk(raws[2], d, ffn), top_k, moe.SILU, ctx)
+    got = ex.forward(x, logits).reshape(T, d)
+    assert np.isnan(got[3]).all()
+    rows = [0, 1, 2] + list(range(4, T, max(1, T // 9))) + [T - 1]
+    full = [[r[e % distinct] for e in range(E)] for r in raws]
+    want, idx, prob = orc.moe_ffn(x[rows].reshape(-1), len(rows), d, ffn, E, top_k, logits[rows], full[0], full[1], full[2], typ, moe.SILU)
+    for j, t in enumerate(rows):
+        H.assert_close_rel(got[t], want[j], MOE_RTOL, f"token {t}")
+    keep = np.arange(T) != 3
+    _, idx, prob = orc.moe_ffn(np.zeros(keep.sum() * 32, np.float32), int(keep.sum()), 32, 32, E, top_k, logits[keep],
+                               *[[np.zeros(32 * 34, np.uint8)] * E] * 3, 8, moe.SILU)
+    again = ex.forward_routed(x[keep], idx, prob).reshape(-1, d)
+    H.assert_close_rel(again[:3], got[keep][:3], 1e-4, "the routing handed in")
