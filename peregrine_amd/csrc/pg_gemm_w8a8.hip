@@ -455,8 +455,8 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__res
 // ask the same memory channels at the same time: each starts at its own unit and wraps round its run (integer
 // sums do not depend on the order).  The epilogue is the reference's (acc as f32) * a_scale[m] * w_scale[n]
 // (src/quant.rs:163).  a_i8 has at least 16 MB rows of a_stride bytes (rows >= m feed accumulators never stored).
-// NB: tiles of 16 weight rows per workgroup (2 for more than 16 activation rows: every activation fragment then
-// meets two weight tiles, which halves what the CUs pull from L2).
+// NB: tiles of 16 weight rows per workgroup (with 2 every activation fragment meets two weight tiles, which halves what
+// the CUs pull from L2; the launcher says when).
 // Up to PG_GEMM_MAX_GROUP weights of equal K in one launch (the fused q|k|v and gate|up products of models::llama):
 // weight g owns the workgroups wg0[g] .. wg0[g + 1] - 1 (unused slots hold INT_MAX).
 struct skinny_wgroup {
@@ -699,17 +699,41 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         cols += w[i]->cols;
     }
     const size_t k_pad = w[0]->k_pad;
-    // Wavefronts per workgroup (K runs): as many as keep every workgroup resident at once -- a second round of
-    // workgroups would stream its weights after the first has drained.  The rings fill the CU's LDS: eight
-    // wavefronts a CU with 16 to 18 KiB each up to 32 rows, four with 30 to 36 KiB where four activation tiles or
-    // two weight tiles share a unit.  Two weight tiles a workgroup (more than 16 rows: halves what the CUs pull
-    // from L2 for the activations) pay while that still gives every CU a workgroup (32 rows, us: 4096 -> 14336
-    // 14.7 against 16.0, but 14336 -> 4096 20.0 against 16.0).
+    // Weight tiles a workgroup (NB), stages of a ring (NST) and wavefronts a workgroup (NW, its K runs).  What counts is that
+    // every workgroup is resident at once and that a CU has many units requested: two or three stages in more wavefronts
+    // beat four stages in fewer, and two weight tiles a workgroup (half the activations' way from L2) pay once 16-row
+    // workgroups are more than one a CU and their runs are not too short.  Drawn from 4500 shapes (m 2 .. 64, K 256 ..
+    // 10000, N 512 .. 16000, every shape that fits the LDS timed): against the rule before, which took four stages and
+    // wavefronts in powers of two up to the LDS of one or two tiles, 3.6 % (m <= 16), 6.3 % (m <= 32) and 13 % (m <= 64) on those
+    // over 8 us.  (us, before and now: 17 x 3412 -> 7951 12.0 / 10.6, 29 x 7580 -> 5374 19.9 / 16.7, 36 x 3853 -> 6403
+    // 17.9 / 13.7, 40 x 531 -> 8375 11.7 / 8.7, 12 x 7381 -> 5018 15.0 / 13.4.)
     const int mb = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
-    const int nb_tiles = (m > 16 && cols / 32 >= (size_t)ctx->num_cu) ? 2 : 1;
-    const int nst = mb == 1 ? 4 : (mb == 2 && nb_tiles == 2 ? 4 : 3);
-    const size_t ring = (size_t)nst * (nb_tiles + mb) * 2048;
-    const int per_cu = ring * 8 <= 160 * 1024 ? 8 : 4;
+    const size_t units = k_pad / 128, g16 = (cols + 15) / 16, cus = (size_t)ctx->num_cu;
+    struct shape { int nb, nst, nw; } sh = {1, mb == 1 ? 4 : 3, 0};
+    if (mb == 1) {
+        if (g16 > 3 * cus && units > 8) sh = {2, 3, 4};
+        else if (g16 > 2 * cus && units > 16) sh = {1, 2, 4};
+        else if (g16 > cus && units > 16) sh = {2, 3, 8};
+    } else if (mb == 2) {
+        if (units <= 8) sh = {1, 3, 2};
+        else if (g16 <= 2 * cus && units <= 16) sh = {1, 3, 4};
+        else if (g16 <= 3 * cus && units <= 16) sh = {1, 2, 4};
+        else if (g16 > 2 * cus) sh = {2, 2, 4};
+        else if (g16 > cus) sh = {2, 2, 8};
+    } else {
+        if (units <= 8) sh = {1, g16 > 2 * cus ? 2 : 3, 2};
+        else if (g16 > 2 * cus) sh = {2, 2, 3};
+        else if (g16 > cus) sh = {2, 3, 4};
+        else if (units <= 16) sh = {1, 3, 4};
+    }
+    if (sh.nw == 0) {  // the narrow ones: as many wavefronts as keep every workgroup resident, on runs of four units or more
+        const int per_cu = mb == 4 ? 4 : 8;
+        sh.nw = per_cu;
+        while (sh.nw > 1 && (g16 * sh.nw > cus * per_cu || units / sh.nw < 4)) sh.nw >>= 1;
+    } else if (2 * units < 3 * (size_t)sh.nw) {
+        sh.nw = 1;  // (two wavefronts want three units)
+    }
+    const int nb_tiles = sh.nb;
     skinny_wgroup grp;
     int wgs = 0;
     for (int i = 0; i < PG_GEMM_MAX_GROUP; ++i) {
@@ -722,37 +746,21 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         if (used) wgs += (int)((w[i]->cols + 16 * nb_tiles - 1) / (16 * nb_tiles));
     }
     const dim3 grid((unsigned)wgs);
-    const size_t slots = (size_t)ctx->num_cu * per_cu, units = k_pad / 128;
-    int nw = per_cu;
-    while (nw > 1 && ((size_t)grid.x * nw > slots || units / nw < 4)) nw >>= 1;
-#define PG_SKINNY_LAUNCH(MBB, NBB, NWW, NSTT)                                                                                \
-    do {                                                                                                                     \
-        auto kern = gemm_w8a8_skinny_kernel<MBB, NBB, NWW, NSTT>;                                                            \
-        const size_t lds = (size_t)NWW * NSTT * (NBB + MBB) * 2048;                                                          \
-        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                          \
+#define PG_SKINNY(MBB, NBB, NSTT, NWW)                                                                                        \
+    if (mb == MBB && sh.nb == NBB && sh.nst == NSTT && sh.nw == NWW) {                                                         \
+        auto kern = gemm_w8a8_skinny_kernel<MBB, NBB, NWW, NSTT>;                                                              \
+        const size_t lds = (size_t)NWW * NSTT * (NBB + MBB) * 2048;                                                            \
+        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
         return pg_launch(ctx, "gemm_w8a8_few_rows", kern, grid, dim3(64 * NWW), lds, a_i8, grp, (int)k_pad, (int)m, a_scales, acc, (size_t)0); \
-    } while (0)
-#define PG_SKINNY_NW8(MBB, NBB, NSTT)                       \
-    switch (nw) {                                           \
-        case 8: PG_SKINNY_LAUNCH(MBB, NBB, 8, NSTT);        \
-        case 4: PG_SKINNY_LAUNCH(MBB, NBB, 4, NSTT);        \
-        case 2: PG_SKINNY_LAUNCH(MBB, NBB, 2, NSTT);        \
-        default: PG_SKINNY_LAUNCH(MBB, NBB, 1, NSTT);       \
     }
-#define PG_SKINNY_NW4(MBB, NBB, NSTT)                       \
-    switch (nw) {                                           \
-        case 4: PG_SKINNY_LAUNCH(MBB, NBB, 4, NSTT);        \
-        case 2: PG_SKINNY_LAUNCH(MBB, NBB, 2, NSTT);        \
-        default: PG_SKINNY_LAUNCH(MBB, NBB, 1, NSTT);       \
-    }
-    if (mb == 1) PG_SKINNY_NW8(1, 1, 4)
-    if (mb == 2 && nb_tiles == 1) PG_SKINNY_NW8(2, 1, 3)
-    if (mb == 2) PG_SKINNY_NW4(2, 2, 4)
-    if (nb_tiles == 1) PG_SKINNY_NW4(4, 1, 3)
-    PG_SKINNY_NW4(4, 2, 3)
-#undef PG_SKINNY_NW8
-#undef PG_SKINNY_NW4
-#undef PG_SKINNY_LAUNCH
+    PG_SKINNY(1, 1, 4, 1) PG_SKINNY(1, 1, 4, 2) PG_SKINNY(1, 1, 4, 4) PG_SKINNY(1, 1, 4, 8)
+    PG_SKINNY(1, 1, 2, 4) PG_SKINNY(1, 2, 3, 4) PG_SKINNY(1, 2, 3, 8)
+    PG_SKINNY(2, 1, 3, 1) PG_SKINNY(2, 1, 3, 2) PG_SKINNY(2, 1, 3, 4) PG_SKINNY(2, 1, 3, 8)
+    PG_SKINNY(2, 1, 2, 4) PG_SKINNY(2, 2, 2, 4) PG_SKINNY(2, 2, 2, 8)
+    PG_SKINNY(4, 1, 3, 1) PG_SKINNY(4, 1, 3, 2) PG_SKINNY(4, 1, 3, 4)
+    PG_SKINNY(4, 1, 2, 1) PG_SKINNY(4, 1, 2, 2) PG_SKINNY(4, 2, 2, 3) PG_SKINNY(4, 2, 3, 4)
+#undef PG_SKINNY
+    return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8 (few rows in one launch): no kernel of %d tiles, %d stages, %d wavefronts", sh.nb, sh.nst, sh.nw);
 }
 
 pg_status pg_launch_gemm_w8a8_skinny(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,

@@ -605,3 +605,24 @@ def test_row_kernels_on_rows_of_any_length(ctx, orc, rows, cols):
     assert (got == ai.astype(np.int64) @ qi.astype(np.int64)).all()
     qt.free_gpu()
     qt_int.free_gpu()
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (2, 2176, 4112), (16, 4224, 8208), (16, 2176, 12304), (5, 1152, 12304), (16, 1024, 12304),   # one tile of rows
+    (17, 1024, 4096), (32, 300, 700), (19, 128, 520), (17, 1153, 8192), (32, 2048, 8208), (20, 2176, 4112), (32, 2176, 12290),
+    (33, 1024, 8208), (64, 1000, 8192), (40, 130, 700), (48, 2048, 4112), (64, 4200, 8208), (33, 1536, 4000),
+])
+def test_few_rows_launch_shapes_bit_exact(ctx, orc, m, k, n):
+    """Both sides of every line of the few-row launch's rule (16-row weight tiles against CUs, units of K), with ragged
+    rows, K and columns.  The integers are exact in f64 and the scales are applied in one order, so the bits are determined."""
+    from peregrine_amd import quant
+    say(f"few rows m={m} k={k} n={n}")
+    rng = np.random.default_rng(m * 7 + k + n)
+    qt = quant.quantize_weights(rng.uniform(-0.05, 0.05, (k, n)).astype(np.float32), k, n, ctx)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, ::53] *= 20.0
+    q, s = orc.quantize_activations(a, m, k)
+    acc = np.asarray(q, np.float64).reshape(m, k) @ np.asarray(qt.data_i8, np.float64).reshape(k, n)
+    want = acc.astype(np.float32) * np.asarray(s, np.float32)[:, None] * np.asarray(qt.scales, np.float32)[None, :]
+    got = np.asarray(quant.matmul_quantized(a, m, k, qt, ctx), np.float32).reshape(m, n)
+    assert (bits(got) == bits(want)).all()
