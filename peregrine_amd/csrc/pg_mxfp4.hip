@@ -17,6 +17,7 @@
 // j of a row is one column of B with block scale byte 127 + se + 5 j, so the instruction itself applies
 // both block scales and sums over K; the five columns of a row are added at the end.  Three activation
 // rows (15 columns) share one pass over the weights.
+#include <math.h>
 #include "pg_internal.h"
 #include "pg_stream_addr.h"
 #include "pg_digits.h"
@@ -1138,6 +1139,19 @@ pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, 
 #undef PG_MTG
 }
 
+// Whether up to 64 pairs are faster one by one than as tiles although pairs share experts (P > 2 E): the decode kernel streams an
+// expert's 3 * hidden * inter FP4 weights per pair at 6.2 TB/s over 15 us of launches, the tiles stream those of the
+// experts that T tokens are expected to hit at 5.2 over 27, but at least the walk of one row tile through both K.
+// (us, pairs against tiles: 8 experts of 960, top 2, 16 tokens 22.0 / 28.2; of 1440, top 4, 6 tokens 28.8 / 34.3, 8 tokens
+// 33.1 / 33.8, 10 tokens 37.3 / 32.2; of 2880, top 2, 10 tokens 60.1 / 47.3.)
+bool pairs_faster(size_t T, size_t E, size_t top_k, size_t hidden, size_t inter) {
+    const double us_per_expert = 3.0 * (double)hidden * (double)inter * (17.0 / 32.0) / 1e6;  // at 1 TB/s
+    const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));
+    const double pairs = 15.0 + (double)(T * top_k) * us_per_expert / 6.2;
+    const double tiles = std::max(20.0 + 0.00415 * (double)(hidden + inter), 27.0 + hit * us_per_expert / 5.2);
+    return pairs < tiles;
+}
+
 // The same product pair by pair on the decode kernel (few pairs).
 bool pairs_fit(int ncp) { return mx_lds_bytes(1, ncp) <= (160u << 10); }
 pg_status moe_product_pairs(pg_ctx *ctx, const float *src, size_t src_rows, size_t k_in, size_t n_out, size_t pairs, int div,
@@ -1181,7 +1195,7 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     const int ncp1 = (int)mx_chunks(hidden / 32), ncp2 = (int)mx_chunks(inter / 32);
     // With few pairs hardly two of them meet in an expert, and a pair is a one-row product: the decode kernel, one
     // workgroup column per pair (exact activations; no expert lists).  Otherwise the experts' token tiles on the tile kernel.
-    const bool by_pairs = P <= 2 * E && P <= 64 && pairs_fit(ncp1) && pairs_fit(ncp2);
+    const bool by_pairs = P <= 64 && (P <= 2 * E || pairs_faster(T, E, top_k, hidden, inter)) && pairs_fit(ncp1) && pairs_fit(ncp2);
     const size_t sz_idx = pg_round_up(P * sizeof(int), 256), sz_p = pg_round_up(P * sizeof(float), 256);
     const size_t sz_lists = pg_round_up(E * T * sizeof(int), 256), sz_counts = pg_round_up((2 * E + 1) * sizeof(int), 256);
     const size_t sz_rec = pg_round_up(max_tiles * tb * (size_t)std::max(ncp1, ncp2) * MT_RECORD, 256);
