@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     float *__restrict__ out = out_arg;
     const uint8_t *const *qs_table = grp.qs_table;
     const uint16_t *const *d_table = grp.d_table;
-    if (grp.qs_table2 && bx >= (n_out_arg + 127) / 128) {  // the expert's second tensor
+    if (grp.nseg < 0 && bx >= (n_out_arg + 127) / 128) {  // the expert's second tensor
         bx -= (n_out_arg + 127) / 128;
         qs_table = grp.qs_table2;
         d_table = grp.d_table2;
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const uint8_t *qs_any = qs_table ? qs_table[e] : qs0;
     const uint16_t *d_any = d_table ? d_table[e] : d0;
     size_t part_stride = part_stride_arg;
-    if (grp.nseg) {  // which tensor of the launch this row group belongs to
+    if (grp.nseg > 0) {  // which tensor of the launch this row group belongs to
         int t = 0;
         while (t + 1 < grp.nseg && bx >= grp.seg_first[t + 1]) ++t;
         bx -= grp.seg_first[t];
@@ -656,10 +656,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // wg0[g] .. wg0[g + 1] - 1 (unused slots hold INT_MAX).
 // Q41 (with QT = 4): Q4_1, whose value q d + m is (q - 8) d + (8 d + m): besides the Q4_0 product every block adds
 // 8 d + m times the block's plain sum of x, one FMA more per output; a unit holds the blocks' f16 m and the tokens' block sums too.
+// Q4_1's offsets and block sums are arguments of its kernels alone: in everybody's they cost the other formats 0.1 to 0.5 us
+// a launch (two rows of a Q8_0 block's gate|up 7.6 -> 8.1 us).
+template <bool Q41> struct skinny_args : pg_skinny_group {
+    void set(const pg_gguf_tensor *const *, int, const pg_mmdigits &) {}
+};
+template <> struct skinny_args<true> : pg_skinny_group {
+    const uint16_t *mo[3];
+    const float *xsum;
+    void set(const pg_gguf_tensor *const *w, int count, const pg_mmdigits &md) {
+        for (int i = 0; i < 3; ++i) mo[i] = i < count ? w[i]->m : nullptr;
+        xsum = md.xsum;
+    }
+};
+
 template <int QT, int NB, int MT, int NW, int NST, bool Q41 = false>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <= 8 ? 4 : 2))) void gguf_skinny_kernel(const pg_skinny_group grp, int nb, int nbp, int m,
-                                                                    const int8_t *__restrict__ digits, const float *__restrict__ xs,
-                                                                    const float *__restrict__ xsum) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <= 8 ? 4 : 2))) void gguf_skinny_kernel(const skinny_args<Q41> grp, int nb, int nbp, int m,
+                                                                    const int8_t *__restrict__ digits, const float *__restrict__ xs) {
     int tg = 0;
 #pragma unroll
     for (int i = 1; i < 3; ++i) tg = (int)blockIdx.x >= grp.wg0[i] ? i : tg;
@@ -697,7 +710,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     const int ntile = (n_out + 7) / 8;
     const int dt = pg_gskinny_scale_tile(n0, lane, ntile);
     const char *d_src = reinterpret_cast<const char *>(dsc) + pg_gskinny_scale_offset(dt, nb, 0, lane);
-    const char *ms_src = Q41 ? reinterpret_cast<const char *>(grp.mo[tg]) + pg_gskinny_scale_offset(dt, nb, 0, lane) : nullptr;
+    const char *ms_src = nullptr;  // Q4_1: the blocks' offsets
+    if constexpr (Q41) ms_src = reinterpret_cast<const char *>(grp.mo[tg]) + pg_gskinny_scale_offset(dt, nb, 0, lane);
     // digits: instruction q covers runs 4 q .. 4 q + 3, run = 2 token + plane; lane -> run 4 q + lane / 16, position lane % 16
     const int8_t *g_src[GQ];
 #pragma unroll
@@ -708,7 +722,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     }
     // token scales: lanes 0 .. 2 MT - 1: token lane / 2, blocks 4 (lane % 2) .. + 3 of the unit
     const float *x_src = xs + (size_t)((lane >> 1) < m ? (lane >> 1) : 0) * nbp + 4 * (lane & 1);
-    const float *sum_src = Q41 ? xsum + (x_src - xs) : nullptr;
+    const float *sum_src = nullptr;
+    if constexpr (Q41) sum_src = grp.xsum + (x_src - xs);
 
     const int rot = cnt > 0 ? (int)((blockIdx.x * 5u) % (unsigned)cnt) : 0;
     auto issue = [&](auto slot, int t) {
@@ -1130,7 +1145,6 @@ pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, c
         const bool used = i < count;
         grp.qs[i] = used ? w[i]->qs : nullptr;
         grp.d[i] = used ? w[i]->d : nullptr;
-        grp.mo[i] = used ? w[i]->m : nullptr;
         grp.y[i] = used ? y[i] : nullptr;
         grp.res[i] = i == 0 ? residual : nullptr;
         grp.n[i] = used ? (int)w[i]->n_out : 0;
@@ -1150,10 +1164,13 @@ pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, c
 #define PG_GSK_LAUNCH(QTT, NBB, MTT, NWW, NSTT)                                                                                \
     do {                                                                                                                       \
         auto kern = gguf_skinny_kernel<QTT == 8 ? 8 : 4, NBB, MTT, NWW, NSTT, QTT == 5>;                                       \
+        skinny_args<QTT == 5> args;                                                                                            \
+        static_cast<pg_skinny_group &>(args) = grp;                                                                            \
+        args.set(w, count, md);                                                                                                \
         const size_t lds = (size_t)NWW * NSTT * (NBB * ((QTT == 8 ? 4096 : 2048) + (QTT == 5 ? 512 : 256)) + MTT * 512 + (QTT == 5 ? 1024 : 512)); \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
         return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_few_rows_mm" : (QTT == 5 ? "gguf_q4_1_few_rows_mm" : "gguf_q4_0_few_rows_mm"), kern, grid, \
-                         dim3(64 * NWW), lds, grp, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs, (const float *)md.xsum); \
+                         dim3(64 * NWW), lds, args, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs); \
     } while (0)
 #define PG_GSK_NW8(QTT, NBB, MTT, NSTT)                     \
     switch (nw) {                                           \
@@ -1195,11 +1212,11 @@ pg_status pg_launch_gguf_mm(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_i
     const size_t gy = experts * (size_t)grp.tiles_per_expert;
     // token tiles that certainly hold work: all of them without expert lists, one per expert with
     bool by_xcd = false;
-    const bool second = grp.qs_table2 != nullptr;
+    const bool second = grp.nseg < 0;
     if (second && (!grp.counts || !keep_parts)) return pg_fail(PG_EINVAL, "gguf_mm: a second tensor per expert needs expert lists and leaves its K chunks unsummed");
     const int ks = pg_gguf_mm_splitk(ctx, second ? pg_mm_pair_rows(n_out) : n_out, k_in, grp.counts ? experts : gy, md.rows, grp.counts != nullptr, &chunk, &by_xcd);
     if (ks > 1 && !part) return pg_fail(PG_EINVAL, "gguf_mm: split-K needs a partial-sum buffer");
-    if (grp.nseg && ((ks > 1 && !keep_parts) || grp.counts || !grp.tiled))
+    if (grp.nseg > 0 && ((ks > 1 && !keep_parts) || grp.counts || !grp.tiled))
         return pg_fail(PG_EINVAL, "gguf_mm: several tensors in one launch leave their K chunks unsummed, take no expert lists and read tile-major copies");
     if (gy > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_mm: too many token tiles");
     dim3 grid(grid_for(n_out, 128) * (second ? 2 : 1), (unsigned)gy, (unsigned)ks);

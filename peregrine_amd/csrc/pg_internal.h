@@ -366,7 +366,6 @@ bool pg_gguf_skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_o
 struct pg_skinny_group {  // the tensors of one few-rows launch (gguf_skinny_kernel)
     const uint8_t *qs[3];
     const uint16_t *d[3];
-    const uint16_t *mo[3];  // Q4_1 only: the blocks' offsets
     float *y[3];
     const float *res[3];  // where set: y = res + product (same shape as y)
     int n[3];
@@ -401,17 +400,24 @@ struct pg_mm_group {
     // Several tensors of equal K in one launch (q|k|v, gate|up): the launch's 128-row groups are the tensors'
     // groups one after the other; tensor t starts at group seg_first[t], has seg_n[t] rows, its own tile-major
     // copy, scales and output (planes seg_stride[t] floats apart).  nseg = 0: the one tensor of the arguments.
+    // nseg = -1: a second tensor per expert of the same shape (gate and up in one launch); its 128-row groups follow the first
+    // ones', its planes go to out2, as far apart as the first ones'.  (In the segments' place: a launch's arguments are
+    // read by every workgroup, and 24 bytes more of them can be measured.)
     int nseg;
     int seg_first[3], seg_n[3];
-    const uint8_t *seg_qs[3];
-    const uint16_t *seg_d[3];
+    union {
+        struct {
+            const uint8_t *seg_qs[3];
+            const uint16_t *seg_d[3];
+        };
+        struct {
+            const uint8_t *const *qs_table2;
+            const uint16_t *const *d_table2;
+            float *out2;
+        };
+    };
     float *seg_out[3];
     size_t seg_stride[3];
-    // A second tensor per expert of the same shape (gate and up in one launch): its 128-row groups follow the first
-    // ones', its planes go to out2, as far apart as the first ones'.
-    const uint8_t *const *qs_table2;
-    const uint16_t *const *d_table2;
-    float *out2;
 };
 // Rows of a launch over two tensors of n_out rows each (whole 128-row groups).
 inline size_t pg_mm_pair_rows(size_t n_out) { return 2 * pg_round_up(n_out, 128); }

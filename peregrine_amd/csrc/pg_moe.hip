@@ -422,7 +422,8 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
         const pg_mmdigits xd = pg_mmdigits_carve(xd_base, T, d);
         PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, T, d, type, xd));
         pg_mm_group gg = {(int)E, table(0), dtable(1), lists, counts, (int)T, tiles, (int)T, (int)top_k, 0, 0, 1};
-        gg.qs_table2 = table(2);  // gate and up in one launch
+        gg.nseg = -1;  // gate and up in one launch
+        gg.qs_table2 = table(2);
         gg.d_table2 = dtable(3);
         gg.out2 = u;
         PG_TRY(pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xd, g, g, true));
