@@ -159,3 +159,12 @@ def test_audit_argument_errors():
         check(lib.pg_audit_gemv_w8a8_m1(4096, 16, 1, 1, 4, 0, *[C.byref(x) for x in v]))   # NCH too small for the row
     with pytest.raises(_ffi.PeregrineError):
         check(lib.pg_audit_gguf_skinny(16, 1000, 0, 4, 1, *[C.byref(x) for x in v]))          # K not a multiple of 256
+
+
+def test_few_rows_w8a8_fills_of_the_wide_launch_shapes():
+    """The shapes of the few-row rule that the test above does not name: two weight tiles for one tile of rows, three wavefronts."""
+    for (mb, nbt, nw), k, n in itertools.product([(1, 2, 4), (1, 2, 8), (4, 2, 3)], [128, 1152, 1300, 4224], RAGGED_N + [8200]):
+        for m in {2, 16 * mb - 15, 16 * mb} - {1}:
+            v = _four()
+            check(lib.pg_audit_gemm_w8a8_skinny(m, k, n, mb, nbt, nw, *[C.byref(x) for x in v]))
+            _inside(v, f"gemm_w8a8_skinny m={m} k={k} n={n} MB={mb} NB={nbt} NW={nw}")
