@@ -980,7 +980,8 @@ def section_moe(B, line):
     hit = int(torch.unique(torch.topk(lg_moe, topk_moe, dim=1).indices).numel())
     t_moe = B.timed(moe_step, 20, 10)  # 5 GB of weights: the first passes also warm the TLBs
     prof, grids = B.profiled(moe_step, 5)
-    mm_total = prof["gguf_mm_q8_0"][0] * prof["gguf_mm_q8_0"][1] / 5  # three launches per step
+    mm_launches = prof["gguf_mm_q8_0"][1] / 5  # gate and up together, down
+    mm_total = prof["gguf_mm_q8_0"][0] * mm_launches
     line["moe_q8_0"] = {
         "workload": "cfg5: Grok-1-shaped MoE FFN, Q8_0 experts (d 6144, ffn 32768, 8 experts, top-2, 64 tokens, SiLU); "
                     "5.13 GB of expert weights, read once per step",
@@ -988,10 +989,10 @@ def section_moe(B, line):
         "frac_of_hbm_peak": round(moe_bytes / (t_moe["ms_per_step"] * 1e-3) / 1e9 / PEAK_HBM_GBS, 4), **B.stats(t_moe, 4),
         "tflops": round(2 * T_moe * topk_moe * 3 * ffn_moe * d_moe / (t_moe["ms_per_step"] * 1e-3) / 1e12, 2),
         "kernels_ms": {k: round(v[0], 5) for k, v in prof.items()},
-        "roofline": {"kernel": "gguf_mm_kernel<Q8_0> (gate, up, down)", "bound": "hbm",
+        "roofline": {"kernel": "gguf_mm_kernel<Q8_0> (gate|up, down)", "bound": "hbm",
                      "achieved": round(3 * E_moe * nblk * 34 / (mm_total * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS,
                      "unit": "GB/s", "frac": round(3 * E_moe * nblk * 34 / (mm_total * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
-                     "traffic": B.traffic_for("gguf_mm_q8_0", grids), "bytes_per_launch": E_moe * nblk * 34,
+                     "traffic": B.traffic_for("gguf_mm_q8_0", grids), "bytes_per_launch": int(3 * E_moe * nblk * 34 / mm_launches),
                      "avg_launch_ms": round(prof["gguf_mm_q8_0"][0], 5)}}
     for w3 in experts:
         for h in w3:
