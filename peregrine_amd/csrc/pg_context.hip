@@ -33,6 +33,13 @@ pg_status pg_use(pg_ctx *ctx) {
     return PG_OK;
 }
 
+pg_status pg_refuse_capture(pg_ctx *ctx, const char *what) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) (void)hipGetLastError();
+    if (st != hipStreamCaptureStatusNone) return pg_fail(PG_EDEVICE, "%s: not permitted while the stream is capturing", what);
+    return PG_OK;
+}
+
 pg_status pg_launch_check(const char *what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return pg_fail(PG_EDEVICE, "launch of %s failed: %s", what, hipGetErrorString(e));
@@ -81,6 +88,7 @@ void pg_dev_pool::drain(bool close) {
 }
 
 pg_status pg_dev_block::alloc(pg_ctx *ctx, size_t want) {
+    PG_TRY(pg_refuse_capture(ctx, "device memory"));
     release();
     // to the next sixteenth of a power of two, so that objects of nearly one size can take each other's blocks
     size_t unit = 4096;

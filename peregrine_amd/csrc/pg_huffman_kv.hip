@@ -1114,10 +1114,17 @@ static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c) {
     return st;
 }
 
+// Whether an append of seq_len tokens cuts a chunk: the host reads its size, which a capturing stream refuses -- ahead of the
+// append to the window, so that nothing has changed then.
+static pg_status append_ok(pg_ctx *ctx, const pg_huffman_kv_cache *c, size_t seq_len) {
+    return c->hot->len + seq_len < c->compress_threshold ? PG_OK : pg_refuse_capture(ctx, "pg_huffman_kv_cache_append: a chunk");
+}
+
 PG_API pg_status pg_huffman_kv_cache_append_dev(pg_ctx *ctx, pg_huffman_kv_cache *c, const float *new_k_dev,
                                                 const float *new_v_dev, size_t seq_len) {
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(c != nullptr, "pg_huffman_kv_cache_append: null cache");
+    PG_TRY(append_ok(ctx, c, seq_len));
     c->touch(ctx);
     PG_TRY(pg_kv_cache_append_dev(ctx, c->hot, new_k_dev, new_v_dev, seq_len));
     return compress_hot(ctx, c);
@@ -1127,6 +1134,7 @@ PG_API pg_status pg_huffman_kv_cache_append(pg_ctx *ctx, pg_huffman_kv_cache *c,
                                             size_t seq_len) {
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(c != nullptr, "pg_huffman_kv_cache_append: null cache");
+    PG_TRY(append_ok(ctx, c, seq_len));
     c->touch(ctx);
     PG_TRY(pg_kv_cache_append(ctx, c->hot, new_k, new_v, seq_len));
     return compress_hot(ctx, c);

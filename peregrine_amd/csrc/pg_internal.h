@@ -32,7 +32,9 @@ struct pg_prof_total {
 // Device blocks that objects of a context gave back and later ones may take (hipMalloc and hipFree cost 6 and 10 us a
 // call and hipFree waits for the device).  A block from the pool is used on the context's stream alone, so whoever
 // takes it next is ordered behind whoever had it; an object that another context has touched gives its memory to
-// hipFree instead.  At most PG_POOL_BYTES lie here; the context's end, or memory running out, empties it.
+// hipFree instead.  At most PG_POOL_BYTES lie here; the context's end, or memory running out, empties it.  While the
+// stream captures, a block is refused whether the pool holds one or not (as hipMalloc refuses it): replays would go on
+// using an address that its object may have given back by then.
 constexpr size_t PG_POOL_BYTES = 256u << 20;
 struct pg_dev_pool {
     std::mutex mu;
@@ -170,6 +172,8 @@ pg_status pg_fail(pg_status st, const char *fmt, ...) __attribute__((format(prin
 
 // Make ctx's device current for the calling thread.
 pg_status pg_use(pg_ctx *ctx);
+// PG_EDEVICE while ctx's stream captures: for calls that take memory or hand the host a result.
+pg_status pg_refuse_capture(pg_ctx *ctx, const char *what);
 // Scratch arena of at least `bytes` (256-byte aligned); contents undefined.
 pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out);
 // Pinned host memory of at least `bytes` (the context's one block; contents undefined).  The caller has waited for

@@ -1712,7 +1712,8 @@ __global__ __launch_bounds__(256) void kv_rows_kernel(T *dst_k, T *dst_v, size_t
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < width; i += (size_t)gridDim.x * 256) d[i] = s[i];
 }
 
-// Room for `needed` positions per head; grows like the reference (at least double, from 16).
+// Room for `needed` positions per head; grows like the reference (at least double, from 16).  A capturing stream refuses
+// the growth, before anything is launched or changed.
 pg_status cache_reserve(pg_ctx *ctx, pg_kv_cache *c, size_t needed) {
     if (needed <= c->capacity) return PG_OK;
     const size_t grown = (c->capacity > 16 ? c->capacity : 16) * 2;
@@ -2188,7 +2189,6 @@ static pg_status block_forward_one_token(pg_ctx *ctx, pg_llama_block *b, const f
         PG_TRY(pg_launch_gguf_gemv(ctx, b->w[1]->ggml_type, kv_dim, d, b->w[1]->qs, b->w[1]->d, one, b->xd_d, kd));
         PG_TRY(pg_launch_gguf_gemv(ctx, b->w[2]->ggml_type, kv_dim, d, b->w[2]->qs, b->w[2]->d, one, b->xd_d, vd));
     }
-    PG_TRY(cache_reserve(ctx, cache, offset + 1));
     if (attention_is_short(ctx, b->nqh, offset + 1, hd)) {
         // RoPE of q and of the new key, and the append of the new key and value, happen inside
         // the attention kernel: one launch less.
@@ -2340,7 +2340,6 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
 
     PG_TRY(norm_digits(h_dev, -1, nullptr, b->attn_norm_w, hm[0]));
     PG_TRY(product(0, md_d));
-    PG_TRY(cache_reserve(ctx, cache, offset + seq));
     rope_args ra = {};
     ra.seg[0] = {part(0), q_rope, q_dim, seq * hd, (int)b->nqh, 1, ks[0], seq * q_dim};
     ra.seg[1] = {part(1), cache->k + offset * hd, kv_dim, cache->capacity * hd, (int)b->nkvh, 1, ks[1], seq * kv_dim};
@@ -2408,6 +2407,7 @@ PG_API pg_status pg_llama_block_forward_dev(pg_ctx *ctx, pg_llama_block *b, cons
         PG_HIP(hipMalloc(reinterpret_cast<void **>(&b->arena), floats * sizeof(float)));
         b->seq_cap = cap;
     }
+    PG_TRY(cache_reserve(ctx, cache, offset + seq));  // (ahead of every launch: a step that a capture refuses leaves nothing in the graph)
     const size_t cap = b->seq_cap;
     if (seq == 1 && b->digit_kind != 0 && hd % 32 == 0 && d <= 8192 && (uintptr_t)h_dev % 16 == 0)
         return block_forward_one_token(ctx, b, h_dev, cache, out_dev);
@@ -2425,7 +2425,6 @@ PG_API pg_status pg_llama_block_forward_dev(pg_ctx *ctx, pg_llama_block *b, cons
     PG_TRY(launch_rmsnorm(ctx, h_dev, nullptr, nullptr, b->attn_norm_w, b->eps, seq, d, normed));
     float *const qkv[3] = {qd, kd, vd};
     PG_TRY(pg_gguf_matmul_rows_multi(ctx, normed, seq, b->w, qkv, 3));
-    PG_TRY(cache_reserve(ctx, cache, offset + seq));
     rope_args ra = {};
     ra.seg[0] = {qd, q_rope, q_dim, seq * hd, (int)b->nqh, 1};
     ra.seg[1] = {kd, cache->k + offset * hd, kv_dim, cache->capacity * hd, (int)b->nkvh, 1};

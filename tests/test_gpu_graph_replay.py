@@ -218,3 +218,37 @@ def test_mxfp4_products_and_moe_replayed_from_a_graph(ctx, orc):
     w.free()
     for e in experts:
         e.free()
+
+
+def test_cache_growth_inside_a_capture_is_refused(ctx, orc):
+    """A cache that would have to grow is refused by the capturing stream also when the context's pool holds blocks of
+    the grown size; the capture stays whole, the cache as it was, and the eager append afterwards grows it."""
+    from peregrine_amd import _ffi
+    hip, lib = Hip(), _ffi.lib
+    heads, hd = 2, 64
+    rows = DevBuf(ctx, host=orc.rng_normal(80, heads * hd * 64))
+
+    def cache(tokens):
+        h = C.c_void_p()
+        _ffi.check(lib.pg_kv_cache_create(ctx.handle, heads, hd, C.byref(h)))
+        _ffi.check(lib.pg_kv_cache_append_dev(ctx.handle, h, rows.ptr, rows.ptr, tokens))
+        return h
+
+    c = cache(32)
+    lib.pg_kv_cache_free(ctx.handle, cache(64))
+    status = []
+    say("capturing an append that would grow its cache")
+    graph, ex = hip.capture(ctx.stream, lambda: status.append(lib.pg_kv_cache_append_dev(ctx.handle, c, rows.ptr, rows.ptr, 1)))
+    hip.lib.hipGraphExecDestroy(ex)
+    hip.lib.hipGraphDestroy(graph)
+    assert status == [_ffi.PG_EDEVICE] and lib.pg_kv_cache_len(c) == 32 and lib.pg_kv_cache_capacity(c) == 32
+    _ffi.check(lib.pg_kv_cache_append_dev(ctx.handle, c, rows.ptr, rows.ptr, 1))
+    assert lib.pg_kv_cache_capacity(c) == 64
+    k = np.empty(heads * 33 * hd, np.float32)
+    v = np.empty_like(k)
+    _ffi.check(lib.pg_kv_cache_download(ctx.handle, c, C.c_void_p(k.ctypes.data), C.c_void_p(v.ctypes.data)))
+    src = rows.to_host(np.float32)
+    for h in range(heads):   # an append's rows are [heads][tokens][head_dim]
+        want = np.concatenate([src[h * 32 * hd : (h + 1) * 32 * hd], src[h * hd : (h + 1) * hd]])
+        assert (k[h * 33 * hd : (h + 1) * 33 * hd] == want).all() and (v[h * 33 * hd : (h + 1) * 33 * hd] == want).all()
+    lib.pg_kv_cache_free(ctx.handle, c)

@@ -1,0 +1,140 @@
+"""What the library does around its launches, followed without a GPU: the library's own objects, linked with a HIP runtime
+on host memory that notes kernels instead of running them (tests/cpp/host_runtime.cpp).  Nothing here looks at a computed
+number."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import helpers as H
+
+CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+LIB = os.path.join(CPP, "_build", "libperegrine_host.so")
+
+
+class Host:
+    """The library on the host runtime, one context to begin with."""
+
+    def __init__(self):
+        from peregrine_amd import _ffi
+        if not os.path.exists(LIB):
+            subprocess.check_call(["make", "-C", CPP])
+        self.lib = C.CDLL(LIB)
+        for name, args in _ffi.SIGNATURES.items():
+            fn = getattr(self.lib, name)
+            fn.argtypes, fn.restype = args, _ffi._OTHER_RESTYPE.get(name, C.c_int)
+        for name in ("pghost_used", "pghost_frees", "pghost_bad_frees", "pghost_recorded", "pghost_num_launches"):
+            getattr(self.lib, name).restype = C.c_size_t
+        self.lib.pghost_limit.argtypes = [C.c_size_t]
+        self.lib.pghost_limit.restype = self.lib.pghost_clear_launches.restype = self.lib.pghost_begin_capture.restype = None
+        self.lib.pghost_begin_capture.argtypes = self.lib.pghost_end_capture.argtypes = [C.c_void_p]
+        self.lib.pghost_launch.argtypes, self.lib.pghost_launch.restype = [C.c_size_t, C.POINTER(C.c_uint)], C.c_char_p
+        self.ctx = self.new("pg_ctx_create", 0, None)
+
+    def ok(self, name, *args):
+        st = getattr(self.lib, name)(*args)
+        assert st == 0, (name, st, self.lib.pg_last_error())
+
+    def new(self, name, *args):
+        h = C.c_void_p()
+        self.ok(name, *args, C.byref(h))
+        return h
+
+    def alloc(self, floats):
+        return self.new("pg_dev_alloc", self.ctx, floats * 4)
+
+    def stream(self, ctx=None):
+        return self.lib.pg_ctx_stream(ctx or self.ctx)
+
+    def launches(self):
+        grid, out = (C.c_uint * 3)(), []
+        for i in range(self.lib.pghost_num_launches()):
+            name = self.lib.pghost_launch(i, grid)
+            out.append((name.decode(), tuple(grid)))
+        return out
+
+    def captured(self, fn, *args):
+        """fn's status on a capturing stream, what the capture recorded, and whether it is still whole."""
+        self.lib.pghost_begin_capture(self.stream())
+        st = getattr(self.lib, fn)(*args)
+        recorded = self.lib.pghost_recorded()
+        return st, recorded, bool(self.lib.pghost_end_capture(self.stream()))
+
+    def cache(self, heads, hd, tokens, ctx=None):
+        c = self.new("pg_kv_cache_create", ctx or self.ctx, heads, hd)
+        if tokens:
+            rows = self.alloc(heads * hd * tokens)
+            self.ok("pg_kv_cache_append_dev", ctx or self.ctx, c, rows, rows, tokens)
+        return c
+
+    def gguf(self, n, k):
+        return self.new("pg_gguf_upload", self.ctx, bytes(H.pack_q4_0(np.zeros(n * k, np.float32))), 2, n, k)
+
+
+@pytest.fixture()
+def host():
+    h = Host()
+    h.lib.pghost_limit(C.c_size_t(-1).value)
+    h.lib.pghost_clear_launches()
+    yield h
+    assert h.lib.pghost_bad_frees() == 0
+    h.lib.pg_ctx_destroy(h.ctx)
+
+
+def test_cache_growth_is_refused_by_a_capture_whatever_the_pool_holds(host):
+    heads, hd = 2, 64
+    c = host.cache(heads, hd, 32)
+    host.lib.pg_kv_cache_free(host.ctx, host.cache(heads, hd, 64))     # two blocks of the grown size in the pool
+    row = host.alloc(heads * hd)
+    st, recorded, whole = host.captured("pg_kv_cache_append_dev", host.ctx, c, row, row, 1)
+    assert st == 2 and b"captur" in host.lib.pg_last_error() and recorded == 0 and whole
+    assert host.lib.pg_kv_cache_len(c) == 32 and host.lib.pg_kv_cache_capacity(c) == 32
+    host.ok("pg_kv_cache_append_dev", host.ctx, c, row, row, 1)        # eagerly it grows
+    assert host.lib.pg_kv_cache_capacity(c) == 64
+    st, recorded, whole = host.captured("pg_kv_cache_append_dev", host.ctx, c, row, row, 1)
+    assert st == 0 and recorded == 1 and whole                         # with room there, it is one launch
+    host.lib.pg_kv_cache_free(host.ctx, c)
+
+
+@pytest.mark.parametrize("seq", [1, 4, 40])
+def test_block_step_that_grows_its_cache_is_refused_by_a_capture(host, seq):
+    d, nqh, nkvh, hd, ffn = 256, 4, 2, 64, 512
+    shapes = [(nqh * hd, d), (nkvh * hd, d), (nkvh * hd, d), (d, nqh * hd), (ffn, d), (ffn, d), (d, ffn)]
+    ws = [host.gguf(n, k) for n, k in shapes]
+    b = host.new("pg_llama_block_create", host.ctx, d, nqh, nkvh, hd, ffn, 512, 10000.0, 1e-5)
+    norm = np.ones(d, np.float32)
+    host.ok("pg_llama_block_set_weights", host.ctx, b, *ws, norm.ctypes.data, norm.ctypes.data)
+    x, out = host.alloc(64 * d), host.alloc(64 * d)
+    c = host.cache(nkvh, hd, 32)
+    host.ok("pg_kv_cache_append_dev", host.ctx, c, x, x, 32)             # (room for 64)
+    host.ok("pg_kv_cache_rollback_to", c, 64 - seq)
+    host.ok("pg_llama_block_forward_dev", host.ctx, b, x, seq, c, out)   # every buffer of the step exists now; the cache is full
+    assert host.lib.pg_kv_cache_len(c) == host.lib.pg_kv_cache_capacity(c) == 64
+    host.lib.pg_kv_cache_free(host.ctx, host.cache(nkvh, hd, 128))
+    st, recorded, whole = host.captured("pg_llama_block_forward_dev", host.ctx, b, x, seq, c, out)
+    assert st == 2 and recorded == 0 and whole
+    assert host.lib.pg_kv_cache_len(c) == 64
+    host.ok("pg_llama_block_forward_dev", host.ctx, b, x, seq, c, out)
+    assert host.lib.pg_kv_cache_capacity(c) == 128
+    host.ok("pg_kv_cache_rollback_to", c, 64)
+    st, recorded, whole = host.captured("pg_llama_block_forward_dev", host.ctx, b, x, seq, c, out)
+    assert st == 0 and recorded > 0 and whole
+    host.lib.pg_kv_cache_free(host.ctx, c)
+    host.lib.pg_llama_block_free(host.ctx, b)
+
+
+def test_coded_cache_append_that_cuts_a_chunk_is_refused_by_a_capture(host):
+    heads, hd = 2, 64
+    c = host.new("pg_huffman_kv_cache_create", host.ctx, heads, hd, 32, 32)
+    rows = host.alloc(heads * hd * 64)
+    for tokens in (31, 1, 31):                                          # 63 tokens: one chunk a side, 31 in the window
+        host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, tokens)
+    assert host.lib.pg_huffman_kv_cache_num_chunks(c) == 1
+    st, recorded, whole = host.captured("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 1)
+    assert st == 2 and recorded == 0 and whole
+    assert host.lib.pg_huffman_kv_cache_len(c) == 63
+    host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 1)
+    assert host.lib.pg_huffman_kv_cache_num_chunks(c) == 2
+    host.lib.pg_huffman_kv_cache_free(host.ctx, c)
