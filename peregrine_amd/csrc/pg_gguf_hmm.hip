@@ -402,8 +402,11 @@ static hmm_plan hmm_plan_for(const pg_ctx *ctx, size_t m, size_t n_total, size_t
     return best;
 }
 
-// Which products this kernel takes, and in how many K chunks: those it is estimated to do in 0.93 of the int8 block
-// product's time or less (nearer than that the two estimates do not tell them apart).  That one takes about 12 us and 5
+// Which products this kernel takes, and in how many K chunks: every one of 96 rows and 18 G (Q8_0: 24 G) multiply-adds, which
+// always ran here and whose callers have its rounding (2^-22 of a row's largest value; the int8 block route's is 2^-16 of a
+// block's, so no estimate moves them there; it costs little: 4096 -> 22016 at 200 / 220 / 226 rows 116 : 116 / 113 : 116 /
+// 122 : 118 us, Q8_0 6528 -> 32772 at 141 208 : 192); and of the smaller ones those that it is estimated to do in 0.93 of the
+// int8 block product's time or less (nearer than that the two estimates do not tell them apart).  That one takes about 12 us and 5
 // (short K) to 6.5 (K of 8192 and more) us per G multiply-adds.  f16 route : int8 route, us: 4096 -> 28672 at 97 / 400 / 1024
 // rows 80 : 87 / 194 : 325 / 432 : 698; 4096 -> 4096 at 256 / 400 / 777 43 : 40 / 55 : 57 / 78 : 86; 14336 -> 4096 at
 // 97 / 256 / 777 71 : 57 / 91 : 105 / 211 : 343; 1024 -> 5632 at 400 / 1024 37 : 27 / 44 : 43.  Up to 64 rows are two full
@@ -414,10 +417,12 @@ bool pg_gguf_hmm_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_tota
         m < 2 || m > ((size_t)1 << 20))
         return false;
     const double int8_us = 12.0 + 1e-9 * (double)m * (double)n_total * (double)k_in * (5.0 + 1.5 * (k_in < 8192 ? (double)k_in : 8192.0) / 8192.0);
-    if (ctx->hmm_mode != 1 && (m <= 64 || int8_us < 30.0)) return false;
+    const bool large = m >= 96 && (double)m * (double)n_total * (double)k_in >= (ggml_type == PG_GGML_Q8_0 ? 2.4e10 : 1.8e10);
+    const bool always = ctx->hmm_mode == 1 || large;
+    if (!always && (m <= 64 || int8_us < 30.0)) return false;
     const hmm_plan plan = hmm_plan_for(ctx, m, n_total, k_in, 0);
     if (ks_out) *ks_out = plan.ks;
-    return ctx->hmm_mode == 1 || plan.us < 0.93 * int8_us;
+    return always || plan.us < 0.93 * int8_us;
 }
 
 size_t pg_gguf_hmm_part_floats(size_t m, size_t n_total, int ks) { return ks > 1 ? (size_t)ks * m * n_total : 0; }

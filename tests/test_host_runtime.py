@@ -138,3 +138,27 @@ def test_coded_cache_append_that_cuts_a_chunk_is_refused_by_a_capture(host):
     host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 1)
     assert host.lib.pg_huffman_kv_cache_num_chunks(c) == 2
     host.lib.pg_huffman_kv_cache_free(host.ctx, c)
+
+
+def f16_route(host, typ, m, n, k):
+    """Whether a product of m rows over an [n, k] tensor runs on the f16 matrix cores."""
+    w = host.new("pg_gguf_upload", host.ctx, bytes(n * k // 32 * {2: 18, 3: 20, 8: 34}[typ]), typ, n, k)
+    x, y = host.alloc(m * k), host.alloc(m * n)
+    host.lib.pghost_clear_launches()
+    host.ok("pg_gguf_matmul_dev", host.ctx, x, m, w, y)
+    host.lib.pg_gguf_free(host.ctx, w)
+    for p in (x, y):
+        host.ok("pg_dev_free", host.ctx, p)
+    return any("gguf_hmm_kernel" in name for name, _ in host.launches())
+
+
+@pytest.mark.parametrize("typ", [2, 3, 8])
+def test_products_of_the_f16_route_stay_there(host, typ):
+    """From 96 rows and 18 G (Q8_0: 24 G) multiply-adds on, a product always ran with its activations in f16 planes (2^-22
+    of a row's largest value): no estimate may hand it to the int8 block route (2^-16 of a block's)."""
+    least = 2.4e10 if typ == 8 else 1.8e10
+    for k, n in ((4096, 22016), (4096, 14336), (2048, 11008), (14336, 4096), (8192, 8200), (1024, 32000), (13312, 1029), (6528, 32772)):
+        first = max(96, int(-(-least // (n * k))))
+        for m in sorted({first, first + 1, first + 10, first + 21, first + 26, first + 45}):
+            if m * n * k <= 4e10:
+                assert f16_route(host, typ, m, n, k), (typ, m, n, k)
