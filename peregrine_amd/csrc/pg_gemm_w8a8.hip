@@ -792,11 +792,15 @@ pg_status pg_launch_gemm_w8a8(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride,
 }
 
 // The W8A32 product over three digit planes in one launch, where it is the better route: up to 32 rows the few-row kernel
-// (three or six tiles of planes), beyond that tiles of 64x64 to 128x128, unless tiles of 256x256 fill the part (then the
-// two low planes stacked and the combining pass below; `takes` says which).  128x128 from one tile a CU on.
+// (three or six tiles of planes), beyond that tiles of 64x64 to 128x128, unless tiles of 256x256 fill the part and are
+// mostly rows (three quarters; then the two low planes stacked and the combining pass below; `takes` says which).  Tiles
+// filled up by a vocabulary's columns are no reason: the padding rows are multiplied too, and two planes of accumulators of
+// m_pad x n written and read.  us, one launch : stacked: 1 x 4096 -> 50257 62 : 161, 32 x 4096 -> 128256 240 : 423,
+// 191 x 4096 -> 50257 144 : 249, 300 x 1024 -> 32000 54 : 93, 2048 x 14336 -> 32000 2890 : 2570.  (With short K the one
+// launch is also the faster one on tiles that are all rows: 512 x 1024 -> 50257 121 : 348, 2048 x 4096 -> 32000 855 : 859.)
 static bool w8a32_large(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
-    const size_t cus = (size_t)ctx->num_cu, t256 = ((m + 255) / 256) * ((w->cols + 255) / 256);
-    return t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus);
+    const size_t cus = (size_t)ctx->num_cu, m_pad = pg_round_up(m, 256), t256 = m_pad / 256 * ((w->cols + 255) / 256);
+    return 4 * m >= 3 * m_pad && (t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus));
 }
 bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     return ctx->gemm_force_tile == 0 && !w8a32_large(ctx, w, m) && w->k_pad < (1ull << 22) && w->cols < (1ull << 30) &&

@@ -582,6 +582,31 @@ def test_matmul_dequant_i8_one_launch(ctx, orc, m, k, n):
     qt.free_gpu()
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 256, 50257), (32, 384, 65536), (33, 130, 128256), (191, 256, 50257), (383, 128, 45825),
+                                   (192, 256, 50257)])   # (the last one: the low planes stacked)
+def test_matmul_dequant_i8_wide_weights(ctx, m, k, n):
+    """W8A32 over a vocabulary's columns: exact small integers in, exact integers out, on rows and columns of every tile's
+    beginning and end; and the float64 product there for random data."""
+    from peregrine_amd import quant
+    say(f"matmul_dequant_i8 wide weights m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + n)
+    rows = np.unique(np.r_[0, m // 2, m - 1, rng.integers(0, m, 5)])
+    cols = np.unique(np.r_[0:40, n // 2, n - 300 : n, rng.integers(0, n, 300)])
+    ai = (np.arange(m * k, dtype=np.float32) % 9 - 4).reshape(m, k)
+    qi = rng.integers(-127, 128, (k, n), dtype=np.int8)
+    qt = quant.QuantizedTensor(qi.reshape(-1), None, np.ones(n, np.float32), k, n)
+    got = quant.matmul_dequant_i8(ai, m, k, qt, ctx).reshape(m, n)
+    w = qi[:, cols].astype(np.float64)
+    assert (got[np.ix_(rows, cols)] == ai[rows].astype(np.float64) @ w).all(), "integer inputs: the product is not exact"
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    got = quant.matmul_dequant_i8(a, m, k, qt, ctx).reshape(m, n)
+    exact = a[rows].astype(np.float64) @ w
+    for i, r in enumerate(rows):
+        H.assert_close_rel(got[r, cols], exact[i], 1e-5, f"row {r} vs exact")
+    assert np.isfinite(got).all() and (np.abs(got).max(axis=1) > 0).all()
+    qt.free_gpu()
+
+
 @pytest.mark.parametrize("rows,cols", [(3, 4), (2, 5), (5, 1023), (4, 1025), (6, 4098), (2, 4099), (700, 4097),
                                        (2, 16381), (600, 16389), (1, 32767), (1, 32772), (3, 3)])
 def test_row_kernels_on_rows_of_any_length(ctx, orc, rows, cols):

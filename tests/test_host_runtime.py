@@ -162,3 +162,39 @@ def test_products_of_the_f16_route_stay_there(host, typ):
         for m in sorted({first, first + 1, first + 10, first + 21, first + 26, first + 45}):
             if m * n * k <= 4e10:
                 assert f16_route(host, typ, m, n, k), (typ, m, n, k)
+
+
+def dequant_i8_call(host, m, k, n):
+    """The kernels of one W8A32 product and the scratch it made the context take."""
+    w = host.alloc(k * n)
+    q = host.new("pg_qtensor_from_f32_dev", host.ctx, w, k, n)
+    host.ok("pg_dev_free", host.ctx, w)
+    x, y = host.alloc(m * k), host.alloc(m * n)
+    host.lib.pghost_clear_launches()
+    before = host.lib.pghost_used()
+    host.ok("pg_matmul_dequant_i8_dev", host.ctx, x, m, k, q, y)
+    taken = host.lib.pghost_used() - before
+    for p in (x, y):
+        host.ok("pg_dev_free", host.ctx, p)
+    host.lib.pg_qtensor_free(host.ctx, q)
+    return [name for name, _ in host.launches()], taken
+
+
+@pytest.mark.parametrize("m", [1, 16, 32, 33, 100, 191, 257, 383])
+@pytest.mark.parametrize("n", [45825, 50257, 65536, 128256])
+def test_w8a32_over_wide_weights_is_one_launch_in_the_planes_scratch(host, m, n):
+    """A vocabulary's columns: few 256-row tiles of many columns are still few rows.  One launch after the rows' digits, and
+    no scratch beyond the three planes (the accumulator planes of the stacked form are 8 bytes per padded row and column)."""
+    k = 1024
+    names, taken = dequant_i8_call(host, m, k, n)
+    assert len(names) == 2 and ("skinny" if m <= 32 else "gemm_w8a8_kernel") in names[1], names
+    m_pad = -(-m // 256) * 256
+    assert taken <= 1.25 * 3 * (m_pad * k + 4 * m_pad) + (2 << 20), taken
+
+
+@pytest.mark.parametrize("m,n,large", [(192, 46080, True), (191, 46080, False), (384, 23040, True), (383, 23040, False), (2048, 5888, True),
+                                       (2048, 5632, False), (192, 65537, False), (192, 98048, False), (192, 98049, True)])
+def test_w8a32_large_products_stack_their_low_planes(host, m, n, large):
+    """Both sides of each condition of the stacked form: 256x256 tiles that fill the part and are mostly rows."""
+    names, _ = dequant_i8_call(host, m, 256, n)
+    assert len(names) == (3 if large else 2), names
