@@ -69,7 +69,7 @@ pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out) {
         ctx->ws = nullptr;
         ctx->ws_bytes = 0;
         size_t want = pg_round_up(bytes + bytes / 4, 1 << 20);
-        PG_HIP(hipMalloc(&ctx->ws, want));
+        PG_HIP(pg_dev_malloc(ctx, &ctx->ws, want));
         ctx->ws_bytes = want;
     }
     *out = ctx->ws;
@@ -85,6 +85,16 @@ void pg_dev_pool::drain(bool close) {
         if (close) open = false;
     }
     for (auto &b : take) (void)hipFree(b.second);
+}
+
+hipError_t pg_dev_malloc(pg_ctx *ctx, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        ctx->pool->drain(false);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
 }
 
 pg_status pg_dev_block::alloc(pg_ctx *ctx, size_t want) {
@@ -111,12 +121,7 @@ pg_status pg_dev_block::alloc(pg_ctx *ctx, size_t want) {
             return PG_OK;
         }
     }
-    hipError_t e = hipMalloc(&p, want);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        pool->drain(false);
-        e = hipMalloc(&p, want);
-    }
+    const hipError_t e = pg_dev_malloc(ctx, &p, want);
     if (e != hipSuccess) {
         p = nullptr;
         pool.reset();
@@ -225,7 +230,7 @@ PG_API void *pg_ctx_stream(pg_ctx *ctx) { return ctx ? static_cast<void *>(ctx->
 PG_API pg_status pg_dev_alloc(pg_ctx *ctx, size_t bytes, void **dptr) {
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(dptr != nullptr, "pg_dev_alloc: dptr is null");
-    PG_HIP(hipMalloc(dptr, bytes ? bytes : 1));
+    PG_HIP(pg_dev_malloc(ctx, dptr, bytes ? bytes : 1));
     return PG_OK;
 }
 

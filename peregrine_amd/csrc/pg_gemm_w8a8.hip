@@ -868,11 +868,11 @@ PG_API pg_status pg_probe_gemm_clock(pg_ctx *ctx, size_t m, size_t k, size_t n, 
     const int tiles_m = (int)(m / BM), ntiles = tiles_m * (int)(n / BN);
     const unsigned grid = (unsigned)(((ntiles + 7) / 8) * 8);
     pg_tmp a, b, sc, out, clk;
-    PG_TRY(a.alloc(m * k));
-    PG_TRY(b.alloc(n * k));
-    PG_TRY(sc.alloc((m > n ? m : n) * sizeof(float)));
-    PG_TRY(out.alloc(m * n * sizeof(float)));
-    PG_TRY(clk.alloc((size_t)grid * 2 * sizeof(long long)));
+    PG_TRY(a.alloc(ctx, m * k));
+    PG_TRY(b.alloc(ctx, n * k));
+    PG_TRY(sc.alloc(ctx, (m > n ? m : n) * sizeof(float)));
+    PG_TRY(out.alloc(ctx, m * n * sizeof(float)));
+    PG_TRY(clk.alloc(ctx, (size_t)grid * 2 * sizeof(long long)));
     PG_TRY(pg_probe_fill_random(ctx, a.p, m * k));
     PG_TRY(pg_probe_fill_random(ctx, b.p, n * k));
     PG_HIP(hipMemsetAsync(sc.p, 0, (m > n ? m : n) * sizeof(float), ctx->stream));

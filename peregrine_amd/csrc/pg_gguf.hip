@@ -990,7 +990,7 @@ pg_status pg_gguf_ensure_tiled(pg_ctx *ctx, const pg_gguf_tensor *w) {
     const size_t bytes = groups * group_bytes, chunks = (group_bytes - 4352) / 16;
     if (groups > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf: too many weight rows for a tile-major copy");
     uint8_t *p = nullptr;
-    hipError_t e = hipMalloc((void **)&p, bytes);
+    hipError_t e = pg_dev_malloc(ctx, (void **)&p, bytes);
     if (e != hipSuccess)
         return pg_fail(e == hipErrorOutOfMemory ? PG_ENOMEM : PG_EDEVICE, "gguf tile-major copy (%zu bytes): %s", bytes, hipGetErrorString(e));
     const dim3 grid(grid_for(chunks, 256), (unsigned)groups);
@@ -1163,8 +1163,8 @@ PG_API pg_status pg_f16_to_f32(pg_ctx *ctx, const uint16_t *bits, size_t n, floa
     if (n == 0) return PG_OK;
     PG_CHECK_ARG(bits && out, "pg_f16_to_f32: null pointer");
     pg_tmp din, dout;
-    PG_TRY(din.alloc(n * 2));
-    PG_TRY(dout.alloc(n * 4));
+    PG_TRY(din.alloc(ctx, n * 2));
+    PG_TRY(dout.alloc(ctx, n * 4));
     PG_HIP(hipMemcpyAsync(din.p, bits, n * 2, hipMemcpyHostToDevice, ctx->stream));
     f16_to_f32_kernel<<<grid_for(n, 256), 256, 0, ctx->stream>>>(din.as<uint16_t>(), n, dout.as<uint32_t>());
     PG_TRY(pg_launch_check("f16_to_f32"));
@@ -1181,8 +1181,8 @@ static pg_status dequant_host(pg_ctx *ctx, const uint8_t *data, size_t num_eleme
     PG_CHECK_ARG(data && out, "%s: null pointer", name);
     const size_t nblocks = num_elements / 32;
     pg_tmp din, dout;
-    PG_TRY(din.alloc(nblocks * block_bytes));
-    PG_TRY(dout.alloc(num_elements * sizeof(float)));
+    PG_TRY(din.alloc(ctx, nblocks * block_bytes));
+    PG_TRY(dout.alloc(ctx, num_elements * sizeof(float)));
     PG_HIP(hipMemcpyAsync(din.p, data, nblocks * block_bytes, hipMemcpyHostToDevice, ctx->stream));
     const unsigned grid = grid_for(nblocks, 128);
     if (ggml_type == PG_GGML_Q8_0)
@@ -1230,12 +1230,12 @@ PG_API pg_status pg_gguf_upload(pg_ctx *ctx, const void *blocks, int ggml_type, 
     t->n_out = n_out;
     t->k_in = k_in;
     pg_tmp raw;
-    pg_status st = raw.alloc(nblocks * bb);
+    pg_status st = raw.alloc(ctx, nblocks * bb);
     hipError_t e = hipSuccess;
     if (st == PG_OK) {
-        e = hipMalloc((void **)&t->qs, nblocks * qb);
-        if (e == hipSuccess) e = hipMalloc((void **)&t->d, (n_out + 7) / 8 * 8 * nb * sizeof(uint16_t));
-        if (e == hipSuccess && ggml_type == PG_GGML_Q4_1) e = hipMalloc((void **)&t->m, (n_out + 7) / 8 * 8 * nb * sizeof(uint16_t));
+        e = pg_dev_malloc(ctx, (void **)&t->qs, nblocks * qb);
+        if (e == hipSuccess) e = pg_dev_malloc(ctx, (void **)&t->d, (n_out + 7) / 8 * 8 * nb * sizeof(uint16_t));
+        if (e == hipSuccess && ggml_type == PG_GGML_Q4_1) e = pg_dev_malloc(ctx, (void **)&t->m, (n_out + 7) / 8 * 8 * nb * sizeof(uint16_t));
         if (e == hipSuccess) e = hipMemcpyAsync(raw.p, blocks, nblocks * bb, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) {
             split_blocks_kernel<<<grid_for((n_out + 7) / 8 * 8 * nb, 256), 256, 0, ctx->stream>>>(raw.as<uint8_t>(), n_out, nb,

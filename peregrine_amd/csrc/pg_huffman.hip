@@ -384,7 +384,7 @@ pg_status decode_device_streams(pg_ctx *ctx, const uint8_t *bit_lengths, std::ve
     const size_t o_count = o_end + pg_round_up(sub * 8, 256), o_excl = o_count + pg_round_up(sub * 4, 256);
     const size_t o_wg = o_excl + pg_round_up(sub * 4, 256), o_flag = o_wg + pg_round_up(wg * 8, 256);
     pg_tmp buf;
-    PG_TRY(buf.alloc(o_flag + 256));
+    PG_TRY(buf.alloc(ctx, o_flag + 256));
     char *base = buf.as<char>();
     std::vector<uint16_t> lut;
     if (bit_lengths) {
@@ -446,7 +446,7 @@ pg_status decode_streams(pg_ctx *ctx, const uint8_t *bit_lengths, const uint8_t 
     }
     if (total == 0) return PG_OK;
     pg_tmp buf;
-    PG_TRY(buf.alloc(total));
+    PG_TRY(buf.alloc(ctx, total));
     std::vector<stream_desc> desc;
     size_t byte_off = 0, out_off = 0, sub = 0, wg = 0;
     for (size_t i = 0; i < nstreams; ++i) {
@@ -536,7 +536,7 @@ PG_API pg_status pg_huffman_decode(pg_ctx *ctx, const uint8_t *bit_lengths, cons
     if (num_symbols == 0) return PG_OK;
     PG_CHECK_ARG(bit_lengths && bitstream && out, "pg_huffman_decode: null pointer");
     pg_tmp dout;
-    PG_TRY(dout.alloc(num_symbols));
+    PG_TRY(dout.alloc(ctx, num_symbols));
     PG_TRY(decode_streams(ctx, bit_lengths, &bitstream, &len, &num_symbols, 1, dout.as<int8_t>()));
     PG_HIP(hipMemcpyAsync(out, dout.p, num_symbols, hipMemcpyDeviceToHost, ctx->stream));
     PG_HIP(hipStreamSynchronize(ctx->stream));
@@ -645,7 +645,7 @@ PG_API pg_status pg_huffman_tensor_to_gpu(pg_ctx *ctx, const pg_huffman_tensor *
     *out = nullptr;
     PG_CHECK_ARG(t->rows > 0 && t->cols > 0, "pg_huffman_tensor_to_gpu: empty tensor");
     pg_tmp dq;
-    PG_TRY(dq.alloc(t->rows * t->cols));
+    PG_TRY(dq.alloc(ctx, t->rows * t->cols));
     PG_TRY(huffman_decode_to_device(ctx, t, dq.as<int8_t>()));
     return pg_qtensor_from_device_q(ctx, dq.as<int8_t>(), t->scales.data(), t->rows, t->cols, out);
 }

@@ -879,7 +879,7 @@ static pg_status decompress_many(pg_ctx *ctx, const pg_huffman_kv_chunk *const *
     PG_CHECK_ARG(items.size() < 65536, "huffman kv: %zu chunks in one pass", items.size());
     const size_t o_items = pg_round_up(total, 256);
     pg_tmp buf;
-    PG_TRY(buf.alloc(o_items + items.size() * sizeof(dequant_item)));
+    PG_TRY(buf.alloc(ctx, o_items + items.size() * sizeof(dequant_item)));
     PG_HIP(hipMemcpyAsync(buf.as<char>() + o_items, items.data(), items.size() * sizeof(dequant_item), hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(pg_huffman_decode_device_streams(ctx, streams.data(), streams.size(), buf.as<int8_t>()));
     PG_TRY(pg_launch(ctx, "huffman_kv_dequant", kv_dequant_kernel, dim3(splits_for(max_head_elems), (unsigned)heads, (unsigned)items.size()),
@@ -920,7 +920,7 @@ PG_API pg_status pg_huffman_kv_compress_chunk(pg_ctx *ctx, const float *data, si
     const size_t total = num_tokens * num_heads * head_dim;
     PG_CHECK_ARG(data || total == 0, "pg_huffman_kv_compress_chunk: null data");
     pg_tmp d;
-    PG_TRY(d.alloc(total * sizeof(float)));
+    PG_TRY(d.alloc(ctx, total * sizeof(float)));
     if (total) PG_HIP(hipMemcpyAsync(d.p, data, total * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(compress_dev(ctx, d.as<float>(), num_tokens * head_dim, num_tokens, num_heads, head_dim, out));
     const hipError_t e = hipStreamSynchronize(ctx->stream);  // d is freed on return
@@ -1007,7 +1007,7 @@ PG_API pg_status pg_huffman_kv_decompress_chunk(pg_ctx *ctx, const pg_huffman_kv
     if (total == 0) return PG_OK;
     PG_CHECK_ARG(out != nullptr, "pg_huffman_kv_decompress_chunk: null output");
     pg_tmp d;
-    PG_TRY(d.alloc(total * sizeof(float)));
+    PG_TRY(d.alloc(ctx, total * sizeof(float)));
     PG_TRY(decompress_dev(ctx, c, d.as<float>(), c->num_tokens * c->head_dim));
     PG_HIP(hipMemcpyAsync(out, d.p, total * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     PG_HIP(hipStreamSynchronize(ctx->stream));
@@ -1183,7 +1183,7 @@ PG_API pg_status pg_huffman_kv_cache_get_kv(pg_ctx *ctx, const pg_huffman_kv_cac
     if (n == 0) return PG_OK;
     PG_CHECK_ARG(k && v, "pg_huffman_kv_cache_get_kv: null output");
     pg_tmp d;
-    PG_TRY(d.alloc(2 * n * sizeof(float)));
+    PG_TRY(d.alloc(ctx, 2 * n * sizeof(float)));
     PG_TRY(pg_huffman_kv_cache_get_kv_dev(ctx, c, d.as<float>(), d.as<float>() + n));
     PG_HIP(hipMemcpyAsync(k, d.p, n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     PG_HIP(hipMemcpyAsync(v, d.as<float>() + n, n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));

@@ -174,6 +174,9 @@ pg_status pg_fail(pg_status st, const char *fmt, ...) __attribute__((format(prin
 pg_status pg_use(pg_ctx *ctx);
 // PG_EDEVICE while ctx's stream captures: for calls that take memory or hand the host a result.
 pg_status pg_refuse_capture(pg_ctx *ctx, const char *what);
+// hipMalloc, which takes back what lies in ctx's pool when memory runs out.  Every device allocation of the library goes
+// through here.
+hipError_t pg_dev_malloc(pg_ctx *ctx, void **p, size_t bytes);
 // Scratch arena of at least `bytes` (256-byte aligned); contents undefined.
 pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out);
 // Pinned host memory of at least `bytes` (the context's one block; contents undefined).  The caller has waited for
@@ -223,8 +226,8 @@ inline pg_status pg_launch(pg_ctx *ctx, const char *name, void (*kernel)(KArgs..
 struct pg_tmp {
     void *p = nullptr;
     ~pg_tmp() { if (p) (void)hipFree(p); }
-    pg_status alloc(size_t bytes) {
-        hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
+    pg_status alloc(pg_ctx *ctx, size_t bytes) {
+        hipError_t e = pg_dev_malloc(ctx, &p, bytes ? bytes : 1);
         if (e != hipSuccess) { p = nullptr; return pg_fail(PG_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e)); }
         return PG_OK;
     }

@@ -1779,9 +1779,9 @@ PG_API pg_status pg_rmsnorm(pg_ctx *ctx, const float *x, size_t rows, size_t dim
     if (rows == 0 || dim == 0) return PG_OK;
     PG_CHECK_ARG(x && w && out, "pg_rmsnorm: null pointer");
     pg_tmp dx, dw, dout;
-    PG_TRY(dx.alloc(rows * dim * sizeof(float)));
-    PG_TRY(dw.alloc(dim * sizeof(float)));
-    PG_TRY(dout.alloc(rows * dim * sizeof(float)));
+    PG_TRY(dx.alloc(ctx, rows * dim * sizeof(float)));
+    PG_TRY(dw.alloc(ctx, dim * sizeof(float)));
+    PG_TRY(dout.alloc(ctx, rows * dim * sizeof(float)));
     PG_HIP(hipMemcpyAsync(dx.p, x, rows * dim * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     PG_HIP(hipMemcpyAsync(dw.p, w, dim * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(pg_rmsnorm_dev(ctx, dx.as<float>(), rows, dim, dw.as<float>(), eps, dout.as<float>()));
@@ -1811,8 +1811,8 @@ PG_API pg_status pg_rope_create(pg_ctx *ctx, size_t head_dim, size_t max_seq_len
         }
     pg_rope *r = new (std::nothrow) pg_rope{nullptr, nullptr, head_dim, max_seq_len};
     if (!r) return pg_fail(PG_ENOMEM, "pg_rope_create: out of host memory");
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&r->cos_t), n * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&r->sin_t), n * sizeof(float));
+    hipError_t e = pg_dev_malloc(ctx, reinterpret_cast<void **>(&r->cos_t), n * sizeof(float));
+    if (e == hipSuccess) e = pg_dev_malloc(ctx, reinterpret_cast<void **>(&r->sin_t), n * sizeof(float));
     if (e == hipSuccess) e = hipMemcpyAsync(r->cos_t, c.data(), n * sizeof(float), hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(r->sin_t, s.data(), n * sizeof(float), hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -1855,8 +1855,8 @@ PG_API pg_status pg_rope_apply(pg_ctx *ctx, const pg_rope *r, const float *x, si
     PG_CHECK_ARG(x && out, "pg_rope_apply: null pointer");
     const size_t bytes = seq_len * r->head_dim * sizeof(float);
     pg_tmp dx, dout;
-    PG_TRY(dx.alloc(bytes));
-    PG_TRY(dout.alloc(bytes));
+    PG_TRY(dx.alloc(ctx, bytes));
+    PG_TRY(dout.alloc(ctx, bytes));
     PG_HIP(hipMemcpyAsync(dx.p, x, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(pg_rope_apply_dev(ctx, r, dx.as<float>(), seq_len, offset, dout.as<float>()));
     PG_HIP(hipMemcpyAsync(out, dout.p, bytes, hipMemcpyDeviceToHost, ctx->stream));
@@ -1921,8 +1921,8 @@ PG_API pg_status pg_kv_cache_append(pg_ctx *ctx, pg_kv_cache *c, const float *ne
     PG_CHECK_ARG(new_k && new_v, "pg_kv_cache_append: null pointer");
     const size_t bytes = c->num_kv_heads * seq_len * c->head_dim * sizeof(float);
     pg_tmp dk, dv;
-    PG_TRY(dk.alloc(bytes));
-    PG_TRY(dv.alloc(bytes));
+    PG_TRY(dk.alloc(ctx, bytes));
+    PG_TRY(dv.alloc(ctx, bytes));
     PG_HIP(hipMemcpyAsync(dk.p, new_k, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_HIP(hipMemcpyAsync(dv.p, new_v, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(pg_kv_cache_append_dev(ctx, c, dk.as<float>(), dv.as<float>(), seq_len));
@@ -1968,8 +1968,8 @@ PG_API pg_status pg_gqa_attention(pg_ctx *ctx, const float *q, const pg_kv_cache
     PG_CHECK_ARG(q && out, "pg_gqa_attention: null pointer");
     const size_t bytes = num_q_heads * seq_q * k_cache->head_dim * sizeof(float);
     pg_tmp dq, dout;
-    PG_TRY(dq.alloc(bytes));
-    PG_TRY(dout.alloc(bytes));
+    PG_TRY(dq.alloc(ctx, bytes));
+    PG_TRY(dout.alloc(ctx, bytes));
     PG_HIP(hipMemcpyAsync(dq.p, q, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_HIP(hipMemcpyAsync(dout.p, out, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(launch_attention(ctx, dq.as<float>(), k_cache, v_cache, num_q_heads, seq_q, scale, mask_kind, offset, window,
@@ -2004,8 +2004,8 @@ PG_API pg_status pg_gqa_attention_local_global(pg_ctx *ctx, const float *q, cons
     PG_CHECK_ARG(q && out, "pg_gqa_attention_local_global: null pointer");
     const size_t bytes = num_q_heads * seq_q * k_cache->head_dim * sizeof(float);
     pg_tmp dq, dout;
-    PG_TRY(dq.alloc(bytes));
-    PG_TRY(dout.alloc(bytes));
+    PG_TRY(dq.alloc(ctx, bytes));
+    PG_TRY(dout.alloc(ctx, bytes));
     PG_HIP(hipMemcpyAsync(dq.p, q, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_HIP(hipMemcpyAsync(dout.p, out, bytes, hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(launch_attention(ctx, dq.as<float>(), k_cache, v_cache, num_q_heads, seq_q, scale, PG_MASK_LOCAL_GLOBAL, offset,
@@ -2034,7 +2034,7 @@ PG_API pg_status pg_llama_block_create(pg_ctx *ctx, size_t model_dim, size_t num
     b->d = model_dim; b->nqh = num_q_heads; b->nkvh = num_kv_heads; b->hd = head_dim; b->ffn = ffn_dim; b->eps = rms_eps;
     pg_status st = pg_rope_create(ctx, head_dim, max_seq_len, rope_base, &b->rope);
     if (st == PG_OK) {
-        hipError_t e = hipMalloc(reinterpret_cast<void **>(&b->attn_norm_w), 2 * model_dim * sizeof(float));
+        hipError_t e = pg_dev_malloc(ctx, reinterpret_cast<void **>(&b->attn_norm_w), 2 * model_dim * sizeof(float));
         if (e != hipSuccess) st = pg_fail(PG_ENOMEM, "pg_llama_block_create: %s", hipGetErrorString(e));
     }
     if (st != PG_OK) {
@@ -2050,7 +2050,7 @@ PG_API pg_status pg_llama_block_create(pg_ctx *ctx, size_t model_dim, size_t num
     const size_t o_tab = o_f + pg_xdigits_bytes(1, ffn_dim);
     const size_t tab_bytes = pg_round_up((2 * items + 4) * sizeof(void *) + items * sizeof(int), 256);
     const size_t total = o_tab + tab_bytes + pg_round_up(model_dim / 32 * sizeof(float), 256);
-    hipError_t e = hipMalloc(&b->dec, total);
+    hipError_t e = pg_dev_malloc(ctx, &b->dec, total);
     if (e == hipSuccess) e = hipMemsetAsync(b->dec, 0, total, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
@@ -2286,7 +2286,7 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
         b->chain = nullptr;
         b->chain_bytes = 0;
         const size_t want = need + need / 4;
-        PG_HIP(hipMalloc(&b->chain, want));
+        PG_HIP(pg_dev_malloc(ctx, &b->chain, want));
         b->chain_bytes = want;
     }
     char *base = static_cast<char *>(b->chain);
@@ -2404,7 +2404,7 @@ PG_API pg_status pg_llama_block_forward_dev(pg_ctx *ctx, pg_llama_block *b, cons
         if (b->arena) (void)hipFree(b->arena);
         b->arena = nullptr;
         b->seq_cap = 0;
-        PG_HIP(hipMalloc(reinterpret_cast<void **>(&b->arena), floats * sizeof(float)));
+        PG_HIP(pg_dev_malloc(ctx, reinterpret_cast<void **>(&b->arena), floats * sizeof(float)));
         b->seq_cap = cap;
     }
     PG_TRY(cache_reserve(ctx, cache, offset + seq));  // (ahead of every launch: a step that a capture refuses leaves nothing in the graph)

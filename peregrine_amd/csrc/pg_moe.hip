@@ -280,7 +280,7 @@ pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n
         ctx->moe_tabs.erase(ctx->moe_tabs.begin());
     }
     void *dev = nullptr;
-    PG_HIP(hipMalloc(&dev, n * sizeof(void *)));
+    PG_HIP(pg_dev_malloc(ctx, &dev, n * sizeof(void *)));
     const hipError_t ce = hipMemcpy(dev, host_tab, n * sizeof(void *), hipMemcpyHostToDevice);
     if (ce != hipSuccess) {
         (void)hipFree(dev);

@@ -945,12 +945,12 @@ PG_API pg_status pg_mxfp4_upload(pg_ctx *ctx, const uint8_t *blocks, const uint8
     t->n_out = out_dim;
     t->k_in = in_dim;
     pg_tmp rb, rs;
-    pg_status st = rb.alloc(nblocks * 16);
-    if (st == PG_OK) st = rs.alloc(nblocks);
+    pg_status st = rb.alloc(ctx, nblocks * 16);
+    if (st == PG_OK) st = rs.alloc(ctx, nblocks);
     hipError_t e = hipSuccess;
     if (st == PG_OK) {
-        e = hipMalloc((void **)&t->qs, nrg * ncp * 64 * 16);
-        if (e == hipSuccess) e = hipMalloc((void **)&t->d, nrg * (ncp / 4) * 64 * 4);
+        e = pg_dev_malloc(ctx, (void **)&t->qs, nrg * ncp * 64 * 16);
+        if (e == hipSuccess) e = pg_dev_malloc(ctx, (void **)&t->d, nrg * (ncp / 4) * 64 * 4);
         if (e == hipSuccess) e = hipMemcpyAsync(rb.p, blocks, nblocks * 16, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(rs.p, scales, nblocks, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) {
@@ -1028,7 +1028,7 @@ PG_API pg_status pg_mxfp4_expert_create(pg_ctx *ctx, size_t hidden, size_t inter
     pg_status st = pg_mxfp4_upload(ctx, mlp1_blocks, mlp1_scales, 2 * intermediate, hidden, &e->mlp1);
     if (st == PG_OK) st = pg_mxfp4_upload(ctx, mlp2_blocks, mlp2_scales, hidden, intermediate, &e->mlp2);
     if (st == PG_OK) {
-        hipError_t he = hipMalloc((void **)&e->bias1, (2 * intermediate + hidden) * sizeof(float));
+        hipError_t he = pg_dev_malloc(ctx, (void **)&e->bias1, (2 * intermediate + hidden) * sizeof(float));
         if (he == hipSuccess) {
             e->bias2 = e->bias1 + 2 * intermediate;
             he = hipMemcpyAsync(e->bias1, mlp1_bias, 2 * intermediate * sizeof(float), hipMemcpyHostToDevice, ctx->stream);

@@ -99,9 +99,9 @@ PG_API pg_status pg_probe_mfma_i8(pg_ctx *ctx, int iters, double *tops, double *
     PG_CHECK_ARG(iters >= 1 && iters <= (1 << 20), "pg_probe_mfma_i8: iters %d", iters);
     const int wgs = ctx->num_cu;  // one workgroup of 8 wavefronts per CU: two per SIMD
     pg_tmp in, out, clk;
-    PG_TRY(in.alloc(6 * 512 * sizeof(v4i)));
-    PG_TRY(out.alloc((size_t)wgs * 512 * sizeof(int)));
-    PG_TRY(clk.alloc((size_t)wgs * 2 * sizeof(long long)));
+    PG_TRY(in.alloc(ctx, 6 * 512 * sizeof(v4i)));
+    PG_TRY(out.alloc(ctx, (size_t)wgs * 512 * sizeof(int)));
+    PG_TRY(clk.alloc(ctx, (size_t)wgs * 2 * sizeof(long long)));
     PG_TRY(pg_probe_fill_random(ctx, in.p, 6 * 512 * sizeof(v4i)));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     PG_HIP(hipEventCreate(&e0));
@@ -146,8 +146,8 @@ PG_API pg_status pg_probe_hbm_read_shaped(pg_ctx *ctx, size_t bytes_per_pass, in
     const size_t chunks_per_wg = (total + wgs - 1) / wgs;
     const size_t pass_bytes = total * 16;
     pg_tmp buf, out;
-    PG_TRY(buf.alloc(pass_bytes * buffers));
-    PG_TRY(out.alloc(256));
+    PG_TRY(buf.alloc(ctx, pass_bytes * buffers));
+    PG_TRY(out.alloc(ctx, 256));
     PG_TRY(pg_probe_fill_random(ctx, buf.p, pass_bytes * buffers));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     PG_HIP(hipEventCreate(&e0));

@@ -278,7 +278,7 @@ pg_status quantize_weights_on_device(pg_ctx *ctx, const float *w_dev, size_t row
                                      int8_t *q_dev, int8_t *q_t_dev, size_t t_stride,
                                      float *scales_dev, size_t cols_pad) {
     pg_tmp amax;
-    PG_TRY(amax.alloc(cols * sizeof(uint32_t)));
+    PG_TRY(amax.alloc(ctx, cols * sizeof(uint32_t)));
     fill_u32_kernel<<<grid_for(cols, 256), 256, 0, ctx->stream>>>(amax.as<uint32_t>(), cols, 0u);
     PG_TRY(pg_launch_check("fill_u32"));
     dim3 g1(grid_for(cols, 256), grid_for(rows, CM_ROWS_PER_BLOCK));
@@ -305,8 +305,8 @@ pg_status qtensor_alloc(pg_ctx *ctx, size_t rows, size_t cols, pg_qtensor **out)
     t->w_t = nullptr;
     t->scales = nullptr;
     const size_t bytes = t->k_pad * t->n_pad;
-    hipError_t e = hipMalloc((void **)&t->w_t, bytes);
-    if (e == hipSuccess) e = hipMalloc((void **)&t->scales, t->n_pad * sizeof(float));
+    hipError_t e = pg_dev_malloc(ctx, (void **)&t->w_t, bytes);
+    if (e == hipSuccess) e = pg_dev_malloc(ctx, (void **)&t->scales, t->n_pad * sizeof(float));
     if (e == hipSuccess) e = hipMemsetAsync(t->w_t, 0, bytes, ctx->stream);
     if (e != hipSuccess) {
         if (t->w_t) (void)hipFree(t->w_t);
@@ -385,9 +385,9 @@ PG_API pg_status pg_quantize_activations(pg_ctx *ctx, const float *a, size_t row
     PG_CHECK_ARG(rows < (1ull << 31), "pg_quantize_activations: too many rows");
     const size_t n = rows * cols;
     pg_tmp da, dq, ds;
-    PG_TRY(da.alloc(n * sizeof(float)));
-    PG_TRY(dq.alloc(n));
-    PG_TRY(ds.alloc(rows * sizeof(float)));
+    PG_TRY(da.alloc(ctx, n * sizeof(float)));
+    PG_TRY(dq.alloc(ctx, n));
+    PG_TRY(ds.alloc(ctx, rows * sizeof(float)));
     if (n) PG_HIP(hipMemcpyAsync(da.p, a, n * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(pg_launch_quantize_activations(ctx, da.as<float>(), rows, cols, dq.as<int8_t>(), cols,
                                           ds.as<float>()));
@@ -405,10 +405,10 @@ PG_API pg_status pg_quantize_weights(pg_ctx *ctx, const float *w, size_t rows, s
     PG_CHECK_ARG(scales != nullptr, "pg_quantize_weights: scales is null");
     PG_CHECK_ARG(n == 0 || (w && q), "pg_quantize_weights: null pointer");
     pg_tmp dw, dq, dqt, ds;
-    PG_TRY(dw.alloc(n * sizeof(float)));
-    PG_TRY(dq.alloc(n));
-    if (q_t) PG_TRY(dqt.alloc(n));
-    PG_TRY(ds.alloc(cols * sizeof(float)));
+    PG_TRY(dw.alloc(ctx, n * sizeof(float)));
+    PG_TRY(dq.alloc(ctx, n));
+    if (q_t) PG_TRY(dqt.alloc(ctx, n));
+    PG_TRY(ds.alloc(ctx, cols * sizeof(float)));
     if (n) PG_HIP(hipMemcpyAsync(dw.p, w, n * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     PG_TRY(quantize_weights_on_device(ctx, dw.as<float>(), rows, cols, dq.as<int8_t>(),
                                       q_t ? dqt.as<int8_t>() : nullptr, rows, ds.as<float>(), cols));
@@ -426,9 +426,9 @@ PG_API pg_status pg_dequantize(pg_ctx *ctx, const int8_t *q, const float *scales
     if (n == 0) return PG_OK;
     PG_CHECK_ARG(q && scales && out, "pg_dequantize: null pointer");
     pg_tmp dq, ds, dout;
-    PG_TRY(dq.alloc(n));
-    PG_TRY(ds.alloc(cols * sizeof(float)));
-    PG_TRY(dout.alloc(n * sizeof(float)));
+    PG_TRY(dq.alloc(ctx, n));
+    PG_TRY(ds.alloc(ctx, cols * sizeof(float)));
+    PG_TRY(dout.alloc(ctx, n * sizeof(float)));
     PG_HIP(hipMemcpyAsync(dq.p, q, n, hipMemcpyHostToDevice, ctx->stream));
     PG_HIP(hipMemcpyAsync(ds.p, scales, cols * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     dequantize_kernel<<<grid_for(n, 256), 256, 0, ctx->stream>>>(dq.as<int8_t>(), ds.as<float>(), rows,
@@ -471,7 +471,7 @@ PG_API pg_status pg_qtensor_upload(pg_ctx *ctx, const int8_t *q, const float *sc
     PG_CHECK_ARG(q && scales, "pg_qtensor_upload: null pointer");
     PG_CHECK_ARG(rows < (1ull << 31) && cols < (1ull << 31), "pg_qtensor_upload: shape too large");
     pg_tmp dq;
-    PG_TRY(dq.alloc(rows * cols));
+    PG_TRY(dq.alloc(ctx, rows * cols));
     PG_HIP(hipMemcpyAsync(dq.p, q, rows * cols, hipMemcpyHostToDevice, ctx->stream));
     return pg_qtensor_from_device_q(ctx, dq.as<int8_t>(), scales, rows, cols, out);
 }
@@ -500,7 +500,7 @@ PG_API pg_status pg_qtensor_from_f32(pg_ctx *ctx, const float *w, size_t rows, s
     *out = nullptr;
     PG_CHECK_ARG(rows > 0 && cols > 0 && w, "pg_qtensor_from_f32: empty tensor or null pointer");
     pg_tmp dw;
-    PG_TRY(dw.alloc(rows * cols * sizeof(float)));
+    PG_TRY(dw.alloc(ctx, rows * cols * sizeof(float)));
     PG_HIP(hipMemcpyAsync(dw.p, w, rows * cols * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     return pg_qtensor_from_f32_dev(ctx, dw.as<float>(), rows, cols, out);
 }
@@ -512,7 +512,7 @@ PG_API pg_status pg_qtensor_download(pg_ctx *ctx, const pg_qtensor *t, int8_t *q
     const size_t rows = t->rows, cols = t->cols;
     if (q) {
         pg_tmp dq;
-        PG_TRY(dq.alloc(rows * cols));
+        PG_TRY(dq.alloc(ctx, rows * cols));
         dim3 g(grid_for(rows, 64), grid_for(cols, 64));
         // w_t is [cols, rows] with stride k_pad; transpose back to [rows, cols].
         transpose_i8_kernel<<<g, 256, 0, ctx->stream>>>(t->w_t, cols, rows, t->k_pad, dq.as<int8_t>(), cols);

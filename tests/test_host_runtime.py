@@ -198,3 +198,43 @@ def test_w8a32_large_products_stack_their_low_planes(host, m, n, large):
     """Both sides of each condition of the stacked form: 256x256 tiles that fill the part and are mostly rows."""
     names, _ = dequant_i8_call(host, m, 256, n)
     assert len(names) == (3 if large else 2), names
+
+
+def test_memory_running_out_empties_the_pool_for_every_allocation(host):
+    """64 MB lie in the pool (a key/value cache's two planes); with 16 MB of device memory left, whatever needs more
+    than that gets it: the workspace, a block's chain and arena, weights, temporaries, the caller's own allocations."""
+    mb = 1 << 20
+    d, nqh, nkvh, hd, ffn, seq = 256, 4, 2, 64, 8192, 400
+    shapes = [(nqh * hd, d), (nkvh * hd, d), (nkvh * hd, d), (d, nqh * hd), (ffn, d), (ffn, d), (d, ffn)]
+    ws = [host.gguf(n, k) for n, k in shapes]
+    b = host.new("pg_llama_block_create", host.ctx, d, nqh, nkvh, hd, ffn, 512, 10000.0, 1e-5)
+    norm = np.ones(d, np.float32)
+    host.ok("pg_llama_block_set_weights", host.ctx, b, *ws, norm.ctypes.data, norm.ctypes.data)
+    c, x = host.cache(nkvh, hd, 32), host.alloc(seq * d)
+    k, n, m = 4096, 8192, 64
+    wf, y, xq = host.alloc(k * n), host.alloc(m * n), host.alloc(2048 * k)
+    q = host.new("pg_qtensor_from_f32_dev", host.ctx, wf, k, 64)
+    i8, scales = np.zeros(k * n, np.int8), np.ones(n, np.float32)
+    out = np.zeros(seq * d, np.float32)
+
+    def upload():
+        host.lib.pg_qtensor_free(host.ctx, host.new("pg_qtensor_upload", host.ctx, i8.ctypes.data, scales.ctypes.data, k, n))
+
+    def rows():
+        big = np.zeros(6 * mb, np.float32)
+        host.ok("pg_rmsnorm", host.ctx, big.ctypes.data, 6 * mb // d, d, norm.ctypes.data, 1e-5, big.ctypes.data)
+
+    for what, use in (("workspace", lambda: host.ok("pg_matmul_dequant_i8_dev", host.ctx, xq, 2048, k, q, y)),
+                      ("block step", lambda: host.ok("pg_llama_block_forward_dev", host.ctx, b, x, seq, c, x)),
+                      ("weights", upload), ("temporaries", rows),
+                      ("a caller's", lambda: host.ok("pg_dev_free", host.ctx, host.alloc(8 * mb)))):
+        planes = host.cache(8, 128, 8192)
+        used = host.lib.pghost_used()
+        host.lib.pg_kv_cache_free(host.ctx, planes)
+        assert host.lib.pghost_used() == used                     # (64 MB in the pool now)
+        host.lib.pghost_limit(used + 16 * mb)
+        use()
+        host.lib.pghost_limit(C.c_size_t(-1).value)
+        assert host.lib.pghost_used() < used + 16 * mb, what
+    host.lib.pg_kv_cache_free(host.ctx, c)
+    host.lib.pg_llama_block_free(host.ctx, b)
