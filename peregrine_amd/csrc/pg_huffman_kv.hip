@@ -17,6 +17,7 @@
 // 0.25 bit a value): the decoder of such a chunk is one launch that starts a thread per 64 values, with no search for
 // code boundaries, and writes the scaled f32 values into the caller's layout.  A chunk made from stored parts has no
 // index and goes through the self-synchronising decoder of the Huffman-coded weights and a scaling launch.
+#include <atomic>
 #include <chrono>
 #include <memory>
 #include <new>
@@ -676,16 +677,25 @@ struct pg_huffman_kv_cache {
     char **table = nullptr;
     size_t table_cap = 0;
     std::vector<pg_dev_block> old_tables;
-    bool foreign() const { return hot->k_mem.foreign || table_mem.foreign; }
-    // Before ctx's stream uses any of it.  (Once another context has, the chunks' blocks are marked one by one.)
+    // Before ctx's stream uses any of it.  `user` = the pool of the context that used the cache last: what its stream has made
+    // since is its own, everything else was marked then, so only another context has anything to mark.  (An address that
+    // a later context's pool takes over belongs to no block any more: the same holds.  Reads may come from several threads.)
+    std::atomic<const pg_dev_pool *> user{nullptr};
     void touch(const pg_ctx *ctx) {
-        const bool was = foreign();
         hot->touch(ctx);
+        if (user.load() == ctx->pool.get()) return;
         table_mem.touch(ctx);
-        if (!foreign() || was) return;
+        for (auto &t : old_tables) t.touch(ctx);
         for (auto *v : {&k_chunks, &v_chunks})
-            for (auto *p : *v) p->block->foreign = true;
-        for (auto &t : old_tables) t.foreign = true;
+            for (auto *p : *v) p->block->touch(ctx);
+        user.store(ctx->pool.get());
+    }
+    bool foreign() const {
+        bool any = hot->k_mem.foreign || hot->v_mem.foreign || table_mem.foreign;
+        for (auto &t : old_tables) any = any || t.foreign;
+        for (auto *v : {&k_chunks, &v_chunks})
+            for (auto *p : *v) any = any || p->block->foreign;
+        return any;
     }
 };
 

@@ -238,3 +238,33 @@ def test_memory_running_out_empties_the_pool_for_every_allocation(host):
         assert host.lib.pghost_used() < used + 16 * mb, what
     host.lib.pg_kv_cache_free(host.ctx, c)
     host.lib.pg_llama_block_free(host.ctx, b)
+
+
+@pytest.mark.parametrize("users", ["a", "ab", "aba", "abab"])
+def test_memory_another_context_has_used_is_not_pooled(host, users):
+    """A cache and a coded cache used on two contexts' streams in turn, from the first of which they are freed: what only
+    the one context used goes to its pool, everything else to hipFree, which waits for both streams -- chunks and tables
+    made after the window was shared among it."""
+    other = host.new("pg_ctx_create", 0, None)
+    ctx = {"a": host.ctx, "b": other}
+    heads, hd = 2, 64
+    rows, out = host.alloc(heads * hd * 256), host.alloc(heads * hd * 256)
+    plain = host.new("pg_kv_cache_create", host.ctx, heads, hd)
+    coded = host.new("pg_huffman_kv_cache_create", host.ctx, heads, hd, 32, 32)
+    for u in users:
+        host.ok("pg_kv_cache_append_dev", ctx[u], plain, rows, rows, 8)       # (room for 32: it never grows)
+        host.ok("pg_huffman_kv_cache_append_dev", ctx[u], coded, rows, rows, 33)   # a chunk each
+    host.ok("pg_huffman_kv_cache_get_kv_dev", host.ctx, coded, out, out)
+    for cache, free, blocks in ((plain, "pg_kv_cache_free", 2), (coded, "pg_huffman_kv_cache_free", 3 + len(users))):
+        before = host.lib.pghost_frees()
+        getattr(host.lib, free)(host.ctx, cache)
+        freed = host.lib.pghost_frees() - before
+        if users == "a":
+            assert freed == 0                                                 # all of it pooled
+        elif cache is plain:
+            assert freed == 2
+        else:
+            # two planes of the window, the table, and the chunks: a reads b's, and b's appends follow a's first
+            own_after = 1 if users == "aba" else 0                            # the chunk that a cut after b's last use
+            assert freed == blocks - own_after, (freed, blocks)
+    host.lib.pg_ctx_destroy(other)
