@@ -710,7 +710,35 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
     const int mb = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
     const size_t units = k_pad / 128, g16 = (cols + 15) / 16, cus = (size_t)ctx->num_cu;
     struct shape { int nb, nst, nw; } sh = {1, mb == 1 ? 4 : 3, 0};
-    if (mb == 1) {
+    const size_t wgs2 = (g16 + 1) / 2;  // workgroups of two weight tiles
+    if (wgs2 > 2 * cus) {
+        // More than 16384 columns (a vocabulary's): two weight tiles a workgroup, and of the rings that the LDS still holds
+        // all at once (160 KiB a CU over the ring: 3, 4, 6 or 8 workgroups) the deepest; past that, rounds of the ring whose
+        // rounds come out fullest.  Short runs of K keep one tile.  Drawn from 384 shapes a row class (m 12, 24, 48; K 256
+        // .. 14000, N 16500 .. 170000), every shape below timed on each: 2.6, 2.4 and 0.9 % over the best one on average
+        // (the lines below, which go to 16000 columns, taken further: 12, 16 and 14 %, up to 40).  us, those : these:
+        // 8 x 1024 -> 50257 15.2 : 13.0, 24 x 4096 -> 24000 26.6 : 22.0, 24 x 768 -> 128256 38.8 : 30.4, 48 x 4096 -> 24000
+        // 36.9 : 28.6, 64 x 8192 -> 32000 73.8 : 64.5, 48 x 768 -> 151936 68.4 : 58.5.
+        if (mb == 1) {
+            if (units <= 4) sh = wgs2 <= 4 * cus ? shape{1, 4, 1} : shape{2, 3, 1};
+            else if (units > 32 && (wgs2 <= 3 * cus || wgs2 > 4 * cus)) sh = {2, 3, 4};
+            else if (wgs2 <= 3 * cus) sh = shape{2, 2, units < 6 ? 2 : 4};
+            else if (wgs2 <= 4 * cus) sh = {2, 3, 2};
+            else if (wgs2 <= 6 * cus) sh = {2, 2, 2};
+            else if (wgs2 <= 8 * cus) sh = {2, 3, 1};
+            else sh = shape{2, 2, units < 6 ? 2 : 4};
+        } else if (mb == 2) {
+            if (wgs2 <= 4 * cus) sh = units <= 4 ? shape{1, 3, 1} : shape{2, 2, 2};
+            else if (wgs2 <= 6 * cus || (wgs2 > 10 * cus && units > 16)) sh = {2, 3, 1};
+            else sh = {2, 2, 1};
+        } else {
+            if (units <= 4) sh = {1, 2, 1};
+            else if (units > 16 && wgs2 > 12 * cus) sh = {2, 2, 3};
+            else if (wgs2 <= 3 * cus || (units > 16 && wgs2 > 8 * cus && wgs2 <= 9 * cus)) sh = {2, 2, 2};
+            else if (wgs2 <= 4 * cus || (wgs2 > 6 * cus && wgs2 <= 8 * cus)) sh = {2, 3, 1};
+            else sh = {2, 2, 1};
+        }
+    } else if (mb == 1) {
         if (g16 > 3 * cus && units > 8) sh = {2, 3, 4};
         else if (g16 > 2 * cus && units > 16) sh = {1, 2, 4};
         else if (g16 > cus && units > 16) sh = {2, 3, 8};
@@ -759,6 +787,8 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
     PG_SKINNY(2, 1, 2, 4) PG_SKINNY(2, 2, 2, 4) PG_SKINNY(2, 2, 2, 8)
     PG_SKINNY(4, 1, 3, 1) PG_SKINNY(4, 1, 3, 2) PG_SKINNY(4, 1, 3, 4)
     PG_SKINNY(4, 1, 2, 1) PG_SKINNY(4, 1, 2, 2) PG_SKINNY(4, 2, 2, 3) PG_SKINNY(4, 2, 3, 4)
+    PG_SKINNY(1, 2, 2, 2) PG_SKINNY(1, 2, 2, 4) PG_SKINNY(1, 2, 3, 1) PG_SKINNY(1, 2, 3, 2)
+    PG_SKINNY(2, 2, 2, 1) PG_SKINNY(2, 2, 2, 2) PG_SKINNY(2, 2, 3, 1) PG_SKINNY(4, 2, 2, 1) PG_SKINNY(4, 2, 2, 2) PG_SKINNY(4, 2, 3, 1)
 #undef PG_SKINNY
     return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8 (few rows in one launch): no kernel of %d tiles, %d stages, %d wavefronts", sh.nb, sh.nst, sh.nw);
 }

@@ -651,3 +651,31 @@ def test_few_rows_launch_shapes_bit_exact(ctx, orc, m, k, n):
     want = acc.astype(np.float32) * np.asarray(s, np.float32)[:, None] * np.asarray(qt.scales, np.float32)[None, :]
     got = np.asarray(quant.matmul_quantized(a, m, k, qt, ctx), np.float32).reshape(m, n)
     assert (bits(got) == bits(want)).all()
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (2, 512, 16400), (16, 512, 32800), (5, 640, 16400), (3, 640, 65552), (16, 768, 24576), (9, 2100, 24592), (16, 640, 32784), (2, 640, 49168),
+    (16, 4200, 16400), (7, 4224, 32784),                                                                              # one tile of rows
+    (17, 500, 32768), (32, 130, 32784), (20, 640, 16400), (31, 640, 32784), (32, 700, 49168), (17, 2176, 81936),       # two
+    (33, 512, 16400), (64, 640, 24576), (48, 640, 24592), (50, 640, 32784), (64, 700, 49168), (33, 640, 65552),        # four
+    (40, 2176, 65552), (64, 2200, 73744), (35, 2176, 98320),
+])
+def test_few_rows_over_wide_weights_bit_exact(ctx, orc, m, k, n):
+    """Both sides of the lines between the few-row launch's shapes beyond 16384 columns (workgroups of 32 columns a CU),
+    ragged rows, K and columns; at columns of the first, middle and last tiles."""
+    from peregrine_amd import quant
+    say(f"few rows over wide weights m={m} k={k} n={n}")
+    rng = np.random.default_rng(m * 7 + k + n)
+    q = rng.integers(-127, 128, (k, n), dtype=np.int8)
+    scales = rng.uniform(0.5e-3, 2e-3, n).astype(np.float32)
+    qt = quant.QuantizedTensor(q.reshape(-1), None, scales, k, n)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, ::53] *= 20.0
+    got = np.asarray(quant.matmul_quantized(a, m, k, qt, ctx), np.float32).reshape(m, n)
+    cols = np.unique(np.r_[0:70, n // 2 : n // 2 + 40, n - 300 : n, rng.integers(0, n, 400)])
+    qa, s = orc.quantize_activations(a, m, k)
+    acc = np.asarray(qa, np.float64).reshape(m, k) @ q[:, cols].astype(np.float64)
+    want = acc.astype(np.float32) * np.asarray(s, np.float32)[:, None] * scales[cols][None, :]
+    assert (bits(got[:, cols]) == bits(want)).all()
+    assert (np.abs(got).max(axis=0) > 0).all(), "a column was left out"
+    qt.free_gpu()

@@ -64,7 +64,7 @@ def test_one_row_w8a8_old_indexing_would_have_been_caught():
 
 def test_few_rows_w8a8_fills_stay_inside_both_planes():
     """gemm_w8a8_skinny_kernel<MB, NB, NW, NST>: every (activation tiles, weight tiles, wavefronts) it is launched with."""
-    combos = [(1, 1), (2, 1), (2, 2), (4, 1), (4, 2)]
+    combos = [(1, 1), (1, 2), (2, 1), (2, 2), (4, 1), (4, 2)]
     for k, n in itertools.product([128, 256, 384, 1000, 4096, 14336], RAGGED_N + [8200]):
         for (mb, nbt), nw in itertools.product(combos, (1, 2, 4, 8)):
             if mb == 4 and nw == 8:
