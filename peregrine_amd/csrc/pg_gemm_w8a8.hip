@@ -866,10 +866,13 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
         return nw == 4 ? go(gemm_w8a8_skinny_kernel<6, 1, 4, 2, true>, lds) : nw == 2 ? go(gemm_w8a8_skinny_kernel<6, 1, 2, 2, true>, lds)
                                                                                         : go(gemm_w8a8_skinny_kernel<6, 1, 1, 2, true>, lds);
     }
-    // One workgroup fits a CU whatever the tile: rounds of workgroups times what a round takes (us at K = 4096: 26 for
-    // 64x64, 29 for 64x128, 40 for 128x128; 700 x 1024 -> 4096 19.8 / 17.2 / 15.3, 2048 x 4096 -> 1024 57 / 33 / 44).
+    // One workgroup fits a CU whatever the tile: rounds of workgroups times what a round takes, 18 for 64x64, 24 for 64x128 and
+    // 40 for 128x128 (us at K = 4096).  Drawn from 180 shapes (m 33 .. 2500, K 256 .. 14336, n 512 .. 130000) with the three
+    // tiles timed on each and held against 280 others: 0.1 % over the best tile on average, 5 % at most (26, 29 and 40, from a
+    // few shapes, took 1.2 % and up to 26 %).  us, the three tiles: 197 x 1024 -> 4096 11.3 / 12.8 / 18.2, 356 x 4096 -> 14336
+    // 106 / 84 / 97, 1000 x 4096 -> 4096 84 / 66 / 63, 311 x 2048 -> 32000 101 / 75 / 84.
     auto cost = [&](size_t bm, size_t bn, size_t us) { return (((m + bm - 1) / bm) * ((n + bn - 1) / bn) + ctx->num_cu - 1) / ctx->num_cu * us; };
-    const size_t c0 = cost(64, 64, 26), c1 = cost(64, 128, 29), c2 = cost(128, 128, 40);
+    const size_t c0 = cost(64, 64, 18), c1 = cost(64, 128, 24), c2 = cost(128, 128, 40);
     if (c2 < c0 && c2 < c1)
         return launch_group<128, 128, 128, 2, 2, 4, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes);
     if (c1 < c0)

@@ -268,3 +268,10 @@ def test_memory_another_context_has_used_is_not_pooled(host, users):
             own_after = 1 if users == "aba" else 0                            # the chunk that a cut after b's last use
             assert freed == blocks - own_after, (freed, blocks)
     host.lib.pg_ctx_destroy(other)
+
+
+@pytest.mark.parametrize("m,k,n,tile", [(197, 1024, 4096, (64, 64)), (356, 4096, 14336, (64, 128)), (1000, 4096, 4096, (128, 128)), (311, 2048, 32000, (64, 128)),
+                                        (155, 1024, 103918, (64, 128)), (888, 11222, 4096, (128, 128))])
+def test_w8a32_tile_is_the_one_that_took_least(host, m, k, n, tile):
+    names, _ = dequant_i8_call(host, m, k, n)
+    assert len(names) == 2 and "gemm_w8a8_kernelILi%dELi%dE" % tile in names[1], names
