@@ -1143,7 +1143,10 @@ pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, 
 // expert's 3 * hidden * inter FP4 weights per pair at 6.2 TB/s over 15 us of launches, the tiles stream those of the
 // experts that T tokens are expected to hit at 5.2 over 27, but at least the walk of one row tile through both K.
 // (us, pairs against tiles: 8 experts of 960, top 2, 16 tokens 22.0 / 28.2; of 1440, top 4, 6 tokens 28.8 / 34.3, 8 tokens
-// 33.1 / 33.8, 10 tokens 37.3 / 32.2; of 2880, top 2, 10 tokens 60.1 / 47.3.)
+// 33.1 / 33.8, 10 tokens 37.3 / 32.2; of 2880, top 2, 10 tokens 60.1 / 47.3.  Both timed on 351 shapes, 4 to 30 experts,
+// hidden and inter 256 to 5760: 0.6 % over the faster one on average.  Where it errs: few output columns under a long K, which
+// the decode kernel streams at less than half that rate -- hidden 512, inter 3360 to 4096, 36 to 40 pairs 43-47 / 35 -- and
+// narrow experts of 2048 x 512, which would gain 15 % as pairs.  Such calls keep the finer digits they have.)
 bool pairs_faster(size_t T, size_t E, size_t top_k, size_t hidden, size_t inter) {
     const double us_per_expert = 3.0 * (double)hidden * (double)inter * (17.0 / 32.0) / 1e6;  // at 1 TB/s
     const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));

@@ -430,6 +430,21 @@ def test_llama_block_many_token_steps_on_the_f16_matrix_cores(ctx, orc, shape, t
         assert name in prof, (name, sorted(prof))
 
 
+@pytest.mark.parametrize("ffn", [4096, 4160, 8192, 8256, 16384, 16448, 32768])
+def test_llama_block_silu_up_rows_at_the_edges_of_their_registers(ctx, orc, ffn):
+    """SiLU.up as f16 planes: a row is held by 512 threads of 2, 4, 8 or 16 float4s; the longest row of each instance and
+    the next one that the f16 route takes (multiples of 64), with K chunks of gate|up to add up and without."""
+    from peregrine_amd import _ffi
+    _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 1))
+    try:
+        ctx.profile_begin()
+        _block_case(ctx, orc, 256, 4, 2, 64, ffn, 2, (20, 3, 17), max_seq=64, seed=ffn)
+        prof = ctx.profile_end()
+    finally:
+        _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 0))
+    assert "swiglu_f16_planes" in prof, sorted(prof)
+
+
 def test_llama_block_q4_1_weights(ctx, orc):
     """Offset blocks (Q4_1): the streaming kernel, one item per row, up to seven rows; more rows take the Q4_0
     matrix-core product on the same nibbles plus a launch that adds the offsets times the rows' block sums."""

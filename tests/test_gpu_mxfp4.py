@@ -285,3 +285,32 @@ def test_mxfp4_moe_tiles_with_few_slots(ctx, orc, hidden, inter):
         assert (other[keep] == got[keep]).all()
     for ex in experts:
         ex.free()
+
+
+@pytest.mark.parametrize("hidden,inter,E,top_k,T,pairs", [
+    (512, 512, 8, 2, 32, True), (512, 512, 8, 5, 13, False),         # 64 and 65 pairs
+    (512, 512, 8, 3, 21, True), (1024, 1024, 4, 2, 25, True), (1024, 1024, 4, 2, 26, False),   # 63; both sides of the estimates
+    (64, 96, 40, 1, 64, True), (64, 96, 33, 5, 13, False),           # up to 64 pairs of more experts than that are always pairs
+])
+def test_mxfp4_moe_pairs_or_tiles(ctx, orc, hidden, inter, E, top_k, T, pairs):
+    """Up to 64 (token, expert) pairs go one by one, also where pairs share experts if the estimates say so; 65 never do.
+    Bounds as for the routed test: exact digits one by one, 20 bits under a block's largest value in tiles."""
+    from peregrine_amd import mxfp4
+    from test_oracle_formats_pins import _mx_expert
+    say(f"mxfp4 moe pairs or tiles hidden={hidden} inter={inter} E={E} top_k={top_k} T={T}")
+    rng = np.random.default_rng(hidden + E + T)
+    raw = [_mx_expert(rng, hidden, inter) for _ in range(E)]
+    experts = [mxfp4.Mxfp4Expert(hidden, inter, 1.702, 7.0, *r, ctx=ctx) for r in raw]
+    x = orc.rng_normal(T + 5, T * hidden).reshape(T, hidden)
+    x[:, ::37] *= 10.0
+    idx = np.stack([rng.permutation(E)[:top_k] for _ in range(T)]).astype(np.int32)
+    w = rng.uniform(0.2, 1.0, (T, top_k)).astype(np.float32)
+    ctx.profile_begin()
+    got = mxfp4.moe_forward_routed(x, idx, w, experts, ctx)
+    prof = ctx.profile_end()
+    assert ("mxfp4_rows_pairs" in prof) == pairs and ("mxfp4_tiles_grouped" in prof) != pairs, sorted(prof)
+    want = orc.mxfp4_moe_routed(x, T, hidden, inter, 1.702, 7.0, top_k, idx, w, raw)
+    for t in range(T):
+        H.assert_close_rel(got[t], want[t], 2e-4, f"token {t}")
+    for ex in experts:
+        ex.free()
