@@ -767,7 +767,7 @@ def section_gguf_many_rows(B, line):
     entry = {"workload": f"row (a), prefill size: Q4_0 dequant-matmul [{m}x{k_in}]->[{m}x{n_out}]; {len(hs)} tensors rotated",
              "value": round(flop / (t["ms_per_step"] * 1e-3) / 1e12, 1), "unit": "TFLOP/s", **B.stats(t),
              "kernels_ms": {k: round(v[0], 5) for k, v in prof.items()},
-             "roofline": {"kernel": "gguf_hmm_kernel<Q4_0, 2, 4> (v_mfma_f32_16x16x32_f16; weights unpacked exactly in registers, "
+             "roofline": {"kernel": "gguf_hmm_kernel<Q4_0, 8> (v_mfma_f32_16x16x32_f16; weights unpacked exactly in registers, "
                                     "activations as two f16 planes: twice the counted flops run on the matrix cores)",
                           "bound": "mfma", "achieved": round(flop / (k_ms * 1e-3) / 1e12, 1), "peak": 2500.0, "unit": "TFLOP/s",
                           "frac": round(flop / (k_ms * 1e-3) / 1e12 / 2500.0, 4), "executed_tflops": round(2 * flop / (k_ms * 1e-3) / 1e12, 1),
