@@ -198,8 +198,9 @@ pg_status pg_gguf_matmul_dev(pg_ctx *ctx, const float *x_dev, size_t m,
  * a hipMalloc, a launch and a wait inside a call that is otherwise stream-ordered and allocation-free.
  * pg_gguf_prepare makes now whatever products over up to `max_rows` activation rows of this tensor (alone, in a
  * group, inside a Llama block or as an expert of pg_moe_ffn) will need, as the reference rearranges weights at load
- * (load_transposed_weight, src/models/llama/model.rs:243-257); afterwards those calls neither allocate nor wait,
- * which a caller that captures them in a HIP graph requires.  max_rows < 2 makes nothing (one-row products read
+ * (load_transposed_weight, src/models/llama/model.rs:243-257); afterwards those calls allocate nothing for the tensor.
+ * (The context's workspace still grows at the first call that needs more of it: a caller that captures them in a HIP
+ * graph makes one eager call of each shape first.)  max_rows < 2 makes nothing (one-row products read
  * the planes as uploaded), and neither does an MXFP4 tensor (all of its products do).  pg_gguf_drop_prepared frees
  * the copy again (it waits for the stream); pg_gguf_device_bytes reports what the tensor holds. */
 pg_status pg_gguf_prepare(pg_ctx *ctx, const pg_gguf_tensor *w, size_t max_rows);

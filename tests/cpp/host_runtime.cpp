@@ -17,7 +17,7 @@ struct state {
     std::map<const void *, std::string> kernels;
     std::map<const void *, void *> variables;
     std::map<void *, size_t> device;  // live allocations
-    size_t used = 0, limit = ~(size_t)0, frees = 0, bad_frees = 0, recorded = 0;
+    size_t used = 0, limit = ~(size_t)0, frees = 0, bad_frees = 0, recorded = 0, copied = 0;
     std::map<hipStream_t, bool> capturing;  // true: capture was broken by a forbidden call
     std::vector<launch_rec> launches;
 };
@@ -57,7 +57,8 @@ TEST_API size_t pghost_used() { guard g(sim().mu); return sim().used; }
 TEST_API size_t pghost_frees() { guard g(sim().mu); return sim().frees; }
 TEST_API size_t pghost_bad_frees() { guard g(sim().mu); return sim().bad_frees; }
 TEST_API size_t pghost_recorded() { guard g(sim().mu); return sim().recorded; }
-TEST_API void pghost_begin_capture(void *stream) { guard g(sim().mu); sim().capturing[(hipStream_t)stream] = false; sim().recorded = 0; }
+TEST_API size_t pghost_copied() { guard g(sim().mu); return sim().copied; }  // of those, copies and fills by the runtime
+TEST_API void pghost_begin_capture(void *stream) { guard g(sim().mu); sim().capturing[(hipStream_t)stream] = false; sim().recorded = sim().copied = 0; }
 TEST_API int pghost_end_capture(void *stream) {  // 1: the capture is whole
     guard g(sim().mu);
     const bool broken = sim().capturing[(hipStream_t)stream];
@@ -113,12 +114,12 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { guard g(
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
     guard g(sim().mu);
     if (sim().capturing.empty()) memcpy(d, s, n);
-    else ++sim().recorded;
+    else { ++sim().recorded; ++sim().copied; }
     return hipSuccess;
 }
 hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
     guard g(sim().mu);
-    if (!sim().capturing.empty()) ++sim().recorded;
+    if (!sim().capturing.empty()) { ++sim().recorded; ++sim().copied; }
     else
         for (size_t i = 0; i < h; ++i) memcpy((char *)d + i * dp, (const char *)s + i * sp, w);
     return hipSuccess;
@@ -126,7 +127,7 @@ hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) {
     guard g(sim().mu);
     if (sim().capturing.empty()) memset(d, v, n);
-    else ++sim().recorded;
+    else { ++sim().recorded; ++sim().copied; }
     return hipSuccess;
 }
 

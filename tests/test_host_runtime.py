@@ -25,7 +25,7 @@ class Host:
         for name, args in _ffi.SIGNATURES.items():
             fn = getattr(self.lib, name)
             fn.argtypes, fn.restype = args, _ffi._OTHER_RESTYPE.get(name, C.c_int)
-        for name in ("pghost_used", "pghost_frees", "pghost_bad_frees", "pghost_recorded", "pghost_num_launches"):
+        for name in ("pghost_used", "pghost_frees", "pghost_bad_frees", "pghost_recorded", "pghost_copied", "pghost_num_launches"):
             getattr(self.lib, name).restype = C.c_size_t
         self.lib.pghost_limit.argtypes = [C.c_size_t]
         self.lib.pghost_limit.restype = self.lib.pghost_clear_launches.restype = self.lib.pghost_begin_capture.restype = None
@@ -275,3 +275,68 @@ def test_memory_another_context_has_used_is_not_pooled(host, users):
 def test_w8a32_tile_is_the_one_that_took_least(host, m, k, n, tile):
     names, _ = dequant_i8_call(host, m, k, n)
     assert len(names) == 2 and "gemm_w8a8_kernelILi%dELi%dE" % tile in names[1], names
+
+
+def same_call_captured(host, name, *args):
+    """A call that has run once at its shape is captured whole, as launches alone."""
+    host.ok(name, host.ctx, *args)
+    st, recorded, whole = host.captured(name, host.ctx, *args)
+    assert st == 0 and whole and recorded > 0 and host.lib.pghost_copied() == 0, (name, st, recorded, whole, host.lib.pghost_copied(), host.lib.pg_last_error())
+
+
+ROWS = [1, 2, 3, 5, 8, 9, 16, 17, 33, 64, 65, 97, 150, 200, 300, 700]
+
+
+@pytest.mark.parametrize("typ", [2, 3, 8])
+@pytest.mark.parametrize("n,k", [(4096, 4096), (1000, 1024), (1029, 6656), (300, 96)])
+def test_block_products_are_captured_after_one_eager_call(host, typ, n, k):
+    w = host.new("pg_gguf_upload", host.ctx, bytes(n * k // 32 * {2: 18, 3: 20, 8: 34}[typ]), typ, n, k)
+    x, y = host.alloc(max(ROWS) * k), host.alloc(max(ROWS) * n)
+    for m in ROWS:
+        same_call_captured(host, "pg_gguf_matmul_dev", x, m, w, y)
+
+
+@pytest.mark.parametrize("n,k", [(4096, 1024), (50257, 256), (300, 4096)])
+def test_int8_products_are_captured_after_one_eager_call(host, n, k):
+    w = host.alloc(n * k)
+    q = host.new("pg_qtensor_from_f32_dev", host.ctx, w, k, n)
+    x, y = host.alloc(max(ROWS) * k), host.alloc(max(ROWS) * n)
+    for m in ROWS:
+        same_call_captured(host, "pg_matmul_quantized_dev", x, m, k, q, y, None)
+        same_call_captured(host, "pg_matmul_dequant_i8_dev", x, m, k, q, y)
+
+
+def test_expert_layers_are_captured_after_one_eager_call(host):
+    d, ffn, E, k = 256, 512, 8, 2
+    tab = lambda n_out, k_in: (C.c_void_p * E)(*[host.new("pg_gguf_upload", host.ctx, bytes(n_out * k_in // 32 * 34), 8, n_out, k_in).value for _ in range(E)])
+    gate, up, down = (C.cast(t, C.POINTER(C.c_void_p)) for t in (tab(ffn, d), tab(ffn, d), tab(d, ffn)))
+    codes, scales, bias = np.zeros(2 * ffn * d // 2, np.uint8), np.zeros(2 * ffn * d // 32, np.uint8), np.zeros(2 * ffn, np.float32)
+    p = lambda a: a.ctypes.data
+    ex = (C.c_void_p * E)(*[host.new("pg_mxfp4_expert_create", host.ctx, d, ffn, 1.702, 7.0, p(codes), p(scales), p(bias), p(codes), p(scales), p(bias)).value
+                            for _ in range(E)])
+    x, logits, out = host.alloc(700 * d), host.alloc(700 * E), host.alloc(700 * d)
+    idx, wt = host.alloc(700 * k), host.alloc(700 * k)
+    for T in ROWS:
+        same_call_captured(host, "pg_moe_ffn_dev", x, T, logits, E, k, gate, up, down, 0, out)
+        same_call_captured(host, "pg_mxfp4_moe_ffn_routed_dev", x, T, idx, wt, k, C.cast(ex, C.POINTER(C.c_void_p)), E, out)
+
+
+@pytest.mark.parametrize("typ,d,ffn", [(2, 256, 512), (8, 1024, 2048), (3, 256, 512)])
+def test_block_steps_are_captured_after_one_eager_call(host, typ, d, ffn):
+    nqh, nkvh, hd = 4, 2, 64
+    shapes = [(nqh * hd, d), (nkvh * hd, d), (nkvh * hd, d), (d, nqh * hd), (ffn, d), (ffn, d), (d, ffn)]
+    ws = [host.new("pg_gguf_upload", host.ctx, bytes(n * k // 32 * {2: 18, 3: 20, 8: 34}[typ]), typ, n, k) for n, k in shapes]
+    b = host.new("pg_llama_block_create", host.ctx, d, nqh, nkvh, hd, ffn, 2048, 10000.0, 1e-5)
+    norm = np.ones(d, np.float32)
+    host.ok("pg_llama_block_set_weights", host.ctx, b, *ws, norm.ctypes.data, norm.ctypes.data)
+    x, out = host.alloc(700 * d), host.alloc(700 * d)
+    c = host.cache(nkvh, hd, 1500)
+    for seq in ROWS:
+        for at in (0, 700):
+            host.ok("pg_kv_cache_rollback_to", c, min(at, host.lib.pg_kv_cache_len(c)))
+            host.ok("pg_llama_block_forward_dev", host.ctx, b, x, seq, c, out)
+            host.ok("pg_kv_cache_rollback_to", c, host.lib.pg_kv_cache_len(c) - seq)
+            st, recorded, whole = host.captured("pg_llama_block_forward_dev", host.ctx, b, x, seq, c, out)
+            assert st == 0 and whole and recorded > 0 and host.lib.pghost_copied() == 0, (seq, at, host.lib.pg_last_error())
+    host.lib.pg_kv_cache_free(host.ctx, c)
+    host.lib.pg_llama_block_free(host.ctx, b)
