@@ -11,7 +11,7 @@
 // encoder.  The host takes part once per batch: it learns the coded sizes (words that the table kernel stores in
 // pinned memory), allocates exactly that much and launches the encoder.  A batch was 10 launches, 12 copies and 8
 // waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
-// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.36.
+// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.28.
 //
 // The encoder knows where every code starts, so it leaves an index beside the stream (a 16-bit offset per 64 values,
 // 0.25 bit a value): the decoder of such a chunk is one launch that starts a thread per 64 values, with no search for
@@ -137,239 +137,299 @@ __global__ __launch_bounds__(KV_WG) void kv_quant_hist_kernel(const kv_batch b, 
     b.hist[((size_t)c * b.nwg + blockIdx.x) * NUM_SYMBOLS + t] = (uint16_t)(lh[0][t] + lh[1][t] + lh[2][t] + lh[3][t]);
 }
 
+// Lane exchange for the merges below: the value of lane ^ D.
+template <int D> __device__ __forceinline__ unsigned lane_xor(unsigned v) {
+    if constexpr (D == 1) return __builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // quad_perm 1 0 3 2
+    else if constexpr (D == 2) return __builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2 3 0 1
+    else if constexpr (D == 4) return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);  // ^ 7, ^ 3
+    else if constexpr (D == 8) return __builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);  // row_ror 8
+    else {
+        const auto two = D == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false) : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return threadIdx.x & D ? two[0] : two[1];
+    }
+}
+template <int D> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+    return (unsigned long long)lane_xor<D>((unsigned)(v >> 32)) << 32 | lane_xor<D>((unsigned)v);
+}
+template <int D, class K> __device__ __forceinline__ void half_cleaner(K &x) {
+    const K o = lane_xor<D>(x);
+    x = ((threadIdx.x & D) != 0) == (o > x) ? o : x;
+}
+
+// Running sum over the lanes of a row of 16.
+__device__ __forceinline__ unsigned row_scan(unsigned v) {
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true);  // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true);
+    return v;
+}
+
+// The Huffman merges of n leaves (ascending weights) on one wavefront; returns the number of rounds.  Two queues, leaves
+// and the nodes made of them, both ascending.  The sum m of the two lightest trees is the smallest weight that a new node
+// can have, so all trees of weight <= m are taken, two by two, before any node that the round makes (a tie goes to the one
+// that was there first: a leaf before a node).  A round sorts the 64 lightest of both queues' heads across the lanes
+// -- min of the one ascending and the other descending is bitonic, six exchanges put it in order -- and pairs
+// neighbours, up to 32 at a time.  K holds weight << 9 | id: 32 bits for chunks below 2^23 values, else 64.
+constexpr unsigned TREE_PAD = NUM_SYMBOLS + 64;  // (a round reads 64 from a queue's head on)
+template <class K>
+__device__ __forceinline__ unsigned merge_trees(unsigned n, const unsigned *leaf_w, unsigned *node_w, unsigned *parent) {
+    const unsigned lane = threadIdx.x & 63;
+    unsigned lh = 0, qh = 0, made = 0, rounds = 0;
+    for (unsigned alive = n; alive > 1; ++rounds) {
+        constexpr unsigned NONE = 0x7FFFFFFFu;  // (not below any sum but the last)
+        const unsigned li = lh + lane, qi = qh + 63 - lane;
+        unsigned lw = leaf_w[li], qw = node_w[qi];
+        lw = li < n ? lw : NONE;
+        qw = qi < made ? qw : NONE;
+        const unsigned l0 = __builtin_amdgcn_readlane(lw, 0), l1 = __builtin_amdgcn_readlane(lw, 1);
+        const unsigned q0 = __builtin_amdgcn_readlane(qw, 63), q1 = __builtin_amdgcn_readlane(qw, 62);
+        const unsigned m = min(min(l0 + l1, l0 + q0), q0 + q1);
+        const unsigned light = __popcll(__ballot(lw <= m)) + __popcll(__ballot(qw <= m));
+        const unsigned taken = min(min(light, alive), 64u) & ~1u;
+        const K lk = (K)lw << 9 | li, qk = (K)qw << 9 | (NUM_SYMBOLS + qi);
+        K x = min(lk, qk);
+        half_cleaner<32>(x);
+        half_cleaner<16>(x);
+        half_cleaner<8>(x);
+        half_cleaner<4>(x);
+        half_cleaner<2>(x);
+        half_cleaner<1>(x);
+        const unsigned id = (unsigned)x & 511u, w = (unsigned)(x >> 9), sum = w + lane_xor<1>(w);
+        if (lane < taken) {
+            parent[id] = made + lane / 2;
+            if (!(lane & 1)) node_w[made + lane / 2] = sum;
+        }
+        const unsigned leaves = __popcll(__ballot(lane < taken && id < NUM_SYMBOLS));
+        lh += leaves;
+        qh += taken - leaves;
+        made += taken / 2;
+        alive -= taken / 2;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // the nodes are read by other lanes
+    }
+    return rounds;
+}
+
 // The chunk's code table and where its 4096-value runs start: one workgroup of 1024 a chunk.
 //
 // Lengths as HuffmanTable::from_frequencies gives them (src/huffman.rs:35-150: two queues over the symbols sorted by
 // frequency, a leaf wins a tie; depths clamped to 12), and where the clamp over-subscribes the code the same repair
 // as table_that_decodes in pg_huffman.hip.
 //
-// The merges are not made one after the other (a chain of up to 255 dependent steps: 80 us on one wavefront) but in
-// rounds: with the trees still apart in queue order, the sum m of the first two is the smallest weight a new tree can
-// have, so all those of weight <= m are taken, two by two, before any tree that the round makes (a tie goes to the one
-// that was there first).  A round pairs them up and merges the sums, ascending as they are, into what is left; some
-// 18 rounds of 0.8 us for a chunk of 262144 normally distributed values, half of the kernel's 28 us.  Each node's parent is kept; depths follow by
-// pointer doubling.
+// One workgroup on its CU, so what counts is the chain of dependent steps, and code that runs once comes in at the pace of
+// the instruction cache's misses: loops, not unrolled bodies.  A chunk of 262144 normally distributed values, cycles: histograms
+// 2 k (read one row at a time 10 k), ranks 4.3 k, merges 14 k for 18 rounds (33 k by eight wavefronts with a binary search in
+// LDS and a barrier a round), depths 2 k, length repair 3.4 k (14 k with its second ranking, unrolled), the rest, which
+// runs beside the host's part, 10 k: 17 us where it was 31, and 278 for 360 of 3000 tokens of 8 x 128 in pieces of 512.
 __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsigned long long *host_bits) {
-    __shared__ unsigned part[4][NUM_SYMBOLS], rank_up[NUM_SYMBOLS], rank_down[NUM_SYMBOLS];
-    __shared__ __attribute__((aligned(16))) unsigned long long keys[NUM_SYMBOLS];
-    __shared__ unsigned tree_w[2][NUM_SYMBOLS], tree_id[2][NUM_SYMBOLS];
+    __shared__ __attribute__((aligned(16))) unsigned freq[NUM_SYMBOLS];
+    __shared__ unsigned rank_up[NUM_SYMBOLS], rank_down[NUM_SYMBOLS];  // by symbol; by place in the ascending order
+    __shared__ unsigned leaf_w[TREE_PAD], node_w[TREE_PAD];
+    __shared__ uint8_t leaf_sym[NUM_SYMBOLS];
     __shared__ unsigned parent[2 * NUM_SYMBOLS];  // of the leaves (by ascending frequency), then of the nodes
-    __shared__ unsigned anc[2][NUM_SYMBOLS], dep[2][NUM_SYMBOLS];
+    __shared__ unsigned up_tree[2][NUM_SYMBOLS];  // of the nodes: levels << 16 | ancestor
     __shared__ unsigned cnt[16], first_code[16], limit[16], offset[16], lane_cnt[4][16];
     __shared__ __attribute__((aligned(16))) uint8_t bl[NUM_SYMBOLS];
     __shared__ uint8_t by_len[NUM_SYMBOLS];
-    __shared__ unsigned over, wsum[16];
+    __shared__ unsigned over, nrounds, wsum[16];
     __shared__ unsigned run_bits[1024];
     __shared__ unsigned long long wave_bits[4];
     const unsigned c = blockIdx.x, t = threadIdx.x, s = t & 255, p = t >> 8;
+    const unsigned lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint16_t *hist = b.hist + (size_t)c * b.nwg * NUM_SYMBOLS;
 
-    unsigned sum = 0;
-    for (unsigned i = p; i < b.nwg; i += 4) sum += hist[(size_t)i * NUM_SYMBOLS + s];
-    part[p][s] = sum;
     if (t < 16) cnt[t] = 0;
-    if (t < NUM_SYMBOLS) rank_up[t] = rank_down[t] = 0;
+    if (p == 0) {
+        freq[s] = ~0u;  // (kept less one: what is not in use then comes behind all others)
+        rank_up[s] = 0;
+        bl[s] = 0;
+    }
     __syncthreads();
-    const unsigned f = part[0][s] + part[1][s] + part[2][s] + part[3][s];
-    // symbols in order of frequency, ties by symbol: one key each, symbols not in use behind all others
-    const unsigned long long key = f ? (unsigned long long)f << 8 | s : ~0ull;
-    if (p == 0) keys[s] = key;
-    const unsigned n = __builtin_amdgcn_readfirstlane(__syncthreads_count(p == 0 && f > 0));  // symbols in use
-    unsigned up = 0;
-#pragma unroll 8
-    for (unsigned o = p * 64; o < p * 64 + 64; ++o) up += keys[o] < key;
-    atomicAdd(&rank_up[s], up);
+    {   // a wavefront adds up every sixteenth row, four rows in flight
+        unsigned sum[4] = {0, 0, 0, 0};
+        const ushort4 *rows = reinterpret_cast<const ushort4 *>(hist);
+        unsigned i = wave;
+        for (; i + 48 < b.nwg; i += 64) {
+            ushort4 h[4];
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) h[k] = rows[(size_t)(i + 16 * k) * 64 + lane];
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) { sum[0] += h[k].x; sum[1] += h[k].y; sum[2] += h[k].z; sum[3] += h[k].w; }
+        }
+        for (; i < b.nwg; i += 16) {
+            const ushort4 h = rows[(size_t)i * 64 + lane];
+            sum[0] += h.x; sum[1] += h.y; sum[2] += h.z; sum[3] += h.w;
+        }
+        if (wave < b.nwg)
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) atomicAdd(&freq[4 * lane + k], sum[k]);
+    }
     __syncthreads();
-    const unsigned lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    constexpr unsigned NONE = 0xFFFFFFFFu;  // (weights stay below 2^31)
+    // symbols in order of frequency, ties by symbol: o comes before s if its weight is below f, or below f + 1 where o < s,
+    // which is one and the same for all of a wavefront's symbols unless o is among them
+    const unsigned f = freq[s] + 1;
+    unsigned n = 0;  // symbols in use
+    {
+        const unsigned block = wave & 3, from = wave >> 2;
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k) n += __popcll(__ballot(freq[64 * k + lane] != ~0u));
+        unsigned up = 0;
+        if (block != from) {
+            const unsigned below = f - (from < block ? 0u : 1u);
+#pragma unroll 4
+            for (unsigned k = 0; k < 64; k += 4) {
+                const uint4 w = *reinterpret_cast<const uint4 *>(freq + from * 64 + k);
+                up += (w.x < below) + (w.y < below) + (w.z < below) + (w.w < below);
+            }
+        } else {
+#pragma unroll 4
+            for (unsigned k = 0; k < 64; k += 4) {
+                const uint4 w = *reinterpret_cast<const uint4 *>(freq + from * 64 + k);
+                up += (w.x < f - (k < lane ? 0u : 1u)) + (w.y < f - (k + 1 < lane ? 0u : 1u)) + (w.z < f - (k + 2 < lane ? 0u : 1u)) +
+                      (w.w < f - (k + 3 < lane ? 0u : 1u));
+            }
+        }
+        if (f > 0) atomicAdd(&rank_up[s], up);
+    }
+    __syncthreads();
     if (p == 0 && f > 0) {
-        tree_w[0][rank_up[s]] = f;
-        tree_id[0][rank_up[s]] = rank_up[s];
+        leaf_w[rank_up[s]] = f;
+        leaf_sym[rank_up[s]] = (uint8_t)s;
     }
     __syncthreads();
-    unsigned cur = 0, made = 0;
-    for (unsigned alive = n; alive > 1;) {
-        unsigned a[4], b2[2];
-#pragma unroll
-        for (unsigned r = 0; r < 4; ++r) a[r] = lane + 64 * r < alive ? tree_w[cur][lane + 64 * r] : NONE;
-        const unsigned m = __builtin_amdgcn_readlane(a[0], 0) + __builtin_amdgcn_readlane(a[0], 1);
-        unsigned taken = 0;
-#pragma unroll
-        for (unsigned r = 0; r < 4; ++r) taken += __popcll(__ballot(a[r] <= m));
-        taken &= ~1u;
-        const unsigned pairs = taken / 2;
-        if (wave < 6) {
-#pragma unroll
-            for (unsigned h = 0; h < 2; ++h) {
-                const unsigned k = lane + 64 * h;
-                b2[h] = k < pairs ? tree_w[cur][2 * k] + tree_w[cur][2 * k + 1] : NONE;
+    if (wave == 0) {
+        const unsigned r = b.total < (1u << 23) ? merge_trees<unsigned>(n, leaf_w, node_w, parent) : merge_trees<unsigned long long>(n, leaf_w, node_w, parent);
+        if (t == 0) nrounds = r;
+    } else if (wave >= 4 && wave < 8) {  // meanwhile the descending order, ties by symbol
+        const unsigned i = t - 256;
+        if (i < n) {
+            const unsigned w = leaf_w[i];
+            unsigned lo = 0, hi = 0;  // leaves below w, and of at most w
+#pragma unroll 1
+            for (unsigned step = 256; step > 0; step >>= 1) {
+                if (lo + step <= n && leaf_w[lo + step - 1] < w) lo += step;
+                if (hi + step <= n && leaf_w[hi + step - 1] <= w) hi += step;
             }
+            rank_down[i] = n - hi + i - lo;
         }
-        if (wave < 4) {  // what is left: 64 trees to a wavefront, each behind the new ones that are lighter
-            const unsigned own = wave == 0 ? a[0] : wave == 1 ? a[1] : wave == 2 ? a[2] : a[3], i = lane + 64 * wave;
-            const unsigned id = tree_id[cur][i];
-            unsigned at = i - taken;
-            for (unsigned k = 0; k < min(pairs, 64u); k += 8)
-#pragma unroll
-                for (unsigned u = 0; u < 8; ++u) at += __builtin_amdgcn_readlane(b2[0], k + u) < own ? 1u : 0u;
-            for (unsigned k = 64; k < pairs; ++k) at += __builtin_amdgcn_readlane(b2[1], k - 64) < own ? 1u : 0u;
-            if (i >= taken && i < alive) {
-                tree_w[cur ^ 1][at] = own;
-                tree_id[cur ^ 1][at] = id;
-            }
-        } else if (wave < 6) {  // the new ones: one to a lane of two wavefronts, each behind what is left of at most its weight
-            const unsigned w = wave == 4 ? b2[0] : b2[1], k = lane + 64 * (wave - 4);
-            unsigned at = taken;
-            for (unsigned step = 128; step > 0; step >>= 1)
-                if (step <= alive - taken) {
-                    const unsigned to = min(at + step, alive);
-                    at = tree_w[cur][to - 1] <= w ? to : at;
-                }
-            if (k < pairs) {
-                at += k - taken;
-                tree_w[cur ^ 1][at] = w;
-                tree_id[cur ^ 1][at] = NUM_SYMBOLS + made + k;
-            }
-        } else if (wave < 8) {
-            const unsigned k = lane + 64 * (wave - 6);
-            if (k < pairs) parent[tree_id[cur][2 * k]] = parent[tree_id[cur][2 * k + 1]] = made + k;
-        }
-        made += pairs;
-        alive -= pairs;
-        cur ^= 1;
-        __syncthreads();
     }
+    __syncthreads();
+    const unsigned rounds = nrounds;
+    unsigned mine = t;
     if (t < NUM_SYMBOLS) {
         const bool root = n < 2 || t >= n - 2;
-        anc[0][t] = root ? t : parent[NUM_SYMBOLS + t];
-        dep[0][t] = root ? 0 : 1;
+        up_tree[0][t] = mine = root ? t : 1u << 16 | parent[NUM_SYMBOLS + t];
     }
     __syncthreads();
-    for (int r = 0; r < 8; ++r) {
+    unsigned last = 0;
+#pragma unroll 1
+    for (unsigned reach = 1; reach < rounds; reach *= 2) {  // (a round adds at most one level)
         if (t < NUM_SYMBOLS) {
-            const unsigned a = anc[r & 1][t];
-            anc[(r + 1) & 1][t] = anc[r & 1][a];
-            dep[(r + 1) & 1][t] = dep[r & 1][t] + dep[r & 1][a];
+            const unsigned a = up_tree[last][mine & 0xFFFFu];
+            up_tree[last ^ 1][t] = mine = (mine & ~0xFFFFu) + a;
         }
+        last ^= 1;
         __syncthreads();
     }
-    unsigned len = 0;  // of symbol s (threads with p == 0)
-    if (p == 0 && f > 0) {
-        len = n < 2 ? 1u : min(dep[0][parent[rank_up[s]]] + 1u, (unsigned)KV_MAX_BITS);
+    unsigned len = 0;  // of leaf t
+    if (t < n) {
+        len = n < 2 ? 1u : min((up_tree[last][parent[t]] >> 16) + 1u, (unsigned)KV_MAX_BITS);
         atomicAdd(&cnt[len], 1u);
     }
     __syncthreads();
-    if (wave == 0) {  // uniform: the counts of the twelve lengths in registers
-        const unsigned mine = cnt[lane & 15];
-        unsigned cn[KV_MAX_BITS + 1];
-        int excess = -KV_LUT;  // of the Kraft sum, in 1 / 4096
-#pragma unroll
-        for (int l = 1; l <= KV_MAX_BITS; ++l) {
-            cn[l] = __builtin_amdgcn_readlane(mine, l);
-            excess += (int)cn[l] * (KV_LUT >> l);
-        }
+    if (wave == 0) {  // the counts of the twelve lengths: lane l holds cn[l]
+        unsigned cn = lane >= 1 && lane <= KV_MAX_BITS ? cnt[lane] : 0u;
+        auto get = [&](int l) { return (unsigned)__builtin_amdgcn_readlane(cn, l); };
+        auto add = [&](int l, unsigned x) { cn += lane == (unsigned)l ? x : 0u; };
+        int excess = pg_wave_sum_i32((int)(cn * (lane <= KV_MAX_BITS ? KV_LUT >> lane : 0))) - KV_LUT;  // of the Kraft sum, in 1 / 4096
         const bool too_many = excess > 0;
-        // While there is too much, lengthen by a bit the least frequent symbol of the deepest level below the limit:
-        // it stays the deepest until it gets there, so whole symbols go to the limit level by level, as many as the
-        // excess holds, and the last one part of the way.
-        int part_level = KV_MAX_BITS;
-#pragma unroll
-        for (int l = KV_MAX_BITS - 1; l >= 1; --l) {
-            const int gain = (KV_LUT >> l) - 1;
-            if (excess > 0 && part_level == KV_MAX_BITS) {
-                const unsigned x = min(cn[l], (unsigned)excess / (unsigned)gain);
-                cn[l] -= x;
-                cn[KV_MAX_BITS] += x;
+        if (too_many) {
+            // While there is too much, lengthen by a bit the least frequent symbol of the deepest level below the limit:
+            // it stays the deepest until it gets there, so whole symbols go to the limit level by level, as many as the
+            // excess holds, and the last one part of the way.
+            int l = KV_MAX_BITS - 1;
+#pragma unroll 1
+            for (; l >= 1 && excess > 0; --l) {
+                const int gain = (KV_LUT >> l) - 1;
+                const unsigned had = get(l);
+                unsigned x = (unsigned)((float)excess / (float)gain);  // (both below 2^21: off by one at the most)
+                if ((int)x * gain > excess) --x;
+                else if ((int)(x + 1) * gain <= excess) ++x;
+                x = min(x, had);
+                add(l, 0u - x);
+                add(KV_MAX_BITS, x);
                 excess -= (int)x * gain;
-                if (excess > 0 && cn[l] > 0) part_level = l;
+                if (excess > 0 && had > x) break;
             }
-        }
-#pragma unroll
-        for (int l = 1; l < KV_MAX_BITS; ++l)
-            if (l >= part_level && excess > 0) {
-                cn[l] -= 1;
-                cn[l + 1] += 1;
+#pragma unroll 1
+            for (; l >= 1 && l < KV_MAX_BITS && excess > 0; ++l) {
+                add(l, ~0u);
+                add(l + 1, 1u);
                 excess -= KV_LUT >> (l + 1);
             }
-        unsigned slack = too_many ? (unsigned)-excess : 0u;
-        if (slack > 0) {  // and give what is left to the most frequent symbols
-            unsigned had[KV_MAX_BITS + 1];
-#pragma unroll
-            for (int l = 1; l <= KV_MAX_BITS; ++l) { had[l] = cn[l]; cn[l] = 0; }
-#pragma unroll
-            for (int l = 1; l <= KV_MAX_BITS; ++l) {
-                for (; had[l] > 0 && l > 1 && (unsigned)(KV_LUT >> l) <= slack; --had[l]) {
-                    bool going = true;
-#pragma unroll
-                    for (int m = l; m >= 1; --m) {
-                        const bool shorter = going && m > 1 && (unsigned)(KV_LUT >> m) <= slack;
-                        if (shorter) slack -= KV_LUT >> m;
-                        else if (going) cn[m] += 1;
-                        going = shorter;
-                    }
+            unsigned slack = (unsigned)-excess;  // and what is left goes to the most frequent symbols
+            const unsigned all = cn;
+#pragma unroll 1
+            for (int from = 2; from <= KV_MAX_BITS && slack > 0; ++from) {
+                unsigned had = (unsigned)__builtin_amdgcn_readlane(all, from);
+#pragma unroll 1
+                for (; had > 0 && (unsigned)(KV_LUT >> from) <= slack; --had) {
+                    int to = from;
+#pragma unroll 1
+                    for (; to > 1 && (unsigned)(KV_LUT >> to) <= slack; --to) slack -= KV_LUT >> to;
+                    add(from, ~0u);
+                    add(to, 1u);
                 }
-                cn[l] += had[l];
             }
         }
-        unsigned code = 0, off = 0;
-#pragma unroll
-        for (int l = 1; l <= KV_MAX_BITS; ++l) {  // src/huffman.rs:152-186
-            code <<= 1;
-            if (t == 0) {
-                first_code[l] = code;
-                offset[l] = off;
-                limit[l] = (code + cn[l]) << (KV_MAX_BITS - l);
+        // src/huffman.rs:152-186: the codes of a length follow those of the shorter ones
+        unsigned kraft = lane <= KV_MAX_BITS ? cn << (KV_MAX_BITS - lane) : 0u, off = cn;
+        const unsigned own = kraft;
+        kraft = row_scan(kraft);
+        off = row_scan(off);
+        if (lane >= 1 && lane <= KV_MAX_BITS + 1) {
+            offset[lane] = off - cn;
+            if (lane <= KV_MAX_BITS) {
+                first_code[lane] = (kraft - own) >> (KV_MAX_BITS - lane);
+                limit[lane] = kraft;
             }
-            code += cn[l];
-            off += cn[l];
         }
-        if (t == 0) {
-            offset[KV_MAX_BITS + 1] = off;
-            over = too_many;
-        }
+        if (lane == 0) over = too_many;
     }
     __syncthreads();
-    if (over) {  // the repaired lengths go out again, shortest to most frequent (ties: lower symbol first)
-        const unsigned long long down_key = f ? (unsigned long long)~f << 8 | s : ~0ull;
-        if (p == 0) keys[s] = down_key;
-        __syncthreads();
-        unsigned down = 0;
-#pragma unroll 8
-        for (unsigned o = p * 64; o < p * 64 + 64; ++o) down += keys[o] < down_key;
-        atomicAdd(&rank_down[s], down);
-        __syncthreads();
-        if (p == 0 && f > 0) {
-            len = 1;
-#pragma unroll
-            for (int l = 2; l <= KV_MAX_BITS; ++l) len += offset[l] <= rank_down[s] ? 1 : 0;
-        }
-    }
-    // The stream's bits go to the host as soon as the lengths are known: it makes room and launches the encoder while the
-    // tables and start bits are written (3000 tokens of 8 x 128 in
-    // pieces of 512: 382 -> 360 us for the whole sequence).
     if (p == 0) {
-        bl[s] = (uint8_t)len;
-        unsigned long long bits = (unsigned long long)f * len;
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) bits += __shfl_xor(bits, d, 64);
-        if (lane == 0) wave_bits[wave] = bits;
+        if (over && t < n) {  // the repaired lengths go out again, shortest to most frequent (ties: lower symbol first)
+            const unsigned down = rank_down[t];
+            len = 1;
+#pragma unroll 1
+            for (int l = 2; l <= KV_MAX_BITS; ++l) len += offset[l] <= down ? 1 : 0;
+        }
+        if (t < n) bl[leaf_sym[t]] = (uint8_t)len;
+        const unsigned long long bits = t < n ? (unsigned long long)leaf_w[t] * len : 0ull;
+        const unsigned lo = (unsigned)pg_wave_sum_i32((int)(bits & 0xFFFFFFull)), hi = (unsigned)pg_wave_sum_i32((int)(bits >> 24));
+        if (lane == 0) wave_bits[wave] = ((unsigned long long)hi << 24) + lo;
     }
+    __syncthreads();
+    // The stream's bits go to the host as soon as the lengths are known: it makes room and launches the encoder while the
+    // tables and start bits are written.
+    if (t == 1023)  // (0 = not there yet)
+        __hip_atomic_store(host_bits + c, wave_bits[0] + wave_bits[1] + wave_bits[2] + wave_bits[3] + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     // the symbol's place among those of its length
     unsigned before = 0;
     if (p == 0) {
+        len = bl[s];
+#pragma unroll 1
         for (unsigned l = 1; l <= KV_MAX_BITS; ++l) {
             const unsigned long long m = __ballot(len == l);
-            if (len == l) before = __popcll(m & ((1ull << (t & 63)) - 1));
-            if ((t & 63) == 0) lane_cnt[t >> 6][l] = __popcll(m);
+            if (len == l) before = __popcll(m & ((1ull << lane) - 1));
+            if (lane == 0) lane_cnt[wave][l] = __popcll(m);
         }
     }
     __syncthreads();
-    if (t == 1023)  // (0 = not there yet)
-        __hip_atomic_store(host_bits + c, wave_bits[0] + wave_bits[1] + wave_bits[2] + wave_bits[3] + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (p == 0) {
         unsigned e = 0;
         if (len) {
-            for (unsigned w = 0; w < (t >> 6); ++w) before += lane_cnt[w][len];
+            for (unsigned w = 0; w < wave; ++w) before += lane_cnt[w][len];
             e = len << 16 | (first_code[len] + before);
             by_len[offset[len] + before] = (uint8_t)s;
         }

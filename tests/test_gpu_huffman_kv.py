@@ -239,3 +239,40 @@ def test_batches_and_run_edges(ctx, orc, heads, hd, chunk, chunks, kind):
     for side, made in ((0, c.k_chunks), (1, c.v_chunks)):
         for i in {0, chunks // 2, chunks - 1}:
             _same_chunk(made[i], o.chunk(side, i)[:3])
+
+
+def _counts(kind):
+    """How often each of the values -127 .. 127 occurs (127 always does: the scale is then 1 and a value its own code)."""
+    i = np.arange(255, dtype=np.int64)
+    if kind == "equal":                                    # every tree ties: more pairs in a round than a wavefront takes
+        return np.full(255, 9)
+    if kind == "ties":                                     # leaves and nodes of one weight, leaf first
+        return 1 << (i // 20)
+    if kind == "fibonacci":                                # one pair a round, the deepest tree
+        c = np.zeros(255, np.int64)
+        c[-26:] = [1, 1] + [0] * 24
+        for j in range(255 - 24, 255):
+            c[j] = c[j - 1] + c[j - 2]
+        return c
+    if kind == "ramp":
+        return i % 83 + 1
+    c = np.zeros(255, np.int64)
+    c[254] = 5                                             # one symbol
+    return c
+
+
+@pytest.mark.parametrize("kind", ["equal", "ties", "fibonacci", "ramp", "one"])
+@pytest.mark.parametrize("total", [0, (1 << 23) - 1, 1 << 23])
+def test_tables_at_the_edges_of_the_merges(ctx, orc, kind, total):
+    """Histograms that the merge rounds can go wrong at, as they are and brought to the total at which their keys
+    become 64 bits wide, and to one value less."""
+    from peregrine_amd import huffman
+    say(f"huffman kv table {kind} total={total}")
+    counts = _counts(kind)
+    if total:
+        counts = counts * (total // counts.sum())
+        counts[254] += total - counts.sum()
+    data = np.repeat(np.arange(-127, 128), counts).astype(np.float32)
+    chunk = huffman.HuffmanKVCache.compress_chunk(data, len(data), 1, 1, ctx)
+    _same_chunk(chunk, orc.huffman_kv_compress_chunk(data, len(data), 1, 1))
+    assert (huffman.HuffmanKVCache.decompress_chunk(chunk) == data).all()
