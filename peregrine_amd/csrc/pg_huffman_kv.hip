@@ -98,9 +98,17 @@ __global__ __launch_bounds__(KV_WG) void kv_quant_hist_kernel(const kv_batch b, 
     const unsigned c = blockIdx.y, t = threadIdx.x, base = blockIdx.x * ENC_PER_WG;
     const unsigned last = min(base + ENC_PER_WG, b.total) - 1;
     const unsigned h0 = base / b.head_elems, h1 = last / b.head_elems;
+    float4 v[ENC_SPT / 4];
+    if (vec)  // four values of one head each
+#pragma unroll
+        for (int j = 0; j < ENC_SPT / 4; ++j) {
+            const unsigned i = base + (j * KV_WG + t) * 4, h = i / b.head_elems;
+            if (i < b.total) v[j] = *reinterpret_cast<const float4 *>(b.head(c, h) + (i - h * b.head_elems));
+        }
     for (unsigned h = h0 + t; h <= h1; h += KV_WG) {
         const float *a = b.amax + ((size_t)c * b.heads + h) * b.splits;
         float m = 0.0f;
+#pragma unroll 8
         for (unsigned s = 0; s < b.splits; ++s) m = fmaxf(m, a[s]);
         const float scale = (m == 0.0f) ? 1.0f : m / 127.0f;
         sc[h - h0] = scale;
@@ -113,12 +121,10 @@ __global__ __launch_bounds__(KV_WG) void kv_quant_hist_kernel(const kv_batch b, 
 #pragma unroll
     for (int j = 0; j < ENC_SPT / 4; ++j) {
         const unsigned i = base + (j * KV_WG + t) * 4;
-        if (vec) {  // four values of one head
+        if (vec) {
             if (i >= b.total) continue;
-            const unsigned h = i / b.head_elems;
-            const float inv = 1.0f / sc[h - h0];
-            const float4 v = *reinterpret_cast<const float4 *>(b.head(c, h) + (i - h * b.head_elems));
-            const int x0 = pg_quant_to_i8(v.x * inv), x1 = pg_quant_to_i8(v.y * inv), x2 = pg_quant_to_i8(v.z * inv), x3 = pg_quant_to_i8(v.w * inv);
+            const float inv = 1.0f / sc[i / b.head_elems - h0];
+            const int x0 = pg_quant_to_i8(v[j].x * inv), x1 = pg_quant_to_i8(v[j].y * inv), x2 = pg_quant_to_i8(v[j].z * inv), x3 = pg_quant_to_i8(v[j].w * inv);
             *reinterpret_cast<unsigned *>(q + i) = (x0 & 255) | (x1 & 255) << 8 | (x2 & 255) << 16 | (unsigned)x3 << 24;
             atomicAdd(mine + x0 + 128, 1u);
             atomicAdd(mine + x1 + 128, 1u);
@@ -162,6 +168,14 @@ __device__ __forceinline__ unsigned row_scan(unsigned v) {
     v += __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true);
     v += __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true);
     v += __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true);
+    return v;
+}
+
+// And over a wavefront's.
+__device__ __forceinline__ unsigned wave_scan(unsigned v) {
+    v = row_scan(v);
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, true);  // row_bcast 15 into rows 1 and 3, then 31 into rows 2 and 3
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, true);
     return v;
 }
 
@@ -462,12 +476,7 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
         }
         __syncthreads();
         const unsigned v = at + t < b.nwg ? run_bits[t] : 0u;
-        unsigned incl = v;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const unsigned o = __shfl_up(incl, d, 64);
-            incl += lane >= (unsigned)d ? o : 0u;
-        }
+        const unsigned incl = wave_scan(v);
         if (lane == 63) wsum[wave] = incl;
         __syncthreads();
         unsigned long long pre = run;
@@ -508,7 +517,7 @@ __device__ __forceinline__ bool push_code(unsigned e, unsigned long long &acc, u
 // has two writers and nothing is zeroed first.
 __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, const kv_places places, char **__restrict__ table) {
     __shared__ unsigned lc[NUM_SYMBOLS], wsum[4];
-    __shared__ unsigned words[ENC_PER_WG * KV_MAX_BITS / 32 + 2];
+    __shared__ unsigned words[ENC_PER_WG * KV_MAX_BITS / 32 + 2], follow[32];
     const unsigned c = places.first + blockIdx.y, g = blockIdx.x, t = threadIdx.x, lane = t & 63;
     if (c >= b.count) {
         const unsigned row = c - b.count;
@@ -519,7 +528,7 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
     const kv_layout lay(b.heads, b.total, true);
     char *dst = places.at[blockIdx.y];
     const unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
-    const unsigned long long first = wg_bit[g], last = wg_bit[g + 1];
+    const unsigned long long first = wg_bit[g], last = wg_bit[g + 1], end = wg_bit[b.nwg];
     lc[t] = b.codes[(size_t)c * NUM_SYMBOLS + t];
     for (unsigned i = t; i < sizeof(words) / 4; i += KV_WG) words[i] = 0;
     const int8_t *q = b.q + (size_t)c * b.q_stride;
@@ -527,18 +536,18 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
     const unsigned count = base >= b.total ? 0u : min(b.total - base, (unsigned)ENC_SPT);
     uint4 v = {0, 0, 0, 0};
     if (count) v = *reinterpret_cast<const uint4 *>(q + base);  // (q is padded to a multiple of 16)
+    // the values that may fill this run's last word up: 31 bits, a value takes at least one
+    const unsigned beyond = (g + 1) * ENC_PER_WG + t;
+    if (t < 32) follow[t] = beyond < b.total ? (uint8_t)q[beyond] ^ 128u : NUM_SYMBOLS;
     __syncthreads();
     const unsigned sw[4] = {v.x, v.y, v.z, v.w};
-    unsigned bits = 0;
+    unsigned e[ENC_SPT], bits = 0;
 #pragma unroll
-    for (unsigned j = 0; j < ENC_SPT; ++j)
-        if (j < count) bits += lc[((sw[j >> 2] >> (8 * (j & 3))) & 255u) ^ 128u] >> 16;
-    unsigned incl = bits;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const unsigned o = __shfl_up(incl, d, 64);
-        incl += lane >= (unsigned)d ? o : 0u;
+    for (unsigned j = 0; j < ENC_SPT; ++j) {
+        e[j] = j < count ? lc[((sw[j >> 2] >> (8 * (j & 3))) & 255u) ^ 128u] : 0u;
+        bits += e[j] >> 16;
     }
+    const unsigned incl = wave_scan(bits);
     if (lane == 63) wsum[t >> 6] = incl;
     __syncthreads();
     unsigned start = incl - bits;  // within the run
@@ -551,7 +560,7 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
         unsigned long long acc = 0;
 #pragma unroll
         for (unsigned j = 0; j < ENC_SPT; ++j)
-            if (j < count && push_code(lc[((sw[j >> 2] >> (8 * (j & 3))) & 255u) ^ 128u], acc, nacc, word)) atomicOr(&words[k++], word);
+            if (push_code(e[j], acc, nacc, word)) atomicOr(&words[k++], word);
         if (nacc && count) atomicOr(&words[k], (unsigned)(acc << (32 - nacc)));
     }
     __syncthreads();
@@ -559,7 +568,7 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
         unsigned nacc = (unsigned)last & 31, k = (unsigned)((last >> 5) - (first >> 5)), word;
         unsigned long long acc = words[k] >> (32 - nacc);
         bool full = false;
-        for (unsigned i = (g + 1) * ENC_PER_WG; !full && i < b.total; ++i) full = push_code(lc[(unsigned)(uint8_t)q[i] ^ 128u], acc, nacc, word);
+        for (unsigned i = 0; !full && i < 32 && follow[i] < NUM_SYMBOLS; ++i) full = push_code(lc[follow[i]], acc, nacc, word);
         words[k] = full ? word : (unsigned)(acc << (32 - nacc));
     }
     __syncthreads();
@@ -573,10 +582,10 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
         const uint4 *lut = reinterpret_cast<const uint4 *>(b.lut + (size_t)c * KV_LUT);
         for (unsigned i = t; i < KV_LUT * 2 / 16; i += KV_WG) reinterpret_cast<uint4 *>(dst + lay.o_lut)[i] = lut[i];
         if (t == 0) {
-            reinterpret_cast<unsigned long long *>(dst + lay.o_wg)[b.nwg] = wg_bit[b.nwg];
+            reinterpret_cast<unsigned long long *>(dst + lay.o_wg)[b.nwg] = end;
             if (table) table[c] = dst;
         }
-        if (t < 4) reinterpret_cast<unsigned *>(dst + lay.o_bits)[(size_t)((wg_bit[b.nwg] + 31) >> 5) + t] = 0;  // the padding
+        if (t < 4) reinterpret_cast<unsigned *>(dst + lay.o_bits)[(size_t)((end + 31) >> 5) + t] = 0;  // the padding
     }
 }
 
@@ -602,6 +611,8 @@ __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a
     constexpr unsigned MAX_WORDS = DEC_PER_WG * KV_MAX_BITS / 32 + 4;
     __shared__ __attribute__((aligned(16))) uint16_t lut[KV_LUT];
     __shared__ unsigned words[MAX_WORDS];
+    constexpr unsigned DEC_SCALES = 64;
+    __shared__ float sc[DEC_SCALES];  // of the first heads that the workgroup meets
     __shared__ unsigned sym[KV_WG * (SUB_SYMS / 4 + 1)];  // four values a word; a thread's words start an odd number apart
     const unsigned t = threadIdx.x, nchunk = a.count * a.wgs;
     if (blockIdx.x >= nchunk) {  // the window
@@ -619,14 +630,28 @@ __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a
     const char *chunk = a.table ? a.table[c] : a.single;
     const kv_layout lay(a.heads, a.total, true);
     const uint4 *lut_g = reinterpret_cast<const uint4 *>(chunk + lay.o_lut);
-    for (unsigned i = t; i < KV_LUT * 2 / 16; i += KV_WG) reinterpret_cast<uint4 *>(lut)[i] = lut_g[i];
+    uint4 lut_v[KV_LUT * 2 / 16 / KV_WG];
+#pragma unroll
+    for (unsigned i = 0; i < KV_LUT * 2 / 16 / KV_WG; ++i) lut_v[i] = lut_g[i * KV_WG + t];
     constexpr unsigned RUNS = DEC_PER_WG / ENC_PER_WG;
     const unsigned long long *wg_bit = reinterpret_cast<const unsigned long long *>(chunk + lay.o_wg);
     const unsigned nwg = (a.total + ENC_PER_WG - 1) / ENC_PER_WG, r0 = g * RUNS, r1 = min(r0 + RUNS, nwg);
     const unsigned long long w0 = wg_bit[r0] >> 5, w1 = (wg_bit[r1] + 31) >> 5;
     const unsigned *stream = reinterpret_cast<const unsigned *>(chunk + lay.o_bits) + w0;
     const unsigned nwords = min((unsigned)(w1 - w0) + 3, MAX_WORDS);  // (up to 16 bytes of padding follow a stream)
-    for (unsigned i = t; i < nwords; i += KV_WG) words[i] = __builtin_bswap32(stream[i]);
+    for (unsigned at = 0; at < nwords; at += 8 * KV_WG) {  // eight loads in flight
+        unsigned w[8];
+#pragma unroll
+        for (unsigned j = 0; j < 8; ++j) w[j] = stream[min(at + j * KV_WG + t, nwords - 1)];
+#pragma unroll
+        for (unsigned j = 0; j < 8; ++j)
+            if (at + j * KV_WG + t < nwords) words[at + j * KV_WG + t] = __builtin_bswap32(w[j]);
+    }
+#pragma unroll
+    for (unsigned i = 0; i < KV_LUT * 2 / 16 / KV_WG; ++i) reinterpret_cast<uint4 *>(lut)[i * KV_WG + t] = lut_v[i];
+    const float *scales = reinterpret_cast<const float *>(chunk);
+    const unsigned h0 = g * DEC_PER_WG / a.head_elems;
+    if (t < DEC_SCALES) sc[t] = h0 + t < a.heads ? scales[h0 + t] : 0.0f;
     const unsigned base = g * DEC_PER_WG, sub = g * KV_WG + t;
     const unsigned count = base + t * SUB_SYMS >= a.total ? 0u : min(a.total - (base + t * SUB_SYMS), (unsigned)SUB_SYMS);
     unsigned pos = 0;
@@ -659,7 +684,6 @@ __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a
         }
     }
     __syncthreads();
-    const float *scales = reinterpret_cast<const float *>(chunk);
     float *out = a.out[c % a.sides] + (size_t)(c / a.sides) * a.chunk_step;
 #pragma unroll 4
     for (unsigned j = 0; j < DEC_PER_WG / (4 * KV_WG); ++j) {
@@ -668,7 +692,7 @@ __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a
         const unsigned four = sym[local / SUB_SYMS * (SUB_SYMS / 4 + 1) + local % SUB_SYMS / 4];
         if (VEC) {
             const unsigned h = i / a.head_elems;
-            const float scale = scales[h];
+            const float scale = h - h0 < DEC_SCALES ? sc[h - h0] : scales[h];
             float4 v;
             v.x = (float)((int)(four & 255u) - 128) * scale;
             v.y = (float)((int)(four >> 8 & 255u) - 128) * scale;
