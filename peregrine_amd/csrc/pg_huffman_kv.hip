@@ -11,7 +11,7 @@
 // encoder.  The host takes part once per batch: it learns the coded sizes (words that the table kernel stores in
 // pinned memory), allocates exactly that much and launches the encoder.  A batch was 10 launches, 12 copies and 8
 // waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
-// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.28.
+// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.25.
 //
 // The encoder knows where every code starts, so it leaves an index beside the stream (a 16-bit offset per 64 values,
 // 0.25 bit a value): the decoder of such a chunk is one launch that starts a thread per 64 values, with no search for
@@ -71,22 +71,43 @@ struct kv_batch {
     __device__ const float *head(unsigned c, unsigned h) const { return data[c % sides] + (size_t)(c / sides) * chunk_step + (size_t)h * head_stride; }
 };
 
-// Largest |v| of every head (NaN ignored, as f32::max does), one value per split: grid (splits, heads, chunks).
-__global__ __launch_bounds__(KV_WG) void kv_absmax_kernel(const kv_batch b, int vec) {
+// New rows on their way into the window, for the batch's first launch to write while it reads them: a head's values from `from`
+// on are `elems` values at src[side] + h * src_stride.  No rows: from is beyond every chunk and parts is 0.
+struct kv_incoming {
+    const float *src[2];
+    float *dst[2];  // where they go, heads `dst_stride` apart
+    size_t src_stride, dst_stride, from, elems;
+    unsigned parts;  // times as many workgroups per (side, head) as a chunk's head has
+};
+
+// Largest |v| of every head (NaN ignored, as f32::max does), one value per split; and the incoming rows' copy.  Grid
+// (heads * splits, chunks + sides * parts).  As two launches the copy took 4 us of an append's 43.
+template <class V>
+__global__ __launch_bounds__(KV_WG) void kv_absmax_kernel(const kv_batch b, const kv_incoming in) {
+    constexpr unsigned VN = sizeof(V) / 4;
     __shared__ float red[4];
-    const float *p = b.head(blockIdx.z, blockIdx.y);
+    const unsigned split = blockIdx.x % b.splits, h = blockIdx.x / b.splits, c = blockIdx.y;
+    if (c >= b.count) {
+        const unsigned side = (c - b.count) / in.parts, part = (c - b.count) % in.parts * b.splits + split;
+        const V *src = reinterpret_cast<const V *>(in.src[side] + (size_t)h * in.src_stride);
+        V *dst = reinterpret_cast<V *>(in.dst[side] + (size_t)h * in.dst_stride);
+        for (size_t i = (size_t)part * KV_WG + threadIdx.x; i < in.elems / VN; i += (size_t)in.parts * b.splits * KV_WG) dst[i] = src[i];
+        return;
+    }
+    const size_t at = (size_t)(c / b.sides) * b.chunk_step;  // of the head's first value in the window
+    const V *p = reinterpret_cast<const V *>(b.head(c, h));
+    const V *q = reinterpret_cast<const V *>(in.src[c % b.sides] + (size_t)h * in.src_stride);
+    const unsigned n = b.head_elems / VN, old = (unsigned)min((size_t)n, (in.from > at ? in.from - at : 0) / VN);
+    const size_t skip = at / VN - in.from / VN;  // of q's values, from window to incoming (wraps where the chunk starts in the window)
     float m = 0.0f;
-    if (vec) {
-        const unsigned n4 = b.head_elems / 4;
-        for (unsigned i = blockIdx.x * KV_WG + threadIdx.x; i < n4; i += gridDim.x * KV_WG) {
-            const float4 v = reinterpret_cast<const float4 *>(p)[i];
-            m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-        }
-    } else {
-        for (unsigned i = blockIdx.x * KV_WG + threadIdx.x; i < b.head_elems; i += gridDim.x * KV_WG) m = fmaxf(m, fabsf(p[i]));
+    for (unsigned i = split * KV_WG + threadIdx.x; i < n; i += b.splits * KV_WG) {
+        const V v = i < old ? p[i] : q[skip + i];
+        const float *x = reinterpret_cast<const float *>(&v);
+#pragma unroll
+        for (unsigned k = 0; k < VN; ++k) m = fmaxf(m, fabsf(x[k]));
     }
     m = pg_block_max_256(m, red);
-    if (threadIdx.x == 0) b.amax[((size_t)blockIdx.z * b.heads + blockIdx.y) * b.splits + blockIdx.x] = m;
+    if (threadIdx.x == 0) b.amax[((size_t)c * b.heads + h) * b.splits + split] = m;
 }
 
 // q = round(v / scale) clamped to +-127 with scale = amax / 127 (1 for an all-zero head), the scales, and the
@@ -835,10 +856,17 @@ struct kv_shift {
     bool done = false;
 };
 
+// New rows behind the window, for compress_batch's first launch to write (written = true).
+struct kv_rows {
+    kv_incoming in;
+    bool written = false;
+};
+
 // compress_chunk of `count` chunks of one shape (none of them empty), chunk c being number c / sides of side c % sides:
 // head h of it starts at data[side] + number * chunk_step + h * head_stride.  Their addresses go to table_dev[0 ..) if given.
+// `rows` (if given) are still to be written to the window behind data[]: the first launch does.
 static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t sides, size_t count, size_t chunk_step, size_t head_stride,
-                                size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift,
+                                size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift, kv_rows *rows,
                                 std::vector<std::unique_ptr<pg_huffman_kv_chunk>> &out) {
     const size_t head_elems = num_tokens * head_dim, total = num_heads * head_elems;
     const size_t nwg = (total + ENC_PER_WG - 1) / ENC_PER_WG;
@@ -874,7 +902,17 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         b.lut = reinterpret_cast<uint16_t *>(base + o_lut);
         uint64_t *sizes = static_cast<uint64_t *>(pin);
         std::fill(sizes, sizes + n, (uint64_t)0);
-        PG_TRY(pg_launch(ctx, "huffman_kv_absmax", kv_absmax_kernel, dim3(b.splits, b.heads, b.count), dim3(KV_WG), 0, b, (int)vec));
+        kv_incoming in = {{b.data[0], b.data[1]}, {nullptr, nullptr}, 0, 0, ~(size_t)0, 0, 0};
+        bool vec_in = vec;
+        if (rows && first == 0) {
+            in = rows->in;
+            vec_in = vec && in.from % 4 == 0 && in.elems % 4 == 0 && in.src_stride % 4 == 0 && in.dst_stride % 4 == 0;
+            for (size_t s = 0; s < 2; ++s) vec_in = vec_in && ((uintptr_t)in.src[s] | (uintptr_t)in.dst[s]) % 16 == 0;
+            in.parts = (unsigned)std::min<size_t>((in.elems + b.splits * ENC_PER_WG - 1) / (b.splits * ENC_PER_WG), KV_MAX_SPLITS);
+        }
+        PG_TRY(pg_launch(ctx, "huffman_kv_absmax", vec_in ? kv_absmax_kernel<float4> : kv_absmax_kernel<float>,
+                         dim3(b.splits * b.heads, b.count + (unsigned)sides * in.parts), dim3(KV_WG), 0, b, in));
+        if (rows) rows->written = true;
         PG_TRY(pg_launch(ctx, "huffman_kv_quant", kv_quant_hist_kernel, dim3(b.nwg, b.count), dim3(KV_WG), 0, b, (int)vec));
         PG_TRY(pg_launch(ctx, "huffman_kv_table", kv_table_kernel, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
         const kv_layout lay(num_heads, total, true);
@@ -933,7 +971,7 @@ static pg_status compress_dev(pg_ctx *ctx, const float *data, size_t head_stride
         return PG_OK;
     }
     std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
-    PG_TRY(compress_batch(ctx, &data, 1, 1, 0, head_stride, num_tokens, num_heads, head_dim, nullptr, nullptr, made));
+    PG_TRY(compress_batch(ctx, &data, 1, 1, 0, head_stride, num_tokens, num_heads, head_dim, nullptr, nullptr, nullptr, made));
     *out = made[0].release();
     return PG_OK;
 }
@@ -1179,7 +1217,8 @@ static pg_status table_reserve(pg_ctx *ctx, pg_huffman_kv_cache *c, size_t chunk
 
 // The reference compresses the oldest chunk_size tokens and shifts the rest to the front, once per
 // chunk; here every chunk that an append cuts, of both sides, is one batch and the window is shifted once.
-static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c) {
+// `rows`: the window's last ones, still to be written.
+static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c, kv_rows *rows) {
     pg_kv_cache *hot = c->hot;
     if (hot->len < c->compress_threshold) return PG_OK;
     const size_t hd = hot->head_dim, stride = hot->capacity * hd, heads = hot->num_kv_heads, tokens = c->chunk_size;
@@ -1189,7 +1228,7 @@ static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c) {
     const float *data[2] = {hot->k, hot->v};
     std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
     kv_shift shift{{hot->k, hot->v}, stride, chunks * tokens * hd, (hot->len - chunks * tokens) * hd};
-    const pg_status st = compress_batch(ctx, data, 2, 2 * chunks, tokens * hd, stride, tokens, heads, hd, c->table + c->k_chunks.size() * 2, &shift, made);
+    const pg_status st = compress_batch(ctx, data, 2, 2 * chunks, tokens * hd, stride, tokens, heads, hd, c->table + c->k_chunks.size() * 2, &shift, rows, made);
     size_t done = 0;
     for (size_t i = 0; i + 1 < made.size(); i += 2) {
         c->k_chunks.push_back(made[i].release());
@@ -1220,8 +1259,20 @@ PG_API pg_status pg_huffman_kv_cache_append_dev(pg_ctx *ctx, pg_huffman_kv_cache
     PG_CHECK_ARG(c != nullptr, "pg_huffman_kv_cache_append: null cache");
     PG_TRY(append_ok(ctx, c, seq_len));
     c->touch(ctx);
-    PG_TRY(pg_kv_cache_append_dev(ctx, c->hot, new_k_dev, new_v_dev, seq_len));
-    return compress_hot(ctx, c);
+    pg_kv_cache *hot = c->hot;
+    const size_t hd = hot->head_dim, had = hot->len;
+    if (seq_len == 0 || had + seq_len < c->compress_threshold) {
+        PG_TRY(pg_kv_cache_append_dev(ctx, hot, new_k_dev, new_v_dev, seq_len));
+        return compress_hot(ctx, c, nullptr);
+    }
+    PG_TRY(pg_kv_cache_append_room(ctx, hot, new_k_dev, new_v_dev, seq_len));
+    const size_t from = had * hd, stride = hot->capacity * hd;
+    float *k = hot->k + from, *v = hot->v + from;
+    kv_rows rows{{{new_k_dev, new_v_dev}, {k, v}, seq_len * hd, stride, from, seq_len * hd, 0}};
+    hot->len += seq_len;
+    const pg_status st = compress_hot(ctx, c, &rows);
+    if (!rows.written) PG_TRY(pg_launch_kv_rows(ctx, k, v, stride, new_k_dev, new_v_dev, seq_len * hd, seq_len * hd, hot->num_kv_heads));
+    return st;
 }
 
 PG_API pg_status pg_huffman_kv_cache_append(pg_ctx *ctx, pg_huffman_kv_cache *c, const float *new_k, const float *new_v,
@@ -1231,7 +1282,7 @@ PG_API pg_status pg_huffman_kv_cache_append(pg_ctx *ctx, pg_huffman_kv_cache *c,
     PG_TRY(append_ok(ctx, c, seq_len));
     c->touch(ctx);
     PG_TRY(pg_kv_cache_append(ctx, c->hot, new_k, new_v, seq_len));
-    return compress_hot(ctx, c);
+    return compress_hot(ctx, c, nullptr);
 }
 
 PG_API pg_status pg_huffman_kv_cache_get_kv_dev(pg_ctx *ctx, const pg_huffman_kv_cache *c, float *k_dev, float *v_dev) {

@@ -136,6 +136,7 @@ struct pg_kv_cache {
     mutable pg_dev_block k_mem, v_mem;
     void touch(const pg_ctx *ctx) const { k_mem.touch(ctx); v_mem.touch(ctx); }
 };
+pg_status pg_kv_cache_append_room(pg_ctx *ctx, pg_kv_cache *c, const float *new_k_dev, const float *new_v_dev, size_t seq_len);
 // dst[h * dst_stride + i] = src[h * src_stride + i] for i < width of every head h, key and value side in one launch (no overlap).
 pg_status pg_launch_kv_rows(pg_ctx *ctx, float *dst_k, float *dst_v, size_t dst_stride, const float *src_k, const float *src_v,
                             size_t src_stride, size_t width, size_t heads);

@@ -1898,15 +1898,20 @@ PG_API pg_status pg_kv_cache_rollback_to(pg_kv_cache *c, size_t new_len) {
     return PG_OK;
 }
 
+// What an append of seq_len > 0 positions does ahead of the rows' copy.
+pg_status pg_kv_cache_append_room(pg_ctx *ctx, pg_kv_cache *c, const float *new_k_dev, const float *new_v_dev, size_t seq_len) {
+    PG_CHECK_ARG(new_k_dev && new_v_dev, "pg_kv_cache_append: null pointer");
+    PG_CHECK_ARG(c->len + seq_len < (1ull << 31), "pg_kv_cache_append: length beyond 2^31");
+    c->touch(ctx);
+    return cache_reserve(ctx, c, c->len + seq_len);
+}
+
 PG_API pg_status pg_kv_cache_append_dev(pg_ctx *ctx, pg_kv_cache *c, const float *new_k_dev, const float *new_v_dev,
                                         size_t seq_len) {
     PG_TRY(pg_use(ctx));
     PG_CHECK_ARG(c != nullptr, "pg_kv_cache_append: null cache");
     if (seq_len == 0) return PG_OK;
-    PG_CHECK_ARG(new_k_dev && new_v_dev, "pg_kv_cache_append: null pointer");
-    PG_CHECK_ARG(c->len + seq_len < (1ull << 31), "pg_kv_cache_append: length beyond 2^31");
-    c->touch(ctx);
-    PG_TRY(cache_reserve(ctx, c, c->len + seq_len));
+    PG_TRY(pg_kv_cache_append_room(ctx, c, new_k_dev, new_v_dev, seq_len));
     const size_t hd = c->head_dim;
     PG_TRY(pg_launch_kv_rows(ctx, c->k + c->len * hd, c->v + c->len * hd, c->capacity * hd, new_k_dev, new_v_dev, seq_len * hd, seq_len * hd,
                              c->num_kv_heads));

@@ -276,3 +276,28 @@ def test_tables_at_the_edges_of_the_merges(ctx, orc, kind, total):
     chunk = huffman.HuffmanKVCache.compress_chunk(data, len(data), 1, 1, ctx)
     _same_chunk(chunk, orc.huffman_kv_compress_chunk(data, len(data), 1, 1))
     assert (huffman.HuffmanKVCache.decompress_chunk(chunk) == data).all()
+
+
+@pytest.mark.parametrize("heads,hd,thr,chunk,appends,skew", [
+    (4, 64, 48, 32, (40, 1, 1, 70, 1, 0, 200), 0),   # chunks of old rows, of old and new ones, of new ones alone
+    (4, 64, 48, 32, (40, 1, 70), 1),                 # rows that start off a 16-byte boundary
+    (3, 7, 5, 5, (3, 1, 1, 1, 24, 2), 0),            # no four values of one head
+    (2, 6, 4, 2, (1, 1, 1, 1, 3, 8), 0),             # whole quadruples in a chunk, not in the window's rows
+    (1, 1, 1, 1, (1100, 3), 0),                      # more chunks than one batch takes
+    (8, 128, 512, 256, (500, 500, 1100), 0),
+])
+def test_device_rows_are_written_with_the_maximum(ctx, orc, heads, hd, thr, chunk, appends, skew):
+    """append_dev where it cuts chunks: the launch that finds the chunks' maxima also writes the new rows."""
+    from peregrine_amd import huffman, _ffi
+    say(f"huffman kv device rows heads={heads} head_dim={hd} threshold={thr} chunk={chunk} appends={appends} skew={skew}")
+    c, o = huffman.HuffmanKVCache(heads, hd, thr, chunk, ctx), orc.HuffmanKVCache(heads, hd, thr, chunk)
+    rng = np.random.default_rng(hd)
+    for n in appends:
+        k, v = (rng.standard_normal(skew + heads * n * hd + 1).astype(np.float32) for _ in range(2))
+        dk, dv = DevBuf(ctx, host=k), DevBuf(ctx, host=v)
+        at = [C.c_void_p(d.ptr.value + 4 * skew) for d in (dk, dv)]
+        _ffi.check(_ffi.lib.pg_huffman_kv_cache_append_dev(ctx.handle, c._h, *at, n))
+        o.append(*(x[skew:skew + heads * n * hd].reshape(heads, n, hd) for x in (k, v)), n)
+        assert (c.len(), c.compressed_len) == (o.len, o.compressed_len)
+        for got, want in zip(c.get_kv(), o.get_kv()):
+            assert (got.view(np.uint32) == want.view(np.uint32)).all()
