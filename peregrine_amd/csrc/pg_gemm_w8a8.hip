@@ -28,6 +28,7 @@
 // MFMAs.
 #include <limits.h>
 #include "pg_internal.h"
+#include "pg_quant_dev.h"
 #include "pg_stream_addr.h"
 
 namespace {
@@ -467,6 +468,8 @@ struct skinny_wgroup {
     int wg0[PG_GEMM_MAX_GROUP];
 };
 
+constexpr int F32_ROWS_NST = 4;  // stages of gemm_w8a8_f32_rows_kernel's rings
+
 // TRI: the W8A32 product.  The activations are three digit planes a_plane bytes apart (weights 1, 256, 65536); tile b is
 // tile b % (MB / 3) of plane b / (MB / 3), and the final pass joins the three sums in f64.
 template <int MB, int NB, int NW, int NST, bool TRI = false>
@@ -597,6 +600,121 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
             if (out) out[o] = (float)sum * a_scales[row] * w_scales[col];
             if (acc_out) acc_out[o] = sum;
         }
+    }
+}
+
+// ---- 2 .. 8 short rows: quantised by every workgroup for itself, in the product's own launch ----------
+// The few-row kernel above with its rows still in f32: a wavefront quantises one of them (quantize_rows_vec4_kernel's
+// arithmetic: the same integers and scale) into LDS while its weights' first units are on their way.  The rows are asked for
+// ahead of the weights -- loads return in order -- and every unit of the prologue is requested whether the wavefront has
+// one or not (its last one again), so that the wait for the rows knows how many loads are behind them.  NW >= m wavefronts,
+// VK 128-bit vectors of a row to a lane; LDS: the rings of weights, then the rows, k_pad + 16 bytes apart (the fragments of
+// 16 rows in 16 bank groups).
+template <int NW, int VK>
+__global__ __launch_bounds__(64 * NW) void gemm_w8a8_f32_rows_kernel(const float *__restrict__ a, const skinny_wgroup grp, int k, int k_pad, int m) {
+    constexpr int TILE = 2048, NST = F32_ROWS_NST, LPS = 2;
+    static_assert(NST == 4, "three units in the prologue");
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    __shared__ float sc[NW];
+    int g = 0;
+#pragma unroll
+    for (int i = 1; i < PG_GEMM_MAX_GROUP; ++i) g = (int)blockIdx.x >= grp.wg0[i] ? i : g;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nvec = k >> 2, tail = k & 3;
+    const float *ar = a + (size_t)min(wave, m - 1) * k;
+    f4u v[VK];
+#pragma unroll
+    for (int i = 0; i < VK; ++i) v[i] = *reinterpret_cast<const f4u *>(ar + 4 * min(lane + 64 * i, nvec - 1));
+    const float tv = ar[lane < tail ? 4 * nvec + lane : 0];
+    __builtin_amdgcn_sched_barrier(0);
+
+    const int8_t *__restrict__ w_t = grp.w[g];
+    const int n = grp.n[g], n0 = ((int)blockIdx.x - grp.wg0[g]) * 16;
+    const int units = k_pad / 128, per = (units + NW - 1) / NW;
+    const int u_begin = min(wave * per, units - 1), cnt = min((wave + 1) * per, units) - wave * per, run = max(cnt, 1);
+    char *ring = lds + wave * NST * TILE;
+    const int8_t *src[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int r = 8 * j + (lane >> 3), ch = (lane & 7) ^ ((r >> 1) & 7);
+        src[j] = w_t + pg_skinny_fill_offset(n0 + r, k_pad, 0, ch);  // (weight rows are padded to 256)
+    }
+    const int rot = (int)((blockIdx.x * 5u) % (unsigned)run);
+    auto issue = [&](auto slot, int t) {
+        const size_t kb = (size_t)pg_skinny_walk_unit(u_begin, run, t, rot) * 128;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + kb), (lptr_t)(ring + decltype(slot)::value * TILE + j * 1024), 16, 0, 2);
+    };
+    issue(std::integral_constant<int, 0>{}, 0);
+    issue(std::integral_constant<int, 1>{}, min(1, run - 1));
+    issue(std::integral_constant<int, 2>{}, min(2, run - 1));
+    __builtin_amdgcn_sched_barrier(0);
+
+    char *rows = lds + NW * NST * TILE;
+    const int stride = k_pad + 16;
+    if (wave < m) {
+        float amax = lane < tail ? fmaxf(0.0f, fabsf(tv)) : 0.0f;
+#pragma unroll
+        for (int i = 0; i < VK; ++i) {
+            const float m4 = fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w)));
+            amax = fmaxf(amax, lane + 64 * i < nvec ? m4 : 0.0f);
+        }
+        amax = pg_wave_max_f32(amax);
+        const float scale = (amax == 0.0f) ? 1.0f : amax / 127.0f;
+        const float inv = 1.0f / scale;
+        if (lane == 0) sc[wave] = scale;
+        int8_t *q = reinterpret_cast<int8_t *>(rows + wave * stride);
+#pragma unroll
+        for (int i = 0; i < VK; ++i) {
+            const int idx = lane + 64 * i;
+            if (idx < nvec) {
+                const int b0 = pg_quant_to_i8(v[i].x * inv) & 0xFF, b1 = pg_quant_to_i8(v[i].y * inv) & 0xFF;
+                const int b2 = pg_quant_to_i8(v[i].z * inv) & 0xFF, b3 = pg_quant_to_i8(v[i].w * inv) & 0xFF;
+                reinterpret_cast<int *>(q)[idx] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
+            }
+        }
+        if (tail && lane < 4) q[4 * nvec + lane] = (int8_t)(lane < tail ? pg_quant_to_i8(tv * inv) : 0);
+        for (int idx = nvec + (tail != 0) + lane; idx < k_pad / 4; idx += 64) reinterpret_cast<int *>(q)[idx] = 0;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");  // (the weights stay in flight)
+
+    // fragment reads: row lane % 16 of the weights' tile and of the rows (beyond m the last one again, never stored)
+    const int fr = lane & 15, fsw = (fr >> 1) & 7;
+    const char *arow = rows + min(fr, m - 1) * stride + (lane >> 4) * 16;
+    int rd[2];
+#pragma unroll
+    for (int st = 0; st < 2; ++st) rd[st] = fr * 128 + (((4 * st + (lane >> 4)) ^ fsw) * 16);
+    v4i acc = v4i{0, 0, 0, 0};
+    for (int t0 = 0; t0 < cnt; t0 += NST) {
+#define PG_F32R_STEP(U)                                                                                        \
+        if (t0 + U < cnt) {                                                                                    \
+            const int t = t0 + U;                                                                              \
+            if (t + NST - 2 < cnt) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * LPS) : "memory");      \
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                              \
+            if (t + NST - 1 < cnt) issue(std::integral_constant<int, (U + NST - 1) % NST>{}, t + NST - 1);     \
+            __builtin_amdgcn_sched_barrier(0);                                                                 \
+            const char *ap = arow + pg_skinny_walk_unit(u_begin, run, t, rot) * 128, *wp = ring + U * TILE;    \
+            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<const v4i *>(ap), *reinterpret_cast<const v4i *>(wp + rd[0]), acc, 0, 0, 0);      \
+            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<const v4i *>(ap + 64), *reinterpret_cast<const v4i *>(wp + rd[1]), acc, 0, 0, 0); \
+            __builtin_amdgcn_sched_barrier(0);                                                                 \
+        }
+        PG_F32R_STEP(0) PG_F32R_STEP(1) PG_F32R_STEP(2) PG_F32R_STEP(3)
+#undef PG_F32R_STEP
+    }
+    __syncthreads();
+    int *red = reinterpret_cast<int *>(lds);  // [NW][4][64]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[(wave * 4 + i) * 64 + lane] = acc[i];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 4 * 64; e += 64 * NW) {
+        const int l = e & 63, i = e >> 6;
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += red[(w * 4 + i) * 64 + l];
+        const int row = 4 * (l >> 4) + i, col = n0 + (l & 15);
+        if (row < m && col < n) grp.out[g][(size_t)row * n + col] = (float)sum * sc[row] * grp.ws[g][col];
     }
 }
 
@@ -796,6 +914,45 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
 pg_status pg_launch_gemm_w8a8_skinny(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                                      const pg_qtensor *w, size_t m, float *out, int32_t *acc) {
     return pg_launch_gemm_w8a8_skinny_group(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, acc);
+}
+
+// 2 .. 8 short rows in f32 (gemm_w8a8_f32_rows_kernel): as long as a workgroup repeats the quantisation in less time than a
+// launch takes, and all workgroups are resident at once.  us, two launches : this one (the first ones wait for the host):
+// 2 x 128 -> 256 5.4 : 3.1, 3 x 768 -> 3072 7.4 : 4.0, 4 x 1024 -> 8192 6.2 : 5.3, 4 x 2048 -> 8192 7.6 : 7.4, 4 x 1024 -> 14336
+// 7.1 : 6.8, 8 x 1536 -> 3072 6.4 : 6.0, 8 x 768 -> 8192 6.3 : 5.9; past the lines 4 x 4096 -> 4096 7.9 : 8.1, 4 x 2048 ->
+// 14336 9.6 : 11.2, 4 x 256 -> 32000 6.1 : 7.8, 8 x 2048 -> 3072 6.3 : 6.4, 8 x 1024 -> 8192 6.1 : 6.4, 8 x 256 -> 14336 5.6 : 6.9.
+bool pg_gemm_w8a8_takes_f32_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
+    size_t cols = 0;
+    for (int i = 0; i < count; ++i) {
+        if (w[i]->k_pad != w[0]->k_pad || w[i]->cols >= (1ull << 30)) return false;
+        cols += w[i]->cols;
+    }
+    const size_t k = w[0]->rows, tiles = cols / 16 / (size_t)ctx->num_cu;  // whole rounds of 16 columns a CU
+    if (m < 2 || m > 8 || k < 4) return false;
+    return m <= 4 ? k < 2052 && tiles < (k < 1028 ? 4 : 2) : k < 1540 && tiles < (k < 772 ? 2 : 1);
+}
+pg_status pg_launch_gemm_w8a8_f32_rows(pg_ctx *ctx, const float *a, const pg_qtensor *const *w, float *const *out, int count, size_t m) {
+    if (count < 1 || count > PG_GEMM_MAX_GROUP || !pg_gemm_w8a8_takes_f32_rows(ctx, w, count, m))
+        return pg_fail(PG_EINVAL, "gemm_w8a8 (rows in f32): m = %zu, %d weights", m, count);
+    skinny_wgroup grp;
+    int wgs = 0;
+    for (int i = 0; i < PG_GEMM_MAX_GROUP; ++i) {
+        const bool used = i < count;
+        grp.w[i] = used ? w[i]->w_t : nullptr;
+        grp.ws[i] = used ? w[i]->scales : nullptr;
+        grp.out[i] = used ? out[i] : nullptr;
+        grp.n[i] = used ? (int)w[i]->cols : 0;
+        grp.wg0[i] = used ? wgs : INT_MAX;
+        if (used) wgs += (int)((w[i]->cols + 15) / 16);
+    }
+    const size_t k = w[0]->rows, k_pad = w[0]->k_pad;
+    auto go = [&](auto kern, int nw) -> pg_status {
+        const size_t lds = (size_t)nw * F32_ROWS_NST * 2048 + m * (k_pad + 16);
+        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
+        return pg_launch(ctx, "gemm_w8a8_f32_rows", kern, dim3((unsigned)wgs), dim3(64 * nw), lds, a, grp, (int)k, (int)k_pad, (int)m);
+    };
+    if (m <= 4) return k < 516 ? go(gemm_w8a8_f32_rows_kernel<4, 2>, 4) : k < 1028 ? go(gemm_w8a8_f32_rows_kernel<4, 4>, 4) : go(gemm_w8a8_f32_rows_kernel<4, 8>, 4);
+    return k < 516 ? go(gemm_w8a8_f32_rows_kernel<8, 2>, 8) : k < 1028 ? go(gemm_w8a8_f32_rows_kernel<8, 4>, 8) : go(gemm_w8a8_f32_rows_kernel<8, 6>, 8);
 }
 
 // a_i8 must have at least round_up(m, 256) rows of a_stride bytes (rows >= m may

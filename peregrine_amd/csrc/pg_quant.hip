@@ -558,7 +558,8 @@ constexpr size_t PG_GEMV_MAX_M = 4;
 // comes from the context's arena, or from `fixed` (of fixed_cap bytes) when that is given: then
 // nothing is allocated and a request that does not fit is an error.
 static pg_status matmul_quantized_on(pg_ctx *ctx, const float *a_dev, size_t m, size_t k, const pg_qtensor *w,
-                                     float *out_dev, int32_t *acc_dev, void *fixed, size_t fixed_cap) {
+                                     float *out_dev, int32_t *acc_dev, void *fixed, size_t fixed_cap, bool remote = false) {
+    if (!acc_dev && !remote && pg_gemm_w8a8_takes_f32_rows(ctx, &w, 1, m)) return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, &w, &out_dev, 1, m);
     if (pg_gemv_w8a8_takes_f32_row(w, m, k, a_dev)) return pg_launch_gemv_w8a8_f32_row(ctx, a_dev, k, w, out_dev, acc_dev);
     const size_t m_pad = pg_round_up(m, PG_MPAD);
     const size_t a_bytes = m_pad * w->k_pad;
@@ -669,6 +670,7 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     for (size_t i = 0; i < count && one_row_group; ++i) one_row_group = pg_gemv_w8a8_takes_f32_row(w[i], m, k, a_dev);
     if (one_row_group)  // one token: every weight's rows in one streaming launch that quantises the row itself
         return pg_launch_gemv_w8a8_f32_row_group(ctx, a_dev, k, w, out_dev, (int)count, nullptr);
+    if (count > 1 && pg_gemm_w8a8_takes_f32_rows(ctx, w, (int)count, m)) return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, w, out_dev, (int)count, m);
     bool skinny_group = count > 1;
     for (size_t i = 0; i < count && skinny_group; ++i) skinny_group = pg_gemm_w8a8_takes_skinny(w[i], m) && w[i]->k_pad == w[0]->k_pad;
     if (skinny_group) {  // 2 .. 64 rows: quantised once, then the weights side by side in one launch
@@ -805,6 +807,7 @@ PG_API pg_status pg_matmul_quantized(pg_ctx *ctx, const float *a, size_t m, size
         a_dev = da.as<float>();
     }
     PG_TRY(dout.alloc(ctx, m * w->cols * sizeof(float)));
-    PG_TRY(pg_matmul_quantized_dev(ctx, a_dev, m, k, w, dout.as<float>(), nullptr));
+    PG_CHECK_ARG(m < (1ull << 24), "pg_matmul_quantized: m = %zu too large", m);
+    PG_TRY(matmul_quantized_on(ctx, a_dev, m, k, w, dout.as<float>(), nullptr, nullptr, 0, a_dev != da.as<float>()));
     return pg_host_out(ctx, out, dout.p, m * w->cols * sizeof(float));
 }

@@ -679,3 +679,43 @@ def test_few_rows_over_wide_weights_bit_exact(ctx, orc, m, k, n):
     assert (bits(got[:, cols]) == bits(want)).all()
     assert (np.abs(got).max(axis=0) > 0).all(), "a column was left out"
     qt.free_gpu()
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (2, 4, 1), (3, 5, 15), (4, 7, 17), (8, 127, 16), (5, 128, 33), (2, 129, 256),                # part vectors, part tiles
+    (4, 515, 64), (4, 516, 64), (2, 1027, 100), (3, 1028, 100), (4, 2051, 40), (4, 2052, 40),    # vectors to a lane; past the rule
+    (8, 515, 64), (6, 516, 64), (8, 1027, 100), (5, 1028, 100), (8, 1539, 40), (7, 1540, 40),
+    (4, 1027, 16383), (4, 1027, 16384), (4, 1028, 8191), (4, 1028, 8192),                         # columns, both sides
+    (5, 771, 8191), (5, 771, 8192), (8, 772, 4095), (8, 772, 4096),
+])
+def test_short_f32_rows_bit_exact(ctx, orc, m, k, n):
+    """Rows that every workgroup quantises for itself, at the edges of a lane's vectors and of the rule, alone and as
+    two weights over one input, on device pointers; with a row of zeros, a NaN and halves that round away from zero."""
+    from devbuf import DevBuf
+    from peregrine_amd import quant, _ffi
+    say(f"short f32 rows m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + 10 * k + n)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, ::53] *= 20.0
+    a[1] = 0.0
+    a[0, :3] = 127.0, 63.5, np.nan
+    a[0] = np.clip(a[0], -127, 127)
+    a_dev = DevBuf(ctx, host=a)
+    qa, s = orc.quantize_activations(a, m, k)
+    cols = [n, max(1, n // 3)] if n < 4096 else [n - 16, 16]
+    qts, wants = [], []
+    for c in cols:
+        q = rng.integers(-127, 128, (k, c), dtype=np.int8)
+        scales = rng.uniform(0.5e-3, 2e-3, c).astype(np.float32)
+        qts.append(quant.QuantizedTensor(q.reshape(-1), None, scales, k, c).to_gpu(ctx))
+        acc = np.asarray(qa, np.float64).reshape(m, k) @ q.astype(np.float64)
+        wants.append(acc.astype(np.float32) * np.asarray(s, np.float32)[:, None] * scales[None, :])
+    outs = [DevBuf(ctx, nbytes=4 * m * c) for c in cols]
+    for qt, want, out, c in zip(qts, wants, outs, cols):
+        _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, a_dev.ptr, m, k, qt._gpu, out.ptr, None))
+        assert (bits(out.to_host(np.float32).reshape(m, c)) == bits(want)).all()
+    outs = [DevBuf(ctx, nbytes=4 * m * c) for c in cols]
+    tab = lambda v: (C.c_void_p * len(v))(*v)
+    _ffi.check(_ffi.lib.pg_matmul_quantized_multi_dev(ctx.handle, a_dev.ptr, m, k, tab([t._gpu.value for t in qts]), 2, tab([o.ptr.value for o in outs])))
+    for want, out, c in zip(wants, outs, cols):
+        assert (bits(out.to_host(np.float32).reshape(m, c)) == bits(want)).all()
