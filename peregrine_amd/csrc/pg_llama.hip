@@ -19,6 +19,7 @@
 #include "pg_internal.h"
 #include "pg_digits.h"
 #include "pg_f16_planes.h"
+#include "pg_quant_dev.h"
 
 struct pg_rope {
     float *cos_t, *sin_t;
@@ -993,6 +994,8 @@ void gqa_attention_mfma_kernel(attn_args aa, int n_items, int nkvh) {
     }
 }
 
+#include "pg_attn_halves.h"
+
 // ---- one query token, head size 64 or 128: the heads of a kv group together ----
 // A workgroup owns (kv head, split of the keys) and serves every query head of the group from one read
 // of the split's keys and values.  HD / 8 lanes share a key, eight dims each -- i .. i+3 and HD/2 + i ..
@@ -1512,6 +1515,58 @@ bool split_mfma_tiles(const pg_ctx *ctx, size_t group, size_t seq_q, size_t nkv,
     return *splits > 1;
 }
 
+// Whether many rows go to gqa_attention_halves_kernel, and how: *chunk tiles to a run, *runs at the most, the planes' bytes and
+// those of the runs' records.
+//
+// Against the f32 kernels (us, f32 : this): 777 tokens behind 100 of 32 / 8 heads of 128 108 : 54, 1024 behind 2048 457 : 176, 1000
+// behind 30000 4648 : 1464, 777 behind 100 of heads of 64 64 : 37; its 2-norm error against 64 bits 3.4e-7 : 5.0e-7, 5.4e-7 :
+// 9.7e-7 and so on down (attention over N(0, 1) keys; 0.5 to 0.8 of the f32 kernels' with outlier channels and steep scores too).
+// The line is drawn by estimates from 200 shapes (4 .. 1000 tokens behind 0 .. 30000): 200 tokens behind 300 79 : 31, 64 behind
+// 2000 44 : 33, but 32 behind 300 16 : 21 and 16 behind 8000 38 : 58; the worst pick among them is 64 behind 8000 of 4 heads of
+// 64, 37 : 40, and of those that stay 128 behind 300, 33 : 27.
+struct halves_plan {
+    size_t blocks, tiles, chunk, runs, plane_bytes, part_bytes;
+};
+bool plan_halves(pg_ctx *ctx, size_t group, size_t seq_q, size_t nkv, size_t hd, int mask_kind, size_t offset, size_t len, bool digits, halves_plan *p) {
+    const size_t kend = mask_kind != 0 && offset + seq_q < len ? offset + seq_q : len, rows = group * seq_q, cus = (size_t)ctx->num_cu;
+    if (rows < 64) return false;
+    p->blocks = (rows + HALVES_ROWS - 1) / HALVES_ROWS;
+    p->tiles = (kend + 31) / 32;
+    p->plane_bytes = pg_round_up(half_scales_offset(hd == 64 ? half_unit_bytes<64>() : half_unit_bytes<128>(), nkv, p->tiles) + nkv * p->tiles * sizeof(float2), 256);
+    if (p->plane_bytes > (256u << 20) || rows * group >= (1ull << 32)) return false;
+    auto tiles_of = [&](size_t b) {
+        const size_t last = std::min(b * HALVES_ROWS + HALVES_ROWS - 1, rows - 1) / group;
+        return mask_kind != 0 ? (std::min(len, offset + last + 1) + 31) / 32 : p->tiles;
+    };
+    const size_t first = tiles_of(0), sum = (first + p->tiles) * p->blocks / 2;  // (key tiles of a block of rows grow evenly)
+    // the shortest runs that leave every workgroup resident at once (two a CU); where the blocks alone are that many, one run
+    size_t chunk = std::max<size_t>((p->tiles + HALVES_RUNS_MAX - 1) / HALVES_RUNS_MAX, std::max<size_t>(4, sum * nkv / (2 * cus)));
+    if (p->blocks * nkv > 2 * cus) chunk = std::max<size_t>(chunk, p->tiles);
+    for (; chunk < p->tiles; chunk += 1 + chunk / 16) {
+        size_t wgs = 0;
+        for (size_t b = 0; b < p->blocks; ++b) wgs += (tiles_of(b) + chunk - 1) / chunk;
+        if (wgs * nkv <= 2 * cus) break;
+    }
+    p->chunk = chunk;
+    p->runs = (p->tiles + chunk - 1) / chunk;
+    if (chunk > (size_t)HALVES_CHUNK_MAX || p->runs > (size_t)HALVES_RUNS_MAX) return false;
+    p->part_bytes = p->runs > 1 ? pg_round_up(rows * nkv * p->runs * (hd + 4) * sizeof(float), 256) : 0;
+    // both sides in us: a tile of 32 keys takes a wavefront 5 to 6 with f32 matrix instructions, one on each of 1024 SIMDs, and here
+    // 1.6, or 1.3 of a workgroup's chain where they do not fill the chip; the planes are written at 2.2 TB/s
+    const double size = hd / 128.0, work = 4.0 * sum * nkv / (4.0 * cus), waves = 4.0 * p->blocks * nkv;
+    size_t c = 0, r = 0;
+    const double f32 = split_mfma_tiles(ctx, group, seq_q, nkv, mask_kind, offset, len, &c, &r)
+                           ? 16 + 6.3 * size * work : 14 + 2.5 * size * (first + p->tiles) * std::max(1.0, waves / (4.0 * cus));
+    const double f16 = (p->runs > 1 ? 20 : 12) + (digits ? 5 : 0) + size * std::max(1.6 * work, 1.3 * chunk) + p->plane_bytes / 2.2e6;
+    if (f16 >= f32) return false;
+    if (p->plane_bytes + p->part_bytes + len / 8 + 512 > ctx->ws_bytes) {  // a capturing stream cannot have the arena grow
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) (void)hipGetLastError();
+        if (st != hipStreamCaptureStatusNone) return false;
+    }
+    return true;
+}
+
 pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, const pg_kv_cache *vc, size_t nqh,
                            size_t seq_q, float scale, int mask_kind, size_t offset, size_t window, size_t sink,
                            float logit_cap, float *out, int accumulate, const pg_xdigits *xd = nullptr, int digit_kind = 0,
@@ -1553,7 +1608,8 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
     // short kernel handles with every load in flight at once.
     const size_t rows = seq_q * nqh, keys_per_round = 256 / (size_t)lanes;
     size_t chunk, splits;
-    bool short_kernel = false, tiled_kernel = false, decode_kernel = false, split_kernel = false;
+    bool short_kernel = false, tiled_kernel = false, decode_kernel = false, split_kernel = false, halves_kernel = false;
+    halves_plan lp = {};
     int dec_u = 1, dec_tps = 1;
     const uintptr_t align_all = (uintptr_t)q | (uintptr_t)out | (uintptr_t)kc->k | (uintptr_t)vc->v |
                                 (rope_fusion ? (uintptr_t)rope_fusion->raw_q | (uintptr_t)rope_fusion->raw_k | (uintptr_t)rope_fusion->raw_v |
@@ -1573,6 +1629,11 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         chunk = tps * u * tile_rows;
         dec_u = (int)u; dec_tps = (int)tps;
         decode_kernel = true;
+    } else if (seq_q > 1 && (hd == 64 || hd == 128) && align_all % 16 == 0 && !attention_is_short(ctx, rows, len, hd) &&
+               plan_halves(ctx, nqh / kc->num_kv_heads, seq_q, kc->num_kv_heads, hd, mask_kind, offset, len, md != nullptr, &lp)) {
+        halves_kernel = true;
+        splits = 1;
+        chunk = len;
     } else if (seq_q > 1 && (hd == 64 || hd == 128) && align_all % 16 == 0 && split_mfma_tiles(ctx, nqh / kc->num_kv_heads, seq_q,
                                                                                                  kc->num_kv_heads, mask_kind, offset, len, &chunk, &splits)) {
         // few rows under a long cache: the matrix-core kernel over runs of key tiles, then the merge
@@ -1595,9 +1656,13 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
     const size_t part_hdr = split_kernel ? 4 : 2;  // floats ahead of a partial row (maximum, exp-sum, padding)
     const size_t part_bytes = splits > 1 || decode_kernel ? pg_round_up(rows * splits * (hd + part_hdr) * sizeof(float), 256) : 0;
     const size_t bits_words = mask_kind == PG_MASK_LOCAL_GLOBAL ? (len + 31) / 32 : 0;
-    if (part_bytes + bits_words) {
+    const size_t half_bytes = halves_kernel ? lp.plane_bytes + lp.part_bytes : 0;
+    char *halves_planes = nullptr;
+    if (part_bytes + bits_words + half_bytes) {
         void *ws = nullptr;
-        PG_TRY(pg_workspace(ctx, part_bytes + bits_words * sizeof(uint32_t), &ws));
+        const size_t o_halves = pg_round_up(part_bytes + bits_words * sizeof(uint32_t), 256);
+        PG_TRY(pg_workspace(ctx, o_halves + half_bytes, &ws));
+        halves_planes = static_cast<char *>(ws) + o_halves;
         if (part_bytes) aa.part = static_cast<float *>(ws);
         if (bits_words) {
             // The global positions become one bit per key position (positions past the cache
@@ -1632,7 +1697,23 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         if (wgs >= (1ull << 31)) return pg_fail(PG_EUNSUPPORTED, "gqa_attention: grid too large");
         PG_TRY(pg_launch(ctx, "gqa_attention_short", gqa_attention_short_kernel, dim3((unsigned)wgs), dim3(256), 0, aa));
     }
-    else if (tiled_kernel && (hd == 64 || hd == 128)) {
+    else if (halves_kernel) {
+        const size_t nkv = kc->num_kv_heads;
+        if (lp.blocks * nkv * lp.runs >= (1ull << 31)) return pg_fail(PG_EUNSUPPORTED, "gqa_attention: grid too large");
+        PG_TRY(pg_launch(ctx, "kv_halves", hd == 64 ? kv_halves_kernel<64> : kv_halves_kernel<128>, dim3((unsigned)lp.tiles, (unsigned)nkv), dim3(256), 0,
+                         aa.kc, aa.vc, aa.k_stride, aa.v_stride, (int)std::min(len, lp.tiles * 32), halves_planes));
+        aa.chunk = (int)lp.chunk;
+        aa.splits = (int)lp.runs;
+        aa.part = reinterpret_cast<float *>(halves_planes + lp.plane_bytes);
+        auto *kern = hd == 64 ? gqa_attention_halves_kernel<64> : gqa_attention_halves_kernel<128>;
+        const size_t lds_bytes = halves_lds_bytes(hd == 64 ? half_unit_bytes<64>() : half_unit_bytes<128>());
+        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds_bytes));
+        PG_TRY(pg_launch(ctx, "gqa_attention_halves", kern, dim3((unsigned)(lp.blocks * nkv * lp.runs)), dim3(256), lds_bytes, aa, (const char *)halves_planes,
+                         (int)lp.blocks, (int)nkv, (int)lp.tiles));
+        if (lp.runs > 1)
+            PG_TRY(pg_launch(ctx, "gqa_attention_halves_combine", hd == 64 ? attn_halves_combine_kernel<64> : attn_halves_combine_kernel<128>,
+                             dim3((unsigned)((rows * (hd / 4) + 255) / 256)), dim3(256), 0, aa));
+    } else if (tiled_kernel && (hd == 64 || hd == 128)) {
         // matrix-core kernel: one workgroup per kv head and pair of 32-row items (first with last, ...);
         // the kv head varies fastest, so with eight kv heads each XCD's L2 keeps one head's keys and values
         const size_t G = nqh / kc->num_kv_heads, n_items = (G * seq_q + 31) / 32, pairs = (n_items + 1) / 2;

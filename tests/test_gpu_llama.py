@@ -474,3 +474,101 @@ def test_llama_block_rollback_and_errors(ctx, orc):
     with pytest.raises(_ffi.PeregrineError):
         llama.LlamaBlock(128, 4, 3, 32, 256, 8, 10000.0, 1e-5, ctx)      # 4 query heads over 3 kv heads
     assert blk.forward(np.zeros((0, 128), np.float32), cache).shape == (0, 128)
+
+
+@pytest.mark.parametrize("nqh,nkvh,hd,seq_q,length,mask,cap", [
+    (4, 4, 128, 300, 300, "causal", None),        # one head per kv head; blocks of 128 rows, the last of 44
+    (32, 8, 128, 129, 2001, "causal", None),      # several runs of key tiles, a tile that is not full
+    (6, 2, 64, 171, 700, "causal", 3.0),          # group 3: 513 rows, a block of one; a logit cap
+    (16, 2, 64, 333, 333, "causal", None),
+    (8, 1, 128, 700, 700, "none", None),
+    (8, 8, 64, 400, 1030, "sliding", None),       # whole runs hidden for some rows
+    (8, 2, 128, 260, 900, "global", None),
+    (4, 2, 128, 512, 513, "causal", None),
+    (8, 2, 64, 1025, 1025, "causal", 20.0),
+])
+def test_gqa_attention_of_halves(ctx, orc, nqh, nkvh, hd, seq_q, length, mask, cap):
+    """Rows and keys as pairs of halves on the f16 matrix cores: edges of the blocks of rows, of the key tiles and of
+    their runs, every mask kind."""
+    from peregrine_amd import llama
+    M = llama.AttentionMask
+    say(f"attention of halves {nqh}/{nkvh} x {hd}, {seq_q} of {length}, {mask}, cap {cap}")
+    at = length - seq_q
+    m = {"causal": M.causal(at), "none": M.none(), "sliding": M.causal_sliding_window(at, 150, 4),
+         "global": M.local_global(at, 40, [0, 7, 64, 300, 301, length - 1, 9999])}[mask]
+    _attention_case(ctx, orc, nqh, nkvh, hd, seq_q, length, m, cap, 500 + seq_q)
+
+
+def _attention_f64(q, k, v, scale, at):
+    nqh, seq, _ = q.shape
+    g = nqh // k.shape[0]
+    hide = np.arange(k.shape[1])[None, :] > at + np.arange(seq)[:, None]
+    out, mag = np.empty((seq, nqh, k.shape[2])), np.empty((seq, nqh, k.shape[2]))
+    for i in range(nqh):
+        s = q[i].astype(np.float64) @ k[i // g].astype(np.float64).T * scale
+        s[hide] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        out[:, i], mag[:, i] = p @ v[i // g].astype(np.float64), p @ np.abs(v[i // g].astype(np.float64))
+    return out, mag
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_gqa_attention_of_halves_over_a_wide_range(ctx, orc, hd):
+    """Tiles of values and keys whose magnitudes lie far apart (a scale to a tile, one unit for the sums), keys of zeros, a scale
+    below zero.  Bound, of the row's sum of p |v|: a score's sum takes 3 hd / 16 steps of up to one rounding of its sum of
+    |q k| each, beside 2^-22 of it for the halves (2^-18 with both p's in a quotient), the second sum 6 steps a tile, 114 in all
+    (2^-17); and, for what is small beside a tile seen before, 2^-37 of the largest value (halves are 2^-39 of the unit apart)."""
+    from peregrine_amd import llama
+    say(f"attention of halves, wide range, head size {hd}")
+    nqh, nkvh, seq, n = 8, 2, 256, 600
+    rng = np.random.default_rng(hd)
+    for scale, spread in ((hd ** -0.5, (1e-3, 1.0, 300.0, 0.0, 1e-6)), (-0.05, (1.0, 1.0))):
+        k, v = (rng.standard_normal((nkvh, n, hd)).astype(np.float32) for _ in range(2))
+        q = rng.standard_normal((nqh, seq, hd)).astype(np.float32)
+        for t in range((n + 31) // 32):
+            v[:, 32 * t:32 * t + 32] *= spread[t % len(spread)]
+            k[:, 32 * t:32 * t + 32] *= (1.0, 0.01, 2.0, 0.0)[t % 4]
+        q[:, ::5] *= 1e-4
+        cache = llama.StandardKVCache(nkvh, hd, ctx)
+        cache.append(k, v, n)
+        got = np.zeros(seq * nqh * hd, np.float32)
+        llama.gqa_attention(q, cache, cache, nqh, nkvh, seq, hd, scale, llama.AttentionMask.causal(n - seq), None, got, ctx)
+        want, mag = _attention_f64(q, k, v, scale, n - seq)
+        err = np.abs(got.reshape(want.shape) - want)
+        sums = max(abs(scale) * (np.abs(q[i]).astype(np.float64) @ np.abs(k[i // 4]).astype(np.float64).T).max() for i in range(nqh))
+        assert (err <= (2.0 ** -18 * sums + 2.0 ** -17) * mag + 2.0 ** -37 * np.abs(v).max()).all(), (err / (mag + 1e-30)).max()
+
+
+def test_gqa_attention_of_halves_not_finite(ctx, orc):
+    """An infinite value comes out where it is weighted, a NaN of a query in its row, an infinite key in the rows that see it;
+    nothing else changes."""
+    from peregrine_amd import llama
+    say("attention of halves, values that are not finite")
+    nqh, nkvh, hd, seq, n = 8, 2, 128, 256, 600
+    rng = np.random.default_rng(5)
+    k, v = (rng.standard_normal((nkvh, n, hd)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((nqh, seq, hd)).astype(np.float32)
+    q[3, 17, 5] = np.nan
+    v[0, 40, 7], v[0, 41, 8] = np.inf, -np.inf
+    k[1, n - 10, 3] = np.inf                     # of the last tokens: seen by the last ten rows only
+
+    def run(q, k, v):
+        cache = llama.StandardKVCache(nkvh, hd, ctx)
+        cache.append(k, v, n)
+        out = np.zeros(seq * nqh * hd, np.float32)
+        llama.gqa_attention(q, cache, cache, nqh, nkvh, seq, hd, hd ** -0.5, llama.AttentionMask.causal(n - seq), None, out, ctx)
+        return out.reshape(seq, nqh, hd)
+    got = run(q, k, v)
+    clean = run(*(np.where(np.isfinite(x), x, 0.0).astype(np.float32) for x in (q, k, v)))
+    assert np.isnan(got[17, 3]).all()
+    got[17, 3] = clean[17, 3]
+    assert (got[:17, :4, 7] == np.inf).all() and (got[18:, :4, 7] == np.inf).all() and (got[18:, :4, 8] == -np.inf).all()
+    got[:, :4, 7:9] = clean[:, :4, 7:9]
+    # a score is +-inf by the sign of the query's element: the row is NaN, or does not see the key
+    sees = q[4:, seq - 10:, 3].T > 0
+    assert np.isnan(got[seq - 10:, 4:][sees]).all() and np.isfinite(got[seq - 10:, 4:][~sees]).all()
+    same = np.ones(got.shape, bool)
+    same[seq - 10:, 4:] = False
+    same[(n - 10 - (n - seq)) // 32 * 32:, 4:] = False
+    np.testing.assert_allclose(got[same], clean[same], rtol=1e-4, atol=1e-5)
