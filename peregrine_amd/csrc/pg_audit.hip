@@ -44,12 +44,11 @@ PG_API pg_status pg_audit_gemv_w8a8_m1(size_t k, size_t n, int nch, int rpw, int
     return PG_OK;
 }
 
-// 2 .. 64 rows in one launch over int8 weights (gemm_w8a8_skinny_kernel<MB, NB, NW, NST>): the weight plane
+// Up to 512 rows, in groups of 16 MB, in one launch over int8 weights (gemm_w8a8_skinny_kernel<MB, NB, NW, NST>): the weight plane
 // [n_pad][k_pad] and the quantised activation rows [m_pad][k_pad].
 PG_API pg_status pg_audit_gemm_w8a8_skinny(size_t m, size_t k, size_t n, int mb, int nb_tiles, int nw, size_t *w_end, size_t *w_bytes,
                                            size_t *a_end, size_t *a_bytes) {
     PG_CHECK_ARG(m > 0 && k > 0 && n > 0 && mb > 0 && nb_tiles > 0 && nw > 0, "pg_audit_gemm_w8a8_skinny: bad arguments");
-    PG_CHECK_ARG((size_t)16 * mb >= m, "pg_audit_gemm_w8a8_skinny: %d activation tiles for %zu rows", mb, m);
     const size_t k_pad = pg_round_up(k, PG_KPAD), n_pad = pg_round_up(n, PG_NPAD), m_pad = pg_round_up(m, PG_MPAD);
     span_check w, a;
     const int wgs = (int)((n + 16 * nb_tiles - 1) / (16 * nb_tiles));
@@ -66,7 +65,8 @@ PG_API pg_status pg_audit_gemm_w8a8_skinny(size_t m, size_t k, size_t n, int mb,
                     for (int j = 0; j < 2; ++j) {
                         const int r = 8 * j + (lane >> 3), ch = (lane & 7) ^ ((r >> 1) & 7);
                         for (int c = 0; c < nb_tiles; ++c) w.touch(pg_skinny_fill_offset(n0 + 16 * c + r, (int)k_pad, unit, ch), 16);
-                        for (int b = 0; b < mb; ++b) a.touch(pg_skinny_fill_offset(16 * b + r, (int)k_pad, unit, ch), 16);
+                        for (int r0 = 0; r0 < (int)m; r0 += 16 * mb)
+                            for (int b = 0; b < mb; ++b) a.touch(pg_skinny_fill_offset(pg_skinny_act_row(r0, b, r, (int)m), (int)k_pad, unit, ch), 16);
                     }
             }
         }

@@ -440,7 +440,7 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__res
     if (acc_out) acc_out[i] = acc;
 }
 
-// ---- 2 .. 64 activation rows: one pass over the weights, no K split between workgroups -------------
+// ---- 2 .. 64 activation rows, or groups of up to 64: one pass over the weights a group, no K split between workgroups ----
 // A workgroup owns 16 weight rows (output columns) and all of K: its NW wavefronts take one K run each and add
 // their 16 x 16 i32 tiles through LDS at the end, so nothing is left for a second launch.  Operands of
 // v_mfma_i32_16x16x64_i8 want lane -> (row lane % 16, 16 k at lane / 16): loaded that way from row-major memory,
@@ -455,7 +455,8 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__res
 // Every weight row is k_pad bytes from the next, so workgroups that all walked K from the start of their runs would
 // ask the same memory channels at the same time: each starts at its own unit and wraps round its run (integer
 // sums do not depend on the order).  The epilogue is the reference's (acc as f32) * a_scale[m] * w_scale[n]
-// (src/quant.rs:163).  a_i8 has at least 16 MB rows of a_stride bytes (rows >= m feed accumulators never stored).
+// (src/quant.rs:163).  a_i8 has at least 16 MB rows of a_stride bytes (rows >= m feed
+// accumulators never stored; with groups of rows, those past the last are the last one again).
 // NB: tiles of 16 weight rows per workgroup (with 2 every activation fragment meets two weight tiles, which halves what
 // the CUs pull from L2; the launcher says when).
 // Up to PG_GEMM_MAX_GROUP weights of equal K in one launch (the fused q|k|v and gate|up products of models::llama):
@@ -470,16 +471,25 @@ struct skinny_wgroup {
 
 constexpr int F32_ROWS_NST = 4;  // stages of gemm_w8a8_f32_rows_kernel's rings
 
-// TRI: the W8A32 product.  The activations are three digit planes a_plane bytes apart (weights 1, 256, 65536); tile b is
+// TRI: the W8A32 product.  The activations are three digit planes apart in memory (weights 1, 256, 65536); tile b is
 // tile b % (MB / 3) of plane b / (MB / 3), and the final pass joins the three sums in f64.
-template <int MB, int NB, int NW, int NST, bool TRI = false>
+// GROUPS: the rows in groups of 16 MB, each over every weight.
+// extra: the digit planes' distance (TRI); groups of rows, and above 32 bits the workgroups of one group (GROUPS).
+template <int MB, int NB, int NW, int NST, bool TRI = false, bool GROUPS = false>
 __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t *__restrict__ a_i8, const skinny_wgroup grp,
                                                                     int k_pad, int m, const float *__restrict__ a_scales,
-                                                                    int32_t *__restrict__ acc_out, size_t a_plane) {
+                                                                    int32_t *__restrict__ acc_out, size_t extra) {
     constexpr int MT = TRI ? MB / 3 : MB;  // tiles of activation rows
+    int wg = blockIdx.x, r0 = 0;
+    if constexpr (GROUPS) {  // (a weight tile's groups of rows: neighbours in time on one XCD)
+        const int j = blockIdx.x >> 3, row_groups = (int)(uint32_t)extra;
+        wg = j / row_groups * 8 + (blockIdx.x & 7);
+        r0 = j % row_groups * 16 * MT;
+        if (wg >= (int)(extra >> 32)) return;
+    }
     int g = 0;
 #pragma unroll
-    for (int i = 1; i < PG_GEMM_MAX_GROUP; ++i) g = (int)blockIdx.x >= grp.wg0[i] ? i : g;
+    for (int i = 1; i < PG_GEMM_MAX_GROUP; ++i) g = wg >= grp.wg0[i] ? i : g;
     const int8_t *__restrict__ w_t = grp.w[g];
     const float *__restrict__ w_scales = grp.ws[g];
     float *__restrict__ out = grp.out[g];
@@ -488,7 +498,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
     static_assert((NST - 1) * LPS < 64 && NST <= 6, "the wait counter holds 63");
     extern __shared__ __attribute__((aligned(1024))) char lds[];  // NW rings of NST units; afterwards the wavefronts' tiles
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n0 = ((int)blockIdx.x - grp.wg0[g]) * 16 * NB;
+    const int n0 = (wg - grp.wg0[g]) * 16 * NB;
     const int units = k_pad / 128, per = (units + NW - 1) / NW;
     const int u_begin = wave * per, u_end = u_begin + per < units ? u_begin + per : units;
     const int cnt = u_end - u_begin;
@@ -501,14 +511,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
 #pragma unroll
         for (int c = 0; c < NB; ++c) src[c][j] = w_t + pg_skinny_fill_offset(n0 + 16 * c + r, k_pad, 0, ch);  // (weight rows are padded to 256)
 #pragma unroll
-        for (int b = 0; b < MB; ++b) src[NB + b][j] = a_i8 + (TRI ? b / MT * a_plane : 0) + pg_skinny_fill_offset(16 * (b % MT) + r, k_pad, 0, ch);
+        for (int b = 0; b < MB; ++b) {
+            const int row = GROUPS ? pg_skinny_act_row(r0, b, r, m) : 16 * (b % MT) + r;
+            src[NB + b][j] = a_i8 + (TRI ? b / MT * extra : 0) + pg_skinny_fill_offset(row, k_pad, 0, ch);
+        }
     }
     // fragment reads: row lane % 16, chunk 4 s + lane / 16 of k-step s
     const int fr = lane & 15, fsw = (fr >> 1) & 7;
     int rd[2];
 #pragma unroll
     for (int st = 0; st < 2; ++st) rd[st] = fr * 128 + (((4 * st + (lane >> 4)) ^ fsw) * 16);
-    const int rot = cnt > 0 ? (int)((blockIdx.x * 5u) % (unsigned)cnt) : 0;
+    const int rot = cnt > 0 ? (int)((wg * 5u) % (unsigned)cnt) : 0;
     auto issue = [&](auto slot, int t) {  // t-th unit of the walk into ring slot `slot`
         const size_t kb = (size_t)pg_skinny_walk_unit(u_begin, cnt, t, rot) * 128;
         char *base = ring + decltype(slot)::value * UNIT;
@@ -581,7 +594,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
             for (int p = 0; p < 3; ++p)
 #pragma unroll
                 for (int w = 0; w < NW; ++w) sum[p] += red[((w * NB * MB + c * MB + p * MT + b) * 4 + i) * 64 + l];
-            const int row = b * 16 + 4 * (l >> 4) + i, col = n0 + 16 * c + (l & 15);
+            const int row = r0 + b * 16 + 4 * (l >> 4) + i, col = n0 + 16 * c + (l & 15);
             if (row < m && col < n) {
                 const double v = 65536.0 * (double)sum[2] + 256.0 * (double)sum[1] + (double)sum[0];
                 out[(size_t)row * n + col] = (float)(v * (double)a_scales[row] * (double)w_scales[col]);
@@ -594,7 +607,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
         int sum = 0;
 #pragma unroll
         for (int w = 0; w < NW; ++w) sum += red[((w * NB * MB + cb) * 4 + i) * 64 + l];
-        const int row = b * 16 + 4 * (l >> 4) + i, col = n0 + 16 * c + (l & 15);
+        const int row = r0 + b * 16 + 4 * (l >> 4) + i, col = n0 + 16 * c + (l & 15);
         if (row < m && col < n) {
             const size_t o = (size_t)row * n + col;
             if (out) out[o] = (float)sum * a_scales[row] * w_scales[col];
@@ -723,29 +736,29 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_f32_rows_kernel(const float
 // double the rate at which one CU can stream from L2 (about 9 GB/s per wavefront).
 // ctx->gemm_force_tile (pg_gemm_w8a8_force_tile) overrides the choice: 1 = 64x64, 2 = 256x256,
 // 3 = 128x256, 4 = 128x64, 5 = 128x128.
+size_t gemm_tiles(const pg_qtensor *const *w, int count, size_t m, size_t bm, size_t bn) {
+    size_t panels = 0;
+    for (int i = 0; i < count; ++i) panels += (w[i]->cols + bn - 1) / bn;
+    return ((m + bm - 1) / bm) * panels;
+}
+int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
+    const size_t cus = (size_t)ctx->num_cu;
+    if (ctx->gemm_force_tile) return ctx->gemm_force_tile;
+    const size_t t256 = gemm_tiles(w, count, m, 256, 256);
+    if (m <= 64) return 1;
+    // one and a half rounds of the largest tile or more -- or a single round that fills at least 70 %
+    // of the CUs: the fused q|k|v product (192 tiles on 256 CUs) runs 56 us so against 65 us as
+    // 384 half-size tiles (the CUs left idle let the busy ones clock higher)
+    if (t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus)) return 2;
+    if (gemm_tiles(w, count, m, 128, 256) >= cus) return 3;
+    // Too few 128x128 tiles for the CUs (k/v projections, N = 1024): halve the tile instead of
+    // leaving half of the chip idle (21.2 -> 16.5 us at 2048 x 4096 -> 1024).
+    return gemm_tiles(w, count, m, 128, 128) < cus ? 4 : 5;
+}
 pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                         const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc,
                         const int32_t *comb = nullptr, size_t comb_plane = 0) {
-    const size_t cus = (size_t)ctx->num_cu;
-    auto tiles = [&](size_t bm, size_t bn) {
-        size_t panels = 0;
-        for (int i = 0; i < count; ++i) panels += (w[i]->cols + bn - 1) / bn;
-        return ((m + bm - 1) / bm) * panels;
-    };
-    int pick = ctx->gemm_force_tile;
-    if (pick == 0) {
-        const size_t t256 = tiles(256, 256);
-        if (m <= 64) pick = 1;
-        // one and a half rounds of the largest tile or more -- or a single round that fills at least 70 %
-        // of the CUs: the fused q|k|v product (192 tiles on 256 CUs) runs 56 us so against 65 us as
-        // 384 half-size tiles (the CUs left idle let the busy ones clock higher)
-        else if (t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus)) pick = 2;
-        else if (tiles(128, 256) >= cus) pick = 3;
-        // Too few 128x128 tiles for the CUs (k/v projections, N = 1024): halve the tile instead of
-        // leaving half of the chip idle (21.2 -> 16.5 us at 2048 x 4096 -> 1024).
-        else if (tiles(128, 128) < cus) pick = 4;
-        else pick = 5;
-    }
+    const int pick = pick_tile(ctx, w, count, m);
     switch (pick) {
         case 1:
             if (comb) return launch_group<64, 64, 128, 2, 2, 2, 2, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
@@ -799,11 +812,64 @@ pg_status pg_launch_gemm_w8a8_few_rows(pg_ctx *ctx, const int8_t *a_i8, size_t a
                      (const int32_t *)part, (int)splits, plane, a_scales, (const float *)w->scales, (int)n, out, acc);
 }
 
-// 2 .. 64 rows in one launch (see gemm_w8a8_skinny_kernel).
-// (33 .. 64 rows, us with the quantisation launch: 4096 -> 14336 24.7 against 30.3 split over K with a finishing pass,
-// 4096 -> 4096 11.1 against 15.8, but 14336 -> 4096 27.8 against 26.2: long, narrow products keep the split.)
-bool pg_gemm_w8a8_takes_skinny(const pg_qtensor *w, size_t m) { return m >= 2 && (m <= 32 || (m <= 64 && w->cols >= w->k_pad)) &&
-           w->k_pad < (1ull << 30) && w->cols < (1ull << 30); }
+// 33 .. 512 rows in one launch of the few-row kernel: groups of 32, 48 or 64 rows, each reading every weight once more (the
+// groups of one weight tile follow each other on one XCD).  What the launch takes against the tiles of gemm_dispatch, both as
+// estimates: few rows over few columns leave most CUs without a tile, and a tile then walks all of K alone.  Fitted to 889
+// products (m 33 .. 400, K 256 .. 14336, one to three weights of 64 .. 16384 columns; every shape below and both other routes
+// timed on each): the launch 10 % mean error, the tiles 8 %, the choice 2.4 % over the best route on average
+// (past 256 rows, where the least is to be had, with a margin).  us, with the
+// quantisation, before : now: 66 x 1024 -> 4096 9.8 : 7.2, 96 x 4096 -> 1024 15.4 : 8.5, 128 x 4096 -> 4096 15.7 : 13.2, 39 x 4096 ->
+// 1024 11.8 : 8.2, 256 x 4096 -> 1024 19.5 : 9.8; the tiles stay: 256 x 1024 -> 4096 8.7 : 11.6, 256 x 4096 -> 4096 17.0 : 22.6.
+namespace {
+struct few_rows_shape { int mb, nb, nst, nw; double factor; };
+constexpr few_rows_shape FEW_ROWS_SHAPES[] = {{2, 1, 2, 2, 0.971}, {2, 1, 3, 4, 0.863}, {2, 1, 3, 8, 0.847}, {2, 2, 2, 4, 0.997}, {2, 2, 2, 8, 0.956},
+                                              {3, 1, 2, 8, 0.903}, {3, 2, 2, 4, 1.033}, {3, 2, 2, 8, 1.0},   {4, 2, 3, 4, 1.009}};
+bool choose_few_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, few_rows_shape *out) {
+    const size_t k_pad = w[0]->k_pad, units = k_pad / 128, cus = (size_t)ctx->num_cu;
+    if (m < 33 || m > 512 || ctx->gemm_force_tile) return false;
+    size_t cols = 0;
+    for (int i = 0; i < count; ++i) {
+        if (w[i]->k_pad != k_pad || w[i]->cols >= (1ull << 20)) return false;
+        cols += w[i]->cols;
+    }
+    // (a long K over one weight: split between workgroups, see pg_launch_gemm_w8a8_few_rows)
+    if (count == 1 && units >= 72 && (m <= 64 || (m <= 256 && k_pad >= 2 * cols))) return false;
+    const double mk = 1e-6 * (double)(m * k_pad);
+    double best = 1e30;
+    for (const few_rows_shape &s : FEW_ROWS_SHAPES) {
+        size_t wgs = 0;
+        for (int i = 0; i < count; ++i) wgs += (w[i]->cols + 16 * s.nb - 1) / (16 * s.nb);
+        wgs *= (m + 16 * s.mb - 1) / (16 * s.mb);
+        const size_t lds_kib = 2 * (size_t)(s.nw * s.nst * (s.nb + s.mb)), per_cu = std::min<size_t>(160 / lds_kib, 32 / s.nw);
+        const double rounds = (double)((wgs + cus * per_cu - 1) / (cus * per_cu)), run = (double)((units + s.nw - 1) / s.nw);
+        const double mb_cu = 1e-6 * (double)((wgs + cus - 1) / cus * units * (s.nb + s.mb) * 2048);  // what the fullest CU loads
+        const double us = s.factor * (4.96 + 1.24 * mk + rounds * (1.5 + 0.253 * run) + 14.0 * mb_cu);
+        if (us < best) {
+            best = us;
+            *out = s;
+        }
+    }
+    static constexpr int BM[] = {64, 256, 128, 128, 128}, BN[] = {64, 256, 256, 64, 128};
+    static constexpr double STEP[] = {0.366, 1.98, 1.26, 0.302, 0.846};  // us per 128 of K and round
+    const int t = pick_tile(ctx, w, count, m) - 1;
+    const size_t rounds = (gemm_tiles(w, count, m, BM[t], BN[t]) + cus - 1) / cus;
+    return best < (m <= 256 ? 0.95 : 0.85) * (7.8 + 1.86 * mk + STEP[t] * (double)(rounds * units));
+}
+}  // namespace
+
+// 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights side by side.
+// (33 .. 64 rows where the estimates say no, us with the quantisation launch: 4096 -> 14336 24.7 against 30.3 split over K with a
+// finishing pass, but 14336 -> 4096 27.8 against 26.2: long, narrow products keep the split.)
+bool pg_gemm_w8a8_takes_skinny(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
+    if (m < 2) return false;
+    bool narrow = false;
+    for (int i = 0; i < count; ++i) {
+        if (w[i]->k_pad != w[0]->k_pad || w[i]->k_pad >= (1ull << 30) || w[i]->cols >= (1ull << 30)) return false;
+        narrow = narrow || w[i]->cols < w[i]->k_pad;
+    }
+    few_rows_shape s;
+    return m <= 32 || choose_few_rows(ctx, w, count, m, &s) || (m <= 64 && !narrow);
+}
 
 // 2 .. 64 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights of equal K side by side.
 pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
@@ -813,9 +879,9 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
     size_t cols = 0;
     for (int i = 0; i < count; ++i) {
         if (a_stride != w[i]->k_pad) return pg_fail(PG_EINVAL, "gemm_w8a8: activation stride %zu != k_pad %zu", a_stride, w[i]->k_pad);
-        if (!pg_gemm_w8a8_takes_skinny(w[i], m)) return pg_fail(PG_EINVAL, "gemm_w8a8 (few rows in one launch): m = %zu", m);
         cols += w[i]->cols;
     }
+    if (!pg_gemm_w8a8_takes_skinny(ctx, w, count, m)) return pg_fail(PG_EINVAL, "gemm_w8a8 (few rows in one launch): m = %zu", m);
     const size_t k_pad = w[0]->k_pad;
     // Weight tiles a workgroup (NB), stages of a ring (NST) and wavefronts a workgroup (NW, its K runs).  What counts is that
     // every workgroup is resident at once and that a CU has many units requested: two or three stages in more wavefronts
@@ -825,11 +891,16 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
     // wavefronts in powers of two up to the LDS of one or two tiles, 3.6 % (m <= 16), 6.3 % (m <= 32) and 13 % (m <= 64) on those
     // over 8 us.  (us, before and now: 17 x 3412 -> 7951 12.0 / 10.6, 29 x 7580 -> 5374 19.9 / 16.7, 36 x 3853 -> 6403
     // 17.9 / 13.7, 40 x 531 -> 8375 11.7 / 8.7, 12 x 7381 -> 5018 15.0 / 13.4.)
-    const int mb = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
+    int mb = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
     const size_t units = k_pad / 128, g16 = (cols + 15) / 16, cus = (size_t)ctx->num_cu;
     struct shape { int nb, nst, nw; } sh = {1, mb == 1 ? 4 : 3, 0};
     const size_t wgs2 = (g16 + 1) / 2;  // workgroups of two weight tiles
-    if (wgs2 > 2 * cus) {
+    few_rows_shape grouped;
+    const bool rows_grouped = choose_few_rows(ctx, w, count, m, &grouped);
+    if (rows_grouped) {
+        mb = grouped.mb;
+        sh = {grouped.nb, grouped.nst, grouped.nw};
+    } else if (wgs2 > 2 * cus) {
         // More than 16384 columns (a vocabulary's): two weight tiles a workgroup, and of the rings that the LDS still holds
         // all at once (160 KiB a CU over the ring: 3, 4, 6 or 8 workgroups) the deepest; past that, rounds of the ring whose
         // rounds come out fullest.  Short runs of K keep one tile.  Drawn from 384 shapes a row class (m 12, 24, 48; K 256
@@ -876,7 +947,7 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         const int per_cu = mb == 4 ? 4 : 8;
         sh.nw = per_cu;
         while (sh.nw > 1 && (g16 * sh.nw > cus * per_cu || units / sh.nw < 4)) sh.nw >>= 1;
-    } else if (2 * units < 3 * (size_t)sh.nw) {
+    } else if (!rows_grouped && 2 * units < 3 * (size_t)sh.nw) {
         sh.nw = 1;  // (two wavefronts want three units)
     }
     const int nb_tiles = sh.nb;
@@ -891,14 +962,24 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         grp.wg0[i] = used ? wgs : INT_MAX;
         if (used) wgs += (int)((w[i]->cols + 16 * nb_tiles - 1) / (16 * nb_tiles));
     }
-    const dim3 grid((unsigned)wgs);
-#define PG_SKINNY(MBB, NBB, NSTT, NWW)                                                                                        \
+#define PG_SKINNY(MBB, NBB, NSTT, NWW, ...)                                                                                   \
     if (mb == MBB && sh.nb == NBB && sh.nst == NSTT && sh.nw == NWW) {                                                         \
-        auto kern = gemm_w8a8_skinny_kernel<MBB, NBB, NWW, NSTT>;                                                              \
+        auto kern = gemm_w8a8_skinny_kernel<MBB, NBB, NWW, NSTT, ##__VA_ARGS__>;                                               \
         const size_t lds = (size_t)NWW * NSTT * (NBB + MBB) * 2048;                                                            \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
-        return pg_launch(ctx, "gemm_w8a8_few_rows", kern, grid, dim3(64 * NWW), lds, a_i8, grp, (int)k_pad, (int)m, a_scales, acc, (size_t)0); \
+        return pg_launch(ctx, "gemm_w8a8_few_rows", kern, grid, dim3(64 * NWW), lds, a_i8, grp, (int)k_pad, (int)m, a_scales, acc, extra); \
     }
+    if (rows_grouped) {
+        const size_t groups = (m + 16 * mb - 1) / (16 * mb), extra = groups | (size_t)wgs << 32;
+        const dim3 grid((unsigned)((wgs + 7) / 8 * 8 * groups));
+#define PG_GROUPS(MBB, NBB, NSTT, NWW) PG_SKINNY(MBB, NBB, NSTT, NWW, false, true)
+        PG_GROUPS(2, 1, 2, 2) PG_GROUPS(2, 1, 3, 4) PG_GROUPS(2, 1, 3, 8) PG_GROUPS(2, 2, 2, 4) PG_GROUPS(2, 2, 2, 8)
+        PG_GROUPS(3, 1, 2, 8) PG_GROUPS(3, 2, 2, 4) PG_GROUPS(3, 2, 2, 8) PG_GROUPS(4, 2, 3, 4)
+#undef PG_GROUPS
+        return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8 (groups of rows in one launch): no kernel of %d tiles, %d stages, %d wavefronts", sh.nb, sh.nst, sh.nw);
+    }
+    const dim3 grid((unsigned)wgs);
+    const size_t extra = 0;
     PG_SKINNY(1, 1, 4, 1) PG_SKINNY(1, 1, 4, 2) PG_SKINNY(1, 1, 4, 4) PG_SKINNY(1, 1, 4, 8)
     PG_SKINNY(1, 1, 2, 4) PG_SKINNY(1, 2, 3, 4) PG_SKINNY(1, 2, 3, 8)
     PG_SKINNY(2, 1, 3, 1) PG_SKINNY(2, 1, 3, 2) PG_SKINNY(2, 1, 3, 4) PG_SKINNY(2, 1, 3, 8)

@@ -256,7 +256,7 @@ pg_status pg_launch_gemm_w8a8_combine(pg_ctx *ctx, const int8_t *a_i8, size_t a_
 // The W8A32 product over three digit planes (plane_bytes apart) in one launch, where it takes it.
 bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
 pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out);
-bool pg_gemm_w8a8_takes_skinny(const pg_qtensor *w, size_t m);
+bool pg_gemm_w8a8_takes_skinny(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m);
 pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                                            const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc);
 pg_status pg_launch_gemm_w8a8_skinny(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,

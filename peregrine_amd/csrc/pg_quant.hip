@@ -563,12 +563,12 @@ static pg_status matmul_quantized_on(pg_ctx *ctx, const float *a_dev, size_t m, 
     if (pg_gemv_w8a8_takes_f32_row(w, m, k, a_dev)) return pg_launch_gemv_w8a8_f32_row(ctx, a_dev, k, w, out_dev, acc_dev);
     const size_t m_pad = pg_round_up(m, PG_MPAD);
     const size_t a_bytes = m_pad * w->k_pad;
-    // 5 .. 256 rows (batched decode, short prefill chunks): split-K product with i32 partial planes
+    // 33 .. 256 rows that the few-row kernel leaves: split-K product with i32 partial planes
     // behind the scales, where the unsplit tiles would leave most CUs idle
     // (up to 64 rows always; up to 256 only for long-K, narrow-N products like a down projection --
     // measured at 128 rows: 14336 -> 4096 35 -> 25 us split, but 4096 -> 4096 12.6 -> 19 us)
     int splits = 1;
-    const bool skinny = pg_gemm_w8a8_takes_skinny(w, m);
+    const bool skinny = pg_gemm_w8a8_takes_skinny(ctx, &w, 1, m);
     if (!skinny && m > PG_GEMV_MAX_M && (m <= 64 || (m <= 256 && w->k_pad >= 2 * w->cols)))
         PG_TRY(pg_launch_gemm_w8a8_few_rows(ctx, nullptr, w->k_pad, nullptr, w, m, nullptr, nullptr, nullptr, &splits));
     const size_t sz_scales = pg_round_up(m_pad * sizeof(float), 256);
@@ -649,9 +649,10 @@ PG_API size_t pg_fixed_scratch_bytes(void) { return PG_FIXED_SCRATCH_BYTES; }
 // column-concatenated weights (fuse_qkv src/models/llama/attention.rs:51-71, fuse_gate_up
 // src/models/llama/decoder.rs:49-67) and slices the result; per-column weight scales and per-row
 // activation scales make every output column independent of its neighbours, so the separate
-// outputs here are bit for bit those of the single products.  The rows are quantised ONCE and,
-// for more than 256 rows, the narrow products share one launch (the weights' column panels side
-// by side in one tile space).
+// outputs here are bit for bit those of the single products.  The rows are quantised ONCE and the
+// narrow products share one launch (the weights side by side in the few-row kernel, or their column
+// panels in one tile space).  (Up to 256 rows each product used to quantise them again: q|k|v of a layer of
+// 2016 and the rest of its seven products 75 -> 40 us at 60 rows, 99 -> 49 at 130.)
 PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, size_t m, size_t k,
                                                const pg_qtensor *const *w, size_t count, float *const *out_dev) {
     PG_TRY(pg_use(ctx));
@@ -671,18 +672,17 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     if (one_row_group)  // one token: every weight's rows in one streaming launch that quantises the row itself
         return pg_launch_gemv_w8a8_f32_row_group(ctx, a_dev, k, w, out_dev, (int)count, nullptr);
     if (count > 1 && pg_gemm_w8a8_takes_f32_rows(ctx, w, (int)count, m)) return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, w, out_dev, (int)count, m);
-    bool skinny_group = count > 1;
-    for (size_t i = 0; i < count && skinny_group; ++i) skinny_group = pg_gemm_w8a8_takes_skinny(w[i], m) && w[i]->k_pad == w[0]->k_pad;
-    if (skinny_group) {  // 2 .. 64 rows: quantised once, then the weights side by side in one launch
-        const size_t k_pad = w[0]->k_pad, a_bytes = pg_round_up(m, PG_MPAD) * k_pad;
+    if (count > 1 && pg_gemm_w8a8_takes_skinny(ctx, w, (int)count, m)) {  // 2 .. 512 rows: quantised once, then the weights side by side in one launch
+        const size_t k_pad = w[0]->k_pad, m_pad = pg_round_up(m, PG_MPAD), a_bytes = m_pad * k_pad;
         void *ws = nullptr;
-        PG_TRY(pg_workspace(ctx, a_bytes + pg_round_up(PG_MPAD * sizeof(float), 256), &ws));
+        PG_TRY(pg_workspace(ctx, a_bytes + pg_round_up(m_pad * sizeof(float), 256), &ws));
         int8_t *a_i8 = static_cast<int8_t *>(ws);
         float *a_scales = reinterpret_cast<float *>(a_i8 + a_bytes);
         PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, k_pad, a_scales));
         return pg_launch_gemm_w8a8_skinny_group(ctx, a_i8, k_pad, a_scales, w, out_dev, (int)count, m, nullptr);  // one launch for all
     }
-    if (count == 1 || m <= 256) {  // few rows: the single products pick their own route (GEMV, split K)
+    // one weight (or one row): the single product picks its own route (GEMV, split K)
+    if (count == 1 || m <= 32) {
         for (size_t i = 0; i < count; ++i) PG_TRY(pg_matmul_quantized_dev(ctx, a_dev, m, k, w[i], out_dev[i], nullptr));
         return PG_OK;
     }

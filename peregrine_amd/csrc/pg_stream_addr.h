@@ -54,6 +54,11 @@ PG_HD int pg_skinny_walk_unit(int u_begin, int cnt, int t, int rot) {
     const int r = t + rot;
     return u_begin + (r >= cnt ? r - cnt : r);
 }
+// activation row behind row `r` of tile `t` of the group of rows from r0: past the rows, the last one again
+PG_HD int pg_skinny_act_row(int r0, int t, int r, int m) {
+    const int row = r0 + 16 * t + r;
+    return row < m ? row : m - 1;
+}
 // byte offset of a 16-byte fill in a [rows][k_pad] plane: row, K unit, chunk within the unit's 128 bytes
 PG_HD size_t pg_skinny_fill_offset(int row, int k_pad, int unit, int ch) { return (size_t)row * k_pad + (size_t)unit * 128 + (size_t)ch * 16; }
 

@@ -719,3 +719,40 @@ def test_short_f32_rows_bit_exact(ctx, orc, m, k, n):
     _ffi.check(_ffi.lib.pg_matmul_quantized_multi_dev(ctx.handle, a_dev.ptr, m, k, tab([t._gpu.value for t in qts]), 2, tab([o.ptr.value for o in outs])))
     for want, out, c in zip(wants, outs, cols):
         assert (bits(out.to_host(np.float32).reshape(m, c)) == bits(want)).all()
+
+
+@pytest.mark.parametrize("m,k,ns", [
+    (33, 100, [17]), (33, 1000, [64, 33, 33]), (47, 4096, [300]), (48, 640, [515]), (49, 640, [515]), (64, 4096, [256, 64, 64]),
+    (65, 384, [1030]), (96, 9300, [48]), (97, 2050, [700, 700]), (128, 1024, [1024]), (129, 511, [2000, 499, 499]), (144, 4096, [129]),
+    (250, 1500, [333]), (256, 4097, [200, 50, 50]), (257, 260, [40]), (385, 2048, [250]), (511, 4096, [96]), (512, 1000, [130, 130]),
+    (513, 1000, [130, 130]), (300, 300, [5000, 1250, 1250]), (40, 9216, [100]), (60, 256, [9000, 9000]),      # other routes beside them
+])
+def test_groups_of_rows_bit_exact(ctx, orc, m, k, ns):
+    """33 to 512 rows in groups of 32, 48 and 64 over one to three weights, whole and part groups, one launch and the tiles beside
+    it; the accumulators too where there is one weight."""
+    from devbuf import DevBuf
+    from peregrine_amd import quant, _ffi
+    say(f"groups of rows m={m} k={k} ns={ns}")
+    rng = np.random.default_rng(m + 10 * k + ns[0])
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, ::53] *= 20.0
+    a[m // 2] = 0.0
+    a_dev = DevBuf(ctx, host=a)
+    qa, s = orc.quantize_activations(a, m, k)
+    qts, wants, accs = [], [], []
+    for c in ns:
+        q = rng.integers(-127, 128, (k, c), dtype=np.int8)
+        scales = rng.uniform(0.5e-3, 2e-3, c).astype(np.float32)
+        qts.append(quant.QuantizedTensor(q.reshape(-1), None, scales, k, c).to_gpu(ctx))
+        acc = np.asarray(qa, np.float64).reshape(m, k) @ q.astype(np.float64)
+        accs.append(acc)
+        wants.append(acc.astype(np.float32) * np.asarray(s, np.float32)[:, None] * scales[None, :])
+    outs = [DevBuf(ctx, nbytes=4 * m * c) for c in ns]
+    tab = lambda v: (C.c_void_p * len(v))(*v)
+    _ffi.check(_ffi.lib.pg_matmul_quantized_multi_dev(ctx.handle, a_dev.ptr, m, k, tab([t._gpu.value for t in qts]), len(ns), tab([o.ptr.value for o in outs])))
+    for want, out, c in zip(wants, outs, ns):
+        assert (bits(out.to_host(np.float32).reshape(m, c)) == bits(want)).all()
+    acc_dev = DevBuf(ctx, nbytes=4 * m * ns[0])
+    _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, a_dev.ptr, m, k, qts[0]._gpu, outs[0].ptr, acc_dev.ptr))
+    assert (bits(outs[0].to_host(np.float32).reshape(m, ns[0])) == bits(wants[0])).all()
+    assert (acc_dev.to_host(np.int32).reshape(m, ns[0]) == accs[0].astype(np.int32)).all()

@@ -77,6 +77,16 @@ def test_few_rows_w8a8_fills_stay_inside_both_planes():
                 _inside(v, f"gemm_w8a8_skinny m={m} k={k} n={n} MB={mb} NB={nbt} NW={nw}")
 
 
+def test_groups_of_few_rows_w8a8_fills_stay_inside_both_planes():
+    """gemm_w8a8_skinny_kernel over groups of 32, 48 and 64 rows: a last group that runs past the padded rows."""
+    for k, n in itertools.product([256, 1000, 4096], [16, 17, 257]):
+        for (mb, nbt), nw in itertools.product([(2, 1), (2, 2), (3, 1), (3, 2), (4, 2)], (2, 4, 8)):
+            for m in (33, 48, 49, 250, 256, 257, 500, 512):
+                v = _four()
+                check(lib.pg_audit_gemm_w8a8_skinny(m, k, n, mb, nbt, nw, *[C.byref(x) for x in v]))
+                _inside(v, f"gemm_w8a8_skinny m={m} k={k} n={n} MB={mb} NB={nbt} NW={nw}")
+
+
 def test_block_gemv_loads_stay_inside_payload_and_scale_planes():
     """gguf_gemv_kernel and the few-rows form: blocks per lane 1 .. 4 (longer rows run as K segments), 2 / 4 / 8 rows
     per wavefront, 1 / 4 / 8 / 16 wavefronts per workgroup, Q4_0 and Q8_0 planes."""
