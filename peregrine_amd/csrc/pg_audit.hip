@@ -112,7 +112,7 @@ PG_API pg_status pg_audit_gguf_gemv(size_t n_out, size_t k_in, int q8, int bpl, 
     return PG_OK;
 }
 
-// 2 .. 16 rows in one launch over a block tensor (gguf_skinny_kernel<QT, NB, MT, NW, NST>): K in units of 8 blocks
+// 2 .. 8 rows in one launch over a block tensor (gguf_skinny_kernel<QT, NB, MT, NW, NST>): K in units of 8 blocks
 // (k_in % 256 == 0), a workgroup of nw wavefronts per `tiles` tiles of 16 weight rows.
 PG_API pg_status pg_audit_gguf_skinny(size_t n_out, size_t k_in, int q8, int nw, int tiles, size_t *qs_end, size_t *qs_bytes,
                                       size_t *d_end, size_t *d_bytes) {

@@ -1051,11 +1051,11 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
         pg_gemv_batch batch = {(int)m, nullptr, nullptr, nullptr, 1};
         return pg_launch_gguf_gemv(ctx, w->ggml_type, w->n_out, w->k_in, w->qs, w->d, batch, xd, y_dev, nullptr, w->m);
     }
-    if (pg_gguf_skinny_takes(ctx, w->ggml_type, m, w->n_out, w->k_in)) {  // up to 16 rows: digits, then one launch
+    if (pg_gguf_one_launch_takes(ctx, w->ggml_type, m, w->n_out, w->k_in)) {  // few rows, small products: digits, then one launch
         PG_TRY(pg_workspace(ctx, pg_mmdigits_bytes(m, w->k_in), &ws));
         const pg_mmdigits md = pg_mmdigits_carve(ws, m, w->k_in);
         PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, m, w->k_in, w->ggml_type, md));
-        return pg_launch_gguf_skinny_group(ctx, w->ggml_type, w->k_in, &w, &y_dev, 1, m, md);
+        return pg_launch_gguf_one_launch(ctx, w->ggml_type, w->k_in, &w, &y_dev, 1, m, md);
     }
     if (pg_gguf_hmm_takes(ctx, w->ggml_type, m, w->n_out, w->k_in, &hks))  // many rows of Q4_0 / Q8_0: the f16 matrix cores
         return pg_gguf_hmm_rows(ctx, x_dev, m, &w, &y_dev, 1, hks);
@@ -1116,7 +1116,7 @@ pg_status pg_gguf_matmul_rows_multi(pg_ctx *ctx, const float *x_dev, size_t m, c
         }
         return PG_OK;
     }
-    {   // many rows, one block type: one launch on the f16 matrix cores
+    {   // one block type: one launch on the f16 matrix cores (many rows) or one after the digits (few)
         bool one_type = count <= PG_HMM_MAX_GROUP;
         size_t n_total = 0;
         for (int i = 0; i < count; ++i) {
@@ -1125,6 +1125,12 @@ pg_status pg_gguf_matmul_rows_multi(pg_ctx *ctx, const float *x_dev, size_t m, c
         }
         int hks = 1;
         if (one_type && pg_gguf_hmm_takes(ctx, w[0]->ggml_type, m, n_total, k_in, &hks)) return pg_gguf_hmm_rows(ctx, x_dev, m, w, y_dev, count, hks);
+        if (one_type && count <= 3 && pg_gguf_one_launch_takes(ctx, w[0]->ggml_type, m, n_total, k_in)) {
+            PG_TRY(pg_workspace(ctx, pg_mmdigits_bytes(m, k_in), &ws));
+            const pg_mmdigits md = pg_mmdigits_carve(ws, m, k_in);
+            PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, m, k_in, w[0]->ggml_type, md));
+            return pg_launch_gguf_one_launch(ctx, w[0]->ggml_type, k_in, w, y_dev, count, m, md);
+        }
     }
     const size_t sz_d = pg_mmdigits_bytes(m, k_in);
     size_t sz_part = 0;

@@ -636,7 +636,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
 }
 
-// ---- up to 16 activation rows over a Q4_0 or Q8_0 tensor in one launch after the digits ------------------------
+// ---- up to 8 activation rows over a Q4_0 or Q8_0 tensor in one launch after the digits --------------------------
 // The product above splits K between workgroups where one token tile meets a wide tensor, and a third launch adds
 // the planes.  Here a workgroup owns 16 NB weight rows and all of K: its NW wavefronts take one run of K each, every
 // wavefront with an LDS ring of its own (no barrier in the loop: it reads only what it loaded itself), and their
@@ -644,34 +644,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // tiles as whole 128-byte lines per row (8 rows an instruction, 16-byte chunk p of row r at position
 // p ^ ((r >> 1) & 7)), their f16 scales, the two digit planes of the 16 token rows (256 bytes a row and plane,
 // chunk c of token t at position c ^ t) and the tokens' block scales; NST - 1 units are in flight while one is
-// consumed.  v_mfma_i32_16x16x32_i8 takes one block per instruction: lane -> (token or weight row lane % 16, 8 k at
-// lane / 16), result lane -> weight row lane % 16, tokens 4 (lane / 16) + i.  The weights are read in the row-major
-// planes every tensor has (no tile-major copy).  Each workgroup starts its walk through K at its own unit.
-// MT: token rows the ring holds (4, 8 or 16: the digits are most of a unit, and the fewer there are the more units
+// consumed.  The weights are read in the row-major planes every tensor has (no tile-major copy).  Each workgroup starts its
+// walk through K at its own unit.
+// MT: token rows the ring holds (4 or 8: the digits are most of a unit, and the fewer there are the more units
 // fit in flight); token slots from MT on read the rows of slots 0 .. MT - 1 again and are never stored.
 // QT = 8 (Q8_0): a weight row is two streams (bytes 0 .. 15 and 16 .. 31 of its blocks, as the upload splits them), 32
 // streams a tile, kept in LDS half-major (stream slot 16 half + row) so that the fragment reads of 16 rows and one
 // half stay free of bank conflicts; no nibbles to unpack.
 // Up to three tensors of equal K in one launch (q|k|v, gate|up of models::llama): tensor g owns the workgroups
 // wg0[g] .. wg0[g + 1] - 1 (unused slots hold INT_MAX).
-// Q41 (with QT = 4): Q4_1, whose value q d + m is (q - 8) d + (8 d + m): besides the Q4_0 product every block adds
-// 8 d + m times the block's plain sum of x, one FMA more per output; a unit holds the blocks' f16 m and the tokens' block sums too.
-// Q4_1's offsets and block sums are arguments of its kernels alone: in everybody's they cost the other formats 0.1 to 0.5 us
-// a launch (two rows of a Q8_0 block's gate|up 7.6 -> 8.1 us).
-template <bool Q41> struct skinny_args : pg_skinny_group {
-    void set(const pg_gguf_tensor *const *, int, const pg_mmdigits &) {}
-};
-template <> struct skinny_args<true> : pg_skinny_group {
-    const uint16_t *mo[3];
-    const float *xsum;
-    void set(const pg_gguf_tensor *const *w, int count, const pg_mmdigits &md) {
-        for (int i = 0; i < 3; ++i) mo[i] = i < count ? w[i]->m : nullptr;
-        xsum = md.xsum;
-    }
-};
-
-template <int QT, int NB, int MT, int NW, int NST, bool Q41 = false>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <= 8 ? 4 : 2))) void gguf_skinny_kernel(const skinny_args<Q41> grp, int nb, int nbp, int m,
+template <int QT, int NB, int MT, int NW, int NST>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_skinny_kernel(const pg_skinny_group grp, int nb, int nbp, int m,
                                                                     const int8_t *__restrict__ digits, const float *__restrict__ xs) {
     int tg = 0;
 #pragma unroll
@@ -682,10 +665,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     const float *__restrict__ res = grp.res[tg];
     const int n_out = grp.n[tg];
     constexpr int WF = QT == 8 ? 4 : 2, W_T = WF * 1024, D_T = 256, DIG = MT * 512, XS_B = 512, GQ = MT / 2;  // WF, GQ: weight, digit fills per unit
-    constexpr int OFF_DS = NB * W_T, OFF_DG = OFF_DS + NB * D_T, OFF_X = OFF_DG + DIG, OFF_MS = OFF_X + XS_B;
-    constexpr int OFF_XSUM = OFF_MS + (Q41 ? NB * D_T : 0), UNIT = OFF_XSUM + (Q41 ? XS_B : 0);
-    constexpr int LPS = WF * NB + 1 + GQ + 1 + (Q41 ? 2 : 0);  // fills per unit
-    static_assert(!Q41 || QT == 4, "Q4_1 is the Q4_0 product and its offsets");
+    constexpr int OFF_DS = NB * W_T, OFF_DG = OFF_DS + NB * D_T, OFF_X = OFF_DG + DIG, UNIT = OFF_X + XS_B;
+    constexpr int LPS = WF * NB + 1 + GQ + 1;  // fills per unit
+    static_assert(MT == 4 || MT == 8, "tokens in quads");
     static_assert((NST - 1) * LPS < 64 && NST <= 6 && NB <= 2, "the wait counter holds 63");
     extern __shared__ __attribute__((aligned(1024))) char lds[];  // NW rings of NST units; afterwards the wavefronts' tiles
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -710,8 +692,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     const int ntile = (n_out + 7) / 8;
     const int dt = pg_gskinny_scale_tile(n0, lane, ntile);
     const char *d_src = reinterpret_cast<const char *>(dsc) + pg_gskinny_scale_offset(dt, nb, 0, lane);
-    const char *ms_src = nullptr;  // Q4_1: the blocks' offsets
-    if constexpr (Q41) ms_src = reinterpret_cast<const char *>(grp.mo[tg]) + pg_gskinny_scale_offset(dt, nb, 0, lane);
     // digits: instruction q covers runs 4 q .. 4 q + 3, run = 2 token + plane; lane -> run 4 q + lane / 16, position lane % 16
     const int8_t *g_src[GQ];
 #pragma unroll
@@ -722,8 +702,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
     }
     // token scales: lanes 0 .. 2 MT - 1: token lane / 2, blocks 4 (lane % 2) .. + 3 of the unit
     const float *x_src = xs + (size_t)((lane >> 1) < m ? (lane >> 1) : 0) * nbp + 4 * (lane & 1);
-    const float *sum_src = nullptr;
-    if constexpr (Q41) sum_src = grp.xsum + (x_src - xs);
 
     const int rot = cnt > 0 ? (int)((blockIdx.x * 5u) % (unsigned)cnt) : 0;
     auto issue = [&](auto slot, int t) {
@@ -739,37 +717,28 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
         for (int q = 0; q < GQ; ++q)
             __builtin_amdgcn_global_load_lds((gptr_t)(g_src[q] + unit * 256), (lptr_t)(base + OFF_DG + q * 1024), 16, 0, 0);
         if (lane < 2 * MT) __builtin_amdgcn_global_load_lds((gptr_t)(x_src + unit * 8), (lptr_t)(base + OFF_X), 16, 0, 0);
-        if constexpr (Q41) {
-            if (lane < 16 * NB) __builtin_amdgcn_global_load_lds((gptr_t)(ms_src + unit * 128), (lptr_t)(base + OFF_MS), 16, 0, 0);
-            if (lane < 2 * MT) __builtin_amdgcn_global_load_lds((gptr_t)(sum_src + unit * 8), (lptr_t)(base + OFF_XSUM), 16, 0, 0);
-        }
     };
 
     // fragment reads of this lane
-    const int fr = lane & 15, g4 = lane >> 4, ft = fr & (MT - 1);
-    const int w_rd = ((QT == 8 ? 16 * (g4 >> 1) : 0) + fr) * 128 + 8 * (g4 & 1), w_sw = (fr >> 1) & 7;  // + ((j ^ w_sw) * 16): bytes 8 (g4 & 1) .. of block j
-    const int dg_rd = OFF_DG + ft * 512 + 8 * (g4 & 1);                     // + plane * 256 + (((2 j + (g4 >> 1)) ^ ft) * 16)
+    const int fr = lane & 15, g4 = lane >> 4;
+    const int w_sw = (fr >> 1) & 7;
     const int ds_rd = OFF_DS + (fr >> 3) * 128 + (fr & 7) * 2;              // + tile c * 256 + j * 16: this lane's weight row
-    const int x_rd = OFF_X + ((4 * g4) & (MT - 1)) * 32;                    // tokens 4 g4 .. + 3, 8 floats each
-    const int left = 4 - 4 * (g4 >> 1);                                     // low nibbles for the even elements' half
 
-    // Up to 8 token rows (QUAD): v_mfma_i32_4x4x4_i8 instead, sixteen independent 4 x 4 x 4 products an instruction.
+    // v_mfma_i32_4x4x4_i8: sixteen independent 4 x 4 x 4 products an instruction.
     // Product b of a lane quad takes weight rows 4 (b % 4) .. + 3 against four tokens for FOUR DIFFERENT blocks of K
     // (block lane / 16 of a group of four): lane -> weight row lane % 16 of block lane / 16, its eight operand
     // dwords the block's 32 k; the token operand comes from lane % 4's token (one more set of instructions for
     // tokens 4 .. 7).  The result registers are the four tokens of the lane's own row and block, so nothing of the
-    // 16 x 16 tile is padding: per block and 16 rows a quarter of the instructions of the form above, which spends
-    // them on 16 token slots whatever the count.  A lane sums blocks lane / 16, + 4, ...; the four partial sums of a
+    // 16 x 16 tile is padding.  A lane sums blocks lane / 16, + 4, ...; the four partial sums of a
     // row meet in the final pass through LDS.
-    constexpr bool QUAD = MT <= 8;
-    constexpr int NQ = QUAD ? MT / 4 : 1, NS = NB * NQ;  // accumulator sets: weight tiles x token quads
+    constexpr int NQ = MT / 4, NS = NB * NQ;  // accumulator sets: weight tiles x token quads
     float acc[NS][4];
 #pragma unroll
     for (int c = 0; c < NS; ++c)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[c][i] = 0.0f;
 
-    auto consume_quad = [&](auto slot) {
+    auto consume = [&](auto slot) {
         const char *base = ring + decltype(slot)::value * UNIT;
         const int tq = lane & 3;  // the token (of each set) whose digits this lane hands to its quad
 #pragma unroll
@@ -777,7 +746,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
             const int blk = 4 * J + g4;
             // the lane's rows (one a tile) and block: 32 weight bytes each as eight dwords in the order of the digit halves
             int wk[NB][8];
-            float dv[NB], cv[NB];
+            float dv[NB];
 #pragma unroll
             for (int c = 0; c < NB; ++c) {
                 const char *wt = base + c * W_T;
@@ -798,10 +767,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
                     }
                 }
                 dv[c] = half_bits_to_float(*reinterpret_cast<const unsigned short *>(base + ds_rd + c * D_T + blk * 16));
-                if constexpr (Q41) {  // (the sum is divided by 16 at the end)
-                    const float mv = half_bits_to_float(*reinterpret_cast<const unsigned short *>(base + ds_rd + (OFF_MS - OFF_DS) + c * D_T + blk * 16));
-                    cv[c] = fmaf(128.0f, dv[c], 16.0f * mv);
-                }
             }
 #pragma unroll
             for (int s2 = 0; s2 < NQ; ++s2) {
@@ -814,11 +779,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
                 int sx[4];  // the scales of tokens 4 s2 .. + 3 for this lane's block (read as integers: see gguf_mm_kernel)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) sx[i] = *reinterpret_cast<const int *>(base + OFF_X + (4 * s2 + i) * 32 + blk * 4);
-                int sm[4] = {0, 0, 0, 0};  // and their block sums
-                if constexpr (Q41) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) sm[i] = *reinterpret_cast<const int *>(base + OFF_XSUM + (4 * s2 + i) * 32 + blk * 4);
-                }
 #pragma unroll
                 for (int c = 0; c < NB; ++c) {
                     v4i ihi = {0, 0, 0, 0}, ilo = {0, 0, 0, 0};
@@ -836,113 +796,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
                     for (int i = 0; i < 4; ++i) {
                         const float fx = (float)(ihi[i] * 256 + ilo[i]) * __int_as_float(sx[i]);
                         acc[c * NQ + s2][i] = fmaf(dv[c], fx, acc[c * NQ + s2][i]);
-                        if constexpr (Q41) acc[c * NQ + s2][i] = fmaf(cv[c], __int_as_float(sm[i]), acc[c * NQ + s2][i]);
                     }
                 }
-            }
-        }
-    };
-
-    auto consume = [&](auto slot) {
-        if constexpr (QUAD) {
-            consume_quad(slot);
-            return;
-        }
-        const char *base = ring + decltype(slot)::value * UNIT;
-        // the scales of this lane's four tokens for the unit's eight blocks (read as integers: see gguf_mm_kernel)
-        int sx[4][8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const v4i t = *reinterpret_cast<const v4i *>(base + x_rd + i * 32 + h * 16);
-                const int t0 = t[0], t1 = t[1], t2 = t[2], t3 = t[3];
-                sx[i][4 * h] = t0; sx[i][4 * h + 1] = t1; sx[i][4 * h + 2] = t2; sx[i][4 * h + 3] = t3;
-            }
-        // Software pipeline over the unit's 8 blocks: while block j is scaled and accumulated on the vector ALU,
-        // the MFMAs of block j + 1 run and the LDS reads of block j + 2 return (one wavefront a SIMD: nothing else
-        // would fill those waits).
-        int sm[Q41 ? 4 : 1][8];  // and their block sums
-        if constexpr (Q41) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const v4i t = *reinterpret_cast<const v4i *>(base + (OFF_XSUM - OFF_X) + x_rd + i * 32 + h * 16);
-                    const int t0 = t[0], t1 = t[1], t2 = t[2], t3 = t[3];
-                    sm[i][4 * h] = t0; sm[i][4 * h + 1] = t1; sm[i][4 * h + 2] = t2; sm[i][4 * h + 3] = t3;
-                }
-        }
-        long dh[2], dl[2];
-        v2i wraw[2][NB];
-        unsigned db[2][NB], mb[2][Q41 ? NB : 1];
-        v4i ihi[2][NB], ilo[2][NB];
-        auto read = [&](int buf, int j) {
-            const int dpos = (((2 * j + (g4 >> 1)) ^ ft) * 16);
-            dh[buf] = *reinterpret_cast<const long *>(base + dg_rd + dpos);
-            dl[buf] = *reinterpret_cast<const long *>(base + dg_rd + 256 + dpos);
-#pragma unroll
-            for (int c = 0; c < NB; ++c) wraw[buf][c] = *reinterpret_cast<const v2i *>(base + c * W_T + w_rd + ((j ^ w_sw) * 16));
-        };
-        auto read_d = [&](int buf, int j) {  // the blocks' weight scales of this lane's rows
-#pragma unroll
-            for (int c = 0; c < NB; ++c) db[buf][c] = *reinterpret_cast<const unsigned short *>(base + ds_rd + c * D_T + j * 16);
-            if constexpr (Q41) {
-#pragma unroll
-                for (int c = 0; c < NB; ++c) mb[buf][c] = *reinterpret_cast<const unsigned short *>(base + ds_rd + (OFF_MS - OFF_DS) + c * D_T + j * 16);
-            }
-        };
-        auto mfmas = [&](int buf, int c) {
-            const v4i zero = {0, 0, 0, 0};
-            {
-                v2i wq = wraw[buf][c];
-                if constexpr (QT == 4) {
-                    wq[0] = nibbles_to_i8x16(wq[0], left);
-                    wq[1] = nibbles_to_i8x16(wq[1], left);
-                }
-                const long wl = __builtin_bit_cast(long, wq);
-                ihi[buf][c] = __builtin_amdgcn_mfma_i32_16x16x32_i8(dh[buf], wl, zero, 0, 0, 0);  // rows = tokens, columns = weight rows
-                ilo[buf][c] = __builtin_amdgcn_mfma_i32_16x16x32_i8(dl[buf], wl, zero, 0, 0, 0);
-            }
-        };
-        auto scale = [&](int buf, int j, int c) {
-            {
-                const float dv = half_bits_to_float(db[buf][c]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float fx = (float)(ihi[buf][c][i] * 256 + ilo[buf][c][i]) * __int_as_float(sx[i][j]);
-                    acc[c][i] = fmaf(dv, fx, acc[c][i]);
-                }
-                if constexpr (Q41) {  // (the sum is divided by 16 at the end)
-                    const float cv = fmaf(128.0f, dv, 16.0f * half_bits_to_float(mb[buf][c]));
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[c][i] = fmaf(cv, __int_as_float(sm[i][j]), acc[c][i]);
-                }
-            }
-        };
-        read(0, 0);
-        read_d(0, 0);
-        read(1, 1);
-#pragma unroll
-        for (int c = 0; c < NB; ++c) mfmas(0, c);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            // tile by tile: the two MFMAs of block j + 1 are issued, then block j of the same tile is scaled while
-            // they run (instructions issue in order: MFMAs back to back would hold the vector work behind them)
-            // (the LDS reads of block j + 2 go first and have the whole step to return; their buffers held block j,
-            // whose MFMAs were issued a step ago)
-            if (j + 1 < 8) read_d((j + 1) & 1, j + 1);
-            if (j + 2 < 8) read(j & 1, j + 2);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int c = 0; c < NB; ++c) {
-                if (j + 1 < 8) {
-                    mfmas((j + 1) & 1, c);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                scale(j & 1, j, c);
-                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
@@ -974,31 +829,238 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, MT <
 #pragma unroll
         for (int i = 0; i < 4; ++i) red[((wave * NS + c) * 4 + i) * 64 + lane] = acc[c][i];
     __syncthreads();
-    if constexpr (QUAD) {
-        for (int e = threadIdx.x; e < NS * 4 * 16; e += 64 * NW) {
-            const int r = e & 15, i = (e >> 4) & 3, c = e >> 6;  // c = tile * NQ + token quad
-            float sum = 0.0f;
+    for (int e = threadIdx.x; e < NS * 4 * 16; e += 64 * NW) {
+        const int r = e & 15, i = (e >> 4) & 3, c = e >> 6;  // c = tile * NQ + token quad
+        float sum = 0.0f;
 #pragma unroll
-            for (int w = 0; w < NW; ++w)  // ascending runs of K, within a run the four block classes in order
+        for (int w = 0; w < NW; ++w)  // ascending runs of K, within a run the four block classes in order
 #pragma unroll
-                for (int q = 0; q < 4; ++q) sum += red[((w * NS + c) * 4 + i) * 64 + 16 * q + r];
-            const int tok = 4 * (c % NQ) + i, row = n0 + 16 * (c / NQ) + r;
-            if (tok < m && row < n_out) {
-                const float v = QT == 4 ? sum * 0.0625f : sum;  // (Q4_0: the weight operand was 16 * (q - 8))
-                y[(size_t)tok * n_out + row] = res ? res[(size_t)tok * n_out + row] + v : v;
-            }
-        }
-        return;
-    }
-    for (int e = threadIdx.x; e < NB * 4 * 64; e += 64 * NW) {
-        const int l = e & 63, i = (e >> 6) & 3, c = e >> 8;
-        float sum = red[(c * 4 + i) * 64 + l];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) sum += red[((w * NB + c) * 4 + i) * 64 + l];  // ascending runs of K
-        const int tok = 4 * (l >> 4) + i, row = n0 + 16 * c + (l & 15);
+            for (int q = 0; q < 4; ++q) sum += red[((w * NS + c) * 4 + i) * 64 + 16 * q + r];
+        const int tok = 4 * (c % NQ) + i, row = n0 + 16 * (c / NQ) + r;
         if (tok < m && row < n_out) {
             const float v = QT == 4 ? sum * 0.0625f : sum;  // (Q4_0: the weight operand was 16 * (q - 8))
             y[(size_t)tok * n_out + row] = res ? res[(size_t)tok * n_out + row] + v : v;
+        }
+    }
+}
+
+// ---- 2 and more activation rows over a small product in one launch after the digits, any K -------------------------
+// gguf_mm_kernel's 32 x 32 tile with gguf_skinny_kernel's split of K: a workgroup owns 32 weight rows x MT tokens and all of
+// K, its NW wavefronts take one run of K each with an LDS ring of their own (no barrier in the loop), and their f32 tiles
+// are added through LDS in a fixed order.  Nothing is left for a third launch, and a small tensor has as many wavefronts as its
+// blocks can feed.  A unit of the ring is four blocks: the tile-major copy's run of the 32 rows (2 or 4 KiB), their f16 scales,
+// the digit planes and block scales of the tokens.  Blocks past the end of K are not added.
+// More than MT tokens: groups of MT, a weight tile's groups behind each other on one XCD.
+// MT = 8, 16: tokens on the accumulator registers (half of MT of them), weight rows on the lanes; MT = 32 the other way
+// round, as gguf_mm_kernel.
+// Q41 (with QT = 4): Q4_1, whose value q d + m is (q - 8) d + (8 d + m): besides the Q4_0 product every block adds 8 d + m times
+// the block's plain sum of x, one FMA more per output; a unit holds the blocks' f16 m and the tokens' block sums too.
+// Q4_1's offsets and block sums are arguments of its kernels alone: in everybody's they cost the other formats 0.1 to 0.5 us
+// a launch.
+template <bool Q41> struct ktile_args : pg_skinny_group {
+    void set(const pg_gguf_tensor *const *, int, const pg_mmdigits &) {}
+};
+template <> struct ktile_args<true> : pg_skinny_group {
+    const uint16_t *mo[3];
+    const float *xsum;
+    void set(const pg_gguf_tensor *const *w, int count, const pg_mmdigits &md) {
+        for (int i = 0; i < 3; ++i) mo[i] = i < count ? w[i]->m : nullptr;
+        xsum = md.xsum;
+    }
+};
+
+template <int QT, int MT, bool Q41> struct KTCfg {
+    static constexpr int W_T = QT == 8 ? 4096 : 2048, OFF_D = W_T, OFF_M = OFF_D + 256, OFF_DG = OFF_M + (Q41 ? 256 : 0);
+    static constexpr int OFF_X = OFF_DG + MT * 256, OFF_S = OFF_X + MT * 16, UNIT = OFF_S + (Q41 ? MT * 16 : 0);
+};
+template <int QT, int MT, int NW, bool Q41>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_ktile_kernel(const ktile_args<Q41> grp, int nb, int nbp, int m,
+                                                                const int8_t *__restrict__ digits, const float *__restrict__ xs, int groups, int wgs) {
+    using C = KTCfg<QT, MT, Q41>;
+    static_assert(!Q41 || QT == 4, "Q4_1 is the Q4_0 product and its offsets");
+    int wg = blockIdx.x, t0 = 0;
+    if (groups > 1) {
+        const int j = blockIdx.x >> 3;
+        wg = j / groups * 8 + (blockIdx.x & 7);
+        t0 = j % groups * MT;
+        if (wg >= wgs) return;
+    }
+    int tg = 0;
+#pragma unroll
+    for (int i = 1; i < 3; ++i) tg = wg >= grp.wg0[i] ? i : tg;
+    const int n_out = grp.n[tg];
+    float *__restrict__ y = grp.y[tg];
+    const float *__restrict__ res = grp.res[tg];
+    extern __shared__ __attribute__((aligned(1024))) char lds[];  // NW rings of two units; afterwards the wavefronts' tiles
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l31 = lane & 31, hh = lane >> 5;
+    const int n0 = (wg - grp.wg0[tg]) * 32, mt = m - t0 < MT ? m - t0 : MT;
+    const int units = (nb + 3) / 4, per = (units + NW - 1) / NW;
+    const int u_begin = wave * per, u_end = u_begin + per < units ? u_begin + per : units;
+    const int cnt = u_end - u_begin;
+    char *ring = lds + (size_t)wave * 2 * C::UNIT;
+
+    // fill duties of this lane
+    const char *w_src = reinterpret_cast<const char *>(grp.qs[tg]) + (size_t)(n0 >> 7) * pg_tiled_group_bytes(nb, QT == 8) +
+                        ((n0 >> 5) & 3) * C::W_T + lane * 16;
+    const int ngroups = (n_out + 7) / 8;
+    const int dg8 = (n0 >> 3) + (lane >> 4) < ngroups ? (n0 >> 3) + (lane >> 4) : ngroups - 1;
+    const size_t d_at = (size_t)dg8 * nb * 16 + (lane & 3) * 4;
+    const int d_jb = (lane >> 2) & 3;
+    const char *d_src = reinterpret_cast<const char *>(grp.d[tg]) + d_at;
+    const char *m_src = nullptr;
+    if constexpr (Q41) m_src = reinterpret_cast<const char *>(grp.mo[tg]) + d_at;
+    // digits: fill q covers runs 8 q .. 8 q + 7 of 128 bytes, run = 2 token + plane (tokens 8 .. 15 (mod 16) keep their planes swapped)
+    const int8_t *g_src[MT / 4];
+    int g_jb[MT / 4];
+#pragma unroll
+    for (int q = 0; q < MT / 4; ++q) {
+        const int run = 8 * q + (lane >> 3), tok = run >> 1, pl = (run & 1) ^ ((tok >> 3) & 1), ch = (lane & 7) ^ (tok & 7);
+        g_jb[q] = ch >> 1;
+        g_src[q] = digits + (size_t)(t0 + (tok < mt ? tok : 0)) * pg_mm_row_bytes(nb) + (size_t)pl * nb * 32 + (ch & 1) * 16;
+    }
+    const size_t x_at = (size_t)(t0 + (lane < mt ? lane : 0)) * nbp;
+
+    const int rot = cnt > 0 ? (int)((wg * 5u) % (unsigned)cnt) : 0;
+    auto issue = [&](auto slot, int t) {
+        const int unit = pg_skinny_walk_unit(u_begin, cnt, t, rot), b0 = 4 * unit;
+        char *base = ring + decltype(slot)::value * C::UNIT;
+        auto blk = [&](int j) { return (size_t)(b0 + j < nb ? b0 + j : nb - 1); };  // past the end: a valid block, never added
+#pragma unroll
+        for (int q = 0; q < C::W_T / 1024; ++q)
+            __builtin_amdgcn_global_load_lds((gptr_t)(w_src + (size_t)unit * (4 * C::W_T) + q * 1024), (lptr_t)(base + q * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((gptr_t)(d_src + blk(d_jb) * 16), (lptr_t)(base + C::OFF_D), 4, 0, 0);
+        if constexpr (Q41) __builtin_amdgcn_global_load_lds((gptr_t)(m_src + blk(d_jb) * 16), (lptr_t)(base + C::OFF_M), 4, 0, 0);
+#pragma unroll
+        for (int q = 0; q < MT / 4; ++q)
+            __builtin_amdgcn_global_load_lds((gptr_t)(g_src[q] + blk(g_jb[q]) * 32), (lptr_t)(base + C::OFF_DG + q * 1024), 16, 0, 0);
+        if (lane < MT) {
+            __builtin_amdgcn_global_load_lds((gptr_t)(xs + x_at + b0), (lptr_t)(base + C::OFF_X), 16, 0, 0);
+            if constexpr (Q41) __builtin_amdgcn_global_load_lds((gptr_t)(grp.xsum + x_at + b0), (lptr_t)(base + C::OFF_S), 16, 0, 0);
+        }
+    };
+
+    constexpr bool ROWS = MT == 32;      // weight rows on the registers
+    constexpr int NR = ROWS ? 16 : MT / 2;
+    float acc[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) acc[r] = 0.0f;
+    const int ws = QT == 8 ? lane : l31, w_rd = ws * 64, w_sw = (ws >> 2) & 3;
+    const int tok = l31 & (MT - 1), dig_rd = C::OFF_DG + tok * 256, dig_sw = tok & 7, dig_hi = ((tok >> 3) & 1) * 128;
+    auto read = [&](const char *base, int j, v4i (&ab)[3]) {
+        ab[0] = *reinterpret_cast<const v4i *>(base + w_rd + ((j ^ w_sw) * 16));
+        ab[1] = *reinterpret_cast<const v4i *>(base + dig_rd + dig_hi + (((2 * j + hh) ^ dig_sw) * 16));
+        ab[2] = *reinterpret_cast<const v4i *>(base + dig_rd + (128 - dig_hi) + (((2 * j + hh) ^ dig_sw) * 16));
+    };
+    auto mfmas = [&](const v4i (&ab)[3], v16i &ihi, v16i &ilo) {
+        v4i a = ab[0];
+        if constexpr (QT == 4) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) a[t] = nibbles_to_i8x16(a[t], 4 - 4 * hh);
+        }
+        v16i zero;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero[r] = 0;
+        ihi = ROWS ? __builtin_amdgcn_mfma_i32_32x32x32_i8(a, ab[1], zero, 0, 0, 0) : __builtin_amdgcn_mfma_i32_32x32x32_i8(ab[1], a, zero, 0, 0, 0);
+        ilo = ROWS ? __builtin_amdgcn_mfma_i32_32x32x32_i8(a, ab[2], zero, 0, 0, 0) : __builtin_amdgcn_mfma_i32_32x32x32_i8(ab[2], a, zero, 0, 0, 0);
+    };
+    auto quad = [&](const char *base, int off, int (&v)[4]) {  // four ints at once (read as integers: see gguf_mm_kernel)
+        const v4i t = *reinterpret_cast<const v4i *>(base + off);
+        const int a0 = t[0], a1 = t[1], a2 = t[2], a3 = t[3];
+        v[0] = a0; v[1] = a1; v[2] = a2; v[3] = a3;
+    };
+    auto consume = [&](auto slot, int t) {
+        const char *base = ring + decltype(slot)::value * C::UNIT;
+        const int left = nb - 4 * pg_skinny_walk_unit(u_begin, cnt, t, rot);
+        // the scales (and Q4_1's block sums) of the tokens for the unit's four blocks: of this lane's token, or of its NR tokens
+        int sx[ROWS ? 1 : NR][4], sm[Q41 ? (ROWS ? 1 : NR) : 1][4];
+#pragma unroll
+        for (int r = 0; r < (ROWS ? 1 : NR); ++r) {
+            const int at = (ROWS ? l31 : 8 * (r >> 2) + 4 * hh + (r & 3)) * 16;
+            quad(base, C::OFF_X + at, sx[r]);
+            if constexpr (Q41) quad(base, C::OFF_S + at, sm[r]);
+        }
+        v4i ab[2][3];
+        v16i ihi[2], ilo[2];
+        auto scale = [&](int j, const v16i &hi, const v16i &lo) {
+            if constexpr (ROWS) {
+                const float sj = __int_as_float(sx[0][j]) * (QT == 4 ? 0.0625f : 1.0f);  // (Q4_0: the weight operand was 16 * (q - 8))
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {  // rows 8 g + 4 hh + {0 .. 3}  <->  registers 4 g .. 4 g + 3
+                    const v2i dd = *reinterpret_cast<const v2i *>(base + C::OFF_D + (g * 4 + j) * 16 + hh * 8);
+                    v2i mm = {0, 0};
+                    if constexpr (Q41) mm = *reinterpret_cast<const v2i *>(base + C::OFF_M + (g * 4 + j) * 16 + hh * 8);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int r = 4 * g + q;
+                        const uint32_t bits = (uint32_t)dd[q >> 1];
+                        const float dv = half_bits_to_float((q & 1) ? bits >> 16 : bits & 0xFFFFu);
+                        const float fx = (float)(hi[r] * 256 + lo[r]) * sj;
+                        acc[r] = fmaf(dv, fx, acc[r]);
+                        if constexpr (Q41) {
+                            const uint32_t mbits = (uint32_t)mm[q >> 1];
+                            const float cv = fmaf(8.0f, dv, half_bits_to_float((q & 1) ? mbits >> 16 : mbits & 0xFFFFu));
+                            acc[r] = fmaf(cv, __int_as_float(sm[0][j]), acc[r]);
+                        }
+                    }
+                }
+            } else {
+                const int at = (l31 >> 3) * 64 + j * 16 + (l31 & 7) * 2;
+                float dv = half_bits_to_float(*reinterpret_cast<const unsigned short *>(base + C::OFF_D + at)), cv = 0.0f;
+                if constexpr (Q41) cv = fmaf(8.0f, dv, half_bits_to_float(*reinterpret_cast<const unsigned short *>(base + C::OFF_M + at)));
+                if constexpr (QT == 4) dv *= 0.0625f;
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    const float fx = (float)(hi[r] * 256 + lo[r]) * __int_as_float(sx[r][j]);
+                    acc[r] = fmaf(dv, fx, acc[r]);
+                    if constexpr (Q41) acc[r] = fmaf(cv, __int_as_float(sm[r][j]), acc[r]);
+                }
+            }
+        };
+        read(base, 0, ab[0]);
+        read(base, 1, ab[1]);
+        mfmas(ab[0], ihi[0], ilo[0]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {  // while block j is scaled the MFMAs of block j + 1 run and the reads of block j + 2 return
+            if (j + 1 < 4) mfmas(ab[(j + 1) & 1], ihi[(j + 1) & 1], ilo[(j + 1) & 1]);
+            if (j + 2 < 4) read(base, j + 2, ab[j & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (j < left) scale(j, ihi[j & 1], ilo[j & 1]);  // (the same for the whole wavefront)
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (cnt > 0) {
+        issue(std::integral_constant<int, 0>{}, 0);
+        auto step = [&](auto slot, int t) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (t + 1 < cnt) issue(std::integral_constant<int, 1 - decltype(slot)::value>{}, t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            consume(slot, t);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int t = 0; t < cnt; t += 2) {
+            step(std::integral_constant<int, 0>{}, t);
+            if (t + 1 < cnt) step(std::integral_constant<int, 1>{}, t + 1);
+        }
+    }
+    __syncthreads();  // the rings are done with: their space takes the wavefronts' tiles
+    float *red = reinterpret_cast<float *>(lds);  // [NW][NR][64], a lane's registers 65 apart
+#pragma unroll
+    for (int r = 0; r < NR; ++r) red[(wave * NR + r) * 65 + lane] = acc[r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < NR * 64; e += 64 * NW) {
+        // ROWS: consecutive threads take consecutive weight rows of one token; otherwise a register's 64 lanes
+        const int r = ROWS ? (e & 3) + 4 * ((e >> 3) & 3) : e >> 6;
+        const int l = ROWS ? (e >> 5) + 32 * ((e >> 2) & 1) : e & 63;
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += red[(w * NR + r) * 65 + l];
+        const int at = 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
+        const int token = ROWS ? l & 31 : at, row = n0 + (ROWS ? at : l & 31);
+        if (token < mt && row < n_out) {
+            const size_t o = (size_t)(t0 + token) * n_out + row;
+            y[o] = res ? res[o] + sum : sum;
         }
     }
 }
@@ -1104,102 +1166,146 @@ int pg_gguf_mm_splitk(const pg_ctx *ctx, size_t n_out, size_t k_in, size_t group
     return (int)ks_real;
 }
 
-// Up to 16 rows over a Q4_0 or Q8_0 tensor whose K is a multiple of 256: the one-launch product (see the kernel).
-// With 9 .. 16 token rows (the 16 x 16 x 32 form) the kernel is bound by instruction issue (about 500 instructions per
-// 8 blocks and weight tile, most of them the per-block scaling of 16 token slots), seven wavefronts fit a CU at two
-// units a ring, and it beats digits + product over K chunks + their sum only where those are short of workgroups
-// (14336 -> 4096: 18.2 against 24.3 us; 4096 -> 4096: 8.8 against 13.3; but 4096 -> 14336: 21.5 against 20.0 - 22.0).
-// Up to 8 token rows (the 4 x 4 x 4 form) a quarter of those instructions remain and the kernel is bound by how many
-// bytes its rings keep in flight: 4 x 4096 -> 14336 takes 9.0 us (with its arithmetic switched off 8.6 - 9.1; in the
-// 16 x 16 x 32 form it took 11.9).
-bool pg_gguf_skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out, size_t k_in) {
-    // (Q4_1 below eight rows stays with the streaming kernel and its finer fixed point)
-    return (ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0 || (ggml_type == PG_GGML_Q4_1 && m >= 8)) && m >= 2 && (m <= 8 || (m <= 16 && n_out / 32 < (size_t)ctx->num_cu)) &&
+// Up to 8 rows over a Q4_0 or Q8_0 tensor whose K is a multiple of 256: gguf_skinny_kernel, bound by how many bytes its rings keep
+// in flight (4 x 4096 -> 14336 takes 9.0 us; with its arithmetic switched off 8.6 - 9.1).  From five rows on it is the better one
+// only where a long K meets few columns (us, this one : gguf_ktile_kernel: 7 x 11776 -> 1804 12.7 : 14.8, 8 x 8704 -> 406 10.7 :
+// 12.3; but 6 x 6144 -> 4297 14.1 : 10.5, 8 x 1536 -> 12190 11.5 : 8.1, 7 x 3584 -> 870 10.1 : 8.5).
+static bool skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out, size_t k_in) {
+    return (ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0) && m >= 2 && (m <= 4 || (m <= 8 && k_in >= 6400 && n_out < 16 * (size_t)ctx->num_cu)) &&
            k_in % 256 == 0 && k_in >= 1024 && n_out >= 1 && n_out < (1u << 30) && k_in < (1u << 24);
 }
 
-pg_status pg_launch_gguf_skinny_group(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_gguf_tensor *const *w, float *const *y, int count,
-                                      size_t m, const pg_mmdigits &md, const float *residual) {
+// Products small enough that digits, K chunks and their sum are three latencies: gguf_ktile_kernel.  Against that route (m 2 .. 400,
+// K 256 .. 14336, N 256 .. 14336, 1450 products) it takes 0.6 to 0.8 of the time up to half a G multiply-adds, is level at 1.5 (more than
+// 64 rows: 1, Q4_1 2) and slower beyond, where a tile of 128 weight rows shares a token's digits; so it is with a long K, or a short one
+// under many columns, over more than two row tiles (71 x 4896 -> 2614 24 : 31, 67 x 512 -> 13720 11.5 : 17).  Q4_1 up to 64 rows: the offsets' launch goes too (0.6 to 0.9 up to 5 G).  us, before : now:
+// 35 x 1088 -> 465 (Q8_0) 12.4 : 7.6, 12 x 4096 -> 4096 (Q4_1) 9.9 : 8.0, 11 x 1056 -> 2116 (Q8_0) 11.5 : 7.6, 32 x 4096 -> 1024
+// (Q4_0) 13.7 : 9.2, 64 x 4096 -> 4096 (Q4_1) 28.5 : 22.
+// What runs on the f16 matrix cores stays there, and Q4_1 below eight rows with the streaming kernel: both have finer digits.
+static bool ktile_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out, size_t k_in, bool planes) {
+    const bool q41 = ggml_type == PG_GGML_Q4_1;
+    if (!(ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0 || q41) || m < (q41 ? 8 : 2) || k_in % 32 != 0 || k_in > 32768 || n_out < 1 || n_out >= (1u << 24))
+        return false;
+    const double g = 1e-9 * (double)m * (double)n_out * (double)k_in * (planes ? 1.5 : 1.0);
+    if (k_in < 512 && n_out > 8192) return false;                                        // (all columns, hardly any K to split)
+    if (m > 64 && (k_in >= (q41 ? 8192 : 6144) || (k_in < 1024 && m * n_out > 500000))) return false;
+    if (g > (q41 ? (m <= 64 ? 5.0 : 1.8) : m <= 64 ? 1.4 : m <= 128 ? 0.9 : 0.7)) return false;
+    return m <= 16 || !pg_gguf_hmm_takes(ctx, q41 ? PG_GGML_Q4_0 : ggml_type, m, n_out, k_in, nullptr);
+}
+
+// Whether a product runs as one launch after the digits.  `planes`: the caller takes the K chunks of the other route unsummed, so that
+// there is no launch for their sum to be saved and the lines lie at two thirds (the Llama block's steps of 10 to 180 tokens over four
+// models: at 1 / 1.5 / 3 of the lines 0 to 1 % slower / best / 1 to 3 % slower; without this kernel 3 to 15 %.  us, before : now:
+// 7 tokens of 1024 47 : 41, 30 of 2048 77 : 69, 45 of 2048 / 5632 93 : 76, 20 of 4096 115 : 102, 180 of 4096 322 : 301).
+bool pg_gguf_one_launch_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out, size_t k_in, bool planes) {
+    return skinny_takes(ctx, ggml_type, m, n_out, k_in) || ktile_takes(ctx, ggml_type, m, n_out, k_in, planes);
+}
+
+static pg_status launch_skinny(pg_ctx *ctx, size_t k_in, bool q8, const pg_skinny_group &grp, int wgs, int tiles, size_t m, const pg_mmdigits &md) {
+    const int nb = (int)(k_in / 32), nbp = (int)pg_round_up(nb, 4);
+    // Wavefronts (runs of K) per workgroup: as many as keep every workgroup resident at once, up to 16 a CU (4 a SIMD).  The rings: units
+    // of 4.75 / 6.75 KiB for 4 / 8 token rows (Q8_0: 2 KiB more), two stages (three on fewer wavefronts: 10.7 - 10.9 against 9.0 us on
+    // 4 x 4096 -> 14336).
+    const size_t unit_bytes = (size_t)tiles * ((q8 ? 4096 : 2048) + 256) + (m <= 4 ? 4 : 8) * 512 + 512, units = (size_t)nb / 8;
+    auto fits = [&](int nw_) {  // LDS is handed out per workgroup: nw wavefronts' rings each
+        const size_t per_cu = std::min<size_t>((160u << 10) / ((size_t)nw_ * 2 * unit_bytes), 16 / nw_);
+        return (size_t)wgs <= (size_t)ctx->num_cu * per_cu;
+    };
+    int nw = 8;
+    while (nw > 1 && (!fits(nw) || units / nw < 4)) nw >>= 1;
+#define PG_GSK(QTT, NBB, MTT, NWW)                                                                                             \
+    if (q8 == (QTT == 8) && tiles == NBB && (m <= 4) == (MTT == 4) && nw == NWW) {                                             \
+        auto kern = gguf_skinny_kernel<QTT, NBB, MTT, NWW, 2>;                                                                 \
+        const size_t lds = (size_t)NWW * 2 * (NBB * ((QTT == 8 ? 4096 : 2048) + 256) + MTT * 512 + 512);                       \
+        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
+        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_few_rows_mm" : "gguf_q4_0_few_rows_mm", kern, dim3((unsigned)wgs), dim3(64 * NWW), lds, \
+                         grp, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs);                               \
+    }
+#define PG_GSK_NW(QTT, NBB, MTT) PG_GSK(QTT, NBB, MTT, 8) PG_GSK(QTT, NBB, MTT, 4) PG_GSK(QTT, NBB, MTT, 2) PG_GSK(QTT, NBB, MTT, 1)
+    PG_GSK_NW(8, 1, 4) PG_GSK_NW(8, 2, 4) PG_GSK_NW(8, 1, 8) PG_GSK_NW(8, 2, 8)
+    PG_GSK_NW(4, 1, 4) PG_GSK_NW(4, 2, 4) PG_GSK_NW(4, 1, 8) PG_GSK_NW(4, 2, 8)
+#undef PG_GSK_NW
+#undef PG_GSK
+    return pg_fail(PG_EUNSUPPORTED, "gguf (few rows in one launch): no kernel of %d tiles, %d wavefronts", tiles, nw);
+}
+
+// The shape of a ktile launch: of the tokens a workgroup takes (MT) and its wavefronts (NW) the pair of least estimated time.  Rounds of
+// workgroups (a CU's LDS over their rings), a wavefront's run of units, and what the fullest CU loads; Q4_1's further FMAs a unit.  Fitted
+// to 1341 products within the lines above: 1 to 2 % over the best of the shapes on average.  (Tokens in groups of 8 or 16 while
+// there are few: the digits of 32 are most of a ring and leave six wavefronts a CU.)
+struct ktile_shape { int mt, nw; double factor; };
+static constexpr ktile_shape KTILE_SHAPES[] = {{32, 2, 1.26}, {32, 3, 1.2}, {32, 6, 1.14}, {16, 4, 1.06}, {16, 8, 1.03}, {8, 4, 1.014}, {8, 8, 1.0}};
+static size_t ktile_unit(int ggml_type, int mt) {
+    return ggml_type == PG_GGML_Q8_0 ? (mt == 32 ? KTCfg<8, 32, false>::UNIT : mt == 16 ? KTCfg<8, 16, false>::UNIT : KTCfg<8, 8, false>::UNIT)
+         : ggml_type == PG_GGML_Q4_1 ? (mt == 32 ? KTCfg<4, 32, true>::UNIT : mt == 16 ? KTCfg<4, 16, true>::UNIT : KTCfg<4, 8, true>::UNIT)
+                                     : (mt == 32 ? KTCfg<4, 32, false>::UNIT : mt == 16 ? KTCfg<4, 16, false>::UNIT : KTCfg<4, 8, false>::UNIT);
+}
+static pg_status launch_ktile(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_gguf_tensor *const *w, int count, const pg_skinny_group &grp, int wgs1,
+                              size_t m, const pg_mmdigits &md) {
+    const int nb = (int)(k_in / 32), nbp = (int)pg_round_up(nb, 4);
+    const bool q8 = ggml_type == PG_GGML_Q8_0, q41 = ggml_type == PG_GGML_Q4_1;
+    const size_t units = ((size_t)nb + 3) / 4, cus = (size_t)ctx->num_cu;
+    ktile_shape sh = KTILE_SHAPES[0];
+    double best = 1e30;
+    for (const ktile_shape &s : KTILE_SHAPES) {
+        if ((s.mt == 8 && m > 32) || (s.mt == 16 && m > 64)) continue;
+        const size_t unit = ktile_unit(ggml_type, s.mt), wgs = (size_t)wgs1 * ((m + s.mt - 1) / s.mt);
+        const size_t per_cu = std::max<size_t>(1, std::min<size_t>((160u << 10) / ((size_t)s.nw * 2 * unit), (s.mt == 32 ? 8 : 16) / s.nw));
+        const double rounds = (double)((wgs + cus * per_cu - 1) / (cus * per_cu)), run = (double)((units + s.nw - 1) / s.nw);
+        const double cu_units = (double)((wgs + cus - 1) / cus * units);
+        const double us = s.factor * (4.58 + 7.06e-6 * (double)(m * k_in) + rounds * (1.51 + 0.325 * run) + cu_units * (10.1e-6 * (double)unit + (q41 ? 0.042 : 0.0)));
+        if (us < best) {
+            best = us;
+            sh = s;
+        }
+    }
+    const int groups = (int)((m + sh.mt - 1) / sh.mt);
+    const dim3 grid(groups == 1 ? (unsigned)wgs1 : (unsigned)((wgs1 + 7) / 8 * 8 * groups));
+#define PG_KT(QTT, MTT, NWW)                                                                                                   \
+    if ((QTT == 8 ? q8 : QTT == 5 ? q41 : !q8 && !q41) && sh.mt == MTT && sh.nw == NWW) {  /* (5 names Q4_1 here) */           \
+        auto kern = gguf_ktile_kernel<QTT == 8 ? 8 : 4, MTT, NWW, QTT == 5>;                                                   \
+        ktile_args<QTT == 5> args;                                                                                             \
+        static_cast<pg_skinny_group &>(args) = grp;                                                                            \
+        args.set(w, count, md);                                                                                                \
+        const size_t lds = (size_t)NWW * 2 * KTCfg<QTT == 8 ? 8 : 4, MTT, QTT == 5>::UNIT;                                     \
+        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
+        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_rows_tile" : QTT == 5 ? "gguf_q4_1_rows_tile" : "gguf_q4_0_rows_tile", kern, grid, \
+                         dim3(64 * NWW), lds, args, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs, groups, wgs1); \
+    }
+#define PG_KTS(QTT) PG_KT(QTT, 32, 2) PG_KT(QTT, 32, 3) PG_KT(QTT, 32, 6) PG_KT(QTT, 16, 4) PG_KT(QTT, 16, 8) PG_KT(QTT, 8, 4) PG_KT(QTT, 8, 8)
+    PG_KTS(8) PG_KTS(4) PG_KTS(5)
+#undef PG_KTS
+#undef PG_KT
+    return pg_fail(PG_EUNSUPPORTED, "gguf (rows in tiles, one launch): no kernel of %d tokens, %d wavefronts", sh.mt, sh.nw);
+}
+
+pg_status pg_launch_gguf_one_launch(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_gguf_tensor *const *w, float *const *y, int count,
+                                    size_t m, const pg_mmdigits &md, const float *residual) {
     if (count < 1 || count > 3) return pg_fail(PG_EINVAL, "gguf (few rows in one launch): %d tensors (1 .. 3)", count);
     size_t n_total = 0;
     for (int i = 0; i < count; ++i) {
         if (w[i]->k_in != k_in || w[i]->ggml_type != ggml_type) return pg_fail(PG_EINVAL, "gguf (few rows in one launch): the tensors differ in K or type");
         n_total += w[i]->n_out;
     }
-    if (!pg_gguf_skinny_takes(ctx, ggml_type, m, n_total, k_in)) return pg_fail(PG_EINVAL, "gguf (few rows in one launch): [%zu x %zu] x %zu", m, k_in, n_total);
-    const int nb = (int)(k_in / 32), nbp = (int)pg_round_up(nb, 4);
-    const bool q8 = ggml_type == PG_GGML_Q8_0;
-    // Wavefronts (runs of K) per workgroup: as many as keep every workgroup resident at once.  The rings: units of
-    // 4.75 / 6.75 / 10.75 KiB for 4 / 8 / 16 token rows (Q8_0: 2 KiB more), as many stages as let eight wavefronts
-    // share a CU's LDS (16 token rows: two stages and six or seven wavefronts; three stages and four were slower).
-    // Two weight tiles a workgroup (32 rows) where that still leaves a workgroup for every CU: the digits, which
+    const bool skinny = skinny_takes(ctx, ggml_type, m, n_total, k_in);
+    if (!skinny && !ktile_takes(ctx, ggml_type, m, n_total, k_in, false)) return pg_fail(PG_EINVAL, "gguf (few rows in one launch): [%zu x %zu] x %zu", m, k_in, n_total);
+    // Two 16-row weight tiles a workgroup of the skinny kernel where that still leaves a workgroup for every CU: the digits, which
     // every workgroup fetches for all of K, then cost half as much per weight byte.
-    const int tiles = (m <= 8 && n_total / 32 >= (size_t)ctx->num_cu) ? 2 : 1;
-    const bool q41 = ggml_type == PG_GGML_Q4_1;
-    const size_t unit_bytes = (size_t)tiles * ((q8 ? 4096 : 2048) + (q41 ? 512 : 256)) + (m <= 4 ? 4 : (m <= 8 ? 8 : 16)) * 512 + (q41 ? 1024 : 512);
-    const int stages = 2;  // (three stages on fewer wavefronts: 10.7 - 10.9 against 9.0 us on 4 x 4096 -> 14336)
-    const size_t lds_cu = 160u << 10;
+    const int tiles = n_total / 32 >= (size_t)ctx->num_cu ? 2 : 1, rows = skinny ? 16 * tiles : 32;
     pg_skinny_group grp;
     int wgs = 0;
     for (int i = 0; i < 3; ++i) {
         const bool used = i < count;
-        grp.qs[i] = used ? w[i]->qs : nullptr;
+        if (used && !skinny) PG_TRY(pg_gguf_ensure_tiled(ctx, w[i]));
+        grp.qs[i] = !used ? nullptr : skinny ? w[i]->qs : w[i]->qs_tiled;
         grp.d[i] = used ? w[i]->d : nullptr;
         grp.y[i] = used ? y[i] : nullptr;
         grp.res[i] = i == 0 ? residual : nullptr;
         grp.n[i] = used ? (int)w[i]->n_out : 0;
         grp.wg0[i] = used ? wgs : INT_MAX;
-        if (used) wgs += (int)((w[i]->n_out + 16 * tiles - 1) / (16 * tiles));
+        if (used) wgs += (int)((w[i]->n_out + rows - 1) / rows);
     }
-    const dim3 grid((unsigned)wgs);
-    // LDS is handed out per workgroup: nw wavefronts' rings each; up to 16 wavefronts a CU (4 a SIMD)
-    const size_t units = (size_t)nb / 8;
-    auto fits = [&](int nw_) {
-        if (m > 8) return (size_t)grid.x * nw_ <= (size_t)ctx->num_cu * (q8 || q41 ? 6 : 7);
-        const size_t per_cu = std::min<size_t>(lds_cu / ((size_t)nw_ * stages * unit_bytes), 16 / nw_);
-        return (size_t)grid.x <= (size_t)ctx->num_cu * per_cu;
-    };
-    int nw = m <= 8 ? 8 : 4;
-    while (nw > 1 && (!fits(nw) || units / nw < 4)) nw >>= 1;
-#define PG_GSK_LAUNCH(QTT, NBB, MTT, NWW, NSTT)                                                                                \
-    do {                                                                                                                       \
-        auto kern = gguf_skinny_kernel<QTT == 8 ? 8 : 4, NBB, MTT, NWW, NSTT, QTT == 5>;                                       \
-        skinny_args<QTT == 5> args;                                                                                            \
-        static_cast<pg_skinny_group &>(args) = grp;                                                                            \
-        args.set(w, count, md);                                                                                                \
-        const size_t lds = (size_t)NWW * NSTT * (NBB * ((QTT == 8 ? 4096 : 2048) + (QTT == 5 ? 512 : 256)) + MTT * 512 + (QTT == 5 ? 1024 : 512)); \
-        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
-        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_few_rows_mm" : (QTT == 5 ? "gguf_q4_1_few_rows_mm" : "gguf_q4_0_few_rows_mm"), kern, grid, \
-                         dim3(64 * NWW), lds, args, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs); \
-    } while (0)
-#define PG_GSK_NW8(QTT, NBB, MTT, NSTT)                     \
-    switch (nw) {                                           \
-        case 8: PG_GSK_LAUNCH(QTT, NBB, MTT, 8, NSTT);      \
-        case 4: PG_GSK_LAUNCH(QTT, NBB, MTT, 4, NSTT);      \
-        case 2: PG_GSK_LAUNCH(QTT, NBB, MTT, 2, NSTT);      \
-        default: PG_GSK_LAUNCH(QTT, NBB, MTT, 1, NSTT);     \
-    }
-#define PG_GSK_NW4(QTT, MTT, NSTT)                        \
-    switch (nw) {                                         \
-        case 4: PG_GSK_LAUNCH(QTT, 1, MTT, 4, NSTT);      \
-        case 2: PG_GSK_LAUNCH(QTT, 1, MTT, 2, NSTT);      \
-        default: PG_GSK_LAUNCH(QTT, 1, MTT, 1, NSTT);     \
-    }
-    if (q8) {
-        if (m <= 4) { if (tiles == 2) PG_GSK_NW8(8, 2, 4, 2) else PG_GSK_NW8(8, 1, 4, 2) }
-        if (m <= 8) { if (tiles == 2) PG_GSK_NW8(8, 2, 8, 2) else PG_GSK_NW8(8, 1, 8, 2) }
-        PG_GSK_NW4(8, 16, 2)
-    }
-    if (q41) {  // (5 names Q4_1 here)
-        if (m <= 8) { if (tiles == 2) PG_GSK_NW8(5, 2, 8, 2) else PG_GSK_NW8(5, 1, 8, 2) }
-        PG_GSK_NW4(5, 16, 2)
-    }
-    if (m <= 4) { if (tiles == 2) PG_GSK_NW8(4, 2, 4, 2) else PG_GSK_NW8(4, 1, 4, 2) }
-    if (m <= 8) { if (tiles == 2) PG_GSK_NW8(4, 2, 8, 2) else PG_GSK_NW8(4, 1, 8, 2) }
-    PG_GSK_NW4(4, 16, 2)
-#undef PG_GSK_NW8
-#undef PG_GSK_NW4
-#undef PG_GSK_LAUNCH
+    return skinny ? launch_skinny(ctx, k_in, ggml_type == PG_GGML_Q8_0, grp, wgs, tiles, m, md) : launch_ktile(ctx, ggml_type, k_in, w, count, grp, wgs, m, md);
 }
 
 pg_status pg_launch_gguf_mm(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const uint8_t *qs,

@@ -2338,9 +2338,8 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
     const size_t n_of[7] = {q_dim, kv_dim, kv_dim, d, ffn, ffn, d}, k_of[7] = {d, d, d, q_dim, d, d, ffn};
     // q|k|v and gate|up are one launch each (the tensors' 128-row groups one after the other): one K split for the launch
     const int first_of[7] = {0, 0, 0, 3, 4, 4, 6}, count_of[7] = {3, 3, 3, 1, 2, 2, 1};
-    // Up to eight tokens: the few-rows product (one launch per tensor group, no K split between workgroups, so every
-    // product leaves one plane; the weights are read in their row-major planes, no tile-major copy).
-    // (Nine to sixteen tokens: only the products over fewer than 32 weight rows per CU, see pg_gguf_skinny_takes.)
+    // Few tokens, or some dozens over small tensors: the one-launch products (no K split between workgroups, so every
+    // product leaves one plane; see pg_gguf_one_launch_takes).
     bool few[7], hm[7];
     int ks[7];
     size_t part_off[7], floats = 0;
@@ -2350,7 +2349,7 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
             groups += (n_of[j] + 127) / 128;
             rows += n_of[j];
         }
-        few[i] = pg_gguf_skinny_takes(ctx, type, seq, rows, k_of[i]);
+        few[i] = pg_gguf_one_launch_takes(ctx, type, seq, rows, k_of[i], i != 6);
         ks[i] = few[i] ? 1 : pg_gguf_mm_splitk(ctx, groups * 128, k_of[i], tiles, seq, false, nullptr);
         // Many tokens: the f16 matrix-core product where it is the faster one (its input then arrives as two f16
         // planes, not as digit planes; the down projection's producer holds a row of the FFN width in registers).
@@ -2393,7 +2392,7 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
         }
         if (few[i]) {
             float *ys[3] = {part(i), count_of[i] > 1 ? part(i + 1) : nullptr, count_of[i] > 2 ? part(i + 2) : nullptr};
-            return pg_launch_gguf_skinny_group(ctx, type, k_of[i], b->w + i, ys, count_of[i], seq, md);
+            return pg_launch_gguf_one_launch(ctx, type, k_of[i], b->w + i, ys, count_of[i], seq, md);
         }
         pg_mm_group g = grp;
         size_t groups = 0;
@@ -2454,7 +2453,7 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
     }
     if (few[6]) {  // the down product adds the residual itself
         float *ys[1] = {out_dev};
-        return pg_launch_gguf_skinny_group(ctx, type, k_of[6], b->w + 6, ys, 1, seq, md_f, h1);
+        return pg_launch_gguf_one_launch(ctx, type, k_of[6], b->w + 6, ys, 1, seq, md_f, h1);
     }
     PG_TRY(product(6, md_f));
     if ((uintptr_t)out_dev % 16 == 0)  // (d is a multiple of 32 and the arena's slices are aligned)

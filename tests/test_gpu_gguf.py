@@ -421,3 +421,33 @@ def test_gguf_q4_1_few_rows(ctx, orc, n_out, k_in, m):
         sl = slice(r * n_out, (r + 1) * n_out)
         H.assert_close_rel(got[sl], want[sl], RTOL_ACHIEVED_MM, f"row {r}")
     gw.free()
+
+
+@pytest.mark.parametrize("typ", [2, 8, 3])
+@pytest.mark.parametrize("n_out,k_in,m", [
+    (31, 256, 8), (33, 288, 9), (127, 320, 16), (129, 1024, 17), (257, 1056, 24), (1000, 4096, 32), (64, 8224, 33),   # tokens in eights and sixteens
+    (515, 2080, 47), (4100, 1152, 48), (96, 14336, 64), (1, 1312, 31), (2050, 544, 63), (6144, 512, 25),
+    (300, 1024, 65), (700, 6112, 96), (33, 992, 130), (129, 2048, 257), (3000, 4096, 40),                             # tokens in thirty-twos
+    (5000, 4096, 130), (9000, 480, 20), (40, 8192, 70),                                                               # other routes beside them
+])
+def test_gguf_rows_in_tiles(ctx, orc, n_out, k_in, m, typ):
+    """Few and some dozens of rows in one launch after the digits: ragged weight rows, K of whole and part stages, whole and part
+    groups of tokens, with outlier channels and a row of zeros."""
+    from peregrine_amd import gguf
+    say(f"gguf_matmul rows in tiles n_out={n_out} k_in={k_in} m={m} type={typ}")
+    w = orc.rng_normal(41 + n_out, n_out * k_in, 0.0, 0.02) + (np.float32(0.03) if typ == 3 else np.float32(0))
+    raw = {2: H.pack_q4_0, 3: H.pack_q4_1, 8: H.pack_q8_0}[typ](w)
+    x = orc.rng_normal(43 + m, m * k_in)
+    x.reshape(m, k_in)[:, :: max(1, k_in // 40)] *= 20
+    x.reshape(m, k_in)[m // 2] = 0
+    gw = gguf.GgufWeight(raw, typ, n_out, k_in, ctx)
+    got, want = gw.matmul(x, m), orc.gguf_matmul(x, m, raw, typ, n_out, k_in)
+    # A row's activations are off by up to blockmax / 65278 each, independently of its weights, so an output's error goes with
+    # |x| |w| and not with what is left of the output after cancellation: with |x| rms(w), the outputs' expected size, for the floor
+    # (an rms over the row's own outputs is no floor where there is one of them).
+    xr, g, v = x.reshape(m, k_in).astype(np.float64), np.asarray(got, np.float64).reshape(m, n_out), np.asarray(want, np.float64).reshape(m, n_out)
+    floor = np.linalg.norm(xr, axis=1) * np.sqrt(np.mean(w.astype(np.float64) ** 2))
+    err = np.abs(g - v) - RTOL_ACHIEVED_MM * np.maximum(np.abs(v), floor[:, None])
+    assert (err <= 0).all(), (np.unravel_index(err.argmax(), err.shape), err.max())
+    assert not g[m // 2].any()
+    gw.free()
