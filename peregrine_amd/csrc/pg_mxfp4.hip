@@ -611,13 +611,20 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
         }
 }
 
-template <int RA, int TB, int BD, bool GROUPED>
-__global__ __launch_bounds__(64 * MT_NW) __attribute__((amdgpu_waves_per_eu(GROUPED && TB == 1 && RA <= 2 ? 4 : 2))) void mxfp4_tiles_kernel(const uint8_t *__restrict__ qs_frag, const uint32_t *__restrict__ sc_frag,
+template <typename F, int... I>
+__device__ __forceinline__ void mt_steps(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int RA, int TB, int BD, bool GROUPED, int NW = MT_NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED && TB == 1 && RA <= 2 ? 4 : 2))) void mxfp4_tiles_kernel(const uint8_t *__restrict__ qs_frag, const uint32_t *__restrict__ sc_frag,
                                                                  const char *__restrict__ bq, float *__restrict__ y, int n_out,
                                                                  int ncp, int m, int n_tt, int ks, int cps, size_t part_stride,
                                                                  int items, int per_xcd, const mt_gather gat, const mt_experts ex) {
-    constexpr int STAGE = TB * MT_RECORD, UNITS = TB * MT_UNITS, ROUNDS = (UNITS + 64 * MT_NW - 1) / (64 * MT_NW);
+    constexpr int STAGE = TB * MT_RECORD, UNITS = TB * MT_UNITS, ROUNDS = (UNITS + 64 * NW - 1) / (64 * NW);
     constexpr bool RING = RA == 4;  // A two chunks ahead in a ring of two; else the next batch of four chunks
+    constexpr int AHEAD = RA == 1 && TB > 1 ? 3 : 1;  // planes read ahead: the fewer products a plane feeds, the less of the LDS latency they cover
+    static_assert(NW == MT_NW || TB > 1, "narrow tiles are staged by all of MT_NW wavefronts");
     static_assert(BD == 1 || BD == 2 || BD == 4, "the staging depth divides the unrolled batch");
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -649,7 +656,7 @@ __global__ __launch_bounds__(64 * MT_NW) __attribute__((amdgpu_waves_per_eu(GROU
         return kc0 + (i < run ? i : i - run);
     };
     const int nrg = (n_out + 15) / 16;                       // >= RA (the launcher's choice of RA)
-    const int rg_mine = (wt * MT_NW + wave) * RA;            // the row groups whose tiles this wavefront stores
+    const int rg_mine = (wt * NW + wave) * RA;            // the row groups whose tiles this wavefront stores
     const int rg0 = pg_mt_first_row_group(rg_mine, RA, nrg);  // the ones it reads: a spare wavefront repeats the last ones
     const size_t a_stride = (size_t)ncp * 64;                // v4i per row group
     const gv4i_ptr qa = (gv4i_ptr)(uintptr_t)qs_frag + (size_t)rg0 * a_stride;
@@ -684,7 +691,7 @@ __global__ __launch_bounds__(64 * MT_NW) __attribute__((amdgpu_waves_per_eu(GROU
     const char *const b_base = bq + (size_t)tt * TB * ncp * MT_RECORD;
     unsigned b_off[ROUNDS];
 #pragma unroll
-    for (int i = 0; i < ROUNDS; ++i) b_off[i] = pg_mt_unit_offset((int)threadIdx.x + i * 64 * MT_NW, UNITS, ncp);
+    for (int i = 0; i < ROUNDS; ++i) b_off[i] = pg_mt_unit_offset((int)threadIdx.x + i * 64 * NW, UNITS, ncp);
     v4i sr[BD][ROUNDS];
 #define PG_MT_FETCH_B(SLOT, C)                                                                                          \
     do {                                                                                                                \
@@ -694,7 +701,7 @@ __global__ __launch_bounds__(64 * MT_NW) __attribute__((amdgpu_waves_per_eu(GROU
 #define PG_MT_PUT_B(STG, SLOT)                                                                                          \
     do {                                                                                                                \
         _Pragma("unroll") for (int i = 0; i < ROUNDS; ++i) {                                                            \
-            const int u = (int)threadIdx.x + i * 64 * MT_NW;                                                            \
+            const int u = (int)threadIdx.x + i * 64 * NW;                                                            \
             if (u < UNITS) *reinterpret_cast<v4i *>(lds + (STG) * STAGE + u * 16) = sr[SLOT][i];                        \
         }                                                                                                               \
     } while (0)
@@ -735,70 +742,48 @@ __global__ __launch_bounds__(64 * MT_NW) __attribute__((amdgpu_waves_per_eu(GROU
                 for (int u = 0; u < 4; ++u) fetch_a(an[RING ? 0 : u], next + u);
             }
         }
-    // One plane of one token group: its two operand halves are read while the previous plane's instructions run.
-    // (The byte selectors of the two scale operands are immediates: chunk within the dword, plane within the dword.)
-#define PG_MT_READ(G, J, B0, B1)                                                                  \
-    do {                                                                                          \
-        B0 = *reinterpret_cast<const v4i *>(st + (G) * MT_RECORD + (J) * MT_FRAG + lane * 16);      \
-        B1 = *reinterpret_cast<const v4i *>(st + (G) * MT_RECORD + (J) * MT_FRAG + 1024 + lane * 16); \
-    } while (0)
-#define PG_MT_MUL(U, G, J, B0, B1)                                                                                          \
-    do {                                                                                                                    \
-        const v8i B = {B0[0], B0[1], B0[2], B0[3], B1[0], B1[1], B1[2], B1[3]};                                             \
-        _Pragma("unroll") for (int r = 0; r < RA; ++r) {                                                                    \
-            const v4i aw = a[RING ? (U) & 1 : (U)][r];                                                                      \
-            const v8i A = {aw[0], aw[1], aw[2], aw[3], 0, 0, 0, 0};                                                         \
-            acc[r][G] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, acc[r][G], 4, 0, (U), (int)sca[r], (J), sbv[G]); \
-            asm volatile("" : "+v"(acc[r][G]));  /* (or the compiler sinks every product to the end of the loop body) */  \
-        }                                                                                                                   \
-    } while (0)
-#define PG_MT_GROUP(U, G)                                                 \
-    do {                                                                  \
-        if ((G) < TB && (!GROUPED || (G) < live)) {                       \
-            PG_MT_READ(G, 1, y0, y1);                                     \
-            PG_MT_MUL(U, G, 0, x0, x1);                                   \
-            __builtin_amdgcn_sched_barrier(0);                            \
-            PG_MT_READ(G, 2, x0, x1);                                     \
-            PG_MT_MUL(U, G, 1, y0, y1);                                   \
-            __builtin_amdgcn_sched_barrier(0);                            \
-            PG_MT_READ(G, 3, y0, y1);                                     \
-            PG_MT_MUL(U, G, 2, x0, x1);                                   \
-            __builtin_amdgcn_sched_barrier(0);                            \
-            if ((G) + 1 < TB) PG_MT_READ((G) + 1 < TB ? (G) + 1 : 0, 0, x0, x1); \
-            PG_MT_MUL(U, G, 3, y0, y1);                                   \
-            __builtin_amdgcn_sched_barrier(0);                            \
-        }                                                                 \
-    } while (0)
-#define PG_MT_CHUNK(U)                                                                                   \
-    do {                                                                                                 \
-        const int c = cb + (U);                                                                          \
-        const char *st = lds + ((U) & 1) * STAGE;                                                        \
-        int sbv[TB];                                                                                     \
-        _Pragma("unroll") for (int g = 0; g < TB; ++g)                                                   \
-            sbv[g] = *reinterpret_cast<const int *>(st + g * MT_RECORD + MT_PLANES * MT_FRAG + lane * 4); \
-        v4i x0, x1, y0, y1;                                                                              \
-        PG_MT_READ(0, 0, x0, x1);                                                                        \
-        __builtin_amdgcn_sched_barrier(0);                                                               \
-        PG_MT_GROUP(U, 0);                                                                               \
-        PG_MT_GROUP(U, 1);                                                                               \
-        PG_MT_GROUP(U, 2);                                                                               \
-        PG_MT_GROUP(U, 3);                                                                               \
-        if (c + 1 < run) {                                                                               \
-            PG_MT_PUT_B(((U) + 1) & 1, ((U) + 1) % BD);                                                  \
-            if (c + 1 + BD < run) PG_MT_FETCH_B(((U) + 1) % BD, chunk_at(c + 1 + BD));                   \
-        }                                                                                                \
-        if (RING && c + 2 < run) fetch_a(a[RING ? (U) & 1 : 0], chunk_at(c + 2));                        \
-        __syncthreads();                                                                                 \
-    } while (0)
-        static_assert(MT_PLANES == 4 && TB <= 4, "the plane steps are written out");
-        PG_MT_CHUNK(0);
-        PG_MT_CHUNK(1);
-        PG_MT_CHUNK(2);
-        PG_MT_CHUNK(3);
-#undef PG_MT_CHUNK
-#undef PG_MT_GROUP
-#undef PG_MT_MUL
-#undef PG_MT_READ
+        // One step = one plane of one token group against the wavefront's RA row groups; the operand halves of the plane AHEAD steps on
+        // are read meanwhile.  (The byte selectors of the two scale operands are immediates: chunk within the dword, plane within the dword.)
+        auto chunk = [&](auto u_) {
+            constexpr int U = decltype(u_)::value;
+            const int c = cb + U;
+            const char *st = lds + (U & 1) * STAGE;
+            int sbv[TB];
+#pragma unroll
+            for (int g = 0; g < TB; ++g) sbv[g] = *reinterpret_cast<const int *>(st + g * MT_RECORD + MT_PLANES * MT_FRAG + lane * 4);
+            v4i b[AHEAD + 1][2];
+            auto read = [&](int step) {
+                const char *f = st + step / MT_PLANES * MT_RECORD + step % MT_PLANES * MT_FRAG + lane * 16;
+                b[step % (AHEAD + 1)][0] = *reinterpret_cast<const v4i *>(f);
+                b[step % (AHEAD + 1)][1] = *reinterpret_cast<const v4i *>(f + 1024);
+            };
+            auto step = [&](auto i_) {
+                constexpr int I = decltype(i_)::value, G = I / MT_PLANES, J = I % MT_PLANES;
+                if (GROUPED && G >= live) return;
+                if (I + AHEAD < TB * MT_PLANES) read(I + AHEAD);
+                const v4i b0 = b[I % (AHEAD + 1)][0], b1 = b[I % (AHEAD + 1)][1];
+                const v8i B = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
+#pragma unroll
+                for (int r = 0; r < RA; ++r) {
+                    const v4i aw = a[RING ? U & 1 : U][r];
+                    const v8i A = {aw[0], aw[1], aw[2], aw[3], 0, 0, 0, 0};
+                    acc[r][G] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, acc[r][G], 4, 0, U, (int)sca[r], J, sbv[G]);
+                    asm volatile("" : "+v"(acc[r][G]));  /* (or the compiler sinks every product to the end of the loop body) */
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) read(i);
+            __builtin_amdgcn_sched_barrier(0);
+            mt_steps(step, std::make_integer_sequence<int, TB * MT_PLANES>{});
+            if (c + 1 < run) {
+                PG_MT_PUT_B((U + 1) & 1, (U + 1) % BD);
+                if (c + 1 + BD < run) PG_MT_FETCH_B((U + 1) % BD, chunk_at(c + 1 + BD));
+            }
+            if (RING && c + 2 < run) fetch_a(a[RING ? U & 1 : 0], chunk_at(c + 2));
+            __syncthreads();
+        };
+        mt_steps(chunk, std::make_integer_sequence<int, 4>{});
         if (more) {
 #pragma unroll
             for (int r = 0; r < RA; ++r) sca[r] = sca_next[r];
@@ -855,14 +840,14 @@ pg_status launch_tiles(pg_ctx *ctx, const pg_gguf_tensor *w, const char *bq, flo
 }
 
 // The grouped form: `max_tiles` token tiles at most (the launch covers them all; those past the experts' last exit).
-template <int RA, int TB, int BD>
+template <int RA, int TB, int BD, int NW = MT_NW>
 pg_status launch_tiles_grouped(pg_ctx *ctx, size_t n_out, int ncp, const char *bq, float *y, size_t n_wt, size_t max_tiles,
                                const mt_gather &gat, const mt_experts &ex) {
     const size_t lds = TB == 1 ? std::max<size_t>(2 * MT_RECORD, 2 * 4 * (2 * 2048 + 256)) : 2 * (size_t)TB * MT_RECORD;  // (mxfp4_narrow_tile<RA, 2>)
-    auto kern = mxfp4_tiles_kernel<RA, TB, BD, true>;
+    auto kern = mxfp4_tiles_kernel<RA, TB, BD, true, NW>;
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
     const size_t per_xcd = (max_tiles + 7) / 8 * n_wt, items = 8 * per_xcd;
-    return pg_launch(ctx, "mxfp4_tiles_grouped", kern, dim3((unsigned)(8 * per_xcd)), dim3(64 * MT_NW), lds, (const uint8_t *)nullptr,
+    return pg_launch(ctx, "mxfp4_tiles_grouped", kern, dim3((unsigned)(8 * per_xcd)), dim3(64 * NW), lds, (const uint8_t *)nullptr,
                      (const uint32_t *)nullptr, bq, y, (int)n_out, ncp, 0, (int)n_wt, 1, ncp, (size_t)0, (int)items, (int)per_xcd, gat, ex);
 }
 
@@ -1115,28 +1100,90 @@ __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__r
 
 // One grouped product: rows `src` (pair / div) of the experts' slots -> records -> tiles against tensor table `which`.
 // With `act`: the rows are the swiglu of src, mlp1's outputs.
-pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, int tb, size_t max_tiles, mt_gather gat, int div,
+// How the tiles of a grouped product are cut: TB groups of 16 slots, RA groups of 16 weight rows a wavefront, NW wavefronts.
+struct mt_shape { int tb, ra, nw; };
+
+// Up to twelve slots an expert on average (narrow tiles, most of them): one group of slots, and the widest row tile that leaves every CU
+// two workgroups.  Beyond, the tiling of least estimated time for both products together: a chunk takes `chunk` and, for every
+// workgroup of the fullest CU, `wg` us (the tail tiles' empty groups are skipped); the experts' slots as binomials.  Timed on 349
+// shapes (10 to 512 tokens, 8 to 32 experts, 512 to 2880 wide), every tiling of each product: 1 to 2 % over the better of the two
+// rules up to 80 tokens, 7 % over the best tiling beyond, where the old rule (slots by the average, rows by two workgroups a CU) is 10 to
+// 20 % over it.  us, before : now: 471 tokens, 8 experts, 2784 x 672 116 : 88, 410, 16, 1312 x 864 105 : 85, 208, 32, 2272 x 1696
+// 139 : 117, 512, 8, 2048 x 2048 206 : 166.
+struct mt_cost { mt_shape s; double chunk, wg; };
+constexpr mt_cost MT_COSTS[] = {{{1, 1, 8}, 0.112, 0.542}, {{2, 1, 8}, 0.128, 0.807}, {{2, 2, 8}, 0.059, 1.192}, {{2, 4, 8}, 0.404, 1.238},
+                                {{2, 4, 4}, 0.784, 0.528}, {{4, 4, 8}, 0.414, 2.23}};
+double expected_tiles(size_t T, size_t E, size_t top_k, int slots) {
+    const double p = (double)top_k / (double)E, mu = (double)T * p, sd = sqrt(std::max(mu * (1.0 - p), 1e-9));
+    double tiles = 1.0 - pow(1.0 - p, (double)T);
+    for (size_t j = 1; j * slots < T; ++j) {
+        const double more = 0.5 * erfc(((double)(j * slots) + 0.5 - mu) / (sd * 1.41421356));
+        if (more < 1e-4) break;
+        tiles += more;
+    }
+    return tiles * (double)E;
+}
+void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const size_t (&n_out)[2], const int (&ncp)[2], mt_shape (&out)[2]) {
+    const size_t P = T * top_k, cus = (size_t)ctx->num_cu;
+    if (P < 12 * E) {
+        const size_t max_tiles = P / 16 + E;
+        for (int i = 0; i < 2; ++i) {
+            const size_t nrg = (n_out[i] + 15) / 16;
+            int ra = 4;
+            while (ra > 1 && ((size_t)ra > nrg || (nrg + MT_NW * ra - 1) / (MT_NW * ra) * max_tiles < 2 * cus)) ra >>= 1;
+            out[i] = {1, ra, MT_NW};
+        }
+        return;
+    }
+    double best = 1e300;
+    for (int tb = 1; tb <= 4; tb *= 2) {
+        const double tiles = expected_tiles(T, E, top_k, 16 * tb);
+        const double live = tb == 1 ? 1.0 : 0.4 + 0.6 * std::min(1.0, ((double)P / 16.0 + 0.5 * (double)E) / (tiles * tb));
+        const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));
+        mt_shape pick[2] = {};
+        double sum = 0.0;
+        for (int i = 0; i < 2; ++i) {
+            const size_t nrg = (n_out[i] + 15) / 16;
+            double least = 1e299;
+            for (const mt_cost &c : MT_COSTS) {
+                if (c.s.tb != tb || (size_t)c.s.ra > nrg) continue;
+                const double w = std::max(1.0, tiles * (double)((nrg + c.s.nw * c.s.ra - 1) / (c.s.nw * c.s.ra)) / (double)cus);
+                const double stream = hit * (double)n_out[i] * ncp[i] * 68.0 / 5.6e6;  // (the weights once)
+                const double us = std::max(stream, 1.0 + ncp[i] * (c.chunk + c.wg * 0.5 * (w + ceil(w)) * live));
+                if (us < least) {
+                    least = us;
+                    pick[i] = c.s;
+                }
+            }
+            sum += least;
+        }
+        if (sum < best) {
+            best = sum;
+            out[0] = pick[0];
+            out[1] = pick[1];
+        }
+    }
+}
+
+pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, const mt_shape &sh, size_t max_tiles, mt_gather gat, int div,
                       const void **tab, size_t experts, int which, char *bq, float *y, const mt_swiglu *act = nullptr) {
     const int nb = (int)(k_in / 32), ncp = (int)mx_chunks((size_t)nb);
     gat.div = div;
-    const size_t groups = max_tiles * tb, threads = groups * 2 * (size_t)ncp * 64;
+    const size_t groups = max_tiles * sh.tb, threads = groups * 2 * (size_t)ncp * 64;
     PG_CHECK_ARG((threads + 255) / 256 < ((size_t)1 << 31), "mxfp4 moe: too many pairs x %zu for one pre-pass", k_in);
     const dim3 grid((unsigned)((threads + 255) / 256));
     if (act) PG_TRY(pg_launch(ctx, "mxfp4_planes_swiglu", mxfp4_planes_kernel<true, true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, *act));
     else PG_TRY(pg_launch(ctx, "mxfp4_planes_gather", mxfp4_planes_kernel<true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, mt_swiglu{}));
-    const size_t nrg = (n_out + 15) / 16;
-    int ra = 4;
-    while (ra > 1 && ((size_t)ra > nrg || (nrg + MT_NW * ra - 1) / (MT_NW * ra) * max_tiles < 2 * (size_t)ctx->num_cu)) ra >>= 1;
-    const size_t n_wt = (nrg + MT_NW * ra - 1) / (MT_NW * ra);
+    const size_t nrg = (n_out + 15) / 16, n_wt = (nrg + sh.nw * sh.ra - 1) / (sh.nw * sh.ra);
     PG_CHECK_ARG(n_wt * max_tiles < ((size_t)1 << 28), "mxfp4 moe: %zu x %zu tiles", n_wt, max_tiles);
     const mt_experts ex = {reinterpret_cast<const uint8_t *const *>(tab + (size_t)(2 * which) * experts),
                            reinterpret_cast<const uint32_t *const *>(tab + (size_t)(2 * which + 1) * experts)};
-#define PG_MTG(RA_, BD1, BD2, BD4) \
-    (tb == 1 ? launch_tiles_grouped<RA_, 1, BD1>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex) \
-     : tb == 2 ? launch_tiles_grouped<RA_, 2, BD2>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex) \
-               : launch_tiles_grouped<RA_, 4, BD4>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex))
-    return ra == 4 ? PG_MTG(4, 4, 2, 1) : (ra == 2 ? PG_MTG(2, 2, 4, 2) : PG_MTG(1, 4, 4, 4));
+#define PG_MTG(TB, RA, BD, NW) \
+    if (sh.tb == TB && sh.ra == RA && sh.nw == NW) return launch_tiles_grouped<RA, TB, BD, NW>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex);
+    PG_MTG(1, 1, 4, 8) PG_MTG(1, 2, 2, 8) PG_MTG(1, 4, 4, 8)
+    PG_MTG(2, 1, 4, 8) PG_MTG(2, 2, 4, 8) PG_MTG(2, 4, 2, 8) PG_MTG(2, 4, 2, 4) PG_MTG(4, 4, 1, 8)
 #undef PG_MTG
+    return pg_fail(PG_EUNSUPPORTED, "mxfp4 moe: no kernel of %d x 16 slots, %d row groups, %d wavefronts", sh.tb, sh.ra, sh.nw);
 }
 
 // Whether up to 64 pairs are faster one by one than as tiles although pairs share experts (P > 2 E): the decode kernel streams an
@@ -1192,10 +1239,11 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     PG_CHECK_ARG((uintptr_t)x_dev % 16 == 0, "pg_mxfp4_moe_ffn: x must be 16-byte aligned");
     PG_CHECK_ARG(T * top_k < (1ull << 20), "pg_mxfp4_moe_ffn: too many (token, expert) pairs");
     const size_t P = T * top_k;
-    // token tiles: groups of 16 slots, as many to a tile as an expert's average share suggests
-    const int tb = P / E <= 16 ? 1 : (P / E <= 32 ? 2 : 4);
-    const size_t max_tiles = P / (16 * (size_t)tb) + E;  // sum over experts of ceil(count / (16 tb)) stays below
     const int ncp1 = (int)mx_chunks(hidden / 32), ncp2 = (int)mx_chunks(inter / 32);
+    mt_shape shape[2];
+    choose_tiles(ctx, T, E, top_k, {2 * inter, hidden}, {ncp1, ncp2}, shape);
+    const int tb = shape[0].tb;
+    const size_t max_tiles = P / (16 * (size_t)tb) + E;  // sum over experts of ceil(count / (16 tb)) stays below
     // With few pairs hardly two of them meet in an expert, and a pair is a one-row product: the decode kernel, one
     // workgroup column per pair (exact activations; no expert lists).  Otherwise the experts' token tiles on the tile kernel.
     const bool by_pairs = P <= 64 && (P <= 2 * E || pairs_faster(T, E, top_k, hidden, inter)) && pairs_fit(ncp1) && pairs_fit(ncp2);
@@ -1230,7 +1278,7 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     if (by_pairs)
         PG_TRY(moe_product_pairs(ctx, x_dev, T, hidden, 2 * inter, P, (int)top_k, tab, E, 0, topk_idx, h));
     else
-        PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, tb, max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
+        PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, shape[0], max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
     const float *const *bias1 = reinterpret_cast<const float *const *>(tab + 4 * E);
     if (by_pairs) {
         PG_TRY(pg_launch(ctx, "mxfp4_moe_swiglu", mxfp4_moe_swiglu_kernel, dim3(grid_for(P * inter, 256)), dim3(256), 0, (const float *)h,
@@ -1238,7 +1286,7 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
         PG_TRY(moe_product_pairs(ctx, act, P, inter, hidden, P, 1, tab, E, 1, topk_idx, yb));
     } else {
         const mt_swiglu sw = {bias1, alpha, clamp};
-        PG_TRY(moe_product(ctx, h, inter, hidden, tb, max_tiles, gat, 1, tab, E, 1, rec, yb, &sw));
+        PG_TRY(moe_product(ctx, h, inter, hidden, shape[1], max_tiles, gat, 1, tab, E, 1, rec, yb, &sw));
     }
     return pg_launch(ctx, "mxfp4_moe_combine", mxfp4_moe_combine_kernel, dim3(grid_for(T * hidden, 256)), dim3(256), 0, (const float *)yb,
                      reinterpret_cast<const float *const *>(tab + 5 * E), (const int *)topk_idx, (const float *)topk_p, T, hidden,

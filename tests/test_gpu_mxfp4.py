@@ -314,3 +314,13 @@ def test_mxfp4_moe_pairs_or_tiles(ctx, orc, hidden, inter, E, top_k, T, pairs):
         H.assert_close_rel(got[t], want[t], 2e-4, f"token {t}")
     for ex in experts:
         ex.free()
+
+
+@pytest.mark.parametrize("hidden,inter,E,top_k,T", [
+    (544, 2112, 16, 4, 90), (1440, 1440, 4, 4, 130), (1056, 1056, 8, 4, 300),   # 32 slots: 16 to 64 weight rows a wavefront, 4 and 8 of them
+    (1120, 544, 8, 4, 40), (352, 96, 2, 2, 70),                                 # 16 slots; few row groups
+    (2080, 1056, 16, 4, 700), (544, 1056, 2, 2, 1500),                          # 64 slots
+])
+def test_mxfp4_moe_tilings(ctx, orc, hidden, inter, E, top_k, T):
+    """Every tiling that the estimates choose from, at ragged row groups and last tiles."""
+    test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, T)
