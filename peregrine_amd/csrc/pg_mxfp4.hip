@@ -1109,10 +1109,11 @@ struct mt_shape { int tb, ra, nw; };
 // shapes (10 to 512 tokens, 8 to 32 experts, 512 to 2880 wide), every tiling of each product: 1 to 2 % over the better of the two
 // rules up to 80 tokens, 7 % over the best tiling beyond, where the old rule (slots by the average, rows by two workgroups a CU) is 10 to
 // 20 % over it.  us, before : now: 471 tokens, 8 experts, 2784 x 672 116 : 88, 410, 16, 1312 x 864 105 : 85, 208, 32, 2272 x 1696
-// 139 : 117, 512, 8, 2048 x 2048 206 : 166.
+// 139 : 117, 512, 8, 2048 x 2048 206 : 166; 64 slots, 32 experts
+// of 2880 x 2880, where tiles of 32 take 246 and 1075: 300 tokens 235, 2000 958.
 struct mt_cost { mt_shape s; double chunk, wg; };
 constexpr mt_cost MT_COSTS[] = {{{1, 1, 8}, 0.112, 0.542}, {{2, 1, 8}, 0.128, 0.807}, {{2, 2, 8}, 0.059, 1.192}, {{2, 4, 8}, 0.404, 1.238},
-                                {{2, 4, 4}, 0.784, 0.528}, {{4, 4, 8}, 0.414, 2.23}};
+                                {{2, 4, 4}, 0.784, 0.528}, {{4, 4, 8}, 0.414, 1.9}};
 double expected_tiles(size_t T, size_t E, size_t top_k, int slots) {
     const double p = (double)top_k / (double)E, mu = (double)T * p, sd = sqrt(std::max(mu * (1.0 - p), 1e-9));
     double tiles = 1.0 - pow(1.0 - p, (double)T);
