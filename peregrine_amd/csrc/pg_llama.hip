@@ -1227,6 +1227,7 @@ __global__ __launch_bounds__(128) void gqa_combine_kernel(const float *__restric
     if constexpr (DIG == 0) {
         for (int i = tid; i < hd; i += 128) {
             float o = 0.f;
+#pragma unroll 8
             for (int s = 0; s < splits; ++s) o += wts[s] * p[s * rec + hdr + i];
             float *dst = out + (size_t)blockIdx.x * hd + i;
             *dst = accumulate ? *dst + o * inv : o * inv;
@@ -1235,6 +1236,7 @@ __global__ __launch_bounds__(128) void gqa_combine_kernel(const float *__restric
         const int qt = blockIdx.x / nqh, qh = blockIdx.x - qt * nqh;
         for (int i4 = tid; i4 < hd / 4; i4 += 128) {  // whole 8-lane groups: hd / 4 is a multiple of 8
             float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
             for (int s = 0; s < splits; ++s) {
                 const float wv = wts[s];
                 const float *src = p + s * rec + hdr + 4 * i4;
@@ -1249,7 +1251,8 @@ __global__ __launch_bounds__(128) void gqa_combine_kernel(const float *__restric
     }
 }
 
-// The same merge for head sizes 64 and 128 and at most MAXS (64 or 128) splits, every load in flight at once:
+// The same merge for head sizes 64 and 128 and at most MAXS (64, 128 or 256) splits, every load in flight at once (207 splits of three
+// tokens at 6599, 48 rows of 128: 20.8 us by the kernel above, one load behind the other, 5 here):
 // thread = (float4 of the row, slice of the splits), the slices' sums meet in LDS.  Splits are still added in
 // ascending order within a slice and the slices in ascending order: the result does not depend on timing.
 // A record is HDR floats (maximum, exp-sum, padding) followed by the row.  DIG as in gqa_combine_kernel.
@@ -1279,7 +1282,8 @@ __global__ __launch_bounds__(256) void gqa_combine_few_kernel(const float *__res
     }
     __syncthreads();
     float mine_m = sm[tid & 63];
-    if constexpr (MAXS > 64) mine_m = fmaxf(mine_m, sm[64 + (tid & 63)]);
+#pragma unroll
+    for (int s0 = 64; s0 < MAXS; s0 += 64) mine_m = fmaxf(mine_m, sm[s0 + (tid & 63)]);
     const float M = wave_max_f32(mine_m);
     const float m_ref = M == -INFINITY ? 0.f : M;
     float L = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1735,7 +1739,7 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         PG_TRY(pg_launch(ctx, "gqa_attention_tiled", kern, grid_t, dim3(256), lds_t, aa));
     } else
         PG_TRY(pg_launch(ctx, "gqa_attention", gqa_attention_kernel, grid, dim3(256), (256 + ATT_RED + chunk) * sizeof(float), aa));
-    if ((decode_kernel || split_kernel) && splits <= 128) {  // (these kernels: `out` is 16-byte aligned, hd is 64 or 128)
+    if ((decode_kernel || split_kernel) && splits <= 256) {  // (these kernels: `out` is 16-byte aligned, hd is 64 or 128)
         // what the merged rows leave as: f32, the streaming product's digits (one-token step), or -- a merge of key
         // runs under a many-token block step -- the matrix-core product's digit planes
         const bool planes = md && !xd && !accumulate;
@@ -1744,8 +1748,10 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         float *dxs = xd ? xd->xs : (planes ? md->xs : nullptr);
         const char *name = xd ? "gqa_combine_digits" : (planes ? "gqa_combine_mm_digits" : "gqa_combine");
 #define PG_COMBINE_FEW(HD_, DG_)                                                                                                   \
-    (split_kernel ? (splits <= 64 ? gqa_combine_few_kernel<HD_, DG_, 4, 64> : gqa_combine_few_kernel<HD_, DG_, 4, 128>)              \
-                  : (splits <= 64 ? gqa_combine_few_kernel<HD_, DG_, 2, 64> : gqa_combine_few_kernel<HD_, DG_, 2, 128>))
+    (split_kernel ? (splits <= 64 ? gqa_combine_few_kernel<HD_, DG_, 4, 64>                                                          \
+                                  : (splits <= 128 ? gqa_combine_few_kernel<HD_, DG_, 4, 128> : gqa_combine_few_kernel<HD_, DG_, 4, 256>)) \
+                  : (splits <= 64 ? gqa_combine_few_kernel<HD_, DG_, 2, 64>                                                          \
+                                  : (splits <= 128 ? gqa_combine_few_kernel<HD_, DG_, 2, 128> : gqa_combine_few_kernel<HD_, DG_, 2, 256>)))
 #define PG_COMBINE_FEW_HD(DG_) (hd == 64 ? PG_COMBINE_FEW(64, DG_) : PG_COMBINE_FEW(128, DG_))
         auto *kern = dg == 0 ? PG_COMBINE_FEW_HD(0) : (dg == 1 ? PG_COMBINE_FEW_HD(1) : (dg == 2 ? PG_COMBINE_FEW_HD(2) : (dg == 3 ? PG_COMBINE_FEW_HD(3) : PG_COMBINE_FEW_HD(4))));
 #undef PG_COMBINE_FEW_HD

@@ -572,3 +572,11 @@ def test_gqa_attention_of_halves_not_finite(ctx, orc):
     same[seq - 10:, 4:] = False
     same[(n - 10 - (n - seq)) // 32 * 32:, 4:] = False
     np.testing.assert_allclose(got[same], clean[same], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("hd,length", [(128, 4090), (128, 4100), (64, 4130), (128, 8190), (64, 8200), (128, 9001)])
+def test_gqa_attention_merges_many_runs(ctx, orc, hd, length):
+    """Two tokens of one kv head under a long cache: a run a key tile, so 128 to 282 records a row; at the lines between the merges
+    of up to 128 and 256 records and the one for any number."""
+    from peregrine_amd.llama import AttentionMask as M
+    _attention_case(ctx, orc, 5, 1, hd, 2, length, M.causal(length - 2), None, 430 + length)
