@@ -17,6 +17,7 @@
 // being consumed: each wavefront's own 32 weight rows and their f16 block scales, and the
 // token digits and scales of the stage, which the four wavefronts share.
 #include <limits.h>
+#include <type_traits>
 #include "pg_internal.h"
 #include "pg_stream_addr.h"
 #include "pg_digits.h"
@@ -243,7 +244,37 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t h) {
     return (float)v;
 }
 
-// grid: x = tiles of 128 weight rows, y = expert * tiles_per_expert + token tile, z = K chunk.
+// Tiles of `slots` pairs that experts' lists fill at most, T pairs each and P together: a launch over experts x ceil(T / slots) of them is
+// mostly workgroups that read a count and leave, a round of the chip each 768 of them (256 tokens, top 1 of 16 experts of 1024 x 4096,
+// Q4_0: 98.8 -> 67.5 us; 2000, 2 of 8, Q8_0: 444 -> 418; 64, 2 of 8 of 3072 x 8192: 155 -> 150; 81 to 2048 tokens 7 % in the mean).
+inline size_t expert_tiles_bound(size_t experts, size_t T, size_t P, size_t slots) {
+    return std::min(std::min(P, (P + experts * (slots - 1)) / slots), experts * ((T + slots - 1) / slots));
+}
+// The expert that tile `tile` of all experts' tiles belongs to (-1: past the last), its number among that expert's and the expert's pairs.
+// By a wavefront, 64 experts at a time: sums of their tiles up to each lane's, within rows of 16 lanes and then across them.
+__device__ __forceinline__ int expert_of_tile(const int *__restrict__ counts, int experts, int slots, int lane, int &tile, int &count) {
+    for (int e0 = 0; e0 < experts; e0 += 64) {
+        const int c = e0 + lane < experts ? counts[e0 + lane] : 0, mine = (int)((unsigned)(c + slots - 1) / (unsigned)slots);
+        int sum = mine;
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x111, 0xf, 0xf, false);  // row_shr:1, 2, 4, 8
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x112, 0xf, 0xf, false);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x114, 0xf, 0xf, false);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x118, 0xf, 0xf, false);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+        const unsigned long long past = __ballot(sum > tile);
+        if (past) {
+            const int l = __builtin_ctzll(past);
+            tile -= __builtin_amdgcn_readlane(sum - mine, l);
+            count = __builtin_amdgcn_readlane(c, l);
+            return e0 + l;
+        }
+        tile -= __builtin_amdgcn_readlane(sum, 63);
+    }
+    return -1;
+}
+
+// grid: x = tiles of 128 weight rows, y = token tile (with lists, of all experts: expert_of_tile), z = K chunk.
 // `chunk` (blocks per K chunk) is a multiple of NBU and no chunk is empty.
 // out: [K chunks][total pairs][n_out] (plain y with one chunk).
 // (Three wavefronts per SIMD, 168 registers each: the MFMA results are written to ordinary VGPRs,
@@ -287,13 +318,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         by = (st / nrgb) * 8 + (w >> 2);
         if (bx >= grp.remap_rg || by >= grp.remap_tiles) return;
     }
-    int e = 0, tt = by;
+    int e = 0, tt = by, count = grp.max_count;
     if (grp.counts) {
-        e = by / grp.tiles_per_expert;
-        tt = by - e * grp.tiles_per_expert;
-    }
-    const int count = grp.counts ? grp.counts[e] : grp.max_count;
-    if (tt * 32 >= count) return;  // the same for every thread of the workgroup
+        e = expert_of_tile(grp.counts, grp.num_experts, 32, lane, tt, count);
+        if (e < 0) return;  // the same for every thread of the workgroup
+    } else if (tt * 32 >= count) return;
     int n_out = n_out_arg;
     float *__restrict__ out = out_arg;
     const uint8_t *const *qs_table = grp.qs_table;
@@ -869,45 +898,82 @@ template <> struct ktile_args<true> : pg_skinny_group {
     }
 };
 
+// Experts' products: tile blockIdx.y of all experts' tiles of MT pairs, 32 rows of one of up to two tensors; pair p reads activation row
+// p / div and writes output row p.
+struct ktile_experts {
+    const uint8_t *const *qs[2];
+    const uint16_t *const *d[2];
+    float *y[2];
+    const int *lists, *counts;
+    int list_stride, div, experts, n, wgs1;  // wgs1: 32-row tiles of one tensor
+};
+
 template <int QT, int MT, bool Q41> struct KTCfg {
     static constexpr int W_T = QT == 8 ? 4096 : 2048, OFF_D = W_T, OFF_M = OFF_D + 256, OFF_DG = OFF_M + (Q41 ? 256 : 0);
     static constexpr int OFF_X = OFF_DG + MT * 256, OFF_S = OFF_X + MT * 16, UNIT = OFF_S + (Q41 ? MT * 16 : 0);
 };
-template <int QT, int MT, int NW, bool Q41>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_ktile_kernel(const ktile_args<Q41> grp, int nb, int nbp, int m,
+template <int QT, int MT, int NW, bool Q41, typename ARGS = ktile_args<Q41>>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_ktile_kernel(const ARGS grp, int nb, int nbp, int m,
                                                                 const int8_t *__restrict__ digits, const float *__restrict__ xs, int groups, int wgs) {
     using C = KTCfg<QT, MT, Q41>;
     static_assert(!Q41 || QT == 4, "Q4_1 is the Q4_0 product and its offsets");
-    int wg = blockIdx.x, t0 = 0;
-    if (groups > 1) {
-        const int j = blockIdx.x >> 3;
-        wg = j / groups * 8 + (blockIdx.x & 7);
-        t0 = j % groups * MT;
-        if (wg >= wgs) return;
-    }
+    constexpr bool EXPERTS = std::is_same_v<ARGS, ktile_experts>;
+    int wg = blockIdx.x, t0 = 0, n0, n_out;
+    const uint8_t *__restrict__ qs;
+    const uint16_t *__restrict__ dsc;
+    float *__restrict__ y;
+    const float *__restrict__ res = nullptr;
+    const int *__restrict__ list = nullptr;  // pairs of this tile's tokens
     int tg = 0;
+    if constexpr (EXPERTS) {
+        int tile = blockIdx.y;
+        const int e = expert_of_tile(grp.counts, grp.experts, MT, threadIdx.x & 63, tile, m);
+        if (e < 0) return;  // the same for every thread of the workgroup
+        t0 = tile * MT;
+        tg = wg >= grp.wgs1;
+        qs = grp.qs[tg][e];
+        dsc = grp.d[tg][e];
+        y = grp.y[tg];
+        n_out = grp.n;
+        n0 = (wg - tg * grp.wgs1) * 32;
+        list = grp.lists + (size_t)e * grp.list_stride + t0;
+    } else {
+        if (groups > 1) {
+            const int j = blockIdx.x >> 3;
+            wg = j / groups * 8 + (blockIdx.x & 7);
+            t0 = j % groups * MT;
+            if (wg >= wgs) return;
+        }
 #pragma unroll
-    for (int i = 1; i < 3; ++i) tg = wg >= grp.wg0[i] ? i : tg;
-    const int n_out = grp.n[tg];
-    float *__restrict__ y = grp.y[tg];
-    const float *__restrict__ res = grp.res[tg];
+        for (int i = 1; i < 3; ++i) tg = wg >= grp.wg0[i] ? i : tg;
+        qs = grp.qs[tg];
+        dsc = grp.d[tg];
+        y = grp.y[tg];
+        res = grp.res[tg];
+        n_out = grp.n[tg];
+        n0 = (wg - grp.wg0[tg]) * 32;
+    }
+    auto row_of = [&](int tok) -> size_t {  // activation row of a token of this tile
+        if constexpr (EXPERTS) return (size_t)(list[tok] / grp.div);
+        else return (size_t)(t0 + tok);
+    };
     extern __shared__ __attribute__((aligned(1024))) char lds[];  // NW rings of two units; afterwards the wavefronts' tiles
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l31 = lane & 31, hh = lane >> 5;
-    const int n0 = (wg - grp.wg0[tg]) * 32, mt = m - t0 < MT ? m - t0 : MT;
+    const int mt = m - t0 < MT ? m - t0 : MT;
     const int units = (nb + 3) / 4, per = (units + NW - 1) / NW;
     const int u_begin = wave * per, u_end = u_begin + per < units ? u_begin + per : units;
     const int cnt = u_end - u_begin;
     char *ring = lds + (size_t)wave * 2 * C::UNIT;
 
     // fill duties of this lane
-    const char *w_src = reinterpret_cast<const char *>(grp.qs[tg]) + (size_t)(n0 >> 7) * pg_tiled_group_bytes(nb, QT == 8) +
+    const char *w_src = reinterpret_cast<const char *>(qs) + (size_t)(n0 >> 7) * pg_tiled_group_bytes(nb, QT == 8) +
                         ((n0 >> 5) & 3) * C::W_T + lane * 16;
     const int ngroups = (n_out + 7) / 8;
     const int dg8 = (n0 >> 3) + (lane >> 4) < ngroups ? (n0 >> 3) + (lane >> 4) : ngroups - 1;
     const size_t d_at = (size_t)dg8 * nb * 16 + (lane & 3) * 4;
     const int d_jb = (lane >> 2) & 3;
-    const char *d_src = reinterpret_cast<const char *>(grp.d[tg]) + d_at;
+    const char *d_src = reinterpret_cast<const char *>(dsc) + d_at;
     const char *m_src = nullptr;
     if constexpr (Q41) m_src = reinterpret_cast<const char *>(grp.mo[tg]) + d_at;
     // digits: fill q covers runs 8 q .. 8 q + 7 of 128 bytes, run = 2 token + plane (tokens 8 .. 15 (mod 16) keep their planes swapped)
@@ -917,9 +983,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4)))
     for (int q = 0; q < MT / 4; ++q) {
         const int run = 8 * q + (lane >> 3), tok = run >> 1, pl = (run & 1) ^ ((tok >> 3) & 1), ch = (lane & 7) ^ (tok & 7);
         g_jb[q] = ch >> 1;
-        g_src[q] = digits + (size_t)(t0 + (tok < mt ? tok : 0)) * pg_mm_row_bytes(nb) + (size_t)pl * nb * 32 + (ch & 1) * 16;
+        g_src[q] = digits + row_of(tok < mt ? tok : 0) * pg_mm_row_bytes(nb) + (size_t)pl * nb * 32 + (ch & 1) * 16;
     }
-    const size_t x_at = (size_t)(t0 + (lane < mt ? lane : 0)) * nbp;
+    const size_t x_at = row_of(lane < mt ? lane : 0) * nbp;
 
     const int rot = cnt > 0 ? (int)((wg * 5u) % (unsigned)cnt) : 0;
     auto issue = [&](auto slot, int t) {
@@ -1059,7 +1125,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4)))
         const int at = 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
         const int token = ROWS ? l & 31 : at, row = n0 + (ROWS ? at : l & 31);
         if (token < mt && row < n_out) {
-            const size_t o = (size_t)(t0 + token) * n_out + row;
+            size_t o = (size_t)(t0 + token) * n_out + row;
+            if constexpr (EXPERTS) o = (size_t)list[token] * n_out + row;
             y[o] = res ? res[o] + sum : sum;
         }
     }
@@ -1279,6 +1346,76 @@ static pg_status launch_ktile(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_
     return pg_fail(PG_EUNSUPPORTED, "gguf (rows in tiles, one launch): no kernel of %d tokens, %d wavefronts", sh.mt, sh.nw);
 }
 
+// The experts' products of a MoE layer as tiles of 8 or 16 tokens of gguf_ktile_kernel (*mt tokens, *nw wavefronts a workgroup) where the two
+// together are estimated below 0.93 of gguf_mm_kernel's: little work, whose K chunks, tail tiles and planes to be added are what costs
+// there.  Both estimates count the expected tiles and the weights read; terms: rounds of workgroups, a wavefront's (here) or workgroup's
+// (there) walk of K, what the fullest CU loads, its tokens' share of the arithmetic, and there the planes.  Fitted to 890 layers (2 to
+// 256 tokens, 4 to 16 experts, 512 to 3072 x 1024 to 16384): 6 % mean error of each.  8.5 % less time over all of them (the best choice
+// each time: 10 %), 13 to 20 % up to 16 tokens; the worst picks 3 to 4 % over.  us, before : now: 4 tokens, 2 of 8 experts of 2048 x 4096
+// (Q8_0) 44.3 : 35.4, 26, 2 of 4 of 1568 x 1696 34.7 : 31.9.
+bool pg_gguf_experts_tiles(const pg_ctx *ctx, int ggml_type, size_t T, size_t E, size_t top_k, size_t d, size_t ffn, int *mt, int *nw) {
+    const size_t P = T * top_k, n_of[2] = {2 * ffn, d}, k_of[2] = {d, ffn};
+    if (d > 32768 || ffn > 32768 || P > 65535) return false;
+    const bool q8 = ggml_type == PG_GGML_Q8_0;
+    const double cus = (double)ctx->num_cu, per_expert = (double)P / (double)E;
+    const double weights = pg_moe_expected_tiles(T, E, top_k, (int)T) * 3.0 * (double)(d * ffn) * (q8 ? 34.0 / 32 : 18.0 / 32);
+    const double common = 17.2 + 13.2e-6 * (double)P * (double)(d + ffn) + 0.066e-6 * weights;
+    auto half = [](double v) { return v < 1.0 ? 1.0 : 0.5 * (v + ceil(v)); };  // (the last round is rarely full)
+    const double heavy = per_expert > 16.0 ? 2.0 : 1.0 + 0.5 * (1.0 + erf((per_expert - 14.0) / 5.0));
+    double there = common;
+    for (int i = 0; i < 2; ++i) {
+        int chunk = 0;
+        const int ks = pg_gguf_mm_splitk(ctx, i ? d : pg_mm_pair_rows(ffn), k_of[i], E, i ? P : T, true, &chunk);
+        const double wgs = pg_moe_expected_tiles(T, E, top_k, 32) * (double)((n_of[i] + 127) / 128 * ks), cu = std::max(1.0, wgs / cus);
+        const double stages = (double)((std::min<size_t>(chunk, k_of[i] / 32) + 3) / 4);
+        there += half(wgs / (3.0 * cus)) * (3.29 + 0.502 * stages) + cu * stages * ((q8 ? 0.0927 : 0.0463) + 0.0587 * heavy);
+        if (ks > 1) there += 0.78e-6 * (double)ks * (double)P * (double)n_of[i];
+    }
+    static constexpr ktile_shape SHAPES[] = {{8, 4, 1.32}, {16, 4, 1.27}};
+    double best = 1e300;
+    for (const ktile_shape &s : SHAPES) {
+        const size_t unit = ktile_unit(ggml_type, s.mt);
+        const double per_cu = (double)std::max<size_t>(1, std::min<size_t>((160u << 10) / ((size_t)s.nw * 2 * unit), 16 / s.nw));
+        double us = common + 0.005e-6 * weights;
+        for (int i = 0; i < 2; ++i) {
+            const size_t units = (k_of[i] / 32 + 3) / 4;
+            const double wgs = pg_moe_expected_tiles(T, E, top_k, s.mt) * (double)((n_of[i] + 31) / 32);
+            us += s.factor * (half(wgs / (cus * per_cu)) * (0.7 + 0.302 * (double)((units + s.nw - 1) / s.nw)) +
+                              half(wgs / cus) * (double)units * (3.53e-6 * (double)unit + 0.00187 * s.mt));
+        }
+        if (us < best) {
+            best = us;
+            *mt = s.mt;
+            *nw = s.nw;
+        }
+    }
+    return best < 0.93 * there;
+}
+
+pg_status pg_launch_gguf_experts_tiles(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const pg_mm_group &grp, size_t P, int mt, int nw,
+                                       const pg_mmdigits &md, float *y) {
+    const int nb = (int)(k_in / 32), nbp = (int)pg_round_up(nb, 4), tensors = grp.nseg < 0 ? 2 : 1;
+    const bool q8 = ggml_type == PG_GGML_Q8_0, two = tensors == 2;
+    const ktile_experts ex = {{grp.qs_table, two ? grp.qs_table2 : nullptr}, {grp.d_table, two ? grp.d_table2 : nullptr}, {y, two ? grp.out2 : nullptr},
+                              grp.lists, grp.counts, grp.list_stride, grp.x_row_div, grp.num_experts, (int)n_out, (int)((n_out + 31) / 32)};
+    const size_t gy = expert_tiles_bound(grp.num_experts, grp.list_stride, P, mt);
+    if (!grp.counts || !grp.tiled || gy > 65535) return pg_fail(PG_EINVAL, "gguf experts (tiles): %zu token tiles", gy);
+    const dim3 grid((unsigned)(ex.wgs1 * tensors), (unsigned)gy);
+#define PG_KE(QTT, MTT, NWW)                                                                                                   \
+    if (q8 == (QTT == 8) && mt == MTT && nw == NWW) {                                                                          \
+        auto kern = gguf_ktile_kernel<QTT, MTT, NWW, false, ktile_experts>;                                                    \
+        const size_t lds = (size_t)NWW * 2 * KTCfg<QTT, MTT, false>::UNIT;                                                     \
+        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
+        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_experts_tile" : "gguf_q4_0_experts_tile", kern, grid, dim3(64 * NWW), lds, ex, nb, nbp, 0, \
+                         (const int8_t *)md.digits, (const float *)md.xs, 1, 0);                                               \
+    }
+#define PG_KES(QTT) PG_KE(QTT, 8, 4) PG_KE(QTT, 16, 4)
+    PG_KES(8) PG_KES(4)
+#undef PG_KES
+#undef PG_KE
+    return pg_fail(PG_EUNSUPPORTED, "gguf experts (tiles): no kernel of %d tokens, %d wavefronts", mt, nw);
+}
+
 pg_status pg_launch_gguf_one_launch(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_gguf_tensor *const *w, float *const *y, int count,
                                     size_t m, const pg_mmdigits &md, const float *residual) {
     if (count < 1 || count > 3) return pg_fail(PG_EINVAL, "gguf (few rows in one launch): %d tensors (1 .. 3)", count);
@@ -1315,7 +1452,7 @@ pg_status pg_launch_gguf_mm(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_i
     const int nb = (int)(k_in / 32), nbp = (int)pg_round_up(nb, 4);
     const size_t experts = grp.counts ? (size_t)grp.num_experts : 1;
     int chunk = 0;
-    const size_t gy = experts * (size_t)grp.tiles_per_expert;
+    size_t gy = experts * (size_t)grp.tiles_per_expert;
     // token tiles that certainly hold work: all of them without expert lists, one per expert with
     bool by_xcd = false;
     const bool second = grp.nseg < 0;
@@ -1325,6 +1462,7 @@ pg_status pg_launch_gguf_mm(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_i
     if (grp.nseg > 0 && ((ks > 1 && !keep_parts) || grp.counts || !grp.tiled))
         return pg_fail(PG_EINVAL, "gguf_mm: several tensors in one launch leave their K chunks unsummed, take no expert lists and read tile-major copies");
     if (gy > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_mm: too many token tiles");
+    if (grp.counts) gy = expert_tiles_bound(experts, grp.list_stride, total_pairs, 32);
     dim3 grid(grid_for(n_out, 128) * (second ? 2 : 1), (unsigned)gy, (unsigned)ks);
     pg_mm_group g2 = grp;
     g2.remap_rg = g2.remap_tiles = 0;

@@ -448,6 +448,11 @@ int pg_gguf_mm_splitk(const pg_ctx *ctx, size_t n_out, size_t k_in, size_t group
 pg_status pg_launch_gguf_mm(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const uint8_t *qs,
                             const uint16_t *d, const pg_mm_group &grp, size_t total_pairs, const pg_mmdigits &md,
                             float *y, float *part, bool keep_parts = false);  // keep_parts: the K chunks' planes are left in `part` unsummed
+bool pg_gguf_experts_tiles(const pg_ctx *ctx, int ggml_type, size_t T, size_t E, size_t top_k, size_t d, size_t ffn, int *mt, int *nw);
+pg_status pg_launch_gguf_experts_tiles(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const pg_mm_group &grp, size_t P, int mt, int nw,
+                                       const pg_mmdigits &md, float *y);
+// Tiles of `slots` pairs that T tokens choosing top_k of E experts are expected to make (their numbers as binomials).
+double pg_moe_expected_tiles(size_t T, size_t E, size_t top_k, int slots);
 // y[i] = part[0][i] + ... + part[ks - 1][i] (planes `stride` floats apart), in that order.
 // Huffman pieces shared by the coded weights and the coded KV cache (pg_huffman.hip).
 struct pg_huffman_dev_stream {

@@ -260,6 +260,17 @@ __global__ void combine_kernel(const float *__restrict__ yb, int planes, size_t 
 
 }  // namespace
 
+double pg_moe_expected_tiles(size_t T, size_t E, size_t top_k, int slots) {
+    const double p = (double)top_k / (double)E, mu = (double)T * p, sd = sqrt(std::max(mu * (1.0 - p), 1e-9));
+    double tiles = 1.0 - pow(1.0 - p, (double)T);
+    for (size_t j = 1; j * slots < T; ++j) {
+        const double more = 0.5 * erfc(((double)(j * slots) + 0.5 - mu) / (sd * 1.41421356));
+        if (more < 1e-4) break;
+        tiles += more;
+    }
+    return tiles * (double)E;
+}
+
 // A table of device pointers (an expert set's planes) in a device buffer kept with the context, one per distinct
 // table; uploaded (blocking: the source is the caller's stack frame) only on a table's first use.
 pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n, const void ***dev_tab) {
@@ -364,8 +375,10 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     // Arena layout.
     // (K chunks' planes stay apart: the launch that reads a product adds them.)
     const size_t pair_rows = pg_mm_pair_rows(ffn);
-    const int ks_up = up_stream ? 1 : pg_gguf_mm_splitk(ctx, pair_rows, d, E, T, true, nullptr);
-    const int ks_down = down_stream ? 1 : pg_gguf_mm_splitk(ctx, d, ffn, E, P, true, nullptr);
+    int mt = 0, nw = 0;
+    const bool as_tiles = !up_stream && !down_stream && pg_gguf_experts_tiles(ctx, type, T, E, top_k, d, ffn, &mt, &nw);
+    const int ks_up = up_stream || as_tiles ? 1 : pg_gguf_mm_splitk(ctx, pair_rows, d, E, T, true, nullptr);
+    const int ks_down = down_stream || as_tiles ? 1 : pg_gguf_mm_splitk(ctx, d, ffn, E, P, true, nullptr);
     const size_t sz_idx = pg_round_up(P * sizeof(int), 256);
     const size_t sz_p = pg_round_up(P * sizeof(float), 256);
     const size_t sz_lists = pg_round_up(E * T * sizeof(int), 256), sz_counts = pg_round_up(E * sizeof(int), 256);
@@ -426,7 +439,8 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
         gg.qs_table2 = table(2);
         gg.d_table2 = dtable(3);
         gg.out2 = u;
-        PG_TRY(pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xd, g, g, true));
+        PG_TRY(as_tiles ? pg_launch_gguf_experts_tiles(ctx, type, ffn, d, gg, P, mt, nw, xd, g)
+                        : pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xd, g, g, true));
     }
     if (down_stream) {
         PG_TRY(pg_launch(ctx, "moe_act_mul", act_mul_kernel, dim3(grid_for(P * ffn, 256)), dim3(256), 0, g, u, P * ffn, act, h));
@@ -442,7 +456,8 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
         PG_TRY(pg_launch(ctx, "moe_act_mm_digits", kern, dim3(grid_for(nb, 32), (unsigned)P), dim3(256), 0, (const float *)g, (const float *)u,
                          ks_up, P * ffn, act, nb, (int)pg_round_up(nb, 4), hd.digits, hd.xs));
         const pg_mm_group gd = {(int)E, table(4), dtable(5), lists, counts, (int)T, tiles, (int)T, 1, 0, 0, 1};
-        PG_TRY(pg_launch_gguf_mm(ctx, type, d, ffn, nullptr, nullptr, gd, P, hd, yb, yb, true));
+        PG_TRY(as_tiles ? pg_launch_gguf_experts_tiles(ctx, type, d, ffn, gd, P, mt, nw, hd, yb)
+                        : pg_launch_gguf_mm(ctx, type, d, ffn, nullptr, nullptr, gd, P, hd, yb, yb, true));
     }
     return pg_launch(ctx, "moe_combine", combine_kernel, dim3(grid_for(T * d, 256)), dim3(256), 0, (const float *)yb, ks_down, P * d,
                      (const float *)topk_p, (int)T, (int)d, (int)top_k, shared_dev, out_dev);

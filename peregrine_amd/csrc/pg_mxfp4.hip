@@ -1114,16 +1114,6 @@ struct mt_shape { int tb, ra, nw; };
 struct mt_cost { mt_shape s; double chunk, wg; };
 constexpr mt_cost MT_COSTS[] = {{{1, 1, 8}, 0.112, 0.542}, {{2, 1, 8}, 0.128, 0.807}, {{2, 2, 8}, 0.059, 1.192}, {{2, 4, 8}, 0.404, 1.238},
                                 {{2, 4, 4}, 0.784, 0.528}, {{4, 4, 8}, 0.414, 1.9}};
-double expected_tiles(size_t T, size_t E, size_t top_k, int slots) {
-    const double p = (double)top_k / (double)E, mu = (double)T * p, sd = sqrt(std::max(mu * (1.0 - p), 1e-9));
-    double tiles = 1.0 - pow(1.0 - p, (double)T);
-    for (size_t j = 1; j * slots < T; ++j) {
-        const double more = 0.5 * erfc(((double)(j * slots) + 0.5 - mu) / (sd * 1.41421356));
-        if (more < 1e-4) break;
-        tiles += more;
-    }
-    return tiles * (double)E;
-}
 void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const size_t (&n_out)[2], const int (&ncp)[2], mt_shape (&out)[2]) {
     const size_t P = T * top_k, cus = (size_t)ctx->num_cu;
     if (P < 12 * E) {
@@ -1138,7 +1128,7 @@ void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const siz
     }
     double best = 1e300;
     for (int tb = 1; tb <= 4; tb *= 2) {
-        const double tiles = expected_tiles(T, E, top_k, 16 * tb);
+        const double tiles = pg_moe_expected_tiles(T, E, top_k, 16 * tb);
         const double live = tb == 1 ? 1.0 : 0.4 + 0.6 * std::min(1.0, ((double)P / 16.0 + 0.5 * (double)E) / (tiles * tb));
         const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));
         mt_shape pick[2] = {};

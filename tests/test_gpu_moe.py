@@ -345,3 +345,28 @@ def test_moe_routing_in_one_launch_and_split_products(ctx, orc, T, E, top_k, d, 
     again = ex.forward_routed(x[keep], idx, prob).reshape(-1, d)
     for t in range(again.shape[0]):
         H.assert_close_rel(again[t], got[keep][t], 1e-4, f"the routing handed in, row {t}")
+
+
+@pytest.mark.parametrize("T,E,top_k,d,ffn,typ", [
+    (2, 4, 1, 512, 512, 8), (8, 2, 2, 544, 1056, 2), (9, 2, 2, 544, 1056, 8), (17, 3, 2, 608, 992, 2),   # tiles of 8 and 16 pairs and past them
+    (33, 5, 2, 1024, 544, 8), (64, 1, 1, 512, 1024, 8), (65, 70, 2, 512, 544, 2), (130, 130, 1, 512, 512, 8),  # past 64 and 128 experts
+])
+def test_moe_tiles_of_all_experts(ctx, orc, T, E, top_k, d, ffn, typ):
+    """Products over tiles found from the experts' counts: every token at the first experts, at the last ones, and spread;
+    a K whose units of four blocks leave a remainder, rows past the last tile of 32 and of 128."""
+    from peregrine_amd import gguf, moe
+    distinct = min(E, 3)                       # (experts repeat: packing 130 of them would take minutes)
+    raws = build(orc, 90 + E, d, ffn, distinct, typ)
+    x = orc.rng_normal(T, T * d).reshape(T, d)
+    spread = orc.rng_normal(T + 1, T * E).reshape(T, E)
+    ramp = np.tile(np.linspace(0.0, 3.0, E, dtype=np.float32), (T, 1))
+    mk = lambda rs, n_out, k_in: (lambda ws: [ws[e % distinct] for e in range(E)])([gguf.GgufWeight(r, typ, n_out, k_in, ctx) for r in rs])
+    ex = moe.MoEExperts(mk(raws[0], ffn, d), mk(raws[1], ffn, d), mk(raws[2], d, ffn), top_k, moe.SILU, ctx)
+    full = [[r[e % distinct] for e in range(E)] for r in raws]
+    for name, logits in (("spread", spread), ("last", ramp), ("first", -ramp)):
+        say(f"moe tiles T={T} E={E} top_k={top_k} typ={typ} {name}")
+        logits = np.ascontiguousarray(logits, np.float32)
+        got = ex.forward(x, logits).reshape(T, d)
+        want, _, _ = orc.moe_ffn(x.reshape(-1), T, d, ffn, E, top_k, logits, *full, typ, moe.SILU)
+        for t in range(T):
+            H.assert_close_rel(got[t], want[t], MOE_RTOL, f"{name}, token {t}")
