@@ -491,9 +491,16 @@ pg_status pg_launch_mxfp4_rows(pg_ctx *ctx, const float *x_dev, size_t m, const 
 // MoE pieces shared by the block-tensor experts (pg_moe.hip) and the MXFP4 experts (pg_mxfp4.hip).
 constexpr int PG_MOE_MAX_EXPERTS = 256;
 pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n, const void ***dev_tab);
+struct pg_moe_digits {  // the first product's activation rows, to be written as digits beside the routing
+    const float *x;
+    size_t k;
+    int ggml_type;
+    const pg_mmdigits *mm;     // one of the two
+    const pg_xdigits *stream;
+};
 pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, const int *idx_dev, const float *weight_dev, size_t T,
                                 size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts,
-                                int *goff, int tile);
+                                int *goff, int tile, const pg_moe_digits *dig = nullptr);
 struct pg_mxfp4_tiles_plan {
     int ra, tb;            // groups of 16 weight rows per wavefront, groups of 16 tokens per workgroup
     int ks, cps;           // runs of K and chunks per run

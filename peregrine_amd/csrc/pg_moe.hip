@@ -49,18 +49,38 @@ __global__ void route_topk_kernel(const float *__restrict__ logits, int T, int E
 // workgroup while the routing is small: as launches of their own they are the launch and little else (copy, lists and
 // offsets of 20 tokens over 32 experts 13.8 us, 4.8 here; softmax, top-k and lists of 64 over 8 11.0, 4.8 here).  The logits pass through
 // LDS (a row per thread, an odd number of words apart) and hold the probabilities afterwards, -1 where taken; the chosen
-// experts stay there as bytes for the lists.  Grid 1; MAX_ROUTE_LDS bytes at most.
+// experts stay there as bytes for the lists.  MAX_ROUTE_LDS bytes at most.
+// DIG: the further workgroups write the activation rows' digits for the first product, 1 / 2 = byte planes of Q4_0 / Q8_0
+// (pg_emit_mm_digits), 3 / 4 = those of the streaming product (pg_emit_digits): neither waits for the other, and as a launch of its
+// own the digits' took 4.6 us (a layer of 26 tokens, 2 of 4 experts of 1568 x 1696, Q8_0: 31.9 -> 29.5 us; 4, 2 of 8 of 2048 x 4096: 35.4 -> 33.3).
 constexpr size_t MAX_ROUTE_LDS = 48u << 10;
 __host__ __device__ inline size_t route_row(size_t E) { return E | 1; }
 inline bool route_in_one(size_t T, size_t E, size_t top_k) {
     // (lists: a wavefront of the 16 takes every 16th expert and looks at 64 pairs at a time: 128 such steps, 4 us, at most)
     return T * top_k * E <= (1u << 17) && T * route_row(E) * sizeof(float) + T * top_k <= MAX_ROUTE_LDS;
 }
-template <bool LOGITS>
+struct route_digits {
+    const float *x;
+    int nb, nbp, blocks;  // blocks of 32 a row, the same rounded up to 4, blocks of all rows
+    int8_t *digits;
+    float *xs;
+};
+template <bool LOGITS, int DIG>
 __global__ __launch_bounds__(1024) void route_lists_kernel(const float *__restrict__ logits, const int *__restrict__ idx_in,
                                                            const float *__restrict__ w_in, int T, int E, int top_k,
                                                            int *__restrict__ topk_idx, float *__restrict__ topk_p,
-                                                           int *__restrict__ lists, int *__restrict__ counts, int *__restrict__ goff, int tile) {
+                                                           int *__restrict__ lists, int *__restrict__ counts, int *__restrict__ goff, int tile,
+                                                           const route_digits rd) {
+    if (DIG && blockIdx.x > 0) {
+        const int i = ((int)blockIdx.x - 1) * 128 + (int)(threadIdx.x >> 3), sub = threadIdx.x & 7;
+        if (i >= rd.blocks) return;  // whole 8-thread groups leave together
+        const int row = i / rd.nb, b = i - row * rd.nb;
+        const float4 v = reinterpret_cast<const float4 *>(rd.x + (size_t)i * 32)[sub];
+        const float f[4] = {v.x, v.y, v.z, v.w};
+        if constexpr (DIG == 1 || DIG == 2) pg_emit_mm_digits<DIG == 1>(f, row, b, sub, rd.nb, rd.nbp, rd.digits, rd.xs);
+        else if constexpr (DIG != 0) pg_emit_digits<DIG == 3>(f, row, b, sub, rd.nb, rd.digits, rd.xs);
+        return;
+    }
     extern __shared__ __attribute__((aligned(16))) float prob[];  // [T][route_row(E)] (LOGITS), then the pairs' experts as bytes
     __shared__ int cnt[MAX_EXPERTS];
     const int row = (int)route_row(E), P = T * top_k;
@@ -305,15 +325,32 @@ pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n
 // The routing of T tokens as the expert products want it: topk_idx / topk_p [T * top_k] (from the router's logits,
 // grok1's softmax -> top-k, or a copy of the caller's own choice with out-of-range and repeated experts made
 // harmless), and per expert the (token, k) pairs routed to it in ascending order (lists [E][T], counts [E]).
-// With `goff` also the first of each expert's tiles of `tile` pairs, and their number in goff[E].
+// With `goff` also the first of each expert's tiles of `tile` pairs, and their number in goff[E]; with `dig` the activation rows' digits too.
 pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, const int *idx_dev, const float *weight_dev, size_t T,
-                                size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts, int *goff, int tile) {
+                                size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts, int *goff, int tile,
+                                const pg_moe_digits *dig) {
     if (lists && route_in_one(T, E, top_k)) {
         const size_t lds = (router_logits_dev ? T * route_row(E) * sizeof(float) : 0) + T * top_k;
-        auto *kern = router_logits_dev ? route_lists_kernel<true> : route_lists_kernel<false>;
-        return pg_launch(ctx, "moe_route_lists", kern, dim3(1), dim3(1024), lds, router_logits_dev, idx_dev, weight_dev, (int)T, (int)E,
-                         (int)top_k, topk_idx, topk_p, lists, counts, goff, tile);
+        route_digits rd = {};
+        if (dig) {
+            const int nb = (int)(dig->k / 32);
+            rd = {dig->x, nb, (int)pg_round_up(nb, 4), (int)T * nb, dig->mm ? dig->mm->digits : dig->stream->digits, dig->mm ? dig->mm->xs : dig->stream->xs};
+        }
+        const dim3 grid(1 + (unsigned)((rd.blocks + 127) / 128));
+        auto go = [&](auto *kern) {
+            return pg_launch(ctx, dig ? "moe_route_lists_digits" : "moe_route_lists", kern, grid, dim3(1024), lds, router_logits_dev, idx_dev, weight_dev,
+                             (int)T, (int)E, (int)top_k, topk_idx, topk_p, lists, counts, goff, tile, rd);
+        };
+        const bool nib = dig && dig->ggml_type == PG_GGML_Q4_0, by_logits = router_logits_dev != nullptr;
+        switch (!dig ? 0 : (dig->mm ? 1 : 3) + !nib) {
+            case 0: return by_logits ? go(route_lists_kernel<true, 0>) : go(route_lists_kernel<false, 0>);
+            case 1: return by_logits ? go(route_lists_kernel<true, 1>) : go(route_lists_kernel<false, 1>);
+            case 2: return by_logits ? go(route_lists_kernel<true, 2>) : go(route_lists_kernel<false, 2>);
+            case 3: return by_logits ? go(route_lists_kernel<true, 3>) : go(route_lists_kernel<false, 3>);
+            default: return by_logits ? go(route_lists_kernel<true, 4>) : go(route_lists_kernel<false, 4>);
+        }
     }
+    if (dig) PG_TRY(dig->mm ? pg_launch_x_to_mm_digits(ctx, dig->x, T, dig->k, dig->ggml_type, *dig->mm) : pg_launch_x_to_digits(ctx, dig->x, T, dig->k, dig->ggml_type, *dig->stream));
     if (router_logits_dev)
         PG_TRY(pg_launch(ctx, "moe_route_topk", route_topk_kernel, dim3(grid_for(T, 64)), dim3(64), 0,
                          router_logits_dev, (int)T, (int)E, (int)top_k, topk_idx, topk_p));
@@ -419,28 +456,27 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     const void **tab = nullptr;
     PG_TRY(pg_moe_cached_table(ctx, host_tab, 6 * E, &tab));
 
-    PG_TRY(pg_launch_moe_routing(ctx, router_logits_dev, idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, lists, counts, nullptr, 1));
+    const pg_xdigits xd = pg_xdigits_carve(xd_base, T, d);
+    const pg_mmdigits xm = pg_mmdigits_carve(xd_base, T, d);  // (the one or the other is used)
+    const pg_moe_digits dig = {x_dev, d, type, up_stream ? nullptr : &xm, up_stream ? &xd : nullptr};
+    PG_TRY(pg_launch_moe_routing(ctx, router_logits_dev, idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, lists, counts, nullptr, 1, &dig));
     auto table = [&](int which) { return reinterpret_cast<const uint8_t *const *>(tab + which * E); };
     auto dtable = [&](int which) { return reinterpret_cast<const uint16_t *const *>(tab + which * E); };
     // Each token reaches an expert at most once, so an expert owns at most T pairs.
     const int tiles = (int)((T + 31) / 32);
     if (up_stream) {  // pair p: activation row p / top_k against expert topk_idx[p]
-        const pg_xdigits xd = pg_xdigits_carve(xd_base, T, d);
-        PG_TRY(pg_launch_x_to_digits(ctx, x_dev, T, d, type, xd));
         const pg_gemv_batch bg = {(int)P, table(0), dtable(1), topk_idx, (int)top_k};
         PG_TRY(pg_launch_gguf_gemv(ctx, type, ffn, d, nullptr, nullptr, bg, xd, g));
         const pg_gemv_batch bu = {(int)P, table(2), dtable(3), topk_idx, (int)top_k};
         PG_TRY(pg_launch_gguf_gemv(ctx, type, ffn, d, nullptr, nullptr, bu, xd, u));
     } else {
-        const pg_mmdigits xd = pg_mmdigits_carve(xd_base, T, d);
-        PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, T, d, type, xd));
         pg_mm_group gg = {(int)E, table(0), dtable(1), lists, counts, (int)T, tiles, (int)T, (int)top_k, 0, 0, 1};
         gg.nseg = -1;  // gate and up in one launch
         gg.qs_table2 = table(2);
         gg.d_table2 = dtable(3);
         gg.out2 = u;
-        PG_TRY(as_tiles ? pg_launch_gguf_experts_tiles(ctx, type, ffn, d, gg, P, mt, nw, xd, g)
-                        : pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xd, g, g, true));
+        PG_TRY(as_tiles ? pg_launch_gguf_experts_tiles(ctx, type, ffn, d, gg, P, mt, nw, xm, g)
+                        : pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xm, g, g, true));
     }
     if (down_stream) {
         PG_TRY(pg_launch(ctx, "moe_act_mul", act_mul_kernel, dim3(grid_for(P * ffn, 256)), dim3(256), 0, g, u, P * ffn, act, h));
