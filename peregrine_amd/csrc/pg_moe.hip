@@ -329,7 +329,7 @@ pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n
 pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, const int *idx_dev, const float *weight_dev, size_t T,
                                 size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts, int *goff, int tile,
                                 const pg_moe_digits *dig) {
-    if (lists && route_in_one(T, E, top_k)) {
+    if (route_in_one(T, E, top_k)) {
         const size_t lds = (router_logits_dev ? T * route_row(E) * sizeof(float) : 0) + T * top_k;
         route_digits rd = {};
         if (dig) {
@@ -357,7 +357,6 @@ pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, con
     else
         PG_TRY(pg_launch(ctx, "moe_copy_routing", copy_routing_kernel, dim3(grid_for(T, 64)), dim3(64), 0,
                          idx_dev, weight_dev, (int)T, (int)E, (int)top_k, topk_idx, topk_p));
-    if (!lists) return PG_OK;  // (a caller that works pair by pair)
     PG_TRY(pg_launch(ctx, "moe_expert_lists", expert_lists_kernel, dim3((unsigned)E), dim3(64), 0, (const int *)topk_idx,
                      (int)(T * top_k), (int)T, lists, counts));
     if (!goff) return PG_OK;

@@ -125,27 +125,87 @@ __device__ __forceinline__ void mx_emit_digits(const float (&f)[4], int b, int s
 // LDS while its first weight loads are in flight.  Each wavefront then walks its K slice in batches of
 // MX_U chunks, the next batch requested before the current one is consumed, and the partial tiles of
 // the KS slices and the 5 planes are added through LDS in a fixed order.
-// PAIRS (T = 1): blockIdx.y is a (token, expert) pair of an MoE layer: the weights are the pair's expert's entry of
-// two pointer tables, the activation row is pair / div, the output row the pair.
+// PAIRS 1 and 2 (T = 1): blockIdx.z and y are a token and one of its gridDim.y entries in an MoE layer: the weights are that expert's
+// entry of two pointer tables, the activation row is the token's (by_token) or the pair's, the output row the pair's.  2: mlp1, whose rows 2 i and 2 i + 1
+// with their biases become value i of the output row, their swiglu (made where mlp2 reads its rows instead it is made once for every 64 of
+// mlp2's rows: 16 tokens, 4 of 32 experts of 2880 x 2880 156 -> 210 us).  With the choice of the experts read as the caller made it
+// (mx_routed), a layer of few pairs is three launches where it was five (4 of 32 experts of 2880 x 2880: one token 23.0 -> 18.8 us, two 32.2 -> 31.2, 16 level;
+// 4 of 16 of 1024 x 1024, two tokens 18.6 -> 14.7).
+struct mt_swiglu {
+    const float *const *bias_tab;
+    float alpha, clamp;
+    // biased = h + bias; gate = biased[2i].min(clamp); linear = biased[2i+1].clamp(-clamp, clamp);
+    // out[i] = gate * (1 / (1 + exp(-alpha * gate))) * (linear + 1)   examples/gpt_oss/moe.rs:155-166
+    __device__ __forceinline__ static float of(float g0, float l0, float alpha, float clamp) {
+        const float gate = fminf(g0, clamp);                                     // f32::min: a NaN operand loses
+        const float linear = l0 != l0 ? l0 : fminf(fmaxf(l0, -clamp), clamp);    // f32::clamp keeps NaN
+        const float activated = gate * (1.0f / (1.0f + expf(-alpha * gate)));
+        return activated * (linear + 1.0f);
+    }
+};
 struct mx_pairs {
     const uint8_t *const *qs_tab;
     const uint32_t *const *sc_tab;
-    const int *expert_of;  // [pairs]
-    int div;
+    const int *idx;  // [tokens][top_k], the caller's
+    int *chosen;     // [pairs], written by mlp1 (16 tokens, 4 of 32 experts: 1 us less than finding each again)
+    int experts, by_token;
+    mt_swiglu act;
 };
+// The experts of a token's entries 0 .. k, one after the other: an entry out of range, or one that an entry before it names, stands for
+// the lowest expert not taken yet (copy_routing_kernel's rule).
+struct mx_routed {
+    unsigned long long taken[4] = {0, 0, 0, 0};
+    __device__ __forceinline__ int next(int e, int experts, bool &named) {
+        named = e >= 0 && e < experts;
+        if (named) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+                if (e >> 6 == w) named = !((taken[w] >> (e & 63)) & 1ull);
+        }
+        if (!named) {
+#pragma unroll
+            for (int w = 3; w >= 0; --w)
+                if (~taken[w]) e = 64 * w + __builtin_ctzll(~taken[w]);
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+            if (e >> 6 == w) taken[w] |= 1ull << (e & 63);
+        return e;
+    }
+};
+static_assert(PG_MOE_MAX_EXPERTS <= 256, "mx_routed holds 256 experts");
+// Entry k (up to 63) of a token, by a wavefront: a lane an entry; only where one up to k is out of range or named twice they are walked.
+__device__ __forceinline__ int mx_expert_of_entry(const int *__restrict__ idx, int k, int experts) {
+    const int lane = threadIdx.x & 63, e = idx[lane < k ? lane : k];
+    bool odd = e < 0 || e >= experts;
+    for (int j = 0; j < k; ++j) odd |= lane > j && lane <= k && e == __builtin_amdgcn_readlane(e, j);
+    if (!__ballot(odd)) return __builtin_amdgcn_readlane(e, k);
+    mx_routed taken;
+    int expert = 0;
+    bool named;
+    for (int j = 0; j <= k; ++j) expert = taken.next(__builtin_amdgcn_readlane(e, j), experts, named);
+    return __builtin_amdgcn_readfirstlane(expert);
+}
 
-template <int T, int RG, int NW, bool PAIRS = false>
+template <int T, int RG, int NW, int PAIRS = 0>
 __global__ __launch_bounds__(64 * NW) void mxfp4_rows_kernel(const uint8_t *__restrict__ qs_frag, const uint32_t *__restrict__ sc_frag,
                                                                   const float *__restrict__ x, float *__restrict__ y,
                                                                   int n_out, int nb, int ncp, int m, const mx_pairs pr) {
     static_assert(!PAIRS || T == 1, "a pair is one activation row");
     constexpr int KS = NW / RG, COLS = MX_PLANES * T;
     size_t x_row0 = (size_t)blockIdx.y * T;  // first activation row of this workgroup
+    float bias = 0.0f;
+    const size_t pair = (size_t)blockIdx.z * gridDim.y + blockIdx.y;
     if (PAIRS) {
-        const int expert = pr.expert_of[blockIdx.y];
+        const int expert = PAIRS == 2 ? mx_expert_of_entry(pr.idx + (size_t)blockIdx.z * gridDim.y, blockIdx.y, pr.experts) : pr.chosen[pair];
+        if (PAIRS == 2 && blockIdx.x == 0 && threadIdx.x == 0) pr.chosen[pair] = expert;
+        if (PAIRS == 2) {  // (asked for now: one of the 16 RG rows a thread of the last step)
+            const int row = (int)blockIdx.x * RG * 16 + (int)threadIdx.x % (RG * 16);
+            bias = pr.act.bias_tab[expert][row < n_out ? row : n_out - 1];
+        }
         qs_frag = pr.qs_tab[expert];
         sc_frag = pr.sc_tab[expert];
-        x_row0 = blockIdx.y / (unsigned)pr.div;
+        x_row0 = pr.by_token ? blockIdx.z : pair;
     }
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int kp = ncp * 128, stride = kp + 16;  // plane stride = 16 (mod 256): the 16 columns of a 128-bit read fall into 16 different bank groups
@@ -267,8 +327,11 @@ __global__ __launch_bounds__(64 * NW) void mxfp4_rows_kernel(const uint8_t *__re
 #pragma unroll
             for (int k = 0; k < KS; ++k)
                 sum += part[((size_t)(g * KS + k) * 64 + 16 * (i >> 2) + t * MX_PLANES + j) * 4 + (i & 3)];
-        const size_t row = ((size_t)blockIdx.x * RG + g) * 16 + i, item = (size_t)blockIdx.y * T + t;  // (PAIRS: the pair)
-        if (row < (size_t)n_out && (PAIRS || item < (size_t)m)) y[item * n_out + row] = sum;
+        const size_t row = ((size_t)blockIdx.x * RG + g) * 16 + i, item = PAIRS ? pair : (size_t)blockIdx.y * T + t;
+        if constexpr (PAIRS == 2) {
+            const float v = sum + bias, linear = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false));
+            if (!(row & 1) && row < (size_t)n_out) y[item * (n_out / 2) + row / 2] = mt_swiglu::of(v, linear, pr.act.alpha, pr.act.clamp);
+        } else if (row < (size_t)n_out && (PAIRS || item < (size_t)m)) y[item * n_out + row] = sum;
     }
 }
 
@@ -287,14 +350,14 @@ pg_status launch_rows(pg_ctx *ctx, const pg_gguf_tensor *w, const float *x, floa
                      reinterpret_cast<const uint32_t *>(w->d), x, y, (int)w->n_out, (int)(w->k_in / 32), ncp, (int)m, mx_pairs{});
 }
 
-// One launch for `pairs` (token, expert) pairs: pair p = row p / div of x against expert expert_of[p]; x has x_rows rows.
-template <int RG, int NW>
-pg_status launch_rows_pairs(pg_ctx *ctx, size_t n_out, size_t k_in, const float *x, size_t x_rows, float *y, size_t pairs, int ncp,
+// One launch for `pairs` (token, expert) pairs, top_k a token; x has x_rows rows.
+template <int RG, int NW, int PAIRS>
+pg_status launch_rows_pairs(pg_ctx *ctx, size_t n_out, size_t k_in, const float *x, size_t x_rows, float *y, size_t pairs, size_t top_k, int ncp,
                             const mx_pairs &pr) {
     const size_t lds = mx_lds_bytes(1, ncp, NW);
-    auto kern = mxfp4_rows_kernel<1, RG, NW, true>;
+    auto kern = mxfp4_rows_kernel<1, RG, NW, PAIRS>;
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
-    const dim3 grid(grid_for((n_out + 15) / 16, RG), (unsigned)pairs);
+    const dim3 grid(grid_for((n_out + 15) / 16, RG), (unsigned)top_k, (unsigned)(pairs / top_k));
     return pg_launch(ctx, "mxfp4_rows_pairs", kern, grid, dim3(64 * NW), lds, (const uint8_t *)nullptr, (const uint32_t *)nullptr, x, y,
                      (int)n_out, (int)(k_in / 32), ncp, (int)x_rows, pr);
 }
@@ -369,19 +432,6 @@ __device__ __forceinline__ int mt_expert_of(const mt_gather &g, int gt) {
 // GATHER: the token groups are the experts' slots (mt_gather) instead of the rows in order.
 // SWIGLU: x holds mlp1's outputs, [pairs][2 * 32 nb], and the values are their bias and swiglu, made on the way (a launch
 // and a round trip of the pairs' rows less: 11.4 -> 8.1 us for 80 pairs of 2880).
-struct mt_swiglu {
-    const float *const *bias_tab;
-    float alpha, clamp;
-    // biased = h + bias; gate = biased[2i].min(clamp); linear = biased[2i+1].clamp(-clamp, clamp);
-    // out[i] = gate * (1 / (1 + exp(-alpha * gate))) * (linear + 1)   examples/gpt_oss/moe.rs:155-166
-    __device__ __forceinline__ static float of(float g0, float l0, float alpha, float clamp) {
-        const float gate = fminf(g0, clamp);                                     // f32::min: a NaN operand loses
-        const float linear = l0 != l0 ? l0 : fminf(fmaxf(l0, -clamp), clamp);    // f32::clamp keeps NaN
-        const float activated = gate * (1.0f / (1.0f + expf(-alpha * gate)));
-        return activated * (linear + 1.0f);
-    }
-};
-
 template <bool GATHER, bool SWIGLU = false>
 __global__ __launch_bounds__(256) void mxfp4_planes_kernel(const float *__restrict__ x, int m, int nb, int ncp, int token_groups,
                                                            char *__restrict__ bq, const mt_gather gat, const mt_swiglu act) {
@@ -1070,30 +1120,45 @@ PG_API pg_status pg_mxfp4_expert_forward(pg_ctx *ctx, const pg_mxfp4_expert *e, 
 // in k order.
 namespace {
 
-// biased = h + bias1[expert]; the gpt-oss swiglu (examples/gpt_oss/moe.rs:155-166) per pair
-__global__ __launch_bounds__(256) void mxfp4_moe_swiglu_kernel(const float *__restrict__ h, const float *const *__restrict__ bias_tab,
-                                                               const int *__restrict__ topk_idx, size_t pairs, size_t inter,
-                                                               float alpha, float clamp, float *__restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= pairs * inter) return;
-    const size_t p = i / inter, c = i - p * inter;
-    const float *bias = bias_tab[topk_idx[p]];
-    out[i] = mt_swiglu::of(h[p * 2 * inter + 2 * c] + bias[2 * c], h[p * 2 * inter + 2 * c + 1] + bias[2 * c + 1], alpha, clamp);
-}
 
 // output[t] += weight * (out + mlp2_bias) over the token's experts in the order given  (examples/gpt_oss/moe.rs:104-108, 330-334)
+// out[t] = sum_k weight (y + bias2), k ascending; idx and weight as the caller chose them or already put in order (mx_routed).  CH
+// entries' loads are in flight together.
+template <int CH>
 __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__restrict__ yb, const float *const *__restrict__ bias_tab,
-                                                                const int *__restrict__ topk_idx, const float *__restrict__ topk_p,
-                                                                size_t tokens, size_t hidden, int top_k, float *__restrict__ out) {
+                                                                const int *__restrict__ idx, const float *__restrict__ weight,
+                                                                size_t tokens, size_t hidden, int top_k, int experts, float *__restrict__ out) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= tokens * hidden) return;
     const size_t t = i / hidden, c = i - t * hidden;
+    mx_routed taken;
     float acc = 0.0f;
-    for (int k = 0; k < top_k; ++k) {
-        const size_t p = t * top_k + k;
-        const float result = yb[p * hidden + c] + bias_tab[topk_idx[p]][c];
-        const float prod = topk_p[p] * result;
-        acc = acc + prod;
+    for (int k0 = 0; k0 < top_k; k0 += CH) {
+        int e[CH];
+        float w[CH], v[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const size_t p = t * top_k + (k0 + j < top_k ? k0 + j : top_k - 1);
+            e[j] = idx[p];
+            w[j] = weight[p];
+            v[j] = yb[p * hidden + c];
+        }
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            bool named = true;
+            if (k0 + j < top_k) e[j] = taken.next(e[j], experts, named);
+            else e[j] = e[0];
+            w[j] = named ? w[j] : 0.0f;
+        }
+        float b[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) b[j] = bias_tab[e[j]][c];
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+            if (k0 + j < top_k) {
+                const float result = v[j] + b[j], prod = w[j] * result;
+                acc = acc + prod;
+            }
     }
     out[i] = acc;
 }
@@ -1195,18 +1260,19 @@ bool pairs_faster(size_t T, size_t E, size_t top_k, size_t hidden, size_t inter)
 
 // The same product pair by pair on the decode kernel (few pairs).
 bool pairs_fit(int ncp) { return mx_lds_bytes(1, ncp) <= (160u << 10); }
-pg_status moe_product_pairs(pg_ctx *ctx, const float *src, size_t src_rows, size_t k_in, size_t n_out, size_t pairs, int div,
-                            const void **tab, size_t experts, int which, const int *topk_idx, float *y) {
+template <int PAIRS>
+pg_status moe_product_pairs(pg_ctx *ctx, const float *src, size_t src_rows, size_t k_in, size_t n_out, size_t pairs, int by_token,
+                            const void **tab, size_t experts, int which, const int *idx, int *chosen, size_t top_k, float *y, const mt_swiglu &act) {
     const int ncp = (int)mx_chunks(k_in / 32);
     const mx_pairs pr = {reinterpret_cast<const uint8_t *const *>(tab + (size_t)(2 * which) * experts),
-                         reinterpret_cast<const uint32_t *const *>(tab + (size_t)(2 * which + 1) * experts), topk_idx, div};
+                         reinterpret_cast<const uint32_t *const *>(tab + (size_t)(2 * which + 1) * experts), idx, chosen, (int)experts, by_token, act};
     // as pg_launch_mxfp4_rows chooses: 16 wavefronts on a row group while there is at most one group per CU, else 8
     // on the fewest row groups that keep every workgroup resident at once
     const size_t groups = (n_out + 15) / 16 * pairs, slots = (size_t)ctx->num_cu * 2;
-    if (groups <= (size_t)ctx->num_cu) return launch_rows_pairs<1, 16>(ctx, n_out, k_in, src, src_rows, y, pairs, ncp, pr);
-    if (groups <= slots) return launch_rows_pairs<1, 8>(ctx, n_out, k_in, src, src_rows, y, pairs, ncp, pr);
-    if ((groups + 1) / 2 <= slots) return launch_rows_pairs<2, 8>(ctx, n_out, k_in, src, src_rows, y, pairs, ncp, pr);
-    return launch_rows_pairs<4, 8>(ctx, n_out, k_in, src, src_rows, y, pairs, ncp, pr);
+    if (groups <= (size_t)ctx->num_cu) return launch_rows_pairs<1, 16, PAIRS>(ctx, n_out, k_in, src, src_rows, y, pairs, top_k, ncp, pr);
+    if (groups <= slots) return launch_rows_pairs<1, 8, PAIRS>(ctx, n_out, k_in, src, src_rows, y, pairs, top_k, ncp, pr);
+    if ((groups + 1) / 2 <= slots) return launch_rows_pairs<2, 8, PAIRS>(ctx, n_out, k_in, src, src_rows, y, pairs, top_k, ncp, pr);
+    return launch_rows_pairs<4, 8, PAIRS>(ctx, n_out, k_in, src, src_rows, y, pairs, top_k, ncp, pr);
 }
 
 }  // namespace
@@ -1241,10 +1307,10 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     const size_t sz_idx = pg_round_up(P * sizeof(int), 256), sz_p = pg_round_up(P * sizeof(float), 256);
     const size_t sz_lists = pg_round_up(E * T * sizeof(int), 256), sz_counts = pg_round_up((2 * E + 1) * sizeof(int), 256);
     const size_t sz_rec = pg_round_up(max_tiles * tb * (size_t)std::max(ncp1, ncp2) * MT_RECORD, 256);
-    const size_t sz_h = pg_round_up(P * 2 * inter * sizeof(float), 256), sz_act = by_pairs ? pg_round_up(P * inter * sizeof(float), 256) : 0;
+    const size_t sz_h = pg_round_up(P * 2 * inter * sizeof(float), 256);
     const size_t sz_y = pg_round_up(P * hidden * sizeof(float), 256);
     void *ws = nullptr;
-    PG_TRY(pg_workspace(ctx, sz_idx + sz_p + sz_lists + sz_counts + sz_rec + sz_h + sz_act + sz_y, &ws));
+    PG_TRY(pg_workspace(ctx, sz_idx + sz_p + sz_lists + sz_counts + sz_rec + sz_h + sz_y, &ws));
     char *p = static_cast<char *>(ws);
     int *topk_idx = reinterpret_cast<int *>(p); p += sz_idx;
     float *topk_p = reinterpret_cast<float *>(p); p += sz_p;
@@ -1252,7 +1318,6 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     int *counts = reinterpret_cast<int *>(p), *goff = counts + E; p += sz_counts;
     char *rec = p; p += sz_rec;
     float *h = reinterpret_cast<float *>(p); p += sz_h;
-    float *act = reinterpret_cast<float *>(p); p += sz_act;
     float *yb = reinterpret_cast<float *>(p);
     // [mlp1 codes | mlp1 scales | mlp2 codes | mlp2 scales | bias1 | bias2], E each
     const void *host_tab[6 * PG_MOE_MAX_EXPERTS];
@@ -1263,25 +1328,19 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
     }
     const void **tab = nullptr;
     PG_TRY(pg_moe_cached_table(ctx, host_tab, 6 * E, &tab));
-    PG_TRY(pg_launch_moe_routing(ctx, nullptr, expert_idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, by_pairs ? nullptr : lists, counts,
-                                 goff, 16 * tb));
-    const mt_gather gat = {lists, counts, goff, (int)T, (int)E, tb, 1};
-    if (by_pairs)
-        PG_TRY(moe_product_pairs(ctx, x_dev, T, hidden, 2 * inter, P, (int)top_k, tab, E, 0, topk_idx, h));
-    else
-        PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, shape[0], max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
-    const float *const *bias1 = reinterpret_cast<const float *const *>(tab + 4 * E);
+    const mt_swiglu sw = {reinterpret_cast<const float *const *>(tab + 4 * E), alpha, clamp};
     if (by_pairs) {
-        PG_TRY(pg_launch(ctx, "mxfp4_moe_swiglu", mxfp4_moe_swiglu_kernel, dim3(grid_for(P * inter, 256)), dim3(256), 0, (const float *)h,
-                         bias1, (const int *)topk_idx, P, inter, alpha, clamp, act));
-        PG_TRY(moe_product_pairs(ctx, act, P, inter, hidden, P, 1, tab, E, 1, topk_idx, yb));
+        PG_TRY(moe_product_pairs<2>(ctx, x_dev, T, hidden, 2 * inter, P, 1, tab, E, 0, expert_idx_dev, topk_idx, top_k, h, sw));
+        PG_TRY(moe_product_pairs<1>(ctx, h, P, inter, hidden, P, 0, tab, E, 1, nullptr, topk_idx, top_k, yb, mt_swiglu{}));
     } else {
-        const mt_swiglu sw = {bias1, alpha, clamp};
+        PG_TRY(pg_launch_moe_routing(ctx, nullptr, expert_idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, lists, counts, goff, 16 * tb));
+        const mt_gather gat = {lists, counts, goff, (int)T, (int)E, tb, 1};
+        PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, shape[0], max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
         PG_TRY(moe_product(ctx, h, inter, hidden, shape[1], max_tiles, gat, 1, tab, E, 1, rec, yb, &sw));
     }
-    return pg_launch(ctx, "mxfp4_moe_combine", mxfp4_moe_combine_kernel, dim3(grid_for(T * hidden, 256)), dim3(256), 0, (const float *)yb,
-                     reinterpret_cast<const float *const *>(tab + 5 * E), (const int *)topk_idx, (const float *)topk_p, T, hidden,
-                     (int)top_k, out_dev);
+    return pg_launch(ctx, "mxfp4_moe_combine", top_k <= 2 ? mxfp4_moe_combine_kernel<2> : mxfp4_moe_combine_kernel<4>, dim3(grid_for(T * hidden, 256)), dim3(256), 0, (const float *)yb,
+                     reinterpret_cast<const float *const *>(tab + 5 * E), by_pairs ? expert_idx_dev : (const int *)topk_idx,
+                     by_pairs ? weight_dev : (const float *)topk_p, T, hidden, (int)top_k, (int)E, out_dev);
 }
 
 PG_API pg_status pg_mxfp4_moe_ffn_routed(pg_ctx *ctx, const float *x, size_t T, const int32_t *expert_idx, const float *weight,

@@ -324,3 +324,45 @@ def test_mxfp4_moe_pairs_or_tiles(ctx, orc, hidden, inter, E, top_k, T, pairs):
 def test_mxfp4_moe_tilings(ctx, orc, hidden, inter, E, top_k, T):
     """Every tiling that the estimates choose from, at ragged row groups and last tiles."""
     test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, T)
+
+
+@pytest.mark.parametrize("hidden,inter,E,top_k,T", [(64, 96, 6, 6, 3), (512, 512, 200, 64, 1), (512, 96, 70, 12, 5), (64, 512, 2, 1, 9)])
+def test_mxfp4_moe_pairs_with_entries_that_name_no_expert(ctx, hidden, inter, E, top_k, T):
+    """Entries out of range or named twice count as the lowest free expert with weight 0: the device entry's rows are those of the
+    routing with them replaced so, in every bit, and the caller's entries stay as they were."""
+    import ctypes as C
+    from devbuf import DevBuf
+    from peregrine_amd import _ffi, mxfp4
+    from test_oracle_formats_pins import _mx_expert
+    say(f"mxfp4 moe odd entries hidden={hidden} inter={inter} E={E} top_k={top_k} T={T}")
+    rng = np.random.default_rng(T + E)
+    some = [mxfp4.Mxfp4Expert(hidden, inter, 1.702, 7.0, *_mx_expert(rng, hidden, inter), ctx=ctx) for _ in range(min(E, 4))]
+    tab = (C.c_void_p * E)(*[some[e % len(some)]._h.value for e in range(E)])
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    idx = np.stack([rng.permutation(E)[:top_k] for _ in range(T)]).astype(np.int32)
+    w = rng.uniform(0.2, 1.0, (T, top_k)).astype(np.float32)
+    idx[0, top_k // 2] = -3
+    idx[T // 2, top_k - 1] = E
+    idx[T - 1, top_k - 1] = idx[T - 1, 0]
+    fixed, fw = idx.copy(), w.copy()
+    for t in range(T):
+        taken = set()
+        for k in range(top_k):
+            e = int(fixed[t, k])
+            if e < 0 or e >= E or e in taken:
+                fixed[t, k] = e = min(set(range(E)) - taken)
+                fw[t, k] = 0.0
+            taken.add(e)
+
+    def rows(idx, w):
+        dx, di, dw, dout = DevBuf(ctx, host=x), DevBuf(ctx, host=idx), DevBuf(ctx, host=w), DevBuf(ctx, T * hidden * 4)
+        _ffi.check(_ffi.lib.pg_mxfp4_moe_ffn_routed_dev(ctx.handle, dx.ptr, T, di.ptr, dw.ptr, top_k, C.cast(tab, C.POINTER(C.c_void_p)), E, dout.ptr))
+        ctx.sync()
+        assert (di.to_host(np.int32).reshape(T, top_k) == idx).all()
+        return dout.to_host(np.float32).reshape(T, hidden)
+    ctx.profile_begin()
+    got = rows(idx, w)
+    assert "mxfp4_rows_pairs" in ctx.profile_end()
+    np.testing.assert_array_equal(got, rows(fixed, fw))
+    for ex in some:
+        ex.free()
