@@ -127,10 +127,11 @@ __device__ __forceinline__ void mx_emit_digits(const float (&f)[4], int b, int s
 // the KS slices and the 5 planes are added through LDS in a fixed order.
 // PAIRS 1 and 2 (T = 1): blockIdx.z and y are a token and one of its gridDim.y entries in an MoE layer: the weights are that expert's
 // entry of two pointer tables, the activation row is the token's (by_token) or the pair's, the output row the pair's.  2: mlp1, whose rows 2 i and 2 i + 1
-// with their biases become value i of the output row, their swiglu (made where mlp2 reads its rows instead it is made once for every 64 of
-// mlp2's rows: 16 tokens, 4 of 32 experts of 2880 x 2880 156 -> 210 us).  With the choice of the experts read as the caller made it
-// (mx_routed), a layer of few pairs is three launches where it was five (4 of 32 experts of 2880 x 2880: one token 23.0 -> 18.8 us, two 32.2 -> 31.2, 16 level;
-// 4 of 16 of 1024 x 1024, two tokens 18.6 -> 14.7).
+// with their biases become value i of the output row, their swiglu (made where mlp2
+// reads its rows it is made once for every 64 of mlp2's rows: 5 us more at 64 pairs of 2880 x 2880).  With the choice of the experts read
+// as the caller made it, a layer of few pairs is three launches where it was five (4 of 32 experts of 2880 x 2880: one token 23.0 -> 18.8
+// us, two 32.0 -> 30.9; 16 tokens, with eleven rounds of workgroups that each look at the entries, 156 -> 158; 4 of 16 of 1024 x 1024,
+// two tokens 18.3 -> 14.2; random layers of 1 to 8 tokens 0.77 to 0.85 of the time, 9 to 24 0.94).
 struct mt_swiglu {
     const float *const *bias_tab;
     float alpha, clamp;
