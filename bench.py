@@ -698,14 +698,15 @@ def section_gguf(B, line):
         mm_bytes = n_out * (k_in // 32) * 18 + 4 * m_q * k_in + 4 * m_q * n_out
         t_mm = B.timed(mm_step, B.dsteps, max(args.warmup, 8))
         prof, grids = B.profiled(mm_step, B.dsteps)
-        # up to 8 rows: one matrix-core launch after the digits (gguf_skinny_kernel); more: product over K chunks + their sum
-        k_name = "gguf_q4_0_few_rows_mm" if "gguf_q4_0_few_rows_mm" in prof else "gguf_mm_q4_0"
+        # one matrix-core launch after the digits: up to 8 rows gguf_skinny_kernel, more gguf_ktile_kernel; large products over K chunks + their sum
+        kernels = {"gguf_q4_0_few_rows_mm": "gguf_skinny_kernel<Q4_0>", "gguf_q4_0_rows_tile": "gguf_ktile_kernel<Q4_0>", "gguf_mm_q4_0": "gguf_mm_kernel<Q4_0>"}
+        k_name = next(k for k in kernels if k in prof)
         k_ms = prof[k_name][0]
         entry = {"workload": f"cfg4: M={m_q} Q4_0 dequant-matmul [{m_q}x4096]->[{m_q}x14336], weights read once",
                  "value": round(mm_bytes / (t_mm["ms_per_step"] * 1e-3) / 1e9, 1), "unit": "GB/s", **B.stats(t_mm),
                  "gflops": round(2 * m_q * n_out * k_in / (t_mm["ms_per_step"] * 1e-3) / 1e9, 1),
                  "kernels_ms": {k: round(v[0], 5) for k, v in prof.items()},
-                 "roofline": {"kernel": "gguf_skinny_kernel<Q4_0>" if k_name == "gguf_q4_0_few_rows_mm" else "gguf_mm_kernel<Q4_0>", "bound": "hbm",
+                 "roofline": {"kernel": kernels[k_name], "bound": "hbm",
                               "achieved": round(mm_bytes / (k_ms * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                               "frac": round(mm_bytes / (k_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
                               "traffic": B.traffic_for(k_name, grids),
@@ -980,8 +981,9 @@ def section_moe(B, line):
     hit = int(torch.unique(torch.topk(lg_moe, topk_moe, dim=1).indices).numel())
     t_moe = B.timed(moe_step, 20, 10)  # 5 GB of weights: the first passes also warm the TLBs
     prof, grids = B.profiled(moe_step, 5)
-    mm_launches = prof["gguf_mm_q8_0"][1] / 5  # gate and up together, down
-    mm_total = prof["gguf_mm_q8_0"][0] * mm_launches
+    k_name = "gguf_mm_q8_0" if "gguf_mm_q8_0" in prof else "gguf_q8_0_experts_tile"
+    mm_launches = prof[k_name][1] / 5  # gate and up together, down
+    mm_total = prof[k_name][0] * mm_launches
     line["moe_q8_0"] = {
         "workload": "cfg5: Grok-1-shaped MoE FFN, Q8_0 experts (d 6144, ffn 32768, 8 experts, top-2, 64 tokens, SiLU); "
                     "5.13 GB of expert weights, read once per step",
@@ -992,8 +994,8 @@ def section_moe(B, line):
         "roofline": {"kernel": "gguf_mm_kernel<Q8_0> (gate|up, down)", "bound": "hbm",
                      "achieved": round(3 * E_moe * nblk * 34 / (mm_total * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS,
                      "unit": "GB/s", "frac": round(3 * E_moe * nblk * 34 / (mm_total * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
-                     "traffic": B.traffic_for("gguf_mm_q8_0", grids), "bytes_per_launch": int(3 * E_moe * nblk * 34 / mm_launches),
-                     "avg_launch_ms": round(prof["gguf_mm_q8_0"][0], 5)}}
+                     "traffic": B.traffic_for(k_name, grids), "bytes_per_launch": int(3 * E_moe * nblk * 34 / mm_launches),
+                     "avg_launch_ms": round(prof[k_name][0], 5)}}
     for w3 in experts:
         for h in w3:
             lib.pg_gguf_free(B.h, h)
