@@ -253,7 +253,10 @@ void gqa_attention_halves_kernel(attn_args aa, const char *__restrict__ planes, 
             s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k0, q[0][i], s, 0, 0, 0);
         }
         const int t = t0 + it, k0 = 32 * t;
-        float u = k_unit * s_unit;  // of the raw scores
+        // The raw scores' unit, kept off the ends of f32's range: a hidden score's -inf times 0, or a zero times inf, is NaN.  (Raw scores
+        // are below 2^38: with the smallest unit all that is seen weighs the same, as it does with a smaller one.)
+        float u = k_unit * s_unit;
+        u = aa.scale > 0.f ? __builtin_amdgcn_fmed3f(u, 0x1p-126f, 0x1p126f) : aa.scale < 0.f ? __builtin_amdgcn_fmed3f(u, -0x1p126f, -0x1p-126f) : u;
         if (aa.logit_cap > 0.f || !(aa.scale > 0.f)) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] = aa.logit_cap > 0.f ? aa.logit_cap * tanhf(s[r] * u / aa.logit_cap) : s[r] * u;

@@ -540,6 +540,36 @@ def test_gqa_attention_of_halves_over_a_wide_range(ctx, orc, hd):
         assert (err <= (2.0 ** -18 * sums + 2.0 ** -17) * mag + 2.0 ** -37 * np.abs(v).max()).all(), (err / (mag + 1e-30)).max()
 
 
+@pytest.mark.parametrize("hd,q_mag,k_mag,cap,scale", [
+    (128, 1e-19, 1e-19, None, 0.1), (64, 1e-19, 1e-19, None, 0.1), (128, 1e-30, 1e-6, None, 0.1), (64, 2e-34, 1e-3, None, 0.1), (128, 1e-6, 1e-34, None, 0.1),
+    (128, 1e-40, 1e-40, None, 0.1), (128, 1e-25, 1e-25, 5.0, 0.1), (64, 1e-25, 1e-25, None, -0.1),
+    (128, 1e30, 1e30, None, 0.1), (64, 1e38, 1e20, None, 0.1), (128, 1e30, 1e30, 30.0, 0.1),
+])
+def test_gqa_attention_of_halves_at_the_ends_of_the_range(ctx, orc, hd, q_mag, k_mag, cap, scale):
+    """Rows and keys both so small that their units' product is below f32, or so large that it is above (queries in one half of the
+    head, keys in the other): every score is 0, or too small to weigh anything, and a row is the mean of the values it sees, with the
+    last tile's hidden keys left out.  Bound: the second sum, 29 tiles of 6 steps (2^-16 of the mean of |v|)."""
+    from peregrine_amd import llama
+    say(f"attention of halves, queries of {q_mag}, keys of {k_mag}, cap {cap}, scale {scale}, head size {hd}")
+    nqh, nkvh, seq, n = 16, 4, 400, 900
+    rng = np.random.default_rng(hd + 1)
+    k, v = (rng.standard_normal((nkvh, n, hd)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((nqh, seq, hd)).astype(np.float32)
+    q[..., hd // 2:] = 0.0
+    k[..., :hd // 2] = 0.0
+    if q_mag < 1.0:
+        q, k = q[..., ::-1].copy() + q, k[..., ::-1].copy() + k
+    q, k = np.clip(q, -3, 3) * np.float32(q_mag), np.clip(k, -3, 3) * np.float32(k_mag)
+    cache = llama.StandardKVCache(nkvh, hd, ctx)
+    cache.append(k, v, n)
+    got = np.zeros(seq * nqh * hd, np.float32)
+    ctx.profile_begin()
+    llama.gqa_attention(q, cache, cache, nqh, nkvh, seq, hd, scale, llama.AttentionMask.causal(n - seq), cap, got, ctx)
+    assert "gqa_attention_halves" in ctx.profile_end()
+    want, mag = _attention_f64(np.zeros_like(q), k, v, scale, n - seq)
+    assert (np.abs(got.reshape(want.shape) - want) <= 2.0 ** -16 * mag).all()
+
+
 def test_gqa_attention_of_halves_not_finite(ctx, orc):
     """An infinite value comes out where it is weighted, a NaN of a query in its row, an infinite key in the rows that see it;
     nothing else changes."""
