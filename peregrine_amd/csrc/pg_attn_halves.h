@@ -3,7 +3,9 @@
 //
 // x * 2^e = hi + lo: hi is x * 2^e rounded to f16, lo the remainder rounded to f16, 22 to 24 significant bits for what is not
 // far below the scale.  e brings the largest magnitude of a query row, or of a tile of 32 keys or values, to [2^14, 2^15);
-// probabilities are taken times 2^7.  hi hi + hi lo + lo hi leaves out lo lo, below 2^-24 of the product.  The matrix
+// halves are 2^-39 of that apart: a key or value that is 2^-s of its tile's largest, s > 15, keeps 39 - s bits where f32 keeps 24.
+// Probabilities are taken times 2^7 and end at 2^-32 of the row's largest (2^-30 where a tile's values are up to 4 times smaller than the
+// sums' unit).  hi hi + hi lo + lo hi leaves out lo lo, below 2^-24 of the product.  The matrix
 // instruction sums 16 products a step in f32: a score of 128 terms takes 24 roundings of a running sum where the f32 instruction,
 // two products a step, takes 64, which is what either's error comes from (the launcher's rule has the measured ones).  Three of these take
 // 3/16 of the f32 instructions' time.
@@ -40,6 +42,7 @@ __device__ __forceinline__ void halves(float x, float s, _Float16 &hi, _Float16 
 //   values  step j * (HD / 32) + dt: lane = 32 h + d % 32 of d-tile dt, keys 16 j + 8 (e / 4) + 4 h + e % 4, e = 0 .. 7
 // (the order in which a lane holds its probabilities); the inverse scales (keys, values) behind all planes: [kv heads][tiles][2].
 // Keys past `len` are zero.  Grid (tiles, kv heads).
+constexpr float HALVES_NO_VALUES = 0x1p-126f;  // the inverse scale of a tile of zeros, the least there is
 template <int HD> constexpr int half_unit_bytes() { return 2 * 32 * HD * 2; }
 __host__ __device__ constexpr int halves_lds_bytes(int unit) { return 4 * unit > 4 * 32 * 68 * 4 ? 4 * unit : 4 * 32 * 68 * 4; }
 __host__ __device__ inline size_t half_scales_offset(int unit, size_t nkv, size_t tiles) { return nkv * tiles * 2 * unit; }
@@ -81,7 +84,7 @@ __global__ __launch_bounds__(256) void kv_halves_kernel(const float *__restrict_
     ym = pg_block_max_256(ym, vmax);
     const float ks = half_scale(xm), vs = half_scale(ym);
     if (threadIdx.x == 0)  // (no values: no say in the sums' unit)
-        reinterpret_cast<float2 *>(planes + half_scales_offset(UB, gridDim.y, tiles))[(size_t)kvh * tiles + tile] = float2{1.0f / ks, ym > 0.0f ? 1.0f / vs : 1.17549435e-38f};
+        reinterpret_cast<float2 *>(planes + half_scales_offset(UB, gridDim.y, tiles))[(size_t)kvh * tiles + tile] = float2{1.0f / ks, ym > 0.0f ? 1.0f / vs : HALVES_NO_VALUES};
 #pragma unroll
     for (int f = 0; f < FR; ++f) {
         v8h kh, kl, vh, vl;
@@ -220,7 +223,10 @@ void gqa_attention_halves_kernel(attn_args aa, const char *__restrict__ planes, 
     }
     for (int i = threadIdx.x; i < cnt; i += 256) inv[i] = reinterpret_cast<const float2 *>(planes + half_scales_offset(UB, nkvh, tiles_all))[(size_t)kvh * tiles_all + t0 + i];
     __syncthreads();
-    float unit = inv[0].y;  // of the sums in o: the largest of the tiles' so far
+    // Of the sums in o.  It follows the tiles' own, up at once and down in steps of more than 4, to 2^-64 of the largest at the lowest (o
+    // then stays inside f32): the probabilities, times a tile's unit over this one, keep their halves' bits also behind a tile of
+    // far larger values that a row may not see at all.
+    float unit = inv[0].y, top = unit;
     float m = -INFINITY, l = 0.f;
     v16f o[NDT];
 #pragma unroll
@@ -280,14 +286,17 @@ void gqa_attention_halves_kernel(attn_args aa, const char *__restrict__ planes, 
         mt *= u;
         // The probabilities' reference m follows the maximum in steps of more than HALVES_SLACK only (most tiles raise some row's
         // maximum a little): up to e^5 times 2^7 a probability is a half all the same.
-        if (__any(mt > m + HALVES_SLACK || m == -INFINITY) || v_unit > unit) {
+        const float want = fmaxf(v_unit, top * 0x1p-64f);
+        const bool new_unit = v_unit > unit || (want < 0.25f * unit && v_unit > HALVES_NO_VALUES);
+        if (__any(mt > m + HALVES_SLACK || m == -INFINITY) || new_unit) {
             const float m_new = mt > m + HALVES_SLACK || m == -INFINITY ? fmaxf(m, mt) : m;
             float alpha = m == -INFINITY ? 1.0f : exp2f((m - m_new) * LOG2E);
             l *= alpha;
             m = m_new;
-            if (v_unit > unit) {  // (uniform, powers of two)
-                alpha *= unit / v_unit;
-                unit = v_unit;
+            if (new_unit) {  // (uniform, powers of two)
+                alpha *= unit / want;
+                unit = want;
+                top = fmaxf(top, want);
             }
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)

@@ -499,10 +499,11 @@ def test_gqa_attention_of_halves(ctx, orc, nqh, nkvh, hd, seq_q, length, mask, c
     _attention_case(ctx, orc, nqh, nkvh, hd, seq_q, length, m, cap, 500 + seq_q)
 
 
-def _attention_f64(q, k, v, scale, at):
+def _attention_f64(q, k, v, scale, at, window=1 << 30):
     nqh, seq, _ = q.shape
     g = nqh // k.shape[0]
-    hide = np.arange(k.shape[1])[None, :] > at + np.arange(seq)[:, None]
+    back = at + np.arange(seq)[:, None] - np.arange(k.shape[1])[None, :]
+    hide = (back < 0) | (back > window)
     out, mag = np.empty((seq, nqh, k.shape[2])), np.empty((seq, nqh, k.shape[2]))
     for i in range(nqh):
         s = q[i].astype(np.float64) @ k[i // g].astype(np.float64).T * scale
@@ -538,6 +539,31 @@ def test_gqa_attention_of_halves_over_a_wide_range(ctx, orc, hd):
         err = np.abs(got.reshape(want.shape) - want)
         sums = max(abs(scale) * (np.abs(q[i]).astype(np.float64) @ np.abs(k[i // 4]).astype(np.float64).T).max() for i in range(nqh))
         assert (err <= (2.0 ** -18 * sums + 2.0 ** -17) * mag + 2.0 ** -37 * np.abs(v).max()).all(), (err / (mag + 1e-30)).max()
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("big", [2.0 ** 20, 2.0 ** 40, 2.0 ** 62])
+def test_gqa_attention_of_halves_behind_larger_values(ctx, orc, hd, big):
+    """Rows whose window begins behind tiles of values `big` times larger, which their block of rows walks all the same, and tiles of
+    zeros between: as exact as without them.  Bound as over a wide range, the halves' 2^-37 of the largest value that a row sees."""
+    from peregrine_amd import llama
+    say(f"attention of halves behind values {big} times larger, head size {hd}")
+    nqh, nkvh, seq, n, window = 16, 4, 400, 1000, 200
+    rng = np.random.default_rng(hd + 2)
+    k, v = (rng.standard_normal((nkvh, n, hd)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((nqh, seq, hd)).astype(np.float32)
+    v[:, :416] *= np.float32(big)                 # row t sees positions 400 + t .. 600 + t, its run of four tiles begins at 384
+    v[:, 448:480] = 0.0
+    cache = llama.StandardKVCache(nkvh, hd, ctx)
+    cache.append(k, v, n)
+    got = np.zeros(seq * nqh * hd, np.float32)
+    ctx.profile_begin()
+    llama.gqa_attention(q, cache, cache, nqh, nkvh, seq, hd, hd ** -0.5, llama.AttentionMask.causal_sliding_window(n - seq, window, 0), None, got, ctx)
+    assert "gqa_attention_halves" in ctx.profile_end()
+    want, mag = _attention_f64(q, k, v, hd ** -0.5, n - seq, window)
+    err, mag = np.abs(got.reshape(want.shape) - want)[16:], mag[16:]
+    sums = max(hd ** -0.5 * (np.abs(q[i]).astype(np.float64) @ np.abs(k[i // 4]).astype(np.float64).T).max() for i in range(nqh))
+    assert (err <= (2.0 ** -18 * sums + 2.0 ** -16) * mag + 2.0 ** -37 * np.abs(v[:, 416:]).max()).all(), (err / (mag + 1e-30)).max()
 
 
 @pytest.mark.parametrize("hd,q_mag,k_mag,cap,scale", [
