@@ -18,6 +18,10 @@
  *     locked (the reference's callers are single-threaded: Tensor is
  *     Rc<RefCell>, src/tensor.rs:864); distinct contexts may be used from
  *     distinct threads;
+ *   - a result may lie over the activation rows it is made from in pg_matmul_quantized_dev,
+ *     pg_matmul_quantized_fixed_scratch_dev, pg_matmul_quantized_multi_dev, pg_matmul_dequant_i8_dev
+ *     and pg_gguf_matmul_dev (at few rows a launch more than into a buffer of its own); elsewhere
+ *     outputs and inputs do not overlap unless the function says so;
  *   - the library keeps no host pointer past the return of a call.
  */
 #ifndef PEREGRINE_HIP_H

@@ -1025,11 +1025,19 @@ static pg_status pg_gguf_hmm_rows(pg_ctx *ctx, const float *x_dev, size_t m, con
 pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const pg_gguf_tensor *w,
                               float *y_dev) {
     void *ws = nullptr;
+    // A result over the rows (K = n_out): only routes that are done with the rows before they store, that is, that write them as
+    // digits first.
+    const bool apart = !pg_overlap(x_dev, m * w->k_in * sizeof(float), y_dev, m * w->n_out * sizeof(float));
     if (w->ggml_type == PG_MXFP4) {
         // The MXFP4 kernel is a decode kernel (three rows per pass over the weights).  From 16 rows on (24 for a
         // tensor under 2^25 weights, where the passes are short) the tile kernel on the same instruction takes over:
         // the weights once per 64 rows, the rows as four planes of base-32 digits.
         if (pg_mxfp4_tiles_takes(w, m)) return pg_launch_mxfp4_tiles(ctx, x_dev, m, w, y_dev);
+        if (!apart) {
+            PG_TRY(pg_workspace(ctx, m * w->k_in * sizeof(float), &ws));
+            PG_HIP(hipMemcpyAsync(ws, x_dev, m * w->k_in * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
+            x_dev = static_cast<const float *>(ws);
+        }
         return pg_launch_mxfp4_rows(ctx, x_dev, m, w, y_dev);
     }
     int hks = 1;
@@ -1038,9 +1046,9 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
     // a K of a few blocks needs the streaming kernel's finer fixed point; so do up to seven rows of Q4_1 (its
     // matrix-core route is three launches more than the streaming one: 27 against 19 us at four rows of 4096 ->
     // 14336, 35 against 59 at sixteen) and Q4_1 rows too long for the offset kernel
-    if (m == 1 && pg_gguf_gemv_takes_f32_row(w->ggml_type, w->n_out, w->k_in, x_dev))
+    if (apart && m == 1 && pg_gguf_gemv_takes_f32_row(w->ggml_type, w->n_out, w->k_in, x_dev))
         return pg_launch_gguf_gemv_f32_row(ctx, w->ggml_type, w->n_out, w->k_in, w->qs, w->d, x_dev, y_dev);
-    if (pg_gguf_gemv_takes_few_rows(w->ggml_type, m, w->n_out, w->k_in, x_dev))
+    if (apart && pg_gguf_gemv_takes_few_rows(w->ggml_type, m, w->n_out, w->k_in, x_dev))
         return pg_launch_gguf_gemv_few_rows(ctx, w->n_out, w->k_in, w->qs, w->d, x_dev, m, y_dev);
     const bool q41 = w->ggml_type == PG_GGML_Q4_1;
     if (m == 1 || (q41 && (m < 8 || w->k_in > 32768)) || w->k_in / 32 < PG_MM_MIN_BLOCKS) {
@@ -1059,7 +1067,7 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
     }
     if (pg_gguf_hmm_takes(ctx, w->ggml_type, m, w->n_out, w->k_in, &hks))  // many rows of Q4_0 / Q8_0: the f16 matrix cores
         return pg_gguf_hmm_rows(ctx, x_dev, m, &w, &y_dev, 1, hks);
-    if (q41 && w->k_in <= 32768 && pg_gguf_hmm_takes(ctx, PG_GGML_Q4_0, m, w->n_out, w->k_in, &hks)) {
+    if (apart && q41 && w->k_in <= 32768 && pg_gguf_hmm_takes(ctx, PG_GGML_Q4_0, m, w->n_out, w->k_in, &hks)) {
         // Q4_1 at that size: the first term d sum (q - 8) x as the Q4_0 product on the f16 matrix cores, then the
         // offsets times the rows' block sums (which the digit launch writes beside its planes)
         PG_TRY(pg_gguf_hmm_rows(ctx, x_dev, m, &w, &y_dev, 1, hks));

@@ -110,6 +110,12 @@ struct pg_qtensor {
     size_t k_pad, n_pad;  // multiples of PG_KPAD / PG_NPAD
 };
 
+// Whether two byte ranges share any.
+inline bool pg_overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a_bytes && b_bytes && x < y + b_bytes && y < x + a_bytes;
+}
+
 // GGUF block tensor split into planes at upload:
 //   qs     [n_out, k_in/32, QB] quant bytes (QB = 16 for Q4_0, 32 for Q8_0)
 //   d      [ceil(n_out/8), k_in/32, 8]  f16 block scales, tiled by 8 weight rows

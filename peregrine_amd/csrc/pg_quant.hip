@@ -559,8 +559,12 @@ constexpr size_t PG_GEMV_MAX_M = 4;
 // nothing is allocated and a request that does not fit is an error.
 static pg_status matmul_quantized_on(pg_ctx *ctx, const float *a_dev, size_t m, size_t k, const pg_qtensor *w,
                                      float *out_dev, int32_t *acc_dev, void *fixed, size_t fixed_cap, bool remote = false) {
-    if (!acc_dev && !remote && pg_gemm_w8a8_takes_f32_rows(ctx, &w, 1, m)) return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, &w, &out_dev, 1, m);
-    if (pg_gemv_w8a8_takes_f32_row(w, m, k, a_dev)) return pg_launch_gemv_w8a8_f32_row(ctx, a_dev, k, w, out_dev, acc_dev);
+    // (the two whose workgroups read f32 rows while others store: only where the result lies apart from them)
+    const size_t a_span = m * k * sizeof(float), out_span = m * w->cols * sizeof(float);
+    const bool apart = !pg_overlap(a_dev, a_span, out_dev, out_span) && (!acc_dev || !pg_overlap(a_dev, a_span, acc_dev, out_span));
+    if (apart && !acc_dev && !remote && pg_gemm_w8a8_takes_f32_rows(ctx, &w, 1, m))
+        return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, &w, &out_dev, 1, m);
+    if (apart && pg_gemv_w8a8_takes_f32_row(w, m, k, a_dev)) return pg_launch_gemv_w8a8_f32_row(ctx, a_dev, k, w, out_dev, acc_dev);
     const size_t m_pad = pg_round_up(m, PG_MPAD);
     const size_t a_bytes = m_pad * w->k_pad;
     // 33 .. 256 rows that the few-row kernel leaves: split-K product with i32 partial planes
@@ -667,11 +671,13 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     if (m == 0) return PG_OK;
     PG_CHECK_ARG(a_dev != nullptr, "pg_matmul_quantized_multi: null pointer");
     PG_CHECK_ARG(m < (1ull << 24), "pg_matmul_quantized_multi: m = %zu too large", m);
-    bool one_row_group = m == 1 && count > 1;
+    bool apart = true;  // an output over the rows: they are quantised before any product stores
+    for (size_t i = 0; i < count; ++i) apart = apart && !pg_overlap(a_dev, m * k * sizeof(float), out_dev[i], m * w[i]->cols * sizeof(float));
+    bool one_row_group = apart && m == 1 && count > 1;
     for (size_t i = 0; i < count && one_row_group; ++i) one_row_group = pg_gemv_w8a8_takes_f32_row(w[i], m, k, a_dev);
     if (one_row_group)  // one token: every weight's rows in one streaming launch that quantises the row itself
         return pg_launch_gemv_w8a8_f32_row_group(ctx, a_dev, k, w, out_dev, (int)count, nullptr);
-    if (count > 1 && pg_gemm_w8a8_takes_f32_rows(ctx, w, (int)count, m)) return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, w, out_dev, (int)count, m);
+    if (apart && count > 1 && pg_gemm_w8a8_takes_f32_rows(ctx, w, (int)count, m)) return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, w, out_dev, (int)count, m);
     if (count > 1 && pg_gemm_w8a8_takes_skinny(ctx, w, (int)count, m)) {  // 2 .. 512 rows: quantised once, then the weights side by side in one launch
         const size_t k_pad = w[0]->k_pad, m_pad = pg_round_up(m, PG_MPAD), a_bytes = m_pad * k_pad;
         void *ws = nullptr;
@@ -681,11 +687,8 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
         PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, k_pad, a_scales));
         return pg_launch_gemm_w8a8_skinny_group(ctx, a_i8, k_pad, a_scales, w, out_dev, (int)count, m, nullptr);  // one launch for all
     }
-    // one weight (or one row): the single product picks its own route (GEMV, split K)
-    if (count == 1 || m <= 32) {
-        for (size_t i = 0; i < count; ++i) PG_TRY(pg_matmul_quantized_dev(ctx, a_dev, m, k, w[i], out_dev[i], nullptr));
-        return PG_OK;
-    }
+    // one weight: the single product picks its own route (GEMV, split K)
+    if (count == 1) return pg_matmul_quantized_dev(ctx, a_dev, m, k, w[0], out_dev[0], nullptr);
     const size_t k_pad = w[0]->k_pad, m_pad = pg_round_up(m, PG_MPAD);
     const size_t a_bytes = m_pad * k_pad;
     void *ws = nullptr;
@@ -693,6 +696,10 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     int8_t *a_i8 = static_cast<int8_t *>(ws);
     float *a_scales = reinterpret_cast<float *>(a_i8 + a_bytes);
     PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, k_pad, a_scales));
+    if (m <= PG_GEMV_MAX_M) {
+        for (size_t i = 0; i < count; ++i) PG_TRY(pg_launch_gemv_w8a8(ctx, a_i8, k_pad, a_scales, w[i], m, out_dev[i], nullptr));
+        return PG_OK;
+    }
     // Weights that fill the chip with 256x256 tiles on their own run on their own (measured: gate and up
     // as two launches 2 x 112 us, as one launch of 896 tiles 242 us: the rounds that leave CUs idle run
     // faster); the narrow ones (q, k, v) share one launch, where k and v alone would leave most CUs idle.

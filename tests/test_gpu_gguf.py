@@ -451,3 +451,31 @@ def test_gguf_rows_in_tiles(ctx, orc, n_out, k_in, m, typ):
     assert (err <= 0).all(), (np.unravel_index(err.argmax(), err.shape), err.max())
     assert not g[m // 2].any()
     gw.free()
+
+
+@pytest.mark.parametrize("kind,m,k,forced", [
+    ("q4_0", 1, 1024, 0), ("q4_0", 1, 4096, 0), ("q4_0", 2, 2048, 0), ("q4_0", 3, 1024, 0), ("q8_0", 1, 1024, 0), ("q8_0", 5, 1024, 0), ("q4_1", 1, 1024, 0),
+    ("q4_1", 12, 1024, 0), ("q4_0", 40, 1024, 0), ("q8_0", 200, 1024, 0), ("q4_0", 40, 1024, 1), ("q8_0", 40, 1024, 1), ("q4_1", 40, 1024, 1),
+    ("mxfp4", 1, 1024, 0), ("mxfp4", 4, 2880, 0), ("mxfp4", 30, 1024, 0),
+])
+def test_product_over_its_own_rows(ctx, kind, m, k, forced):
+    """A result over the rows it is made from: the same, up to the digits of another route (each within half the contract), as in a
+    buffer of its own."""
+    from devbuf import DevBuf
+    from peregrine_amd import _ffi, gguf, mxfp4
+    say(f"{kind} over its own rows m={m} k={k} forced={forced}")
+    rng = np.random.default_rng(m + k)
+    if kind == "mxfp4":
+        w = mxfp4.upload(rng.integers(0, 256, k * k // 2, dtype=np.uint8), rng.integers(116, 119, k * k // 32, dtype=np.uint8), k, k, ctx)
+    else:
+        pack, t = {"q4_0": (H.pack_q4_0, gguf.Q4_0), "q4_1": (H.pack_q4_1, gguf.Q4_1), "q8_0": (H.pack_q8_0, gguf.Q8_0)}[kind]
+        w = gguf.GgufWeight(pack((rng.standard_normal(k * k) * 0.02).astype(np.float32)), t, k, k, ctx)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    over, apart = DevBuf(ctx, host=x), DevBuf(ctx, nbytes=4 * m * k)
+    _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, forced))
+    try:
+        _ffi.check(_ffi.lib.pg_gguf_matmul_dev(ctx.handle, over.ptr, m, w._h, apart.ptr))
+        _ffi.check(_ffi.lib.pg_gguf_matmul_dev(ctx.handle, over.ptr, m, w._h, over.ptr))
+    finally:
+        _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 0))
+    H.assert_close_rel(over.to_host(np.float32), apart.to_host(np.float32), RTOL_CONTRACT, kind)

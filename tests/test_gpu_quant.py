@@ -756,3 +756,43 @@ def test_groups_of_rows_bit_exact(ctx, orc, m, k, ns):
     _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, a_dev.ptr, m, k, qts[0]._gpu, outs[0].ptr, acc_dev.ptr))
     assert (bits(outs[0].to_host(np.float32).reshape(m, ns[0])) == bits(wants[0])).all()
     assert (acc_dev.to_host(np.int32).reshape(m, ns[0]) == accs[0].astype(np.int32)).all()
+
+
+@pytest.mark.parametrize("m,k", [(1, 768), (1, 4096), (2, 128), (3, 768), (4, 2048), (5, 768), (8, 1536), (8, 640), (17, 512), (40, 1024), (1, 20000)])
+@pytest.mark.parametrize("shift", [0, 1, -1])
+def test_w8a8_over_its_own_rows_bit_exact(ctx, orc, m, k, shift):
+    """A result over the rows it is made from, whole or one row further on: no workgroup may store before every other has read
+    the rows.  A weight alone, in the fixed scratch, and the first and the last of two over one input."""
+    from devbuf import DevBuf
+    from peregrine_amd import quant, _ffi
+    say(f"W8A8 over its own rows m={m} k={k} shift={shift}")
+    rng = np.random.default_rng(m + 10 * k)
+    n = k if k < 20000 else 3000
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    q = rng.integers(-127, 128, (k, n), dtype=np.int8)
+    scales = rng.uniform(0.5e-3, 2e-3, n).astype(np.float32)
+    qt = quant.QuantizedTensor(q.reshape(-1), None, scales, k, n).to_gpu(ctx)
+    other = quant.QuantizedTensor(np.ascontiguousarray(q[:, ::-1]).reshape(-1), None, scales, k, n).to_gpu(ctx)
+    qa, s = orc.quantize_activations(a, m, k)
+    acc = np.asarray(qa, np.float64).reshape(m, k) @ q.astype(np.float64)
+    want = acc.astype(np.float32) * np.asarray(s, np.float32)[:, None] * scales[None, :]
+    wants = want, acc[:, ::-1].astype(np.float32) * np.asarray(s, np.float32)[:, None] * scales[None, :]
+    L = _ffi.lib
+    tab = lambda v: (C.c_void_p * len(v))(*v)
+
+    def check(call, w):
+        buf = DevBuf(ctx, host=np.concatenate([np.zeros(k, np.float32), a.reshape(-1), np.zeros(k, np.float32)]))
+        aside = DevBuf(ctx, nbytes=4 * m * n)
+        rows = buf.ptr.value + 4 * k
+        _ffi.check(call(C.c_void_p(rows), rows + 4 * k * shift, aside.ptr.value))
+        got = buf.to_host(np.float32)[k + k * shift:][: m * n].reshape(m, n)
+        assert (bits(got) == bits(wants[w])).all()
+        return aside.to_host(np.float32).reshape(m, n)
+
+    check(lambda x, out, _: L.pg_matmul_quantized_dev(ctx.handle, x, m, k, qt._gpu, C.c_void_p(out), None), 0)
+    check(lambda x, out, _: L.pg_matmul_quantized_fixed_scratch_dev(ctx.handle, x, m, k, qt._gpu, C.c_void_p(out)), 0)
+    both = tab([qt._gpu.value, other._gpu.value])
+    aside = check(lambda x, out, at: L.pg_matmul_quantized_multi_dev(ctx.handle, x, m, k, both, 2, tab([out, at])), 0)
+    assert (bits(aside) == bits(wants[1])).all()
+    aside = check(lambda x, out, at: L.pg_matmul_quantized_multi_dev(ctx.handle, x, m, k, both, 2, tab([at, out])), 1)
+    assert (bits(aside) == bits(wants[0])).all()
