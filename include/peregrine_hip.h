@@ -189,9 +189,10 @@ void pg_gguf_free(pg_ctx *ctx, pg_gguf_tensor *t);
 /* The dequantise-then-matmul of models::llama, fused:
  * y [m, n_out] = x [m, k_in] . dequant(w)^T, i.e. Tensor::matmul
  * (src/tensor.rs:1342-1353) applied to the transposed dequantised weight.
- * The first call with m > 1 on a Q4_0 / Q8_0 tensor (and an expert's first pg_moe_ffn) adds a
- * second, tile-major copy of the quant payload to the handle (freed by pg_gguf_free): a
- * handle must not see its first such call from two threads at once. */
+ * The first call with m > 16 (m > 8 from 8192 weight rows on; less where k_in is below 1024 or no
+ * multiple of 256 and the product a large one) on a block tensor, and an expert's first
+ * pg_moe_ffn, adds a second, tile-major copy of the quant payload to the handle (freed by
+ * pg_gguf_free): a handle must not see its first such call from two threads at once. */
 pg_status pg_gguf_matmul(pg_ctx *ctx, const float *x, size_t m, const pg_gguf_tensor *w,
                          float *y);
 pg_status pg_gguf_matmul_dev(pg_ctx *ctx, const float *x_dev, size_t m,
@@ -201,7 +202,7 @@ pg_status pg_gguf_matmul_dev(pg_ctx *ctx, const float *x_dev, size_t m,
  * payload plane (as many bytes again as the payload).  Left alone, the first product that needs the copy makes it:
  * a hipMalloc, a launch and a wait inside a call that is otherwise stream-ordered and allocation-free.
  * pg_gguf_prepare makes now whatever products over up to `max_rows` activation rows of this tensor (alone, in a
- * group, inside a Llama block or as an expert of pg_moe_ffn) will need, as the reference rearranges weights at load
+ * group, inside a Llama block or as an expert of pg_moe_ffn) will need or, up to sixteen, read faster, as the reference rearranges weights at load
  * (load_transposed_weight, src/models/llama/model.rs:243-257); afterwards those calls allocate nothing for the tensor.
  * (The context's workspace still grows at the first call that needs more of it: a caller that captures them in a HIP
  * graph makes one eager call of each shape first.)  max_rows < 2 makes nothing (one-row products read

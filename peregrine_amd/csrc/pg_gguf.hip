@@ -977,6 +977,11 @@ __global__ void tile_weights_kernel(const uint8_t *__restrict__ qs, int n_out, i
 
 static std::mutex g_tiled_mutex;
 
+const uint8_t *pg_gguf_tiled(const pg_gguf_tensor *w) {
+    std::lock_guard<std::mutex> lock(g_tiled_mutex);
+    return w->qs_tiled;
+}
+
 pg_status pg_gguf_ensure_tiled(pg_ctx *ctx, const pg_gguf_tensor *w) {
     // One maker at a time, and the pointer is published only once the copy is complete, so another
     // context, stream or thread that finds it set may read it at once.

@@ -912,7 +912,7 @@ template <int QT, int MT, bool Q41> struct KTCfg {
     static constexpr int W_T = QT == 8 ? 4096 : 2048, OFF_D = W_T, OFF_M = OFF_D + 256, OFF_DG = OFF_M + (Q41 ? 256 : 0);
     static constexpr int OFF_X = OFF_DG + MT * 256, OFF_S = OFF_X + MT * 16, UNIT = OFF_S + (Q41 ? MT * 16 : 0);
 };
-template <int QT, int MT, int NW, bool Q41, typename ARGS = ktile_args<Q41>>
+template <int QT, int MT, int NW, bool Q41, typename ARGS = ktile_args<Q41>, bool UPLOADED = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_ktile_kernel(const ARGS grp, int nb, int nbp, int m,
                                                                 const int8_t *__restrict__ digits, const float *__restrict__ xs, int groups, int wgs) {
     using C = KTCfg<QT, MT, Q41>;
@@ -967,8 +967,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4)))
     char *ring = lds + (size_t)wave * 2 * C::UNIT;
 
     // fill duties of this lane
-    const char *w_src = reinterpret_cast<const char *>(qs) + (size_t)(n0 >> 7) * pg_tiled_group_bytes(nb, QT == 8) +
-                        ((n0 >> 5) & 3) * C::W_T + lane * 16;
+    const char *w_src[UPLOADED ? 2 : 1];  // UPLOADED: of fill q's row (lane / 4 of 16, q odd the second 16), else of the tile-major copy
+    const int w_jb = (lane & 3) ^ ((lane >> 4) & 3);
+#pragma unroll
+    for (int i = 0; i < (UPLOADED ? 2 : 1); ++i) {
+        const int row = n0 + 16 * i + (lane >> 2);
+        w_src[i] = reinterpret_cast<const char *>(qs) +
+                   (UPLOADED ? (size_t)(row < n_out ? row : n_out - 1) * (QT == 8 ? 2 : 1) * nb * 16  // (rows past the end: never stored)
+                             : (size_t)(n0 >> 7) * pg_tiled_group_bytes(nb, QT == 8) + ((n0 >> 5) & 3) * C::W_T + lane * 16);
+    }
     const int ngroups = (n_out + 7) / 8;
     const int dg8 = (n0 >> 3) + (lane >> 4) < ngroups ? (n0 >> 3) + (lane >> 4) : ngroups - 1;
     const size_t d_at = (size_t)dg8 * nb * 16 + (lane & 3) * 4;
@@ -994,7 +1001,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4)))
         auto blk = [&](int j) { return (size_t)(b0 + j < nb ? b0 + j : nb - 1); };  // past the end: a valid block, never added
 #pragma unroll
         for (int q = 0; q < C::W_T / 1024; ++q)
-            __builtin_amdgcn_global_load_lds((gptr_t)(w_src + (size_t)unit * (4 * C::W_T) + q * 1024), (lptr_t)(base + q * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(UPLOADED ? w_src[q & 1] + (blk(w_jb) + (size_t)(q >> 1) * nb) * 16 : w_src[0] + (size_t)unit * (4 * C::W_T) + q * 1024),
+                                             (lptr_t)(base + q * 1024), 16, 0, 0);
         __builtin_amdgcn_global_load_lds((gptr_t)(d_src + blk(d_jb) * 16), (lptr_t)(base + C::OFF_D), 4, 0, 0);
         if constexpr (Q41) __builtin_amdgcn_global_load_lds((gptr_t)(m_src + blk(d_jb) * 16), (lptr_t)(base + C::OFF_M), 4, 0, 0);
 #pragma unroll
@@ -1236,9 +1244,12 @@ int pg_gguf_mm_splitk(const pg_ctx *ctx, size_t n_out, size_t k_in, size_t group
 // Up to 8 rows over a Q4_0 or Q8_0 tensor whose K is a multiple of 256: gguf_skinny_kernel, bound by how many bytes its rings keep
 // in flight (4 x 4096 -> 14336 takes 9.0 us; with its arithmetic switched off 8.6 - 9.1).  From five rows on it is the better one
 // only where a long K meets few columns (us, this one : gguf_ktile_kernel: 7 x 11776 -> 1804 12.7 : 14.8, 8 x 8704 -> 406 10.7 :
-// 12.3; but 6 x 6144 -> 4297 14.1 : 10.5, 8 x 1536 -> 12190 11.5 : 8.1, 7 x 3584 -> 870 10.1 : 8.5).
+// 12.3; but 6 x 6144 -> 4297 14.1 : 10.5, 8 x 1536 -> 12190 11.5 : 8.1, 7 x 3584 -> 870 10.1 : 8.5), and of Q8_0 over a vocabulary
+// (6 x 8192 -> 32768 54.5 : 72.4 from the planes as uploaded, 49.2 : 59.7 from the copy; 5 x 4096 -> 128256 104 : 116 and 99.6 : 98.9).
 static bool skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out, size_t k_in) {
-    return (ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0) && m >= 2 && (m <= 4 || (m <= 8 && k_in >= 6400 && n_out < 16 * (size_t)ctx->num_cu)) &&
+    const size_t cus = (size_t)ctx->num_cu;
+    const bool few_columns = k_in >= 6400 && n_out < 16 * cus, vocabulary = ggml_type == PG_GGML_Q8_0 && n_out > 64 * cus && m * n_out * k_in > 1400000000;
+    return (ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0) && m >= 2 && (m <= 4 || (m <= 8 && (few_columns || vocabulary))) &&
            k_in % 256 == 0 && k_in >= 1024 && n_out >= 1 && n_out < (1u << 30) && k_in < (1u << 24);
 }
 
@@ -1253,6 +1264,10 @@ static bool ktile_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out
     const bool q41 = ggml_type == PG_GGML_Q4_1;
     if (!(ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0 || q41) || m < (q41 ? 8 : 2) || k_in % 32 != 0 || k_in > 32768 || n_out < 1 || n_out >= (1u << 24))
         return false;
+    // Up to eight rows, up to sixteen of fewer than 8192 columns: always, so that no product of so few rows needs the tile-major copy
+    // (launch_ktile).  us over weights with a copy, gguf_mm_kernel : this: Q4_0 8 x 4096 -> 50257 36.7 : 32.9, 16 x 14336 -> 8000
+    // 27.8 : 25.2, Q8_0 7 x 14336 -> 14336 45.1 : 45.1, 16 x 14336 -> 8000 32.2 : 32.6, the worst 8 x 14336 -> 12600 42.8 : 45.0.
+    if (m <= (n_out < 32 * (size_t)ctx->num_cu ? 16u : 8u) && k_in % 256 == 0 && k_in >= 1024) return true;
     if (q41 && m > 896) return false;  // (1216 -> 972, us, before : now: 512 rows 25.4 : 16.8, 700 25.8 : 20.5, 1008 28.5 : 29.1)
     const double g = 1e-9 * (double)m * (double)n_out * (double)k_in * (planes ? 1.5 : 1.0);
     if (k_in < 512 && n_out > 8192) return false;                                        // (all columns, hardly any K to split)
@@ -1309,7 +1324,7 @@ static size_t ktile_unit(int ggml_type, int mt) {
                                      : (mt == 32 ? KTCfg<4, 32, false>::UNIT : mt == 16 ? KTCfg<4, 16, false>::UNIT : KTCfg<4, 8, false>::UNIT);
 }
 static pg_status launch_ktile(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_gguf_tensor *const *w, int count, const pg_skinny_group &grp, int wgs1,
-                              size_t m, const pg_mmdigits &md) {
+                              size_t m, const pg_mmdigits &md, bool uploaded) {
     const int nb = (int)(k_in / 32), nbp = (int)pg_round_up(nb, 4);
     const bool q8 = ggml_type == PG_GGML_Q8_0, q41 = ggml_type == PG_GGML_Q4_1;
     const size_t units = ((size_t)nb + 3) / 4, cus = (size_t)ctx->num_cu;
@@ -1331,7 +1346,8 @@ static pg_status launch_ktile(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_
     const dim3 grid(groups == 1 ? (unsigned)wgs1 : (unsigned)((wgs1 + 7) / 8 * 8 * groups));
 #define PG_KT(QTT, MTT, NWW)                                                                                                   \
     if ((QTT == 8 ? q8 : QTT == 5 ? q41 : !q8 && !q41) && sh.mt == MTT && sh.nw == NWW) {  /* (5 names Q4_1 here) */           \
-        auto kern = gguf_ktile_kernel<QTT == 8 ? 8 : 4, MTT, NWW, QTT == 5>;                                                   \
+        auto kern = uploaded ? gguf_ktile_kernel<QTT == 8 ? 8 : 4, MTT, NWW, QTT == 5, ktile_args<QTT == 5>, true>              \
+                             : gguf_ktile_kernel<QTT == 8 ? 8 : 4, MTT, NWW, QTT == 5>;                                        \
         ktile_args<QTT == 5> args;                                                                                             \
         static_cast<pg_skinny_group &>(args) = grp;                                                                            \
         args.set(w, count, md);                                                                                                \
@@ -1430,12 +1446,19 @@ pg_status pg_launch_gguf_one_launch(pg_ctx *ctx, int ggml_type, size_t k_in, con
     // Two 16-row weight tiles a workgroup of the skinny kernel where that still leaves a workgroup for every CU: the digits, which
     // every workgroup fetches for all of K, then cost half as much per weight byte.
     const int tiles = n_total / 32 >= (size_t)ctx->num_cu ? 2 : 1, rows = skinny ? 16 * tiles : 32;
+    // The planes as uploaded, or everybody's tile-major copy where all have one: the same values in the same order, so the same bits.
+    // Up to sixteen rows do not make the copy (as many bytes as the tensor again, a wait, and a refusal under a capture; without
+    // it 180 products took 2 % longer on average, the worst a third: Q8_0 13 x 11168 -> 3856 19.8 : 26.4).
+    bool uploaded = skinny;
+    for (int i = 0; i < count && !skinny; ++i) {
+        if (m > 16) PG_TRY(pg_gguf_ensure_tiled(ctx, w[i]));
+        uploaded = uploaded || !pg_gguf_tiled(w[i]);
+    }
     pg_skinny_group grp;
     int wgs = 0;
     for (int i = 0; i < 3; ++i) {
         const bool used = i < count;
-        if (used && !skinny) PG_TRY(pg_gguf_ensure_tiled(ctx, w[i]));
-        grp.qs[i] = !used ? nullptr : skinny ? w[i]->qs : w[i]->qs_tiled;
+        grp.qs[i] = !used ? nullptr : uploaded ? w[i]->qs : w[i]->qs_tiled;
         grp.d[i] = used ? w[i]->d : nullptr;
         grp.y[i] = used ? y[i] : nullptr;
         grp.res[i] = i == 0 ? residual : nullptr;
@@ -1443,7 +1466,7 @@ pg_status pg_launch_gguf_one_launch(pg_ctx *ctx, int ggml_type, size_t k_in, con
         grp.wg0[i] = used ? wgs : INT_MAX;
         if (used) wgs += (int)((w[i]->n_out + rows - 1) / rows);
     }
-    return skinny ? launch_skinny(ctx, k_in, ggml_type == PG_GGML_Q8_0, grp, wgs, tiles, m, md) : launch_ktile(ctx, ggml_type, k_in, w, count, grp, wgs, m, md);
+    return skinny ? launch_skinny(ctx, k_in, ggml_type == PG_GGML_Q8_0, grp, wgs, tiles, m, md) : launch_ktile(ctx, ggml_type, k_in, w, count, grp, wgs, m, md, uploaded);
 }
 
 pg_status pg_launch_gguf_mm(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const uint8_t *qs,

@@ -124,7 +124,7 @@ struct pg_gguf_tensor {
     uint16_t *d;
     uint16_t *m;  // Q4_1 only: the blocks' f16 offsets, tiled like d; else null
     // Q4_0 / Q8_0: a second copy of qs in the order gguf_mm_kernel's workgroups fetch it
-    // (pg_gguf_ensure_tiled makes it on the tensor's first product over more than one row).
+    // (pg_gguf_ensure_tiled makes it at load time or on the first product that needs it: over more than 8 or 16 rows).
     mutable uint8_t *qs_tiled;
     int ggml_type;
     size_t n_out, k_in;
@@ -446,6 +446,7 @@ __host__ __device__ static inline size_t pg_tiled_group_bytes(int nb, bool q8) {
 }
 // Makes w->qs_tiled if it is missing (one allocation and one kernel on the context's stream).
 pg_status pg_gguf_ensure_tiled(pg_ctx *ctx, const pg_gguf_tensor *w);
+const uint8_t *pg_gguf_tiled(const pg_gguf_tensor *w);  // the copy, or null while there is none
 // Number of K chunks the product is split into (partial sums: [chunks][pairs][n_out] floats);
 // `groups` = token tiles that certainly hold work (all tiles of a plain product, one per expert).
 // `act_rows` = activation rows the product reads, `grouped` = with expert lists.

@@ -194,6 +194,31 @@ def test_prepare_makes_the_derived_copies_up_front(ctx, orc, typ):
     eager.free()
 
 
+@pytest.mark.parametrize("kind,m,n,k", [
+    ("q4_0", 5, 300, 2048), ("q4_0", 8, 9000, 1024), ("q4_0", 16, 8191, 1280), ("q4_0", 2, 100, 288), ("q4_0", 11, 33, 4192), ("q4_0", 16, 1, 1056),
+    ("q8_0", 5, 300, 2048), ("q8_0", 8, 9000, 1024), ("q8_0", 16, 8191, 1280), ("q8_0", 3, 129, 928), ("q8_0", 13, 31, 14336), ("q8_0", 6, 20000, 11776),
+    ("q4_1", 8, 300, 2048), ("q4_1", 16, 8000, 1024), ("q4_1", 9, 95, 4256),
+])
+def test_few_rows_read_the_planes_as_uploaded(ctx, orc, kind, m, n, k):
+    """Products of up to sixteen rows (a K that is no multiple of 256 up to the one launch's line) make no tile-major copy, and the bits
+    are those over the copy: part tiles of weight rows, a K that ends inside a unit of four blocks."""
+    from peregrine_amd import gguf
+    say(f"{kind} planes as uploaded m={m} n={n} k={k}")
+    pack, t = {"q4_0": (H.pack_q4_0, gguf.Q4_0), "q4_1": (H.pack_q4_1, gguf.Q4_1), "q8_0": (H.pack_q8_0, gguf.Q8_0)}[kind]
+    rng = np.random.default_rng(m + n + k)
+    raw = pack((rng.standard_normal(min(n, 500) * k) * 0.02).astype(np.float32))
+    raw = (bytes(raw) * (n // min(n, 500) + 1))[: n * len(raw) // min(n, 500)]     # (rows over again: packing is slow)
+    w = gguf.GgufWeight(raw, t, n, k, ctx)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    got = w.matmul(x, m).reshape(m, n)
+    assert w.device_bytes()[1] == 0
+    few = min(n, 500)
+    H.assert_close_rel(got[:, n - few:], orc.gguf_matmul(x, m, raw[(n - few) * (len(raw) // n):], int(t), few, k), RTOL_ACHIEVED_MM, kind)
+    w.prepare(m)
+    assert w.device_bytes()[1] > 0
+    assert (bits(w.matmul(x, m).reshape(m, n)) == bits(got)).all()
+
+
 def test_gguf_matmul_special_inputs(ctx, orc):
     from peregrine_amd import gguf
     n_out, k_in = 40, 128
