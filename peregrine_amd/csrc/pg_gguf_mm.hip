@@ -1255,7 +1255,7 @@ static bool skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_ou
 
 // Products small enough that digits, K chunks and their sum are three latencies: gguf_ktile_kernel.  Against that route (m 2 .. 400,
 // K 256 .. 14336, N 256 .. 14336, 1450 products) it takes 0.6 to 0.8 of the time up to half a G multiply-adds, is level at 1.5 (more than
-// 64 rows: 1, Q4_1 2) and slower beyond, where a tile of 128 weight rows shares a token's digits; so it is with a long K, or a short one
+// 64 rows: 1; Q4_1 1.8 to 700 rows and 1 beyond, from 245 products of 66 to 1800 rows: 0.5 % over the better route on average, 18 % at most) and slower beyond, where a tile of 128 weight rows shares a token's digits; so it is with a long K, or a short one
 // under many columns, over more than two row tiles (71 x 4896 -> 2614 24 : 31, 67 x 512 -> 13720 11.5 : 17).  Q4_1 up to 64 rows: the offsets' launch goes too (0.6 to 0.9 up to 5 G).  us, before : now:
 // 35 x 1088 -> 465 (Q8_0) 12.4 : 7.6, 12 x 4096 -> 4096 (Q4_1) 9.9 : 8.0, 11 x 1056 -> 2116 (Q8_0) 11.5 : 7.6, 32 x 4096 -> 1024
 // (Q4_0) 13.7 : 9.2, 64 x 4096 -> 4096 (Q4_1) 28.5 : 22.
@@ -1268,11 +1268,10 @@ static bool ktile_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out
     // (launch_ktile).  us over weights with a copy, gguf_mm_kernel : this: Q4_0 8 x 4096 -> 50257 36.7 : 32.9, 16 x 14336 -> 8000
     // 27.8 : 25.2, Q8_0 7 x 14336 -> 14336 45.1 : 45.1, 16 x 14336 -> 8000 32.2 : 32.6, the worst 8 x 14336 -> 12600 42.8 : 45.0.
     if (m <= (n_out < 32 * (size_t)ctx->num_cu ? 16u : 8u) && k_in % 256 == 0 && k_in >= 1024) return true;
-    if (q41 && m > 896) return false;  // (1216 -> 972, us, before : now: 512 rows 25.4 : 16.8, 700 25.8 : 20.5, 1008 28.5 : 29.1)
     const double g = 1e-9 * (double)m * (double)n_out * (double)k_in * (planes ? 1.5 : 1.0);
     if (k_in < 512 && n_out > 8192) return false;                                        // (all columns, hardly any K to split)
     if (m > 64 && (k_in >= (q41 ? 8192 : 6144) || (k_in < 1024 && m * n_out > 500000))) return false;
-    if (g > (q41 ? (m <= 64 ? 5.0 : 1.8) : m <= 64 ? 1.4 : m <= 128 ? 0.9 : 0.7)) return false;
+    if (g > (q41 ? (m <= 64 ? 5.0 : m <= 700 ? 1.8 : 1.0) : m <= 64 ? 1.4 : m <= 128 ? 0.9 : 0.7)) return false;
     return m <= 16 || !pg_gguf_hmm_takes(ctx, q41 ? PG_GGML_Q4_0 : ggml_type, m, n_out, k_in, nullptr);
 }
 

@@ -478,6 +478,24 @@ def test_gguf_rows_in_tiles(ctx, orc, n_out, k_in, m, typ):
     gw.free()
 
 
+@pytest.mark.parametrize("m,n,k,tiles", [(700, 1216, 2080, True), (701, 700, 2080, False), (701, 684, 2080, True), (897, 900, 1216, True), (1100, 300, 1216, True)])
+def test_q4_1_many_rows_either_side_of_the_tiles_line(ctx, orc, m, n, k, tiles):
+    """The one launch of tiles by its work (1.8 G multiply-adds to 700 rows, 1 G beyond, whatever their number), and the product with
+    an offsets' launch past it; the first, a middle and the last rows against the oracle."""
+    from peregrine_amd import gguf
+    say(f"q4_1 m={m} n={n} k={k}")
+    w = orc.rng_normal(m + n, n * k, 0.0, 0.02) + np.float32(0.03)
+    raw = H.pack_q4_1(w)
+    x = orc.rng_normal(m, m * k)
+    gw = gguf.GgufWeight(raw, gguf.Q4_1, n, k, ctx)
+    ctx.profile_begin()
+    got = gw.matmul(x, m).reshape(m, n)
+    assert ("gguf_q4_1_rows_tile" in ctx.profile_end()) == tiles
+    for r in (0, m // 2, m - 1):
+        H.assert_close_rel(got[r], orc.gguf_matmul(x.reshape(m, k)[r], 1, raw, 3, n, k), RTOL_ACHIEVED_MM, f"row {r}")
+    gw.free()
+
+
 @pytest.mark.parametrize("kind,m,k,forced", [
     ("q4_0", 1, 1024, 0), ("q4_0", 1, 4096, 0), ("q4_0", 2, 2048, 0), ("q4_0", 3, 1024, 0), ("q8_0", 1, 1024, 0), ("q8_0", 5, 1024, 0), ("q4_1", 1, 1024, 0),
     ("q4_1", 12, 1024, 0), ("q4_0", 40, 1024, 0), ("q8_0", 200, 1024, 0), ("q4_0", 40, 1024, 1), ("q8_0", 40, 1024, 1), ("q4_1", 40, 1024, 1),
