@@ -824,6 +824,15 @@ namespace {
 struct few_rows_shape { int mb, nb, nst, nw; double factor; };
 constexpr few_rows_shape FEW_ROWS_SHAPES[] = {{2, 1, 2, 2, 0.971}, {2, 1, 3, 4, 0.863}, {2, 1, 3, 8, 0.847}, {2, 2, 2, 4, 0.997}, {2, 2, 2, 8, 0.956},
                                               {3, 1, 2, 8, 0.903}, {3, 2, 2, 4, 1.033}, {3, 2, 2, 8, 1.0},   {4, 2, 3, 4, 1.009}};
+// What the tiles' K loops of one launch over all the weights take, us (see choose_few_rows).
+double tiles_us(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
+    static constexpr int BM[] = {64, 256, 128, 128, 128}, BN[] = {64, 256, 256, 64, 128};
+    static constexpr double STEP[] = {0.366, 1.98, 1.26, 0.302, 0.846};  // per 128 of K and round
+    if (count == 0) return 0.0;
+    const int t = pick_tile(ctx, w, count, m) - 1;
+    const size_t cus = (size_t)ctx->num_cu, rounds = (gemm_tiles(w, count, m, BM[t], BN[t]) + cus - 1) / cus;
+    return STEP[t] * (double)(rounds * (w[0]->k_pad / 128));
+}
 bool choose_few_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, few_rows_shape *out) {
     const size_t k_pad = w[0]->k_pad, units = k_pad / 128, cus = (size_t)ctx->num_cu;
     if (m < 33 || m > 512 || ctx->gemm_force_tile) return false;
@@ -849,13 +858,30 @@ bool choose_few_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, s
             *out = s;
         }
     }
-    static constexpr int BM[] = {64, 256, 128, 128, 128}, BN[] = {64, 256, 256, 64, 128};
-    static constexpr double STEP[] = {0.366, 1.98, 1.26, 0.302, 0.846};  // us per 128 of K and round
-    const int t = pick_tile(ctx, w, count, m) - 1;
-    const size_t rounds = (gemm_tiles(w, count, m, BM[t], BN[t]) + cus - 1) / cus;
-    return best < (m <= 256 ? 0.95 : 0.85) * (7.8 + 1.86 * mk + STEP[t] * (double)(rounds * units));
+    return best < (m <= 256 ? 0.95 : 0.85) * (7.8 + 1.86 * mk + tiles_us(ctx, w, count, m));
 }
 }  // namespace
+
+// Several weights that share the tiles' launch: whether those of long K and few columns are better off in a launch of their own, split
+// over K (pg_launch_gemm_w8a8_few_rows, estimated from 16 such products), because the others then need a round of tiles less, or
+// because few tiles walk a long K.
+// apart[i] says which.  us, all in one : apart: 135 x 10836 -> 628, 8185 75.7 : 63.8, 213 x 13535 -> 1432, 7172 96.9 :
+// 84.6, 36 x 13303 -> 1942, 6355 80.2 : 49.9, 46 x 13309 -> 294, 9512 81.2 : 57.0; of 110 such groups the worst it leaves is 34 x 7988 -> 8097,
+// 679, 708, 51.4 against 48.1 with each weight split.
+bool pg_gemm_w8a8_split_apart(pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, bool *apart) {
+    const pg_qtensor *rest[PG_GEMM_MAX_GROUP];
+    int n_rest = 0;
+    double split_us = 0.0;
+    for (int i = 0; i < count; ++i) {
+        int splits = 1;
+        apart[i] = m > 32 && (m <= 64 || (m <= 256 && w[i]->k_pad >= 2 * w[i]->cols)) && !ctx->gemm_force_tile &&
+                   pg_launch_gemm_w8a8_few_rows(ctx, nullptr, w[i]->k_pad, nullptr, w[i], m, nullptr, nullptr, nullptr, &splits) == PG_OK && splits > 1;
+        if (apart[i]) split_us += 9.5 + 0.05e-3 * (double)(m * w[i]->cols);
+        else rest[n_rest++] = w[i];
+    }
+    const double cold = m <= 64 ? 1.95 : 1.55;  // (a step of the tiles over weights that no cache holds)
+    return n_rest < count && split_us + cold * tiles_us(ctx, rest, n_rest, m) < 0.95 * cold * tiles_us(ctx, w, count, m);
+}
 
 // 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights side by side.
 // (33 .. 64 rows where the estimates say no, us with the quantisation launch: 4096 -> 14336 24.7 against 30.3 split over K with a

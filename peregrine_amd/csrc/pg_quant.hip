@@ -690,9 +690,17 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     // one weight: the single product picks its own route (GEMV, split K)
     if (count == 1) return pg_matmul_quantized_dev(ctx, a_dev, m, k, w[0], out_dev[0], nullptr);
     const size_t k_pad = w[0]->k_pad, m_pad = pg_round_up(m, PG_MPAD);
-    const size_t a_bytes = m_pad * k_pad;
+    const size_t a_bytes = m_pad * k_pad, sz_scales = pg_round_up(m_pad * sizeof(float), 256);
+    bool apart_of[PG_GEMM_MAX_GROUP];
+    const bool split = pg_gemm_w8a8_split_apart(ctx, w, (int)count, m, apart_of);
+    size_t part_bytes = 0;
+    for (size_t i = 0; i < count && split; ++i) {
+        int splits = 1;
+        if (apart_of[i]) PG_TRY(pg_launch_gemm_w8a8_few_rows(ctx, nullptr, k_pad, nullptr, w[i], m, nullptr, nullptr, nullptr, &splits));
+        part_bytes = std::max(part_bytes, (size_t)splits * m * w[i]->cols * sizeof(int32_t));
+    }
     void *ws = nullptr;
-    PG_TRY(pg_workspace(ctx, a_bytes + pg_round_up(m_pad * sizeof(float), 256), &ws));
+    PG_TRY(pg_workspace(ctx, a_bytes + sz_scales + part_bytes, &ws));
     int8_t *a_i8 = static_cast<int8_t *>(ws);
     float *a_scales = reinterpret_cast<float *>(a_i8 + a_bytes);
     PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, k_pad, a_scales));
@@ -708,7 +716,10 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     int n_small = 0;
     for (size_t i = 0; i < count; ++i) {
         const size_t t256 = ((m + 255) / 256) * ((w[i]->cols + 255) / 256);
-        if (t256 >= (size_t)ctx->num_cu) {
+        if (split && apart_of[i]) {
+            PG_TRY(pg_launch_gemm_w8a8_few_rows(ctx, a_i8, k_pad, a_scales, w[i], m, out_dev[i], nullptr,
+                                                reinterpret_cast<int32_t *>(a_i8 + a_bytes + sz_scales), nullptr));
+        } else if (t256 >= (size_t)ctx->num_cu) {
             PG_TRY(pg_launch_gemm_w8a8(ctx, a_i8, k_pad, a_scales, w[i], m, out_dev[i], nullptr));
         } else {
             small_w[n_small] = w[i];

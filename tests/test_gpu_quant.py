@@ -796,3 +796,28 @@ def test_w8a8_over_its_own_rows_bit_exact(ctx, orc, m, k, shift):
     assert (bits(aside) == bits(wants[1])).all()
     aside = check(lambda x, out, at: L.pg_matmul_quantized_multi_dev(ctx.handle, x, m, k, both, 2, tab([at, out])), 1)
     assert (bits(aside) == bits(wants[0])).all()
+
+
+@pytest.mark.parametrize("m,k,ns,apart", [(46, 13300, [294, 9512], 2), (135, 10836, [628, 8185], 1), (63, 13958, [8390, 421, 363], 3), (65, 10836, [628, 8185], 0)])
+def test_several_weights_some_split_over_k_bit_exact(ctx, orc, m, k, ns, apart):
+    """Weights of one launch whose long, narrow (or, to 64 rows, any) ones go apart, split over K: how many do, and the bits."""
+    from peregrine_amd import quant, _ffi
+    say(f"several weights, split over K m={m} k={k} ns={ns}")
+    rng = np.random.default_rng(m + 10 * k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a_dev = DevBuf(ctx, host=a)
+    qa, s = orc.quantize_activations(a, m, k)
+    qts, wants = [], []
+    for c in ns:
+        q = rng.integers(-127, 128, (k, c), dtype=np.int8)
+        scales = rng.uniform(0.5e-3, 2e-3, c).astype(np.float32)
+        qts.append(quant.QuantizedTensor(q.reshape(-1), None, scales, k, c).to_gpu(ctx))
+        acc = np.asarray(qa, np.float64).reshape(m, k) @ q.astype(np.float64)
+        wants.append(acc.astype(np.float32) * np.asarray(s, np.float32)[:, None] * scales[None, :])
+    outs = [DevBuf(ctx, nbytes=4 * m * c) for c in ns]
+    tab = lambda v: (C.c_void_p * len(v))(*v)
+    ctx.profile_begin()
+    _ffi.check(_ffi.lib.pg_matmul_quantized_multi_dev(ctx.handle, a_dev.ptr, m, k, tab([t._gpu.value for t in qts]), len(ns), tab([o.ptr.value for o in outs])))
+    assert ctx.profile_end().get("gemm_w8a8_finish", (0, 0))[1] == apart
+    for want, out, c in zip(wants, outs, ns):
+        assert (bits(out.to_host(np.float32).reshape(m, c)) == bits(want)).all()
