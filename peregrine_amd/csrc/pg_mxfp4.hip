@@ -129,9 +129,10 @@ __device__ __forceinline__ void mx_emit_digits(const float (&f)[4], int b, int s
 // entry of two pointer tables, the activation row is the token's (by_token) or the pair's, the output row the pair's.  2: mlp1, whose rows 2 i and 2 i + 1
 // with their biases become value i of the output row, their swiglu (made where mlp2
 // reads its rows it is made once for every 64 of mlp2's rows: 5 us more at 64 pairs of 2880 x 2880).  With the choice of the experts read
-// as the caller made it, a layer of few pairs is three launches where it was five (4 of 32 experts of 2880 x 2880: one token 23.0 -> 18.8
-// us, two 32.0 -> 30.9; 16 tokens, with eleven rounds of workgroups that each look at the entries, 156 -> 158; 4 of 16 of 1024 x 1024,
-// two tokens 18.3 -> 14.2; random layers of 1 to 8 tokens 0.77 to 0.85 of the time, 9 to 24 0.94).
+// as the caller made it, a layer of few pairs is three launches where it was five.  The expert and its tables are found by scalar loads
+// behind the requests for the activation row: looked up ahead of them, by a lane an entry, that chain was in front of every one of up to
+// eleven rounds of workgroups.  us, five launches : the look-up in front : now, 4 of 32 experts of 2880 x 2880: one token 24.5 : 20.5 : 19.6, two 33.5 :
+// 32.0 : 28.5, 16 tokens 160.0 : 163.3 : 154.7; 16 tokens of 1440 x 2880 88.8 : 92.4 : 86.0; 4 of 16 of 1024 x 1024, two tokens 19.2 : 15.2 : 14.7.
 struct mt_swiglu {
     const float *const *bias_tab;
     float alpha, clamp;
@@ -175,8 +176,27 @@ struct mx_routed {
     }
 };
 static_assert(PG_MOE_MAX_EXPERTS <= 256, "mx_routed holds 256 experts");
-// Entry k (up to 63) of a token, by a wavefront: a lane an entry; only where one up to k is out of range or named twice they are walked.
+// What the kernel does not write, at addresses that are the same for a wavefront: through the scalar cache.
+template <typename T> __device__ __forceinline__ T mx_uniform(const T *p) {
+    typedef const T __attribute__((address_space(4))) *ptr;
+    return *(ptr)(uintptr_t)p;
+}
+// Entry k (up to 63) of a token, by a wavefront: the first four as scalars, later ones a lane an entry; only where one up to k is out
+// of range or named twice they are walked.
 __device__ __forceinline__ int mx_expert_of_entry(const int *__restrict__ idx, int k, int experts) {
+    if (k < 4) {
+        int a[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = mx_uniform(idx + (j < k ? j : k));
+        bool fine = true;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            fine = fine && (unsigned)a[j] < (unsigned)experts;
+#pragma unroll
+            for (int l = j + 1; l < 4; ++l) fine = fine && (a[j] != a[l] || l > k);
+        }
+        if (fine) return a[3];  // (entry k, clamped)
+    }
     const int lane = threadIdx.x & 63, e = idx[lane < k ? lane : k];
     bool odd = e < 0 || e >= experts;
     for (int j = 0; j < k; ++j) odd |= lane > j && lane <= k && e == __builtin_amdgcn_readlane(e, j);
@@ -197,17 +217,7 @@ __global__ __launch_bounds__(64 * NW) void mxfp4_rows_kernel(const uint8_t *__re
     size_t x_row0 = (size_t)blockIdx.y * T;  // first activation row of this workgroup
     float bias = 0.0f;
     const size_t pair = (size_t)blockIdx.z * gridDim.y + blockIdx.y;
-    if (PAIRS) {
-        const int expert = PAIRS == 2 ? mx_expert_of_entry(pr.idx + (size_t)blockIdx.z * gridDim.y, blockIdx.y, pr.experts) : pr.chosen[pair];
-        if (PAIRS == 2 && blockIdx.x == 0 && threadIdx.x == 0) pr.chosen[pair] = expert;
-        if (PAIRS == 2) {  // (asked for now: one of the 16 RG rows a thread of the last step)
-            const int row = (int)blockIdx.x * RG * 16 + (int)threadIdx.x % (RG * 16);
-            bias = pr.act.bias_tab[expert][row < n_out ? row : n_out - 1];
-        }
-        qs_frag = pr.qs_tab[expert];
-        sc_frag = pr.sc_tab[expert];
-        x_row0 = pr.by_token ? blockIdx.z : pair;
-    }
+    if (PAIRS) x_row0 = pr.by_token ? blockIdx.z : pair;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int kp = ncp * 128, stride = kp + 16;  // plane stride = 16 (mod 256): the 16 columns of a 128-bit read fall into 16 different bank groups
     char *const dig = lds;
@@ -220,8 +230,8 @@ __global__ __launch_bounds__(64 * NW) void mxfp4_rows_kernel(const uint8_t *__re
     rg = rg < nrg ? rg : nrg - 1;  // a spare wavefront repeats the last group; its result is not stored
     const int cps = ((ncp + KS - 1) / KS + 3) & ~3;  // chunks per K slice, whole scale dwords
     const int c0 = ksi * cps, c1 = (c0 + cps < ncp) ? c0 + cps : ncp;
-    const gv4i_ptr qa = (gv4i_ptr)(uintptr_t)qs_frag + (size_t)rg * ncp * 64 + lane;
-    const uint32_t *__restrict__ sa = sc_frag + (size_t)rg * (ncp / 4) * 64 + lane;
+    gv4i_ptr qa = nullptr;
+    const uint32_t *__restrict__ sa = nullptr;
 
     v4i abuf[2][MX_U];
     uint32_t sabuf[2][MX_U / 4];
@@ -270,6 +280,18 @@ __global__ __launch_bounds__(64 * NW) void mxfp4_rows_kernel(const uint8_t *__re
     }
     asm volatile("" ::: "memory");  // (keeps the compiler from moving these loads down to their uses)
     __builtin_amdgcn_sched_barrier(0);
+    if (PAIRS) {  // (the pair's expert and its tables, scalar loads, while the activation blocks fly)
+        const int expert = PAIRS == 2 ? mx_expert_of_entry(pr.idx + (size_t)blockIdx.z * gridDim.y, blockIdx.y, pr.experts) : mx_uniform(pr.chosen + pair);
+        if (PAIRS == 2 && blockIdx.x == 0 && threadIdx.x == 0) pr.chosen[pair] = expert;
+        qs_frag = mx_uniform(pr.qs_tab + expert);
+        sc_frag = mx_uniform(pr.sc_tab + expert);
+        if (PAIRS == 2) {  // (asked for now: one of the 16 RG rows a thread of the last step)
+            const int row = (int)blockIdx.x * RG * 16 + (int)threadIdx.x % (RG * 16);
+            bias = mx_uniform(pr.act.bias_tab + expert)[row < n_out ? row : n_out - 1];
+        }
+    }
+    qa = (gv4i_ptr)(uintptr_t)qs_frag + (size_t)rg * ncp * 64 + lane;
+    sa = sc_frag + (size_t)rg * (ncp / 4) * 64 + lane;
     load_batch(abuf[0], sabuf[0], c0 < ncp ? c0 : 0);  // (an empty slice consumes nothing)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

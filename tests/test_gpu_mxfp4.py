@@ -326,7 +326,8 @@ def test_mxfp4_moe_tilings(ctx, orc, hidden, inter, E, top_k, T):
     test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, T)
 
 
-@pytest.mark.parametrize("hidden,inter,E,top_k,T", [(64, 96, 6, 6, 3), (512, 512, 200, 64, 1), (512, 96, 70, 12, 5), (64, 512, 2, 1, 9)])
+@pytest.mark.parametrize("hidden,inter,E,top_k,T", [(64, 96, 6, 6, 3), (512, 512, 200, 64, 1), (512, 96, 70, 12, 5), (64, 512, 2, 1, 9), (64, 96, 9, 4, 6), (96, 64, 5, 3, 8),
+                                                   (64, 96, 8, 5, 4), (96, 64, 4, 2, 7)])
 def test_mxfp4_moe_pairs_with_entries_that_name_no_expert(ctx, hidden, inter, E, top_k, T):
     """Entries out of range or named twice count as the lowest free expert with weight 0: the device entry's rows are those of the
     routing with them replaced so, in every bit, and the caller's entries stay as they were."""
