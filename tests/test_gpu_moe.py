@@ -157,12 +157,13 @@ def test_moe_full_size_distinct_experts_against_the_oracle(ctx, orc):
         w.free()
 
 
-def test_moe_many_tokens_per_expert(ctx, orc):
-    """More than 32 tokens reach one expert (two token tiles), another expert gets none, and the
-    widths are not multiples of the kernel's 128-row / 4-block tiles."""
+@pytest.mark.parametrize("T,d,ffn,kernel", [(75, 96, 224, "gguf_gemv_q4_0"), (75, 544, 1056, "gguf_q4_0_experts_tile"), (300, 1056, 1568, "gguf_mm_q4_0")])
+def test_moe_many_tokens_per_expert(ctx, orc, T, d, ffn, kernel):
+    """More than 32 tokens reach one expert (two token tiles and more), another expert gets none, and the
+    widths are not multiples of the kernels' 128- or 32-row / 4-block tiles; a K of a few blocks streams."""
     from peregrine_amd import gguf, moe
-    T, d, ffn, E, top_k = 75, 96, 224, 5, 2
-    say("moe many tokens per expert")
+    E, top_k = 5, 2
+    say(f"moe many tokens per expert T={T} d={d} ffn={ffn}")
     raws = build(orc, 90, d, ffn, E, 2)
     x = orc.rng_normal(5, T * d)
     logits = orc.rng_normal(6, T * E).reshape(T, E)
@@ -170,7 +171,10 @@ def test_moe_many_tokens_per_expert(ctx, orc):
     logits[:, 4] = -30.0   # expert 4 is never chosen
     mk = lambda rs, n_out, k_in: [gguf.GgufWeight(r, 2, n_out, k_in, ctx) for r in rs]
     ex = moe.MoEExperts(mk(raws[0], ffn, d), mk(raws[1], ffn, d), mk(raws[2], d, ffn), top_k, moe.SILU, ctx)
+    ctx.profile_begin()
     got = ex.forward(x, logits)
+    prof = ctx.profile_end()
+    assert kernel in prof, sorted(prof)
     want, idx, prob = orc.moe_ffn(x, T, d, ffn, E, top_k, logits, raws[0], raws[1], raws[2], 2, 0)
     assert (idx == 3).sum() > 32 and (idx == 4).sum() == 0
     for t in range(T):
