@@ -1241,6 +1241,9 @@ int pg_gguf_mm_splitk(const pg_ctx *ctx, size_t n_out, size_t k_in, size_t group
     return (int)ks_real;
 }
 
+// Rows up to which a product leaves its tensor without a tile-major copy.
+static size_t few_rows_of(const pg_ctx *ctx, size_t n_out) { return n_out < 32 * (size_t)ctx->num_cu ? 16 : 8; }
+
 // Up to 8 rows over a Q4_0 or Q8_0 tensor whose K is a multiple of 256: gguf_skinny_kernel, bound by how many bytes its rings keep
 // in flight (4 x 4096 -> 14336 takes 9.0 us; with its arithmetic switched off 8.6 - 9.1).  From five rows on it is the better one
 // only where a long K meets few columns (us, this one : gguf_ktile_kernel: 7 x 11776 -> 1804 12.7 : 14.8, 8 x 8704 -> 406 10.7 :
@@ -1267,7 +1270,7 @@ static bool ktile_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out
     // Up to eight rows, up to sixteen of fewer than 8192 columns: always, so that no product of so few rows needs the tile-major copy
     // (launch_ktile).  us over weights with a copy, gguf_mm_kernel : this: Q4_0 8 x 4096 -> 50257 36.7 : 32.9, 16 x 14336 -> 8000
     // 27.8 : 25.2, Q8_0 7 x 14336 -> 14336 45.1 : 45.1, 16 x 14336 -> 8000 32.2 : 32.6, the worst 8 x 14336 -> 12600 42.8 : 45.0.
-    if (m <= (n_out < 32 * (size_t)ctx->num_cu ? 16u : 8u) && k_in % 256 == 0 && k_in >= 1024) return true;
+    if (m <= few_rows_of(ctx, n_out) && k_in % 256 == 0 && k_in >= 1024) return true;
     const double g = 1e-9 * (double)m * (double)n_out * (double)k_in * (planes ? 1.5 : 1.0);
     if (k_in < 512 && n_out > 8192) return false;                                        // (all columns, hardly any K to split)
     if (m > 64 && (k_in >= (q41 ? 8192 : 6144) || (k_in < 1024 && m * n_out > 500000))) return false;
@@ -1446,11 +1449,11 @@ pg_status pg_launch_gguf_one_launch(pg_ctx *ctx, int ggml_type, size_t k_in, con
     // every workgroup fetches for all of K, then cost half as much per weight byte.
     const int tiles = n_total / 32 >= (size_t)ctx->num_cu ? 2 : 1, rows = skinny ? 16 * tiles : 32;
     // The planes as uploaded, or everybody's tile-major copy where all have one: the same values in the same order, so the same bits.
-    // Up to sixteen rows do not make the copy (as many bytes as the tensor again, a wait, and a refusal under a capture; without
-    // it 180 products took 2 % longer on average, the worst a third: Q8_0 13 x 11168 -> 3856 19.8 : 26.4).
+    // Up to eight rows, up to sixteen of fewer than 8192 columns, do not make the copy (as many bytes as the tensor again, a wait, and a
+    // refusal under a capture; without it 180 products took 2 % longer on average, the worst a third: Q8_0 13 x 11168 -> 3856 19.8 : 26.4).
     bool uploaded = skinny;
     for (int i = 0; i < count && !skinny; ++i) {
-        if (m > 16) PG_TRY(pg_gguf_ensure_tiled(ctx, w[i]));
+        if (m > few_rows_of(ctx, n_total)) PG_TRY(pg_gguf_ensure_tiled(ctx, w[i]));
         uploaded = uploaded || !pg_gguf_tiled(w[i]);
     }
     pg_skinny_group grp;
