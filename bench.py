@@ -991,7 +991,7 @@ def section_moe(B, line):
         "frac_of_hbm_peak": round(moe_bytes / (t_moe["ms_per_step"] * 1e-3) / 1e9 / PEAK_HBM_GBS, 4), **B.stats(t_moe, 4),
         "tflops": round(2 * T_moe * topk_moe * 3 * ffn_moe * d_moe / (t_moe["ms_per_step"] * 1e-3) / 1e12, 2),
         "kernels_ms": {k: round(v[0], 5) for k, v in prof.items()},
-        "roofline": {"kernel": "gguf_mm_kernel<Q8_0> (gate|up, down)", "bound": "hbm",
+        "roofline": {"kernel": {"gguf_mm_q8_0": "gguf_mm_kernel<Q8_0>", "gguf_q8_0_experts_tile": "gguf_ktile_kernel<Q8_0>"}[k_name] + " (gate|up, down)", "bound": "hbm",
                      "achieved": round(3 * E_moe * nblk * 34 / (mm_total * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS,
                      "unit": "GB/s", "frac": round(3 * E_moe * nblk * 34 / (mm_total * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
                      "traffic": B.traffic_for(k_name, grids), "bytes_per_launch": int(3 * E_moe * nblk * 34 / mm_launches),

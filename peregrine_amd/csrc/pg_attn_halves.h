@@ -107,11 +107,11 @@ __global__ __launch_bounds__(256) void kv_halves_kernel(const float *__restrict_
 // A workgroup takes 128 rows of a kv head (row index = token * group + head in group), 32 to a wavefront, and a run of aa.chunk
 // of the key tiles that they see.  Per tile S^T = K Q^T and O^T += V^T P^T with the columns = rows of the query, as in the f32
 // kernel above: the tile of S^T that a lane holds is, register by register, the operand of the second product.  The ring
-// holds three units (a tile's keys or its values): one consumed, one landed or landing, one asked for when everybody has left its
-// place; 48 KiB for HD = 128: two workgroups a CU (by their registers), not in step with each other, so that the softmax of one runs beside the
+// holds four units (a tile's keys or its values): one consumed, two landed or landing, one asked for when everybody has left its
+// place; 64 KiB for HD = 128: two workgroups a CU (by their registers), not in step with each other, so that the softmax of one runs beside the
 // matrix instructions of the other.  Rows that one run covers are finished here, others leave (maximum, exp-sum, unnormalised
 // row) in aa.part for attn_halves_combine_kernel.
-constexpr int HALVES_ROWS = 128, HALVES_CHUNK_MAX = 512, HALVES_RING = 4;
+constexpr int HALVES_ROWS = 128, HALVES_CHUNK_MAX = 512, HALVES_RING = 4;  // (CHUNK_MAX: the tiles of a run, by the array of their scales)
 constexpr float HALVES_SLACK = 5.0f, LOG2E = 1.44269504f;
 __device__ __forceinline__ int halves_tiles(const attn_args &aa, int blk, int nrows) {  // key tiles that a block of rows sees
     const int last_qt = min(blk * HALVES_ROWS + HALVES_ROWS - 1, nrows - 1) / aa.group;

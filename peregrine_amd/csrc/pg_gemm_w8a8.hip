@@ -897,7 +897,7 @@ bool pg_gemm_w8a8_takes_skinny(const pg_ctx *ctx, const pg_qtensor *const *w, in
     return m <= 32 || choose_few_rows(ctx, w, count, m, &s) || (m <= 64 && !narrow);
 }
 
-// 2 .. 64 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights of equal K side by side.
+// 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights of equal K side by side.
 pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                                            const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc) {
     if (count < 1 || count > PG_GEMM_MAX_GROUP || (acc && count != 1))

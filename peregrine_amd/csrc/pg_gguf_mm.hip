@@ -671,7 +671,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // wavefront with an LDS ring of its own (no barrier in the loop: it reads only what it loaded itself), and their
 // f32 tiles are added through LDS in a fixed order at the end.  A unit of the ring is 8 blocks (256 k): the weight
 // tiles as whole 128-byte lines per row (8 rows an instruction, 16-byte chunk p of row r at position
-// p ^ ((r >> 1) & 7)), their f16 scales, the two digit planes of the 16 token rows (256 bytes a row and plane,
+// p ^ ((r >> 1) & 7)), their f16 scales, the two digit planes of the MT token rows (256 bytes a row and plane,
 // chunk c of token t at position c ^ t) and the tokens' block scales; NST - 1 units are in flight while one is
 // consumed.  The weights are read in the row-major planes every tensor has (no tile-major copy).  Each workgroup starts its
 // walk through K at its own unit.
@@ -878,7 +878,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4)))
 // K, its NW wavefronts take one run of K each with an LDS ring of their own (no barrier in the loop), and their f32 tiles
 // are added through LDS in a fixed order.  Nothing is left for a third launch, and a small tensor has as many wavefronts as its
 // blocks can feed.  A unit of the ring is four blocks: the tile-major copy's run of the 32 rows (2 or 4 KiB), their f16 scales,
-// the digit planes and block scales of the tokens.  Blocks past the end of K are not added.
+// the digit planes and block scales of the tokens.  Blocks past the end of K are not added.  UPLOADED: the weights' 16-byte chunks
+// come from the planes as uploaded instead, 64 bytes of a row to four lanes, into the same places (see pg_launch_gguf_one_launch).
 // More than MT tokens: groups of MT, a weight tile's groups behind each other on one XCD.
 // MT = 8, 16: tokens on the accumulator registers (half of MT of them), weight rows on the lanes; MT = 32 the other way
 // round, as gguf_mm_kernel.

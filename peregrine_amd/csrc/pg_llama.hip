@@ -1528,6 +1528,10 @@ bool split_mfma_tiles(const pg_ctx *ctx, size_t group, size_t seq_q, size_t nkv,
 // The line is drawn by estimates from 200 shapes (4 .. 1000 tokens behind 0 .. 30000): 200 tokens behind 300 79 : 31, 64 behind
 // 2000 44 : 33, but 32 behind 300 16 : 21 and 16 behind 8000 38 : 58; the worst pick among them is 64 behind 8000 of 4 heads of
 // 64, 37 : 40, and of those that stay 128 behind 300, 33 : 27.
+//
+// Two limits leave calls to the f32 kernels that would take a third of the time here: planes of more than 256 MiB (32 736 positions of 8
+// heads of 128), and blocks of rows for more than the places on the chip, which take all key tiles in one run, over more than
+// HALVES_CHUNK_MAX of them (2048 tokens of 32 / 8 heads and more that see more than 16 384 positions).
 struct halves_plan {
     size_t blocks, tiles, chunk, runs, plane_bytes, part_bytes;
 };
