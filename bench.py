@@ -3,7 +3,8 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W]
 
-Prints ONE JSON line.  Headline (`value`): W8A8 prefill GEMM throughput, in TOP/s, over the
+Prints ONE JSON line (the values; the record with every workload's description and every kernel's time goes to
+stderr).  Headline (`value`): W8A8 prefill GEMM throughput, in TOP/s, over the
 seven projections of one Llama-3-8B layer at M = 2048 tokens (q, k, v, o, gate, up, down;
 893 353 197 568 integer ops per step), run as models::llama runs them: q|k|v and gate|up as fused
 products over one input (four calls, each = per-row activation quantisation + i8 MFMA GEMM +
@@ -424,8 +425,31 @@ def main():
 
     line["launch_work_items"] = LAUNCHES_SEEN
     line["cpu_baseline"] = cpu_baseline(B.orc, cpu_w, cpu_a) if B.cpu else None
-    print(json.dumps(line), flush=True)
+    print("full record: " + json.dumps(line), file=sys.stderr, flush=True)
+    print(json.dumps(short_line(line)), flush=True)
     B.ctx.close()
+
+
+# What stays of a section in the line: a log's last 8 KB are to hold all of it.
+HEADLINE = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "median_ms", "min_ms", "std_ms", "higher_is_better", "scaling", "vs_baseline",
+            "dtype", "data", "config", "pct_int8_mfma_peak", "roofline", "ceilings", "cpu_baseline")
+LEFT_OUT = ("workload", "what", "sample", "note", "config", "cores", "kind", "std_ms", "min_ms", "median_ms", "bytes_per_step", "bytes_per_launch", "flop_per_launch",
+            "launches_per_step", "peak", "bound", "steps", "traffic", "avg_launch_ms", "kernels_ms", "kernels_ms_x_launches", "kernels_us", "launch_work_items", "gemm_vs_vendor_library")
+
+
+def short_line(line):
+    """The headline's fields whole, of every other section its values without the prose and the single kernels' times, of its
+    roofline the fraction and of its CPU baseline the value."""
+    def brief(v):
+        if isinstance(v, dict):
+            one = {"roofline": "frac", "cpu_baseline": "value"}
+            return {k: x[one[k]] if k in one and isinstance(x, dict) and one[k] in x else brief(x) for k, x in v.items() if k not in LEFT_OUT}
+        if isinstance(v, list):
+            return [{**({"of": x["workload"][:28]} if isinstance(x, dict) and "workload" in x else {}), **brief(x)} if isinstance(x, dict) else brief(x) for x in v]
+        if isinstance(v, float):
+            return float(f"{v:.5g}")
+        return v[:40] if isinstance(v, str) else v
+    return {k: v if k in HEADLINE else brief(v) for k, v in line.items() if k not in LEFT_OUT or k in HEADLINE}
 
 
 def probe_shapes(B):
