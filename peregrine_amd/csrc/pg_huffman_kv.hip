@@ -164,12 +164,17 @@ __global__ __launch_bounds__(KV_WG) void kv_quant_hist_kernel(const kv_batch b, 
     b.hist[((size_t)c * b.nwg + blockIdx.x) * NUM_SYMBOLS + t] = (uint16_t)(lh[0][t] + lh[1][t] + lh[2][t] + lh[3][t]);
 }
 
-// Lane exchange for the merges below: the value of lane ^ D.
+// Lane exchange for the sorts below: the value of lane ^ D.
 template <int D> __device__ __forceinline__ unsigned lane_xor(unsigned v) {
     if constexpr (D == 1) return __builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // quad_perm 1 0 3 2
     else if constexpr (D == 2) return __builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2 3 0 1
-    else if constexpr (D == 4) return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);  // ^ 7, ^ 3
+    else if constexpr (D == 3) return __builtin_amdgcn_mov_dpp((int)v, 0x1B, 0xF, 0xF, true);   // quad_perm 3 2 1 0
+    else if constexpr (D == 7) return __builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+    else if constexpr (D == 15) return __builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true); // row_mirror
+    else if constexpr (D == 4) return lane_xor<3>(lane_xor<7>(v));
     else if constexpr (D == 8) return __builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);  // row_ror 8
+    else if constexpr (D == 31) return lane_xor<16>(lane_xor<15>(v));
+    else if constexpr (D == 63) return lane_xor<32>(lane_xor<31>(v));
     else {
         const auto two = D == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false) : __builtin_amdgcn_permlane32_swap(v, v, false, false);
         return threadIdx.x & D ? two[0] : two[1];
@@ -178,9 +183,34 @@ template <int D> __device__ __forceinline__ unsigned lane_xor(unsigned v) {
 template <int D> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
     return (unsigned long long)lane_xor<D>((unsigned)(v >> 32)) << 32 | lane_xor<D>((unsigned)v);
 }
-template <int D, class K> __device__ __forceinline__ void half_cleaner(K &x) {
-    const K o = lane_xor<D>(x);
-    x = ((threadIdx.x & D) != 0) == (o > x) ? o : x;
+// The smaller of both for end = 0, the larger for end = ~0: one instruction, their median with `end`.
+__device__ __forceinline__ unsigned end_of(unsigned x, unsigned o, unsigned end) { return max(min(x, o), min(max(x, o), end)); }
+__device__ __forceinline__ unsigned long long end_of(unsigned long long x, unsigned long long o, unsigned end) { return (end != 0) == (o > x) ? o : x; }
+// The smaller of a lane and lane ^ D stays where bit B of the lane is clear, the larger where it is set.
+template <int D, int B, class K> __device__ __forceinline__ void order_pair(K &x) {
+    const unsigned end = threadIdx.x & B ? ~0u : 0u;
+    if constexpr (sizeof(K) == 4 && (D == 16 || D == 32)) {  // the swap leaves both in every lane
+        const auto two = D == 16 ? __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)x, false, false) : __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)x, false, false);
+        x = end_of(two[0], two[1], end);
+    } else x = end_of(x, lane_xor<D>(x), end);
+}
+// A bitonic sequence of 64 lanes into ascending order.
+template <class K> __device__ __forceinline__ void order_bitonic(K &x) {
+    order_pair<32, 32>(x);
+    order_pair<16, 16>(x);
+    order_pair<8, 8>(x);
+    order_pair<4, 4>(x);
+    order_pair<2, 2>(x);
+    order_pair<1, 1>(x);
+}
+// Any 64 into ascending order: runs of 2, 4, .. 64 by meeting their mirror image.
+template <class K> __device__ __forceinline__ void order_wave(K &x) {
+    order_pair<1, 1>(x);
+    order_pair<3, 2>(x); order_pair<1, 1>(x);
+    order_pair<7, 4>(x); order_pair<2, 2>(x); order_pair<1, 1>(x);
+    order_pair<15, 8>(x); order_pair<4, 4>(x); order_pair<2, 2>(x); order_pair<1, 1>(x);
+    order_pair<31, 16>(x); order_pair<8, 8>(x); order_pair<4, 4>(x); order_pair<2, 2>(x); order_pair<1, 1>(x);
+    order_pair<63, 32>(x); order_pair<16, 16>(x); order_pair<8, 8>(x); order_pair<4, 4>(x); order_pair<2, 2>(x); order_pair<1, 1>(x);
 }
 
 // Running sum over the lanes of a row of 16.
@@ -200,180 +230,168 @@ __device__ __forceinline__ unsigned wave_scan(unsigned v) {
     return v;
 }
 
-// The Huffman merges of n leaves (ascending weights) on one wavefront; returns the number of rounds.  Two queues, leaves
-// and the nodes made of them, both ascending.  The sum m of the two lightest trees is the smallest weight that a new node
-// can have, so all trees of weight <= m are taken, two by two, before any node that the round makes (a tie goes to the one
-// that was there first: a leaf before a node).  A round sorts the 64 lightest of both queues' heads across the lanes
-// -- min of the one ascending and the other descending is bitonic, six exchanges put it in order -- and pairs
-// neighbours, up to 32 at a time.  K holds weight << 9 | id: 32 bits for chunks below 2^23 values, else 64.
-constexpr unsigned TREE_PAD = NUM_SYMBOLS + 64;  // (a round reads 64 from a queue's head on)
+// LDS that one wavefront writes and reads: its accesses happen in program order, so only the compiler has to keep it.
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// The Huffman merges of n leaves on one wavefront; returns the number of rounds.  Two queues, leaves and the nodes made of
+// them, both ascending, of keys weight << 9 | id (ids of nodes from NUM_SYMBOLS on), with NONE behind their ends.  The sum m of
+// the two lightest trees is the smallest weight that a new node can have, so all trees of weight <= m are taken, two
+// by two, before any node that the round makes (a tie goes to the one that was there first: a leaf before a node).  A
+// round puts the 64 lightest of both queues' heads in order across the lanes -- min of the one ascending and the other
+// descending is bitonic, six exchanges of two instructions -- and pairs neighbours, up to 32 at a time.
+constexpr unsigned TREE_PAD = NUM_SYMBOLS + 64;  // (a round reads 64 from a queue's head on; what is not taken is written behind)
 template <class K>
-__device__ __forceinline__ unsigned merge_trees(unsigned n, const unsigned *leaf_w, unsigned *node_w, unsigned *parent) {
+__device__ __forceinline__ unsigned merge_trees(unsigned n, const K *leaf_key, K *node_key, unsigned *parent) {
     const unsigned lane = threadIdx.x & 63;
     unsigned lh = 0, qh = 0, made = 0, rounds = 0;
     for (unsigned alive = n; alive > 1; ++rounds) {
-        constexpr unsigned NONE = 0x7FFFFFFFu;  // (not below any sum but the last)
-        const unsigned li = lh + lane, qi = qh + 63 - lane;
-        unsigned lw = leaf_w[li], qw = node_w[qi];
-        lw = li < n ? lw : NONE;
-        qw = qi < made ? qw : NONE;
-        const unsigned l0 = __builtin_amdgcn_readlane(lw, 0), l1 = __builtin_amdgcn_readlane(lw, 1);
-        const unsigned q0 = __builtin_amdgcn_readlane(qw, 63), q1 = __builtin_amdgcn_readlane(qw, 62);
-        const unsigned m = min(min(l0 + l1, l0 + q0), q0 + q1);
-        const unsigned light = __popcll(__ballot(lw <= m)) + __popcll(__ballot(qw <= m));
-        const unsigned taken = min(min(light, alive), 64u) & ~1u;
-        const K lk = (K)lw << 9 | li, qk = (K)qw << 9 | (NUM_SYMBOLS + qi);
-        K x = min(lk, qk);
-        half_cleaner<32>(x);
-        half_cleaner<16>(x);
-        half_cleaner<8>(x);
-        half_cleaner<4>(x);
-        half_cleaner<2>(x);
-        half_cleaner<1>(x);
+        K x = min(leaf_key[lh + lane], node_key[qh + 63 - lane]);
+        order_bitonic(x);
         const unsigned id = (unsigned)x & 511u, w = (unsigned)(x >> 9), sum = w + lane_xor<1>(w);
-        if (lane < taken) {
-            parent[id] = made + lane / 2;
-            if (!(lane & 1)) node_w[made + lane / 2] = sum;
-        }
-        const unsigned leaves = __popcll(__ballot(lane < taken && id < NUM_SYMBOLS));
+        const unsigned m = __builtin_amdgcn_readlane(sum, 0);
+        const unsigned taken = min((unsigned)__popcll(__ballot(w <= m)), alive) & ~1u, node = made + lane / 2;  // (two at least)
+        const bool in = lane < taken;
+        node_key[in ? node : TREE_PAD] = (K)sum << 9 | (NUM_SYMBOLS + node);
+        const unsigned leaves = __popcll(__ballot(id < NUM_SYMBOLS) & ~0ull >> (64 - taken));
+        parent[in ? id : 2 * NUM_SYMBOLS - 1] = node;
         lh += leaves;
         qh += taken - leaves;
         made += taken / 2;
         alive -= taken / 2;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // the nodes are read by other lanes
+        wave_lds_fence();  // the nodes are read by other lanes
     }
     return rounds;
 }
 
-// The chunk's code table and where its 4096-value runs start: one workgroup of 1024 a chunk.
+// The chunk's code table and where its 4096-value runs start: one workgroup of 1024 a chunk.  K holds weight << 9 | id: 32
+// bits for chunks below 2^23 values, else 64.
 //
 // Lengths as HuffmanTable::from_frequencies gives them (src/huffman.rs:35-150: two queues over the symbols sorted by
 // frequency, a leaf wins a tie; depths clamped to 12), and where the clamp over-subscribes the code the same repair
 // as table_that_decodes in pg_huffman.hip.
 //
-// One workgroup on its CU, so what counts is the chain of dependent steps, and code that runs once comes in at the pace of
-// the instruction cache's misses: loops, not unrolled bodies.  A chunk of 262144 normally distributed values, cycles: histograms
-// 2 k (read one row at a time 10 k), ranks 4.3 k, merges 14 k for 18 rounds (33 k by eight wavefronts with a binary search in
-// LDS and a barrier a round), depths 2 k, length repair 3.4 k (14 k with its second ranking, unrolled), the rest, which
-// runs beside the host's part, 10 k: 17 us where it was 31, and 278 for 360 of 3000 tokens of 8 x 128 in pieces of 512.
+// One workgroup on its CU, so what counts is the chain of dependent steps.  What one wavefront can do alone it does
+// without a barrier (merges, depths, counts, repair), exchanges are DPP moves with one instruction each to order a pair, and
+// the histograms stay in registers until the runs' bits are known.  A chunk of 262144 normally distributed values, cycles
+// (with every symbol compared with every other, exchanges by compare and select, queues that a round pads itself, and
+// branches around its stores): histograms 2.5 k, order 1.8 k (4.5 k), merges 7.4 k for 18 rounds (13.9 k), depths and counts 2 k, repair 1.5 k
+// (3.2 k), codes and runs 2 k (6 k), decode table 0.8 k (2 k): 9.8 us where it was 15.9; 16384 values 8.6 (13.0).
+constexpr unsigned KEPT_ROWS = 4;  // histograms a wavefront keeps: 16 wavefronts, so all of a chunk of up to 64 of them
+template <class K>
 __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsigned long long *host_bits) {
+    constexpr K NONE = ~(K)0;
     __shared__ __attribute__((aligned(16))) unsigned freq[NUM_SYMBOLS];
-    __shared__ unsigned rank_up[NUM_SYMBOLS], rank_down[NUM_SYMBOLS];  // by symbol; by place in the ascending order
-    __shared__ unsigned leaf_w[TREE_PAD], node_w[TREE_PAD];
-    __shared__ uint8_t leaf_sym[NUM_SYMBOLS];
+    __shared__ K order[2][NUM_SYMBOLS];
+    __shared__ unsigned rank_down[NUM_SYMBOLS];  // by place in the ascending order
+    __shared__ K leaf_key[TREE_PAD], node_key[TREE_PAD + 1];
+    __shared__ unsigned leaf_w[NUM_SYMBOLS];
+    __shared__ uint8_t leaf_sym[NUM_SYMBOLS], leaf_len[NUM_SYMBOLS];
     __shared__ unsigned parent[2 * NUM_SYMBOLS];  // of the leaves (by ascending frequency), then of the nodes
-    __shared__ unsigned up_tree[2][NUM_SYMBOLS];  // of the nodes: levels << 16 | ancestor
-    __shared__ unsigned cnt[16], first_code[16], limit[16], offset[16], lane_cnt[4][16];
+    __shared__ unsigned up_tree[NUM_SYMBOLS];     // of the nodes: levels << 16 | ancestor
+    __shared__ __attribute__((aligned(16))) unsigned cnt[16], first_code[16], limit[16], offset[16];
+    __shared__ unsigned lane_cnt[4][16];
     __shared__ __attribute__((aligned(16))) uint8_t bl[NUM_SYMBOLS];
     __shared__ uint8_t by_len[NUM_SYMBOLS];
-    __shared__ unsigned over, nrounds, wsum[16];
+    __shared__ unsigned over, wsum[16];
     __shared__ unsigned run_bits[1024];
-    __shared__ unsigned long long wave_bits[4];
     const unsigned c = blockIdx.x, t = threadIdx.x, s = t & 255, p = t >> 8;
     const unsigned lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const uint16_t *hist = b.hist + (size_t)c * b.nwg * NUM_SYMBOLS;
+    const uint2 *rows = reinterpret_cast<const uint2 *>(b.hist + (size_t)c * b.nwg * NUM_SYMBOLS);  // four counts of 16 bits
+    const bool kept = b.nwg <= 16 * KEPT_ROWS;
 
-    if (t < 16) cnt[t] = 0;
+    // a wavefront adds up every sixteenth row, four rows in flight
+    uint2 h[KEPT_ROWS];
+#pragma unroll
+    for (unsigned k = 0; k < KEPT_ROWS; ++k) h[k] = wave + 16 * k < b.nwg ? rows[(size_t)(wave + 16 * k) * 64 + lane] : uint2{0, 0};
+    if (t < 16) {
+        cnt[t] = 0;
+        limit[t] = ~0u;
+    }
     if (p == 0) {
         freq[s] = ~0u;  // (kept less one: what is not in use then comes behind all others)
-        rank_up[s] = 0;
         bl[s] = 0;
     }
+    if (t < TREE_PAD) leaf_key[t] = node_key[t] = NONE;
     __syncthreads();
-    {   // a wavefront adds up every sixteenth row, four rows in flight
+    {
         unsigned sum[4] = {0, 0, 0, 0};
-        const ushort4 *rows = reinterpret_cast<const ushort4 *>(hist);
-        unsigned i = wave;
-        for (; i + 48 < b.nwg; i += 64) {
-            ushort4 h[4];
+        for (unsigned i = wave;;) {
 #pragma unroll
-            for (unsigned k = 0; k < 4; ++k) h[k] = rows[(size_t)(i + 16 * k) * 64 + lane];
+            for (unsigned k = 0; k < KEPT_ROWS; ++k) { sum[0] += h[k].x & 0xFFFFu; sum[1] += h[k].x >> 16; sum[2] += h[k].y & 0xFFFFu; sum[3] += h[k].y >> 16; }
+            i += 16 * KEPT_ROWS;
+            if (i >= b.nwg) break;
 #pragma unroll
-            for (unsigned k = 0; k < 4; ++k) { sum[0] += h[k].x; sum[1] += h[k].y; sum[2] += h[k].z; sum[3] += h[k].w; }
-        }
-        for (; i < b.nwg; i += 16) {
-            const ushort4 h = rows[(size_t)i * 64 + lane];
-            sum[0] += h.x; sum[1] += h.y; sum[2] += h.z; sum[3] += h.w;
+            for (unsigned k = 0; k < KEPT_ROWS; ++k) h[k] = i + 16 * k < b.nwg ? rows[(size_t)(i + 16 * k) * 64 + lane] : uint2{0, 0};
         }
         if (wave < b.nwg)
 #pragma unroll
             for (unsigned k = 0; k < 4; ++k) atomicAdd(&freq[4 * lane + k], sum[k]);
     }
     __syncthreads();
-    // symbols in order of frequency, ties by symbol: o comes before s if its weight is below f, or below f + 1 where o < s,
-    // which is one and the same for all of a wavefront's symbols unless o is among them
-    const unsigned f = freq[s] + 1;
+    // Symbols in order of frequency, ties by symbol: four wavefronts put 64 each in order, then runs of 128 and 256 meet their
+    // mirror image through LDS.  Place t of the ascending order ends up with thread t.
     unsigned n = 0;  // symbols in use
-    {
-        const unsigned block = wave & 3, from = wave >> 2;
 #pragma unroll
-        for (unsigned k = 0; k < 4; ++k) n += __popcll(__ballot(freq[64 * k + lane] != ~0u));
-        unsigned up = 0;
-        if (block != from) {
-            const unsigned below = f - (from < block ? 0u : 1u);
-#pragma unroll 4
-            for (unsigned k = 0; k < 64; k += 4) {
-                const uint4 w = *reinterpret_cast<const uint4 *>(freq + from * 64 + k);
-                up += (w.x < below) + (w.y < below) + (w.z < below) + (w.w < below);
-            }
-        } else {
-#pragma unroll 4
-            for (unsigned k = 0; k < 64; k += 4) {
-                const uint4 w = *reinterpret_cast<const uint4 *>(freq + from * 64 + k);
-                up += (w.x < f - (k < lane ? 0u : 1u)) + (w.y < f - (k + 1 < lane ? 0u : 1u)) + (w.z < f - (k + 2 < lane ? 0u : 1u)) +
-                      (w.w < f - (k + 3 < lane ? 0u : 1u));
+    for (unsigned k = 0; k < 4; ++k) n += __popcll(__ballot(freq[64 * k + lane] != ~0u));
+    {
+        const unsigned f = freq[s] + 1;
+        K x = f ? (K)f << 8 | s : NONE;
+        if (p == 0) {
+            order_wave(x);
+            order[0][t] = x;
+        }
+        __syncthreads();
+        if (p == 0) {
+            x = end_of(x, order[0][t ^ 127], t & 64 ? ~0u : 0u);
+            order_bitonic(x);
+            order[1][t] = x;
+        }
+        __syncthreads();
+        if (p == 0) {
+            x = end_of(x, order[1][t ^ 255], t & 128 ? ~0u : 0u);
+            order[0][t] = x;
+        }
+        __syncthreads();
+        if (p == 0) {
+            x = end_of(x, order[0][t ^ 64], t & 64 ? ~0u : 0u);
+            order_bitonic(x);
+            if (t < n) {
+                leaf_w[t] = (unsigned)(x >> 8);
+                leaf_key[t] = x >> 8 << 9 | t;
+                leaf_sym[t] = (uint8_t)x;
             }
         }
-        if (f > 0) atomicAdd(&rank_up[s], up);
-    }
-    __syncthreads();
-    if (p == 0 && f > 0) {
-        leaf_w[rank_up[s]] = f;
-        leaf_sym[rank_up[s]] = (uint8_t)s;
     }
     __syncthreads();
     if (wave == 0) {
-        const unsigned r = b.total < (1u << 23) ? merge_trees<unsigned>(n, leaf_w, node_w, parent) : merge_trees<unsigned long long>(n, leaf_w, node_w, parent);
-        if (t == 0) nrounds = r;
-    } else if (wave >= 4 && wave < 8) {  // meanwhile the descending order, ties by symbol
-        const unsigned i = t - 256;
-        if (i < n) {
-            const unsigned w = leaf_w[i];
-            unsigned lo = 0, hi = 0;  // leaves below w, and of at most w
-#pragma unroll 1
-            for (unsigned step = 256; step > 0; step >>= 1) {
-                if (lo + step <= n && leaf_w[lo + step - 1] < w) lo += step;
-                if (hi + step <= n && leaf_w[hi + step - 1] <= w) hi += step;
-            }
-            rank_down[i] = n - hi + i - lo;
+        const unsigned rounds = merge_trees<K>(n, leaf_key, node_key, parent);
+        // the nodes' levels below the root: everyone takes over its ancestor's way up (a round adds at most one level)
+        unsigned up[4];
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k) {
+            const unsigned node = 64 * k + lane, of = parent[NUM_SYMBOLS + node];
+            up[k] = node + 2 < n ? 1u << 16 | of : node;
+            up_tree[node] = up[k];
         }
-    }
-    __syncthreads();
-    const unsigned rounds = nrounds;
-    unsigned mine = t;
-    if (t < NUM_SYMBOLS) {
-        const bool root = n < 2 || t >= n - 2;
-        up_tree[0][t] = mine = root ? t : 1u << 16 | parent[NUM_SYMBOLS + t];
-    }
-    __syncthreads();
-    unsigned last = 0;
-#pragma unroll 1
-    for (unsigned reach = 1; reach < rounds; reach *= 2) {  // (a round adds at most one level)
-        if (t < NUM_SYMBOLS) {
-            const unsigned a = up_tree[last][mine & 0xFFFFu];
-            up_tree[last ^ 1][t] = mine = (mine & ~0xFFFFu) + a;
+        for (unsigned reach = 1; reach < rounds; reach *= 2) {
+            wave_lds_fence();
+            unsigned a[4];
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) a[k] = up_tree[up[k] & 0xFFFFu];
+            wave_lds_fence();
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) up_tree[64 * k + lane] = up[k] = (up[k] & ~0xFFFFu) + a[k];
         }
-        last ^= 1;
-        __syncthreads();
-    }
-    unsigned len = 0;  // of leaf t
-    if (t < n) {
-        len = n < 2 ? 1u : min((up_tree[last][parent[t]] >> 16) + 1u, (unsigned)KV_MAX_BITS);
-        atomicAdd(&cnt[len], 1u);
-    }
-    __syncthreads();
-    if (wave == 0) {  // the counts of the twelve lengths: lane l holds cn[l]
-        unsigned cn = lane >= 1 && lane <= KV_MAX_BITS ? cnt[lane] : 0u;
+        wave_lds_fence();
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k) {
+            const unsigned leaf = 64 * k + lane, of = parent[leaf], levels = up_tree[leaf < n && n > 1 ? of : 0] >> 16;
+            const unsigned len = leaf >= n ? 0u : n < 2 ? 1u : min(levels + 1u, (unsigned)KV_MAX_BITS);
+            leaf_len[leaf] = (uint8_t)len;
+            atomicAdd(&cnt[len], 1u);
+        }
+        wave_lds_fence();
+        unsigned cn = lane >= 1 && lane <= KV_MAX_BITS ? cnt[lane] : 0u;  // lane l holds the number of codes of length l
         auto get = [&](int l) { return (unsigned)__builtin_amdgcn_readlane(cn, l); };
         auto add = [&](int l, unsigned x) { cn += lane == (unsigned)l ? x : 0u; };
         int excess = pg_wave_sum_i32((int)(cn * (lane <= KV_MAX_BITS ? KV_LUT >> lane : 0))) - KV_LUT;  // of the Kraft sum, in 1 / 4096
@@ -404,12 +422,16 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
             }
             unsigned slack = (unsigned)-excess;  // and what is left goes to the most frequent symbols
             const unsigned all = cn;
+            unsigned from = 1;
 #pragma unroll 1
-            for (int from = 2; from <= KV_MAX_BITS && slack > 0; ++from) {
+            for (;;) {  // the next length with symbols that the slack can shorten
+                const unsigned long long can = __ballot(lane > from && lane <= KV_MAX_BITS && all > 0 && (unsigned)(KV_LUT >> (lane & 15)) <= slack);
+                if (!can) break;
+                from = (unsigned)__ffsll((unsigned long long)can) - 1;
                 unsigned had = (unsigned)__builtin_amdgcn_readlane(all, from);
 #pragma unroll 1
                 for (; had > 0 && (unsigned)(KV_LUT >> from) <= slack; --had) {
-                    int to = from;
+                    unsigned to = from;
 #pragma unroll 1
                     for (; to > 1 && (unsigned)(KV_LUT >> to) <= slack; --to) slack -= KV_LUT >> to;
                     add(from, ~0u);
@@ -430,83 +452,125 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
             }
         }
         if (lane == 0) over = too_many;
+    } else if (wave >= 4 && wave < 8) {  // meanwhile the descending order, ties by symbol
+        const unsigned i = t - 256;
+        if (i < n) {
+            const unsigned w = leaf_w[i];
+            unsigned lo = 0, hi = 0;  // leaves below w, and of at most w
+#pragma unroll 1
+            for (unsigned step = 256; step > 0; step >>= 1) {
+                if (lo + step <= n && leaf_w[lo + step - 1] < w) lo += step;
+                if (hi + step <= n && leaf_w[hi + step - 1] <= w) hi += step;
+            }
+            rank_down[i] = n - hi + i - lo;
+        }
     }
     __syncthreads();
-    if (p == 0) {
-        if (over && t < n) {  // the repaired lengths go out again, shortest to most frequent (ties: lower symbol first)
+    if (t < n) {
+        unsigned len = leaf_len[t];
+        if (over) {  // the repaired lengths go out again, shortest to most frequent (ties: lower symbol first)
             const unsigned down = rank_down[t];
             len = 1;
-#pragma unroll 1
+#pragma unroll
             for (int l = 2; l <= KV_MAX_BITS; ++l) len += offset[l] <= down ? 1 : 0;
         }
-        if (t < n) bl[leaf_sym[t]] = (uint8_t)len;
-        const unsigned long long bits = t < n ? (unsigned long long)leaf_w[t] * len : 0ull;
-        const unsigned lo = (unsigned)pg_wave_sum_i32((int)(bits & 0xFFFFFFull)), hi = (unsigned)pg_wave_sum_i32((int)(bits >> 24));
-        if (lane == 0) wave_bits[wave] = ((unsigned long long)hi << 24) + lo;
+        bl[leaf_sym[t]] = (uint8_t)len;
     }
     __syncthreads();
-    // The stream's bits go to the host as soon as the lengths are known: it makes room and launches the encoder while the
-    // tables and start bits are written.
-    if (t == 1023)  // (0 = not there yet)
-        __hip_atomic_store(host_bits + c, wave_bits[0] + wave_bits[1] + wave_bits[2] + wave_bits[3] + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     // the symbol's place among those of its length
-    unsigned before = 0;
+    unsigned before = 0, len = 0;
     if (p == 0) {
         len = bl[s];
-#pragma unroll 1
+        unsigned of_len = 0;  // lane l: symbols of length l
+#pragma unroll
         for (unsigned l = 1; l <= KV_MAX_BITS; ++l) {
             const unsigned long long m = __ballot(len == l);
-            if (len == l) before = __popcll(m & ((1ull << lane) - 1));
-            if (lane == 0) lane_cnt[wave][l] = __popcll(m);
+            if (len == l) before = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+            if (lane == l) of_len = __popcll(m);
         }
+        if (lane < 16) lane_cnt[wave][lane] = of_len;
+    }
+    const unsigned lens = reinterpret_cast<const unsigned *>(bl)[lane];
+    const unsigned lens_lo = (lens & 255u) | (lens & 0xFF00u) << 8, lens_hi = (lens >> 16 & 255u) | (lens & 0xFF000000u) >> 8;
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    auto u2 = [](unsigned v) { return __builtin_bit_cast(u16x2, v); };
+    auto bits_of = [&](uint2 v) {
+        return (unsigned)pg_wave_sum_i32((int)__builtin_amdgcn_udot2(u2(v.x), u2(lens_lo), __builtin_amdgcn_udot2(u2(v.y), u2(lens_hi), 0u, false), false));
+    };
+    unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
+    if (kept) {
+#pragma unroll
+        for (unsigned k = 0; k < KEPT_ROWS; ++k)
+            if (wave + 16 * k < b.nwg) {
+                const unsigned bits = bits_of(h[k]);
+                if (lane == 0) run_bits[wave + 16 * k] = bits;
+            }
     }
     __syncthreads();
     if (p == 0) {
         unsigned e = 0;
         if (len) {
-            for (unsigned w = 0; w < wave; ++w) before += lane_cnt[w][len];
+#pragma unroll
+            for (unsigned w = 0; w < 3; ++w) before += w < wave ? lane_cnt[w][len] : 0u;
             e = len << 16 | (first_code[len] + before);
             by_len[offset[len] + before] = (uint8_t)s;
         }
         b.codes[(size_t)c * NUM_SYMBOLS + s] = e;
     }
+    // where the runs start, and the stream's bits
+    unsigned long long run = 0;
+    if (kept) {
+        if (wave == 4) {
+            const unsigned v = lane < b.nwg ? run_bits[lane] : 0u, incl = wave_scan(v);
+            if (lane < b.nwg) wg_bit[lane] = incl - v;
+            run = (unsigned)__builtin_amdgcn_readlane(incl, 63);
+            if (lane == 0) wg_bit[b.nwg] = run;
+        }
+    } else {
+        for (unsigned at = 0; at < b.nwg; at += 1024) {
+            for (unsigned i = at + wave; i < min(at + 1024u, b.nwg); i += 16) {
+                const unsigned bits = bits_of(rows[(size_t)i * 64 + lane]);
+                if (lane == 0) run_bits[i - at] = bits;
+            }
+            __syncthreads();
+            const unsigned v = at + t < b.nwg ? run_bits[t] : 0u;
+            const unsigned incl = wave_scan(v);
+            if (lane == 63) wsum[wave] = incl;
+            __syncthreads();
+            unsigned long long pre = run;
+            for (unsigned w = 0; w < wave; ++w) pre += wsum[w];
+            if (at + t < b.nwg) wg_bit[at + t] = pre + incl - v;
+            for (unsigned w = 0; w < 16; ++w) run += wsum[w];
+            __syncthreads();
+        }
+        if (t == 256) wg_bit[b.nwg] = run;
+    }
+    // The stream's bits go to the host as soon as they are known: it makes room and launches the encoder meanwhile.
+    const bool tells = t == 256;
     __syncthreads();
+    if (tells) __hip_atomic_store(host_bits + c, run + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // (0 = not there yet)
     {   // decode table, four entries a thread: length << 8 | symbol; codes nobody has decode as (length 0, value 0)
+        const unsigned x = t * 4;
+        unsigned l = 1;  // (the limits ascend)
+#pragma unroll
+        for (int i = 1; i <= KV_MAX_BITS; ++i) l += x >= limit[i] ? 1 : 0;
         ushort4 e;
         uint16_t *ev = reinterpret_cast<uint16_t *>(&e);
-#pragma unroll
-        for (unsigned k = 0; k < 4; ++k) {
-            const unsigned x = t * 4 + k;
-            unsigned l = 1;  // (the limits ascend)
-#pragma unroll
-            for (int i = 1; i <= KV_MAX_BITS; ++i) l += x >= limit[i] ? 1 : 0;
+        auto entry = [&](unsigned x, unsigned l) {
             const unsigned at = l > KV_MAX_BITS ? 0 : offset[l] + (x >> (KV_MAX_BITS - l)) - first_code[l];
-            ev[k] = l > KV_MAX_BITS ? (uint16_t)128 : (uint16_t)(l << 8 | by_len[at]);
+            return l > KV_MAX_BITS ? (uint16_t)128 : (uint16_t)(l << 8 | by_len[at]);
+        };
+        if (l <= KV_MAX_BITS - 2 || l > KV_MAX_BITS) {  // one code for the four, or none
+            ev[0] = ev[1] = ev[2] = ev[3] = entry(x, l);
+        } else {
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) {
+                while (l <= KV_MAX_BITS && x + k >= limit[l]) ++l;
+                ev[k] = entry(x + k, l);
+            }
         }
         reinterpret_cast<ushort4 *>(b.lut + (size_t)c * KV_LUT)[t] = e;
     }
-    // bits of every run of 4096 values, and their running sum
-    const uchar4 lens = reinterpret_cast<const uchar4 *>(bl)[lane];
-    unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
-    unsigned long long run = 0;
-    for (unsigned at = 0; at < b.nwg; at += 1024) {
-        for (unsigned i = at + wave; i < min(at + 1024u, b.nwg); i += 16) {
-            const ushort4 h = reinterpret_cast<const ushort4 *>(hist + (size_t)i * NUM_SYMBOLS)[lane];
-            const int bits = pg_wave_sum_i32((int)(h.x * lens.x + h.y * lens.y + h.z * lens.z + h.w * lens.w));
-            if (lane == 0) run_bits[i - at] = (unsigned)bits;
-        }
-        __syncthreads();
-        const unsigned v = at + t < b.nwg ? run_bits[t] : 0u;
-        const unsigned incl = wave_scan(v);
-        if (lane == 63) wsum[wave] = incl;
-        __syncthreads();
-        unsigned long long pre = run;
-        for (unsigned w = 0; w < wave; ++w) pre += wsum[w];
-        if (at + t < b.nwg) wg_bit[at + t] = pre + incl - v;
-        for (unsigned w = 0; w < 16; ++w) run += wsum[w];
-        __syncthreads();
-    }
-    if (t == 0) wg_bit[b.nwg] = run;
 }
 
 // Where up to KV_PLACES chunks of a batch, from number `first` on, are written to.
@@ -914,7 +978,7 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
                          dim3(b.splits * b.heads, b.count + (unsigned)sides * in.parts), dim3(KV_WG), 0, b, in));
         if (rows) rows->written = true;
         PG_TRY(pg_launch(ctx, "huffman_kv_quant", kv_quant_hist_kernel, dim3(b.nwg, b.count), dim3(KV_WG), 0, b, (int)vec));
-        PG_TRY(pg_launch(ctx, "huffman_kv_table", kv_table_kernel, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
+        PG_TRY(pg_launch(ctx, "huffman_kv_table", b.total < (1u << 23) ? kv_table_kernel<unsigned> : kv_table_kernel<unsigned long long>, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
         const kv_layout lay(num_heads, total, true);
         PG_TRY(wait_for_words(ctx, sizes, n));
         size_t bytes = 0;

@@ -213,6 +213,7 @@ def test_cache_on_device_pointers(ctx, orc):
     (1, 1, 4095, 2), (1, 1, 4096, 2), (1, 1, 4097, 2),     # a histogram run of 4096 values, one less, one more
     (1, 4, 4096, 1), (1, 4, 4097, 1), (3, 1, 5462, 1),     # a decoder workgroup of 16384, and 2 (with a head cut by the runs) past it
     (1, 64, 1, 45), (5, 3, 2, 40),                         # more chunks in one batch than one encoder launch places
+    (1, 1, 262144, 1), (1, 1, 262145, 1),                  # 64 histograms, which the table kernel keeps, and one more
     (2, 2, 70000, 1),                                      # 69 runs of a head's values, several rounds of the maximum
 ])
 @pytest.mark.parametrize("kind", ["normal", "steep", "two"])
