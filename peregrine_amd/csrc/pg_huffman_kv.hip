@@ -5,8 +5,8 @@
 //   HuffmanKVCache::compress_chunk / decompress_chunk                             reference: src/huffman.rs:612-680
 //   HuffmanKVCache::len / get_kv                                                  reference: src/huffman.rs:683-724
 //
-// Everything is device work here, and all the chunks that one append cuts (both sides) are one batch of four
-// launches: the heads' absolute maxima; the int8 values with a histogram per 4096 of them; the code table, one
+// Everything is device work here, and all the chunks that one append cuts (both sides) are one batch of three or four
+// launches: the heads' absolute maxima and the int8 values with a histogram per 4096 of them (one launch, or for large batches two); the code table, one
 // workgroup a chunk, which also turns the small histograms into the bit at which each 4096 values start; and the
 // encoder.  The host takes part once per batch: it learns the coded sizes (words that the table kernel stores in
 // pinned memory), allocates exactly that much and launches the encoder.  A batch was 10 launches, 12 copies and 8
@@ -80,6 +80,25 @@ struct kv_incoming {
     unsigned parts;  // times as many workgroups per (side, head) as a chunk's head has
 };
 
+// Lane exchange by DPP: the value of lane ^ D.
+template <int D> __device__ __forceinline__ unsigned lane_xor(unsigned v) {
+    if constexpr (D == 1) return __builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // quad_perm 1 0 3 2
+    else if constexpr (D == 2) return __builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2 3 0 1
+    else if constexpr (D == 3) return __builtin_amdgcn_mov_dpp((int)v, 0x1B, 0xF, 0xF, true);   // quad_perm 3 2 1 0
+    else if constexpr (D == 7) return __builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+    else if constexpr (D == 15) return __builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true); // row_mirror
+    else if constexpr (D == 4) return lane_xor<3>(lane_xor<7>(v));
+    else if constexpr (D == 8) return __builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);  // row_ror 8
+    else if constexpr (D == 31) return lane_xor<16>(lane_xor<15>(v));
+    else if constexpr (D == 63) return lane_xor<32>(lane_xor<31>(v));
+    else {
+        const auto two = D == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false) : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return threadIdx.x & D ? two[0] : two[1];
+    }
+}
+template <int D> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+    return (unsigned long long)lane_xor<D>((unsigned)(v >> 32)) << 32 | lane_xor<D>((unsigned)v);
+}
 // Largest |v| of every head (NaN ignored, as f32::max does), one value per split; and the incoming rows' copy.  Grid
 // (heads * splits, chunks + sides * parts).  As two launches the copy took 4 us of an append's 43.
 template <class V>
@@ -164,25 +183,114 @@ __global__ __launch_bounds__(KV_WG) void kv_quant_hist_kernel(const kv_batch b, 
     b.hist[((size_t)c * b.nwg + blockIdx.x) * NUM_SYMBOLS + t] = (uint16_t)(lh[0][t] + lh[1][t] + lh[2][t] + lh[3][t]);
 }
 
-// Lane exchange for the sorts below: the value of lane ^ D.
-template <int D> __device__ __forceinline__ unsigned lane_xor(unsigned v) {
-    if constexpr (D == 1) return __builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // quad_perm 1 0 3 2
-    else if constexpr (D == 2) return __builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2 3 0 1
-    else if constexpr (D == 3) return __builtin_amdgcn_mov_dpp((int)v, 0x1B, 0xF, 0xF, true);   // quad_perm 3 2 1 0
-    else if constexpr (D == 7) return __builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
-    else if constexpr (D == 15) return __builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true); // row_mirror
-    else if constexpr (D == 4) return lane_xor<3>(lane_xor<7>(v));
-    else if constexpr (D == 8) return __builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);  // row_ror 8
-    else if constexpr (D == 31) return lane_xor<16>(lane_xor<15>(v));
-    else if constexpr (D == 63) return lane_xor<32>(lane_xor<31>(v));
-    else {
-        const auto two = D == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false) : __builtin_amdgcn_permlane32_swap(v, v, false, false);
-        return threadIdx.x & D ? two[0] : two[1];
+// Both of the above in one launch, for heads of which every workgroup can afford to look at the whole: a workgroup takes
+// 4096 values, finds the maximum of each head that they meet by itself (what the workgroups of a head read in common
+// comes out of the L2), quantises its values and counts them.  New rows are read where the caller has them; workgroups behind
+// the chunks' write them to the window.  Grid 8 * ceil(nwg / 8) * chunks + sides * heads * parts.
+//
+// Taken while the repeated reads cost less than a launch: us, both launches : this, by chunks of heads x values: 2 x 4 x 4096
+// 7.0 : 4.0; 4 x 8 x 32768 7.2 : 5.6; 2 x 8 x 49152 7.4 : 6.2; 2 x 8 x 65536 7.3 : 7.0; but 8 x 8 x 32768 7.8 : 8.0, 8 x 32 x 16384 9.7 : 11.4,
+// 2 x 2 x 262144 7.7 : 15.8.  (Runs dealt to the XCDs one by one: 8 x 8 x 32768 13.1.)
+constexpr unsigned WHOLE_WG = 1024;
+constexpr size_t WHOLE_HEAD = 65536, WHOLE_READS = 12u << 20;  // values of a head, and that all workgroups read together, at the most
+template <class V>
+__global__ __launch_bounds__(WHOLE_WG) __attribute__((amdgpu_waves_per_eu(8, 8))) void kv_whole_kernel(const kv_batch b, const kv_incoming in) {
+    constexpr unsigned VN = sizeof(V) / 4, PER = ENC_PER_WG / WHOLE_WG / VN;
+    __shared__ unsigned lh[4][NUM_SYMBOLS];
+    __shared__ float sc[ENC_PER_WG];  // scales of the heads the workgroup meets (every value its own head at the most)
+    __shared__ unsigned red[2][WHOLE_WG / 64];
+    const unsigned t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const unsigned per_xcd = (b.nwg + 7) / 8;  // workgroup id % 8 = XCD: each takes consecutive runs, so that few of them read a head
+    if (blockIdx.x >= 8 * per_xcd * b.count) {
+        const unsigned g = blockIdx.x - 8 * per_xcd * b.count, row = g / in.parts, side = row / b.heads, h = row % b.heads;
+        const V *src = reinterpret_cast<const V *>(in.src[side] + (size_t)h * in.src_stride);
+        V *dst = reinterpret_cast<V *>(in.dst[side] + (size_t)h * in.dst_stride);
+        for (size_t i = (size_t)(g % in.parts) * WHOLE_WG + t; i < in.elems / VN; i += (size_t)in.parts * WHOLE_WG) dst[i] = src[i];
+        return;
     }
+    const unsigned c = blockIdx.x / (8 * per_xcd), run = (blockIdx.x & 7) * per_xcd + blockIdx.x / 8 % per_xcd, base = run * ENC_PER_WG;
+    if (run >= b.nwg) return;
+    const unsigned last = min(base + ENC_PER_WG, b.total) - 1, h0 = base / b.head_elems, h1 = last / b.head_elems;
+    const size_t at = (size_t)(c / b.sides) * b.chunk_step;  // of the head's first value in the window
+    const unsigned n = b.head_elems / VN, old = (unsigned)min((size_t)n, (in.from > at ? in.from - at : 0) / VN);
+    const size_t skip = at / VN - in.from / VN;  // of the incoming values, from window to incoming (wraps where the chunk starts in the window)
+    const float *src = in.src[c % b.sides];
+    auto load = [&](unsigned h, unsigned i) {
+        return i < old ? reinterpret_cast<const V *>(b.head(c, h))[i] : reinterpret_cast<const V *>(src + (size_t)h * in.src_stride)[skip + i];
+    };
+    V v[PER];
+#pragma unroll
+    for (unsigned j = 0; j < PER; ++j) {
+        const unsigned i = base + (j * WHOLE_WG + t) * VN, h = i / b.head_elems;
+        if (i < b.total) v[j] = load(h, (i - h * b.head_elems) / VN);
+    }
+    if (t < 4 * NUM_SYMBOLS) (&lh[0][0])[t] = 0;
+    // |v| of all but NaN is in order as bits
+    auto max_of = [&](unsigned h, unsigned from, unsigned step) {
+        float m = 0.0f;
+#pragma unroll 8
+        for (unsigned i = from; i < n; i += step) {
+            const V x = load(h, i);
+            const float *f = reinterpret_cast<const float *>(&x);
+#pragma unroll
+            for (unsigned k = 0; k < VN; ++k) m = fmaxf(m, fabsf(f[k]));
+        }
+        unsigned r = __float_as_uint(m);
+        r = max(r, lane_xor<1>(r));
+        r = max(r, lane_xor<2>(r));
+        r = max(r, lane_xor<4>(r));
+        r = max(r, lane_xor<8>(r));
+        r = max(r, lane_xor<16>(r));
+        return max(r, lane_xor<32>(r));
+    };
+    auto scale_is = [&](unsigned h, unsigned bits) {
+        const float m = __uint_as_float(bits), scale = (m == 0.0f) ? 1.0f : m / 127.0f;
+        sc[h - h0] = scale;
+        if (base <= h * b.head_elems) b.scales[(size_t)c * b.heads + h] = scale;  // the workgroup of the head's first value
+    };
+    if (b.head_elems >= 2048) {  // three heads at the most
+        for (unsigned h = h0; h <= h1; ++h) {
+            const unsigned r = max_of(h, t, WHOLE_WG);
+            if (lane == 0) red[(h - h0) & 1][wave] = r;
+            __syncthreads();
+            if (wave == 0) {
+                unsigned m = red[(h - h0) & 1][lane & 15];
+                m = max(m, lane_xor<1>(m));
+                m = max(m, lane_xor<2>(m));
+                m = max(m, lane_xor<4>(m));
+                m = max(m, lane_xor<8>(m));
+                if (lane == 0) scale_is(h, m);
+            }
+        }
+    } else {
+        for (unsigned h = h0 + wave; h <= h1; h += WHOLE_WG / 64) {
+            const unsigned r = max_of(h, lane, 64);
+            if (lane == 0) scale_is(h, r);
+        }
+    }
+    __syncthreads();
+    unsigned *mine = lh[wave & 3];
+    int8_t *q = b.q + (size_t)c * b.q_stride;
+#pragma unroll
+    for (unsigned j = 0; j < PER; ++j) {
+        const unsigned i = base + (j * WHOLE_WG + t) * VN;
+        if (i >= b.total) continue;
+        const float inv = 1.0f / sc[i / b.head_elems - h0];
+        const float *f = reinterpret_cast<const float *>(&v[j]);
+        unsigned four = 0;
+#pragma unroll
+        for (unsigned k = 0; k < VN; ++k) {
+            const int x = pg_quant_to_i8(f[k] * inv);
+            four |= (x & 255u) << (8 * k);
+            atomicAdd(mine + x + 128, 1u);
+        }
+        if (VN == 4) *reinterpret_cast<unsigned *>(q + i) = four;
+        else q[i] = (int8_t)four;
+    }
+    __syncthreads();
+    if (t < NUM_SYMBOLS) b.hist[((size_t)c * b.nwg + run) * NUM_SYMBOLS + t] = (uint16_t)(lh[0][t] + lh[1][t] + lh[2][t] + lh[3][t]);
 }
-template <int D> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
-    return (unsigned long long)lane_xor<D>((unsigned)(v >> 32)) << 32 | lane_xor<D>((unsigned)v);
-}
+
 // The smaller of both for end = 0, the larger for end = ~0: one instruction, their median with `end`.
 __device__ __forceinline__ unsigned end_of(unsigned x, unsigned o, unsigned end) { return max(min(x, o), min(max(x, o), end)); }
 __device__ __forceinline__ unsigned long long end_of(unsigned long long x, unsigned long long o, unsigned end) { return (end != 0) == (o > x) ? o : x; }
@@ -972,12 +1080,18 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
             in = rows->in;
             vec_in = vec && in.from % 4 == 0 && in.elems % 4 == 0 && in.src_stride % 4 == 0 && in.dst_stride % 4 == 0;
             for (size_t s = 0; s < 2; ++s) vec_in = vec_in && ((uintptr_t)in.src[s] | (uintptr_t)in.dst[s]) % 16 == 0;
-            in.parts = (unsigned)std::min<size_t>((in.elems + b.splits * ENC_PER_WG - 1) / (b.splits * ENC_PER_WG), KV_MAX_SPLITS);
         }
-        PG_TRY(pg_launch(ctx, "huffman_kv_absmax", vec_in ? kv_absmax_kernel<float4> : kv_absmax_kernel<float>,
-                         dim3(b.splits * b.heads, b.count + (unsigned)sides * in.parts), dim3(KV_WG), 0, b, in));
+        if (head_elems <= WHOLE_HEAD && n * nwg <= 2 * (size_t)ctx->num_cu && n * nwg * head_elems <= WHOLE_READS) {
+            in.parts = (unsigned)((in.elems + 4 * ENC_PER_WG - 1) / (4 * ENC_PER_WG));
+            PG_TRY(pg_launch(ctx, "huffman_kv_quant", vec_in ? kv_whole_kernel<float4> : kv_whole_kernel<float>,
+                             dim3((b.nwg + 7) / 8 * 8 * b.count + (unsigned)(sides * num_heads) * in.parts), dim3(WHOLE_WG), 0, b, in));
+        } else {
+            in.parts = (unsigned)std::min<size_t>((in.elems + b.splits * ENC_PER_WG - 1) / (b.splits * ENC_PER_WG), KV_MAX_SPLITS);
+            PG_TRY(pg_launch(ctx, "huffman_kv_absmax", vec_in ? kv_absmax_kernel<float4> : kv_absmax_kernel<float>,
+                             dim3(b.splits * b.heads, b.count + (unsigned)sides * in.parts), dim3(KV_WG), 0, b, in));
+            PG_TRY(pg_launch(ctx, "huffman_kv_quant", kv_quant_hist_kernel, dim3(b.nwg, b.count), dim3(KV_WG), 0, b, (int)vec));
+        }
         if (rows) rows->written = true;
-        PG_TRY(pg_launch(ctx, "huffman_kv_quant", kv_quant_hist_kernel, dim3(b.nwg, b.count), dim3(KV_WG), 0, b, (int)vec));
         PG_TRY(pg_launch(ctx, "huffman_kv_table", b.total < (1u << 23) ? kv_table_kernel<unsigned> : kv_table_kernel<unsigned long long>, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
         const kv_layout lay(num_heads, total, true);
         PG_TRY(wait_for_words(ctx, sizes, n));

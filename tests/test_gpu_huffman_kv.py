@@ -214,6 +214,9 @@ def test_cache_on_device_pointers(ctx, orc):
     (1, 4, 4096, 1), (1, 4, 4097, 1), (3, 1, 5462, 1),     # a decoder workgroup of 16384, and 2 (with a head cut by the runs) past it
     (1, 64, 1, 45), (5, 3, 2, 40),                         # more chunks in one batch than one encoder launch places
     (1, 1, 262144, 1), (1, 1, 262145, 1),                  # 64 histograms, which the table kernel keeps, and one more
+    (1, 1, 65536, 1), (1, 1, 65537, 1),                    # the longest head whose maximum every workgroup finds, and one more
+    (3, 1, 2047, 2), (3, 1, 2048, 2),                      # heads by a wavefront, and by the workgroup
+    (1, 1, 4096, 256), (1, 1, 4096, 257),                  # as many workgroups as take that route, and more
     (2, 2, 70000, 1),                                      # 69 runs of a head's values, several rounds of the maximum
 ])
 @pytest.mark.parametrize("kind", ["normal", "steep", "two"])
@@ -286,6 +289,8 @@ def test_tables_at_the_edges_of_the_merges(ctx, orc, kind, total):
     (2, 6, 4, 2, (1, 1, 1, 1, 3, 8), 0),             # whole quadruples in a chunk, not in the window's rows
     (1, 1, 1, 1, (1100, 3), 0),                      # more chunks than one batch takes
     (8, 128, 512, 256, (500, 500, 1100), 0),
+    (1, 2, 40000, 40000, (30000, 20000, 1), 0),      # heads that a launch of their own finds the maximum of
+    (1, 1, 70001, 70001, (30001, 50000), 0),
 ])
 def test_device_rows_are_written_with_the_maximum(ctx, orc, heads, hd, thr, chunk, appends, skew):
     """append_dev where it cuts chunks: the launch that finds the chunks' maxima also writes the new rows."""
