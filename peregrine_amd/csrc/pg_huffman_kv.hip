@@ -9,7 +9,8 @@
 // launches: the heads' absolute maxima and the int8 values with a histogram per 4096 of them (one launch, or for large batches two); the code table, one
 // workgroup a chunk, which also turns the small histograms into the bit at which each 4096 values start; and the
 // encoder.  The host takes part once per batch: it learns the coded sizes (words that the table kernel stores in
-// pinned memory), allocates exactly that much and launches the encoder.  A batch was 10 launches, 12 copies and 8
+// pinned memory); a cache's first batch gets exactly that much memory, later ones what the one before took and 1 / 64, and are
+// encoded a second time if they take more.  A batch was 10 launches, 12 copies and 8
 // waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
 // 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.25.
 //
@@ -686,6 +687,7 @@ constexpr unsigned KV_PLACES = 32;
 struct kv_places {
     unsigned first;
     char *at[KV_PLACES];
+    unsigned long long max_bits;  // that there is room for: a longer stream is not written
     // the window's rows that move to the front in the same launch (workgroups behind the chunks', which read the int8
     // values only): heads of both sides, `rest` values each, from `from` values on
     float *hot[2];
@@ -722,6 +724,7 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
     char *dst = places.at[blockIdx.y];
     const unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
     const unsigned long long first = wg_bit[g], last = wg_bit[g + 1], end = wg_bit[b.nwg];
+    if (end > places.max_bits) return;  // (the same for all of a chunk's workgroups)
     lc[t] = b.codes[(size_t)c * NUM_SYMBOLS + t];
     for (unsigned i = t; i < sizeof(words) / 4; i += KV_WG) words[i] = 0;
     const int8_t *q = b.q + (size_t)c * b.q_stride;
@@ -948,6 +951,7 @@ struct pg_huffman_kv_cache {
     pg_kv_cache *hot = nullptr;
     std::vector<pg_huffman_kv_chunk *> k_chunks, v_chunks;
     size_t compressed_len = 0, compress_threshold = 0, chunk_size = 0;
+    size_t expect = 0;  // bytes that a chunk's stream is expected to take (compress_batch)
     // The chunks' addresses on the device, key and value side in turn (written by the encoder).  An outgrown table
     // may still be read by work in flight and stays until the cache goes.
     pg_dev_block table_mem;
@@ -1037,8 +1041,11 @@ struct kv_rows {
 // compress_chunk of `count` chunks of one shape (none of them empty), chunk c being number c / sides of side c % sides:
 // head h of it starts at data[side] + number * chunk_step + h * head_stride.  Their addresses go to table_dev[0 ..) if given.
 // `rows` (if given) are still to be written to the window behind data[]: the first launch does.
+// `expect` (if given): room for streams of that many bytes is made and the encoder launched before their sizes are known, so that it
+// follows the table at once instead of 8 us later; a batch with a longer stream is encoded again once they are.  0 = wait
+// for the sizes first.  Set to what a batch like the last one needs and 1 / 64 more.
 static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t sides, size_t count, size_t chunk_step, size_t head_stride,
-                                size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift, kv_rows *rows,
+                                size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift, kv_rows *rows, size_t *expect,
                                 std::vector<std::unique_ptr<pg_huffman_kv_chunk>> &out) {
     const size_t head_elems = num_tokens * head_dim, total = num_heads * head_elems;
     const size_t nwg = (total + ENC_PER_WG - 1) / ENC_PER_WG;
@@ -1094,40 +1101,61 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         if (rows) rows->written = true;
         PG_TRY(pg_launch(ctx, "huffman_kv_table", b.total < (1u << 23) ? kv_table_kernel<unsigned> : kv_table_kernel<unsigned long long>, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
         const kv_layout lay(num_heads, total, true);
+        // the encoder, and with `again` unset the window's move: chunk c has room for bytes_of(c) of stream
+        auto encode = [&](auto bytes_of, bool again, std::shared_ptr<pg_dev_block> &block, std::vector<char *> &at) -> pg_status {
+            size_t bytes = 0, largest = 0;
+            for (size_t c = 0; c < n; ++c) {
+                bytes += lay.size(bytes_of(c));
+                largest = std::max<size_t>(largest, bytes_of(c));
+            }
+            block = std::make_shared<pg_dev_block>();
+            PG_TRY(block->alloc(ctx, bytes));
+            at.resize(n);
+            bytes = 0;
+            for (size_t c = 0; c < n; ++c) {
+                at[c] = static_cast<char *>(block->p) + bytes;
+                bytes += lay.size(bytes_of(c));
+            }
+            for (size_t c0 = 0; c0 < n; c0 += KV_PLACES) {
+                kv_places places;
+                places.first = (unsigned)c0;
+                places.max_bits = 8ull * largest;
+                const size_t here = std::min<size_t>(KV_PLACES, n - c0);
+                std::copy(at.begin() + c0, at.begin() + c0 + here, places.at);
+                size_t rows = 0;
+                if (shift && !again && first + c0 + here == count && shift->rest <= shift->from && here + sides * num_heads <= 65535) {  // (no row reads what it writes)
+                    places.hot[0] = shift->hot[0];
+                    places.hot[1] = shift->hot[1];
+                    places.hot_stride = shift->stride;
+                    places.from = shift->from;
+                    places.rest = shift->rest;
+                    rows = sides * num_heads;
+                    shift->done = true;
+                }
+                PG_TRY(pg_launch(ctx, "huffman_kv_encode", kv_encode_kernel, dim3(b.nwg, (unsigned)(here + rows)), dim3(KV_WG), 0, b, places,
+                                 table_dev ? table_dev + first : nullptr));
+            }
+            return PG_OK;
+        };
+        std::shared_ptr<pg_dev_block> block;
+        std::vector<char *> at;
+        const size_t room = expect ? *expect : 0;
+        if (room) PG_TRY(encode([&](size_t) { return room; }, false, block, at));
         PG_TRY(wait_for_words(ctx, sizes, n));
-        size_t bytes = 0;
-        for (size_t c = 0; c < n; ++c) bytes += lay.size((sizes[c] - 1 + 7) / 8);
-        auto block = std::make_shared<pg_dev_block>();
-        PG_TRY(block->alloc(ctx, bytes));
-        char *at = static_cast<char *>(block->p);
-        for (size_t c0 = 0; c0 < n; c0 += KV_PLACES) {
-            kv_places places;
-            places.first = (unsigned)c0;
-            const size_t here = std::min<size_t>(KV_PLACES, n - c0);
-            for (size_t c = c0; c < c0 + here; ++c) {
-                std::unique_ptr<pg_huffman_kv_chunk> ch(new (std::nothrow) pg_huffman_kv_chunk());
-                if (!ch) return pg_fail(PG_ENOMEM, "host allocation failed");
-                ch->num_tokens = num_tokens; ch->num_heads = num_heads; ch->head_dim = head_dim;
-                ch->block = block;
-                ch->dev = at;
-                ch->bytes = (size_t)((sizes[c] - 1 + 7) / 8);
-                ch->decodable = ch->indexed = true;
-                places.at[c - c0] = at;
-                at += lay.size(ch->bytes);
-                out.push_back(std::move(ch));
-            }
-            size_t rows = 0;
-            if (shift && first + c0 + here == count && shift->rest <= shift->from && here + sides * num_heads <= 65535) {  // (no row reads what it writes)
-                places.hot[0] = shift->hot[0];
-                places.hot[1] = shift->hot[1];
-                places.hot_stride = shift->stride;
-                places.from = shift->from;
-                places.rest = shift->rest;
-                rows = sides * num_heads;
-                shift->done = true;
-            }
-            PG_TRY(pg_launch(ctx, "huffman_kv_encode", kv_encode_kernel, dim3(b.nwg, (unsigned)(here + rows)), dim3(KV_WG), 0, b, places,
-                             table_dev ? table_dev + first : nullptr));
+        auto stream_bytes = [&](size_t c) { return (size_t)((sizes[c] - 1 + 7) / 8); };
+        size_t longest = 0;
+        for (size_t c = 0; c < n; ++c) longest = std::max(longest, stream_bytes(c));
+        if (longest > room) PG_TRY(encode(stream_bytes, room != 0, block, at));
+        if (expect) *expect = longest + longest / 64;
+        for (size_t c = 0; c < n; ++c) {
+            std::unique_ptr<pg_huffman_kv_chunk> ch(new (std::nothrow) pg_huffman_kv_chunk());
+            if (!ch) return pg_fail(PG_ENOMEM, "host allocation failed");
+            ch->num_tokens = num_tokens; ch->num_heads = num_heads; ch->head_dim = head_dim;
+            ch->block = block;
+            ch->dev = at[c];
+            ch->bytes = stream_bytes(c);
+            ch->decodable = ch->indexed = true;
+            out.push_back(std::move(ch));
         }
     }
     return PG_OK;
@@ -1149,7 +1177,7 @@ static pg_status compress_dev(pg_ctx *ctx, const float *data, size_t head_stride
         return PG_OK;
     }
     std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
-    PG_TRY(compress_batch(ctx, &data, 1, 1, 0, head_stride, num_tokens, num_heads, head_dim, nullptr, nullptr, nullptr, made));
+    PG_TRY(compress_batch(ctx, &data, 1, 1, 0, head_stride, num_tokens, num_heads, head_dim, nullptr, nullptr, nullptr, nullptr, made));
     *out = made[0].release();
     return PG_OK;
 }
@@ -1406,7 +1434,7 @@ static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c, kv_rows *rows
     const float *data[2] = {hot->k, hot->v};
     std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
     kv_shift shift{{hot->k, hot->v}, stride, chunks * tokens * hd, (hot->len - chunks * tokens) * hd};
-    const pg_status st = compress_batch(ctx, data, 2, 2 * chunks, tokens * hd, stride, tokens, heads, hd, c->table + c->k_chunks.size() * 2, &shift, rows, made);
+    const pg_status st = compress_batch(ctx, data, 2, 2 * chunks, tokens * hd, stride, tokens, heads, hd, c->table + c->k_chunks.size() * 2, &shift, rows, &c->expect, made);
     size_t done = 0;
     for (size_t i = 0; i + 1 < made.size(); i += 2) {
         c->k_chunks.push_back(made[i].release());

@@ -307,3 +307,26 @@ def test_device_rows_are_written_with_the_maximum(ctx, orc, heads, hd, thr, chun
         assert (c.len(), c.compressed_len) == (o.len, o.compressed_len)
         for got, want in zip(c.get_kv(), o.get_kv()):
             assert (got.view(np.uint32) == want.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("heads,hd,thr,chunk", [(2, 16, 24, 16), (3, 7, 5, 5), (4, 64, 96, 64)])
+def test_streams_longer_than_the_last(ctx, orc, heads, hd, thr, chunk):
+    """Batches whose streams take more than the one before led to expect are coded twice, the window moved once; up to
+    two batches of more chunks than one encoder launch places."""
+    from peregrine_amd import huffman
+    say(f"huffman kv lengthening streams heads={heads} head_dim={hd} threshold={thr} chunk={chunk}")
+    rng = np.random.default_rng(heads)
+    c, o = huffman.HuffmanKVCache(heads, hd, thr, chunk, ctx), orc.HuffmanKVCache(heads, hd, thr, chunk)
+    for kind, n in (("two", 3 * chunk), ("two", chunk + 1), ("normal", 2 * chunk), ("two", chunk), ("normal", chunk - 1), ("few", 40 * chunk), ("normal", 41 * chunk)):
+        if kind == "normal":
+            k, v = (rng.standard_normal((heads, n, hd)).astype(np.float32) for _ in range(2))
+        else:
+            k, v = (rng.integers(0, 2 if kind == "two" else 9, (heads, n, hd)).astype(np.float32) for _ in range(2))
+        c.append(k, v, n)
+        o.append(k, v, n)
+        assert (c.len(), c.compressed_len, c.hot_len) == (o.len, o.compressed_len, o.hot_len)
+        for got, want in zip(c.get_kv(), o.get_kv()):
+            assert (got.view(np.uint32) == want.view(np.uint32)).all()
+    for side, chunks in ((0, c.k_chunks), (1, c.v_chunks)):
+        for i, ch in enumerate(chunks):
+            _same_chunk(ch, o.chunk(side, i)[:3])
