@@ -27,6 +27,7 @@
 // just finished and reads the next stage's first fragments under the remaining
 // MFMAs.
 #include <limits.h>
+#include <type_traits>
 #include "pg_internal.h"
 #include "pg_quant_dev.h"
 #include "pg_stream_addr.h"
@@ -248,14 +249,6 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
             clk[2 * blockIdx.x + 1] = wall_clock64() - clk_w0;
         }
     }
-    // How outputs are stored (see below); rows that do not begin on a line leave the hint off: the halves of a line then come
-    // with different stores, and the hint takes each to memory by itself.  us, with it : without: 1355 x 2253 -> 11567 78 : 58,
-    // 2015 x 8071 -> 4709 143 : 131, 1131 x 1035 -> 8180 41 : 34.
-    const bool lines = ((uintptr_t)(acc_out ? (const void *)acc_out : (const void *)out) & 127) == 0 && (N & 31) == 0;
-    auto put = [&](auto v, auto *dst) {
-        if (lines) __builtin_nontemporal_store(v, dst);
-        else *dst = v;
-    };
     // ---- epilogue.  Accumulator register r of a 32x32 tile holds
     // row 8*(r/4) + 4*(lane/32) + r%4, column lane%32.  (The scales were requested before the
     // K loop: loading them here would put several dependent memory round trips on every tile.)
@@ -273,13 +266,27 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
                     const int mr = 8 * (r >> 2) + (r & 3);
                     const double v = 65536.0 * (double)acc[2 * TM + i][j][r] + 256.0 * (double)acc[TM + i][j][r] + (double)acc[i][j][r];
                     if (whole || (m0 + wm * WM + 32 * i + 4 * half + mr < M && n < N))
-                        put((float)(v * (double)lds_as[wm * WM + 32 * i + 4 * half + mr] * ws), dst + (size_t)mr * N);
+                        __builtin_nontemporal_store((float)(v * (double)lds_as[wm * WM + 32 * i + 4 * half + mr] * ws), dst + (size_t)mr * N);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
         return;
     }
+    // How whole tiles are stored (see below); rows that do not begin on a line leave the hint off: the halves of a line then come
+    // with different stores, and the hint takes each to memory by itself.  us, with it : without: 1355 x 2253 -> 11567 78 : 58,
+    // 2015 x 8071 -> 4709 143 : 131, 1131 x 1035 -> 8180 41 : 34.
+    const bool lines = ((uintptr_t)(acc_out ? (const void *)acc_out : (const void *)out) & 127) == 0 && (N & 31) == 0;
+    // (The two kinds of whole-tile epilogue are code of their own: a branch at every store cost a layer of
+    // 2048 rows 3 %.  The one-launch W8A32 product keeps the hint: its tiles take longer than their stores either way.)
+    auto put = [](auto hint, auto v, auto *dst) {
+        if constexpr (decltype(hint)::value) __builtin_nontemporal_store(v, dst);
+        else *dst = v;
+    };
+    auto either = [&](auto epilogue) {
+        if (lines) epilogue(std::true_type{});
+        else epilogue(std::false_type{});
+    };
     if (!COMB && out && !acc_out && m0 + BM <= M && n0 + BN <= N) {
         // A whole tile inside the matrix, f32 output only (every tile of the prefill shapes):
         // straight-line code, the 16 row scales of a 32-row tile as four 128-bit LDS reads.
@@ -287,6 +294,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
         // it per launch otherwise displace the operands of this and the next launch from L2
         // and the Infinity Cache (whole prefill layer 0.633 -> 0.59 ms).  The same hint on the
         // operand fills costs 7 - 15 %.
+        either([&](auto hint) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             float as[16];
@@ -301,15 +309,17 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
                 float *dst = out + (size_t)(m0 + wm * WM + 32 * i + 4 * half) * N + (n0 + wn * WN + 32 * j + l31);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
-                    put((float)acc[i][j][r] * as[r] * ws, dst + (size_t)(8 * (r >> 2) + (r & 3)) * N);
+                    put(hint, (float)acc[i][j][r] * as[r] * ws, dst + (size_t)(8 * (r >> 2) + (r & 3)) * N);
                 __builtin_amdgcn_sched_barrier(0);  // one tile's stores at a time: bounded live ranges
             }
         }
+        });
         return;
     }
     if (COMB && out && !acc_out && m0 + BM <= M && n0 + BN <= N) {
         // The W8A32 product's last pass on a whole tile: the two other digits' accumulators are fetched in the
         // order the stores go out (a lane's rows of one column, four at a time).
+        either([&](auto hint) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             float as[16];
@@ -334,26 +344,29 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const double v = 65536.0 * (double)acc[i][j][r0 + r] + 256.0 * (double)c1[r] + (double)c0[r];
-                        put((float)(v * (double)as[r0 + r] * ws), out + base + (size_t)(8 * ((r0 + r) >> 2) + ((r0 + r) & 3)) * N);
+                        put(hint, (float)(v * (double)as[r0 + r] * ws), out + base + (size_t)(8 * ((r0 + r) >> 2) + ((r0 + r) & 3)) * N);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 __builtin_amdgcn_sched_barrier(0);  // one tile at a time: bounded live ranges
             }
         }
+        });
         return;
     }
     if (acc_out && !out && m0 + BM <= M && n0 + BN <= N) {  // the same for the integer-only output of the W8A32 passes
+        either([&](auto hint) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 int32_t *dst = acc_out + (size_t)(m0 + wm * WM + 32 * i + 4 * half) * N + (n0 + wn * WN + 32 * j + l31);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) put(acc[i][j][r], dst + (size_t)(8 * (r >> 2) + (r & 3)) * N);
+                for (int r = 0; r < 16; ++r) put(hint, acc[i][j][r], dst + (size_t)(8 * (r >> 2) + (r & 3)) * N);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        });
         return;
     }
 #pragma unroll
