@@ -87,7 +87,8 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     constexpr int KS = BK / 32;                      // k-steps per stage
     constexpr int TA = NP * TM;                      // activation tiles per wavefront, plane by plane
     constexpr int NF = TA + TN, NMFMA = TA * TN;
-    static_assert(LA >= 1 && LB >= 1 && KS % 2 == 0 && BM <= 64 * NW && BN <= 64 * NW, "unsupported tile configuration");
+    static_assert(NP * BM % (RPL * NW) == 0 && BN % (RPL * NW) == 0 && KS % 2 == 0 && PG_MPAD % BM == 0 && BM <= 64 * NW && BN <= 64 * NW,
+                  "unsupported tile configuration");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 
     // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a contiguous
@@ -121,7 +122,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
         const int row = RPL * (wave + NW * i) + lr;
-        b_goff[i] = row * ldb + 16 * (pc ^ swz<BK>(row));
+        b_goff[i] = (PG_NPAD % BN == 0 ? row : min(row, N - 1 - n0)) * ldb + 16 * (pc ^ swz<BK>(row));  // (panels that do not divide the padding)
     }
     // A split product (few activation rows): blockIdx.y owns kt_per_split k-tiles of BK bytes and
     // writes its i32 partial sums to plane blockIdx.y of acc_out.  Otherwise gridDim.y == 1.
@@ -751,51 +752,103 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_f32_rows_kernel(const float
     }
 }
 
-// Tile choice (measured on MI355X at M = 2048): the larger the tile the fewer bytes each
-// CU pulls from L2 per MFMA, but every CU needs a tile.  8 wavefronts per workgroup also
-// double the rate at which one CU can stream from L2 (about 9 GB/s per wavefront).
-// ctx->gemm_force_tile (pg_gemm_w8a8_force_tile) overrides the choice: 1 = 64x64, 2 = 256x256,
-// 3 = 128x256, 4 = 128x64, 5 = 128x128.
 size_t gemm_tiles(const pg_qtensor *const *w, int count, size_t m, size_t bm, size_t bn) {
     size_t panels = 0;
     for (int i = 0; i < count; ++i) panels += (w[i]->cols + bn - 1) / bn;
     return ((m + bm - 1) / bm) * panels;
 }
-int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
-    const size_t cus = (size_t)ctx->num_cu;
-    if (ctx->gemm_force_tile) return ctx->gemm_force_tile;
-    const size_t t256 = gemm_tiles(w, count, m, 256, 256);
-    if (m <= 64) return 1;
-    // one and a half rounds of the largest tile or more -- or a single round that fills at least 70 %
-    // of the CUs: the fused q|k|v product (192 tiles on 256 CUs) runs 56 us so against 65 us as
-    // 384 half-size tiles (the CUs left idle let the busy ones clock higher)
-    if (t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus)) return 2;
-    if (gemm_tiles(w, count, m, 128, 256) >= cus) return 3;
-    // Too few 128x128 tiles for the CUs (k/v projections, N = 1024): halve the tile instead of
-    // leaving half of the chip idle (21.2 -> 16.5 us at 2048 x 4096 -> 1024).
-    return gemm_tiles(w, count, m, 128, 128) < cus ? 4 : 5;
+// The tile kernels and what a launch of each takes with the quantisation before it, us: the longer of what the fullest CU does
+// (its tiles one after another, as many as its LDS holds at a time: a step of 128 of K by how many are resident, and a round's
+// ends; 0.29 less of it in proportion to the places that the rounds leave empty, which the busy CUs' clock makes good) and what all
+// tiles bring through L2, the weights from HBM and the output back, as the fourth root of the sum of their fourth powers.
+// Fitted to 690 products (m 65 .. 4200, K 128 .. 14336, n 64 .. 24000, each kernel timed on each, the weights from HBM): 5 to 7 %
+// mean error where a kernel is within 30 % of the best; the choice takes 1.1 % more than the best kernel on average, 6 % at the 95th
+// percentile (half of them against a fit to the others: 1.4 and 8 %).
+//
+// What the shapes are: eight wavefronts or more for everything beyond 64x64 and as many stages as the LDS holds, or two and
+// three workgroups a CU, because a CU's stream from L2 grows with what it has in flight.  Against four wavefronts a tile and two or three stages, and
+// lines on the number of tiles (the largest that fill 70 % of the CUs), products of more than 700 rows take 0.84 of the time, 257 to
+// 700 0.9.  us, before : now: 2015 x 8071 -> 4709 142 : 99, 1262 x 13674 -> 4132 153 : 101, 473 x 6624 -> 9376 80 : 51,
+// 353 x 3968 -> 3968 25 : 21, 717 x 1568 -> 3104 16.9 : 14.4, 2048 x 14336 -> 4096 157 : 147; 2048 x 4096 -> 14336 as before.
+struct tile_kernel {
+    int code;  // of pg_gemm_w8a8_force_tile
+    unsigned bm, bn, resident;  // (workgroups a CU holds)
+    double step[3], round, fixed, l2, weights, output;  // per MB through L2, M weights, M outputs
+};
+constexpr tile_kernel TILES[] = {{1, 64, 64, 3, {0.308, 0.350, 0.396}, 1.15, 3.45, 0.0631, 0.053, 0.232},  // three stages
+                                 {2, 256, 256, 1, {1.608}, 10.1, 5.80, 0.0, 0.430, 0.585},
+                                 {3, 128, 256, 1, {0.981}, 5.53, 4.16, 0.0066, 0.289, 0.606},
+                                 {4, 128, 64, 2, {0.424, 0.620}, 1.65, 3.30, 0.0547, 0.078, 0.522},
+                                 {5, 128, 128, 1, {0.584}, 3.15, 3.24, 0.0247, 0.238, 0.445},
+                                 {6, 128, 192, 1, {0.777}, 4.29, 3.90, 0.0242, 0.221, 0.589},
+                                 {7, 256, 128, 1, {0.982}, 4.80, 2.35, 0.0514, 0.074, 0.677},
+                                 {8, 256, 192, 1, {1.311}, 8.35, 4.63, 0.0, 0.494, 0.597},
+                                 {1, 64, 64, 2, {0.285, 0.381}, 1.21, 3.51, 0.0595, 0.0, 0.0}};  // four stages
+constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
+double quantise_us(const pg_qtensor *w, size_t m) { return 3.0 + 0.8e-6 * (double)(m * w->rows); }
+// The kernel of least estimated time (its index), and that time.  (A call of few microseconds waits for this: 32-bit
+// divisions, and no roots for what is longer anyway.)
+int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, double *us = nullptr) {
+    const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w[0]->k_pad / 128), rows64 = (unsigned)((m + 63) / 64);
+    unsigned panels64 = 0, panels128 = 0, panels192 = 0, panels256 = 0;
+    size_t cols = 0;
+    for (int i = 0; i < count; ++i) {
+        const unsigned n = (unsigned)w[i]->cols;
+        panels64 += (n + 63) / 64;
+        panels128 += (n + 127) / 128;
+        panels192 += (n + 191) / 192;
+        panels256 += (n + 255) / 256;
+        cols += n;
+    }
+    const double weights = 1e-6 * (double)(w[0]->rows * cols), output = 1e-6 * (double)(m * cols);
+    int best = -1;
+    double best_us = 0.0;
+    for (int i = 0; i < NTILES; ++i) {
+        const tile_kernel &t = TILES[i];
+        if (ctx->gemm_force_tile && t.code != ctx->gemm_force_tile) continue;
+        const unsigned rows = (rows64 + t.bm / 64 - 1) / (t.bm / 64), panels = t.bn == 64 ? panels64 : t.bn == 128 ? panels128 : t.bn == 192 ? panels192 : panels256;
+        const size_t tiles = (size_t)rows * panels;
+        const size_t most = tiles <= ~0u - cus ? ((unsigned)tiles + cus - 1) / cus : (tiles + cus - 1) / cus;
+        const size_t full = t.resident == 1 ? most : t.resident == 2 ? most / 2 : most / 3, rest = most - full * t.resident;
+        double cu = (double)full * (kt * t.step[t.resident - 1] + 0.5 * (t.resident + 1) * t.round);
+        if (rest) cu += kt * t.step[rest - 1] + 0.5 * (double)(rest + 1) * t.round;
+        cu *= 1.0 - 0.29 * (1.0 - (double)tiles / (double)(most * cus));
+        const double all = 128e-6 * (double)(tiles * kt) * (t.bm + t.bn) * t.l2 + weights * t.weights + output * t.output;
+        if (best >= 0 && t.fixed + std::max(cu, all) >= best_us) continue;
+        const double c2 = cu * cu, a2 = all * all, time = t.fixed + sqrt(sqrt(c2 * c2 + a2 * a2));
+        if (best < 0 || time < best_us) {
+            best = i;
+            best_us = time;
+        }
+    }
+    // Short K and 128x128 tiles for all CUs but a few: one round of them, where smaller ones need a second or fourth.  (636 x 416 -> 6368
+    // 13.3 : 12.1, 280 x 320 -> 10624 10.4 : 9.9, 1295 x 503 -> 2849 13.7 : 12.5, 1024 x 256 -> 4096 11.4 : 10.1; 216 tiles 12.4 : 12.1, 212 10.6 : 11.)
+    const size_t t128 = (size_t)((rows64 + 1) / 2) * panels128;
+    if (!ctx->gemm_force_tile && w[0]->k_pad <= 512 && t128 <= cus && 20 * t128 >= 19 * cus) best = 4;
+    if (us) *us = quantise_us(w[0], m) + best_us;
+    return best;
 }
 pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                         const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc,
                         const int32_t *comb = nullptr, size_t comb_plane = 0) {
-    const int pick = pick_tile(ctx, w, count, m);
+    // (the combining pass is for products that fill the part with 256x256 tiles: w8a32_large)
+    const int pick = comb && !ctx->gemm_force_tile ? 1 : pick_tile(ctx, w, count, m);
     switch (pick) {
-        case 1:
-            if (comb) return launch_group<64, 64, 128, 2, 2, 2, 2, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
-            return launch_group<64, 64, 128, 2, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
-        case 2:
-            if (comb) return launch_group<256, 256, 128, 2, 2, 4, 2, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
-            return launch_group<256, 256, 128, 2, 2, 4, 2>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
-        case 3:
-            if (comb) return launch_group<128, 256, 128, 2, 2, 4, 2, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
-            return launch_group<128, 256, 128, 2, 2, 4, 2>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
-        case 4:
-            if (comb) return launch_group<128, 64, 128, 3, 2, 2, 2, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
-            return launch_group<128, 64, 128, 3, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
-        case 5:
-            if (comb) return launch_group<128, 128, 128, 3, 2, 2, 2, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
-            return launch_group<128, 128, 128, 3, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
-        default: return pg_fail(PG_EINVAL, "gemm_w8a8: unknown tile override %d", pick);
+#define PG_TILE(CODE, ...)                                                                                                                    \
+        case CODE:                                                                                                                            \
+            if (comb) return launch_group<__VA_ARGS__, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);   \
+            return launch_group<__VA_ARGS__>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
+        PG_TILE(0, 64, 64, 128, 3, 2, 2, 3)
+        PG_TILE(1, 256, 256, 128, 2, 2, 4, 2)
+        PG_TILE(2, 128, 256, 128, 3, 2, 4, 2)
+        PG_TILE(3, 128, 64, 128, 3, 4, 2, 4)
+        PG_TILE(4, 128, 128, 128, 4, 2, 4, 2)
+        PG_TILE(5, 128, 192, 128, 3, 4, 2, 2)
+        PG_TILE(6, 256, 128, 128, 3, 4, 4, 4)
+        PG_TILE(7, 256, 192, 128, 2, 4, 2, 2)
+        PG_TILE(8, 64, 64, 128, 4, 2, 2, 2)
+#undef PG_TILE
+        default: return pg_fail(PG_EINVAL, "gemm_w8a8: unknown tile override %d", ctx->gemm_force_tile);
     }
 }
 
@@ -836,56 +889,62 @@ pg_status pg_launch_gemm_w8a8_few_rows(pg_ctx *ctx, const int8_t *a_i8, size_t a
 // groups of one weight tile follow each other on one XCD).  What the launch takes against the tiles of gemm_dispatch, both as
 // estimates: few rows over few columns leave most CUs without a tile, and a tile then walks all of K alone.  Fitted to 889
 // products (m 33 .. 400, K 256 .. 14336, one to three weights of 64 .. 16384 columns; every shape below and both other routes
-// timed on each): the launch 10 % mean error, the tiles 8 %, the choice 2.4 % over the best route on average
-// (past 256 rows, where the least is to be had, with a margin).  us, with the
+// timed on each): the launch 10 % mean error.  From 65 rows on it is held against 0.85 of pick_tile's estimate: of 66 products of
+// more than 9 us, 1 % over the better route on average (lines at 0.75 to 1 of it: 1.6 to 2.4 %).  us, with the
 // quantisation, before : now: 66 x 1024 -> 4096 9.8 : 7.2, 96 x 4096 -> 1024 15.4 : 8.5, 128 x 4096 -> 4096 15.7 : 13.2, 39 x 4096 ->
 // 1024 11.8 : 8.2, 256 x 4096 -> 1024 19.5 : 9.8; the tiles stay: 256 x 1024 -> 4096 8.7 : 11.6, 256 x 4096 -> 4096 17.0 : 22.6.
 namespace {
 struct few_rows_shape { int mb, nb, nst, nw; double factor; };
 constexpr few_rows_shape FEW_ROWS_SHAPES[] = {{2, 1, 2, 2, 0.971}, {2, 1, 3, 4, 0.863}, {2, 1, 3, 8, 0.847}, {2, 2, 2, 4, 0.997}, {2, 2, 2, 8, 0.956},
                                               {3, 1, 2, 8, 0.903}, {3, 2, 2, 4, 1.033}, {3, 2, 2, 8, 1.0},   {4, 2, 3, 4, 1.009}};
-// What the tiles' K loops of one launch over all the weights take, us (see choose_few_rows).
-double tiles_us(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
-    static constexpr int BM[] = {64, 256, 128, 128, 128}, BN[] = {64, 256, 256, 64, 128};
-    static constexpr double STEP[] = {0.366, 1.98, 1.26, 0.302, 0.846};  // per 128 of K and round
-    if (count == 0) return 0.0;
-    const int t = pick_tile(ctx, w, count, m) - 1;
-    const size_t cus = (size_t)ctx->num_cu, rounds = (gemm_tiles(w, count, m, BM[t], BN[t]) + cus - 1) / cus;
-    return STEP[t] * (double)(rounds * (w[0]->k_pad / 128));
-}
-bool choose_few_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, few_rows_shape *out) {
-    const size_t k_pad = w[0]->k_pad, units = k_pad / 128, cus = (size_t)ctx->num_cu;
-    if (m < 33 || m > 512 || ctx->gemm_force_tile) return false;
+// The shape of least estimated time, and that time (a call of few microseconds waits for this: 32-bit divisions); 0: not for these weights.
+double few_rows_us(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, few_rows_shape *out) {
+    const size_t k_pad = w[0]->k_pad;
+    const unsigned units = (unsigned)(k_pad / 128), cus = (unsigned)ctx->num_cu, rows = (unsigned)m;
+    if (m < 33 || m > 512 || ctx->gemm_force_tile) return 0.0;
+    unsigned g16 = 0, g32 = 0;
     size_t cols = 0;
     for (int i = 0; i < count; ++i) {
-        if (w[i]->k_pad != k_pad || w[i]->cols >= (1ull << 20)) return false;
+        if (w[i]->k_pad != k_pad || w[i]->cols >= (1ull << 20)) return 0.0;
         cols += w[i]->cols;
+        g16 += (unsigned)(w[i]->cols + 15) / 16;
+        g32 += (unsigned)(w[i]->cols + 31) / 32;
     }
     // (a long K over one weight: split between workgroups, see pg_launch_gemm_w8a8_few_rows)
-    if (count == 1 && units >= 72 && (m <= 64 || (m <= 256 && k_pad >= 2 * cols))) return false;
-    const double mk = 1e-6 * (double)(m * k_pad);
-    double best = 1e30;
+    if (count == 1 && units >= 72 && (m <= 64 || (m <= 256 && k_pad >= 2 * cols))) return 0.0;
+    const double rows_us = 4.96 + 1.24e-6 * (double)(m * k_pad);
+    double best = 0.0;
     for (const few_rows_shape &s : FEW_ROWS_SHAPES) {
-        size_t wgs = 0;
-        for (int i = 0; i < count; ++i) wgs += (w[i]->cols + 16 * s.nb - 1) / (16 * s.nb);
-        wgs *= (m + 16 * s.mb - 1) / (16 * s.mb);
-        const size_t lds_kib = 2 * (size_t)(s.nw * s.nst * (s.nb + s.mb)), per_cu = std::min<size_t>(160 / lds_kib, 32 / s.nw);
-        const double rounds = (double)((wgs + cus * per_cu - 1) / (cus * per_cu)), run = (double)((units + s.nw - 1) / s.nw);
-        const double mb_cu = 1e-6 * (double)((wgs + cus - 1) / cus * units * (s.nb + s.mb) * 2048);  // what the fullest CU loads
-        const double us = s.factor * (4.96 + 1.24 * mk + rounds * (1.5 + 0.253 * run) + 14.0 * mb_cu);
-        if (us < best) {
+        const unsigned wgs = (s.nb == 1 ? g16 : g32) * ((rows + 16 * s.mb - 1) / (16 * s.mb));
+        const unsigned per_cu = std::min(80u / (unsigned)(s.nw * s.nst * (s.nb + s.mb)), 32u / s.nw);
+        const unsigned rounds = (wgs + cus * per_cu - 1) / (cus * per_cu), run = (units + s.nw - 1) / s.nw;
+        const double mb_cu = 2048e-6 * (double)((wgs + cus - 1) / cus) * units * (s.nb + s.mb);  // what the fullest CU loads
+        const double us = s.factor * (rows_us + rounds * (1.5 + 0.253 * run) + 14.0 * mb_cu);
+        if (best == 0.0 || us < best) {
             best = us;
             *out = s;
         }
     }
-    return best < (m <= 256 ? 0.95 : 0.85) * (7.8 + 1.86 * mk + tiles_us(ctx, w, count, m));
+    return best;
+}
+bool choose_few_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, few_rows_shape *out) {
+    const double us = few_rows_us(ctx, w, count, m, out);
+    if (us == 0.0) return false;
+    if (m <= 64) {  // held against the kernel of one weight tile for all rows, as rounds of 64x64 tiles
+        const size_t cus = (size_t)ctx->num_cu, k_pad = w[0]->k_pad;
+        return us < 0.95 * (7.8 + 1.86e-6 * (double)(m * k_pad) + 0.366 * (double)((gemm_tiles(w, count, m, 64, 64) + cus - 1) / cus * (k_pad / 128)));
+    }
+    double tiles = 0.0;
+    pick_tile(ctx, w, count, m, &tiles);
+    return us < 0.85 * tiles;
 }
 }  // namespace
 
 // Several weights that share the tiles' launch: whether those of long K and few columns are better off in a launch of their own, split
 // over K (pg_launch_gemm_w8a8_few_rows, estimated from 16 such products), because the others then need a round of tiles less, or
 // because few tiles walk a long K.
-// apart[i] says which.  us, all in one : apart: 135 x 10836 -> 628, 8185 75.7 : 63.8, 213 x 13535 -> 1432, 7172 96.9 :
+// apart[i] says which.  The lines are those of tiles that took longer than today's: the one launch has come level since where most of
+// the outputs go apart, and ahead where few do (135 x 10836 -> 628, 8185 58.7 : 62).  Then: us, all in one : apart: 135 x 10836 -> 628, 8185 75.7 : 63.8, 213 x 13535 -> 1432, 7172 96.9 :
 // 84.6, 36 x 13303 -> 1942, 6355 80.2 : 49.9, 46 x 13309 -> 294, 9512 81.2 : 57.0; of 110 such groups the worst it leaves is 34 x 7988 -> 8097,
 // 679, 708, 51.4 against 48.1 with each weight split.
 bool pg_gemm_w8a8_split_apart(pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, bool *apart) {
@@ -899,8 +958,17 @@ bool pg_gemm_w8a8_split_apart(pg_ctx *ctx, const pg_qtensor *const *w, int count
         if (apart[i]) split_us += 9.5 + 0.05e-3 * (double)(m * w[i]->cols);
         else rest[n_rest++] = w[i];
     }
-    const double cold = m <= 64 ? 1.95 : 1.55;  // (a step of the tiles over weights that no cache holds)
-    return n_rest < count && split_us + cold * tiles_us(ctx, rest, n_rest, m) < 0.95 * cold * tiles_us(ctx, w, count, m);
+    // rounds of the tiles that lines on their number choose, 128 of K at a time
+    auto tiles_us = [&](const pg_qtensor *const *of, int n) {
+        if (n == 0) return 0.0;
+        const size_t cus = (size_t)ctx->num_cu, t256 = gemm_tiles(of, n, m, 256, 256);
+        const bool largest = m > 64 && (t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus));
+        const tile_kernel *t = m <= 64 ? &TILES[0] : largest ? &TILES[1] : gemm_tiles(of, n, m, 128, 256) >= cus ? &TILES[2] : gemm_tiles(of, n, m, 128, 128) < cus ? &TILES[3] : &TILES[4];
+        static constexpr double STEP[] = {0.366, 1.98, 1.26, 0.302, 0.846};
+        return STEP[t - TILES] * (double)((gemm_tiles(of, n, m, t->bm, t->bn) + cus - 1) / cus * (of[0]->k_pad / 128));
+    };
+    const double cold = m <= 64 ? 1.95 : 1.55;  // (a step over weights that no cache holds)
+    return n_rest < count && split_us + cold * tiles_us(rest, n_rest) < 0.95 * cold * tiles_us(w, count);
 }
 
 // 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights side by side.
@@ -927,7 +995,9 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         if (a_stride != w[i]->k_pad) return pg_fail(PG_EINVAL, "gemm_w8a8: activation stride %zu != k_pad %zu", a_stride, w[i]->k_pad);
         cols += w[i]->cols;
     }
-    if (!pg_gemm_w8a8_takes_skinny(ctx, w, count, m)) return pg_fail(PG_EINVAL, "gemm_w8a8 (few rows in one launch): m = %zu", m);
+    few_rows_shape grouped;
+    const bool rows_grouped = m > 64 ? few_rows_us(ctx, w, count, m, &grouped) > 0.0 : choose_few_rows(ctx, w, count, m, &grouped);  // (from 65 on the caller has chosen)
+    if (m > 64 ? !rows_grouped : !pg_gemm_w8a8_takes_skinny(ctx, w, count, m)) return pg_fail(PG_EINVAL, "gemm_w8a8 (few rows in one launch): m = %zu", m);
     const size_t k_pad = w[0]->k_pad;
     // Weight tiles a workgroup (NB), stages of a ring (NST) and wavefronts a workgroup (NW, its K runs).  What counts is that
     // every workgroup is resident at once and that a CU has many units requested: two or three stages in more wavefronts
@@ -941,8 +1011,6 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
     const size_t units = k_pad / 128, g16 = (cols + 15) / 16, cus = (size_t)ctx->num_cu;
     struct shape { int nb, nst, nw; } sh = {1, mb == 1 ? 4 : 3, 0};
     const size_t wgs2 = (g16 + 1) / 2;  // workgroups of two weight tiles
-    few_rows_shape grouped;
-    const bool rows_grouped = choose_few_rows(ctx, w, count, m, &grouped);
     if (rows_grouped) {
         mb = grouped.mb;
         sh = {grouped.nb, grouped.nst, grouped.nw};

@@ -732,7 +732,7 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
 
 // Which tile the W8A8 matrix-core product last ran with on this context, and an override of the
 // dispatcher's choice (0 = automatic; 1 = 64x64, 2 = 256x256, 3 = 128x256, 4 = 128x64,
-// 5 = 128x128 output tiles).  For tests and tuning runs: every tile shape gives the same bits.
+// 5 = 128x128, 6 = 128x192, 7 = 256x128, 8 = 256x192 output tiles).  For tests and tuning runs: every tile shape gives the same bits.
 PG_API pg_status pg_gemm_w8a8_last_tile(const pg_ctx *ctx, int *bm, int *bn, int *k_splits) {
     PG_CHECK_ARG(ctx != nullptr, "null context");
     if (bm) *bm = ctx->gemm_last_bm;
@@ -743,7 +743,7 @@ PG_API pg_status pg_gemm_w8a8_last_tile(const pg_ctx *ctx, int *bm, int *bn, int
 
 PG_API pg_status pg_gemm_w8a8_force_tile(pg_ctx *ctx, int tile) {
     PG_CHECK_ARG(ctx != nullptr, "null context");
-    PG_CHECK_ARG(tile >= 0 && tile <= 5, "pg_gemm_w8a8_force_tile: tile %d (0 .. 5)", tile);
+    PG_CHECK_ARG(tile >= 0 && tile <= 8, "pg_gemm_w8a8_force_tile: tile %d (0 .. 8)", tile);
     ctx->gemm_force_tile = tile;
     return PG_OK;
 }

@@ -370,6 +370,57 @@ def test_every_gemm_tile_gives_the_same_bits(ctx, orc, m, k, n):
     qt.free_gpu()
 
 
+@pytest.mark.parametrize("m,k,n", [(257, 128, 510),       # panels of 192 columns that end behind the weight's padding; one step of K
+                                    (512, 300, 768), (90, 700, 193), (300, 640, 1030)])
+def test_wide_gemm_tiles_give_the_same_bits(ctx, orc, m, k, n):
+    """The tiles of codes 6 to 8, and 64x64 with three stages (many tiles) and four (few), as the others above."""
+    from peregrine_amd import quant, _ffi
+    a = outlier_acts(orc, 17 + m, m, k)
+    w = orc.rng_normal(18 + n, k * n, 0.0, 0.02)
+    q, q_t, s = orc.quantize_weights(w, k, n)
+    qt = quant.QuantizedTensor(q, q_t, s, k, n).to_gpu(ctx)
+    want, want_acc = orc.matmul_quantized(a, m, k, q_t, s, n)
+    da = DevBuf(ctx, host=a)
+    dout, dacc = DevBuf(ctx, m * n * 4 + 4), DevBuf(ctx, m * n * 4)
+    try:
+        for code, tile in {6: (128, 192), 7: (256, 128), 8: (256, 192), 1: (64, 64)}.items():
+            say(f"gemm tile {tile} on m={m} k={k} n={n}")
+            _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, code))
+            for acc_ptr, skew in ((dacc.ptr, 0), (None, 0), (None, 4)):   # an output off the lines is stored plainly
+                out = C.c_void_p(dout.ptr.value + skew)
+                _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, da.ptr, m, k, qt._gpu, out, acc_ptr))
+                ctx.sync()
+                bm, bn, sp = last_tile(ctx)
+                assert sp > 1 or (bm, bn) == tile
+                got = dout.to_host(np.float32)[skew // 4:skew // 4 + m * n]
+                assert (bits(got) == bits(want)).all(), f"tile {tile}: f32 outputs differ"
+            assert (dacc.to_host(np.int32) == want_acc).all(), f"tile {tile}: accumulators differ"
+    finally:
+        _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, 0))
+    qt.free_gpu()
+
+
+@pytest.mark.parametrize("m,k,n,tile", [(400, 1024, 4096, None), (2100, 640, 2000, None), (1600, 4100, 3300, None), (1200, 9000, 4100, None),
+                                         (1400, 4000, 2000, None), (1024, 512, 3968, (128, 128)), (600, 3744, 10144, None)])
+def test_chosen_gemm_tiles_against_numpy(ctx, orc, m, k, n, tile):
+    """Products whose kernel the estimates choose, exact integers against an int64 product."""
+    from peregrine_amd import quant, _ffi
+    rng = np.random.default_rng(m)
+    a = rng.integers(-127, 128, (m, k)).astype(np.float32)
+    a[:, 0] = 127.0                                        # so that the row scale is 1
+    qi = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    qt = quant.QuantizedTensor(qi.reshape(-1), np.ascontiguousarray(qi.T).reshape(-1), np.ones(n, np.float32), k, n).to_gpu(ctx)
+    da, dout = DevBuf(ctx, host=a), DevBuf(ctx, m * n * 4)
+    _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, da.ptr, m, k, qt._gpu, dout.ptr, None))
+    ctx.sync()
+    say(f"gemm m={m} k={k} n={n} ran {last_tile(ctx)}")
+    assert tile is None or last_tile(ctx)[:2] == tile
+    got = dout.to_host(np.float32).reshape(m, n)
+    want = (a.astype(np.float64) @ qi.astype(np.float64)).astype(np.float32)   # |sum| < 2^53; rounded once, as (float)acc is
+    assert (bits(got) == bits(want)).all()
+    qt.free_gpu()
+
+
 def run_multi(ctx, da, m, k, qts, douts):
     from peregrine_amd import _ffi
     wtab = (C.c_void_p * len(qts))(*[q._gpu.value for q in qts])
