@@ -854,18 +854,21 @@ pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const 
 
 }  // namespace
 
-// Few activation rows (5 .. 256: batched decode, short prefill chunks): one or two tiles of activations against
-// every weight row is far too few workgroups to stream the weights (64 on 256 CUs at N = 4096),
-// so K is split until about two workgroups per CU exist; the partial i32 sums go to `part`
-// ([splits][m][n]) and a second launch adds them and applies the scales.  Returns the number of
-// splits through *splits_out when called with part == nullptr (sizing), else runs.
+// Some dozens of rows over a long K (33 .. 256): one or two tiles of activations against every weight row is far too few
+// workgroups to stream the weights (64 on 256 CUs at N = 4096), so K is split until every place of a CU is taken, not one more
+// (a workgroup too many is a round); the partial i32 sums go to `part` ([splits][m][n]) and a second launch adds them and applies the
+// scales.  64x64 tiles of four stages, two workgroups a CU, or for much work and more than two tiles of rows 128x128 with eight
+// wavefronts, one a CU: over 36 products (K 9300 .. 14300) 0.87 of the time of 64x128 and 128x128 tiles of four wavefronts, split beyond
+// the places.  us, before : now: 135 x 10836 -> 628 21.4 : 18.5, 213 x 13535 -> 1432 34.0 : 25.8, 96 x 12787 -> 2221 31.6 : 22.8,
+// 87 x 12661 -> 4291 45.4 : 32.4, 46 x 13300 -> 9512 44.1 : 39.7.  Returns the number of splits through *splits_out when called with
+// part == nullptr (sizing), else runs.
 pg_status pg_launch_gemm_w8a8_few_rows(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                                        const pg_qtensor *w, size_t m, float *out, int32_t *acc, int32_t *part,
                                        int *splits_out) {
     const size_t n = w->cols, kt = w->k_pad / 128;
-    const size_t bm = m <= 32 ? 32 : (m <= 64 ? 64 : 128);
-    const size_t tiles = ((m + bm - 1) / bm) * ((n + 127) / 128);
-    size_t splits = (2 * (size_t)ctx->num_cu + tiles - 1) / tiles;
+    const bool large = m > 128 && m * w->k_pad * n > 7000000000ull;
+    const size_t tile = large ? 128 : 64, tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
+    size_t splits = (large ? 1 : 2) * (size_t)ctx->num_cu / tiles;
     if (splits > kt / 2) splits = kt / 2;  // at least two k-tiles per workgroup
     if (splits > 16) splits = 16;
     if (splits < 1) splits = 1;
@@ -874,12 +877,8 @@ pg_status pg_launch_gemm_w8a8_few_rows(pg_ctx *ctx, const int8_t *a_i8, size_t a
     if (splits_out) *splits_out = (int)splits;
     if (!part) return PG_OK;
     if (a_stride != w->k_pad) return pg_fail(PG_EINVAL, "gemm_w8a8: activation stride %zu != k_pad %zu", a_stride, w->k_pad);
-    if (bm == 32)
-        PG_TRY((launch<32, 128, 128, 3, 1, 4, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)splits, (int)kt_per)));
-    else if (bm == 64)
-        PG_TRY((launch<64, 128, 128, 3, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)splits, (int)kt_per)));
-    else
-        PG_TRY((launch<128, 128, 128, 3, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)splits, (int)kt_per)));
+    if (large) PG_TRY((launch<128, 128, 128, 4, 2, 4, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)splits, (int)kt_per)));
+    else PG_TRY((launch<64, 64, 128, 4, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)splits, (int)kt_per)));
     const size_t plane = m * n;
     return pg_launch(ctx, "gemm_w8a8_finish", splitk_finish_kernel, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0,
                      (const int32_t *)part, (int)splits, plane, a_scales, (const float *)w->scales, (int)n, out, acc);
