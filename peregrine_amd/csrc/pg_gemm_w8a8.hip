@@ -495,11 +495,11 @@ constexpr int F32_ROWS_NST = 4;  // stages of gemm_w8a8_f32_rows_kernel's rings
 // TRI: the W8A32 product.  The activations are three digit planes apart in memory (weights 1, 256, 65536); tile b is
 // tile b % (MB / 3) of plane b / (MB / 3), and the final pass joins the three sums in f64.
 // GROUPS: the rows in groups of 16 MB, each over every weight.
-// extra: the digit planes' distance (TRI); groups of rows, and above 32 bits the workgroups of one group (GROUPS).
+// extra: groups of rows, and above 32 bits the workgroups of one group (GROUPS); plane: the digit planes' distance (TRI).
 template <int MB, int NB, int NW, int NST, bool TRI = false, bool GROUPS = false>
 __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t *__restrict__ a_i8, const skinny_wgroup grp,
                                                                     int k_pad, int m, const float *__restrict__ a_scales,
-                                                                    int32_t *__restrict__ acc_out, size_t extra) {
+                                                                    int32_t *__restrict__ acc_out, size_t extra, size_t plane) {
     constexpr int MT = TRI ? MB / 3 : MB;  // tiles of activation rows
     int wg = blockIdx.x, r0 = 0;
     if constexpr (GROUPS) {  // (a weight tile's groups of rows: neighbours in time on one XCD)
@@ -533,8 +533,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
         for (int c = 0; c < NB; ++c) src[c][j] = w_t + pg_skinny_fill_offset(n0 + 16 * c + r, k_pad, 0, ch);  // (weight rows are padded to 256)
 #pragma unroll
         for (int b = 0; b < MB; ++b) {
-            const int row = GROUPS ? pg_skinny_act_row(r0, b, r, m) : 16 * (b % MT) + r;
-            src[NB + b][j] = a_i8 + (TRI ? b / MT * extra : 0) + pg_skinny_fill_offset(row, k_pad, 0, ch);
+            const int row = GROUPS ? pg_skinny_act_row(r0, b % MT, r, m) : 16 * (b % MT) + r;
+            src[NB + b][j] = a_i8 + (TRI ? b / MT * plane : 0) + pg_skinny_fill_offset(row, k_pad, 0, ch);
         }
     }
     // fragment reads: row lane % 16, chunk 4 s + lane / 16 of k-step s
@@ -1080,7 +1080,7 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         auto kern = gemm_w8a8_skinny_kernel<MBB, NBB, NWW, NSTT, ##__VA_ARGS__>;                                               \
         const size_t lds = (size_t)NWW * NSTT * (NBB + MBB) * 2048;                                                            \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
-        return pg_launch(ctx, "gemm_w8a8_few_rows", kern, grid, dim3(64 * NWW), lds, a_i8, grp, (int)k_pad, (int)m, a_scales, acc, extra); \
+        return pg_launch(ctx, "gemm_w8a8_few_rows", kern, grid, dim3(64 * NWW), lds, a_i8, grp, (int)k_pad, (int)m, a_scales, acc, extra, (size_t)0); \
     }
     if (rows_grouped) {
         const size_t groups = (m + 16 * mb - 1) / (16 * mb), extra = groups | (size_t)wgs << 32;
@@ -1173,7 +1173,7 @@ pg_status pg_launch_gemm_w8a8(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride,
 }
 
 // The W8A32 product over three digit planes in one launch, where it is the better route: up to 32 rows the few-row kernel
-// (three or six tiles of planes), beyond that tiles of 64x64 to 128x128, unless tiles of 256x256 fill the part and are
+// (three or six tiles of planes), beyond that what pick_w8a32 says, unless tiles of 256x256 fill the part and are
 // mostly rows (three quarters; then the two low planes stacked and the combining pass below; `takes` says which).  Tiles
 // filled up by a vocabulary's columns are no reason: the padding rows are multiplied too, and two planes of accumulators of
 // m_pad x n written and read.  us, one launch : stacked: 1 x 4096 -> 50257 62 : 161, 32 x 4096 -> 128256 240 : 423,
@@ -1187,11 +1187,48 @@ bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     return ctx->gemm_force_tile == 0 && !w8a32_large(ctx, w, m) && w->k_pad < (1ull << 22) && w->cols < (1ull << 30) &&
            2 * pg_round_up(m, PG_MPAD) * w->k_pad + 128 * w->k_pad < (1ull << 31);
 }
+// From 33 rows on: tiles, or up to 512 rows groups of 16 or 32 of them in the few-row kernel (whose wavefronts cut K), whichever is
+// estimated to take the least.  Estimates as in pick_tile, with what each kernel's idle places give back fitted too; 434 products (m 33 ..
+// 2048, K and n 256 .. 8192, weights from HBM and from the Infinity Cache, each kernel timed on each): 5 to 6 % mean error where a
+// kernel is within 30 % of the best, the choice 1 % over the best one on average.  Against tiles of 64x64 with three stages, 64x128 and
+// 128x128 with two by rounds of workgroups: 33 to 64 rows 0.67 of the time, 65 to 256 0.81, 257 to 700 0.92, beyond 0.93.  us, before :
+// now: 54 x 2150 -> 488 14.9 : 9.4, 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.
+struct w8a32_kernel {
+    unsigned bm, bn, resident, runs;  // rows, columns, workgroups a CU holds, parts of K within a workgroup
+    double step[2], round, fixed, l2, output, idle;
+};
+constexpr w8a32_kernel W8A32[] = {{32, 64, 2, 1, {0.376, 0.414}, 1.87, 3.44, 0.0677, 0.0, 0.152},   {32, 128, 1, 1, {0.506}, 2.46, 2.82, 0.0219, 2.59, 0.276},
+                                  {32, 128, 2, 1, {0.703, 0.782}, 1.54, 3.30, 0.0493, 1.41, 0.239}, {64, 128, 1, 1, {0.826}, 3.02, 2.80, 0.0448, 1.43, 0.299},
+                                  {128, 128, 1, 1, {1.478}, 6.02, 0.61, 0.0155, 2.71, 0.282},       {64, 256, 1, 1, {1.295}, 8.34, 0.0, 0.0537, 3.04, 0.291},
+                                  {16, 32, 1, 4, {0.634}, 0.0, 4.67, 0.0541, 11.3, 0.263},          {16, 16, 1, 8, {0.872}, 0.0, 3.74, 0.0530, 17.3, 0.0},
+                                  {32, 32, 1, 4, {1.044}, 1.29, 3.48, 0.0491, 8.49, 0.129}};  // the last three: groups of rows
+static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+    const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w->k_pad / 128);
+    const double output = 1e-6 * (double)(m * w->cols);
+    int best = 0;
+    double best_us = 0.0;
+    for (int i = 0; i < (int)(sizeof(W8A32) / sizeof(W8A32[0])); ++i) {
+        const w8a32_kernel &t = W8A32[i];
+        if (t.runs > 1 && m > 512) continue;
+        const size_t wgs = ((m + t.bm - 1) / t.bm) * ((w->cols + t.bn - 1) / t.bn), most = (wgs + cus - 1) / cus, full = most / t.resident, rest = most % t.resident;
+        const double steps = (double)((kt + t.runs - 1) / t.runs);
+        double cu = (double)full * (steps * t.step[t.resident - 1] + 0.5 * (t.resident + 1) * t.round);
+        if (rest) cu += steps * t.step[rest - 1] + 0.5 * (double)(rest + 1) * t.round;
+        cu *= 1.0 - t.idle * (1.0 - (double)wgs / (double)(most * cus));
+        const double all = 128e-6 * (double)(wgs * kt) * (3 * t.bm + t.bn) * t.l2 + output * t.output;
+        if (i && t.fixed + std::max(cu, all) >= best_us) continue;
+        const double c2 = cu * cu, a2 = all * all, us = t.fixed + sqrt(sqrt(c2 * c2 + a2 * a2));
+        if (!i || us < best_us) {
+            best = i;
+            best_us = us;
+        }
+    }
+    return best;
+}
 pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out) {
     if (!pg_gemm_w8a32_takes(ctx, w, m)) return pg_fail(PG_EINVAL, "gemm_w8a32: m = %zu", m);
     const size_t k_pad = w->k_pad, n = w->cols;
-    if (m <= 32) {
-        skinny_wgroup grp;
+    auto one_weight = [&](skinny_wgroup &grp) {
         for (int i = 0; i < PG_GEMM_MAX_GROUP; ++i) {
             grp.w[i] = i ? nullptr : w->w_t;
             grp.ws[i] = i ? nullptr : w->scales;
@@ -1199,6 +1236,10 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
             grp.n[i] = i ? 0 : (int)n;
             grp.wg0[i] = i ? INT_MAX : 0;
         }
+    };
+    if (m <= 32) {
+        skinny_wgroup grp;
+        one_weight(grp);
         // rings of 24 KiB (three tiles of planes, three stages) or 28 (six, two stages): six and five wavefronts a CU
         const dim3 grid((unsigned)((n + 15) / 16));
         const size_t slots = (size_t)ctx->num_cu * (m <= 16 ? 6 : 5), units = k_pad / 128;
@@ -1206,7 +1247,7 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
         while (nw > 1 && ((size_t)grid.x * nw > slots || units / nw < 2)) nw >>= 1;
         auto go = [&](auto kern, size_t lds) -> pg_status {
             PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
-            return pg_launch(ctx, "gemm_w8a32_few_rows", kern, grid, dim3(64 * nw), lds, planes, grp, (int)k_pad, (int)m, a_scales, (int32_t *)nullptr, plane_bytes);
+            return pg_launch(ctx, "gemm_w8a32_few_rows", kern, grid, dim3(64 * nw), lds, planes, grp, (int)k_pad, (int)m, a_scales, (int32_t *)nullptr, (size_t)0, plane_bytes);
         };
         if (m <= 16) {
             const size_t lds = (size_t)nw * 3 * 4 * 2048;
@@ -1217,18 +1258,26 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
         return nw == 4 ? go(gemm_w8a8_skinny_kernel<6, 1, 4, 2, true>, lds) : nw == 2 ? go(gemm_w8a8_skinny_kernel<6, 1, 2, 2, true>, lds)
                                                                                         : go(gemm_w8a8_skinny_kernel<6, 1, 1, 2, true>, lds);
     }
-    // One workgroup fits a CU whatever the tile: rounds of workgroups times what a round takes, 18 for 64x64, 24 for 64x128 and
-    // 40 for 128x128 (us at K = 4096).  Drawn from 180 shapes (m 33 .. 2500, K 256 .. 14336, n 512 .. 130000) with the three
-    // tiles timed on each and held against 280 others: 0.1 % over the best tile on average, 5 % at most (26, 29 and 40, from a
-    // few shapes, took 1.2 % and up to 26 %).  us, the three tiles: 197 x 1024 -> 4096 11.3 / 12.8 / 18.2, 356 x 4096 -> 14336
-    // 106 / 84 / 97, 1000 x 4096 -> 4096 84 / 66 / 63, 311 x 2048 -> 32000 101 / 75 / 84.
-    auto cost = [&](size_t bm, size_t bn, size_t us) { return (((m + bm - 1) / bm) * ((n + bn - 1) / bn) + ctx->num_cu - 1) / ctx->num_cu * us; };
-    const size_t c0 = cost(64, 64, 18), c1 = cost(64, 128, 24), c2 = cost(128, 128, 40);
-    if (c2 < c0 && c2 < c1)
-        return launch_group<128, 128, 128, 2, 2, 4, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes);
-    if (c1 < c0)
-        return launch_group<64, 128, 128, 2, 2, 4, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes);
-    return launch_group<64, 64, 128, 3, 2, 2, 1, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes);
+    auto tiles = [&](auto run) { return run(ctx, planes, k_pad, a_scales, &w, &out, 1, m, nullptr, 1, 0, nullptr, 0, plane_bytes); };
+    auto groups = [&](auto kern, size_t mt, size_t nb, int nw, int nst) -> pg_status {
+        skinny_wgroup grp;
+        one_weight(grp);
+        const size_t wgs = (n + 16 * nb - 1) / (16 * nb), row_groups = (m + 16 * mt - 1) / (16 * mt), lds = (size_t)nw * nst * (3 * mt + nb) * 2048;
+        PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
+        return pg_launch(ctx, "gemm_w8a32_few_rows", kern, dim3((unsigned)((wgs + 7) / 8 * 8 * row_groups)), dim3(64 * nw), lds, planes, grp, (int)k_pad, (int)m,
+                         a_scales, (int32_t *)nullptr, row_groups | wgs << 32, plane_bytes);
+    };
+    switch (pick_w8a32(ctx, w, m)) {
+        case 0: return tiles(launch_group<32, 64, 128, 3, 1, 2, 1, false, 3>);
+        case 1: return tiles(launch_group<32, 128, 128, 3, 1, 4, 1, false, 3>);
+        case 2: return tiles(launch_group<32, 128, 128, 2, 1, 4, 2, false, 3>);
+        case 3: return tiles(launch_group<64, 128, 128, 3, 2, 4, 2, false, 3>);
+        case 4: return tiles(launch_group<128, 128, 128, 2, 4, 4, 4, false, 3>);
+        case 5: return tiles(launch_group<64, 256, 128, 2, 2, 4, 2, false, 3>);
+        case 6: return groups(gemm_w8a8_skinny_kernel<3, 2, 4, 3, true, true>, 1, 2, 4, 3);
+        case 7: return groups(gemm_w8a8_skinny_kernel<3, 1, 8, 2, true, true>, 1, 1, 8, 2);
+        default: return groups(gemm_w8a8_skinny_kernel<6, 2, 4, 2, true, true>, 2, 2, 4, 2);
+    }
 }
 
 // The W8A32 product's last pass: `a_i8` is the digit plane of weight 65536, `comb` holds the accumulators of

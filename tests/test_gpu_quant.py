@@ -633,6 +633,31 @@ def test_matmul_dequant_i8_one_launch(ctx, orc, m, k, n):
     qt.free_gpu()
 
 
+@pytest.mark.parametrize("m,k,n", [
+    (519, 2221, 73), (186, 408, 2870), (211, 102, 3608), (1060, 665, 1904), (770, 105, 2959), (526, 1666, 3890),   # each of the tiles
+    (124, 1073, 515), (512, 174, 73), (212, 174, 73), (74, 396, 1118), (33, 128, 17), (513, 1000, 64),             # groups of rows, their ends
+])
+def test_matmul_dequant_i8_on_every_kernel(ctx, orc, m, k, n):
+    """Each kernel of the one launch from 33 rows on, at ragged sizes the estimates give it.  Small integers are exact; random
+    rows are within the activation step (2^-23 of the row's largest value a value) and one rounding of the float64 product."""
+    from peregrine_amd import quant
+    say(f"matmul_dequant_i8 kernels m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + k)
+    qi = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    s = rng.uniform(0.5e-3, 2e-3, n).astype(np.float32)
+    ones = quant.QuantizedTensor(qi.reshape(-1), np.ascontiguousarray(qi.T).reshape(-1), np.ones(n, np.float32), k, n)
+    ai = rng.integers(-9, 10, (m, k)).astype(np.float32)
+    got = quant.matmul_dequant_i8(ai, m, k, ones, ctx).reshape(m, n)
+    assert (got == (ai.astype(np.float64) @ qi.astype(np.float64))).all()
+    qt = quant.QuantizedTensor(qi.reshape(-1), np.ascontiguousarray(qi.T).reshape(-1), s, k, n)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    got = quant.matmul_dequant_i8(a, m, k, qt, ctx).reshape(m, n).astype(np.float64)
+    w = qi.astype(np.float64) * s.astype(np.float64)
+    want = a.astype(np.float64) @ w
+    bound = np.abs(a).max(1, keepdims=True) * 2.0 ** -23 * np.abs(w).sum(0, keepdims=True) + np.abs(want) * 2.0 ** -23
+    assert (np.abs(got - want) <= bound).all()
+
+
 @pytest.mark.parametrize("m,k,n", [(1, 256, 50257), (32, 384, 65536), (33, 130, 128256), (191, 256, 50257), (383, 128, 45825),
                                    (192, 256, 50257)])   # (the last one: the low planes stacked)
 def test_matmul_dequant_i8_wide_weights(ctx, m, k, n):
