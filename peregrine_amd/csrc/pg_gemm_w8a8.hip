@@ -1202,6 +1202,16 @@ constexpr w8a32_kernel W8A32[] = {{32, 64, 2, 1, {0.376, 0.414}, 1.87, 3.44, 0.0
                                   {128, 128, 1, 1, {1.478}, 6.02, 0.61, 0.0155, 2.71, 0.282},       {64, 256, 1, 1, {1.295}, 8.34, 0.0, 0.0537, 3.04, 0.291},
                                   {16, 32, 1, 4, {0.634}, 0.0, 4.67, 0.0541, 11.3, 0.263},          {16, 16, 1, 8, {0.872}, 0.0, 3.74, 0.0530, 17.3, 0.0},
                                   {32, 32, 1, 4, {1.044}, 1.29, 3.48, 0.0491, 8.49, 0.129}};  // the last three: groups of rows
+// Up to 32 rows: the kernels of 16 and 32 rows a group (-1: the one that takes all rows in a workgroup, up to four wavefronts) from the K on
+// where eight runs of it, or 32 columns a workgroup, are the shorter walk; 110 products of 2 .. 32 rows.  us, before : now: 17 x 6011 -> 420
+// 17.2 : 10.9, 31 x 7127 -> 2249 20.0 : 16.3, 27 x 3326 -> 6259 19.2 : 15.5, 3 x 4650 -> 6594 17.5 : 12.9, 2 x 6124 -> 287 12.0 : 10.3;
+// it stays: 15 x 6884 -> 2276 13.7 : 13.8, 12 x 2076 -> 3367 8.7 : 9.1, 20 x 1242 -> 1104 9.3 : 8.8 and shorter.
+static int pick_w8a32_few(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+    const size_t k = w->k_pad, n = w->cols, cus = (size_t)ctx->num_cu;
+    if (n > 32 * cus) return -1;  // (a vocabulary: the last line's 8192 columns)
+    if (m <= 16) return n > 16 * cus ? (k >= 1536 ? 6 : -1) : m <= 8 && k >= 3072 ? 7 : -1;
+    return n <= 8 * cus ? (k >= 1536 ? 7 : -1) : n <= 16 * cus ? (k >= 1536 ? 6 : -1) : k >= 2560 ? 8 : -1;
+}
 static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w->k_pad / 128);
     const double output = 1e-6 * (double)(m * w->cols);
@@ -1237,7 +1247,8 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
             grp.wg0[i] = i ? INT_MAX : 0;
         }
     };
-    if (m <= 32) {
+    const int pick = m <= 32 ? pick_w8a32_few(ctx, w, m) : pick_w8a32(ctx, w, m);
+    if (pick < 0) {
         skinny_wgroup grp;
         one_weight(grp);
         // rings of 24 KiB (three tiles of planes, three stages) or 28 (six, two stages): six and five wavefronts a CU
@@ -1267,7 +1278,7 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
         return pg_launch(ctx, "gemm_w8a32_few_rows", kern, dim3((unsigned)((wgs + 7) / 8 * 8 * row_groups)), dim3(64 * nw), lds, planes, grp, (int)k_pad, (int)m,
                          a_scales, (int32_t *)nullptr, row_groups | wgs << 32, plane_bytes);
     };
-    switch (pick_w8a32(ctx, w, m)) {
+    switch (pick) {
         case 0: return tiles(launch_group<32, 64, 128, 3, 1, 2, 1, false, 3>);
         case 1: return tiles(launch_group<32, 128, 128, 3, 1, 4, 1, false, 3>);
         case 2: return tiles(launch_group<32, 128, 128, 2, 1, 4, 2, false, 3>);

@@ -636,6 +636,7 @@ def test_matmul_dequant_i8_one_launch(ctx, orc, m, k, n):
 @pytest.mark.parametrize("m,k,n", [
     (519, 2221, 73), (186, 408, 2870), (211, 102, 3608), (1060, 665, 1904), (770, 105, 2959), (526, 1666, 3890),   # each of the tiles
     (124, 1073, 515), (512, 174, 73), (212, 174, 73), (74, 396, 1118), (33, 128, 17), (513, 1000, 64),             # groups of rows, their ends
+    (9, 1530, 4100), (8, 3000, 70), (17, 1500, 30), (32, 1409, 2049), (31, 2500, 4097),                             # few rows of long K
 ])
 def test_matmul_dequant_i8_on_every_kernel(ctx, orc, m, k, n):
     """Each kernel of the one launch from 33 rows on, at ragged sizes the estimates give it.  Small integers are exact; random
