@@ -326,6 +326,13 @@ def test_mxfp4_moe_tilings(ctx, orc, hidden, inter, E, top_k, T):
     test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, T)
 
 
+@pytest.mark.parametrize("E,T", [(63, 30), (64, 41), (65, 30), (127, 60), (128, 200), (129, 23), (256, 300)])
+def test_mxfp4_moe_finds_the_expert_of_a_tile(ctx, orc, E, T):
+    """The offsets of 64 experts are looked through at a time: the last expert of a run, the first of the next, and one run more for
+    the end of the last tile."""
+    test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, 64, 96, E, 3, T)
+
+
 @pytest.mark.parametrize("hidden,inter,E,top_k,T", [(64, 96, 6, 6, 3), (512, 512, 200, 64, 1), (512, 96, 70, 12, 5), (64, 512, 2, 1, 9), (64, 96, 9, 4, 6), (96, 64, 5, 3, 8),
                                                    (64, 96, 8, 5, 4), (96, 64, 4, 2, 7)])
 def test_mxfp4_moe_pairs_with_entries_that_name_no_expert(ctx, hidden, inter, E, top_k, T):
