@@ -249,8 +249,10 @@ PG_API pg_status pg_audit_mxfp4_tiles(int num_cu, size_t out_dim, size_t in_dim,
     for (size_t tg = 0; tg < p.groups; ++tg)
         for (int b = 0; b < 4 * ncp; ++b)
             for (int col = 0; col < 16; col += 15) {
-                for (int sub = 0; sub < 2; ++sub)
-                    for (int j = 0; j < PG_MT_PLANES; ++j) rec.touch(pg_mt_plane_store(tg, ncp, b, sub, col, j), 16);
+                for (int j = 0; j < PG_MT_PLANES; ++j) {
+                    rec.touch(pg_mt_plane_store(tg, ncp, b, col, j), 16);
+                    rec.touch(pg_mt_plane_tail(tg, ncp, b, col, j), 8);
+                }
                 rec.touch(pg_mt_scale_store(tg, ncp, b, col), 4);
             }
     // the tiles: every work item, wavefront and chunk of its run; lanes 0 and 63, threads 0 and 511

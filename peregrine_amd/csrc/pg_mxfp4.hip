@@ -17,6 +17,10 @@
 // j of a row is one column of B with block scale byte 127 + se + 5 j, so the instruction itself applies
 // both block scales and sums over K; the five columns of a row are added at the end.  Three activation
 // rows (15 columns) share one pass over the weights.
+//
+// From some dozens of rows on the digits are FP6 (E2M3), which holds n / 8 for every integer to 16 as well: beside an FP4 operand
+// the instruction then takes half the cycles (random operands, all CUs: 4.2 PFLOP/s in FP8, 6.6 in FP6).
+//   B  lane l holds column l % 16, k = 32 (l / 16) .. + 31, element e in bits 6 e .. 6 e + 5 of its 24 bytes.
 #include <math.h>
 #include "pg_internal.h"
 #include "pg_stream_addr.h"
@@ -26,7 +30,11 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef int v3i __attribute__((ext_vector_type(3)));
+typedef int v6i __attribute__((ext_vector_type(6)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 typedef const v4i __attribute__((address_space(1))) *gv4i_ptr;
 
 constexpr int MX_PLANES = 5;  // digit planes per activation row
@@ -420,11 +428,12 @@ namespace {
 // From a few dozen rows on the product is matrix-core work, and the instruction still does all of it: the block
 // scales of both sides are applied inside, so there is no rescaling of accumulators and nothing to dequantise.
 // An activation block becomes MT_PLANES balanced base-32 digits per value (20 bits under the block's largest
-// magnitude, |error| <= 2^-20 of it), each plane a B operand whose block scale carries the digit's weight; the
+// magnitude, |error| <= 2^-20 of it), each plane a B operand whose block scale carries the digit's weight (FP6: against 64 bits the
+// products' error is that of the same digits in FP8 to 1 %, 0.999 of it on average over 36 shapes); the
 // planes accumulate into the same tile, so a row costs MT_PLANES instructions per 16 x 16 x 128 tile and no
 // final sum.  A pre-pass writes the planes once, in the operand's own fragment order: per token group of 16
 // and chunk of 128 k one record of MT_RECORD bytes,
-//   [plane][half][64 lanes][16 B]   lane = token % 16 + 16 q holds k = 64 half + 16 q .. + 15 of the chunk
+//   [plane][64 lanes][16 B] [64 lanes][8 B]   lane = token % 16 + 16 (block of the chunk): the block's 32 digits of 6 bits
 //   [64 lanes] scale dwords         lane = token % 16 + 16 (block of the chunk), byte j = plane j
 constexpr int MT_PLANES = PG_MT_PLANES;
 constexpr int MT_NW = PG_MT_NW;            // wavefronts per workgroup
@@ -463,7 +472,7 @@ __device__ __forceinline__ mt_place mt_find(const mt_gather &g, int gt) {
 }
 
 // One thread = 16 consecutive k of one token (half a block).  A wavefront = the 16 tokens of a group x two blocks x
-// their halves, tokens on consecutive lanes: what it writes are whole 256-byte runs of the records, and the
+// their halves, tokens on consecutive lanes: what it writes are whole 256- and 128-byte runs of the records, and the
 // 256 bytes it reads of every token row are two full lines.
 // GATHER: the token groups are the experts' slots (mt_gather) instead of the rows in order.
 // SWIGLU: x holds mlp1's outputs, [pairs][2 * 32 nb], and the values are their bias and swiglu, made on the way (a launch
@@ -541,52 +550,59 @@ __global__ __launch_bounds__(256) void mxfp4_planes_kernel(const float *__restri
     // instruction's own sum over k exact, which numbers spread over the format's exponent range do not (a split
     // into E4M3 values of decreasing size, four significant bits a plane, stopped at 2e-4 of the output's rms
     // however many planes it was given).
-    int packed[MT_PLANES][4];
+    float r[16];
 #pragma unroll
-    for (int e4 = 0; e4 < 4; ++e4) {
-        float r[4], d[MT_PLANES][4];
+    for (int e = 0; e < 16; ++e) {
+        const float tt = f[e] * inv;
+        r[e] = (tt != tt) ? 0.0f : rintf(tt);
+    }
+    char *const head = bq + pg_mt_plane_store(tg, ncp, b, col, 0), *const tail = bq + pg_mt_plane_tail(tg, ncp, b, col, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float tt = f[4 * e4 + e] * inv;
-            r[e] = (tt != tt) ? 0.0f : rintf(tt);
-        }
+    for (int j = MT_PLANES - 1; j >= 0; --j) {
+        // The conversion takes two runs of 16 and interleaves them: even elements, odd elements; this thread's sixteen are the first
+        // 96 bits.  Integers in [-16, 16] over the scale of 8 are exact in E2M3.
+        v16f even = {}, odd = {};
 #pragma unroll
-        for (int j = MT_PLANES - 1; j >= 1; --j) {
-            const float down = __builtin_bit_cast(float, (127 - 5 * j) << 23), up = -__builtin_bit_cast(float, (127 + 5 * j) << 23);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                d[j][e] = rintf(r[e] * down);
-                r[e] = fmaf(d[j][e], up, r[e]);
+        for (int e = 0; e < 16; ++e) {
+            float d = r[e];
+            if (j > 0) {
+                const float down = __builtin_bit_cast(float, (127 - 5 * j) << 23), up = -__builtin_bit_cast(float, (127 + 5 * j) << 23);
+                d = rintf(r[e] * down);
+                r[e] = fmaf(d, up, r[e]);
             }
+            if (e & 1) odd[e >> 1] = d;
+            else even[e >> 1] = d;
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) d[0][e] = r[e];
-#pragma unroll
-        for (int j = 0; j < MT_PLANES; ++j) {  // integers in [-16, 16] are exact in E4M3
-            int pk = __builtin_amdgcn_cvt_pk_fp8_f32(d[j][0], d[j][1], 0, false);
-            packed[j][e4] = __builtin_amdgcn_cvt_pk_fp8_f32(d[j][2], d[j][3], pk, true);
+        const v6i pk = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(even, odd, 8.0f);
+        if (sub == 0) {
+            *reinterpret_cast<v3i *>(head + j * MT_FRAG) = v3i{pk[0], pk[1], pk[2]};
+        } else {
+            *reinterpret_cast<int *>(head + j * MT_FRAG + 12) = pk[0];
+            *reinterpret_cast<v2i *>(tail + j * MT_FRAG) = v2i{pk[1], pk[2]};
         }
     }
-#pragma unroll
-    for (int j = 0; j < MT_PLANES; ++j)
-        *reinterpret_cast<v4i *>(bq + pg_mt_plane_store(tg, ncp, b, sub, col, j)) = v4i{packed[j][0], packed[j][1], packed[j][2], packed[j][3]};
     if (sub == 0) {  // a NaN / inf block poisons every product it enters: scale byte 255 is NaN
         unsigned word = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) word |= (unsigned)(j >= MT_PLANES ? 127 : (bad ? 255 : 127 + se + 5 * j)) << (8 * j);
+        for (int j = 0; j < 4; ++j) word |= (unsigned)(j >= MT_PLANES ? 127 : (bad ? 255 : 130 + se + 5 * j)) << (8 * j);
         *reinterpret_cast<unsigned *>(bq + pg_mt_scale_store(tg, ncp, b, col)) = word;
     }
 }
 
-// A workgroup = MT_NW wavefronts x RA groups of 16 weight rows, against TB groups of 16 tokens, over one run of
+// A workgroup = NW wavefronts x RA groups of 16 weight rows, against TB groups of 16 tokens, over one run of
 // chunks (all of K, or one of `ks` runs whose partial tiles a later launch adds).  The weights go from memory
-// straight into the A operand's registers (each wavefront streams its own rows: two chunks ahead for the widest
-// row tile, a batch of four chunks ahead otherwise); the token records of a chunk are shared through LDS (staged
-// through registers BD chunks ahead, two stages, one barrier per chunk).  Narrow tiles do little arithmetic per
-// chunk, so what they need is requests in flight: the deeper staging is theirs.
+// straight into the A operand's registers, a ring of two chunks for the widest row tile and of four otherwise; the token records of
+// a chunk are shared through LDS (staged through registers BD chunks ahead, two stages, one barrier per chunk).  Narrow tiles do
+// little arithmetic per chunk, so what they need is requests in flight: the deeper staging is theirs.
 // GROUPED: the token tiles are the experts' (mt_gather), the weights come from the expert's entry of two pointer
-// tables, an output row is the pair the slot holds; one run of K; items walk the row tiles of one token tile first
-// (that tile's records stay in the XCD's L2).
+// tables, an output row is the pair the slot holds; one run of K.
+// Weights that several tiles read are loaded plainly, the others with the hint that nothing reads them again: hinted, they left the
+// L2 before the next tile came (480 tokens over 8 experts of 2048 x 2048, top 4: the two products 83 + 57 us, plain 78 + 54; but 90
+// tokens over 32 of 2880 x 2880, one tile an expert, 67 + 36 hinted and 72 + 42 plain).
+// What bounds a many-token product now is the matrix cores at about half their rate, the rest a chunk's barrier and LDS reads and
+// the last, partly filled round.  421 tokens over 8 experts of 1280 x 1376, top 4, us: 42.4 + 29.8 in FP8 digits and batches
+// of chunks under conditions; FP6 37.6 + 26.7; loads without conditions, plain and in XCD order, 25.8 + 19.4.  The 480 tokens above:
+// 86 + 57, 74 + 47, 66 + 43, and on four wavefronts instead of eight 50 + 31.
 struct mt_experts {
     const uint8_t *const *qs_tab;
     const uint32_t *const *sc_tab;
@@ -601,15 +617,17 @@ struct mt_experts {
 template <int RA, int NPM>
 __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, const uint32_t *__restrict__ sa, const char *__restrict__ bq,
                                                   int ncp, int turn, v4f (&acc)[RA]) {
-    constexpr int NI = MT_PLANES / NPM, CHUNK = NI * 2048 + 256, STAGE = 4 * CHUNK;
+    constexpr int NI = MT_PLANES / NPM, CHUNK = NI * MT_FRAG + 256, STAGE = 4 * CHUNK;
     const int lane = threadIdx.x & 63, t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const size_t a_stride = (size_t)ncp * 64;
-    // this thread's units of a batch: operand unit (chunk t / 128, half, lane) of every instruction, and a unit of the scales
-    const int oc = t >> 7, ol = t & 63, ocol = ol & 15;
-    const unsigned o_src = (unsigned)oc * MT_RECORD + (ocol % NPM) * MT_FRAG + ((t >> 6) & 1) * 1024 + (ocol / NPM + 16 * (ol >> 4)) * 16;
-    const unsigned o_dst = (unsigned)oc * CHUNK + ((t >> 6) & 1) * 1024 + ol * 16;
+    // this thread's units of a batch: operand unit (chunk t / 128, first 16 or last 8 bytes, lane) of every instruction, and a unit of
+    // the scales; of the last 8 bytes it reads the 16 that they are a half of
+    const int oc = t >> 7, ol = t & 63, ocol = ol & 15, from = ocol / NPM + 16 * (ol >> 4);
+    const bool last8 = (wave & 1) != 0;
+    const unsigned o_src = (unsigned)oc * MT_RECORD + (ocol % NPM) * MT_FRAG + (last8 ? 1024 + (from >> 1) * 16 : from * 16);
+    const unsigned o_dst = (unsigned)oc * CHUNK + (last8 ? 1024 + ol * 8 : ol * 16);
     const unsigned s_src = (unsigned)(lane >> 4) * MT_RECORD + MT_PLANES * MT_FRAG + (lane & 15) * 16;
-    const unsigned s_dst = (unsigned)(lane >> 4) * CHUNK + NI * 2048 + (lane & 15) * 16;
+    const unsigned s_dst = (unsigned)(lane >> 4) * CHUNK + NI * MT_FRAG + (lane & 15) * 16;
     v4i so[NI], ss;
     auto fetch_b = [&](int c) {
         const char *at = bq + (size_t)c * MT_RECORD;
@@ -619,7 +637,11 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
     };
     auto put_b = [&](int stage) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) *reinterpret_cast<v4i *>(lds + stage * STAGE + o_dst + i * 2048) = so[i];
+        for (int i = 0; i < NI; ++i) {
+            char *const at = lds + stage * STAGE + o_dst + i * MT_FRAG;
+            if (last8) *reinterpret_cast<v2i *>(at) = from & 1 ? v2i{so[i][2], so[i][3]} : v2i{so[i][0], so[i][1]};
+            else *reinterpret_cast<v4i *>(at) = so[i];
+        }
         if (wave == 0) *reinterpret_cast<v4i *>(lds + stage * STAGE + s_dst) = ss;
     };
     auto chunk_at = [&](int i) { return i + turn < ncp ? i + turn : i + turn - ncp; };
@@ -634,7 +656,7 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
         for (int r = 0; r < RA; ++r) sc[r] = sa[((size_t)r * (ncp / 4) + (c >> 2)) * 64 + lane];
     };
     const int col = lane & 15;
-    const unsigned sc_at = NI * 2048 + (col / NPM + 16 * (lane >> 4)) * 4, shift = 8 * (col % NPM);
+    const unsigned sc_at = NI * MT_FRAG + (col / NPM + 16 * (lane >> 4)) * 4, shift = 8 * (col % NPM);
 #pragma unroll
     for (int r = 0; r < RA; ++r) acc[r] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     fetch_b(chunk_at(0));
@@ -650,14 +672,14 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
         const char *st = lds + s * STAGE;
 #define PG_MT_STEP(U, I)                                                                                                   \
     do {                                                                                                                   \
-        const v4i b0 = *reinterpret_cast<const v4i *>(st + (U) * CHUNK + (I) * 2048 + lane * 16);                          \
-        const v4i b1 = *reinterpret_cast<const v4i *>(st + (U) * CHUNK + (I) * 2048 + 1024 + lane * 16);                   \
+        const v4i b0 = *reinterpret_cast<const v4i *>(st + (U) * CHUNK + (I) * MT_FRAG + lane * 16);                       \
+        const v2i b1 = *reinterpret_cast<const v2i *>(st + (U) * CHUNK + (I) * MT_FRAG + 1024 + lane * 8);                 \
         const int sb = (int)(*reinterpret_cast<const unsigned *>(st + (U) * CHUNK + sc_at) >> shift);                      \
-        const v8i B = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};                                            \
+        const v8i B = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], 0, 0};                                                    \
         _Pragma("unroll") for (int r = 0; r < RA; ++r) {                                                                   \
             const v4i aw = a[U][r];                                                                                        \
             const v8i A = {aw[0], aw[1], aw[2], aw[3], 0, 0, 0, 0};                                                        \
-            acc[r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, acc[r], 4, 0, (U), (int)sca[r], NPM * (I), sb); \
+            acc[r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, acc[r], 4, 2, (U), (int)sca[r], NPM * (I), sb); \
             asm volatile("" : "+v"(acc[r]) : : "memory");  /* (or every chunk's operands are read first: 32 to 64 registers) */ \
         }                                                                                                                  \
     } while (0)
@@ -709,9 +731,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED
                                                                  int ncp, int m, int n_tt, int ks, int cps, size_t part_stride,
                                                                  int items, int per_xcd, const mt_gather gat, const mt_experts ex) {
     constexpr int STAGE = TB * MT_RECORD, UNITS = TB * MT_UNITS, ROUNDS = (UNITS + 64 * NW - 1) / (64 * NW);
-    constexpr bool RING = RA == 4;  // A two chunks ahead in a ring of two; else the next batch of four chunks
+    constexpr bool NT = TB == 1 || (!GROUPED && TB == 2);
+    constexpr int DA = RA == 4 ? 2 : 4;  // weights read ahead, in chunks: a ring of registers
     constexpr int AHEAD = RA == 1 && TB > 1 ? 3 : 1;  // planes read ahead: the fewer products a plane feeds, the less of the LDS latency they cover
-    static_assert(NW == MT_NW || TB > 1, "narrow tiles are staged by all of MT_NW wavefronts");
     static_assert(BD == 1 || BD == 2 || BD == 4, "the staging depth divides the unrolled batch");
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -721,11 +743,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED
     if ((int)(blockIdx.x >> 3) >= per_xcd || item >= items) return;
     int tt = item % n_tt, split = (item / n_tt) % ks, wt = item / (n_tt * ks), live = TB;
     mt_place at = {0, 0, 0};
-    if (GROUPED) {  // n_tt = the row tiles here; token tile 8 i + x belongs to XCD x (the unused tail tiles spread evenly)
+    if (GROUPED) {  // n_tt = the row tiles here
         const int slot = (int)(blockIdx.x >> 3);
-        wt = slot % n_tt;
-        tt = (slot / n_tt) * 8 + (int)(blockIdx.x & 7);
         split = 0;
+        if (TB > 1) {  // every XCD walks its own run of tiles in order: an expert's weights are read by one or two of the eight
+            const int all = gat.goff[gat.experts] * n_tt, mine = (all + 7) / 8, it = (int)(blockIdx.x & 7) * mine + slot;
+            if (slot >= mine || it >= all) return;
+            tt = it / n_tt;
+            wt = it % n_tt;
+        } else {  // hardly an expert has a second tile: token tile 8 i + x belongs to XCD x (the unused tail tiles spread evenly)
+            tt = (slot / n_tt) * 8 + (int)(blockIdx.x & 7);
+            wt = slot % n_tt;
+        }
         at = mt_find(gat, tt);
         if (at.expert < 0) return;
         qs_frag = ex.qs_tab[at.expert];
@@ -784,20 +813,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED
 #define PG_MT_FETCH_B(SLOT, C)                                                                                          \
     do {                                                                                                                \
         _Pragma("unroll") for (int i = 0; i < ROUNDS; ++i)                                                              \
-            sr[SLOT][i] = *reinterpret_cast<const v4i *>(b_base + b_off[i] + (unsigned)(C) * MT_RECORD);                \
+            sr[SLOT][i] = *reinterpret_cast<const v4i *>(b_base + b_off[i] + (unsigned)(C) * MT_RECORD), __builtin_amdgcn_sched_barrier(0); \
     } while (0)
 #define PG_MT_PUT_B(STG, SLOT)                                                                                          \
     do {                                                                                                                \
         _Pragma("unroll") for (int i = 0; i < ROUNDS; ++i) {                                                            \
             const int u = (int)threadIdx.x + i * 64 * NW;                                                            \
-            if (u < UNITS) *reinterpret_cast<v4i *>(lds + (STG) * STAGE + u * 16) = sr[SLOT][i];                        \
+            if ((i + 1) * 64 * NW <= UNITS || u < UNITS) *reinterpret_cast<v4i *>(lds + (STG) * STAGE + u * 16) = sr[SLOT][i]; \
         }                                                                                                               \
     } while (0)
-    v4i a[RING ? 2 : 4][RA], an[RING ? 1 : 4][RA];
+    v4i a[DA][RA];
     uint32_t sca[RA], sca_next[RA];
     auto fetch_a = [&](v4i (&dst)[RA], int c) {
 #pragma unroll
-        for (int r = 0; r < RA; ++r) dst[r] = __builtin_nontemporal_load(qa + (size_t)r * a_stride + (size_t)c * 64 + lane);
+        for (int r = 0; r < RA; ++r) dst[r] = NT ? __builtin_nontemporal_load(qa + (size_t)r * a_stride + (size_t)c * 64 + lane) : qa[(size_t)r * a_stride + (size_t)c * 64 + lane];
     };
     v4f acc[RA][TB];
 #pragma unroll
@@ -813,22 +842,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED
         PG_MT_FETCH_B(BD > 2 ? 3 : 0, c0 + 3);
     }
 #pragma unroll
-    for (int u = 0; u < (RING ? 2 : 4); ++u) fetch_a(a[u], c0 + u);
+    for (int u = 0; u < DA; ++u) fetch_a(a[u], c0 + u);
 #pragma unroll
     for (int r = 0; r < RA; ++r) sca[r] = sa[((size_t)r * (ncp / 4) + (c0 >> 2)) * 64 + lane];
     PG_MT_PUT_B(0, 0);
     if (BD < run) PG_MT_FETCH_B(0, chunk_at(BD));
     __syncthreads();
-    for (int cb = 0; cb < run; cb += 4) {
-        const bool more = cb + 4 < run;
-        if (more) {
+    // Which loads a batch makes is known when it is compiled (the last batch is code of its own): with a condition around them the
+    // compiler cannot count what is under way, and a chunk's weights waited for everything that was read after them as well.
+    auto batch = [&](int cb, auto last_) {
+        constexpr bool LAST = decltype(last_)::value;
+        if (!LAST) {
             const int next = chunk_at(cb + 4);
 #pragma unroll
             for (int r = 0; r < RA; ++r) sca_next[r] = sa[((size_t)r * (ncp / 4) + (next >> 2)) * 64 + lane];
-            if (!RING) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) fetch_a(an[RING ? 0 : u], next + u);
-            }
         }
         // One step = one plane of one token group against the wavefront's RA row groups; the operand halves of the plane AHEAD steps on
         // are read meanwhile.  (The byte selectors of the two scale operands are immediates: chunk within the dword, plane within the dword.)
@@ -839,23 +866,25 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED
             int sbv[TB];
 #pragma unroll
             for (int g = 0; g < TB; ++g) sbv[g] = *reinterpret_cast<const int *>(st + g * MT_RECORD + MT_PLANES * MT_FRAG + lane * 4);
-            v4i b[AHEAD + 1][2];
+            v4i b[AHEAD + 1];
+            v2i bt[AHEAD + 1];
             auto read = [&](int step) {
-                const char *f = st + step / MT_PLANES * MT_RECORD + step % MT_PLANES * MT_FRAG + lane * 16;
-                b[step % (AHEAD + 1)][0] = *reinterpret_cast<const v4i *>(f);
-                b[step % (AHEAD + 1)][1] = *reinterpret_cast<const v4i *>(f + 1024);
+                const char *f = st + step / MT_PLANES * MT_RECORD + step % MT_PLANES * MT_FRAG;
+                b[step % (AHEAD + 1)] = *reinterpret_cast<const v4i *>(f + lane * 16);
+                bt[step % (AHEAD + 1)] = *reinterpret_cast<const v2i *>(f + 1024 + lane * 8);
             };
             auto step = [&](auto i_) {
                 constexpr int I = decltype(i_)::value, G = I / MT_PLANES, J = I % MT_PLANES;
                 if (GROUPED && G >= live) return;
                 if (I + AHEAD < TB * MT_PLANES) read(I + AHEAD);
-                const v4i b0 = b[I % (AHEAD + 1)][0], b1 = b[I % (AHEAD + 1)][1];
-                const v8i B = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
+                const v4i b0 = b[I % (AHEAD + 1)];
+                const v2i b1 = bt[I % (AHEAD + 1)];
+                const v8i B = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], 0, 0};
 #pragma unroll
                 for (int r = 0; r < RA; ++r) {
-                    const v4i aw = a[RING ? U & 1 : U][r];
+                    const v4i aw = a[U % DA][r];
                     const v8i A = {aw[0], aw[1], aw[2], aw[3], 0, 0, 0, 0};
-                    acc[r][G] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, acc[r][G], 4, 0, U, (int)sca[r], J, sbv[G]);
+                    acc[r][G] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, acc[r][G], 4, 2, U, (int)sca[r], J, sbv[G]);
                     asm volatile("" : "+v"(acc[r][G]));  /* (or the compiler sinks every product to the end of the loop body) */
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -864,25 +893,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED
             for (int i = 0; i < AHEAD; ++i) read(i);
             __builtin_amdgcn_sched_barrier(0);
             mt_steps(step, std::make_integer_sequence<int, TB * MT_PLANES>{});
-            if (c + 1 < run) {
+            if (!LAST || U < 3) {
                 PG_MT_PUT_B((U + 1) & 1, (U + 1) % BD);
-                if (c + 1 + BD < run) PG_MT_FETCH_B((U + 1) % BD, chunk_at(c + 1 + BD));
+                __builtin_amdgcn_sched_barrier(0);
+                if (!LAST || U + 1 + BD < 4) PG_MT_FETCH_B((U + 1) % BD, chunk_at(c + 1 + BD < run ? c + 1 + BD : run - 1));
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (RING && c + 2 < run) fetch_a(a[RING ? U & 1 : 0], chunk_at(c + 2));
-            __syncthreads();
+            if (!LAST || U + DA < 4) fetch_a(a[U % DA], chunk_at(c + DA));
+            asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");  // (the loads stay in flight)
         };
         mt_steps(chunk, std::make_integer_sequence<int, 4>{});
-        if (more) {
+        if (!LAST) {
 #pragma unroll
             for (int r = 0; r < RA; ++r) sca[r] = sca_next[r];
-            if (!RING) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int r = 0; r < RA; ++r) a[RING ? 0 : u][r] = an[RING ? 0 : u][r];
-            }
         }
-    }
+    };
+#pragma unroll 1
+    for (int cb = 0; cb + 4 < run; cb += 4) batch(cb, std::false_type{});
+    batch(run - 4, std::true_type{});
 #undef PG_MT_FETCH_B
 #undef PG_MT_PUT_B
     // D: lane holds token lane % 16 of its group, weight rows 4 (lane / 16) .. + 3 of the row group
@@ -931,7 +959,7 @@ pg_status launch_tiles(pg_ctx *ctx, const pg_gguf_tensor *w, const char *bq, flo
 template <int RA, int TB, int BD, int NW = MT_NW>
 pg_status launch_tiles_grouped(pg_ctx *ctx, size_t n_out, int ncp, const char *bq, float *y, size_t n_wt, size_t max_tiles,
                                const mt_gather &gat, const mt_experts &ex) {
-    const size_t lds = TB == 1 ? std::max<size_t>(2 * MT_RECORD, 2 * 4 * (2 * 2048 + 256)) : 2 * (size_t)TB * MT_RECORD;  // (mxfp4_narrow_tile<RA, 2>)
+    const size_t lds = TB == 1 ? std::max<size_t>(2 * MT_RECORD, 2 * 4 * (2 * MT_FRAG + 256)) : 2 * (size_t)TB * MT_RECORD;  // (mxfp4_narrow_tile<RA, 2>)
     auto kern = mxfp4_tiles_kernel<RA, TB, BD, true, NW>;
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
     const size_t per_xcd = (max_tiles + 7) / 8 * n_wt, items = 8 * per_xcd;
@@ -1206,20 +1234,27 @@ __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__r
 // How the tiles of a grouped product are cut: TB groups of 16 slots, RA groups of 16 weight rows a wavefront, NW wavefronts.
 struct mt_shape { int tb, ra, nw; };
 
-// Up to twelve slots an expert on average (narrow tiles, most of them): one group of slots, and the widest row tile that leaves every CU
-// two workgroups.  Beyond, the tiling of least estimated time for both products together: a chunk takes `chunk` and, for every
-// workgroup of the fullest CU, `wg` us (the tail tiles' empty groups are skipped); the experts' slots as binomials.  Timed on 349
-// shapes (10 to 512 tokens, 8 to 32 experts, 512 to 2880 wide), every tiling of each product: 1 to 2 % over the better of the two
-// rules up to 80 tokens, 7 % over the best tiling beyond, where the old rule (slots by the average, rows by two workgroups a CU) is 10 to
-// 20 % over it.  us, before : now: 471 tokens, 8 experts, 2784 x 672 116 : 88, 410, 16, 1312 x 864 105 : 85, 208, 32, 2272 x 1696
-// 139 : 117, 512, 8, 2048 x 2048 206 : 166; 64 slots, 32 experts
-// of 2880 x 2880, where tiles of 32 take 246 and 1075: 300 tokens 235, 2000 958.
-struct mt_cost { mt_shape s; double chunk, wg; };
-constexpr mt_cost MT_COSTS[] = {{{1, 1, 8}, 0.112, 0.542}, {{2, 1, 8}, 0.128, 0.807}, {{2, 2, 8}, 0.059, 1.192}, {{2, 4, 8}, 0.404, 1.238},
-                                {{2, 4, 4}, 0.784, 0.528}, {{4, 4, 8}, 0.414, 1.9}};
+// The tiling of least estimated time for both products together.  `load` workgroups stand on the fullest CU (between the average and
+// the whole number above it); a launch takes begin + load * each, a chunk of it `chunk` + load * wg (tail tiles skip their empty
+// groups, of which only the part `fixed` is paid), and no less than the weights of the experts that are hit at `rate` TB/s, the two
+// joined by a fourth power.  The experts' slots are binomials.  Timed on 720 shapes (16 to 1700 tokens, 4 to 32 experts, 256 to
+// 3800 wide), ten tilings of each product: the choice is 2 % over the best one on average; 64 slots, and 32 on eight wavefronts,
+// were the best by 0.4 % where they were at all.
+// Where hardly a tile is half full (six slots an expert on average, or twelve if the weights alone take 40 us), the estimates err by
+// up to 40 % for 32 slots, which pay for 16: one group of slots, and the widest row tile that leaves every CU two workgroups.  (60
+// tokens over 32 experts of 2144 x 1280, top 2: 60 us, by the estimates 75; 90 over 32 of 2880 x 2880, top 4: 131, as 32 slots 143.)
+struct mt_cost { mt_shape s; double begin, chunk, wg, fixed, each, rate; };
+constexpr mt_cost MT_COSTS[] = {{{1, 1, 8}, 1.33, 0.197, 0.466, 0.00, 0.92, 8.00},
+                                {{1, 2, 8}, 1.01, 0.089, 0.703, 0.00, 1.80, 6.92},
+                                {{1, 4, 8}, 0.00, 0.000, 1.070, 0.00, 3.66, 5.53},
+                                {{2, 1, 4}, 2.95, 0.183, 0.279, 0.34, 0.61, 3.86},
+                                {{2, 2, 4}, 3.35, 0.176, 0.319, 0.04, 0.92, 4.93},
+                                {{2, 4, 4}, 3.81, 0.183, 0.528, 0.00, 1.53, 5.23}};
 void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const size_t (&n_out)[2], const int (&ncp)[2], mt_shape (&out)[2]) {
     const size_t P = T * top_k, cus = (size_t)ctx->num_cu;
-    if (P < 12 * E) {
+    const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));
+    auto bytes = [&](int i) { return hit * (double)n_out[i] * ncp[i] * 68.0; };
+    if (P < 6 * E || (P < 12 * E && (bytes(0) + bytes(1)) / 5.6e6 > 40.0)) {
         const size_t max_tiles = P / 16 + E;
         for (int i = 0; i < 2; ++i) {
             const size_t nrg = (n_out[i] + 15) / 16;
@@ -1230,10 +1265,9 @@ void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const siz
         return;
     }
     double best = 1e300;
-    for (int tb = 1; tb <= 4; tb *= 2) {
+    for (int tb = 1; tb <= 2; ++tb) {
         const double tiles = pg_moe_expected_tiles(T, E, top_k, 16 * tb);
-        const double live = tb == 1 ? 1.0 : 0.4 + 0.6 * std::min(1.0, ((double)P / 16.0 + 0.5 * (double)E) / (tiles * tb));
-        const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));
+        const double live = std::min(1.0, ((double)P / 16.0 + 0.5 * hit) / (tiles * tb));
         mt_shape pick[2] = {};
         double sum = 0.0;
         for (int i = 0; i < 2; ++i) {
@@ -1242,8 +1276,9 @@ void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const siz
             for (const mt_cost &c : MT_COSTS) {
                 if (c.s.tb != tb || (size_t)c.s.ra > nrg) continue;
                 const double w = std::max(1.0, tiles * (double)((nrg + c.s.nw * c.s.ra - 1) / (c.s.nw * c.s.ra)) / (double)cus);
-                const double stream = hit * (double)n_out[i] * ncp[i] * 68.0 / 5.6e6;  // (the weights once)
-                const double us = std::max(stream, 1.0 + ncp[i] * (c.chunk + c.wg * 0.5 * (w + ceil(w)) * live));
+                const double load = 0.5 * (w + ceil(w));
+                const double work = c.begin + load * c.each + ncp[i] * (c.chunk + load * c.wg * (c.fixed + (1.0 - c.fixed) * live));
+                const double us = pow(pow(work, 4.0) + pow(3.0 + bytes(i) / (c.rate * 1e6), 4.0), 0.25);
                 if (us < least) {
                     least = us;
                     pick[i] = c.s;
@@ -1274,8 +1309,7 @@ pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, 
                            reinterpret_cast<const uint32_t *const *>(tab + (size_t)(2 * which + 1) * experts)};
 #define PG_MTG(TB, RA, BD, NW) \
     if (sh.tb == TB && sh.ra == RA && sh.nw == NW) return launch_tiles_grouped<RA, TB, BD, NW>(ctx, n_out, ncp, bq, y, n_wt, max_tiles, gat, ex);
-    PG_MTG(1, 1, 4, 8) PG_MTG(1, 2, 2, 8) PG_MTG(1, 4, 4, 8)
-    PG_MTG(2, 1, 4, 8) PG_MTG(2, 2, 4, 8) PG_MTG(2, 4, 2, 8) PG_MTG(2, 4, 2, 4) PG_MTG(4, 4, 1, 8)
+    PG_MTG(1, 1, 4, 8) PG_MTG(1, 2, 2, 8) PG_MTG(1, 4, 4, 8) PG_MTG(2, 1, 4, 4) PG_MTG(2, 2, 1, 4) PG_MTG(2, 4, 1, 4)
 #undef PG_MTG
     return pg_fail(PG_EUNSUPPORTED, "mxfp4 moe: no kernel of %d x 16 slots, %d row groups, %d wavefronts", sh.tb, sh.ra, sh.nw);
 }

@@ -77,8 +77,9 @@ PG_HD int pg_mx_chunk(int c, int ncp) { return c < ncp ? c : ncp - 1; }
 PG_HD int pg_mx_scale_word(int c, int ncp) { return (c < ncp ? c : ncp - 4) >> 2; }
 
 // ---- MXFP4 over many rows (mxfp4_planes_kernel writes the token records, mxfp4_tiles_kernel reads them and the weights)
-// A record = one token group of 16 and one chunk of 128 k: PG_MT_PLANES operand fragments of 2 KiB, then 64 scale dwords.
-constexpr int PG_MT_PLANES = 4, PG_MT_FRAG = 2048, PG_MT_RECORD = PG_MT_PLANES * PG_MT_FRAG + 256, PG_MT_NW = 8;
+// A record = one token group of 16 and one chunk of 128 k: PG_MT_PLANES operand fragments of 64 lanes x 24 bytes (the lanes' first 16,
+// then their last 8), then 64 scale dwords.
+constexpr int PG_MT_PLANES = 4, PG_MT_FRAG = 1536, PG_MT_RECORD = PG_MT_PLANES * PG_MT_FRAG + 256, PG_MT_NW = 8;
 // chunks a row of nb blocks is padded to: whole scale dwords (4 chunks of 4 blocks)
 PG_HD size_t pg_mx_chunks(size_t nb) { return ((nb + 3) / 4 + 3) & ~(size_t)3; }
 // first of the `ra` row groups a wavefront reads, from the first one it owns: past the tensor's end it repeats the last ones
@@ -91,10 +92,13 @@ PG_HD unsigned pg_mt_unit_offset(int u, int units, int ncp) {
     u = u < units ? u : units - 1;
     return (unsigned)(u / (PG_MT_RECORD / 16)) * (unsigned)ncp * PG_MT_RECORD + (unsigned)(u % (PG_MT_RECORD / 16)) * 16;
 }
-// byte offset of the 16 bytes of plane j that hold k = 32 (b % 4) + 16 sub .. + 15 of chunk b / 4 for token `col` of group tg
-PG_HD size_t pg_mt_plane_store(size_t tg, int ncp, int b, int sub, int col, int j) {
-    const int k0 = 32 * (b & 3) + 16 * sub, half = k0 >> 6, q = (k0 & 63) >> 4;
-    return (tg * ncp + (size_t)(b >> 2)) * PG_MT_RECORD + (size_t)j * PG_MT_FRAG + half * 1024 + (col + 16 * q) * 16;
+// byte offset of the lane of plane j that holds block b of token `col` of group tg: its 32 digits of 6 bits, the first 16 bytes here
+// (elements 0 .. 15 in 12 of them), the last 8 at pg_mt_plane_tail
+PG_HD size_t pg_mt_plane_store(size_t tg, int ncp, int b, int col, int j) {
+    return (tg * ncp + (size_t)(b >> 2)) * PG_MT_RECORD + (size_t)j * PG_MT_FRAG + (size_t)(col + 16 * (b & 3)) * 16;
+}
+PG_HD size_t pg_mt_plane_tail(size_t tg, int ncp, int b, int col, int j) {
+    return (tg * ncp + (size_t)(b >> 2)) * PG_MT_RECORD + (size_t)j * PG_MT_FRAG + 1024 + (size_t)(col + 16 * (b & 3)) * 8;
 }
 // byte offset of the scale dword of block b for token `col` of group tg
 PG_HD size_t pg_mt_scale_store(size_t tg, int ncp, int b, int col) {

@@ -326,6 +326,35 @@ def test_mxfp4_moe_tilings(ctx, orc, hidden, inter, E, top_k, T):
     test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, T)
 
 
+@pytest.mark.parametrize("hidden,inter,E,top_k,T", [(96, 480, 130, 4, 194), (96, 992, 130, 4, 194)])
+def test_mxfp4_moe_narrow_tilings(ctx, orc, hidden, inter, E, top_k, T):
+    """32 and 64 weight rows a wavefront over tiles of 16 slots: six tokens an expert, so full tiles and both narrow forms."""
+    test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, T)
+
+
+@pytest.mark.parametrize("m", [24, 40, 70])
+def test_mxfp4_tiles_digits_at_their_ends(ctx, m):
+    """The largest digits of every plane, and the largest scales: one weight of 1 a row, so a product is its block's first value.  A
+    block is held in units of 2^-19 of the power of two above its largest value, which the first is: half a unit is at most 2^-19
+    of it, and the result is rounded once more (2^-24)."""
+    from peregrine_amd import mxfp4
+    k, n = 160, 33
+    rng = np.random.default_rng(m)
+    b = np.zeros((n, k // 2), np.uint8)
+    b[:, 0] = 0x02                                         # element 0: 1.0
+    s = np.full(n * k // 32, 97, np.uint8)                 # 2^-30
+    ends = [3.4028234663852886e38, -3.4028234663852886e38, 1.0, -1.0, 2.0 ** -60, 2.0 ** 20 - 1, 541200.0, -541200.0, 16.0, 17.0, 528.0, -16912.0]
+    x = np.zeros((m, k), np.float32)
+    x[:, 0] = np.resize(np.array(ends, np.float32), m)
+    x[:, 1:32] = x[:, :1] * rng.uniform(-1, 1, (m, 31)).astype(np.float32)
+    x[:, 40] = 7.0                                         # (a block without weights)
+    w = mxfp4.upload(b.reshape(-1), s, n, k, ctx)
+    got = w.matmul(x, m).reshape(m, n).astype(np.float64)
+    want = x[:, :1].astype(np.float64) * 2.0 ** -30
+    assert (np.abs(got - want) <= np.abs(want) * (2.0 ** -19 + 2.0 ** -24)).all()
+    w.free()
+
+
 @pytest.mark.parametrize("E,T", [(63, 30), (64, 41), (65, 30), (127, 60), (128, 200), (129, 23), (256, 300)])
 def test_mxfp4_moe_finds_the_expert_of_a_tile(ctx, orc, E, T):
     """The offsets of 64 experts are looked through at a time: the last expert of a run, the first of the next, and one run more for
