@@ -36,6 +36,10 @@ typedef int v6i __attribute__((ext_vector_type(6)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef const v4i __attribute__((address_space(1))) *gv4i_ptr;
+// (a pointer out of a table is not known to lead to global memory: the compiler reads through it by flat loads, which count as LDS
+// reads too, and every wait for LDS then waits for memory)
+typedef const uint32_t __attribute__((address_space(1))) *gu32_ptr;
+typedef const float __attribute__((address_space(1))) *gf32_ptr;
 
 constexpr int MX_PLANES = 5;  // digit planes per activation row
 constexpr int MX_U = 8;       // chunks (of 4 blocks) per batch of weight loads in flight
@@ -611,11 +615,12 @@ struct mt_experts {
 // A token tile with at most 16 / NPM slots in use: the spare columns of the B operand take NPM planes of each token (column
 // = token * NPM + plane), so a chunk is 4 / NPM instructions instead of four, and only the operand bytes of those tokens
 // pass through LDS, a batch of four chunks at a time (one barrier a batch).  The planes' sums are joined at the end.
-// Twenty tokens over 32 experts of 2880 x 2880, top 4 (2.7 slots a tile): the two products 71 + 40 -> 51 + 29 us, 250 and
-// 125 MB at 4.9 and 4.3 TB/s; before, the instructions and LDS reads of 16 slots took 40 us beside the stream, and 142
-// registers left one workgroup a CU with 64 KB of weights on their way (now 128 and two).
+// Bound by the weights' stream: twenty tokens over 32 experts of 2880 x 2880, top 4 (2.7 slots a tile), 250 and 125 MB in 49 and
+// 27.6 us, 5.1 and 4.5 TB/s (as full tiles 71 + 40; with the next batch beside the current one in registers, copied, 51 + 30.5;
+// scales by flat loads and the ring 51 + 28.8): a ring keeps four chunks under way at every moment and takes 95 registers
+// where two batches took 128.
 template <int RA, int NPM>
-__device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, const uint32_t *__restrict__ sa, const char *__restrict__ bq,
+__device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, const gu32_ptr sa, const char *__restrict__ bq,
                                                   int ncp, int turn, v4f (&acc)[RA]) {
     constexpr int NI = MT_PLANES / NPM, CHUNK = NI * MT_FRAG + 256, STAGE = 4 * CHUNK;
     const int lane = threadIdx.x & 63, t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -645,13 +650,13 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
         if (wave == 0) *reinterpret_cast<v4i *>(lds + stage * STAGE + s_dst) = ss;
     };
     auto chunk_at = [&](int i) { return i + turn < ncp ? i + turn : i + turn - ncp; };
-    v4i a[4][RA], an[4][RA];
+    v4i a[4][RA];  // a ring: a chunk's weights are read as soon as the same place of the batch before is used
     uint32_t sca[RA], sca_next[RA];
-    auto fetch_a = [&](v4i (&dst)[4][RA], uint32_t (&sc)[RA], int c) {
+    auto fetch_a = [&](int u, int c) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int r = 0; r < RA; ++r) dst[u][r] = __builtin_nontemporal_load(qa + (size_t)r * a_stride + (size_t)(c + u) * 64 + lane);
+        for (int r = 0; r < RA; ++r) a[u][r] = __builtin_nontemporal_load(qa + (size_t)r * a_stride + (size_t)(c + u) * 64 + lane);
+    };
+    auto fetch_s = [&](uint32_t (&sc)[RA], int c) {
 #pragma unroll
         for (int r = 0; r < RA; ++r) sc[r] = sa[((size_t)r * (ncp / 4) + (c >> 2)) * 64 + lane];
     };
@@ -660,15 +665,16 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
 #pragma unroll
     for (int r = 0; r < RA; ++r) acc[r] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     fetch_b(chunk_at(0));
-    fetch_a(a, sca, chunk_at(0));
+    fetch_s(sca, chunk_at(0));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) fetch_a(u, chunk_at(0));
     put_b(0);
-    if (4 < ncp) fetch_b(chunk_at(4));
-    __syncthreads();
-#pragma unroll 1
-    for (int cb = 0, s = 0; cb < ncp; cb += 4, s ^= 1) {
-        const bool more = cb + 4 < ncp;
-        if (more) fetch_a(an, sca_next, chunk_at(cb + 4));
-        __builtin_amdgcn_sched_barrier(0);
+    fetch_b(chunk_at(4 < ncp ? 4 : 0));
+    asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");
+    auto batch = [&](int cb, int s, auto last_) {
+        constexpr bool LAST = decltype(last_)::value;
+        const int next = chunk_at(cb + 4 < ncp ? cb + 4 : 0);
+        if (!LAST) fetch_s(sca_next, next);
         const char *st = lds + s * STAGE;
 #define PG_MT_STEP(U, I)                                                                                                   \
     do {                                                                                                                   \
@@ -687,6 +693,8 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
     do {                                    \
         PG_MT_STEP(U, 0);                   \
         if constexpr (NI == 2) PG_MT_STEP(U, 1); \
+        if (!LAST) fetch_a(U, next);        \
+        __builtin_amdgcn_sched_barrier(0);  \
     } while (0)
         static_assert(NI == 1 || NI == 2, "the instructions of a chunk are written out");
         PG_MT_STEPS(0);
@@ -695,20 +703,20 @@ __device__ __forceinline__ void mxfp4_narrow_tile(char *lds, const gv4i_ptr qa, 
         PG_MT_STEPS(3);
 #undef PG_MT_STEPS
 #undef PG_MT_STEP
-        if (more) {
+        if (!LAST) {
             put_b(s ^ 1);
-            if (cb + 8 < ncp) fetch_b(chunk_at(cb + 8));
+            fetch_b(chunk_at(cb + 8 < ncp ? cb + 8 : 0));
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");  // (not __syncthreads(): the loads stay in flight)
-        if (more) {
+        if (!LAST) {
 #pragma unroll
             for (int r = 0; r < RA; ++r) sca[r] = sca_next[r];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int r = 0; r < RA; ++r) a[u][r] = an[u][r];
         }
-    }
+    };
+    int s = 0;
+#pragma unroll 1
+    for (int cb = 0; cb + 4 < ncp; cb += 4, s ^= 1) batch(cb, s, std::false_type{});
+    batch(ncp - 4, s, std::true_type{});
 #pragma unroll
     for (int r = 0; r < RA; ++r)  // every lane of a token's columns: the sum over the planes
 #pragma unroll
@@ -777,7 +785,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(GROUPED
     const int rg0 = pg_mt_first_row_group(rg_mine, RA, nrg);  // the ones it reads: a spare wavefront repeats the last ones
     const size_t a_stride = (size_t)ncp * 64;                // v4i per row group
     const gv4i_ptr qa = (gv4i_ptr)(uintptr_t)qs_frag + (size_t)rg0 * a_stride;
-    const uint32_t *const sa = sc_frag + (size_t)rg0 * (ncp / 4) * 64;
+    const gu32_ptr sa = (gu32_ptr)(uintptr_t)sc_frag + (size_t)rg0 * (ncp / 4) * 64;
     if constexpr (GROUPED && TB == 1) {
         const int first = (tt - at.first_tile) * 16, used = at.used - first;
         if (used <= 8) {
@@ -1218,7 +1226,7 @@ __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__r
         }
         float b[CH];
 #pragma unroll
-        for (int j = 0; j < CH; ++j) b[j] = bias_tab[e[j]][c];
+        for (int j = 0; j < CH; ++j) b[j] = ((gf32_ptr)(uintptr_t)bias_tab[e[j]])[c];
 #pragma unroll
         for (int j = 0; j < CH; ++j)
             if (k0 + j < top_k) {
@@ -1234,22 +1242,23 @@ __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__r
 // How the tiles of a grouped product are cut: TB groups of 16 slots, RA groups of 16 weight rows a wavefront, NW wavefronts.
 struct mt_shape { int tb, ra, nw; };
 
-// The tiling of least estimated time for both products together.  `load` workgroups stand on the fullest CU (between the average and
-// the whole number above it); a launch takes begin + load * each, a chunk of it `chunk` + load * wg (tail tiles skip their empty
-// groups, of which only the part `fixed` is paid), and no less than the weights of the experts that are hit at `rate` TB/s, the two
-// joined by a fourth power.  The experts' slots are binomials.  Timed on 720 shapes (16 to 1700 tokens, 4 to 32 experts, 256 to
-// 3800 wide), ten tilings of each product: the choice is 2 % over the best one on average; 64 slots, and 32 on eight wavefronts,
-// were the best by 0.4 % where they were at all.
+// The tiling of least estimated time for both products together.  `load` workgroups stand on the fullest CU (the average and the part
+// `whole` of what is missing to the number above it); a launch takes begin + load * each, a chunk of it `chunk` + load * wg, of which
+// empty groups of tail tiles and empty slots of single-group tiles cost only the part `fixed`; the weights of the experts that are hit
+// come at `rate` TB/s.  The two times are joined by a square for tiles of 16 slots and by a seventh power for 32, whose arithmetic
+// hides the stream better.  The experts' slots are binomials.  Timed on 770 shapes (16 to 1700 tokens, 4 to 32 experts, 256 to 3800
+// wide), every tiling of each product: the choice is 2 % over the best one on average; 64 slots, and 32 on eight wavefronts, would
+// give another 0.4 %.
 // Where hardly a tile is half full (six slots an expert on average, or twelve if the weights alone take 40 us), the estimates err by
 // up to 40 % for 32 slots, which pay for 16: one group of slots, and the widest row tile that leaves every CU two workgroups.  (60
-// tokens over 32 experts of 2144 x 1280, top 2: 60 us, by the estimates 75; 90 over 32 of 2880 x 2880, top 4: 131, as 32 slots 143.)
-struct mt_cost { mt_shape s; double begin, chunk, wg, fixed, each, rate; };
-constexpr mt_cost MT_COSTS[] = {{{1, 1, 8}, 1.33, 0.197, 0.466, 0.00, 0.92, 8.00},
-                                {{1, 2, 8}, 1.01, 0.089, 0.703, 0.00, 1.80, 6.92},
-                                {{1, 4, 8}, 0.00, 0.000, 1.070, 0.00, 3.66, 5.53},
-                                {{2, 1, 4}, 2.95, 0.183, 0.279, 0.34, 0.61, 3.86},
-                                {{2, 2, 4}, 3.35, 0.176, 0.319, 0.04, 0.92, 4.93},
-                                {{2, 4, 4}, 3.81, 0.183, 0.528, 0.00, 1.53, 5.23}};
+// tokens over 32 experts of 2144 x 1280, top 2: 58 us, as 32 slots 75; 90 over 32 of 2880 x 2880, top 4: 124, as 32 slots 143.)
+struct mt_cost { mt_shape s; double begin, chunk, wg, fixed, each, rate, whole; };
+constexpr mt_cost MT_COSTS[] = {{{1, 1, 8}, 0.97, 0.113, 0.387, 0.14, 0.95, 7.23, 0.65},
+                                {{1, 2, 8}, 0.66, 0.010, 0.674, 0.24, 1.63, 7.18, 0.75},
+                                {{1, 4, 8}, 0.00, 0.000, 1.014, 0.27, 3.22, 6.42, 1.00},
+                                {{2, 1, 4}, 3.07, 0.105, 0.289, 0.40, 0.50, 3.54, 0.69},
+                                {{2, 2, 4}, 3.21, 0.164, 0.314, 0.11, 0.86, 4.64, 0.71},
+                                {{2, 4, 4}, 3.72, 0.148, 0.505, 0.00, 1.49, 5.03, 0.77}};
 void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const size_t (&n_out)[2], const int (&ncp)[2], mt_shape (&out)[2]) {
     const size_t P = T * top_k, cus = (size_t)ctx->num_cu;
     const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));
@@ -1267,7 +1276,8 @@ void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const siz
     double best = 1e300;
     for (int tb = 1; tb <= 2; ++tb) {
         const double tiles = pg_moe_expected_tiles(T, E, top_k, 16 * tb);
-        const double live = std::min(1.0, ((double)P / 16.0 + 0.5 * hit) / (tiles * tb));
+        const double live = tb == 1 ? (double)P / (16.0 * tiles) : std::min(1.0, ((double)P / 16.0 + 0.5 * hit) / (tiles * tb));
+        const double joined = tb == 1 ? 2.0 : 7.0;
         mt_shape pick[2] = {};
         double sum = 0.0;
         for (int i = 0; i < 2; ++i) {
@@ -1276,9 +1286,9 @@ void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const siz
             for (const mt_cost &c : MT_COSTS) {
                 if (c.s.tb != tb || (size_t)c.s.ra > nrg) continue;
                 const double w = std::max(1.0, tiles * (double)((nrg + c.s.nw * c.s.ra - 1) / (c.s.nw * c.s.ra)) / (double)cus);
-                const double load = 0.5 * (w + ceil(w));
+                const double load = w + c.whole * (ceil(w) - w);
                 const double work = c.begin + load * c.each + ncp[i] * (c.chunk + load * c.wg * (c.fixed + (1.0 - c.fixed) * live));
-                const double us = pow(pow(work, 4.0) + pow(3.0 + bytes(i) / (c.rate * 1e6), 4.0), 0.25);
+                const double us = pow(pow(work, joined) + pow(3.0 + bytes(i) / (c.rate * 1e6), joined), 1.0 / joined);
                 if (us < least) {
                     least = us;
                     pick[i] = c.s;
