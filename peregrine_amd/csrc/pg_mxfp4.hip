@@ -1197,25 +1197,29 @@ namespace {
 
 // output[t] += weight * (out + mlp2_bias) over the token's experts in the order given  (examples/gpt_oss/moe.rs:104-108, 330-334)
 // out[t] = sum_k weight (y + bias2), k ascending; idx and weight as the caller chose them or already put in order (mx_routed).  CH
-// entries' loads are in flight together.
+// entries' loads are in flight together.  `per` workgroups a token, so its entries, their experts and the bias rows' addresses are
+// the same for a workgroup and are scalars; a thread owns four columns (hidden is a multiple of 32).  Bound by three dependent
+// reads, entry, table and bias: 421 tokens x 4 of 1280 columns 7.7 -> 5.7 us (one column a thread), 20 x 4 of 2880 4.8 -> 4.7.
 template <int CH>
 __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__restrict__ yb, const float *const *__restrict__ bias_tab,
                                                                 const int *__restrict__ idx, const float *__restrict__ weight,
-                                                                size_t tokens, size_t hidden, int top_k, int experts, float *__restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= tokens * hidden) return;
-    const size_t t = i / hidden, c = i - t * hidden;
+                                                                unsigned per, unsigned hidden, int top_k, int experts, float *__restrict__ out) {
+    typedef const v4f __attribute__((address_space(1))) *gv4f_ptr;
+    const size_t t = blockIdx.x / per;
+    const unsigned c = (blockIdx.x % per) * blockDim.x + threadIdx.x;
+    if (c >= hidden / 4) return;
     mx_routed taken;
-    float acc = 0.0f;
+    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int k0 = 0; k0 < top_k; k0 += CH) {
         int e[CH];
-        float w[CH], v[CH];
+        float w[CH];
+        v4f v[CH], b[CH];
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
             const size_t p = t * top_k + (k0 + j < top_k ? k0 + j : top_k - 1);
-            e[j] = idx[p];
+            v[j] = *reinterpret_cast<const v4f *>(yb + p * hidden + c * 4);
+            e[j] = __builtin_amdgcn_readfirstlane(idx[p]);
             w[j] = weight[p];
-            v[j] = yb[p * hidden + c];
         }
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
@@ -1224,17 +1228,25 @@ __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__r
             else e[j] = e[0];
             w[j] = named ? w[j] : 0.0f;
         }
-        float b[CH];
 #pragma unroll
-        for (int j = 0; j < CH; ++j) b[j] = ((gf32_ptr)(uintptr_t)bias_tab[e[j]])[c];
+        for (int j = 0; j < CH; ++j) b[j] = ((gv4f_ptr)(uintptr_t)mx_uniform(bias_tab + e[j]))[c];
 #pragma unroll
         for (int j = 0; j < CH; ++j)
             if (k0 + j < top_k) {
-                const float result = v[j] + b[j], prod = w[j] * result;
-                acc = acc + prod;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const float result = v[j][x] + b[j][x], prod = w[j] * result;
+                    acc[x] = acc[x] + prod;
+                }
             }
     }
-    out[i] = acc;
+    float *const o = out + t * hidden + c * 4;
+    if (((uintptr_t)out & 15) == 0) {
+        *reinterpret_cast<v4f *>(o) = acc;
+    } else {  // (the caller's pointer may be any float's)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) o[x] = acc[x];
+    }
 }
 
 // One grouped product: rows `src` (pair / div) of the experts' slots -> records -> tiles against tensor table `which`.
@@ -1420,9 +1432,11 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
         PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, shape[0], max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
         PG_TRY(moe_product(ctx, h, inter, hidden, shape[1], max_tiles, gat, 1, tab, E, 1, rec, yb, &sw));
     }
-    return pg_launch(ctx, "mxfp4_moe_combine", top_k <= 2 ? mxfp4_moe_combine_kernel<2> : mxfp4_moe_combine_kernel<4>, dim3(grid_for(T * hidden, 256)), dim3(256), 0, (const float *)yb,
-                     reinterpret_cast<const float *const *>(tab + 5 * E), by_pairs ? expert_idx_dev : (const int *)topk_idx,
-                     by_pairs ? weight_dev : (const float *)topk_p, T, hidden, (int)top_k, (int)E, out_dev);
+    const unsigned wg = (unsigned)std::min<size_t>(256, pg_round_up(hidden / 4, 64)), per = grid_for(hidden / 4, wg);
+    PG_CHECK_ARG(T * per < ((size_t)1 << 31), "pg_mxfp4_moe_ffn: %zu tokens of %zu outputs in one launch", T, hidden);
+    return pg_launch(ctx, "mxfp4_moe_combine", top_k <= 2 ? mxfp4_moe_combine_kernel<2> : mxfp4_moe_combine_kernel<4>, dim3((unsigned)(T * per)), dim3(wg), 0,
+                     (const float *)yb, reinterpret_cast<const float *const *>(tab + 5 * E), by_pairs ? expert_idx_dev : (const int *)topk_idx,
+                     by_pairs ? weight_dev : (const float *)topk_p, per, (unsigned)hidden, (int)top_k, (int)E, out_dev);
 }
 
 PG_API pg_status pg_mxfp4_moe_ffn_routed(pg_ctx *ctx, const float *x, size_t T, const int32_t *expert_idx, const float *weight,

@@ -374,3 +374,40 @@ def test_moe_tiles_of_all_experts(ctx, orc, T, E, top_k, d, ffn, typ):
         want, _, _ = orc.moe_ffn(x.reshape(-1), T, d, ffn, E, top_k, logits, *full, typ, moe.SILU)
         for t in range(T):
             H.assert_close_rel(got[t], want[t], MOE_RTOL, f"{name}, token {t}")
+
+
+@pytest.mark.parametrize("T,d,top_k", [(3, 160, 3), (7, 1056, 2), (65, 2080, 1)])
+@pytest.mark.parametrize("form", ["block", "mxfp4"])
+def test_layer_outputs_at_any_float(ctx, orc, form, T, d, top_k):
+    """The sum over a token's experts goes out four columns at a time where the output allows it: the same bits at an output that
+    begins one float further on, and nothing written before or behind it.  One and three workgroups a token, odd numbers of entries."""
+    import ctypes as C
+    from peregrine_amd import gguf, moe, mxfp4, _ffi
+    from devbuf import DevBuf
+    E, ffn = 4, 96
+    rng = np.random.default_rng(T + d)
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    idx = np.stack([rng.permutation(E)[:top_k] for _ in range(T)]).astype(np.int32)
+    w = rng.uniform(0.2, 1.0, (T, top_k)).astype(np.float32)
+    dx, di, dw = DevBuf(ctx, host=x), DevBuf(ctx, host=idx), DevBuf(ctx, host=w)
+    if form == "block":
+        raws = build(orc, 77, d, ffn, E, 8)
+        mk = lambda rs, n_out, k_in: [gguf.GgufWeight(r, 8, n_out, k_in, ctx) for r in rs]
+        ex = moe.MoEExperts(mk(raws[0], ffn, d), mk(raws[1], ffn, d), mk(raws[2], d, ffn), top_k, moe.SILU, ctx)
+        (g, _g), (u, _u), (dn, _d) = ex._table(ex.gate), ex._table(ex.up), ex._table(ex.down)
+        call = lambda out: _ffi.lib.pg_moe_ffn_routed_dev(ctx.handle, dx.ptr, T, di.ptr, dw.ptr, E, top_k, g, u, dn, moe.SILU, None, out)
+    else:
+        from test_oracle_formats_pins import _mx_expert
+        some = [mxfp4.Mxfp4Expert(d, ffn, 1.702, 7.0, *_mx_expert(rng, d, ffn), ctx=ctx) for _ in range(E)]
+        tab = (C.c_void_p * E)(*[e._h.value for e in some])
+        call = lambda out: _ffi.lib.pg_mxfp4_moe_ffn_routed_dev(ctx.handle, dx.ptr, T, di.ptr, dw.ptr, top_k, C.cast(tab, C.POINTER(C.c_void_p)), E, out)
+    rows = []
+    for off in (0, 1):
+        buf = DevBuf(ctx, host=np.full(T * d + 8, 7.5, np.float32))
+        _ffi.check(call(C.c_void_p(C.cast(buf.ptr, C.c_void_p).value + 4 * off)))
+        ctx.sync()
+        got = buf.to_host(np.float32)
+        assert (got[:off] == 7.5).all() and (got[off + T * d:] == 7.5).all()
+        rows.append(got[off:off + T * d])
+    assert np.isfinite(rows[0]).all() and (rows[0] != 7.5).any()
+    np.testing.assert_array_equal(rows[0], rows[1])
