@@ -139,12 +139,33 @@ __global__ __launch_bounds__(1024) void route_lists_kernel(const float *__restri
     const int lane = threadIdx.x & 63;
     for (int e = threadIdx.x >> 6; e < E; e += 16) {
         int base = 0;
-        for (int p0 = 0; p0 < P; p0 += 64) {
-            const int p = p0 + lane;
-            const bool own = p < P && chosen[p] == e;
-            const unsigned long long mask = __ballot(own);
-            if (own) lists[(size_t)e * T + base + __popcll(mask & ((1ull << lane) - 1ull))] = p;
-            base += __popcll(mask);
+        // Past two looks of a pair a lane, four pairs a lane: a look waits for LDS once (1684 pairs 7.5 -> 6.2 us, 480 6.4 -> 5.6; 20 pairs
+        // 5.3, by fours 5.6).
+        if (P <= 128) {
+            for (int p0 = 0; p0 < P; p0 += 64) {
+                const int p = p0 + lane;
+                const bool own = p < P && chosen[p] == e;
+                const unsigned long long mask = __ballot(own);
+                if (own) lists[(size_t)e * T + base + __popcll(mask & ((1ull << lane) - 1ull))] = p;
+                base += __popcll(mask);
+            }
+        } else {
+            for (int p0 = 0; p0 < P; p0 += 256) {
+                const int p = p0 + 4 * lane;
+                const unsigned four = p < P ? *reinterpret_cast<const unsigned *>(chosen + p) : 0u;
+                int before = base;
+                bool own[4];
+    #pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    own[i] = p + i < P && (int)(four >> (8 * i) & 255u) == e;
+                    const unsigned long long mask = __ballot(own[i]);
+                    before += __popcll(mask & ((1ull << lane) - 1ull));
+                    base += __popcll(mask);
+                }
+    #pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (own[i]) lists[(size_t)e * T + before++] = p + i;
+            }
         }
         if (lane == 0) {
             counts[e] = base;
@@ -364,7 +385,7 @@ pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, con
                                 size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts, int *goff, int tile,
                                 const pg_moe_digits *dig) {
     if (route_in_one(T, E, top_k)) {
-        const size_t lds = (router_logits_dev ? T * route_row(E) * sizeof(float) : 0) + T * top_k;
+        const size_t lds = pg_round_up((router_logits_dev ? T * route_row(E) * sizeof(float) : 0) + T * top_k, 4);  // (read four bytes at a time)
         route_digits rd = {};
         if (dig) {
             const int nb = (int)(dig->k / 32);
