@@ -12,7 +12,7 @@
 // pinned memory); a cache's first batch gets exactly that much memory, later ones what the one before took and 1 / 64, and are
 // encoded a second time if they take more.  A batch was 10 launches, 12 copies and 8
 // waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
-// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.25.
+// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.18.
 //
 // The encoder knows where every code starts, so it leaves an index beside the stream (a 16-bit offset per 64 values,
 // 0.25 bit a value): the decoder of such a chunk is one launch that starts a thread per 64 values, with no search for
@@ -800,8 +800,10 @@ struct kv_decode_args {
 
 // A thread decodes SUB_SYMS values from the bit the index names: table and stream in LDS (the workgroup's part of the
 // stream is contiguous), a 64-bit window in registers with the next word already read; the values go through LDS so
-// that the f32 stores are whole lines.  What it takes is the chain of 64 table look-ups: 20 chunks of 262144 values in
-// 19 us, where the search for code boundaries, the scans, the write pass and the scaling launch took 170.
+// that the f32 stores are whole lines.  What it takes is the chain of 64 table look-ups, about 100 ns each:
+// 20 chunks of 262144 values in 14.3 us, 8 of 16384 in 10.8 (16.8 and 13.5 with the window filled up under a branch after every value;
+// the search for code boundaries, the scans, the write pass and the scaling launch took 170).  Loads marked as global memory instead
+// of flat ones are 0.4 us slower here.
 template <bool VEC>
 __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a) {
     constexpr unsigned MAX_WORDS = DEC_PER_WG * KV_MAX_BITS / 32 + 4;
@@ -864,16 +866,19 @@ __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a
         for (unsigned j = 0; j < count; j += 4) {
             unsigned four = 0;
 #pragma unroll
-            for (unsigned i = 0; i < 4; ++i) {
-                const unsigned e = lut[buf >> (64 - KV_MAX_BITS)], l = e >> 8;
-                four |= (e & 255u) << (8 * i);
-                buf <<= l;
-                avail -= l;
-                if (avail <= 32) {
-                    buf |= (unsigned long long)next << (32 - avail);
-                    avail += 32;
-                    k = min(k + 1, MAX_WORDS - 1);
-                    next = words[k];
+            for (unsigned i = 0; i < 4; i += 2) {
+                // more than 32 bits hold two codes: the window is filled up once for both, and without a branch
+                const bool low = avail <= 32;
+                buf |= (unsigned long long)(low ? next : 0u) << ((32 - avail) & 63);
+                avail += low ? 32 : 0;
+                k = min(k + (low ? 1u : 0u), MAX_WORDS - 1);
+                next = words[k];
+#pragma unroll
+                for (unsigned x = 0; x < 2; ++x) {
+                    const unsigned e = lut[buf >> (64 - KV_MAX_BITS)], l = e >> 8;
+                    four |= (e & 255u) << (8 * (i + x));
+                    buf <<= l;
+                    avail -= l;
                 }
             }
             o[j / 4] = four;
