@@ -1198,26 +1198,27 @@ namespace {
 // output[t] += weight * (out + mlp2_bias) over the token's experts in the order given  (examples/gpt_oss/moe.rs:104-108, 330-334)
 // out[t] = sum_k weight (y + bias2), k ascending; idx and weight as the caller chose them or already put in order (mx_routed).  CH
 // entries' loads are in flight together.  `per` workgroups a token, so its entries, their experts and the bias rows' addresses are
-// the same for a workgroup and are scalars; a thread owns four columns (hidden is a multiple of 32).  Bound by three dependent
-// reads, entry, table and bias: 421 tokens x 4 of 1280 columns 7.7 -> 5.7 us (one column a thread), 20 x 4 of 2880 4.8 -> 4.7.
-template <int CH>
+// the same for a workgroup and are scalars; a thread owns one V: four columns (hidden is a multiple of 32), of few outputs
+// one (9 x 4 of 1088 columns 5.2 -> 4.0 us, by fours 5.5).  Bound by three dependent reads, entry, table and bias: 421 tokens x 4 of 1280 columns 7.7 -> 5.7 us (one column a thread), 20 x 4 of 2880 4.8 -> 4.7.
+template <typename V, int CH>
 __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__restrict__ yb, const float *const *__restrict__ bias_tab,
                                                                 const int *__restrict__ idx, const float *__restrict__ weight,
                                                                 unsigned per, unsigned hidden, int top_k, int experts, float *__restrict__ out) {
-    typedef const v4f __attribute__((address_space(1))) *gv4f_ptr;
+    typedef const V __attribute__((address_space(1))) *gV_ptr;
+    constexpr unsigned W = sizeof(V) / 4;
     const size_t t = blockIdx.x / per;
     const unsigned c = (blockIdx.x % per) * blockDim.x + threadIdx.x;
-    if (c >= hidden / 4) return;
+    if (c >= hidden / W) return;
     mx_routed taken;
-    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    float acc[W] = {};
     for (int k0 = 0; k0 < top_k; k0 += CH) {
         int e[CH];
         float w[CH];
-        v4f v[CH], b[CH];
+        V v[CH], b[CH];
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
             const size_t p = t * top_k + (k0 + j < top_k ? k0 + j : top_k - 1);
-            v[j] = *reinterpret_cast<const v4f *>(yb + p * hidden + c * 4);
+            v[j] = reinterpret_cast<const V *>(yb + p * hidden)[c];
             e[j] = __builtin_amdgcn_readfirstlane(idx[p]);
             w[j] = weight[p];
         }
@@ -1229,23 +1230,23 @@ __global__ __launch_bounds__(256) void mxfp4_moe_combine_kernel(const float *__r
             w[j] = named ? w[j] : 0.0f;
         }
 #pragma unroll
-        for (int j = 0; j < CH; ++j) b[j] = ((gv4f_ptr)(uintptr_t)mx_uniform(bias_tab + e[j]))[c];
+        for (int j = 0; j < CH; ++j) b[j] = ((gV_ptr)(uintptr_t)mx_uniform(bias_tab + e[j]))[c];
 #pragma unroll
         for (int j = 0; j < CH; ++j)
             if (k0 + j < top_k) {
 #pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const float result = v[j][x] + b[j][x], prod = w[j] * result;
+                for (unsigned x = 0; x < W; ++x) {
+                    const float result = reinterpret_cast<const float *>(&v[j])[x] + reinterpret_cast<const float *>(&b[j])[x], prod = w[j] * result;
                     acc[x] = acc[x] + prod;
                 }
             }
     }
-    float *const o = out + t * hidden + c * 4;
-    if (((uintptr_t)out & 15) == 0) {
-        *reinterpret_cast<v4f *>(o) = acc;
+    float *const o = out + t * hidden + c * W;
+    if (W == 4 && ((uintptr_t)out & 15) == 0) {
+        *reinterpret_cast<v4f *>(o) = v4f{acc[0], acc[1 % W], acc[2 % W], acc[3 % W]};
     } else {  // (the caller's pointer may be any float's)
 #pragma unroll
-        for (int x = 0; x < 4; ++x) o[x] = acc[x];
+        for (unsigned x = 0; x < W; ++x) o[x] = acc[x];
     }
 }
 
@@ -1432,9 +1433,13 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
         PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, shape[0], max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
         PG_TRY(moe_product(ctx, h, inter, hidden, shape[1], max_tiles, gat, 1, tab, E, 1, rec, yb, &sw));
     }
-    const unsigned wg = (unsigned)std::min<size_t>(256, pg_round_up(hidden / 4, 64)), per = grid_for(hidden / 4, wg);
+    const bool four = T * hidden >= 65536;
+    const size_t columns = four ? hidden / 4 : hidden;
+    const unsigned wg = (unsigned)std::min<size_t>(256, pg_round_up(columns, 64)), per = grid_for(columns, wg);
     PG_CHECK_ARG(T * per < ((size_t)1 << 31), "pg_mxfp4_moe_ffn: %zu tokens of %zu outputs in one launch", T, hidden);
-    return pg_launch(ctx, "mxfp4_moe_combine", top_k <= 2 ? mxfp4_moe_combine_kernel<2> : mxfp4_moe_combine_kernel<4>, dim3((unsigned)(T * per)), dim3(wg), 0,
+    auto kern = four ? (top_k <= 2 ? mxfp4_moe_combine_kernel<v4f, 2> : mxfp4_moe_combine_kernel<v4f, 4>)
+                     : (top_k <= 2 ? mxfp4_moe_combine_kernel<float, 2> : mxfp4_moe_combine_kernel<float, 4>);
+    return pg_launch(ctx, "mxfp4_moe_combine", kern, dim3((unsigned)(T * per)), dim3(wg), 0,
                      (const float *)yb, reinterpret_cast<const float *const *>(tab + 5 * E), by_pairs ? expert_idx_dev : (const int *)topk_idx,
                      by_pairs ? weight_dev : (const float *)topk_p, per, (unsigned)hidden, (int)top_k, (int)E, out_dev);
 }

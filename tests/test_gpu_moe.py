@@ -376,7 +376,7 @@ def test_moe_tiles_of_all_experts(ctx, orc, T, E, top_k, d, ffn, typ):
             H.assert_close_rel(got[t], want[t], MOE_RTOL, f"{name}, token {t}")
 
 
-@pytest.mark.parametrize("T,d,top_k", [(3, 160, 3), (7, 1056, 2), (65, 2080, 1)])
+@pytest.mark.parametrize("T,d,top_k", [(3, 160, 3), (7, 1056, 2), (65, 2080, 1), (63, 1056, 3)])
 @pytest.mark.parametrize("form", ["block", "mxfp4"])
 def test_layer_outputs_at_any_float(ctx, orc, form, T, d, top_k):
     """The sum over a token's experts goes out four columns at a time where the output allows it: the same bits at an output that
