@@ -635,11 +635,12 @@ def test_matmul_dequant_i8_one_launch(ctx, orc, m, k, n):
 
 @pytest.mark.parametrize("m,k,n", [
     (519, 2221, 73), (186, 408, 2870), (211, 102, 3608), (1060, 665, 1904), (770, 105, 2959), (526, 1666, 3890),   # each of the tiles
+    (391, 631, 2419), (580, 209, 3254), (1071, 1731, 3635),
     (124, 1073, 515), (512, 174, 73), (212, 174, 73), (74, 396, 1118), (33, 128, 17), (513, 1000, 64),             # groups of rows, their ends
     (9, 1530, 4100), (8, 3000, 70), (17, 1500, 30), (32, 1409, 2049), (31, 2500, 4097),                             # few rows of long K
 ])
 def test_matmul_dequant_i8_on_every_kernel(ctx, orc, m, k, n):
-    """Each kernel of the one launch from 33 rows on, at ragged sizes the estimates give it.  Small integers are exact; random
+    """Each kernel of the one launch from 33 rows on, at ragged sizes that are given to it.  Small integers are exact; random
     rows are within the activation step (2^-23 of the row's largest value a value) and one rounding of the float64 product."""
     from peregrine_amd import quant
     say(f"matmul_dequant_i8 kernels m={m} k={k} n={n}")
