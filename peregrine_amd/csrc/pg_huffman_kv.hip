@@ -9,8 +9,8 @@
 // launches: the heads' absolute maxima and the int8 values with a histogram per 4096 of them (one launch, or for large batches two); the code table, one
 // workgroup a chunk, which also turns the small histograms into the bit at which each 4096 values start; and the
 // encoder.  The host takes part once per batch: it learns the coded sizes (words that the table kernel stores in
-// pinned memory); a cache's first batch gets exactly that much memory, later ones what the one before took and 1 / 64, and are
-// encoded a second time if they take more.  A batch was 10 launches, 12 copies and 8
+// pinned memory); a cache's first batch gets exactly that much memory, later ones what the one before took and 1 / 64, or, if
+// they take more, exactly as much once the sizes are known.  A batch was 10 launches, 12 copies and 8
 // waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
 // 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.18.
 //
@@ -682,12 +682,14 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
     }
 }
 
+__host__ __device__ inline unsigned long long kv_stream_bytes(unsigned long long bits) { return (bits + 7) / 8; }
+
 // Where up to KV_PLACES chunks of a batch, from number `first` on, are written to.
 constexpr unsigned KV_PLACES = 32;
 struct kv_places {
     unsigned first;
     char *at[KV_PLACES];
-    unsigned long long max_bits;  // that there is room for: a longer stream is not written
+    unsigned long long room;  // GUESSED: bytes that every chunk of the batch has for its stream
     // the window's rows that move to the front in the same launch (workgroups behind the chunks', which read the int8
     // values only): heads of both sides, `rest` values each, from `from` values on
     float *hot[2];
@@ -710,10 +712,18 @@ __device__ __forceinline__ bool push_code(unsigned e, unsigned long long &acc, u
 // known; its threads put their codes together in LDS and the workgroup stores the words that START in its
 // range, whole: the bits that the last of them takes from the next run it encodes itself (up to 31 values), so no word
 // has two writers and nothing is zeroed first.
+// GUESSED: launched before the host knows the sizes.  Unless every stream of the batch fits its room, the launch does nothing at
+// all -- no stream is written and the window does not move -- and the host, which decides by the same sizes, takes over.
+template <bool GUESSED>
 __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, const kv_places places, char **__restrict__ table) {
     __shared__ unsigned lc[NUM_SYMBOLS], wsum[4];
     __shared__ unsigned words[ENC_PER_WG * KV_MAX_BITS / 32 + 2], follow[32];
     const unsigned c = places.first + blockIdx.y, g = blockIdx.x, t = threadIdx.x, lane = t & 63;
+    if constexpr (GUESSED) {
+        bool fits = true;
+        for (unsigned i = lane; i < b.count; i += 64) fits = fits && kv_stream_bytes(b.wg_bit[(size_t)i * (b.nwg + 1) + b.nwg]) <= places.room;
+        if (__ballot(!fits)) return;  // (the same for all workgroups)
+    }
     if (c >= b.count) {
         const unsigned row = c - b.count;
         float *p = places.hot[row / b.heads] + (size_t)(row % b.heads) * places.hot_stride;
@@ -724,7 +734,6 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
     char *dst = places.at[blockIdx.y];
     const unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
     const unsigned long long first = wg_bit[g], last = wg_bit[g + 1], end = wg_bit[b.nwg];
-    if (end > places.max_bits) return;  // (the same for all of a chunk's workgroups)
     lc[t] = b.codes[(size_t)c * NUM_SYMBOLS + t];
     for (unsigned i = t; i < sizeof(words) / 4; i += KV_WG) words[i] = 0;
     const int8_t *q = b.q + (size_t)c * b.q_stride;
@@ -1030,7 +1039,7 @@ static pg_status wait_for_words(pg_ctx *ctx, const uint64_t *words, size_t n) {
     return PG_OK;
 }
 
-// The window's move to the front, for compress_batch to fold into its last launch (done = true) where it can.
+// The window's move to the front, for compress_batch to fold into its last launch where it can (done = true once it is certain).
 struct kv_shift {
     float *hot[2];
     size_t stride, from, rest;
@@ -1047,14 +1056,16 @@ struct kv_rows {
 // head h of it starts at data[side] + number * chunk_step + h * head_stride.  Their addresses go to table_dev[0 ..) if given.
 // `rows` (if given) are still to be written to the window behind data[]: the first launch does.
 // `expect` (if given): room for streams of that many bytes is made and the encoder launched before their sizes are known, so that it
-// follows the table at once instead of 8 us later; a batch with a longer stream is encoded again once they are.  0 = wait
-// for the sizes first.  Set to what a batch like the last one needs and 1 / 64 more.
+// follows the table at once instead of 8 us later; where a stream is longer that launch does nothing (GUESSED), and the batch is
+// encoded once the sizes are known.  0 = wait for the sizes first.  Set to what a batch like the last one needs and 1 / 64 more.
+// Whatever fails -- memory on the device or on the host -- fails before the window moves: the cache is then as it was.
 static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t sides, size_t count, size_t chunk_step, size_t head_stride,
                                 size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift, kv_rows *rows, size_t *expect,
                                 std::vector<std::unique_ptr<pg_huffman_kv_chunk>> &out) {
     const size_t head_elems = num_tokens * head_dim, total = num_heads * head_elems;
     const size_t nwg = (total + ENC_PER_WG - 1) / ENC_PER_WG;
     const size_t most = std::max<size_t>(1, std::min<size_t>(KV_BATCH_SYMBOLS / total, KV_BATCH_CHUNKS) / sides) * sides;
+    out.reserve(count);
     for (size_t first = 0; first < count; first += most) {
         kv_batch b;
         const size_t n = std::min(most, count - first);
@@ -1084,6 +1095,14 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         b.wg_bit = reinterpret_cast<unsigned long long *>(base + o_bit);
         b.codes = reinterpret_cast<unsigned *>(base + o_codes);
         b.lut = reinterpret_cast<uint16_t *>(base + o_lut);
+        std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made(n);
+        for (auto &ch : made) {
+            ch.reset(new (std::nothrow) pg_huffman_kv_chunk());
+            if (!ch) return pg_fail(PG_ENOMEM, "host allocation failed");
+        }
+        auto block = std::make_shared<pg_dev_block>();
+        std::vector<char *> at(n);
+        bool moves = false;  // the encoder's launch moves the window
         uint64_t *sizes = static_cast<uint64_t *>(pin);
         std::fill(sizes, sizes + n, (uint64_t)0);
         kv_incoming in = {{b.data[0], b.data[1]}, {nullptr, nullptr}, 0, 0, ~(size_t)0, 0, 0};
@@ -1106,61 +1125,57 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         if (rows) rows->written = true;
         PG_TRY(pg_launch(ctx, "huffman_kv_table", b.total < (1u << 23) ? kv_table_kernel<unsigned> : kv_table_kernel<unsigned long long>, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
         const kv_layout lay(num_heads, total, true);
-        // the encoder, and with `again` unset the window's move: chunk c has room for bytes_of(c) of stream
-        auto encode = [&](auto bytes_of, bool again, std::shared_ptr<pg_dev_block> &block, std::vector<char *> &at) -> pg_status {
-            size_t bytes = 0, largest = 0;
-            for (size_t c = 0; c < n; ++c) {
-                bytes += lay.size(bytes_of(c));
-                largest = std::max<size_t>(largest, bytes_of(c));
-            }
-            block = std::make_shared<pg_dev_block>();
+        // the encoder and the window's move: chunk c has room for bytes_of(c) of stream
+        auto encode = [&](auto bytes_of, unsigned long long guess) -> pg_status {
+            size_t bytes = 0;
+            for (size_t c = 0; c < n; ++c) bytes += lay.size(bytes_of(c));
             PG_TRY(block->alloc(ctx, bytes));
-            at.resize(n);
             bytes = 0;
             for (size_t c = 0; c < n; ++c) {
                 at[c] = static_cast<char *>(block->p) + bytes;
                 bytes += lay.size(bytes_of(c));
             }
+            moves = false;
             for (size_t c0 = 0; c0 < n; c0 += KV_PLACES) {
                 kv_places places;
                 places.first = (unsigned)c0;
-                places.max_bits = 8ull * largest;
+                places.room = guess;
                 const size_t here = std::min<size_t>(KV_PLACES, n - c0);
                 std::copy(at.begin() + c0, at.begin() + c0 + here, places.at);
                 size_t rows = 0;
-                if (shift && !again && first + c0 + here == count && shift->rest <= shift->from && here + sides * num_heads <= 65535) {  // (no row reads what it writes)
+                if (shift && first + c0 + here == count && shift->rest <= shift->from && here + sides * num_heads <= 65535) {  // (no row reads what it writes)
                     places.hot[0] = shift->hot[0];
                     places.hot[1] = shift->hot[1];
                     places.hot_stride = shift->stride;
                     places.from = shift->from;
                     places.rest = shift->rest;
                     rows = sides * num_heads;
-                    shift->done = true;
+                    moves = true;
                 }
-                PG_TRY(pg_launch(ctx, "huffman_kv_encode", kv_encode_kernel, dim3(b.nwg, (unsigned)(here + rows)), dim3(KV_WG), 0, b, places,
-                                 table_dev ? table_dev + first : nullptr));
+                PG_TRY(pg_launch(ctx, "huffman_kv_encode", guess ? kv_encode_kernel<true> : kv_encode_kernel<false>, dim3(b.nwg, (unsigned)(here + rows)),
+                                 dim3(KV_WG), 0, b, places, table_dev ? table_dev + first : nullptr));
             }
             return PG_OK;
         };
-        std::shared_ptr<pg_dev_block> block;
-        std::vector<char *> at;
         const size_t room = expect ? *expect : 0;
-        if (room) PG_TRY(encode([&](size_t) { return room; }, false, block, at));
-        PG_TRY(wait_for_words(ctx, sizes, n));
-        auto stream_bytes = [&](size_t c) { return (size_t)((sizes[c] - 1 + 7) / 8); };
+        pg_status guessed = PG_OK;
+        if (room) guessed = encode([&](size_t) { return room; }, room);
+        PG_TRY(wait_for_words(ctx, sizes, n));  // (also after a failure: the table kernel writes them until then)
+        PG_TRY(guessed);
+        auto stream_bytes = [&](size_t c) { return (size_t)kv_stream_bytes(sizes[c] - 1); };
         size_t longest = 0;
         for (size_t c = 0; c < n; ++c) longest = std::max(longest, stream_bytes(c));
-        if (longest > room) PG_TRY(encode(stream_bytes, room != 0, block, at));
+        if (!room || longest > room) PG_TRY(encode(stream_bytes, 0));
+        if (shift && moves) shift->done = true;
         if (expect) *expect = longest + longest / 64;
         for (size_t c = 0; c < n; ++c) {
-            std::unique_ptr<pg_huffman_kv_chunk> ch(new (std::nothrow) pg_huffman_kv_chunk());
-            if (!ch) return pg_fail(PG_ENOMEM, "host allocation failed");
+            pg_huffman_kv_chunk *ch = made[c].get();
             ch->num_tokens = num_tokens; ch->num_heads = num_heads; ch->head_dim = head_dim;
             ch->block = block;
             ch->dev = at[c];
             ch->bytes = stream_bytes(c);
             ch->decodable = ch->indexed = true;
-            out.push_back(std::move(ch));
+            out.push_back(std::move(made[c]));
         }
     }
     return PG_OK;
@@ -1436,6 +1451,8 @@ static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c, kv_rows *rows
     const size_t chunks = (hot->len - c->compress_threshold) / tokens + 1;  // compress_threshold >= chunk_size: every chunk is whole
     PG_TRY(chunk_shape_ok("huffman kv append", tokens, heads, hd));
     PG_TRY(table_reserve(ctx, c, c->k_chunks.size() * 2 + 2 * chunks));
+    for (auto *v : {&c->k_chunks, &c->v_chunks})
+        if (v->size() + chunks > v->capacity()) v->reserve(std::max(v->size() + chunks, 2 * v->capacity()));
     const float *data[2] = {hot->k, hot->v};
     std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
     kv_shift shift{{hot->k, hot->v}, stride, chunks * tokens * hd, (hot->len - chunks * tokens) * hd};

@@ -1,12 +1,14 @@
 // The HIP runtime calls of libperegrine_hip on host memory, for tests without a GPU: the library's own objects are linked
 // with this file instead of the runtime, kernels are not run but noted (name and grid), and what the library does around
 // its launches -- its allocations, its pools, its choice of kernels, what it asks of a capturing stream -- can be
-// followed.  `pghost_*` are the test's handles: a limit on device memory, a stream's capture state, the launches.
+// followed.  `pghost_*` are the test's handles: a limit on device memory, allocations that fail, a stream's capture state, the
+// launches, the size of coded streams.
 #include <hip/hip_runtime_api.h>
 #include <stdlib.h>
 #include <string.h>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -17,6 +19,8 @@ struct state {
     std::map<const void *, std::string> kernels;
     std::map<const void *, void *> variables;
     std::map<void *, size_t> device;  // live allocations
+    size_t mallocs_left = ~(size_t)0, news_left = ~(size_t)0;  // that succeed: device allocations, host objects
+    unsigned long long stream_bytes[2] = {1000, 1000};         // of a coded chunk, by side (chunks take turns)
     size_t used = 0, limit = ~(size_t)0, frees = 0, bad_frees = 0, recorded = 0, copied = 0;
     std::map<hipStream_t, bool> capturing;  // true: capture was broken by a forbidden call
     std::vector<launch_rec> launches;
@@ -38,10 +42,12 @@ void note(const void *fn, dim3 grid, dim3 block, void **args) {
     if (!sim().capturing.empty()) { ++sim().recorded; return; }
     // the one kernel whose result the host reads before its next launch: a chunk's bits plus one, in pinned memory
     if (name.find("kv_table_kernel") != std::string::npos)
-        for (unsigned i = 0; i < grid.x; ++i) (*static_cast<unsigned long long **>(args[1]))[i] = 8 * 1000 + 1;
+        for (unsigned i = 0; i < grid.x; ++i) (*static_cast<unsigned long long **>(args[1]))[i] = 8 * sim().stream_bytes[i & 1] + 1;
 }
 hipError_t take(void **p, size_t bytes) {
     if (forbidden()) return hipErrorStreamCaptureUnsupported;
+    if (sim().mallocs_left == 0) return hipErrorOutOfMemory;
+    if (sim().mallocs_left != ~(size_t)0) --sim().mallocs_left;
     if (bytes > sim().limit - (sim().used < sim().limit ? sim().used : sim().limit)) return hipErrorOutOfMemory;
     *p = aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
     if (!*p) return hipErrorOutOfMemory;
@@ -53,6 +59,8 @@ hipError_t take(void **p, size_t bytes) {
 
 #define TEST_API extern "C" __attribute__((visibility("default")))
 TEST_API void pghost_limit(size_t bytes) { guard g(sim().mu); sim().limit = bytes; }
+TEST_API void pghost_fail_after(size_t mallocs, size_t news) { guard g(sim().mu); sim().mallocs_left = mallocs; sim().news_left = news; }
+TEST_API void pghost_stream_bytes(size_t k, size_t v) { guard g(sim().mu); sim().stream_bytes[0] = k; sim().stream_bytes[1] = v; }
 TEST_API size_t pghost_used() { guard g(sim().mu); return sim().used; }
 TEST_API size_t pghost_frees() { guard g(sim().mu); return sim().frees; }
 TEST_API size_t pghost_bad_frees() { guard g(sim().mu); return sim().bad_frees; }
@@ -71,6 +79,14 @@ TEST_API const char *pghost_launch(size_t i, unsigned *grid) {
     guard g(sim().mu);
     memcpy(grid, sim().launches[i].grid, sizeof sim().launches[i].grid);
     return sim().launches[i].name.c_str();
+}
+
+// the library's objects, which it asks for without exceptions
+void *operator new(size_t bytes, const std::nothrow_t &) noexcept {
+    guard g(sim().mu);
+    if (sim().news_left == 0) return nullptr;
+    if (sim().news_left != ~(size_t)0) --sim().news_left;
+    return malloc(bytes ? bytes : 1);
 }
 
 extern "C" {

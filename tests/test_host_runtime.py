@@ -14,6 +14,9 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
 LIB = os.path.join(CPP, "_build", "libperegrine_host.so")
 
 
+NO_LIMIT = C.c_size_t(-1).value
+
+
 class Host:
     """The library on the host runtime, one context to begin with."""
 
@@ -28,6 +31,8 @@ class Host:
         for name in ("pghost_used", "pghost_frees", "pghost_bad_frees", "pghost_recorded", "pghost_copied", "pghost_num_launches"):
             getattr(self.lib, name).restype = C.c_size_t
         self.lib.pghost_limit.argtypes = [C.c_size_t]
+        self.lib.pghost_fail_after.argtypes = self.lib.pghost_stream_bytes.argtypes = [C.c_size_t, C.c_size_t]
+        self.lib.pghost_fail_after.restype = self.lib.pghost_stream_bytes.restype = None
         self.lib.pghost_limit.restype = self.lib.pghost_clear_launches.restype = self.lib.pghost_begin_capture.restype = None
         self.lib.pghost_begin_capture.argtypes = self.lib.pghost_end_capture.argtypes = [C.c_void_p]
         self.lib.pghost_launch.argtypes, self.lib.pghost_launch.restype = [C.c_size_t, C.POINTER(C.c_uint)], C.c_char_p
@@ -76,7 +81,9 @@ class Host:
 @pytest.fixture()
 def host():
     h = Host()
-    h.lib.pghost_limit(C.c_size_t(-1).value)
+    h.lib.pghost_limit(NO_LIMIT)
+    h.lib.pghost_fail_after(NO_LIMIT, NO_LIMIT)
+    h.lib.pghost_stream_bytes(1000, 1000)
     h.lib.pghost_clear_launches()
     yield h
     assert h.lib.pghost_bad_frees() == 0
@@ -138,6 +145,52 @@ def test_coded_cache_append_that_cuts_a_chunk_is_refused_by_a_capture(host):
     host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 1)
     assert host.lib.pg_huffman_kv_cache_num_chunks(c) == 2
     host.lib.pg_huffman_kv_cache_free(host.ctx, c)
+
+
+def coded_cache(host, heads=8, hd=128, tokens=256, pieces=2):
+    """A coded cache that has cut a chunk a side per piece, and the rows of another."""
+    c = host.new("pg_huffman_kv_cache_create", host.ctx, heads, hd, tokens, tokens)
+    rows = host.alloc(heads * hd * 2 * tokens)
+    for _ in range(pieces):
+        host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, tokens)
+    return c, rows
+
+
+@pytest.mark.parametrize("mallocs,news", [(n, NO_LIMIT) for n in range(6)] + [(NO_LIMIT, n) for n in range(3)])
+@pytest.mark.parametrize("was,now", [(100000, 120000), (100000, 100000), (100000, 5000)])
+def test_append_that_runs_out_of_memory_leaves_the_coded_cache_whole(host, mallocs, news, was, now):
+    """Every allocation of an append that cuts a chunk fails in turn.  What failed has moved nothing: the only encoder
+    launches that carry the window's move are those that do nothing where streams do not suit their rooms, and these
+    did not.  The next append cuts what this one could not."""
+    host.lib.pghost_stream_bytes(was, was)
+    c, rows = coded_cache(host)
+    host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 255)
+    drained = host.alloc(1)                                              # (an allocation that fails empties the pool)
+    host.lib.pghost_limit(host.lib.pghost_used())
+    assert host.lib.pg_dev_alloc(host.ctx, 1 << 20, C.byref(C.c_void_p())) == 3
+    host.lib.pghost_limit(NO_LIMIT)
+    host.lib.pghost_stream_bytes(now, now)
+    host.lib.pghost_clear_launches()
+    host.lib.pghost_fail_after(mallocs, news)
+    st = host.lib.pg_huffman_kv_cache_append_dev(host.ctx, c, rows, rows, 2)
+    host.lib.pghost_fail_after(NO_LIMIT, NO_LIMIT)
+    shape = lambda: (host.lib.pg_huffman_kv_cache_len(c), host.lib.pg_huffman_kv_cache_compressed_len(c), host.lib.pg_huffman_kv_cache_num_chunks(c))
+    encoders = [name for name, _ in host.launches() if "kv_encode_kernel" in name]
+    if st == 0:
+        assert shape() == (769, 768, 3)
+    else:
+        assert st == 3 and shape()[1:] == (512, 2)
+        assert shape()[0] in (767, 769)                                  # (767: there was no room for the new rows)
+        assert all("kv_encode_kernelILb1E" in name for name in encoders) and (now != was or not encoders), encoders
+        n = 769 - shape()[0]
+        host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, n)
+        if n == 0:
+            host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 1)
+        assert shape()[1:] == (768, 3)
+    if (mallocs, news) == (0, NO_LIMIT) or news == 0:
+        assert st == 3                                                   # (the test does reach failures)
+    host.lib.pg_huffman_kv_cache_free(host.ctx, c)
+    host.ok("pg_dev_free", host.ctx, drained)
 
 
 def f16_route(host, typ, m, n, k):
