@@ -1057,7 +1057,7 @@ struct kv_rows {
 // `rows` (if given) are still to be written to the window behind data[]: the first launch does.
 // `expect` (if given): room for streams of that many bytes is made and the encoder launched before their sizes are known, so that it
 // follows the table at once instead of 8 us later; where a stream is longer that launch does nothing (GUESSED), and the batch is
-// encoded once the sizes are known.  0 = wait for the sizes first.  Set to what a batch like the last one needs and 1 / 64 more.
+// encoded once the sizes are known, as where there was no memory for the guess.  0 = wait for the sizes first.  Set to what a batch like the last one needs and 1 / 64 more.
 // Whatever fails -- memory on the device or on the host -- fails before the window moves: the cache is then as it was.
 static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t sides, size_t count, size_t chunk_step, size_t head_stride,
                                 size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift, kv_rows *rows, size_t *expect,
@@ -1161,11 +1161,11 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         pg_status guessed = PG_OK;
         if (room) guessed = encode([&](size_t) { return room; }, room);
         PG_TRY(wait_for_words(ctx, sizes, n));  // (also after a failure: the table kernel writes them until then)
-        PG_TRY(guessed);
+        if (guessed != PG_ENOMEM) PG_TRY(guessed);
         auto stream_bytes = [&](size_t c) { return (size_t)kv_stream_bytes(sizes[c] - 1); };
         size_t longest = 0;
         for (size_t c = 0; c < n; ++c) longest = std::max(longest, stream_bytes(c));
-        if (!room || longest > room) PG_TRY(encode(stream_bytes, 0));
+        if (!room || guessed != PG_OK || longest > room) PG_TRY(encode(stream_bytes, 0));
         if (shift && moves) shift->done = true;
         if (expect) *expect = longest + longest / 64;
         for (size_t c = 0; c < n; ++c) {

@@ -193,6 +193,20 @@ def test_append_that_runs_out_of_memory_leaves_the_coded_cache_whole(host, mallo
     host.ok("pg_dev_free", host.ctx, drained)
 
 
+def test_append_that_fits_is_taken_where_a_guess_would_not(host):
+    """After streams of 100000 bytes, two of 5000 with memory for them, but not for two like the last."""
+    host.lib.pghost_stream_bytes(100000, 100000)
+    c, rows = coded_cache(host)
+    host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 255)
+    host.lib.pghost_stream_bytes(5000, 5000)
+    host.lib.pghost_limit(host.lib.pghost_used())
+    assert host.lib.pg_dev_alloc(host.ctx, 1 << 20, C.byref(C.c_void_p())) == 3   # (the pool is empty now)
+    host.lib.pghost_limit(host.lib.pghost_used() + 120000)
+    host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, 1)
+    assert host.lib.pg_huffman_kv_cache_num_chunks(c) == 3
+    host.lib.pg_huffman_kv_cache_free(host.ctx, c)
+
+
 def f16_route(host, typ, m, n, k):
     """Whether a product of m rows over an [n, k] tensor runs on the f16 matrix cores."""
     w = host.new("pg_gguf_upload", host.ctx, bytes(n * k // 32 * {2: 18, 3: 20, 8: 34}[typ]), typ, n, k)
