@@ -9,8 +9,8 @@
 // launches: the heads' absolute maxima and the int8 values with a histogram per 4096 of them (one launch, or for large batches two); the code table, one
 // workgroup a chunk, which also turns the small histograms into the bit at which each 4096 values start; and the
 // encoder.  The host takes part once per batch: it learns the coded sizes (words that the table kernel stores in
-// pinned memory); a cache's first batch gets exactly that much memory, later ones what the one before took and 1 / 64, or, if
-// they take more, exactly as much once the sizes are known.  A batch was 10 launches, 12 copies and 8
+// pinned memory) and allocates exactly that much, or, from a cache's second batch on, has launched the encoder into what the
+// batch before took and 1 / 64 where that suits (at most 1 / 32 too much; compress_batch).  A batch was 10 launches, 12 copies and 8
 // waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
 // 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.18.
 //
@@ -689,7 +689,9 @@ constexpr unsigned KV_PLACES = 32;
 struct kv_places {
     unsigned first;
     char *at[KV_PLACES];
-    unsigned long long room;  // GUESSED: bytes that every chunk of the batch has for its stream
+    // GUESSED: bytes that every chunk of a side has for its stream; what all chunks have to need, in units of 256 bytes
+    unsigned long long room[2];
+    unsigned least;
     // the window's rows that move to the front in the same launch (workgroups behind the chunks', which read the int8
     // values only): heads of both sides, `rest` values each, from `from` values on
     float *hot[2];
@@ -712,17 +714,24 @@ __device__ __forceinline__ bool push_code(unsigned e, unsigned long long &acc, u
 // known; its threads put their codes together in LDS and the workgroup stores the words that START in its
 // range, whole: the bits that the last of them takes from the next run it encodes itself (up to 31 values), so no word
 // has two writers and nothing is zeroed first.
-// GUESSED: launched before the host knows the sizes.  Unless every stream of the batch fits its room, the launch does nothing at
-// all -- no stream is written and the window does not move -- and the host, which decides by the same sizes, takes over.
+// GUESSED: launched before the host knows the sizes.  Unless every stream of the batch fits its room, and the rooms are not much too
+// large, the launch does nothing at all -- no stream is written and the window does not move -- and the host, which decides by
+// the same sizes, takes over.
 template <bool GUESSED>
 __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, const kv_places places, char **__restrict__ table) {
     __shared__ unsigned lc[NUM_SYMBOLS], wsum[4];
     __shared__ unsigned words[ENC_PER_WG * KV_MAX_BITS / 32 + 2], follow[32];
     const unsigned c = places.first + blockIdx.y, g = blockIdx.x, t = threadIdx.x, lane = t & 63;
+    const kv_layout lay(b.heads, b.total, true);
     if constexpr (GUESSED) {
         bool fits = true;
-        for (unsigned i = lane; i < b.count; i += 64) fits = fits && kv_stream_bytes(b.wg_bit[(size_t)i * (b.nwg + 1) + b.nwg]) <= places.room;
-        if (__ballot(!fits)) return;  // (the same for all workgroups)
+        unsigned need = 0;
+        for (unsigned i = lane; i < b.count; i += 64) {
+            const unsigned long long bytes = kv_stream_bytes(b.wg_bit[(size_t)i * (b.nwg + 1) + b.nwg]);
+            fits = fits && bytes <= places.room[i % b.sides];
+            need += (unsigned)(lay.size(bytes) / 256);
+        }
+        if (__ballot(!fits) || (unsigned)pg_wave_sum_i32((int)need) < places.least) return;  // (the same for all workgroups)
     }
     if (c >= b.count) {
         const unsigned row = c - b.count;
@@ -730,7 +739,6 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
         for (size_t i = (size_t)g * KV_WG + t; i < places.rest; i += (size_t)gridDim.x * KV_WG) p[i] = p[places.from + i];
         return;
     }
-    const kv_layout lay(b.heads, b.total, true);
     char *dst = places.at[blockIdx.y];
     const unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
     const unsigned long long first = wg_bit[g], last = wg_bit[g + 1], end = wg_bit[b.nwg];
@@ -965,7 +973,7 @@ struct pg_huffman_kv_cache {
     pg_kv_cache *hot = nullptr;
     std::vector<pg_huffman_kv_chunk *> k_chunks, v_chunks;
     size_t compressed_len = 0, compress_threshold = 0, chunk_size = 0;
-    size_t expect = 0;  // bytes that a chunk's stream is expected to take (compress_batch)
+    size_t expect[2] = {0, 0};  // bytes that a chunk's stream is expected to take, by side (compress_batch)
     // The chunks' addresses on the device, key and value side in turn (written by the encoder).  An outgrown table
     // may still be read by work in flight and stays until the cache goes.
     pg_dev_block table_mem;
@@ -1055,9 +1063,12 @@ struct kv_rows {
 // compress_chunk of `count` chunks of one shape (none of them empty), chunk c being number c / sides of side c % sides:
 // head h of it starts at data[side] + number * chunk_step + h * head_stride.  Their addresses go to table_dev[0 ..) if given.
 // `rows` (if given) are still to be written to the window behind data[]: the first launch does.
-// `expect` (if given): room for streams of that many bytes is made and the encoder launched before their sizes are known, so that it
-// follows the table at once instead of 8 us later; where a stream is longer that launch does nothing (GUESSED), and the batch is
-// encoded once the sizes are known, as where there was no memory for the guess.  0 = wait for the sizes first.  Set to what a batch like the last one needs and 1 / 64 more.
+// `expect` (if given): room for streams of that many bytes, by side, is made and the encoder launched before their sizes are known, so
+// that it follows the table at once instead of 8 us later.  Where a stream is longer, or the rooms take more than 1 / 32 over what
+// the chunks need, that launch does nothing (GUESSED), and the batch is encoded into exactly what it needs once the sizes
+// are known, as where there was no memory for the guess.  0 = wait for the sizes first.  Set to what a batch like the last
+// one needs and 1 / 64 more: of normally distributed rows, in appends of 1 to 4 chunks of 16384 to 262144 values, one batch in
+// 16 does not suit its guess.
 // Whatever fails -- memory on the device or on the host -- fails before the window moves: the cache is then as it was.
 static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t sides, size_t count, size_t chunk_step, size_t head_stride,
                                 size_t num_tokens, size_t num_heads, size_t head_dim, char **table_dev, kv_shift *shift, kv_rows *rows, size_t *expect,
@@ -1126,10 +1137,12 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         PG_TRY(pg_launch(ctx, "huffman_kv_table", b.total < (1u << 23) ? kv_table_kernel<unsigned> : kv_table_kernel<unsigned long long>, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
         const kv_layout lay(num_heads, total, true);
         // the encoder and the window's move: chunk c has room for bytes_of(c) of stream
-        auto encode = [&](auto bytes_of, unsigned long long guess) -> pg_status {
+        unsigned least = 0;
+        auto encode = [&](auto bytes_of, bool guess) -> pg_status {
             size_t bytes = 0;
             for (size_t c = 0; c < n; ++c) bytes += lay.size(bytes_of(c));
             PG_TRY(block->alloc(ctx, bytes));
+            least = (unsigned)((bytes / 256 * 32 + 32) / 33);
             bytes = 0;
             for (size_t c = 0; c < n; ++c) {
                 at[c] = static_cast<char *>(block->p) + bytes;
@@ -1139,7 +1152,9 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
             for (size_t c0 = 0; c0 < n; c0 += KV_PLACES) {
                 kv_places places;
                 places.first = (unsigned)c0;
-                places.room = guess;
+                places.room[0] = expect ? expect[0] : 0;
+                places.room[1] = expect ? expect[1] : 0;
+                places.least = least;
                 const size_t here = std::min<size_t>(KV_PLACES, n - c0);
                 std::copy(at.begin() + c0, at.begin() + c0 + here, places.at);
                 size_t rows = 0;
@@ -1157,17 +1172,22 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
             }
             return PG_OK;
         };
-        const size_t room = expect ? *expect : 0;
-        pg_status guessed = PG_OK;
-        if (room) guessed = encode([&](size_t) { return room; }, room);
+        const bool guesses = expect && expect[0] && expect[sides - 1];
+        pg_status guessed = PG_ENOMEM;
+        if (guesses) guessed = encode([&](size_t c) { return expect[c % sides]; }, true);
         PG_TRY(wait_for_words(ctx, sizes, n));  // (also after a failure: the table kernel writes them until then)
         if (guessed != PG_ENOMEM) PG_TRY(guessed);
         auto stream_bytes = [&](size_t c) { return (size_t)kv_stream_bytes(sizes[c] - 1); };
-        size_t longest = 0;
-        for (size_t c = 0; c < n; ++c) longest = std::max(longest, stream_bytes(c));
-        if (!room || guessed != PG_OK || longest > room) PG_TRY(encode(stream_bytes, 0));
+        size_t longest[2] = {0, 0}, need = 0;
+        for (size_t c = 0; c < n; ++c) {
+            longest[c % sides] = std::max(longest[c % sides], stream_bytes(c));
+            need += lay.size(stream_bytes(c)) / 256;
+        }
+        bool suits = guessed == PG_OK && need >= least;
+        for (size_t s = 0; s < sides; ++s) suits = suits && longest[s] <= expect[s];
+        if (!suits) PG_TRY(encode(stream_bytes, false));
         if (shift && moves) shift->done = true;
-        if (expect) *expect = longest + longest / 64;
+        for (size_t s = 0; expect && s < sides; ++s) expect[s] = longest[s] + longest[s] / 64;
         for (size_t c = 0; c < n; ++c) {
             pg_huffman_kv_chunk *ch = made[c].get();
             ch->num_tokens = num_tokens; ch->num_heads = num_heads; ch->head_dim = head_dim;
@@ -1456,7 +1476,7 @@ static pg_status compress_hot(pg_ctx *ctx, pg_huffman_kv_cache *c, kv_rows *rows
     const float *data[2] = {hot->k, hot->v};
     std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made;
     kv_shift shift{{hot->k, hot->v}, stride, chunks * tokens * hd, (hot->len - chunks * tokens) * hd};
-    const pg_status st = compress_batch(ctx, data, 2, 2 * chunks, tokens * hd, stride, tokens, heads, hd, c->table + c->k_chunks.size() * 2, &shift, rows, &c->expect, made);
+    const pg_status st = compress_batch(ctx, data, 2, 2 * chunks, tokens * hd, stride, tokens, heads, hd, c->table + c->k_chunks.size() * 2, &shift, rows, c->expect, made);
     size_t done = 0;
     for (size_t i = 0; i + 1 < made.size(); i += 2) {
         c->k_chunks.push_back(made[i].release());

@@ -330,3 +330,27 @@ def test_streams_longer_than_the_last(ctx, orc, heads, hd, thr, chunk):
     for side, chunks in ((0, c.k_chunks), (1, c.v_chunks)):
         for i, ch in enumerate(chunks):
             _same_chunk(ch, o.chunk(side, i)[:3])
+
+
+@pytest.mark.parametrize("heads,hd,thr,chunk", [(2, 16, 24, 16), (4, 64, 96, 64), (8, 128, 512, 256)])
+def test_sides_of_different_streams(ctx, orc, heads, hd, thr, chunk):
+    """Keys and values that code to very different lengths, alike from append to append, in turn the one and the other, and in
+    batches of which one chunk alone outgrows its room: what the device makes of its sizes is what the host does."""
+    from peregrine_amd import huffman
+    say(f"huffman kv sides heads={heads} head_dim={hd} threshold={thr} chunk={chunk}")
+    rng = np.random.default_rng(heads + 7)
+    c, o = huffman.HuffmanKVCache(heads, hd, thr, chunk, ctx), orc.HuffmanKVCache(heads, hd, thr, chunk)
+    few = lambda n: rng.integers(0, 2, (heads, n, hd)).astype(np.float32)
+    many = lambda n: rng.standard_normal((heads, n, hd)).astype(np.float32)
+    late = lambda n: np.concatenate([few(n - n // 3), many(n // 3)], 1)
+    for k, v, n in ((few, many, thr), (few, many, chunk), (few, many, chunk + 3), (many, few, chunk), (many, few, 2 * chunk), (many, late, 3 * chunk),
+                    (late, many, 3 * chunk), (few, few, chunk), (few, few, chunk), (many, many, 35 * chunk), (many, many, 35 * chunk)):
+        k, v = k(n), v(n)
+        c.append(k, v, n)
+        o.append(k, v, n)
+        assert (c.len(), c.compressed_len, c.hot_len) == (o.len, o.compressed_len, o.hot_len)
+        for got, want in zip(c.get_kv(), o.get_kv()):
+            assert (got.view(np.uint32) == want.view(np.uint32)).all()
+    for side, chunks in ((0, c.k_chunks), (1, c.v_chunks)):
+        for i in {0, len(chunks) // 2, len(chunks) - 1}:
+            _same_chunk(chunks[i], o.chunk(side, i)[:3])

@@ -207,6 +207,36 @@ def test_append_that_fits_is_taken_where_a_guess_would_not(host):
     host.lib.pg_huffman_kv_cache_free(host.ctx, c)
 
 
+@pytest.mark.parametrize("first,then", [((100000, 100000), (5000, 5000)), ((30000, 220000), (30000, 220000)), ((5000, 5000), (100000, 100000)),
+                                        ((100000, 100000), (97500, 97500)), ((100000, 100000), (99000, 101500)), ((40000, 200000), (39000, 190000))])
+def test_coded_chunks_take_the_memory_their_streams_need(host, first, then):
+    """Streams of one length, then of another, the sides' of their own: a batch holds at most 1 / 32 more than scales, tables,
+    index and streams (and the step of the allocations: a sixteenth of a power of two)."""
+    heads, hd, tokens = 8, 128, 256
+    host.lib.pghost_stream_bytes(*first)
+    c, rows = coded_cache(host, heads, hd, tokens)
+    host.lib.pghost_stream_bytes(*then)
+    total = heads * hd * tokens
+    chunk = lambda b: 256 + 256 + 8192 + (total // 4096 + 1) * 8 + total // 64 * 2 + b + 512
+    for n in range(3):
+        drained = host.lib.pghost_used()
+        host.lib.pghost_limit(drained)
+        assert host.lib.pg_dev_alloc(host.ctx, 1 << 30, C.byref(C.c_void_p())) == 3
+        host.lib.pghost_limit(NO_LIMIT)
+        before = host.lib.pghost_used()
+        host.lib.pghost_clear_launches()
+        host.ok("pg_huffman_kv_cache_append_dev", host.ctx, c, rows, rows, tokens)
+        encoders = [name for name, _ in host.launches() if "kv_encode_kernel" in name]
+        assert len(encoders) in (1, 2) and "ILb1E" in encoders[0], encoders
+        host.lib.pghost_limit(host.lib.pghost_used())                    # (a guess that did not suit lies in the pool)
+        assert host.lib.pg_dev_alloc(host.ctx, 1 << 30, C.byref(C.c_void_p())) == 3
+        host.lib.pghost_limit(NO_LIMIT)
+        taken, need = host.lib.pghost_used() - before, sum(chunk(b) for b in then)
+        assert taken <= need * (1 + 1 / 32) * (1 + 1 / 8), (taken, need)
+        assert n == 0 or len(encoders) == 1                              # and like the last, one launch
+    host.lib.pg_huffman_kv_cache_free(host.ctx, c)
+
+
 def f16_route(host, typ, m, n, k):
     """Whether a product of m rows over an [n, k] tensor runs on the f16 matrix cores."""
     w = host.new("pg_gguf_upload", host.ctx, bytes(n * k // 32 * {2: 18, 3: 20, 8: 34}[typ]), typ, n, k)
