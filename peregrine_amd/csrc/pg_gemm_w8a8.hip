@@ -939,37 +939,6 @@ bool choose_few_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, s
 }
 }  // namespace
 
-// Several weights that share the tiles' launch: whether those of long K and few columns are better off in a launch of their own, split
-// over K (pg_launch_gemm_w8a8_few_rows, estimated from 16 such products), because the others then need a round of tiles less, or
-// because few tiles walk a long K.
-// apart[i] says which.  The lines are those of tiles that took longer than today's: the one launch has come level since where most of
-// the outputs go apart, and ahead where few do (135 x 10836 -> 628, 8185 58.7 : 62).  Then: us, all in one : apart: 135 x 10836 -> 628, 8185 75.7 : 63.8, 213 x 13535 -> 1432, 7172 96.9 :
-// 84.6, 36 x 13303 -> 1942, 6355 80.2 : 49.9, 46 x 13309 -> 294, 9512 81.2 : 57.0; of 110 such groups the worst it leaves is 34 x 7988 -> 8097,
-// 679, 708, 51.4 against 48.1 with each weight split.
-bool pg_gemm_w8a8_split_apart(pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, bool *apart) {
-    const pg_qtensor *rest[PG_GEMM_MAX_GROUP];
-    int n_rest = 0;
-    double split_us = 0.0;
-    for (int i = 0; i < count; ++i) {
-        int splits = 1;
-        apart[i] = m > 32 && (m <= 64 || (m <= 256 && w[i]->k_pad >= 2 * w[i]->cols)) && !ctx->gemm_force_tile &&
-                   pg_launch_gemm_w8a8_few_rows(ctx, nullptr, w[i]->k_pad, nullptr, w[i], m, nullptr, nullptr, nullptr, &splits) == PG_OK && splits > 1;
-        if (apart[i]) split_us += 9.5 + 0.05e-3 * (double)(m * w[i]->cols);
-        else rest[n_rest++] = w[i];
-    }
-    // rounds of the tiles that lines on their number choose, 128 of K at a time
-    auto tiles_us = [&](const pg_qtensor *const *of, int n) {
-        if (n == 0) return 0.0;
-        const size_t cus = (size_t)ctx->num_cu, t256 = gemm_tiles(of, n, m, 256, 256);
-        const bool largest = m > 64 && (t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus));
-        const tile_kernel *t = m <= 64 ? &TILES[0] : largest ? &TILES[1] : gemm_tiles(of, n, m, 128, 256) >= cus ? &TILES[2] : gemm_tiles(of, n, m, 128, 128) < cus ? &TILES[3] : &TILES[4];
-        static constexpr double STEP[] = {0.366, 1.98, 1.26, 0.302, 0.846};
-        return STEP[t - TILES] * (double)((gemm_tiles(of, n, m, t->bm, t->bn) + cus - 1) / cus * (of[0]->k_pad / 128));
-    };
-    const double cold = m <= 64 ? 1.95 : 1.55;  // (a step over weights that no cache holds)
-    return n_rest < count && split_us + cold * tiles_us(rest, n_rest) < 0.95 * cold * tiles_us(w, count);
-}
-
 // 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights side by side.
 // (33 .. 64 rows where the estimates say no, us with the quantisation launch: 4096 -> 14336 24.7 against 30.3 split over K with a
 // finishing pass, but 14336 -> 4096 27.8 against 26.2: long, narrow products keep the split.)

@@ -268,7 +268,6 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
 pg_status pg_launch_gemm_w8a8_skinny(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                                      const pg_qtensor *w, size_t m, float *out, int32_t *acc);
 // 2 .. 8 rows of up to some thousand columns in f32, quantised inside the product's own launch (the same integers and scales).
-bool pg_gemm_w8a8_split_apart(pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, bool *apart);
 bool pg_gemm_w8a8_takes_f32_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m);
 pg_status pg_launch_gemm_w8a8_f32_rows(pg_ctx *ctx, const float *a, const pg_qtensor *const *w, float *const *out, int count, size_t m);
 pg_status pg_launch_gemm_w8a8_few_rows(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,

@@ -691,16 +691,8 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     if (count == 1) return pg_matmul_quantized_dev(ctx, a_dev, m, k, w[0], out_dev[0], nullptr);
     const size_t k_pad = w[0]->k_pad, m_pad = pg_round_up(m, PG_MPAD);
     const size_t a_bytes = m_pad * k_pad, sz_scales = pg_round_up(m_pad * sizeof(float), 256);
-    bool apart_of[PG_GEMM_MAX_GROUP];
-    const bool split = pg_gemm_w8a8_split_apart(ctx, w, (int)count, m, apart_of);
-    size_t part_bytes = 0;
-    for (size_t i = 0; i < count && split; ++i) {
-        int splits = 1;
-        if (apart_of[i]) PG_TRY(pg_launch_gemm_w8a8_few_rows(ctx, nullptr, k_pad, nullptr, w[i], m, nullptr, nullptr, nullptr, &splits));
-        part_bytes = std::max(part_bytes, (size_t)splits * m * w[i]->cols * sizeof(int32_t));
-    }
     void *ws = nullptr;
-    PG_TRY(pg_workspace(ctx, a_bytes + sz_scales + part_bytes, &ws));
+    PG_TRY(pg_workspace(ctx, a_bytes + sz_scales, &ws));
     int8_t *a_i8 = static_cast<int8_t *>(ws);
     float *a_scales = reinterpret_cast<float *>(a_i8 + a_bytes);
     PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, k_pad, a_scales));
@@ -710,16 +702,15 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     }
     // Weights that fill the chip with 256x256 tiles on their own run on their own (measured: gate and up
     // as two launches 2 x 112 us, as one launch of 896 tiles 242 us: the rounds that leave CUs idle run
-    // faster); the narrow ones (q, k, v) share one launch, where k and v alone would leave most CUs idle.
+    // faster); the narrow ones (q, k, v) share one launch, where k and v alone would leave most CUs idle.  (Of 33 to 256 rows too, over
+    // a long K: weights split over K in launches of their own took 49.9 us where one launch takes 43.8, 46 x 13300 -> 294, 9512, 67.9 : 54.3,
+    // 135 x 10836 -> 628, 8185, 60.6 : 45.2, 63 x 13958 -> 8390, 421, 363; and of 178 groups two gained by it, 3 and 9 %.)
     const pg_qtensor *small_w[PG_GEMM_MAX_GROUP];
     float *small_out[PG_GEMM_MAX_GROUP];
     int n_small = 0;
     for (size_t i = 0; i < count; ++i) {
         const size_t t256 = ((m + 255) / 256) * ((w[i]->cols + 255) / 256);
-        if (split && apart_of[i]) {
-            PG_TRY(pg_launch_gemm_w8a8_few_rows(ctx, a_i8, k_pad, a_scales, w[i], m, out_dev[i], nullptr,
-                                                reinterpret_cast<int32_t *>(a_i8 + a_bytes + sz_scales), nullptr));
-        } else if (t256 >= (size_t)ctx->num_cu) {
+        if (t256 >= (size_t)ctx->num_cu) {
             PG_TRY(pg_launch_gemm_w8a8(ctx, a_i8, k_pad, a_scales, w[i], m, out_dev[i], nullptr));
         } else {
             small_w[n_small] = w[i];
