@@ -752,46 +752,56 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_f32_rows_kernel(const float
     }
 }
 
-size_t gemm_tiles(const pg_qtensor *const *w, int count, size_t m, size_t bm, size_t bn) {
-    size_t panels = 0;
-    for (int i = 0; i < count; ++i) panels += (w[i]->cols + bn - 1) / bn;
-    return ((m + bm - 1) / bm) * panels;
-}
-// The tile kernels and what a launch of each takes with the quantisation before it, us: the longer of what the fullest CU does
-// (its tiles one after another, as many as its LDS holds at a time: a step of 128 of K by how many are resident, and a round's
-// ends; 0.29 less of it in proportion to the places that the rounds leave empty, which the busy CUs' clock makes good) and what all
-// tiles bring through L2, the weights from HBM and the output back, as the fourth root of the sum of their fourth powers.
-// Fitted to 690 products (m 65 .. 4200, K 128 .. 14336, n 64 .. 24000, each kernel timed on each, the weights from HBM): 5 to 7 %
-// mean error where a kernel is within 30 % of the best; the choice takes 1.1 % more than the best kernel on average, 6 % at the 95th
-// percentile (half of them against a fit to the others: 1.4 and 8 %).
+// From 33 rows on W8A8 has three routes, and each kernel of each an estimate of what the product takes with the quantisation before it, us;
+// the least is taken (pg_gemm_w8a8_route).  All were fitted together to 1150 single products (m 33 .. 4200, K 64 .. 16384, n 64 .. 131072, every
+// kernel of every route timed on each, the weights from HBM), least squares on the relative error, the more the nearer a kernel is to the
+// best, and in full where it would be taken wrongly.  The choice takes 0.9 % more than the best kernel on average to 64 rows, 1.7 % to 256, 1.2 % to
+// 700, 0.9 % beyond (4, 9, 6 and 5 % at the 95th percentile; a third of them against a fit to the others: 1.2, 2.0, 1.6, 0.8 % on average), and
+// 1 % on 197 groups of two and three weights that are in none of the fits.  A change to a kernel asks for all of it again.  Against the lines
+// and estimates that they replace (fitted to no more than 24000 columns, a CU's workgroups counted over the part): of 820 products over 8 us,
+// 137 more than 5 % faster, 18 that much slower.  us, those : these: 200 x 10240 -> 50257 197 : 165, 225 x 4026 -> 1099 17.4 : 12.5,
+// 64 x 1024 -> 50257 32 : 19, 62 x 5302 -> 14499 28.4 : 22.7, 111 x 7102 -> 49915 123 : 87; but 65 x 444 -> 92928 25.8 : 29.6.
+//
+// The tiles: the longer of what the fullest CU does (its tiles one after another, as many as its LDS holds at a time: a step of 128 of
+// K by how many are resident, and a round's ends; less of it in proportion to the places that the rounds leave empty, which the
+// busy CUs' clock makes good) and what all tiles bring through L2, the weights from HBM and the output back (more where rows do not begin on
+// a line, and where it is more than a cache takes), as the fourth root of the sum of their fourth powers.
 //
 // What the shapes are: eight wavefronts or more for everything beyond 64x64 and as many stages as the LDS holds, or two and
 // three workgroups a CU, because a CU's stream from L2 grows with what it has in flight.  Against four wavefronts a tile and two or three stages, and
 // lines on the number of tiles (the largest that fill 70 % of the CUs), products of more than 700 rows take 0.84 of the time, 257 to
-// 700 0.9.  us, before : now: 2015 x 8071 -> 4709 142 : 99, 1262 x 13674 -> 4132 153 : 101, 473 x 6624 -> 9376 80 : 51,
+// 700 0.9.  us, those : these: 2015 x 8071 -> 4709 142 : 99, 1262 x 13674 -> 4132 153 : 101, 473 x 6624 -> 9376 80 : 51,
 // 353 x 3968 -> 3968 25 : 21, 717 x 1568 -> 3104 16.9 : 14.4, 2048 x 14336 -> 4096 157 : 147; 2048 x 4096 -> 14336 as before.
 struct tile_kernel {
     int code;  // of pg_gemm_w8a8_force_tile
     unsigned bm, bn, resident;  // (workgroups a CU holds)
-    double step[3], round, fixed, l2, weights, output;  // per MB through L2, M weights, M outputs
+    double step[3], round, fixed, l2, weights, output, ragged, idle, past;  // per MB through L2, M weights, M outputs, M of them off the lines, past 20 M
 };
-constexpr tile_kernel TILES[] = {{1, 64, 64, 3, {0.308, 0.350, 0.396}, 1.15, 3.45, 0.0631, 0.053, 0.232},  // three stages
-                                 {2, 256, 256, 1, {1.608}, 10.1, 5.80, 0.0, 0.430, 0.585},
-                                 {3, 128, 256, 1, {0.981}, 5.53, 4.16, 0.0066, 0.289, 0.606},
-                                 {4, 128, 64, 2, {0.424, 0.620}, 1.65, 3.30, 0.0547, 0.078, 0.522},
-                                 {5, 128, 128, 1, {0.584}, 3.15, 3.24, 0.0247, 0.238, 0.445},
-                                 {6, 128, 192, 1, {0.777}, 4.29, 3.90, 0.0242, 0.221, 0.589},
-                                 {7, 256, 128, 1, {0.982}, 4.80, 2.35, 0.0514, 0.074, 0.677},
-                                 {8, 256, 192, 1, {1.311}, 8.35, 4.63, 0.0, 0.494, 0.597},
-                                 {1, 64, 64, 2, {0.285, 0.381}, 1.21, 3.51, 0.0595, 0.0, 0.0}};  // four stages
+constexpr tile_kernel TILES[] = {{1, 64, 64, 3, {0.309, 0.425, 0.380}, 0.960, 3.04, 0.0485, 0.139, 0.500, 0.037, 0.290, 0.744},  // three stages
+                                 {2, 256, 256, 1, {1.587}, 8.972, 4.36, 0.0543, 0.146, 0.548, 0.287, 0.308, 0.100},
+                                 {3, 128, 256, 1, {0.928}, 4.625, 3.29, 0.0432, 0.152, 0.636, 0.313, 0.175, 0.011},
+                                 {4, 128, 64, 2, {0.436, 0.710}, 1.607, 2.49, 0.0314, 0.191, 0.566, 0.174, 0.309, 0.667},
+                                 {5, 128, 128, 1, {0.589}, 2.936, 2.22, 0.0289, 0.194, 0.647, 0.362, 0.240, 0.030},
+                                 {6, 128, 192, 1, {0.759}, 3.683, 3.16, 0.0338, 0.197, 0.698, 0.345, 0.214, 0.006},
+                                 {7, 256, 128, 1, {1.010}, 4.271, 1.76, 0.0487, 0.140, 0.562, 0.225, 0.312, 0.108},
+                                 {8, 256, 192, 1, {1.226}, 7.611, 3.84, 0.0523, 0.200, 0.500, 0.361, 0.232, 0.132},
+                                 {1, 64, 64, 2, {0.291, 0.419}, 1.251, 2.36, 0.0389, 0.149, 0.500, 0.242, 0.239, 0.778}};  // four stages
 constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
 double quantise_us(const pg_qtensor *w, size_t m) { return 3.0 + 0.8e-6 * (double)(m * w->rows); }
-// The kernel of least estimated time (its index), and that time.  (A call of few microseconds waits for this: 32-bit
+// What the fullest CU takes for its share of `wgs` workgroups of `steps` steps, `resident` of them at a time.
+double fullest_cu(size_t wgs, unsigned cus, unsigned resident, const double *step, double steps, double round, double idle) {
+    const size_t most = wgs <= ~0u - cus ? ((unsigned)wgs + cus - 1) / cus : (wgs + cus - 1) / cus;
+    const size_t full = resident == 1 ? most : resident == 2 ? most / 2 : most / 3, rest = most - full * resident;
+    double cu = (double)full * (steps * step[resident - 1] + 0.5 * (resident + 1) * round);
+    if (rest) cu += steps * step[rest - 1] + 0.5 * (double)(rest + 1) * round;
+    return cu * (1.0 - idle * (1.0 - (double)wgs / (double)(most * cus)));
+}
+// The tile of least estimated time (its index), and that time.  (A call of few microseconds waits for this: 32-bit
 // divisions, and no roots for what is longer anyway.)
 int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, double *us = nullptr) {
     const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w[0]->k_pad / 128), rows64 = (unsigned)((m + 63) / 64);
     unsigned panels64 = 0, panels128 = 0, panels192 = 0, panels256 = 0;
-    size_t cols = 0;
+    size_t cols = 0, off_lines = 0;
     for (int i = 0; i < count; ++i) {
         const unsigned n = (unsigned)w[i]->cols;
         panels64 += (n + 63) / 64;
@@ -799,8 +809,9 @@ int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m
         panels192 += (n + 191) / 192;
         panels256 += (n + 255) / 256;
         cols += n;
+        off_lines += n % 32 ? n : 0;
     }
-    const double weights = 1e-6 * (double)(w[0]->rows * cols), output = 1e-6 * (double)(m * cols);
+    const double weights = 1e-6 * (double)(w[0]->rows * cols), output = 1e-6 * (double)(m * cols), ragged = 1e-6 * (double)(m * off_lines), past = std::max(0.0, output - 20.0);
     int best = -1;
     double best_us = 0.0;
     for (int i = 0; i < NTILES; ++i) {
@@ -808,12 +819,8 @@ int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m
         if (ctx->gemm_force_tile && t.code != ctx->gemm_force_tile) continue;
         const unsigned rows = (rows64 + t.bm / 64 - 1) / (t.bm / 64), panels = t.bn == 64 ? panels64 : t.bn == 128 ? panels128 : t.bn == 192 ? panels192 : panels256;
         const size_t tiles = (size_t)rows * panels;
-        const size_t most = tiles <= ~0u - cus ? ((unsigned)tiles + cus - 1) / cus : (tiles + cus - 1) / cus;
-        const size_t full = t.resident == 1 ? most : t.resident == 2 ? most / 2 : most / 3, rest = most - full * t.resident;
-        double cu = (double)full * (kt * t.step[t.resident - 1] + 0.5 * (t.resident + 1) * t.round);
-        if (rest) cu += kt * t.step[rest - 1] + 0.5 * (double)(rest + 1) * t.round;
-        cu *= 1.0 - 0.29 * (1.0 - (double)tiles / (double)(most * cus));
-        const double all = 128e-6 * (double)(tiles * kt) * (t.bm + t.bn) * t.l2 + weights * t.weights + output * t.output;
+        const double cu = fullest_cu(tiles, cus, t.resident, t.step, kt, t.round, t.idle);
+        const double all = 128e-6 * (double)(tiles * kt) * (t.bm + t.bn) * t.l2 + weights * t.weights + output * t.output + ragged * t.ragged + past * t.past;
         if (best >= 0 && t.fixed + std::max(cu, all) >= best_us) continue;
         const double c2 = cu * cu, a2 = all * all, time = t.fixed + sqrt(sqrt(c2 * c2 + a2 * a2));
         if (best < 0 || time < best_us) {
@@ -821,18 +828,15 @@ int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m
             best_us = time;
         }
     }
-    // Short K and 128x128 tiles for all CUs but a few: one round of them, where smaller ones need a second or fourth.  (636 x 416 -> 6368
-    // 13.3 : 12.1, 280 x 320 -> 10624 10.4 : 9.9, 1295 x 503 -> 2849 13.7 : 12.5, 1024 x 256 -> 4096 11.4 : 10.1; 216 tiles 12.4 : 12.1, 212 10.6 : 11.)
-    const size_t t128 = (size_t)((rows64 + 1) / 2) * panels128;
-    if (!ctx->gemm_force_tile && w[0]->k_pad <= 512 && t128 <= cus && 20 * t128 >= 19 * cus) best = 4;
     if (us) *us = quantise_us(w[0], m) + best_us;
     return best;
 }
+// `pick`: the tile's index, or -1 for the one of least estimated time.
 pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                         const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc,
-                        const int32_t *comb = nullptr, size_t comb_plane = 0) {
+                        int pick = -1, const int32_t *comb = nullptr, size_t comb_plane = 0) {
     // (the combining pass is for products that fill the part with 256x256 tiles: w8a32_large)
-    const int pick = comb && !ctx->gemm_force_tile ? 1 : pick_tile(ctx, w, count, m);
+    if (pick < 0) pick = comb && !ctx->gemm_force_tile ? 1 : pick_tile(ctx, w, count, m);
     switch (pick) {
 #define PG_TILE(CODE, ...)                                                                                                                    \
         case CODE:                                                                                                                            \
@@ -854,108 +858,125 @@ pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const 
 
 }  // namespace
 
-// Some dozens of rows over a long K (33 .. 256): one or two tiles of activations against every weight row is far too few
+// Some dozens of rows over few columns or a long K (33 .. 256): one or two tiles of activations against every weight row is far too few
 // workgroups to stream the weights (64 on 256 CUs at N = 4096), so K is split until every place of a CU is taken, not one more
 // (a workgroup too many is a round); the partial i32 sums go to `part` ([splits][m][n]) and a second launch adds them and applies the
-// scales.  64x64 tiles of four stages, two workgroups a CU, or for much work and more than two tiles of rows 128x128 with eight
-// wavefronts, one a CU: over 36 products (K 9300 .. 14300) 0.87 of the time of 64x128 and 128x128 tiles of four wavefronts, split beyond
-// the places.  us, before : now: 135 x 10836 -> 628 21.4 : 18.5, 213 x 13535 -> 1432 34.0 : 25.8, 96 x 12787 -> 2221 31.6 : 22.8,
-// 87 x 12661 -> 4291 45.4 : 32.4, 46 x 13300 -> 9512 44.1 : 39.7.  Returns the number of splits through *splits_out when called with
-// part == nullptr (sizing), else runs.
-pg_status pg_launch_gemm_w8a8_few_rows(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
-                                       const pg_qtensor *w, size_t m, float *out, int32_t *acc, int32_t *part,
-                                       int *splits_out) {
-    const size_t n = w->cols, kt = w->k_pad / 128;
-    const bool large = m > 128 && m * w->k_pad * n > 7000000000ull;
-    const size_t tile = large ? 128 : 64, tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
-    size_t splits = (large ? 1 : 2) * (size_t)ctx->num_cu / tiles;
-    if (splits > kt / 2) splits = kt / 2;  // at least two k-tiles per workgroup
-    if (splits > 16) splits = 16;
-    if (splits < 1) splits = 1;
-    const size_t kt_per = (kt + splits - 1) / splits;
-    splits = (kt + kt_per - 1) / kt_per;   // no empty split
-    if (splits_out) *splits_out = (int)splits;
-    if (!part) return PG_OK;
+// scales.  128x128 tiles with eight wavefronts, one a CU, or 64x64 of four stages, two a CU: over 36 products (K 9300 .. 14300) 0.87 of the time of
+// 64x128 and 128x128 tiles of four wavefronts, split beyond the places.  us, those : these: 135 x 10836 -> 628 21.4 : 18.5, 213 x
+// 13535 -> 1432 34.0 : 25.8, 96 x 12787 -> 2221 31.6 : 22.8, 87 x 12661 -> 4291 45.4 : 32.4, 46 x 13300 -> 9512 44.1 : 39.7.
+// Estimated as the tiles are, with what the last launch reads.
+namespace {
+struct split_kernel {
+    unsigned tile, resident;
+    double step[2], round, fixed, l2, weights, parts, idle;  // parts: per M of partial sums
+};
+constexpr split_kernel SPLITS[] = {{128, 1, {0.646}, 0.0, 6.60, 0.0, 0.185, 2.356, 0.0}, {64, 2, {0.775, 0.426}, 1.375, 3.67, 0.0508, 0.129, 2.403, 0.0}};
+// The runs of K, none of them empty, and the k-tiles of one.
+unsigned split_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, const split_kernel &s, unsigned *per) {
+    const size_t tiles = ((m + s.tile - 1) / s.tile) * ((w->cols + s.tile - 1) / s.tile), kt = w->k_pad / 128;
+    // (at least two k-tiles a run)
+    const size_t runs = std::max<size_t>(1, std::min<size_t>({s.resident * (size_t)ctx->num_cu / tiles, kt / 2, 16}));
+    *per = (unsigned)((kt + runs - 1) / runs);
+    return (unsigned)((kt + *per - 1) / *per);
+}
+}  // namespace
+size_t pg_gemm_w8a8_split_bytes(const pg_ctx *ctx, const pg_qtensor *w, size_t m, int index) {
+    unsigned per;
+    return (size_t)split_runs(ctx, w, m, SPLITS[index], &per) * m * w->cols * sizeof(int32_t);
+}
+pg_status pg_launch_gemm_w8a8_split(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales, const pg_qtensor *w, size_t m,
+                                    float *out, int32_t *acc, int32_t *part, int index) {
     if (a_stride != w->k_pad) return pg_fail(PG_EINVAL, "gemm_w8a8: activation stride %zu != k_pad %zu", a_stride, w->k_pad);
-    if (large) PG_TRY((launch<128, 128, 128, 4, 2, 4, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)splits, (int)kt_per)));
-    else PG_TRY((launch<64, 64, 128, 4, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)splits, (int)kt_per)));
-    const size_t plane = m * n;
+    unsigned per;
+    const unsigned runs = split_runs(ctx, w, m, SPLITS[index], &per);
+    if (index == 0) PG_TRY((launch<128, 128, 128, 4, 2, 4, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)runs, (int)per)));
+    else PG_TRY((launch<64, 64, 128, 4, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)runs, (int)per)));
+    const size_t n = w->cols, plane = m * n;
     return pg_launch(ctx, "gemm_w8a8_finish", splitk_finish_kernel, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0,
-                     (const int32_t *)part, (int)splits, plane, a_scales, (const float *)w->scales, (int)n, out, acc);
+                     (const int32_t *)part, (int)runs, plane, a_scales, (const float *)w->scales, (int)n, out, acc);
 }
 
 // 33 .. 512 rows in one launch of the few-row kernel: groups of 32, 48 or 64 rows, each reading every weight once more (the
-// groups of one weight tile follow each other on one XCD).  What the launch takes against the tiles of gemm_dispatch, both as
-// estimates: few rows over few columns leave most CUs without a tile, and a tile then walks all of K alone.  Fitted to 889
-// products (m 33 .. 400, K 256 .. 14336, one to three weights of 64 .. 16384 columns; every shape below and both other routes
-// timed on each): the launch 10 % mean error.  From 65 rows on it is held against 0.85 of pick_tile's estimate: of 66 products of
-// more than 9 us, 1 % over the better route on average (lines at 0.75 to 1 of it: 1.6 to 2.4 %).  us, with the
-// quantisation, before : now: 66 x 1024 -> 4096 9.8 : 7.2, 96 x 4096 -> 1024 15.4 : 8.5, 128 x 4096 -> 4096 15.7 : 13.2, 39 x 4096 ->
-// 1024 11.8 : 8.2, 256 x 4096 -> 1024 19.5 : 9.8; the tiles stay: 256 x 1024 -> 4096 8.7 : 11.6, 256 x 4096 -> 4096 17.0 : 22.6.
+// groups of one weight tile follow each other on one XCD).  Few rows over few columns leave most CUs without a tile, and a tile then walks all
+// of K alone.  Estimated as a round's start and run of K and what the fullest CU loads, the outputs and the weights, as the root of the sum of
+// their squares.  What a CU has is counted by XCD: all groups of a weight tile are on one, so 85 weight tiles x 3 groups are 33
+// workgroups for the 32 CUs of some (counted over the part they are a round: 110 x 5660 -> 1350 16.3 as that, 12.3 as groups of 32 rows
+// and 32 columns; 225 x 4026 -> 1099 17.1 : 12.5).  us, with the quantisation, against the tiles: 66 x 1024 -> 4096 9.8 : 7.2, 96 x 4096 -> 1024
+// 15.4 : 8.5, 128 x 4096 -> 4096 15.7 : 13.2, 39 x 4096 -> 1024 11.8 : 8.2.  (All rows of 33 .. 64 in one workgroup, a weight tile each, was
+// a route of its own up to 64 rows over wide weights: 64 x 1024 -> 50257 32 : 18, 40 x 10240 -> 50257 168 : 116, and of 187 products none
+// that it was 3 % faster on.)
 namespace {
-struct few_rows_shape { int mb, nb, nst, nw; double factor; };
-constexpr few_rows_shape FEW_ROWS_SHAPES[] = {{2, 1, 2, 2, 0.971}, {2, 1, 3, 4, 0.863}, {2, 1, 3, 8, 0.847}, {2, 2, 2, 4, 0.997}, {2, 2, 2, 8, 0.956},
-                                              {3, 1, 2, 8, 0.903}, {3, 2, 2, 4, 1.033}, {3, 2, 2, 8, 1.0},   {4, 2, 3, 4, 1.009}};
-// The shape of least estimated time, and that time (a call of few microseconds waits for this: 32-bit divisions); 0: not for these weights.
-double few_rows_us(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, few_rows_shape *out) {
+struct few_rows_shape {
+    int mb, nb, nst, nw;
+    double fixed, rows, round, run, loads, output, weights;
+};
+constexpr few_rows_shape FEW_ROWS_SHAPES[] = {{2, 1, 2, 2, 4.432, 0.831, 1.238, 0.528, 9.694, 2.673, 0.122},
+                                              {2, 1, 3, 4, 4.793, 1.442, 1.463, 0.080, 13.909, 0.837, 0.094},
+                                              {2, 1, 3, 8, 4.937, 1.323, 1.189, 0.0, 14.333, 3.440, 0.117},
+                                              {2, 2, 2, 4, 4.587, 1.174, 1.253, 0.590, 9.910, 3.003, 0.120},
+                                              {2, 2, 2, 8, 4.630, 1.283, 1.316, 0.324, 14.129, 3.255, 0.082},
+                                              {3, 1, 2, 8, 4.754, 1.333, 1.235, 0.317, 12.997, 4.109, 0.082},
+                                              {3, 2, 2, 4, 4.815, 1.023, 1.662, 0.593, 12.034, 3.146, 0.071},
+                                              {3, 2, 2, 8, 4.739, 1.238, 1.548, 0.353, 14.674, 3.660, 0.059},
+                                              {4, 2, 3, 4, 4.903, 1.548, 2.224, 0.303, 12.576, 4.001, 0.056}};
+}  // namespace
+
+// The route of a product of m rows over `count` weights side by side: 2 to 32 rows the few-row kernel, all rows in a workgroup
+// (index -1); beyond, the least estimate.
+pg_w8a8_route pg_gemm_w8a8_route(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
     const size_t k_pad = w[0]->k_pad;
-    const unsigned units = (unsigned)(k_pad / 128), cus = (unsigned)ctx->num_cu, rows = (unsigned)m;
-    if (m < 33 || m > 512 || ctx->gemm_force_tile) return 0.0;
     unsigned g16 = 0, g32 = 0;
     size_t cols = 0;
+    bool narrow = true;  // of 2^20 columns at most
     for (int i = 0; i < count; ++i) {
-        if (w[i]->k_pad != k_pad || w[i]->cols >= (1ull << 20)) return 0.0;
+        if (w[i]->k_pad != k_pad || k_pad >= (1ull << 30) || w[i]->cols >= (1ull << 30)) return {PG_W8A8_TILES, -1};
         cols += w[i]->cols;
+        narrow = narrow && w[i]->cols < (1ull << 20);
         g16 += (unsigned)(w[i]->cols + 15) / 16;
         g32 += (unsigned)(w[i]->cols + 31) / 32;
     }
-    // (a long K over one weight: split between workgroups, see pg_launch_gemm_w8a8_few_rows)
-    if (count == 1 && units >= 72 && (m <= 64 || (m <= 256 && k_pad >= 2 * cols))) return 0.0;
-    const double rows_us = 4.96 + 1.24e-6 * (double)(m * k_pad);
-    double best = 0.0;
-    for (const few_rows_shape &s : FEW_ROWS_SHAPES) {
-        const unsigned wgs = (s.nb == 1 ? g16 : g32) * ((rows + 16 * s.mb - 1) / (16 * s.mb));
-        const unsigned per_cu = std::min(80u / (unsigned)(s.nw * s.nst * (s.nb + s.mb)), 32u / s.nw);
-        const unsigned rounds = (wgs + cus * per_cu - 1) / (cus * per_cu), run = (units + s.nw - 1) / s.nw;
-        const double mb_cu = 2048e-6 * (double)((wgs + cus - 1) / cus) * units * (s.nb + s.mb);  // what the fullest CU loads
-        const double us = s.factor * (rows_us + rounds * (1.5 + 0.253 * run) + 14.0 * mb_cu);
-        if (best == 0.0 || us < best) {
-            best = us;
-            *out = s;
+    if (m >= 2 && m <= 32) return {PG_W8A8_ROWS, -1};
+    pg_w8a8_route best = {PG_W8A8_TILES, -1};
+    if (m < 33 || ctx->gemm_force_tile) return best;
+    double best_us;
+    best.index = pick_tile(ctx, w, count, m, &best_us);
+    const double weights = 1e-6 * (double)(w[0]->rows * cols);
+    auto better = [&](double us, pg_w8a8_kind kind, size_t i) {
+        if (us >= best_us) return;
+        best_us = us;
+        best = {kind, (int)i};
+    };
+    if (m <= 512 && narrow) {  // (a call of few microseconds waits for this: 32-bit divisions)
+        const unsigned units = (unsigned)(k_pad / 128), cus = (unsigned)ctx->num_cu / 8, rows = (unsigned)m;  // of one XCD
+        const double output = 1e-6 * (double)(m * cols), digits = 1e-6 * (double)(m * k_pad);
+        for (size_t i = 0; i < sizeof(FEW_ROWS_SHAPES) / sizeof(FEW_ROWS_SHAPES[0]); ++i) {
+            const few_rows_shape &s = FEW_ROWS_SHAPES[i];
+            const unsigned wgs = ((s.nb == 1 ? g16 : g32) + 7) / 8 * ((rows + 16 * s.mb - 1) / (16 * s.mb));
+            const unsigned per_cu = std::min(80u / (unsigned)(s.nw * s.nst * (s.nb + s.mb)), 32u / s.nw);
+            const unsigned rounds = (wgs + cus * per_cu - 1) / (cus * per_cu), run = (units + s.nw - 1) / s.nw;
+            const double walk = rounds * (s.round + s.run * run);
+            const double loads = 2048e-6 * (double)((wgs + cus - 1) / cus) * units * (s.nb + s.mb) * s.loads + output * s.output + weights * s.weights;
+            better(s.fixed + s.rows * digits + sqrt(walk * walk + loads * loads), PG_W8A8_ROWS, i);
         }
     }
+    if (m <= 256 && count == 1)
+        for (size_t i = 0; i < sizeof(SPLITS) / sizeof(SPLITS[0]); ++i) {
+            const split_kernel &s = SPLITS[i];
+            unsigned per;
+            const unsigned runs = split_runs(ctx, w[0], m, s, &per);
+            if (runs < 2) continue;
+            const size_t tiles = ((m + s.tile - 1) / s.tile) * ((cols + s.tile - 1) / s.tile);
+            const double cu = fullest_cu(tiles * runs, (unsigned)ctx->num_cu, s.resident, s.step, per, s.round, s.idle);
+            const double all = 128e-6 * (double)(tiles * (k_pad / 128)) * (2 * s.tile) * s.l2 + weights * s.weights;
+            const double c2 = cu * cu, a2 = all * all;
+            better(quantise_us(w[0], m) + s.fixed + sqrt(sqrt(c2 * c2 + a2 * a2)) + 1e-6 * (double)(m * cols * runs) * s.parts, PG_W8A8_SPLIT, i);
+        }
     return best;
 }
-bool choose_few_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m, few_rows_shape *out) {
-    const double us = few_rows_us(ctx, w, count, m, out);
-    if (us == 0.0) return false;
-    if (m <= 64) {  // held against the kernel of one weight tile for all rows, as rounds of 64x64 tiles
-        const size_t cus = (size_t)ctx->num_cu, k_pad = w[0]->k_pad;
-        return us < 0.95 * (7.8 + 1.86e-6 * (double)(m * k_pad) + 0.366 * (double)((gemm_tiles(w, count, m, 64, 64) + cus - 1) / cus * (k_pad / 128)));
-    }
-    double tiles = 0.0;
-    pick_tile(ctx, w, count, m, &tiles);
-    return us < 0.85 * tiles;
-}
-}  // namespace
 
-// 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights side by side.
-// (33 .. 64 rows where the estimates say no, us with the quantisation launch: 4096 -> 14336 24.7 against 30.3 split over K with a
-// finishing pass, but 14336 -> 4096 27.8 against 26.2: long, narrow products keep the split.)
-bool pg_gemm_w8a8_takes_skinny(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m) {
-    if (m < 2) return false;
-    bool narrow = false;
-    for (int i = 0; i < count; ++i) {
-        if (w[i]->k_pad != w[0]->k_pad || w[i]->k_pad >= (1ull << 30) || w[i]->cols >= (1ull << 30)) return false;
-        narrow = narrow || w[i]->cols < w[i]->k_pad;
-    }
-    few_rows_shape s;
-    return m <= 32 || choose_few_rows(ctx, w, count, m, &s) || (m <= 64 && !narrow);
-}
-
-// 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights of equal K side by side.
+// 2 .. 512 rows in one launch (see gemm_w8a8_skinny_kernel); `count` weights of equal K side by side.  `index`: of the route.
 pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
-                                           const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc) {
+                                           const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc, int index) {
     if (count < 1 || count > PG_GEMM_MAX_GROUP || (acc && count != 1))
         return pg_fail(PG_EINVAL, "gemm_w8a8 (few rows in one launch): %d weights (1 .. %d; the accumulators of one only)", count, PG_GEMM_MAX_GROUP);
     size_t cols = 0;
@@ -963,33 +984,32 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         if (a_stride != w[i]->k_pad) return pg_fail(PG_EINVAL, "gemm_w8a8: activation stride %zu != k_pad %zu", a_stride, w[i]->k_pad);
         cols += w[i]->cols;
     }
-    few_rows_shape grouped;
-    const bool rows_grouped = m > 64 ? few_rows_us(ctx, w, count, m, &grouped) > 0.0 : choose_few_rows(ctx, w, count, m, &grouped);  // (from 65 on the caller has chosen)
-    if (m > 64 ? !rows_grouped : !pg_gemm_w8a8_takes_skinny(ctx, w, count, m)) return pg_fail(PG_EINVAL, "gemm_w8a8 (few rows in one launch): m = %zu", m);
+    const bool rows_grouped = index >= 0;
+    if (rows_grouped ? m > 512 : m < 2 || m > 32) return pg_fail(PG_EINVAL, "gemm_w8a8 (few rows in one launch): m = %zu", m);
     const size_t k_pad = w[0]->k_pad;
     // Weight tiles a workgroup (NB), stages of a ring (NST) and wavefronts a workgroup (NW, its K runs).  What counts is that
     // every workgroup is resident at once and that a CU has many units requested: two or three stages in more wavefronts
     // beat four stages in fewer, and two weight tiles a workgroup (half the activations' way from L2) pay once 16-row
-    // workgroups are more than one a CU and their runs are not too short.  Drawn from 4500 shapes (m 2 .. 64, K 256 ..
+    // workgroups are more than one a CU and their runs are not too short.  Drawn from 3000 shapes (m 2 .. 32, K 256 ..
     // 10000, N 512 .. 16000, every shape that fits the LDS timed): against the rule before, which took four stages and
-    // wavefronts in powers of two up to the LDS of one or two tiles, 3.6 % (m <= 16), 6.3 % (m <= 32) and 13 % (m <= 64) on those
-    // over 8 us.  (us, before and now: 17 x 3412 -> 7951 12.0 / 10.6, 29 x 7580 -> 5374 19.9 / 16.7, 36 x 3853 -> 6403
-    // 17.9 / 13.7, 40 x 531 -> 8375 11.7 / 8.7, 12 x 7381 -> 5018 15.0 / 13.4.)
-    int mb = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
+    // wavefronts in powers of two up to the LDS of one or two tiles, 3.6 % (m <= 16) and 6.3 % (m <= 32) on those
+    // over 8 us.  (us, before and now: 17 x 3412 -> 7951 12.0 / 10.6, 29 x 7580 -> 5374 19.9 / 16.7, 12 x 7381 -> 5018 15.0 / 13.4.)
+    // Past 32 rows the route says the shape.
+    int mb = m <= 16 ? 1 : 2;
     const size_t units = k_pad / 128, g16 = (cols + 15) / 16, cus = (size_t)ctx->num_cu;
     struct shape { int nb, nst, nw; } sh = {1, mb == 1 ? 4 : 3, 0};
     const size_t wgs2 = (g16 + 1) / 2;  // workgroups of two weight tiles
     if (rows_grouped) {
+        const few_rows_shape &grouped = FEW_ROWS_SHAPES[index];
         mb = grouped.mb;
         sh = {grouped.nb, grouped.nst, grouped.nw};
     } else if (wgs2 > 2 * cus) {
         // More than 16384 columns (a vocabulary's): two weight tiles a workgroup, and of the rings that the LDS still holds
         // all at once (160 KiB a CU over the ring: 3, 4, 6 or 8 workgroups) the deepest; past that, rounds of the ring whose
-        // rounds come out fullest.  Short runs of K keep one tile.  Drawn from 384 shapes a row class (m 12, 24, 48; K 256
-        // .. 14000, N 16500 .. 170000), every shape below timed on each: 2.6, 2.4 and 0.9 % over the best one on average
-        // (the lines below, which go to 16000 columns, taken further: 12, 16 and 14 %, up to 40).  us, those : these:
-        // 8 x 1024 -> 50257 15.2 : 13.0, 24 x 4096 -> 24000 26.6 : 22.0, 24 x 768 -> 128256 38.8 : 30.4, 48 x 4096 -> 24000
-        // 36.9 : 28.6, 64 x 8192 -> 32000 73.8 : 64.5, 48 x 768 -> 151936 68.4 : 58.5.
+        // rounds come out fullest.  Short runs of K keep one tile.  Drawn from 384 shapes a row class (m 12, 24; K 256
+        // .. 14000, N 16500 .. 170000), every shape below timed on each: 2.6 and 2.4 % over the best one on average
+        // (the lines below, which go to 16000 columns, taken further: 12 and 16 %, up to 40).  us, those : these:
+        // 8 x 1024 -> 50257 15.2 : 13.0, 24 x 4096 -> 24000 26.6 : 22.0, 24 x 768 -> 128256 38.8 : 30.4.
         if (mb == 1) {
             if (units <= 4) sh = wgs2 <= 4 * cus ? shape{1, 4, 1} : shape{2, 3, 1};
             else if (units > 32 && (wgs2 <= 3 * cus || wgs2 > 4 * cus)) sh = {2, 3, 4};
@@ -998,37 +1018,25 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
             else if (wgs2 <= 6 * cus) sh = {2, 2, 2};
             else if (wgs2 <= 8 * cus) sh = {2, 3, 1};
             else sh = shape{2, 2, units < 6 ? 2 : 4};
-        } else if (mb == 2) {
+        } else {
             if (wgs2 <= 4 * cus) sh = units <= 4 ? shape{1, 3, 1} : shape{2, 2, 2};
             else if (wgs2 <= 6 * cus || (wgs2 > 10 * cus && units > 16)) sh = {2, 3, 1};
-            else sh = {2, 2, 1};
-        } else {
-            if (units <= 4) sh = {1, 2, 1};
-            else if (units > 16 && wgs2 > 12 * cus) sh = {2, 2, 3};
-            else if (wgs2 <= 3 * cus || (units > 16 && wgs2 > 8 * cus && wgs2 <= 9 * cus)) sh = {2, 2, 2};
-            else if (wgs2 <= 4 * cus || (wgs2 > 6 * cus && wgs2 <= 8 * cus)) sh = {2, 3, 1};
             else sh = {2, 2, 1};
         }
     } else if (mb == 1) {
         if (g16 > 3 * cus && units > 8) sh = {2, 3, 4};
         else if (g16 > 2 * cus && units > 16) sh = {1, 2, 4};
         else if (g16 > cus && units > 16) sh = {2, 3, 8};
-    } else if (mb == 2) {
+    } else {
         if (units <= 8) sh = {1, 3, 2};
         else if (g16 <= 2 * cus && units <= 16) sh = {1, 3, 4};
         else if (g16 <= 3 * cus && units <= 16) sh = {1, 2, 4};
         else if (g16 > 2 * cus) sh = {2, 2, 4};
         else if (g16 > cus) sh = {2, 2, 8};
-    } else {
-        if (units <= 8) sh = {1, g16 > 2 * cus ? 2 : 3, 2};
-        else if (g16 > 2 * cus) sh = {2, 2, 3};
-        else if (g16 > cus) sh = {2, 3, 4};
-        else if (units <= 16) sh = {1, 3, 4};
     }
     if (sh.nw == 0) {  // the narrow ones: as many wavefronts as keep every workgroup resident, on runs of four units or more
-        const int per_cu = mb == 4 ? 4 : 8;
-        sh.nw = per_cu;
-        while (sh.nw > 1 && (g16 * sh.nw > cus * per_cu || units / sh.nw < 4)) sh.nw >>= 1;
+        sh.nw = 8;
+        while (sh.nw > 1 && (g16 * sh.nw > cus * 8 || units / sh.nw < 4)) sh.nw >>= 1;
     } else if (!rows_grouped && 2 * units < 3 * (size_t)sh.nw) {
         sh.nw = 1;  // (two wavefronts want three units)
     }
@@ -1066,17 +1074,15 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
     PG_SKINNY(1, 1, 2, 4) PG_SKINNY(1, 2, 3, 4) PG_SKINNY(1, 2, 3, 8)
     PG_SKINNY(2, 1, 3, 1) PG_SKINNY(2, 1, 3, 2) PG_SKINNY(2, 1, 3, 4) PG_SKINNY(2, 1, 3, 8)
     PG_SKINNY(2, 1, 2, 4) PG_SKINNY(2, 2, 2, 4) PG_SKINNY(2, 2, 2, 8)
-    PG_SKINNY(4, 1, 3, 1) PG_SKINNY(4, 1, 3, 2) PG_SKINNY(4, 1, 3, 4)
-    PG_SKINNY(4, 1, 2, 1) PG_SKINNY(4, 1, 2, 2) PG_SKINNY(4, 2, 2, 3) PG_SKINNY(4, 2, 3, 4)
     PG_SKINNY(1, 2, 2, 2) PG_SKINNY(1, 2, 2, 4) PG_SKINNY(1, 2, 3, 1) PG_SKINNY(1, 2, 3, 2)
-    PG_SKINNY(2, 2, 2, 1) PG_SKINNY(2, 2, 2, 2) PG_SKINNY(2, 2, 3, 1) PG_SKINNY(4, 2, 2, 1) PG_SKINNY(4, 2, 2, 2) PG_SKINNY(4, 2, 3, 1)
+    PG_SKINNY(2, 2, 2, 1) PG_SKINNY(2, 2, 2, 2) PG_SKINNY(2, 2, 3, 1)
 #undef PG_SKINNY
     return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8 (few rows in one launch): no kernel of %d tiles, %d stages, %d wavefronts", sh.nb, sh.nst, sh.nw);
 }
 
 pg_status pg_launch_gemm_w8a8_skinny(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
-                                     const pg_qtensor *w, size_t m, float *out, int32_t *acc) {
-    return pg_launch_gemm_w8a8_skinny_group(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, acc);
+                                     const pg_qtensor *w, size_t m, float *out, int32_t *acc, int index) {
+    return pg_launch_gemm_w8a8_skinny_group(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, acc, index);
 }
 
 // 2 .. 8 short rows in f32 (gemm_w8a8_f32_rows_kernel): as long as a workgroup repeats the quantisation in less time than a
@@ -1134,11 +1140,11 @@ pg_status pg_launch_gemm_w8a8_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_st
 
 pg_status pg_launch_gemm_w8a8(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride,
                               const float *a_scales, const pg_qtensor *w, size_t m, float *out,
-                              int32_t *acc) {
+                              int32_t *acc, int pick) {
     if (a_stride != w->k_pad) return pg_fail(PG_EINVAL, "gemm_w8a8: activation stride %zu != k_pad %zu", a_stride, w->k_pad);
     if (w->k_pad >= (1ull << 22) || m >= (1ull << 24) || w->cols >= (1ull << 30))
         return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8: shape exceeds the kernel's 32-bit tile offsets");
-    return gemm_dispatch(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, acc);
+    return gemm_dispatch(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, acc, pick);
 }
 
 // The W8A32 product over three digit planes in one launch, where it is the better route: up to 32 rows the few-row kernel
@@ -1276,7 +1282,7 @@ pg_status pg_launch_gemm_w8a8_combine(pg_ctx *ctx, const int8_t *a_i8, size_t a_
     if (a_stride != w->k_pad) return pg_fail(PG_EINVAL, "gemm_w8a8: activation stride %zu != k_pad %zu", a_stride, w->k_pad);
     if (w->k_pad >= (1ull << 22) || m >= (1ull << 24) || w->cols >= (1ull << 30))
         return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8: shape exceeds the kernel's 32-bit tile offsets");
-    return gemm_dispatch(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, nullptr, comb, comb_plane);
+    return gemm_dispatch(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, nullptr, -1, comb, comb_plane);
 }
 
 // The shader clock inside the K loop of the 256x256 tile (the gate|up product's kernel): the

@@ -247,32 +247,35 @@ pg_status pg_probe_fill_random(pg_ctx *ctx, void *dev, size_t bytes);
 // Kernel launchers implemented per translation unit (device pointers, stream ordered).
 pg_status pg_launch_quantize_activations(pg_ctx *ctx, const float *a, size_t rows, size_t cols,
                                          int8_t *q, size_t q_stride, float *row_scales);
+// (pick: the index of a route of tiles, or -1: the tile of least estimated time)
 pg_status pg_launch_gemm_w8a8(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride,
                               const float *a_scales, const pg_qtensor *w, size_t m,
-                              float *out, int32_t *acc);
+                              float *out, int32_t *acc, int pick = -1);
 // The same activation rows against up to PG_GEMM_MAX_GROUP weights of equal K in ONE launch: the
 // weights' column panels form one tile space (a fused QKV or gate|up product without a fused
 // copy of the weights).  out[i] is [m, w[i]->cols].
 pg_status pg_launch_gemm_w8a8_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                                     const pg_qtensor *const *w, float *const *out, int count, size_t m);
-// 5 .. 64 activation rows: K split over workgroups, i32 partial sums in `part`, then one finishing
-// launch.  With part == nullptr only reports the number of splits (for sizing `part`).
 pg_status pg_launch_gemm_w8a8_combine(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                                       const pg_qtensor *w, size_t m, float *out, const int32_t *comb, size_t comb_plane);
 // The W8A32 product over three digit planes (plane_bytes apart) in one launch, where it takes it.
 bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
 pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out);
-bool pg_gemm_w8a8_takes_skinny(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m);
+// How W8A8 products of two rows and more run: tiles, the few-row kernel (2 .. 512 rows), or tiles with K split over workgroups (33 .. 256 rows
+// over one weight: i32 partial sums in `part`, pg_gemm_w8a8_split_bytes of them, and a finishing launch); `index` names the kernel.
+enum pg_w8a8_kind { PG_W8A8_TILES, PG_W8A8_ROWS, PG_W8A8_SPLIT };
+struct pg_w8a8_route { pg_w8a8_kind kind; int index; };
+pg_w8a8_route pg_gemm_w8a8_route(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m);
+size_t pg_gemm_w8a8_split_bytes(const pg_ctx *ctx, const pg_qtensor *w, size_t m, int index);
+pg_status pg_launch_gemm_w8a8_split(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales, const pg_qtensor *w, size_t m,
+                                    float *out, int32_t *acc, int32_t *part, int index);
 pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
-                                           const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc);
+                                           const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc, int index);
 pg_status pg_launch_gemm_w8a8_skinny(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
-                                     const pg_qtensor *w, size_t m, float *out, int32_t *acc);
+                                     const pg_qtensor *w, size_t m, float *out, int32_t *acc, int index);
 // 2 .. 8 rows of up to some thousand columns in f32, quantised inside the product's own launch (the same integers and scales).
 bool pg_gemm_w8a8_takes_f32_rows(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m);
 pg_status pg_launch_gemm_w8a8_f32_rows(pg_ctx *ctx, const float *a, const pg_qtensor *const *w, float *const *out, int count, size_t m);
-pg_status pg_launch_gemm_w8a8_few_rows(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
-                                       const pg_qtensor *w, size_t m, float *out, int32_t *acc, int32_t *part,
-                                       int *splits_out);
 pg_status pg_launch_gemv_w8a8(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride,
                               const float *a_scales, const pg_qtensor *w, size_t m,
                               float *out, int32_t *acc);

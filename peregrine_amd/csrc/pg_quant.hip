@@ -567,16 +567,13 @@ static pg_status matmul_quantized_on(pg_ctx *ctx, const float *a_dev, size_t m, 
     if (apart && pg_gemv_w8a8_takes_f32_row(w, m, k, a_dev)) return pg_launch_gemv_w8a8_f32_row(ctx, a_dev, k, w, out_dev, acc_dev);
     const size_t m_pad = pg_round_up(m, PG_MPAD);
     const size_t a_bytes = m_pad * w->k_pad;
-    // 33 .. 256 rows that the few-row kernel leaves: split-K product with i32 partial planes
-    // behind the scales, where the unsplit tiles would leave most CUs idle
-    // (up to 64 rows always; up to 256 only for long-K, narrow-N products like a down projection --
-    // measured at 128 rows: 14336 -> 4096 35 -> 25 us split, but 4096 -> 4096 12.6 -> 19 us)
-    int splits = 1;
-    const bool skinny = pg_gemm_w8a8_takes_skinny(ctx, &w, 1, m);
-    if (!skinny && m > PG_GEMV_MAX_M && (m <= 64 || (m <= 256 && w->k_pad >= 2 * w->cols)))
-        PG_TRY(pg_launch_gemm_w8a8_few_rows(ctx, nullptr, w->k_pad, nullptr, w, m, nullptr, nullptr, nullptr, &splits));
     const size_t sz_scales = pg_round_up(m_pad * sizeof(float), 256);
-    const size_t part_bytes = splits > 1 ? (size_t)splits * m * w->cols * sizeof(int32_t) : 0;
+    pg_w8a8_route route = pg_gemm_w8a8_route(ctx, &w, 1, m);
+    size_t part_bytes = route.kind == PG_W8A8_SPLIT ? pg_gemm_w8a8_split_bytes(ctx, w, m, route.index) : 0;
+    if (part_bytes && fixed && a_bytes + sz_scales + part_bytes > fixed_cap) {  // (the partial planes are no reason to refuse)
+        route = {PG_W8A8_TILES, -1};
+        part_bytes = 0;
+    }
     const size_t need = a_bytes + sz_scales + part_bytes;
     void *ws = fixed;
     if (fixed) {
@@ -589,13 +586,13 @@ static pg_status matmul_quantized_on(pg_ctx *ctx, const float *a_dev, size_t m, 
     int8_t *a_i8 = static_cast<int8_t *>(ws);
     float *a_scales = reinterpret_cast<float *>(a_i8 + a_bytes);
     PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, w->k_pad, a_scales));
-    if (skinny) return pg_launch_gemm_w8a8_skinny(ctx, a_i8, w->k_pad, a_scales, w, m, out_dev, acc_dev);
+    if (route.kind == PG_W8A8_ROWS) return pg_launch_gemm_w8a8_skinny(ctx, a_i8, w->k_pad, a_scales, w, m, out_dev, acc_dev, route.index);
     if (m <= PG_GEMV_MAX_M)
         return pg_launch_gemv_w8a8(ctx, a_i8, w->k_pad, a_scales, w, m, out_dev, acc_dev);
-    if (splits > 1)
-        return pg_launch_gemm_w8a8_few_rows(ctx, a_i8, w->k_pad, a_scales, w, m, out_dev, acc_dev,
-                                            reinterpret_cast<int32_t *>(a_i8 + a_bytes + sz_scales), nullptr);
-    return pg_launch_gemm_w8a8(ctx, a_i8, w->k_pad, a_scales, w, m, out_dev, acc_dev);
+    if (route.kind == PG_W8A8_SPLIT)
+        return pg_launch_gemm_w8a8_split(ctx, a_i8, w->k_pad, a_scales, w, m, out_dev, acc_dev,
+                                         reinterpret_cast<int32_t *>(a_i8 + a_bytes + sz_scales), route.index);
+    return pg_launch_gemm_w8a8(ctx, a_i8, w->k_pad, a_scales, w, m, out_dev, acc_dev, route.index);
 }
 
 PG_API pg_status pg_matmul_quantized_dev(pg_ctx *ctx, const float *a_dev, size_t m, size_t k,
@@ -678,17 +675,18 @@ PG_API pg_status pg_matmul_quantized_multi_dev(pg_ctx *ctx, const float *a_dev, 
     if (one_row_group)  // one token: every weight's rows in one streaming launch that quantises the row itself
         return pg_launch_gemv_w8a8_f32_row_group(ctx, a_dev, k, w, out_dev, (int)count, nullptr);
     if (apart && count > 1 && pg_gemm_w8a8_takes_f32_rows(ctx, w, (int)count, m)) return pg_launch_gemm_w8a8_f32_rows(ctx, a_dev, w, out_dev, (int)count, m);
-    if (count > 1 && pg_gemm_w8a8_takes_skinny(ctx, w, (int)count, m)) {  // 2 .. 512 rows: quantised once, then the weights side by side in one launch
+    // one weight: the single product picks its own route (GEMV, split K)
+    if (count == 1) return pg_matmul_quantized_dev(ctx, a_dev, m, k, w[0], out_dev[0], nullptr);
+    const pg_w8a8_route route = pg_gemm_w8a8_route(ctx, w, (int)count, m);
+    if (route.kind == PG_W8A8_ROWS) {  // 2 .. 512 rows: quantised once, then the weights side by side in one launch
         const size_t k_pad = w[0]->k_pad, m_pad = pg_round_up(m, PG_MPAD), a_bytes = m_pad * k_pad;
         void *ws = nullptr;
         PG_TRY(pg_workspace(ctx, a_bytes + pg_round_up(m_pad * sizeof(float), 256), &ws));
         int8_t *a_i8 = static_cast<int8_t *>(ws);
         float *a_scales = reinterpret_cast<float *>(a_i8 + a_bytes);
         PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, k_pad, a_scales));
-        return pg_launch_gemm_w8a8_skinny_group(ctx, a_i8, k_pad, a_scales, w, out_dev, (int)count, m, nullptr);  // one launch for all
+        return pg_launch_gemm_w8a8_skinny_group(ctx, a_i8, k_pad, a_scales, w, out_dev, (int)count, m, nullptr, route.index);  // one launch for all
     }
-    // one weight: the single product picks its own route (GEMV, split K)
-    if (count == 1) return pg_matmul_quantized_dev(ctx, a_dev, m, k, w[0], out_dev[0], nullptr);
     const size_t k_pad = w[0]->k_pad, m_pad = pg_round_up(m, PG_MPAD);
     const size_t a_bytes = m_pad * k_pad, sz_scales = pg_round_up(m_pad * sizeof(float), 256);
     void *ws = nullptr;

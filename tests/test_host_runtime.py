@@ -374,6 +374,53 @@ def test_w8a32_tile_is_the_one_that_took_least(host, m, k, n, tile):
     assert len(names) == 2 and "gemm_w8a8_kernelILi%dELi%dE" % tile in names[1], names
 
 
+def int8_call(host, m, k, ns):
+    """The kernels of one W8A8 product over one weight or several."""
+    qs = []
+    for n in ns:
+        w = host.alloc(k * n)
+        qs.append(host.new("pg_qtensor_from_f32_dev", host.ctx, w, k, n))
+        host.ok("pg_dev_free", host.ctx, w)
+    x, outs = host.alloc(m * k), [host.alloc(m * n) for n in ns]
+    host.lib.pghost_clear_launches()
+    if len(ns) == 1:
+        host.ok("pg_matmul_quantized_dev", host.ctx, x, m, k, qs[0], outs[0], None)
+    else:
+        tab = lambda of: (C.c_void_p * len(of))(*[p.value for p in of])
+        host.ok("pg_matmul_quantized_multi_dev", host.ctx, x, m, k, tab(qs), len(ns), tab(outs))
+    for p in [x] + outs:
+        host.ok("pg_dev_free", host.ctx, p)
+    for q in qs:
+        host.lib.pg_qtensor_free(host.ctx, q)
+    return [name for name, _ in host.launches()]
+
+
+def tile(bm, bn):
+    return "gemm_w8a8_kernelILi%dELi%dE" % (bm, bn)
+
+
+def rows_in_groups(mb, nb, nw, nst):
+    return "gemm_w8a8_skinny_kernelILi%dELi%dELi%dELi%dELb0ELb1E" % (mb, nb, nw, nst)
+
+
+@pytest.mark.parametrize("m,k,ns,kernel,finish", [
+    (225, 4026, [1099], rows_in_groups(3, 2, 8, 2), False),           # 12.6 us; groups of 48 rows, a weight tile each, 17.4: 69 weight tiles x 5 on 8 XCDs
+    (110, 5660, [1350], rows_in_groups(2, 2, 8, 2), False),           # 12.3; 16.3
+    (197, 6464, [298, 507], rows_in_groups(2, 2, 8, 2), False),       # 13.2; 18.5
+    (200, 10240, [50257], tile(256, 256), False),                     # 165; 197 on 128x64
+    (111, 7102, [49915], tile(128, 256), False),                      # 87; 120
+    (100, 4096, [50257], tile(128, 256), False),                      # 56; 70
+    (40, 1024, [50257], tile(64, 64), False),                         # 19.5; all rows in a workgroup 29.6
+    (62, 5302, [14499], tile(64, 64), False),                         # 22.7; 28.4
+    (163, 12022, [6319], tile(128, 128), True),                       # 43.1; 58.2 on 64x64
+    (132, 9671, [2828, 7938], tile(64, 64), False),                   # 50; 70 with one apart
+])
+def test_int8_product_of_some_rows_takes_a_kernel_that_was_clearly_faster(host, m, k, ns, kernel, finish):
+    """Products of which another kernel took at least a tenth longer than this one (us, both sides beside them)."""
+    names = int8_call(host, m, k, ns)
+    assert kernel in names[1] and len(names) == 2 + finish and ("splitk_finish" in names[-1]) == finish, names
+
+
 def same_call_captured(host, name, *args):
     """A call that has run once at its shape is captured whole, as launches alone."""
     host.ok(name, host.ctx, *args)
