@@ -1164,21 +1164,26 @@ bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
 }
 // From 33 rows on: the tiles of 64x64 to 128x128 by rounds of workgroups, one a CU, times what a round takes (18, 24 and 40: us at K =
 // 4096; drawn from 180 shapes to 2500 rows and 130000 columns, 0.1 % over the best of the three), unless other tiles, or up to 512 rows groups
-// of 16 or 32 of them in the few-row kernel (whose wavefronts cut K), are estimated to take less than 0.92 of that: the estimates err
-// by 5 to 6 %, and they were fitted to 434 products of 33 .. 2048 rows, K and n 256 .. 8192 (weights from HBM and from the Infinity
-// Cache, each kernel timed on each), so past 8192 columns the three tiles stay.  The estimates as in pick_tile, with what each kernel's idle
-// places give back fitted too.  Against the three tiles alone: 33 to 64 rows 0.71 of the time, 65 to 256 0.85, 257 to 700 0.95, beyond 0.96
-// (without the margin 0.70, 0.83, 0.93 and 0.94, and up to 5 % more where it errs).  us, before : now: 54 x 2150 -> 488 14.9 : 9.4,
-// 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.
+// of 16 or 32 of them in the few-row kernel (whose wavefronts cut K), are estimated to take less than 0.9 of that.  The estimates as in
+// pick_tile, a group's workgroups counted by XCD as in the few-row route (by the part, 467 x 8337 -> 534 went to groups of 32 rows, 58.6 us where
+// 64x64 takes 39 and 32x64 34), fitted to 480 products of 33 .. 2048 rows, K to 16384 and n to 131072 (weights from HBM and from the Infinity
+// Cache, each kernel timed on each): of those none takes longer than with the three tiles alone; 33 to 64 rows 0.78 of the time, 65 to
+// 256 0.84, 257 to 700 0.94, beyond 0.99 (without the margin 0.77, 0.83, 0.92 and 0.97, and now and then 5 % more).  us, those : these: 54 x 2150 -> 488
+// 14.9 : 9.4, 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.
 struct w8a32_kernel {
-    unsigned bm, bn, resident, runs;  // rows, columns, workgroups a CU holds, parts of K within a workgroup
-    double step[2], round, fixed, l2, output, idle;
+    unsigned bm, bn, resident, runs;  // rows, columns, workgroups a CU holds, parts of K within a workgroup (more than one: groups of rows)
+    double step[2], round, fixed, l2, weights, output, ragged, idle;
 };
-constexpr w8a32_kernel W8A32[] = {{32, 64, 2, 1, {0.376, 0.414}, 1.87, 3.44, 0.0677, 0.0, 0.152},   {32, 128, 1, 1, {0.506}, 2.46, 2.82, 0.0219, 2.59, 0.276},
-                                  {32, 128, 2, 1, {0.703, 0.782}, 1.54, 3.30, 0.0493, 1.41, 0.239}, {64, 128, 1, 1, {0.826}, 3.02, 2.80, 0.0448, 1.43, 0.299},
-                                  {128, 128, 1, 1, {1.478}, 6.02, 0.61, 0.0155, 2.71, 0.282},       {64, 256, 1, 1, {1.295}, 8.34, 0.0, 0.0537, 3.04, 0.291},
-                                  {16, 32, 1, 4, {0.634}, 0.0, 4.67, 0.0541, 11.3, 0.263},          {16, 16, 1, 8, {0.872}, 0.0, 3.74, 0.0530, 17.3, 0.0},
-                                  {32, 32, 1, 4, {1.044}, 1.29, 3.48, 0.0491, 8.49, 0.129},         {64, 64, 1, 1, {0.509}, 2.68, 2.96, 0.0714, 0.0, 0.217}};  // 6 .. 8: groups of rows
+constexpr w8a32_kernel W8A32[] = {{32, 64, 2, 1, {0.355, 0.394}, 1.94, 2.37, 0.0567, 0.126, 0.500, 0.0, 0.020},
+                                  {32, 128, 1, 1, {0.486}, 2.93, 1.45, 0.0318, 0.230, 0.500, 0.0, 0.214},
+                                  {32, 128, 2, 1, {0.768, 0.757}, 1.46, 2.19, 0.0530, 0.100, 1.149, 0.048, 0.270},
+                                  {64, 128, 1, 1, {0.740}, 2.73, 1.43, 0.0475, 0.100, 1.285, 0.0, 0.170},
+                                  {128, 128, 1, 1, {1.301}, 3.29, 0.42, 0.0726, 0.100, 1.219, 0.536, 0.060},
+                                  {64, 256, 1, 1, {1.152}, 5.35, 0.0, 0.0723, 0.125, 1.154, 1.556, 0.090},
+                                  {16, 32, 1, 4, {0.748}, 0.93, 1.90, 0.0, 0.100, 0.500, 0.0, 0.193},
+                                  {16, 16, 1, 8, {1.127}, 0.0, 2.33, 0.0376, 0.100, 14.382, 0.999, 0.122},
+                                  {32, 32, 1, 4, {1.189}, 1.26, 1.98, 0.0, 0.100, 0.500, 0.0, 0.116},
+                                  {64, 64, 1, 1, {0.568}, 2.20, 1.93, 0.0, 0.226, 3.431, 0.0, 0.231}};
 // Up to 32 rows: the kernels of 16 and 32 rows a group (-1: the one that takes all rows in a workgroup, up to four wavefronts) from the K on
 // where eight runs of it, or 32 columns a workgroup, are the shorter walk; 110 products of 2 .. 32 rows.  us, before : now: 17 x 6011 -> 420
 // 17.2 : 10.9, 31 x 7127 -> 2249 20.0 : 16.3, 27 x 3326 -> 6259 19.2 : 15.5, 3 x 4650 -> 6594 17.5 : 12.9, 2 x 6124 -> 287 12.0 : 10.3;
@@ -1192,22 +1197,21 @@ static int pick_w8a32_few(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
 static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w->k_pad / 128);
     const double output = 1e-6 * (double)(m * w->cols), digits = 3.0 + 1.3e-6 * (double)(m * w->k_pad);  // (the launch before, in the margin's us)
+    const double weights = 1e-6 * (double)(w->rows * w->cols), ragged = w->cols % 32 ? output : 0.0;
     auto estimate = [&](int i) {
         const w8a32_kernel &t = W8A32[i];
-        const size_t wgs = ((m + t.bm - 1) / t.bm) * ((w->cols + t.bn - 1) / t.bn), most = (wgs + cus - 1) / cus, full = most / t.resident, rest = most % t.resident;
-        const double steps = (double)((kt + t.runs - 1) / t.runs);
-        double cu = (double)full * (steps * t.step[t.resident - 1] + 0.5 * (t.resident + 1) * t.round);
-        if (rest) cu += steps * t.step[rest - 1] + 0.5 * (double)(rest + 1) * t.round;
-        cu *= 1.0 - t.idle * (1.0 - (double)wgs / (double)(most * cus));
-        const double all = 128e-6 * (double)(wgs * kt) * (3 * t.bm + t.bn) * t.l2 + output * t.output;
+        size_t columns = (w->cols + t.bn - 1) / t.bn;
+        if (t.runs > 1) columns = (columns + 7) / 8 * 8;
+        const size_t wgs = (m + t.bm - 1) / t.bm * columns;
+        const double cu = fullest_cu(wgs, cus, t.resident, t.step, (kt + t.runs - 1) / t.runs, t.round, t.idle);
+        const double all = 128e-6 * (double)(wgs * kt) * (3 * t.bm + t.bn) * t.l2 + weights * t.weights + output * t.output + ragged * t.ragged;
         const double c2 = cu * cu, a2 = all * all;
         return digits + t.fixed + sqrt(sqrt(c2 * c2 + a2 * a2));
     };
     auto rounds = [&](size_t bm, size_t bn, size_t us) { return (((m + bm - 1) / bm) * ((w->cols + bn - 1) / bn) + cus - 1) / cus * us; };
     const size_t c0 = rounds(64, 64, 18), c1 = rounds(64, 128, 24), c2 = rounds(128, 128, 40);
     int best = c2 < c0 && c2 < c1 ? 4 : c1 < c0 ? 3 : 9;
-    if (w->cols > 32 * (size_t)cus) return best;
-    double best_us = 0.92 * estimate(best);
+    double best_us = 0.9 * estimate(best);
     for (int i = 0; i < (int)(sizeof(W8A32) / sizeof(W8A32[0])); ++i) {
         if (W8A32[i].runs > 1 && m > 512) continue;
         const double us = estimate(i);
