@@ -116,3 +116,28 @@ def build_gguf(metadata, tensors, version=3, magic=0x46554747):
     for name, typ, shape, raw in tensors:
         body[offsets[name]: offsets[name] + len(raw)] = raw
     return head + b"\0" * (data_start - len(head)) + bytes(body), data_start, offsets
+
+
+# Small ragged products and the kernel each runs on, by the dispatch's own choice: a name's part, as the compiler spells it.
+def _tile(bm, bn, nst):
+    return "gemm_w8a8_kernelILi%dELi%dELi128ELi%dE" % (bm, bn, nst)
+
+
+def _rows(mb, nb, nw, nst, tri):
+    return "gemm_w8a8_skinny_kernelILi%dELi%dELi%dELi%dELb%dELb1E" % (mb, nb, nw, nst, tri)
+
+
+INT8_ROUTES = [
+    (410, 69, 4953, _tile(64, 64, 3)), (249, 184, 3406, _tile(64, 64, 4)), (143, 70, 6288, _tile(128, 64, 3)), (292, 404, 9829, _tile(128, 128, 4)),
+    (257, 1191, 11804, _tile(128, 192, 3)), (1117, 478, 6849, _tile(128, 256, 3)), (907, 67, 4767, _tile(256, 128, 3)), (1910, 664, 5893, _tile(256, 192, 2)),
+    (36, 12871, 303, _tile(64, 64, 4)), (34, 9736, 451, _tile(64, 64, 4)), (71, 12547, 2629, _tile(128, 128, 4)),                     # K split
+    (492, 136, 24, _rows(2, 1, 2, 2, 0)), (46, 72, 7032, _rows(2, 1, 2, 2, 0)), (85, 259, 2159, _rows(2, 1, 4, 3, 0)), (209, 192, 214, _rows(2, 1, 8, 3, 0)),
+    (41, 292, 4200, _rows(2, 2, 4, 2, 0)), (268, 294, 422, _rows(2, 2, 8, 2, 0)), (38, 2820, 2221, _rows(3, 1, 8, 2, 0)), (37, 2520, 15993, _rows(3, 2, 4, 2, 0)),
+    (109, 513, 2335, _rows(3, 2, 8, 2, 0)), (52, 2329, 4970, _rows(4, 2, 4, 3, 0)),
+]
+INT8_SPLIT = {(36, 12871, 303), (34, 9736, 451), (71, 12547, 2629)}
+W8A32_ROUTES = [
+    (201, 2071, 1346, _tile(32, 64, 3)), (527, 1156, 1895, _tile(32, 128, 3)), (168, 84, 4949, _tile(32, 128, 2)), (305, 70, 3790, _tile(64, 128, 3)),
+    (539, 77, 3716, _tile(128, 128, 2)), (52, 70, 38752, _tile(64, 256, 2)), (162, 81, 39168, _tile(64, 256, 2)), (118, 71, 452, _tile(64, 64, 3)),
+    (45, 834, 20, _rows(3, 1, 8, 2, 1)), (47, 70, 18, _rows(3, 2, 4, 3, 1)), (43, 390, 2670, _rows(6, 2, 4, 2, 1)),
+]

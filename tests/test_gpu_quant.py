@@ -373,7 +373,7 @@ def test_every_gemm_tile_gives_the_same_bits(ctx, orc, m, k, n):
 @pytest.mark.parametrize("m,k,n", [(257, 128, 510),       # panels of 192 columns that end behind the weight's padding; one step of K
                                     (512, 300, 768), (90, 700, 193), (300, 640, 1030)])
 def test_wide_gemm_tiles_give_the_same_bits(ctx, orc, m, k, n):
-    """The tiles of codes 6 to 8, and 64x64 with three stages (many tiles) and four (few), as the others above."""
+    """The tiles of codes 6 to 8, and 64x64, as the others above (from 33 rows on a tile that is asked for is what runs)."""
     from peregrine_amd import quant, _ffi
     a = outlier_acts(orc, 17 + m, m, k)
     w = orc.rng_normal(18 + n, k * n, 0.0, 0.02)
@@ -391,7 +391,7 @@ def test_wide_gemm_tiles_give_the_same_bits(ctx, orc, m, k, n):
                 _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, da.ptr, m, k, qt._gpu, out, acc_ptr))
                 ctx.sync()
                 bm, bn, sp = last_tile(ctx)
-                assert sp > 1 or (bm, bn) == tile
+                assert sp == 1 and (bm, bn) == tile
                 got = dout.to_host(np.float32)[skew // 4:skew // 4 + m * n]
                 assert (bits(got) == bits(want)).all(), f"tile {tile}: f32 outputs differ"
             assert (dacc.to_host(np.int32) == want_acc).all(), f"tile {tile}: accumulators differ"
@@ -418,6 +418,26 @@ def test_chosen_gemm_tiles_against_numpy(ctx, orc, m, k, n, tile):
     got = dout.to_host(np.float32).reshape(m, n)
     want = (a.astype(np.float64) @ qi.astype(np.float64)).astype(np.float32)   # |sum| < 2^53; rounded once, as (float)acc is
     assert (bits(got) == bits(want)).all()
+    qt.free_gpu()
+
+
+@pytest.mark.parametrize("m,k,n,kernel", H.INT8_ROUTES)
+def test_int8_routes_against_numpy(ctx, orc, m, k, n, kernel):
+    """The same on ragged products of every kernel from 33 rows on (test_host_runtime.py says that these kernels run), with the
+    accumulators."""
+    from peregrine_amd import quant, _ffi
+    say(f"int8 route m={m} k={k} n={n} {kernel}")
+    rng = np.random.default_rng(m + k)
+    a = rng.integers(-127, 128, (m, k)).astype(np.float32)
+    a[:, 0] = 127.0
+    qi = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    qt = quant.QuantizedTensor(qi.reshape(-1), np.ascontiguousarray(qi.T).reshape(-1), np.ones(n, np.float32), k, n).to_gpu(ctx)
+    da, dout, dacc = DevBuf(ctx, host=a), DevBuf(ctx, m * n * 4), DevBuf(ctx, m * n * 4)
+    want = a.astype(np.float64) @ qi.astype(np.float64)
+    for acc in (None, dacc.ptr):
+        _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, da.ptr, m, k, qt._gpu, dout.ptr, acc))
+        assert (bits(dout.to_host(np.float32).reshape(m, n)) == bits(want.astype(np.float32))).all()
+    assert (dacc.to_host(np.int32).reshape(m, n) == want).all()
     qt.free_gpu()
 
 
@@ -634,13 +654,13 @@ def test_matmul_dequant_i8_one_launch(ctx, orc, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [
-    (519, 2221, 73), (186, 408, 2870), (211, 102, 3608), (1060, 665, 1904), (770, 105, 2959), (526, 1666, 3890),   # each of the tiles
+    (519, 2221, 73), (186, 408, 2870), (211, 102, 3608), (1060, 665, 1904), (770, 105, 2959), (526, 1666, 3890),   # the tiles
     (391, 631, 2419), (580, 209, 3254), (1071, 1731, 3635),
     (124, 1073, 515), (512, 174, 73), (212, 174, 73), (74, 396, 1118), (33, 128, 17), (513, 1000, 64),             # groups of rows, their ends
     (9, 1530, 4100), (8, 3000, 70), (17, 1500, 30), (32, 1409, 2049), (31, 2500, 4097),                             # few rows of long K
-])
+] + [r[:3] for r in H.W8A32_ROUTES])
 def test_matmul_dequant_i8_on_every_kernel(ctx, orc, m, k, n):
-    """Each kernel of the one launch from 33 rows on, at ragged sizes that are given to it.  Small integers are exact; random
+    """Each kernel of the one launch from 33 rows on, at ragged sizes (the last ones: test_host_runtime.py says which runs).  Small integers are exact; random
     rows are within the activation step (2^-23 of the row's largest value a value) and one rounding of the float64 product."""
     from peregrine_amd import quant
     say(f"matmul_dequant_i8 kernels m={m} k={k} n={n}")

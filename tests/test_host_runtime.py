@@ -421,6 +421,23 @@ def test_int8_product_of_some_rows_takes_a_kernel_that_was_clearly_faster(host, 
     assert kernel in names[1] and len(names) == 2 + finish and ("splitk_finish" in names[-1]) == finish, names
 
 
+@pytest.mark.parametrize("m,k,n,kernel", H.INT8_ROUTES)
+def test_int8_products_run_on_the_kernels_that_they_are_tested_on(host, m, k, n, kernel):
+    """What the results of these products are compared for (test_gpu_quant.py): every kernel from 33 rows on."""
+    names = int8_call(host, m, k, [n])
+    assert kernel in names[1] and len(names) == (3 if (m, k, n) in H.INT8_SPLIT else 2), names
+
+
+@pytest.mark.parametrize("m,k,n,kernel", H.W8A32_ROUTES)
+def test_w8a32_products_run_on_the_kernels_that_they_are_tested_on(host, m, k, n, kernel):
+    names, _ = dequant_i8_call(host, m, k, n)
+    assert kernel in names[1] and len(names) == 2, names
+
+
+def test_the_tested_int8_kernels_are_all_there_are():
+    assert len({r[3] for r in H.INT8_ROUTES}) == 8 + 9 and len({r[3] for r in H.W8A32_ROUTES}) == 10   # (256x256: the prefill shapes)
+
+
 @pytest.mark.parametrize("m,k,n,kernel", [(467, 8337, 534, "kernelILi32ELi64E"), (257, 2717, 783, "kernelILi32ELi64E")])
 def test_w8a32_groups_of_rows_are_counted_by_xcd(host, m, k, n, kernel):
     """34.1 us against 58.6 in groups of 32 rows, whose 17 weight tiles x 15 groups are up to 45 workgroups for an XCD's 32
