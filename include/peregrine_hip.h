@@ -595,7 +595,7 @@ pg_status pg_probe_gemm_clock(pg_ctx *ctx, size_t m, size_t k, size_t n, double 
  * the output tile (rows x columns) and the number of K splits of the most recent W8A8 GEMM
  * launch on this context, and an override of the dispatcher's tile choice (0 = automatic,
  * 1 = 64x64, 2 = 256x256, 3 = 128x256, 4 = 128x64, 5 = 128x128, 6 = 128x192, 7 = 256x128, 8 = 256x192).  Every tile gives the same
- * bits; tests use the pair to prove each kernel instantiation ran. */
+ * bits (the W8A32 product's last pass has the first five, 256x256 for the others); tests use the pair to prove each kernel instantiation ran. */
 pg_status pg_gemm_w8a8_last_tile(const pg_ctx *ctx, int *bm, int *bn, int *k_splits);
 pg_status pg_gemm_w8a8_force_tile(pg_ctx *ctx, int tile);
 /* The one-row product that takes the activation row in f32: the workgroup shape (wavefronts per workgroup 4, 8 or

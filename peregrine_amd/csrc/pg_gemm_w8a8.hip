@@ -835,13 +835,21 @@ int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m
 pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                         const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc,
                         int pick = -1, const int32_t *comb = nullptr, size_t comb_plane = 0) {
-    // (the combining pass is for products that fill the part with 256x256 tiles: w8a32_large)
-    if (pick < 0) pick = comb && !ctx->gemm_force_tile ? 1 : pick_tile(ctx, w, count, m);
+    if (comb) {  // (for products that fill the part with 256x256 tiles: w8a32_large; the first five codes for tests)
+#define PG_COMB(CODE, ...) \
+    if (code == CODE) return launch_group<__VA_ARGS__, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
+        const int code = ctx->gemm_force_tile >= 1 && ctx->gemm_force_tile <= 5 ? ctx->gemm_force_tile : 2;
+        PG_COMB(1, 64, 64, 128, 3, 2, 2, 3)
+        PG_COMB(2, 256, 256, 128, 2, 2, 4, 2)
+        PG_COMB(3, 128, 256, 128, 3, 2, 4, 2)
+        PG_COMB(4, 128, 64, 128, 3, 4, 2, 4)
+        PG_COMB(5, 128, 128, 128, 4, 2, 4, 2)
+#undef PG_COMB
+    }
+    if (pick < 0) pick = pick_tile(ctx, w, count, m);
     switch (pick) {
-#define PG_TILE(CODE, ...)                                                                                                                    \
-        case CODE:                                                                                                                            \
-            if (comb) return launch_group<__VA_ARGS__, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);   \
-            return launch_group<__VA_ARGS__>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
+#define PG_TILE(INDEX, ...) \
+        case INDEX: return launch_group<__VA_ARGS__>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc);
         PG_TILE(0, 64, 64, 128, 3, 2, 2, 3)
         PG_TILE(1, 256, 256, 128, 2, 2, 4, 2)
         PG_TILE(2, 128, 256, 128, 3, 2, 4, 2)
@@ -1167,7 +1175,7 @@ bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
 // of 16 or 32 of them in the few-row kernel (whose wavefronts cut K), are estimated to take less than 0.9 of that.  The estimates as in
 // pick_tile, a group's workgroups counted by XCD as in the few-row route (by the part, 467 x 8337 -> 534 went to groups of 32 rows, 58.6 us where
 // 64x64 takes 39 and 32x64 34), fitted to 480 products of 33 .. 2048 rows, K to 16384 and n to 131072 (weights from HBM and from the Infinity
-// Cache, each kernel timed on each): of those none takes longer than with the three tiles alone; 33 to 64 rows 0.78 of the time, 65 to
+// Cache, each kernel timed on each): of those none takes over 2 % longer than with the three tiles alone; 33 to 64 rows 0.78 of the time, 65 to
 // 256 0.84, 257 to 700 0.94, beyond 0.99 (without the margin 0.77, 0.83, 0.92 and 0.97, and now and then 5 % more).  us, those : these: 54 x 2150 -> 488
 // 14.9 : 9.4, 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.
 struct w8a32_kernel {

@@ -438,6 +438,14 @@ def test_the_tested_int8_kernels_are_all_there_are():
     assert len({r[3] for r in H.INT8_ROUTES}) == 8 + 9 and len({r[3] for r in H.W8A32_ROUTES}) == 10   # (256x256: the prefill shapes)
 
 
+@pytest.mark.parametrize("code,bm,bn", [(0, 256, 256), (1, 64, 64), (2, 256, 256), (3, 128, 256), (4, 128, 64), (5, 128, 128), (6, 256, 256), (7, 256, 256), (8, 256, 256)])
+def test_w8a32_last_pass_by_tile_override(host, code, bm, bn):
+    host.ok("pg_gemm_w8a8_force_tile", host.ctx, code)
+    names, _ = dequant_i8_call(host, 2048, 128, 5888)
+    host.ok("pg_gemm_w8a8_force_tile", host.ctx, 0)
+    assert len(names) == 3 and "gemm_w8a8_kernelILi%dELi%dE" % (bm, bn) in names[2] and "ELb0ELb1ELi1E" in names[2], names
+
+
 @pytest.mark.parametrize("m,k,n,kernel", [(467, 8337, 534, "kernelILi32ELi64E"), (257, 2717, 783, "kernelILi32ELi64E")])
 def test_w8a32_groups_of_rows_are_counted_by_xcd(host, m, k, n, kernel):
     """34.1 us against 58.6 in groups of 32 rows, whose 17 weight tiles x 15 groups are up to 45 workgroups for an XCD's 32
