@@ -370,6 +370,7 @@ def test_memory_another_context_has_used_is_not_pooled(host, users):
 @pytest.mark.parametrize("m,k,n,tile", [(197, 1024, 4096, (64, 64)), (356, 4096, 14336, (64, 128)), (1000, 4096, 4096, (128, 128)), (311, 2048, 32000, (64, 128)),
                                         (155, 1024, 103918, (64, 128)), (888, 11222, 4096, (128, 128))])
 def test_w8a32_tile_is_the_one_that_took_least(host, m, k, n, tile):
+    """Of 64x64, 64x128 and 128x128; another kernel has to be estimated below 0.9 of it."""
     names, _ = dequant_i8_call(host, m, k, n)
     assert len(names) == 2 and "gemm_w8a8_kernelILi%dELi%dE" % tile in names[1], names
 
