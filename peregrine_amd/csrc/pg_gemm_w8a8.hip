@@ -1172,11 +1172,12 @@ bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
 }
 // From 33 rows on: the tiles of 64x64 to 128x128 by rounds of workgroups, one a CU, times what a round takes (18, 24 and 40: us at K =
 // 4096; drawn from 180 shapes to 2500 rows and 130000 columns, 0.1 % over the best of the three), unless other tiles, or up to 512 rows groups
-// of 16 or 32 of them in the few-row kernel (whose wavefronts cut K), are estimated to take less than 0.9 of that.  The estimates as in
+// of 16 or 32 of them in the few-row kernel (whose wavefronts cut K), are estimated to take less than 0.93 of that, past 700 rows 0.9 (they err
+// more there: at 0.92 one of 85 took 5 % longer).  The estimates as in
 // pick_tile, a group's workgroups counted by XCD as in the few-row route (by the part, 467 x 8337 -> 534 went to groups of 32 rows, 58.6 us where
 // 64x64 takes 39 and 32x64 34), fitted to 480 products of 33 .. 2048 rows, K to 16384 and n to 131072 (weights from HBM and from the Infinity
-// Cache, each kernel timed on each): of those none takes over 2 % longer than with the three tiles alone; 33 to 64 rows 0.78 of the time, 65 to
-// 256 0.84, 257 to 700 0.94, beyond 0.99 (without the margin 0.77, 0.83, 0.92 and 0.97, and now and then 5 % more).  us, those : these: 54 x 2150 -> 488
+// Cache, each kernel timed on each): of those none takes over 2 % longer than with the three tiles alone; 33 to 64 rows 0.77 of the time, 65 to
+// 256 0.83, 257 to 700 0.93, beyond 0.99 (without the margins 0.77, 0.83, 0.92 and 0.97, and now and then 5 % more).  us, those : these: 54 x 2150 -> 488
 // 14.9 : 9.4, 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.
 struct w8a32_kernel {
     unsigned bm, bn, resident, runs;  // rows, columns, workgroups a CU holds, parts of K within a workgroup (more than one: groups of rows)
@@ -1219,7 +1220,7 @@ static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     auto rounds = [&](size_t bm, size_t bn, size_t us) { return (((m + bm - 1) / bm) * ((w->cols + bn - 1) / bn) + cus - 1) / cus * us; };
     const size_t c0 = rounds(64, 64, 18), c1 = rounds(64, 128, 24), c2 = rounds(128, 128, 40);
     int best = c2 < c0 && c2 < c1 ? 4 : c1 < c0 ? 3 : 9;
-    double best_us = 0.9 * estimate(best);
+    double best_us = (m <= 700 ? 0.93 : 0.9) * estimate(best);
     for (int i = 0; i < (int)(sizeof(W8A32) / sizeof(W8A32[0])); ++i) {
         if (W8A32[i].runs > 1 && m > 512) continue;
         const double us = estimate(i);

@@ -370,7 +370,7 @@ def test_memory_another_context_has_used_is_not_pooled(host, users):
 @pytest.mark.parametrize("m,k,n,tile", [(197, 1024, 4096, (64, 64)), (356, 4096, 14336, (64, 128)), (1000, 4096, 4096, (128, 128)), (311, 2048, 32000, (64, 128)),
                                         (155, 1024, 103918, (64, 128)), (888, 11222, 4096, (128, 128))])
 def test_w8a32_tile_is_the_one_that_took_least(host, m, k, n, tile):
-    """Of 64x64, 64x128 and 128x128; another kernel has to be estimated below 0.9 of it."""
+    """Of 64x64, 64x128 and 128x128; another kernel has to be estimated below 0.93 of it (past 700 rows 0.9)."""
     names, _ = dequant_i8_call(host, m, k, n)
     assert len(names) == 2 and "gemm_w8a8_kernelILi%dELi%dE" % tile in names[1], names
 
@@ -447,10 +447,10 @@ def test_w8a32_last_pass_by_tile_override(host, code, bm, bn):
     assert len(names) == 3 and "gemm_w8a8_kernelILi%dELi%dE" % (bm, bn) in names[2] and "ELb0ELb1ELi1E" in names[2], names
 
 
-@pytest.mark.parametrize("m,k,n,kernel", [(467, 8337, 534, "kernelILi32ELi64E"), (257, 2717, 783, "kernelILi32ELi64E")])
+@pytest.mark.parametrize("m,k,n,kernel", [(467, 8337, 534, "kernelILi32ELi64E"), (257, 2717, 783, "kernelILi32ELi64E"), (56, 8914, 7775, "kernelILi32ELi64E")])
 def test_w8a32_groups_of_rows_are_counted_by_xcd(host, m, k, n, kernel):
     """34.1 us against 58.6 in groups of 32 rows, whose 17 weight tiles x 15 groups are up to 45 workgroups for an XCD's 32
-    CUs; 16.5 against 20.4."""
+    CUs; 16.5 against 20.4.  (The last one by the margin: 30.7 against 36.3 on 64x64.)"""
     names, _ = dequant_i8_call(host, m, k, n)
     assert kernel in names[1], names
 
