@@ -3,13 +3,20 @@
 //   acc[m, n] = sum_k a_i8[m, k] * w_t[n, k]              (i32, exact)
 //   out[m, n] = ((float)acc * a_scale[m]) * w_scale[n]    (src/quant.rs:163)
 //
-// Both operands are K-contiguous, which is the natural operand layout of
-// v_mfma_i32_32x32x32_i8: lane l supplies 16 consecutive k-bytes of row l%32
-// (half-wave l/32 takes the upper 16 of each 32-wide k step).  The same
-// (lane, byte) -> k mapping is used for A and B, so the sum is over matching k.
+// Both operands are K-contiguous, which is the natural operand layout of v_mfma_i32_16x16x64_i8: lane l supplies 16
+// consecutive k-bytes of row l % 16, its group l / 16 the next 16 of a 64-wide k-step.  The same (lane, byte) -> k mapping is
+// used for A and B, so the sum is over matching k.
+//
+// Why 16x16x64 and not 32x32x32: on a full chip the power limit sets the rate, and for the same multiply-adds it writes
+// half the accumulators.  On random bytes in registers it holds 3.9 to 4.0 POP/s, 32x32x32 3.5 (5.0 both on zeros); the
+// fragments read from LDS are as many.  us, 32x32x32 : 16x16x64, weights from HBM: W8A8 2048 x 4096 -> 14336 134 : 124, 2048 x
+// 14336 -> 4096 158 : 149, 2048 x 4096 -> 6144 63 : 58, 1760 x 12387 -> 15665 356 : 327, 960 x 4001 -> 710 18.8 : 17.5 (120 drawn products of 33
+// rows and more 0.98, 40 drawn layers 0.965 of the time); W8A32 2048 x 4096 -> 14336 416 : 395, 888 x 11222 -> 4096 154 : 134, 356 x 4096 -> 14336
+// 92 : 85, 197 x 1024 -> 4096 10.9 : 10.4 (100 drawn 0.98; four wavefronts a workgroup alone on their CU, which issue it every 18
+// cycles instead of 16, up to 2 % longer: 202 x 5949 -> 1265 25.4 : 26.0).
 //
 // Workgroup = NWM x NWN wavefronts over a BM x BN output tile; each wavefront
-// holds (BM/NWM/32) x (BN/NWN/32) accumulator tiles of 32x32.  K is consumed in
+// holds (BM/NWM/16) x (BN/NWN/16) accumulator tiles of 16x16.  K is consumed in
 // steps of BK bytes through NST LDS stages filled by direct global->LDS loads
 // (global_load_lds_dwordx4): no VGPRs are spent on staging and the fill of later
 // stages overlaps the MFMAs on the current one.
@@ -35,7 +42,6 @@
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 typedef const void __attribute__((address_space(1))) *gptr_t;
 typedef void __attribute__((address_space(3))) *lptr_t;
 
@@ -80,11 +86,11 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
                       int tiles_m, int ntiles, int kt_per_split, long long *__restrict__ clk) {
     constexpr int NW = NWM * NWN;
     constexpr int WM = BM / NWM, WN = BN / NWN;      // wavefront tile
-    constexpr int TM = WM / 32, TN = WN / 32;        // 32x32 MFMA tiles per wavefront
+    constexpr int TM = WM / 16, TN = WN / 16;        // 16x16 MFMA tiles per wavefront
     constexpr int CPR = BK / 16, RPL = 64 / CPR;     // chunks per row, rows per wave-load
     constexpr int LA = NP * BM / RPL / NW, LB = BN / RPL / NW, LPS = LA + LB;  // wave-loads per wave per stage
     constexpr int STAGE = (NP * BM + BN) * BK;            // bytes per LDS stage
-    constexpr int KS = BK / 32;                      // k-steps per stage
+    constexpr int KS = BK / 64;                      // k-steps per stage
     constexpr int TA = NP * TM;                      // activation tiles per wavefront, plane by plane
     constexpr int NF = TA + TN, NMFMA = TA * TN;
     static_assert(NP * BM % (RPL * NW) == 0 && BN % (RPL * NW) == 0 && KS % 2 == 0 && PG_MPAD % BM == 0 && BM <= 64 * NW && BN <= 64 * NW,
@@ -136,9 +142,9 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     int a_off[KS], b_off[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-        const int ra = wm * WM + l31, rb = wn * WN + l31;
-        a_off[ks] = ra * BK + (((2 * ks + half) ^ swz<BK>(ra)) * 16);
-        b_off[ks] = NP * BM * BK + rb * BK + (((2 * ks + half) ^ swz<BK>(rb)) * 16);
+        const int ra = wm * WM + (lane & 15), rb = wn * WN + (lane & 15), chunk = 4 * ks + (lane >> 4);
+        a_off[ks] = ra * BK + ((chunk ^ swz<BK>(ra)) * 16);
+        b_off[ks] = NP * BM * BK + rb * BK + ((chunk ^ swz<BK>(rb)) * 16);
     }
 
     // The scales of this tile's rows and columns go to LDS (behind the stages) now, so that
@@ -150,13 +156,13 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
         if (t < BN) lds_ws[t] = w_scales[n0 + t < N ? n0 + t : N - 1];
     }
 
-    v16i acc[TA][TN];
+    v4i acc[TA][TN];
 #pragma unroll
     for (int i = 0; i < TA; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = 0;
 
     auto issue = [&](int stage, int k0) {
         char *base = lds + stage * STAGE;
@@ -170,17 +176,16 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     auto read_frags = [&](int buf, int stage, int ks) {
         const char *base = lds + stage * STAGE;
 #pragma unroll
-        for (int i = 0; i < TA; ++i) fa[buf][i] = *reinterpret_cast<const v4i *>(base + a_off[ks] + (i / TM * BM + i % TM * 32) * BK);
+        for (int i = 0; i < TA; ++i) fa[buf][i] = *reinterpret_cast<const v4i *>(base + a_off[ks] + (i / TM * BM + i % TM * 16) * BK);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) fb[buf][j] = *reinterpret_cast<const v4i *>(base + b_off[ks] + j * 32 * BK);
+        for (int j = 0; j < TN; ++j) fb[buf][j] = *reinterpret_cast<const v4i *>(base + b_off[ks] + j * 16 * BK);
     };
     auto mfmas = [&](int buf, int lo, int hi) {  // MFMAs lo..hi-1 of the TA x TN set, row-major
 #pragma unroll
         for (int i = 0; i < TA; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-                if (i * TN + j >= lo && i * TN + j < hi)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[buf][i], fb[buf][j], acc[i][j], 0, 0, 0);
+                if (i * TN + j >= lo && i * TN + j < hi) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[buf][i], fb[buf][j], acc[i][j], 0, 0, 0);
     };
     // Before the barrier: this wavefront's LDS reads have returned (lgkmcnt) and all but
     // `ahead` of its youngest stage fills have landed (vmcnt).  After it, every wavefront's
@@ -250,152 +255,97 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
             clk[2 * blockIdx.x + 1] = wall_clock64() - clk_w0;
         }
     }
-    // ---- epilogue.  Accumulator register r of a 32x32 tile holds
-    // row 8*(r/4) + 4*(lane/32) + r%4, column lane%32.  (The scales were requested before the
-    // K loop: loading them here would put several dependent memory round trips on every tile.)
+    // ---- epilogue.  Lane l of a 16x16 tile holds column l % 16 of rows 4 (l / 16) + r.  Two tiles side by side exchange rows of 16
+    // lanes, after which either half-wave has all 32 columns of a row and what is stored is whole lines: value v of register r
+    // is row 8 (lane / 32) + 4 v + r, column lane % 32.  (The scales were requested before the K loop: loading them here would put
+    // several dependent memory round trips on every tile.)
+    //
+    // Tiles inside the matrix are straight-line code (a bounds branch per element: 136 us where this took 118), the row scales of
+    // 16 rows as two 128-bit LDS reads.  Their stores are non-temporal: this kernel never reads the output back, and 117 MB of
+    // it per launch otherwise displace the operands of this and the next launch from L2 and the Infinity Cache (whole prefill
+    // layer 0.633 -> 0.59 ms).  The same hint on the operand fills costs 7 - 15 %.  Rows that do not begin on a line leave the hint off:
+    // the halves of a line then come with different stores, and the hint takes each to memory by itself.  us, with it : without: 1355 x
+    // 2253 -> 11567 78 : 58, 2015 x 8071 -> 4709 143 : 131, 1131 x 1035 -> 8180 41 : 34.  (The kinds of epilogue are code of their own: a branch at
+    // every store cost a layer of 2048 rows 3 %.  The one-launch W8A32 product keeps the hint: its tiles take longer than their stores
+    // either way.)
+    static_assert(TN % 2 == 0, "pairs of column tiles");
+    enum { F32, I32, BOTH };
+    auto store = [&](auto hint, auto inside, auto what) {
+        constexpr int WHAT = decltype(what)::value;
+        auto put = [](auto v, auto *dst) {
+            if constexpr (decltype(hint)::value) __builtin_nontemporal_store(v, dst);
+            else *dst = v;
+        };
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            float as[8];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                const float4 x = *reinterpret_cast<const float4 *>(lds_as + wm * WM + 16 * i + 8 * half + 4 * v);
+                as[4 * v] = x.x; as[4 * v + 1] = x.y; as[4 * v + 2] = x.z; as[4 * v + 3] = x.w;
+            }
+#pragma unroll
+            for (int j = 0; j < TN; j += 2) {
+                const int col = n0 + wn * WN + 16 * j + l31, row0 = m0 + wm * WM + 16 * i + 8 * half;
+                const float ws = lds_ws[wn * WN + 16 * j + l31];
+                const size_t at = (size_t)row0 * N + col;
+                auto stored = [&](int k) { return decltype(inside)::value || (row0 + k < M && col < N); };
+                int c0[8], c1[8];
+                if constexpr (COMB) {  // the two other digits' accumulators, in the order the stores go out (outside the matrix: its last ones)
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const int32_t *c = grp.comb + (decltype(inside)::value ? at + (size_t)k * N : (size_t)min(row0 + k, M - 1) * N + min(col, N - 1));
+                        c0[k] = __builtin_nontemporal_load(c);
+                        c1[k] = __builtin_nontemporal_load(c + grp.comb_plane);
+                    }
+                }
+                int a[NP][8];
+#pragma unroll
+                for (int p = 0; p < NP; ++p)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int x = acc[p * TM + i][j][r], y = acc[p * TM + i][j + 1][r];
+                        const auto two = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+                        a[p][r] = (int)two[0];
+                        a[p][4 + r] = (int)two[1];
+                    }
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    if (!stored(k)) continue;
+                    const size_t o = at + (size_t)k * N;
+                    float f;
+                    if constexpr (NP == 3) f = (float)((65536.0 * (double)a[2][k] + 256.0 * (double)a[1][k] + (double)a[0][k]) * (double)as[k] * (double)ws);
+                    else if constexpr (COMB) f = (float)((65536.0 * (double)a[0][k] + 256.0 * (double)c1[k] + (double)c0[k]) * (double)as[k] * (double)ws);
+                    else f = (float)a[0][k] * as[k] * ws;
+                    if (WHAT == F32) put(f, out + o);
+                    else if (WHAT == I32) put(a[0][k], acc_out + o);
+                    else {
+                        if (out) out[o] = f;
+                        if (acc_out) acc_out[o] = a[0][k];
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);  // one pair of tiles at a time: bounded live ranges
+            }
+        }
+    };
+    using yes = std::true_type;
+    using no = std::false_type;
+    using f32 = std::integral_constant<int, F32>;
+    const bool whole = m0 + BM <= M && n0 + BN <= N;
     if constexpr (NP == 3) {
-        const bool whole = m0 + BM <= M && n0 + BN <= N;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int n = n0 + wn * WN + 32 * j + l31;
-                const double ws = (double)lds_ws[wn * WN + 32 * j + l31];
-                float *dst = out + (size_t)(m0 + wm * WM + 32 * i + 4 * half) * N + n;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int mr = 8 * (r >> 2) + (r & 3);
-                    const double v = 65536.0 * (double)acc[2 * TM + i][j][r] + 256.0 * (double)acc[TM + i][j][r] + (double)acc[i][j][r];
-                    if (whole || (m0 + wm * WM + 32 * i + 4 * half + mr < M && n < N))
-                        __builtin_nontemporal_store((float)(v * (double)lds_as[wm * WM + 32 * i + 4 * half + mr] * ws), dst + (size_t)mr * N);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
+        if (whole) store(yes{}, yes{}, f32{});
+        else store(yes{}, no{}, f32{});
         return;
     }
-    // How whole tiles are stored (see below); rows that do not begin on a line leave the hint off: the halves of a line then come
-    // with different stores, and the hint takes each to memory by itself.  us, with it : without: 1355 x 2253 -> 11567 78 : 58,
-    // 2015 x 8071 -> 4709 143 : 131, 1131 x 1035 -> 8180 41 : 34.
     const bool lines = ((uintptr_t)(acc_out ? (const void *)acc_out : (const void *)out) & 127) == 0 && (N & 31) == 0;
-    // (The two kinds of whole-tile epilogue are code of their own: a branch at every store cost a layer of
-    // 2048 rows 3 %.  The one-launch W8A32 product keeps the hint: its tiles take longer than their stores either way.)
-    auto put = [](auto hint, auto v, auto *dst) {
-        if constexpr (decltype(hint)::value) __builtin_nontemporal_store(v, dst);
-        else *dst = v;
-    };
-    auto either = [&](auto epilogue) {
-        if (lines) epilogue(std::true_type{});
-        else epilogue(std::false_type{});
-    };
-    if (!COMB && out && !acc_out && m0 + BM <= M && n0 + BN <= N) {
-        // A whole tile inside the matrix, f32 output only (every tile of the prefill shapes):
-        // straight-line code, the 16 row scales of a 32-row tile as four 128-bit LDS reads.
-        // The stores are non-temporal: this kernel never reads the output back, and 117 MB of
-        // it per launch otherwise displace the operands of this and the next launch from L2
-        // and the Infinity Cache (whole prefill layer 0.633 -> 0.59 ms).  The same hint on the
-        // operand fills costs 7 - 15 %.
-        either([&](auto hint) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            float as[16];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 v = *reinterpret_cast<const float4 *>(lds_as + wm * WM + 32 * i + 8 * g + 4 * half);
-                as[4 * g] = v.x; as[4 * g + 1] = v.y; as[4 * g + 2] = v.z; as[4 * g + 3] = v.w;
-            }
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const float ws = lds_ws[wn * WN + 32 * j + l31];
-                float *dst = out + (size_t)(m0 + wm * WM + 32 * i + 4 * half) * N + (n0 + wn * WN + 32 * j + l31);
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    put(hint, (float)acc[i][j][r] * as[r] * ws, dst + (size_t)(8 * (r >> 2) + (r & 3)) * N);
-                __builtin_amdgcn_sched_barrier(0);  // one tile's stores at a time: bounded live ranges
-            }
-        }
-        });
-        return;
-    }
-    if (COMB && out && !acc_out && m0 + BM <= M && n0 + BN <= N) {
-        // The W8A32 product's last pass on a whole tile: the two other digits' accumulators are fetched in the
-        // order the stores go out (a lane's rows of one column, four at a time).
-        either([&](auto hint) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            float as[16];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 v = *reinterpret_cast<const float4 *>(lds_as + wm * WM + 32 * i + 8 * g + 4 * half);
-                as[4 * g] = v.x; as[4 * g + 1] = v.y; as[4 * g + 2] = v.z; as[4 * g + 3] = v.w;
-            }
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const double ws = (double)lds_ws[wn * WN + 32 * j + l31];
-                const size_t base = (size_t)(m0 + wm * WM + 32 * i + 4 * half) * N + (n0 + wn * WN + 32 * j + l31);
-#pragma unroll
-                for (int r0 = 0; r0 < 16; r0 += 4) {  // four rows at a time (the 256x256 tile has no registers to spare)
-                    int c0[4], c1[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const size_t idx = base + (size_t)(8 * ((r0 + r) >> 2) + ((r0 + r) & 3)) * N;
-                        c0[r] = __builtin_nontemporal_load(grp.comb + idx);
-                        c1[r] = __builtin_nontemporal_load(grp.comb + grp.comb_plane + idx);
-                    }
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const double v = 65536.0 * (double)acc[i][j][r0 + r] + 256.0 * (double)c1[r] + (double)c0[r];
-                        put(hint, (float)(v * (double)as[r0 + r] * ws), out + base + (size_t)(8 * ((r0 + r) >> 2) + ((r0 + r) & 3)) * N);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                __builtin_amdgcn_sched_barrier(0);  // one tile at a time: bounded live ranges
-            }
-        }
-        });
-        return;
-    }
-    if (acc_out && !out && m0 + BM <= M && n0 + BN <= N) {  // the same for the integer-only output of the W8A32 passes
-        either([&](auto hint) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                int32_t *dst = acc_out + (size_t)(m0 + wm * WM + 32 * i + 4 * half) * N + (n0 + wn * WN + 32 * j + l31);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) put(hint, acc[i][j][r], dst + (size_t)(8 * (r >> 2) + (r & 3)) * N);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        });
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int n = n0 + wn * WN + 32 * j + l31;
-            if (n < N) {
-                const float ws = lds_ws[wn * WN + 32 * j + l31];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * WM + 32 * i + 8 * (r >> 2) + 4 * half + (r & 3);
-                    if (m < M) {
-                        const int a = acc[i][j][r];
-                        const float as = lds_as[wm * WM + 32 * i + 8 * (r >> 2) + 4 * half + (r & 3)];
-                        if (COMB && out) {
-                            const size_t idx = (size_t)m * N + n;
-                            const double v = 65536.0 * (double)a + 256.0 * (double)grp.comb[grp.comb_plane + idx] + (double)grp.comb[idx];
-                            out[idx] = (float)(v * (double)as * (double)ws);
-                        } else if (out) {
-                            out[(size_t)m * N + n] = (float)a * as * ws;
-                        }
-                        if (acc_out) acc_out[(size_t)m * N + n] = a;
-                    }
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);  // one tile's stores at a time: bounded live ranges
-        }
+    if (whole && out && !acc_out) {
+        if (lines) store(yes{}, yes{}, f32{});
+        else store(no{}, yes{}, f32{});
+    } else if (!COMB && whole && !out && acc_out) {  // the integer-only output of the W8A32 passes and of the split product
+        if (lines) store(yes{}, yes{}, std::integral_constant<int, I32>{});
+        else store(no{}, yes{}, std::integral_constant<int, I32>{});
+    } else {
+        store(no{}, no{}, std::integral_constant<int, BOTH>{});
     }
 }
 
@@ -1178,7 +1128,9 @@ bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
 // 64x64 takes 39 and 32x64 34), fitted to 480 products of 33 .. 2048 rows, K to 16384 and n to 131072 (weights from HBM and from the Infinity
 // Cache, each kernel timed on each): of those none takes over 2 % longer than with the three tiles alone; 33 to 64 rows 0.77 of the time, 65 to
 // 256 0.83, 257 to 700 0.93, beyond 0.99 (without the margins 0.77, 0.83, 0.92 and 0.97, and now and then 5 % more).  us, those : these: 54 x 2150 -> 488
-// 14.9 : 9.4, 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.
+// 14.9 : 9.4, 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.  (Fitted while the tiles ran on
+// 32x32x32 matrix instructions and 128x128 on sixteen wavefronts.  It is eight of 32 x 64 now: ten fragment reads a k-step for 24 instructions
+// where it was eight for twelve; us, then : now: 1000 x 4096 -> 4096 64 : 58, 888 x 11222 -> 4096 154 : 134, 2317 x 3643 -> 2853 114 : 107.)
 struct w8a32_kernel {
     unsigned bm, bn, resident, runs;  // rows, columns, workgroups a CU holds, parts of K within a workgroup (more than one: groups of rows)
     double step[2], round, fixed, l2, weights, output, ragged, idle;
@@ -1279,7 +1231,7 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
         case 1: return tiles(launch_group<32, 128, 128, 3, 1, 4, 1, false, 3>);
         case 2: return tiles(launch_group<32, 128, 128, 2, 1, 4, 2, false, 3>);
         case 3: return tiles(launch_group<64, 128, 128, 3, 2, 4, 2, false, 3>);
-        case 4: return tiles(launch_group<128, 128, 128, 2, 4, 4, 4, false, 3>);
+        case 4: return tiles(launch_group<128, 128, 128, 2, 4, 2, 2, false, 3>);
         case 5: return tiles(launch_group<64, 256, 128, 2, 2, 4, 2, false, 3>);
         case 6: return groups(gemm_w8a8_skinny_kernel<3, 2, 4, 3, true, true>, 1, 2, 4, 3);
         case 7: return groups(gemm_w8a8_skinny_kernel<3, 1, 8, 2, true, true>, 1, 1, 8, 2);

@@ -441,6 +441,31 @@ def test_int8_routes_against_numpy(ctx, orc, m, k, n, kernel):
     qt.free_gpu()
 
 
+@pytest.mark.parametrize("semantics,m,k,n", [("w8a8", 1024, 96, 12800), ("w8a8", 1005, 96, 12770), ("w8a8", 1009, 160, 12799), ("w8a32", 1024, 96, 11520),
+                                             ("w8a32", 1005, 96, 11390), ("w8a32", 385, 100, 600), ("w8a32", 384, 96, 640)])
+def test_int8_tiles_store_whole_and_cut_tiles(ctx, orc, semantics, m, k, n):
+    """Products of more than a tile either way, with and without cut tiles and rows that begin on a line: the f32 output, the accumulators,
+    both, and W8A32 in one launch and over two planes of accumulators.  Small integers: every result is exact."""
+    from peregrine_amd import quant, _ffi
+    say(f"int8 tiles {semantics} m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + n)
+    a = rng.integers(-127, 128, (m, k)).astype(np.float32)
+    a[:, 0] = 127.0                                        # so that W8A8's row scale is 1
+    qi = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    qt = quant.QuantizedTensor(qi.reshape(-1), np.ascontiguousarray(qi.T).reshape(-1), np.ones(n, np.float32), k, n).to_gpu(ctx)
+    want = a @ qi.astype(np.float32)                       # |sums| < 2^24: exact in any order
+    da, dout, dacc = DevBuf(ctx, host=a), DevBuf(ctx, m * n * 4), DevBuf(ctx, m * n * 4)
+    if semantics == "w8a32":
+        _ffi.check(_ffi.lib.pg_matmul_dequant_i8_dev(ctx.handle, da.ptr, m, k, qt._gpu, dout.ptr))
+        assert (dout.to_host(np.float32).reshape(m, n) == want).all()
+    else:
+        for acc in (None, dacc.ptr):
+            _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, da.ptr, m, k, qt._gpu, dout.ptr, acc))
+            assert (dout.to_host(np.float32).reshape(m, n) == want).all()
+        assert (dacc.to_host(np.int32).reshape(m, n) == want.astype(np.int32)).all()
+    qt.free_gpu()
+
+
 def run_multi(ctx, da, m, k, qts, douts):
     from peregrine_amd import _ffi
     wtab = (C.c_void_p * len(qts))(*[q._gpu.value for q in qts])
