@@ -354,3 +354,25 @@ def test_sides_of_different_streams(ctx, orc, heads, hd, thr, chunk):
     for side, chunks in ((0, c.k_chunks), (1, c.v_chunks)):
         for i in {0, len(chunks) // 2, len(chunks) - 1}:
             _same_chunk(chunks[i], o.chunk(side, i)[:3])
+
+
+@pytest.mark.parametrize("heads,hd,thr,chunk", [
+    (2, 8, 36, 4),     # chains of 9 steps of 16 bytes: two rounds of 4 loads and one more
+    (3, 7, 40, 8),     # rows that 16 bytes do not divide, the last chains shorter
+    (1, 1, 33, 1),     # one value a chain step
+    (2, 64, 520, 512), # a move shorter than its distance
+    (8, 128, 300, 256),
+])
+def test_the_window_moves_and_grows_in_one_launch(ctx, orc, heads, hd, thr, chunk):
+    """What stays in the window is the same bits after each move to the front, whatever the number of steps, and after each growth."""
+    from peregrine_amd import huffman
+    say(f"huffman kv window heads={heads} head_dim={hd} threshold={thr} chunk={chunk}")
+    rng = np.random.default_rng(thr)
+    c, o = huffman.HuffmanKVCache(heads, hd, thr, chunk, ctx), orc.HuffmanKVCache(heads, hd, thr, chunk)
+    for n in (3, thr - 4, 1, chunk, chunk // 2 + 1, 2 * chunk + 1, 1, 2 * thr):
+        k, v = (rng.standard_normal((heads, n, hd)).astype(np.float32) for _ in range(2))
+        c.append(k, v, n)
+        o.append(k, v, n)
+        assert (c.len(), c.compressed_len, c.hot_len) == (o.len, o.compressed_len, o.hot_len)
+        for got, want in zip(c.get_kv(), o.get_kv()):
+            assert (got.view(np.uint32) == want.view(np.uint32)).all()
