@@ -12,7 +12,7 @@
 // pinned memory) and allocates exactly that much, or, from a cache's second batch on, has launched the encoder into what the
 // batch before took and 1 / 64 where that suits (at most 1 / 32 too much; compress_batch).  A batch was 10 launches, 12 copies and 8
 // waits per pair of chunks before, and the tables were built on the host from copied histograms: 3000 tokens of
-// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.18.
+// 8 x 128, appended 512 at a time in chunks of 256 and read back, took 3.9-4.5 ms, of which 0.8 ms of kernels; now 0.16.
 //
 // The encoder knows where every code starts, so it leaves an index beside the stream (a 16-bit offset per 64 values,
 // 0.25 bit a value): the decoder of such a chunk is one launch that starts a thread per 64 values, with no search for
@@ -31,6 +31,7 @@ namespace {
 constexpr int NUM_SYMBOLS = 256;
 constexpr int KV_MAX_BITS = 12;                // longest code (src/huffman.rs:30)
 constexpr int KV_LUT = 1 << KV_MAX_BITS;
+constexpr int KV_LEVELS = 96;                  // words: by length, the first 12 bits beyond its codes, then where its symbols start less its first code; the symbols by code
 constexpr int KV_WG = 256;
 constexpr int ENC_SPT = 16;                    // symbols per thread of the encoder
 constexpr int ENC_PER_WG = KV_WG * ENC_SPT;    // symbols per workgroup: one histogram and one start bit each
@@ -68,7 +69,7 @@ struct kv_batch {
     uint16_t *hist;               // [count][nwg][256]
     unsigned long long *wg_bit;   // [count][nwg + 1] start bits, then the total
     unsigned *codes;              // [count][256] length << 16 | code
-    uint16_t *lut;                // [count][KV_LUT]
+    unsigned *levels;             // [count][KV_LEVELS] what the decode table is made of
     __device__ const float *head(unsigned c, unsigned h) const { return data[c % sides] + (size_t)(c / sides) * chunk_step + (size_t)h * head_stride; }
 };
 
@@ -384,7 +385,9 @@ __device__ __forceinline__ unsigned merge_trees(unsigned n, const K *leaf_key, K
 // the histograms stay in registers until the runs' bits are known.  A chunk of 262144 normally distributed values, cycles
 // (with every symbol compared with every other, exchanges by compare and select, queues that a round pads itself, and
 // branches around its stores): histograms 2.5 k, order 1.8 k (4.5 k), merges 7.4 k for 18 rounds (13.9 k), depths and counts 2 k, repair 1.5 k
-// (3.2 k), codes and runs 2 k (6 k), decode table 0.8 k (2 k): 9.8 us where it was 15.9; 16384 values 8.6 (13.0).
+// (3.2 k), codes and runs 2 k (6 k): 9.3 us where it was 15.9; 16384 values 8.1 (13.0).  The decode table is left to the encoder's launch,
+// which the host does not wait for, and the host hears of the stream's bits before codes and runs: an append's next one is
+// on its way 1.3 us earlier.
 constexpr unsigned KEPT_ROWS = 4;  // histograms a wavefront keeps: 16 wavefronts, so all of a chunk of up to 64 of them
 template <class K>
 __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsigned long long *host_bits) {
@@ -400,8 +403,8 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
     __shared__ __attribute__((aligned(16))) unsigned cnt[16], first_code[16], limit[16], offset[16];
     __shared__ unsigned lane_cnt[4][16];
     __shared__ __attribute__((aligned(16))) uint8_t bl[NUM_SYMBOLS];
-    __shared__ uint8_t by_len[NUM_SYMBOLS];
-    __shared__ unsigned over, wsum[16];
+    __shared__ __attribute__((aligned(16))) uint8_t by_len[NUM_SYMBOLS];
+    __shared__ unsigned over, wsum[16], stream_sum[4][2];
     __shared__ unsigned run_bits[1024];
     const unsigned c = blockIdx.x, t = threadIdx.x, s = t & 255, p = t >> 8;
     const unsigned lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -575,6 +578,7 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
         }
     }
     __syncthreads();
+    unsigned out_len = 0;
     if (t < n) {
         unsigned len = leaf_len[t];
         if (over) {  // the repaired lengths go out again, shortest to most frequent (ties: lower symbol first)
@@ -583,9 +587,25 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
 #pragma unroll
             for (int l = 2; l <= KV_MAX_BITS; ++l) len += offset[l] <= down ? 1 : 0;
         }
+        out_len = len;
         bl[leaf_sym[t]] = (uint8_t)len;
     }
+    // The stream's bits go to the host as soon as they are known: it makes room and launches the encoder meanwhile, and the caller has its
+    // next append on the way (microseconds that the device otherwise waits out behind the encoder).
+    if (p == 0) {
+        const unsigned long long bits = t < n ? (unsigned long long)leaf_w[t] * out_len : 0ull;  // (below 2^35)
+        const unsigned lo = (unsigned)pg_wave_sum_i32((int)(bits & 0xFFFFFu)), hi = (unsigned)pg_wave_sum_i32((int)(bits >> 20));
+        if (lane == 0) {
+            stream_sum[wave][0] = lo;
+            stream_sum[wave][1] = hi;
+        }
+    }
     __syncthreads();
+    if (t == 1023) {
+        unsigned long long bits = 1;  // (0 = not there yet)
+        for (unsigned w = 0; w < 4; ++w) bits += stream_sum[w][0] + ((unsigned long long)stream_sum[w][1] << 20);
+        __hip_atomic_store(host_bits + c, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     // the symbol's place among those of its length
     unsigned before = 0, len = 0;
     if (p == 0) {
@@ -654,32 +674,30 @@ __global__ __launch_bounds__(1024) void kv_table_kernel(const kv_batch b, unsign
         }
         if (t == 256) wg_bit[b.nwg] = run;
     }
-    // The stream's bits go to the host as soon as they are known: it makes room and launches the encoder meanwhile.
-    const bool tells = t == 256;
     __syncthreads();
-    if (tells) __hip_atomic_store(host_bits + c, run + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // (0 = not there yet)
-    {   // decode table, four entries a thread: length << 8 | symbol; codes nobody has decode as (length 0, value 0)
-        const unsigned x = t * 4;
-        unsigned l = 1;  // (the limits ascend)
+    if (t < KV_LEVELS) b.levels[(size_t)c * KV_LEVELS + t] = t < 16 ? limit[t] : t < 32 ? offset[t - 16] - first_code[t - 16] : reinterpret_cast<const unsigned *>(by_len)[t - 32];
+}
+
+// Four entries of the decode table, length << 8 | symbol; codes nobody has decode as (length 0, value 0).
+__device__ __forceinline__ ushort4 lut_entries(const unsigned *levels, unsigned x) {
+    const unsigned *limit = levels, *start = levels + 16;
+    const uint8_t *by_len = reinterpret_cast<const uint8_t *>(levels + 32);
+    unsigned l = 1;  // (the limits ascend)
 #pragma unroll
-        for (int i = 1; i <= KV_MAX_BITS; ++i) l += x >= limit[i] ? 1 : 0;
-        ushort4 e;
-        uint16_t *ev = reinterpret_cast<uint16_t *>(&e);
-        auto entry = [&](unsigned x, unsigned l) {
-            const unsigned at = l > KV_MAX_BITS ? 0 : offset[l] + (x >> (KV_MAX_BITS - l)) - first_code[l];
-            return l > KV_MAX_BITS ? (uint16_t)128 : (uint16_t)(l << 8 | by_len[at]);
-        };
-        if (l <= KV_MAX_BITS - 2 || l > KV_MAX_BITS) {  // one code for the four, or none
-            ev[0] = ev[1] = ev[2] = ev[3] = entry(x, l);
-        } else {
+    for (int i = 1; i <= KV_MAX_BITS; ++i) l += x >= limit[i] ? 1 : 0;
+    ushort4 e;
+    uint16_t *ev = reinterpret_cast<uint16_t *>(&e);
+    auto entry = [&](unsigned x, unsigned l) { return l > KV_MAX_BITS ? (uint16_t)128 : (uint16_t)(l << 8 | by_len[start[l] + (x >> (KV_MAX_BITS - l))]); };
+    if (l <= KV_MAX_BITS - 2 || l > KV_MAX_BITS) {  // one code for the four, or none
+        ev[0] = ev[1] = ev[2] = ev[3] = entry(x, l);
+    } else {
 #pragma unroll
-            for (unsigned k = 0; k < 4; ++k) {
-                while (l <= KV_MAX_BITS && x + k >= limit[l]) ++l;
-                ev[k] = entry(x + k, l);
-            }
+        for (unsigned k = 0; k < 4; ++k) {
+            while (l <= KV_MAX_BITS && x + k >= limit[l]) ++l;
+            ev[k] = entry(x + k, l);
         }
-        reinterpret_cast<ushort4 *>(b.lut + (size_t)c * KV_LUT)[t] = e;
     }
+    return e;
 }
 
 __host__ __device__ inline unsigned long long kv_stream_bytes(unsigned long long bits) { return (bits + 7) / 8; }
@@ -702,17 +720,17 @@ struct kv_places {
 // p[i] = p[from + i] for i < rest, where rest may be the longer: a thread takes whole chains i, i + from, i + 2 from, .. , so that what it
 // overwrites only it reads, and it has read it before.  (A launch per `from` values moved took 3.2 us each.)
 template <class V> __device__ __forceinline__ void move_to_front(V *p, size_t from, size_t rest, size_t first, size_t step) {
-    constexpr int AHEAD = 4;
-    for (size_t i = first; i < min(from, rest); i += step)
-        for (size_t j = i; j < rest; j += AHEAD * from) {
-            V v[AHEAD];
-#pragma unroll
-            for (int k = 0; k < AHEAD; ++k)
-                if (j + k * from < rest) v[k] = p[j + (k + 1) * from];
-#pragma unroll
-            for (int k = 0; k < AHEAD; ++k)
-                if (j + k * from < rest) p[j + k * from] = v[k];
+    for (size_t i = first; i < min(from, rest); i += step) {
+        size_t j = i;
+        for (; j + 3 * from < rest; j += 4 * from) {
+            const V v0 = p[j + from], v1 = p[j + 2 * from], v2 = p[j + 3 * from], v3 = p[j + 4 * from];
+            p[j] = v0;
+            p[j + from] = v1;
+            p[j + 2 * from] = v2;
+            p[j + 3 * from] = v3;
         }
+        for (; j < rest; j += from) p[j] = p[j + from];
+    }
 }
 
 // Appends the code `e` (length << 16 | code) to a right-aligned window; returns the next whole word if one is full.
@@ -727,10 +745,12 @@ __device__ __forceinline__ bool push_code(unsigned e, unsigned long long &acc, u
     return true;
 }
 
-// HuffmanTable::encode (src/huffman.rs:216-251) in parallel: grid (nwg, chunks).  A workgroup's bit range is
+// HuffmanTable::encode (src/huffman.rs:216-251) in parallel: grid (nwg + 1, chunks).  A workgroup's bit range is
 // known; its threads put their codes together in LDS and the workgroup stores the words that START in its
 // range, whole: the bits that the last of them takes from the next run it encodes itself (up to 31 values), so no word
-// has two writers and nothing is zeroed first.
+// has two writers and nothing is zeroed first.  The last workgroup of a chunk writes its head and the decode table.  What bounds it is
+// latency: with all loads ahead of the first wait and the head beside the runs, 20 chunks of 262144 values take 5.7 us (one
+// after another 6.7).
 // GUESSED: launched before the host knows the sizes.  Unless every stream of the batch fits its room, and the rooms are not much too
 // large, the launch does nothing at all -- no stream is written and the window does not move -- and the host, which decides by
 // the same sizes, takes over.
@@ -740,36 +760,56 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
     __shared__ unsigned words[ENC_PER_WG * KV_MAX_BITS / 32 + 2], follow[32];
     const unsigned c = places.first + blockIdx.y, g = blockIdx.x, t = threadIdx.x, lane = t & 63;
     const kv_layout lay(b.heads, b.total, true);
+    // all that a run needs is requested at once, ahead of the first use of any of it
+    const unsigned cc = min(c, b.count - 1);
+    const unsigned long long stream_bits = b.wg_bit[(size_t)min(lane, b.count - 1) * (b.nwg + 1) + b.nwg];
+    const unsigned long long *wg_bit = b.wg_bit + (size_t)cc * (b.nwg + 1);
+    const unsigned long long first = wg_bit[g], last = wg_bit[min(g + 1, b.nwg)];
+    const unsigned code = b.codes[(size_t)cc * NUM_SYMBOLS + t];
+    const int8_t *q = b.q + (size_t)cc * b.q_stride;
+    const unsigned base = g * ENC_PER_WG + t * ENC_SPT;
+    const unsigned count = base >= b.total ? 0u : min(b.total - base, (unsigned)ENC_SPT);
+    const uint4 v = *reinterpret_cast<const uint4 *>(q + (count ? base : 0));  // (q is padded to a multiple of 16)
+    const unsigned beyond = (g + 1) * ENC_PER_WG + (t & 31);
+    const uint8_t after = (uint8_t)q[min(beyond, b.total - 1)];
     if constexpr (GUESSED) {
-        bool fits = true;
-        unsigned need = 0;
-        for (unsigned i = lane; i < b.count; i += 64) {
-            const unsigned long long bytes = kv_stream_bytes(b.wg_bit[(size_t)i * (b.nwg + 1) + b.nwg]);
-            fits = fits && bytes <= places.room[i % b.sides];
-            need += (unsigned)(lay.size(bytes) / 256);
+        const bool second = b.sides == 2 && (lane & 1);  // (of the sides, also 64 chunks on)
+        const unsigned long long room0 = places.room[0], room1 = places.room[1], room = second ? room1 : room0;
+        const unsigned long long bytes = kv_stream_bytes(stream_bits);
+        bool fits = lane >= b.count || bytes <= room;
+        unsigned need = lane >= b.count ? 0u : (unsigned)(lay.size(bytes) / 256);
+        for (unsigned i = lane + 64; i < b.count; i += 64) {
+            const unsigned long long more = kv_stream_bytes(b.wg_bit[(size_t)i * (b.nwg + 1) + b.nwg]);
+            fits = fits && more <= room;
+            need += (unsigned)(lay.size(more) / 256);
         }
         if (__ballot(!fits) || (unsigned)pg_wave_sum_i32((int)need) < places.least) return;  // (the same for all workgroups)
     }
     if (c >= b.count) {
         const unsigned row = c - b.count;
-        float *p = places.hot[row / b.heads] + (size_t)(row % b.heads) * places.hot_stride;
+        float *p = (row < b.heads ? places.hot[0] : places.hot[1]) + (size_t)(row % b.heads) * places.hot_stride;
         if (places.vec) move_to_front(reinterpret_cast<float4 *>(p), places.from / 4, places.rest / 4, (size_t)g * KV_WG + t, (size_t)gridDim.x * KV_WG);
         else move_to_front(p, places.from, places.rest, (size_t)g * KV_WG + t, (size_t)gridDim.x * KV_WG);
         return;
     }
     char *dst = places.at[blockIdx.y];
-    const unsigned long long *wg_bit = b.wg_bit + (size_t)c * (b.nwg + 1);
-    const unsigned long long first = wg_bit[g], last = wg_bit[g + 1], end = wg_bit[b.nwg];
-    lc[t] = b.codes[(size_t)c * NUM_SYMBOLS + t];
+    if (g == b.nwg) {  // the chunk's head, with the decode table
+        if (t < KV_LEVELS) words[t] = b.levels[(size_t)c * KV_LEVELS + t];
+        for (unsigned h = t; h < b.heads; h += KV_WG) reinterpret_cast<float *>(dst)[h] = b.scales[(size_t)c * b.heads + h];
+        dst[lay.o_book + t] = (char)(code >> 16);
+        if (t == 0) {
+            reinterpret_cast<unsigned long long *>(dst + lay.o_wg)[b.nwg] = first;
+            if (table) table[c] = dst;
+        }
+        if (t < 4) reinterpret_cast<unsigned *>(dst + lay.o_bits)[(size_t)((first + 31) >> 5) + t] = 0;  // the padding
+        __syncthreads();
+        for (unsigned i = t; i < KV_LUT / 4; i += KV_WG) reinterpret_cast<ushort4 *>(dst + lay.o_lut)[i] = lut_entries(words, 4 * i);
+        return;
+    }
+    lc[t] = code;
     for (unsigned i = t; i < sizeof(words) / 4; i += KV_WG) words[i] = 0;
-    const int8_t *q = b.q + (size_t)c * b.q_stride;
-    const unsigned base = g * ENC_PER_WG + t * ENC_SPT;
-    const unsigned count = base >= b.total ? 0u : min(b.total - base, (unsigned)ENC_SPT);
-    uint4 v = {0, 0, 0, 0};
-    if (count) v = *reinterpret_cast<const uint4 *>(q + base);  // (q is padded to a multiple of 16)
     // the values that may fill this run's last word up: 31 bits, a value takes at least one
-    const unsigned beyond = (g + 1) * ENC_PER_WG + t;
-    if (t < 32) follow[t] = beyond < b.total ? (uint8_t)q[beyond] ^ 128u : NUM_SYMBOLS;
+    if (t < 32) follow[t] = beyond < b.total ? after ^ 128u : NUM_SYMBOLS;
     __syncthreads();
     const unsigned sw[4] = {v.x, v.y, v.z, v.w};
     unsigned e[ENC_SPT], bits = 0;
@@ -807,17 +847,6 @@ __global__ __launch_bounds__(KV_WG) void kv_encode_kernel(const kv_batch b, cons
     const unsigned nwords = (unsigned)(((last + 31) >> 5) - (first >> 5));
     for (unsigned i = t + (r ? 1 : 0); i < nwords; i += KV_WG) out[i] = __builtin_bswap32(words[i]);
     if (t == 0) reinterpret_cast<unsigned long long *>(dst + lay.o_wg)[g] = first;
-    if (g == 0) {  // the chunk's head
-        for (unsigned h = t; h < b.heads; h += KV_WG) reinterpret_cast<float *>(dst)[h] = b.scales[(size_t)c * b.heads + h];
-        dst[lay.o_book + t] = (char)(lc[t] >> 16);
-        const uint4 *lut = reinterpret_cast<const uint4 *>(b.lut + (size_t)c * KV_LUT);
-        for (unsigned i = t; i < KV_LUT * 2 / 16; i += KV_WG) reinterpret_cast<uint4 *>(dst + lay.o_lut)[i] = lut[i];
-        if (t == 0) {
-            reinterpret_cast<unsigned long long *>(dst + lay.o_wg)[b.nwg] = end;
-            if (table) table[c] = dst;
-        }
-        if (t < 4) reinterpret_cast<unsigned *>(dst + lay.o_bits)[(size_t)((end + 31) >> 5) + t] = 0;  // the padding
-    }
 }
 
 // Chunks with an index, decoded, scaled and laid out, and the window copied behind them.  Chunk c (address table[c], or
@@ -872,6 +901,12 @@ __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a
     const unsigned long long w0 = wg_bit[r0] >> 5, w1 = (wg_bit[r1] + 31) >> 5;
     const unsigned *stream = reinterpret_cast<const unsigned *>(chunk + lay.o_bits) + w0;
     const unsigned nwords = min((unsigned)(w1 - w0) + 3, MAX_WORDS);  // (up to 16 bytes of padding follow a stream)
+    const float *scales = reinterpret_cast<const float *>(chunk);
+    const unsigned h0 = g * DEC_PER_WG / a.head_elems;
+    const float scale_t = scales[min(h0 + (t & (DEC_SCALES - 1)), a.heads - 1)];
+    const unsigned base = g * DEC_PER_WG, sub = g * KV_WG + t;
+    const unsigned count = base + t * SUB_SYMS >= a.total ? 0u : min(a.total - (base + t * SUB_SYMS), (unsigned)SUB_SYMS), from = count ? sub : 0;
+    const unsigned pos = (unsigned)(wg_bit[from / (ENC_PER_WG / SUB_SYMS)] - (w0 << 5)) + reinterpret_cast<const uint16_t *>(chunk + lay.o_sub)[from];
     for (unsigned at = 0; at < nwords; at += 8 * KV_WG) {  // eight loads in flight
         unsigned w[8];
 #pragma unroll
@@ -882,14 +917,7 @@ __global__ __launch_bounds__(KV_WG) void kv_decode_kernel(const kv_decode_args a
     }
 #pragma unroll
     for (unsigned i = 0; i < KV_LUT * 2 / 16 / KV_WG; ++i) reinterpret_cast<uint4 *>(lut)[i * KV_WG + t] = lut_v[i];
-    const float *scales = reinterpret_cast<const float *>(chunk);
-    const unsigned h0 = g * DEC_PER_WG / a.head_elems;
-    if (t < DEC_SCALES) sc[t] = h0 + t < a.heads ? scales[h0 + t] : 0.0f;
-    const unsigned base = g * DEC_PER_WG, sub = g * KV_WG + t;
-    const unsigned count = base + t * SUB_SYMS >= a.total ? 0u : min(a.total - (base + t * SUB_SYMS), (unsigned)SUB_SYMS);
-    unsigned pos = 0;
-    if (count)
-        pos = (unsigned)(wg_bit[sub / (ENC_PER_WG / SUB_SYMS)] - (w0 << 5)) + reinterpret_cast<const uint16_t *>(chunk + lay.o_sub)[sub];
+    if (t < DEC_SCALES) sc[t] = scale_t;
     __syncthreads();
     if (count) {
         unsigned k = pos >> 5;
@@ -1112,10 +1140,9 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         auto take = [&](size_t bytes) { const size_t at = off; off += pg_round_up(bytes, 256); return at; };
         const size_t o_amax = take(n * num_heads * b.splits * 4), o_scales = take(n * num_heads * 4), o_q = take(n * b.q_stride);
         const size_t o_hist = take(n * nwg * NUM_SYMBOLS * 2), o_bit = take(n * (nwg + 1) * 8), o_codes = take(n * NUM_SYMBOLS * 4);
-        const size_t o_lut = take(n * KV_LUT * 2);
+        const size_t o_levels = take(n * KV_LEVELS * 4);
         void *ws = nullptr, *pin = nullptr;
         PG_TRY(pg_workspace(ctx, off, &ws));
-        PG_TRY(pg_pinned(ctx, n * sizeof(uint64_t), &pin));
         char *base = static_cast<char *>(ws);
         b.amax = reinterpret_cast<float *>(base + o_amax);
         b.scales = reinterpret_cast<float *>(base + o_scales);
@@ -1123,17 +1150,7 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
         b.hist = reinterpret_cast<uint16_t *>(base + o_hist);
         b.wg_bit = reinterpret_cast<unsigned long long *>(base + o_bit);
         b.codes = reinterpret_cast<unsigned *>(base + o_codes);
-        b.lut = reinterpret_cast<uint16_t *>(base + o_lut);
-        std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made(n);
-        for (auto &ch : made) {
-            ch.reset(new (std::nothrow) pg_huffman_kv_chunk());
-            if (!ch) return pg_fail(PG_ENOMEM, "host allocation failed");
-        }
-        auto block = std::make_shared<pg_dev_block>();
-        std::vector<char *> at(n);
-        bool moves = false;  // the encoder's launch moves the window
-        uint64_t *sizes = static_cast<uint64_t *>(pin);
-        std::fill(sizes, sizes + n, (uint64_t)0);
+        b.levels = reinterpret_cast<unsigned *>(base + o_levels);
         kv_incoming in = {{b.data[0], b.data[1]}, {nullptr, nullptr}, 0, 0, ~(size_t)0, 0, 0};
         bool vec_in = vec;
         if (rows && first == 0) {
@@ -1152,6 +1169,18 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
             PG_TRY(pg_launch(ctx, "huffman_kv_quant", kv_quant_hist_kernel, dim3(b.nwg, b.count), dim3(KV_WG), 0, b, (int)vec));
         }
         if (rows) rows->written = true;
+        // (while the device is at it)
+        PG_TRY(pg_pinned(ctx, n * sizeof(uint64_t), &pin));
+        std::vector<std::unique_ptr<pg_huffman_kv_chunk>> made(n);
+        for (auto &ch : made) {
+            ch.reset(new (std::nothrow) pg_huffman_kv_chunk());
+            if (!ch) return pg_fail(PG_ENOMEM, "host allocation failed");
+        }
+        auto block = std::make_shared<pg_dev_block>();
+        std::vector<char *> at(n);
+        bool moves = false;  // the encoder's launch moves the window
+        uint64_t *sizes = static_cast<uint64_t *>(pin);
+        std::fill(sizes, sizes + n, (uint64_t)0);
         PG_TRY(pg_launch(ctx, "huffman_kv_table", b.total < (1u << 23) ? kv_table_kernel<unsigned> : kv_table_kernel<unsigned long long>, dim3(b.count), dim3(1024), 0, b, (unsigned long long *)sizes));
         const kv_layout lay(num_heads, total, true);
         // the encoder and the window's move: chunk c has room for bytes_of(c) of stream
@@ -1186,7 +1215,7 @@ static pg_status compress_batch(pg_ctx *ctx, const float *const *data, size_t si
                     rows = sides * num_heads;
                     moves = true;
                 }
-                PG_TRY(pg_launch(ctx, "huffman_kv_encode", guess ? kv_encode_kernel<true> : kv_encode_kernel<false>, dim3(b.nwg, (unsigned)(here + rows)),
+                PG_TRY(pg_launch(ctx, "huffman_kv_encode", guess ? kv_encode_kernel<true> : kv_encode_kernel<false>, dim3(b.nwg + 1, (unsigned)(here + rows)),
                                  dim3(KV_WG), 0, b, places, table_dev ? table_dev + first : nullptr));
             }
             return PG_OK;
