@@ -72,6 +72,39 @@ struct gemm_wgroup {
     long long comb_plane;  // (NP planes of activations: bytes from one of those to the next)
 };
 
+// The order of a launch's tiles: strips of `strip` row tiles, a strip's tiles by column panel, its row tiles fastest.  Each XCD takes a run of
+// consecutive ones and works on as many at a time as its CUs hold; the nearer those are to a square, the fewer rows of A and B they
+// fetch between them (strip_for).  With all row tiles fastest (one strip), tall products brought most of A into each of the eight L2s
+// for a few column panels.  us, one strip : strips: 4541 x 403 -> 14373 129 : 99, 2848 x 628 -> 17709 105 : 82, 5882 x 207 -> 1607 28.7 : 23.5,
+// 2048 x 14336 -> 4096 109 : 107; 250 drawn products of 200 to 6000 rows 0.966 of the time, 60 drawn layers 0.994.
+// Divisions by the launch's numbers: the high half of a product with (2^32 - 1) / d, rounded down, is the quotient or one less.  (Divisions proper
+// are 25 vector instructions each ahead of a tile's first load: 0.3 us for three.)
+struct tile_order {
+    int ntiles, chunk, strip, strips, per, last;  // chunk: tiles of an XCD; per: tiles of a whole strip; last: row tiles of the last
+    unsigned by_per, by_strip, by_last;
+    tile_order(int tiles_m, int panels, int strip_) : ntiles(tiles_m * panels), chunk((ntiles + 7) / 8), strip(strip_), strips(1), per(ntiles), last(tiles_m), by_per(0), by_strip(0) {
+        if (strip < tiles_m) {
+            strips = (tiles_m + strip - 1) / strip;
+            per = strip * panels;
+            last = tiles_m - (strips - 1) * strip;
+            by_per = ~0u / (unsigned)per;
+            by_strip = ~0u / (unsigned)strip;
+        }
+        by_last = ~0u / (unsigned)last;
+    }
+    __device__ static int over(int t, int d, unsigned by) {
+        const int q = (int)__umulhi((unsigned)t, by);
+        return q + (t - q * d >= d ? 1 : 0);
+    }
+    __device__ __forceinline__ void place(int t, int &mt, int &np) const {
+        const int s = over(t, per, by_per), r = t - s * per;
+        const bool end = s == strips - 1;
+        const int height = end ? last : strip;
+        np = over(r, height, end ? by_last : by_strip);
+        mt = s * strip + r - np * height;
+    }
+};
+
 // NP = 3: the W8A32 product in one launch.  The activations are three digit planes (weights 1, 256, 65536); a stage holds
 // BM rows of each, every weight fragment meets all three, and the epilogue joins the three accumulators as COMB does.
 // One pass over the weights and no accumulator planes in memory: for tiles up to 128x128, where 3 x TM x TN
@@ -81,9 +114,9 @@ struct gemm_wgroup {
 // wall-clock ticks its K loop took, clk[2 * blockIdx.x] and clk[2 * blockIdx.x + 1].
 template <int BM, int BN, int BK, int NST, int NWM, int NWN, int OCC, bool CLK = false, bool COMB = false, int NP = 1>
 __global__ __launch_bounds__(64 * NWM * NWN) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
-void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup grp, int ldb,
+void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const tile_order order, const gemm_wgroup grp, int ldb,
                       const float *__restrict__ a_scales, int32_t *__restrict__ acc_out, int M, int K,
-                      int tiles_m, int ntiles, int kt_per_split, long long *__restrict__ clk) {
+                      int kt_per_split, long long *__restrict__ clk) {
     constexpr int NW = NWM * NWN;
     constexpr int WM = BM / NWM, WN = BN / NWN;      // wavefront tile
     constexpr int TM = WM / 16, TN = WN / 16;        // 16x16 MFMA tiles per wavefront
@@ -98,11 +131,11 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 
     // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a contiguous
-    // run of tiles (m fastest) so the tiles sharing an L2 also share A/B panels.
-    const int chunk = (ntiles + 7) / 8;
-    const int t = (blockIdx.x % 8) * chunk + blockIdx.x / 8;
-    if (t >= ntiles) return;
-    const int np = t / tiles_m;  // n-panel of the launch; which weight owns it (uniform: scalar code)
+    // run of tiles (tile_order) so the tiles sharing an L2 also share A/B panels.
+    const int t = (int)(blockIdx.x % 8) * order.chunk + (int)(blockIdx.x / 8);
+    if (t >= order.ntiles) return;
+    int np, mt;  // np: n-panel of the launch; which weight owns it (uniform: scalar code)
+    order.place(t, mt, np);
     int g = 0;
 #pragma unroll
     for (int i = 1; i < PG_GEMM_MAX_GROUP; ++i) g = np >= grp.panel0[i] ? i : g;
@@ -110,7 +143,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     const float *__restrict__ w_scales = grp.ws[g];
     float *__restrict__ out = grp.out[g];
     const int N = grp.n[g];
-    const int m0 = (t % tiles_m) * BM, n0 = (np - grp.panel0[g]) * BN;
+    const int m0 = mt * BM, n0 = (np - grp.panel0[g]) * BN;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -349,6 +382,23 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const gemm_wgroup g
     }
 }
 
+// Row tiles of a strip: the fewest rows of A and B that the `window` consecutive tiles of an XCD fetch (one strip unless that is 1 / 16 more).
+int strip_for(int tiles_m, int window, int a_rows, int b_rows) {
+    auto rows = [&](int h) { return std::min(h, window) * a_rows + (window + h - 1) / h * b_rows; };
+    int best = tiles_m, least = rows(tiles_m);
+    // (no strips fetch less than the square would; a small product waits for this)
+    if ((double)least * least <= 4.6 * (double)window * (double)a_rows * (double)b_rows) return best;
+    least -= least / 16;
+    for (int strips = 2; strips <= tiles_m && strips <= 64; ++strips) {
+        const int h = (tiles_m + strips - 1) / strips;
+        if (rows(h) < least) {
+            best = h;
+            least = rows(h);
+        }
+    }
+    return best;
+}
+
 template <int BM, int BN, int BK, int NST, int NWM, int NWN, int OCC, bool COMB = false, int NP = 1>
 pg_status launch_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                        const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc,
@@ -367,18 +417,19 @@ pg_status launch_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const f
     }
     grp.comb = comb;
     grp.comb_plane = (long long)(NP > 1 ? a_plane : comb_plane);
-    const int ntiles = tiles_m * panels;
+    const int ntiles = tiles_m * panels, window = std::min((ntiles + 7) / 8, std::max(1, ctx->num_cu / 8 * (4 * OCC / (NWM * NWN))));
+    const tile_order order(tiles_m, panels, strip_for(tiles_m, window, NP * BM, BN));
     const size_t lds = (size_t)NST * (NP * BM + BN) * BK + (BM + BN) * sizeof(float);
     auto kern = gemm_w8a8_kernel<BM, BN, BK, NST, NWM, NWN, OCC, false, COMB, NP>;
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
-    const unsigned grid = (unsigned)(((ntiles + 7) / 8) * 8);
+    const unsigned grid = (unsigned)(order.chunk * 8);
     const size_t k_pad = w[0]->k_pad;
     if (splits == 1) kt_per_split = (int)(k_pad / BK);
     ctx->gemm_last_bm = BM;
     ctx->gemm_last_bn = BN;
     ctx->gemm_last_splits = splits;
-    PG_TRY(pg_launch(ctx, NP == 3 ? "gemm_w8a32" : "gemm_w8a8", kern, dim3(grid, (unsigned)splits), dim3(64 * NWM * NWN), lds, a_i8, (int)a_stride, grp,
-                     (int)k_pad, a_scales, acc, (int)m, (int)k_pad, tiles_m, ntiles, kt_per_split, (long long *)nullptr));
+    PG_TRY(pg_launch(ctx, NP == 3 ? "gemm_w8a32" : "gemm_w8a8", kern, dim3(grid, (unsigned)splits), dim3(64 * NWM * NWN), lds, a_i8, (int)a_stride, order, grp,
+                     (int)k_pad, a_scales, acc, (int)m, (int)k_pad, kt_per_split, (long long *)nullptr));
     return pg_launch_check("gemm_w8a8");
 }
 
@@ -1282,8 +1333,8 @@ PG_API pg_status pg_probe_gemm_clock(pg_ctx *ctx, size_t m, size_t k, size_t n, 
     auto kern = gemm_w8a8_kernel<BM, BN, BK, NST, 2, 4, 2, true>;
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));
     for (int rep = 0; rep < 20; ++rep)  // the clock settles over the first launches; the last one is read
-        PG_TRY(pg_launch(ctx, "gemm_w8a8_clock_probe", kern, dim3(grid), dim3(512), lds, a.as<int8_t>(), (int)k, grp, (int)k, sc.as<float>(),
-                         (int32_t *)nullptr, (int)m, (int)k, tiles_m, ntiles, (int)(k / BK), clk.as<long long>()));
+        PG_TRY(pg_launch(ctx, "gemm_w8a8_clock_probe", kern, dim3(grid), dim3(512), lds, a.as<int8_t>(), (int)k, tile_order(tiles_m, (int)(n / BN), tiles_m), grp, (int)k, sc.as<float>(),
+                         (int32_t *)nullptr, (int)m, (int)k, (int)(k / BK), clk.as<long long>()));
     PG_HIP(hipStreamSynchronize(ctx->stream));
     std::vector<long long> h((size_t)grid * 2);
     PG_HIP(hipMemcpy(h.data(), clk.p, h.size() * sizeof(long long), hipMemcpyDeviceToHost));

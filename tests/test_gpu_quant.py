@@ -466,6 +466,32 @@ def test_int8_tiles_store_whole_and_cut_tiles(ctx, orc, semantics, m, k, n):
     qt.free_gpu()
 
 
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7, 8, "w8a32"])
+@pytest.mark.parametrize("m,n", [(4300, 2690), (1030, 5000)])
+def test_int8_tiles_in_strips(ctx, tile, m, n):
+    """Every tile shape over more row tiles than a strip holds, the last strip shorter: each tile is made once, where it belongs.  Small
+    integers: every result is exact."""
+    from peregrine_amd import quant, _ffi
+    say(f"int8 tiles in strips {tile} m={m} n={n}")
+    k = 70
+    rng = np.random.default_rng(m)
+    a = rng.integers(-127, 128, (m, k)).astype(np.float32)
+    a[:, 0] = 127.0                                        # so that W8A8's row scale is 1
+    qi = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    qt = quant.QuantizedTensor(qi.reshape(-1), np.ascontiguousarray(qi.T).reshape(-1), np.ones(n, np.float32), k, n).to_gpu(ctx)
+    da, dout = DevBuf(ctx, host=a), DevBuf(ctx, m * n * 4)
+    if tile == "w8a32":
+        _ffi.check(_ffi.lib.pg_matmul_dequant_i8_dev(ctx.handle, da.ptr, m, k, qt._gpu, dout.ptr))
+    else:
+        _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, tile))
+        try:
+            _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, da.ptr, m, k, qt._gpu, dout.ptr, None))
+        finally:
+            _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, 0))
+    assert (dout.to_host(np.float32).reshape(m, n) == a @ qi.astype(np.float32)).all()   # |sums| < 2^24: exact in any order
+    qt.free_gpu()
+
+
 def run_multi(ctx, da, m, k, qts, douts):
     from peregrine_amd import _ffi
     wtab = (C.c_void_p * len(qts))(*[q._gpu.value for q in qts])
