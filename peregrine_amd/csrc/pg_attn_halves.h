@@ -119,7 +119,7 @@ __device__ __forceinline__ int halves_tiles(const attn_args &aa, int blk, int nr
 }
 template <int HD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void gqa_attention_halves_kernel(attn_args aa, const char *__restrict__ planes, int n_blocks, int nkvh, int tiles_all) {
+void gqa_attention_halves_kernel(const char *__restrict__ planes, int n_blocks, attn_args aa, int nkvh, int tiles_all) {
     constexpr int NDT = HD / 32, NQ = HD / 16, PLANE = HD * 64, UB = half_unit_bytes<HD>(), LPU = UB / 4096, NS = HALVES_RING;
     extern __shared__ __attribute__((aligned(1024))) char half_lds[];  // [NS][UB]; afterwards the wavefronts' tiles of 32 rows x 64 + 4 values
     __shared__ float2 inv[HALVES_CHUNK_MAX];  // the tiles' inverse scales

@@ -149,7 +149,7 @@ struct gemv_wgroup {
 // workgroups).
 template <int NCH, int RPW, int NW>
 __global__ __launch_bounds__(64 * NW) void gemv_w8a8_m1_f32x_kernel(
-    const gemv_wgroup grp, int k_pad, const float *__restrict__ x_f32, int k, int32_t *__restrict__ acc_out) {
+    const float *__restrict__ x_f32, int k, const gemv_wgroup grp, int k_pad, int32_t *__restrict__ acc_out) {
     constexpr int NT = 64 * NW, NV = (NCH * 256 + NT - 1) / NT;  // float4 of the row per thread
     __shared__ int xq[NCH * 256];  // the quantised row, zero beyond k: NCH KiB >= k_pad bytes
     __shared__ float red[NW];
@@ -244,8 +244,8 @@ pg_status launch_m1_f32x(pg_ctx *ctx, const float *x_f32, size_t k, const pg_qte
         grp.wg0[i] = used ? wgs : INT_MAX;
         if (used) wgs += (int)(w[i]->n_pad / (NW * RPW));  // n_pad is a multiple of 256
     }
-    PG_TRY(pg_launch(ctx, "gemv_w8a8", gemv_w8a8_m1_f32x_kernel<NCH, RPW, NW>, dim3((unsigned)wgs), dim3(64 * NW), 0, grp,
-                     (int)w[0]->k_pad, x_f32, (int)k, acc));
+    PG_TRY(pg_launch(ctx, "gemv_w8a8", gemv_w8a8_m1_f32x_kernel<NCH, RPW, NW>, dim3((unsigned)wgs), dim3(64 * NW), 0, x_f32, (int)k, grp,
+                     (int)w[0]->k_pad, acc));
     return pg_launch_check("gemv_w8a8_m1_f32x");
 }
 

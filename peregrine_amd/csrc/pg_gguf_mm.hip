@@ -683,8 +683,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // Up to three tensors of equal K in one launch (q|k|v, gate|up of models::llama): tensor g owns the workgroups
 // wg0[g] .. wg0[g + 1] - 1 (unused slots hold INT_MAX).
 template <int QT, int NB, int MT, int NW, int NST>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_skinny_kernel(const pg_skinny_group grp, int nb, int nbp, int m,
-                                                                    const int8_t *__restrict__ digits, const float *__restrict__ xs) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_skinny_kernel(const int8_t *__restrict__ digits, const float *__restrict__ xs,
+                                                                    const pg_skinny_group grp, int nb, int nbp, int m) {
     int tg = 0;
 #pragma unroll
     for (int i = 1; i < 3; ++i) tg = (int)blockIdx.x >= grp.wg0[i] ? i : tg;
@@ -914,8 +914,8 @@ template <int QT, int MT, bool Q41> struct KTCfg {
     static constexpr int OFF_X = OFF_DG + MT * 256, OFF_S = OFF_X + MT * 16, UNIT = OFF_S + (Q41 ? MT * 16 : 0);
 };
 template <int QT, int MT, int NW, bool Q41, typename ARGS = ktile_args<Q41>, bool UPLOADED = false>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_ktile_kernel(const ARGS grp, int nb, int nbp, int m,
-                                                                const int8_t *__restrict__ digits, const float *__restrict__ xs, int groups, int wgs) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 4))) void gguf_ktile_kernel(const int8_t *__restrict__ digits, const float *__restrict__ xs, const ARGS grp,
+                                                                int nb, int nbp, int m, int groups, int wgs) {
     using C = KTCfg<QT, MT, Q41>;
     static_assert(!Q41 || QT == 4, "Q4_1 is the Q4_0 product and its offsets");
     constexpr bool EXPERTS = std::is_same_v<ARGS, ktile_experts>;
@@ -1305,7 +1305,7 @@ static pg_status launch_skinny(pg_ctx *ctx, size_t k_in, bool q8, const pg_skinn
         const size_t lds = (size_t)NWW * 2 * (NBB * ((QTT == 8 ? 4096 : 2048) + 256) + MTT * 512 + 512);                       \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
         return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_few_rows_mm" : "gguf_q4_0_few_rows_mm", kern, dim3((unsigned)wgs), dim3(64 * NWW), lds, \
-                         grp, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs);                               \
+                         (const int8_t *)md.digits, (const float *)md.xs, grp, nb, nbp, (int)m);                               \
     }
 #define PG_GSK_NW(QTT, NBB, MTT) PG_GSK(QTT, NBB, MTT, 8) PG_GSK(QTT, NBB, MTT, 4) PG_GSK(QTT, NBB, MTT, 2) PG_GSK(QTT, NBB, MTT, 1)
     PG_GSK_NW(8, 1, 4) PG_GSK_NW(8, 2, 4) PG_GSK_NW(8, 1, 8) PG_GSK_NW(8, 2, 8)
@@ -1357,7 +1357,7 @@ static pg_status launch_ktile(pg_ctx *ctx, int ggml_type, size_t k_in, const pg_
         const size_t lds = (size_t)NWW * 2 * KTCfg<QTT == 8 ? 8 : 4, MTT, QTT == 5>::UNIT;                                     \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
         return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_rows_tile" : QTT == 5 ? "gguf_q4_1_rows_tile" : "gguf_q4_0_rows_tile", kern, grid, \
-                         dim3(64 * NWW), lds, args, nb, nbp, (int)m, (const int8_t *)md.digits, (const float *)md.xs, groups, wgs1); \
+                         dim3(64 * NWW), lds, (const int8_t *)md.digits, (const float *)md.xs, args, nb, nbp, (int)m, groups, wgs1); \
     }
 #define PG_KTS(QTT) PG_KT(QTT, 32, 2) PG_KT(QTT, 32, 3) PG_KT(QTT, 32, 6) PG_KT(QTT, 16, 4) PG_KT(QTT, 16, 8) PG_KT(QTT, 8, 4) PG_KT(QTT, 8, 8)
     PG_KTS(8) PG_KTS(4) PG_KTS(5)
@@ -1426,8 +1426,8 @@ pg_status pg_launch_gguf_experts_tiles(pg_ctx *ctx, int ggml_type, size_t n_out,
         auto kern = gguf_ktile_kernel<QTT, MTT, NWW, false, ktile_experts>;                                                    \
         const size_t lds = (size_t)NWW * 2 * KTCfg<QTT, MTT, false>::UNIT;                                                     \
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds));                                                            \
-        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_experts_tile" : "gguf_q4_0_experts_tile", kern, grid, dim3(64 * NWW), lds, ex, nb, nbp, 0, \
-                         (const int8_t *)md.digits, (const float *)md.xs, 1, 0);                                               \
+        return pg_launch(ctx, QTT == 8 ? "gguf_q8_0_experts_tile" : "gguf_q4_0_experts_tile", kern, grid, dim3(64 * NWW), lds, \
+                         (const int8_t *)md.digits, (const float *)md.xs, ex, nb, nbp, 0, 1, 0);                               \
     }
 #define PG_KES(QTT) PG_KE(QTT, 8, 4) PG_KE(QTT, 16, 4)
     PG_KES(8) PG_KES(4)

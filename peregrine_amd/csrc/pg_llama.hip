@@ -235,7 +235,7 @@ __global__ __launch_bounds__(128) void rope_kernel(rope_args ra) {
 // The same for head sizes that are multiples of 8 with every pointer and stride a multiple of four floats: a
 // thread takes dims 4j .. 4j+3 and their partners half + 4j .. as 128-bit loads and stores, 256 / (hd / 8)
 // heads of one token to a workgroup (the operations per element are those of rope_kernel, in its order).
-__global__ __launch_bounds__(256) void rope_v4_kernel(rope_args ra, int total_heads) {
+__global__ __launch_bounds__(256) void rope_v4_kernel(int total_heads, rope_args ra) {
     const int t = blockIdx.x, per = ra.hd >> 3;
     const int idx = blockIdx.y * 256 + threadIdx.x;
     int h = idx / per, s = 0;
@@ -723,7 +723,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 // HD + 4 floats, or an empty record where its rows see none of the run's keys.
 template <int HD, bool SPLIT = false>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void gqa_attention_mfma_kernel(attn_args aa, int n_items, int nkvh) {
+void gqa_attention_mfma_kernel(int n_items, int nkvh, attn_args aa) {
     constexpr int NDT = HD / 32, QR = HD / 2;
     typedef float vdt __attribute__((ext_vector_type(NDT)));
     __shared__ float part_l[SPLIT ? 1 : (NDT * 16 + 2) * 64];
@@ -1025,7 +1025,7 @@ __device__ __forceinline__ float lanes_sum_f32(float v) {  // over aligned group
 __device__ __forceinline__ float exp_neg(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
 template <int HD, int U>
-__global__ __launch_bounds__(256) void gqa_decode_kernel(attn_args aa, int nkv, int tps) {
+__global__ __launch_bounds__(256) void gqa_decode_kernel(int nkv, int tps, attn_args aa) {
     constexpr int LPK = HD / 8, KPW = 64 / LPK, ROWS = 4 * KPW, GC = ATT_DEC_GC, HALF = HD / 2, TK = U * ROWS;
     __shared__ __attribute__((aligned(16))) float xch[GC][ROWS][HD];  // 32 KB: each key row's partial output rows
     __shared__ float wm[GC][ROWS], wl[GC][ROWS];
@@ -1697,8 +1697,8 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         if (kc->num_kv_heads * splits >= (1ull << 31)) return pg_fail(PG_EUNSUPPORTED, "gqa_attention: grid too large");
         auto *kern = hd == 64 ? (dec_u == 4 ? gqa_decode_kernel<64, 4> : (dec_u == 2 ? gqa_decode_kernel<64, 2> : gqa_decode_kernel<64, 1>))
                               : (dec_u == 4 ? gqa_decode_kernel<128, 4> : (dec_u == 2 ? gqa_decode_kernel<128, 2> : gqa_decode_kernel<128, 1>));
-        PG_TRY(pg_launch(ctx, "gqa_decode", kern, dim3((unsigned)(kc->num_kv_heads * splits)), dim3(256), 0, aa, (int)kc->num_kv_heads,
-                         dec_tps));
+        PG_TRY(pg_launch(ctx, "gqa_decode", kern, dim3((unsigned)(kc->num_kv_heads * splits)), dim3(256), 0, (int)kc->num_kv_heads,
+                         dec_tps, aa));
     } else if (short_kernel) {
         const size_t sets = kc->num_kv_heads * splits, members = (nqh / kc->num_kv_heads) * seq_q;
         const size_t wgs = (sets + 7) / 8 * 8 * members;
@@ -1716,8 +1716,8 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         auto *kern = hd == 64 ? gqa_attention_halves_kernel<64> : gqa_attention_halves_kernel<128>;
         const size_t lds_bytes = halves_lds_bytes(hd == 64 ? half_unit_bytes<64>() : half_unit_bytes<128>());
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds_bytes));
-        PG_TRY(pg_launch(ctx, "gqa_attention_halves", kern, dim3((unsigned)(lp.blocks * nkv * lp.runs)), dim3(256), lds_bytes, aa, (const char *)halves_planes,
-                         (int)lp.blocks, (int)nkv, (int)lp.tiles));
+        PG_TRY(pg_launch(ctx, "gqa_attention_halves", kern, dim3((unsigned)(lp.blocks * nkv * lp.runs)), dim3(256), lds_bytes, (const char *)halves_planes,
+                         (int)lp.blocks, aa, (int)nkv, (int)lp.tiles));
         if (lp.runs > 1)
             PG_TRY(pg_launch(ctx, "gqa_attention_halves_combine", hd == 64 ? attn_halves_combine_kernel<64> : attn_halves_combine_kernel<128>,
                              dim3((unsigned)((rows * (hd / 4) + 255) / 256)), dim3(256), 0, aa));
@@ -1729,11 +1729,11 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         auto *kern = split_kernel ? (hd == 64 ? gqa_attention_mfma_kernel<64, true> : gqa_attention_mfma_kernel<128, true>)
                                   : (hd == 64 ? gqa_attention_mfma_kernel<64> : gqa_attention_mfma_kernel<128>);
         if (split_kernel)  // one wavefront per workgroup: (kv head, item, run)
-            PG_TRY(pg_launch(ctx, "gqa_attention_mfma_split", kern, dim3((unsigned)(n_items * kc->num_kv_heads * splits)), dim3(64), 0, aa,
-                             (int)n_items, (int)kc->num_kv_heads));
+            PG_TRY(pg_launch(ctx, "gqa_attention_mfma_split", kern, dim3((unsigned)(n_items * kc->num_kv_heads * splits)), dim3(64), 0,
+                             (int)n_items, (int)kc->num_kv_heads, aa));
         else
-            PG_TRY(pg_launch(ctx, "gqa_attention_mfma", kern, dim3((unsigned)(pairs * kc->num_kv_heads)), dim3(128), 0, aa, (int)n_items,
-                             (int)kc->num_kv_heads));
+            PG_TRY(pg_launch(ctx, "gqa_attention_mfma", kern, dim3((unsigned)(pairs * kc->num_kv_heads)), dim3(128), 0, (int)n_items,
+                             (int)kc->num_kv_heads, aa));
     } else if (tiled_kernel) {
         const size_t G = nqh / kc->num_kv_heads, row_sets = (G * seq_q + ATT_T_ROWS - 1) / ATT_T_ROWS;
         const dim3 grid_t((unsigned)row_sets, (unsigned)kc->num_kv_heads);
@@ -1854,7 +1854,7 @@ pg_status launch_rope(pg_ctx *ctx, const rope_args &ra, size_t seq, size_t heads
     }
     if (vec) {
         const size_t threads = heads * (size_t)(ra.hd / 8);
-        return pg_launch(ctx, "rope", rope_v4_kernel, dim3((unsigned)seq, (unsigned)((threads + 255) / 256)), dim3(256), 0, ra, (int)heads);
+        return pg_launch(ctx, "rope", rope_v4_kernel, dim3((unsigned)seq, (unsigned)((threads + 255) / 256)), dim3(256), 0, (int)heads, ra);
     }
     return pg_launch(ctx, "rope", rope_kernel, dim3((unsigned)seq, (unsigned)heads), dim3(128), 0, ra);
 }
