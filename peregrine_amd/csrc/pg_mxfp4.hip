@@ -22,6 +22,7 @@
 // the instruction then takes half the cycles (random operands, all CUs: 4.2 PFLOP/s in FP8, 6.6 in FP6).
 //   B  lane l holds column l % 16, k = 32 (l / 16) .. + 31, element e in bits 6 e .. 6 e + 5 of its 24 bytes.
 #include <math.h>
+#include <type_traits>
 #include "pg_internal.h"
 #include "pg_stream_addr.h"
 #include "pg_digits.h"
@@ -475,18 +476,145 @@ __device__ __forceinline__ mt_place mt_find(const mt_gather &g, int gt) {
     return at;
 }
 
+// The caller's routing on its way into the first product's planes, for calls of few pairs: every workgroup works out by itself what its slots
+// hold (the pairs' entries in LDS, each expert's count, one ballot for the tile's expert), and one more writes what the later launches
+// read -- what route_lists_kernel makes, entries that break the rules replaced as there.  A launch of its own was 4.9 us and the gap
+// behind it.  us, with it : in the planes' launch: 20 tokens, top 4 of 32 experts of 2880 x 2880 97 : 94, 64 tokens 114 : 111; 19, top 4 of 8 of
+// 544 x 864 29.0 : 26.5; 64, top 4 of 16 of 576 x 864 34.0 : 31.4; 200, top 1 of 4 of 704 x 512 28.9 : 27.3; 64, top 4 of 64 of 3808 x 3008
+// 252 : 249; 70 drawn calls 0.936 of the time.  Beyond, a pair would no longer be a thread nor an expert a lane.
+constexpr int MT_ROUTE_PAIRS = 256, MT_ROUTE_EXPERTS = 64;  // at most: a pair a thread, an expert a lane
+struct mt_route {
+    const int *idx;
+    const float *w;
+    int tokens, top_k, tile;  // tile: slots of a token tile
+    int *topk_idx;
+    float *topk_p;
+    int *lists, *counts, *goff;
+};
+struct mt_route_lds {
+    int pair[MT_ROUTE_PAIRS], count[MT_ROUTE_EXPERTS], broken;
+    uint8_t zero[MT_ROUTE_PAIRS];     // pairs of weight 0
+    uint16_t slots[4][16];            // by wavefront: the pairs of its 16 slots
+};
+// The pairs' experts and the experts' counts (256 threads).
+__device__ __forceinline__ void mt_route_read(const mt_route &rt, int experts, mt_route_lds &l) {
+    const int t = threadIdx.x, P = rt.tokens * rt.top_k;
+    int e = t < P ? rt.idx[t] : 0;
+    if (t < P) l.pair[t] = e;
+    l.zero[t] = 0;
+    if (t < MT_ROUTE_EXPERTS) l.count[t] = 0;
+    if (t == 0) l.broken = 0;
+    __syncthreads();
+    if (t < P) {
+        bool ok = (unsigned)e < (unsigned)experts;
+        for (int j = t % rt.top_k; j > 0; --j) ok = ok && l.pair[t - j] != e;
+        if (!ok) l.broken = 1;
+    }
+    __syncthreads();
+    if (l.broken) {  // a token a thread, its entries in order
+        if (t < rt.tokens) {
+            int *mine = l.pair + t * rt.top_k;
+            auto taken = [&](int x, int k) {
+                bool is = false;
+                for (int j = 0; j < k; ++j) is |= mine[j] == x;
+                return is;
+            };
+            for (int k = 0; k < rt.top_k; ++k) {
+                int x = mine[k];
+                if ((unsigned)x < (unsigned)experts && !taken(x, k)) continue;
+                x = 0;
+                while (taken(x, k)) ++x;  // top_k <= experts: a free expert exists
+                mine[k] = x;
+                l.zero[t * rt.top_k + k] = 1;
+            }
+        }
+        __syncthreads();
+        e = l.pair[t < P ? t : 0];
+    }
+    if (t < P) atomicAdd(&l.count[e], 1);
+    __syncthreads();
+}
+// Running sum over a wavefront's lanes.
+__device__ __forceinline__ int mt_wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);  // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, true);  // row_bcast 15 into rows 1 and 3, then 31 into rows 2 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, true);
+    return v;
+}
+// What the later launches read, by one workgroup.
+__device__ __forceinline__ void mt_route_write(const mt_route &rt, int experts, const mt_route_lds &l) {
+    const int t = threadIdx.x, lane = t & 63, P = rt.tokens * rt.top_k;
+    if (t < P) {
+        rt.topk_idx[t] = l.pair[t];
+        rt.topk_p[t] = l.zero[t] ? 0.0f : rt.w[t];
+    }
+    if (t < 64) {
+        const int c = lane < experts ? l.count[lane] : 0, tiles = (c + rt.tile - 1) / rt.tile, through = mt_wave_scan(tiles);
+        if (lane < experts) {
+            rt.counts[lane] = c;
+            rt.goff[lane] = through - tiles;
+        }
+        if (lane == 63) rt.goff[experts] = through;
+    }
+    for (int e = t >> 6; e < experts; e += 4) {
+        int base = 0;
+        for (int p0 = 0; p0 < P; p0 += 64) {
+            const int p = p0 + lane;
+            const bool own = p < P && l.pair[p] == e;
+            const unsigned long long mask = __ballot(own);
+            if (own) rt.lists[(size_t)e * rt.tokens + base + __popcll(mask & ((1ull << lane) - 1ull))] = p;
+            base += __popcll(mask);
+        }
+    }
+}
+// mt_find from the counts, and the pairs of 16 slots of the tile (slot `first` of its expert on) in l.slots.
+__device__ __forceinline__ mt_place mt_route_find(const mt_route &rt, int experts, mt_route_lds &l, int gt, int sub) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, P = rt.tokens * rt.top_k;
+    const int c = lane < experts ? l.count[lane] : 0, tiles = (c + rt.tile - 1) / rt.tile, through = mt_wave_scan(tiles);
+    const unsigned long long here = __ballot(through - tiles <= gt && gt < through);
+    mt_place at = {-1, 0, 0};
+    if (!here) return at;
+    at.expert = __ffsll((unsigned long long)here) - 1;
+    at.first_tile = __builtin_amdgcn_readlane(through - tiles, at.expert);
+    at.used = __builtin_amdgcn_readlane(c, at.expert);
+    const int first = (gt - at.first_tile) * rt.tile + 16 * sub;
+    int base = 0;
+    for (int p0 = 0; p0 < P; p0 += 64) {
+        const int p = p0 + lane;
+        const bool own = p < P && l.pair[p] == at.expert;
+        const unsigned long long mask = __ballot(own);
+        const int slot = base + __popcll(mask & ((1ull << lane) - 1ull)) - first;
+        if (own && (unsigned)slot < 16u) l.slots[wave][slot] = (uint16_t)p;
+        base += __popcll(mask);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (its LDS accesses happen in order)
+    return at;
+}
+
 // One thread = 16 consecutive k of one token (half a block).  A wavefront = the 16 tokens of a group x two blocks x
 // their halves, tokens on consecutive lanes: what it writes are whole 256- and 128-byte runs of the records, and the
 // 256 bytes it reads of every token row are two full lines.
 // GATHER: the token groups are the experts' slots (mt_gather) instead of the rows in order.
 // SWIGLU: x holds mlp1's outputs, [pairs][2 * 32 nb], and the values are their bias and swiglu, made on the way (a launch
 // and a round trip of the pairs' rows less: 11.4 -> 8.1 us for 80 pairs of 2880).
-template <bool GATHER, bool SWIGLU = false>
+// ROUTE: the routing too (mt_route), by workgroup 0 and, each for itself, the others.
+template <bool GATHER, bool SWIGLU = false, bool ROUTE = false>
 __global__ __launch_bounds__(256) void mxfp4_planes_kernel(const float *__restrict__ x, int m, int nb, int ncp, int token_groups,
-                                                           char *__restrict__ bq, const mt_gather gat, const mt_swiglu act) {
-    static_assert(GATHER || !SWIGLU, "pairs have experts");
+                                                           char *__restrict__ bq, const mt_gather gat, const mt_swiglu act, const mt_route rt) {
+    static_assert((GATHER || !SWIGLU) && (GATHER || !ROUTE) && !(SWIGLU && ROUTE), "pairs have experts, the first product's a routing to make");
     const float *bias = nullptr;
-    const size_t wv = ((size_t)blockIdx.x * 256 + threadIdx.x) >> 6;  // (token group, pair of blocks)
+    __shared__ std::conditional_t<ROUTE, mt_route_lds, char> route;
+    if constexpr (ROUTE) {
+        mt_route_read(rt, gat.experts, route);
+        if (blockIdx.x == 0) {
+            mt_route_write(rt, gat.experts, route);
+            return;
+        }
+    }
+    const size_t wv = ((size_t)(blockIdx.x - (ROUTE ? 1 : 0)) * 256 + threadIdx.x) >> 6;  // (token group, pair of blocks)
     const int lane = threadIdx.x & 63, col = lane & 15, sub = (lane >> 4) & 1, npair = 2 * ncp;
     const size_t tg = wv / npair;
     if (tg >= (size_t)token_groups) return;  // (whole wavefronts)
@@ -495,12 +623,15 @@ __global__ __launch_bounds__(256) void mxfp4_planes_kernel(const float *__restri
     bool valid = t < (size_t)m && b < nb;
     if (GATHER) {
         const int gt = (int)(tg / gat.tb);
-        const mt_place at = mt_find(gat, __builtin_amdgcn_readfirstlane(gt));
+        mt_place at;
+        if constexpr (ROUTE) at = mt_route_find(rt, gat.experts, route, __builtin_amdgcn_readfirstlane(gt), __builtin_amdgcn_readfirstlane((int)(tg % gat.tb)));
+        else at = mt_find(gat, __builtin_amdgcn_readfirstlane(gt));
         const int e = at.expert;
         if (e < 0) return;  // past the last expert's tiles (whole wavefronts)
         const int slot = ((gt - at.first_tile) * gat.tb + (int)(tg % gat.tb)) * 16 + col;
         valid = slot < at.used && b < nb;
-        t = valid ? (size_t)(gat.lists[(size_t)e * gat.stride + slot] / gat.div) : 0;
+        if constexpr (ROUTE) t = valid ? (size_t)(route.slots[threadIdx.x >> 6][col] / gat.div) : 0;
+        else t = valid ? (size_t)(gat.lists[(size_t)e * gat.stride + slot] / gat.div) : 0;
         if (SWIGLU) bias = act.bias_tab[e];
     }
     float f[16];
@@ -1018,7 +1149,7 @@ pg_status pg_launch_mxfp4_tiles(pg_ctx *ctx, const float *x_dev, size_t m, const
     const size_t threads = p.groups * 2 * (size_t)ncp * 64;  // a wavefront per token group and pair of blocks
     PG_CHECK_ARG((threads + 255) / 256 < ((size_t)1 << 31), "mxfp4: %zu rows x %zu is too much for one pre-pass", m, w->k_in);
     PG_TRY(pg_launch(ctx, "mxfp4_planes", mxfp4_planes_kernel<false>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, x_dev, (int)m, nb,
-                     ncp, (int)p.groups, bq, mt_gather{}, mt_swiglu{}));
+                     ncp, (int)p.groups, bq, mt_gather{}, mt_swiglu{}, mt_route{}));
     // the staging depth: the less arithmetic a chunk holds, the more chunks ahead
 #define PG_MT_LAUNCH(RA_, BD1, BD2, BD4) \
     (p.tb == 1 ? launch_tiles<RA_, 1, BD1>(ctx, w, bq, part, m, ncp, p) \
@@ -1318,14 +1449,15 @@ void choose_tiles(const pg_ctx *ctx, size_t T, size_t E, size_t top_k, const siz
 }
 
 pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, const mt_shape &sh, size_t max_tiles, mt_gather gat, int div,
-                      const void **tab, size_t experts, int which, char *bq, float *y, const mt_swiglu *act = nullptr) {
+                      const void **tab, size_t experts, int which, char *bq, float *y, const mt_swiglu *act = nullptr, const mt_route *rt = nullptr) {
     const int nb = (int)(k_in / 32), ncp = (int)mx_chunks((size_t)nb);
     gat.div = div;
     const size_t groups = max_tiles * sh.tb, threads = groups * 2 * (size_t)ncp * 64;
     PG_CHECK_ARG((threads + 255) / 256 < ((size_t)1 << 31), "mxfp4 moe: too many pairs x %zu for one pre-pass", k_in);
     const dim3 grid((unsigned)((threads + 255) / 256));
-    if (act) PG_TRY(pg_launch(ctx, "mxfp4_planes_swiglu", mxfp4_planes_kernel<true, true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, *act));
-    else PG_TRY(pg_launch(ctx, "mxfp4_planes_gather", mxfp4_planes_kernel<true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, mt_swiglu{}));
+    if (act) PG_TRY(pg_launch(ctx, "mxfp4_planes_swiglu", mxfp4_planes_kernel<true, true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, *act, mt_route{}));
+    else if (rt) PG_TRY(pg_launch(ctx, "mxfp4_planes_route", mxfp4_planes_kernel<true, false, true>, dim3(grid.x + 1), dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, mt_swiglu{}, *rt));
+    else PG_TRY(pg_launch(ctx, "mxfp4_planes_gather", mxfp4_planes_kernel<true>, grid, dim3(256), 0, src, 0, nb, ncp, (int)groups, bq, gat, mt_swiglu{}, mt_route{}));
     const size_t nrg = (n_out + 15) / 16, n_wt = (nrg + sh.nw * sh.ra - 1) / (sh.nw * sh.ra);
     PG_CHECK_ARG(n_wt * max_tiles < ((size_t)1 << 28), "mxfp4 moe: %zu x %zu tiles", n_wt, max_tiles);
     const mt_experts ex = {reinterpret_cast<const uint8_t *const *>(tab + (size_t)(2 * which) * experts),
@@ -1428,9 +1560,11 @@ PG_API pg_status pg_mxfp4_moe_ffn_routed_dev(pg_ctx *ctx, const float *x_dev, si
         PG_TRY(moe_product_pairs<2>(ctx, x_dev, T, hidden, 2 * inter, P, 1, tab, E, 0, expert_idx_dev, topk_idx, top_k, h, sw));
         PG_TRY(moe_product_pairs<1>(ctx, h, P, inter, hidden, P, 0, tab, E, 1, nullptr, topk_idx, top_k, yb, mt_swiglu{}));
     } else {
-        PG_TRY(pg_launch_moe_routing(ctx, nullptr, expert_idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, lists, counts, goff, 16 * tb));
+        const bool route = P <= (size_t)MT_ROUTE_PAIRS && E <= (size_t)MT_ROUTE_EXPERTS;
+        if (!route) PG_TRY(pg_launch_moe_routing(ctx, nullptr, expert_idx_dev, weight_dev, T, E, top_k, topk_idx, topk_p, lists, counts, goff, 16 * tb));
+        const mt_route rt = {expert_idx_dev, weight_dev, (int)T, (int)top_k, 16 * tb, topk_idx, topk_p, lists, counts, goff};
         const mt_gather gat = {lists, counts, goff, (int)T, (int)E, tb, 1};
-        PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, shape[0], max_tiles, gat, (int)top_k, tab, E, 0, rec, h));
+        PG_TRY(moe_product(ctx, x_dev, hidden, 2 * inter, shape[0], max_tiles, gat, (int)top_k, tab, E, 0, rec, h, nullptr, route ? &rt : nullptr));
         PG_TRY(moe_product(ctx, h, inter, hidden, shape[1], max_tiles, gat, 1, tab, E, 1, rec, yb, &sw));
     }
     const bool four = T * hidden >= 65536;

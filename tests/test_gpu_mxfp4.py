@@ -362,6 +362,49 @@ def test_mxfp4_moe_finds_the_expert_of_a_tile(ctx, orc, E, T):
     test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, 64, 96, E, 3, T)
 
 
+@pytest.mark.parametrize("E,top_k,T", [(8, 3, 85), (8, 3, 86), (8, 4, 64), (9, 4, 65), (64, 4, 64), (65, 4, 40), (3, 3, 85), (5, 2, 120), (40, 8, 32)])
+def test_mxfp4_moe_routing_beside_the_planes(ctx, orc, E, top_k, T):
+    """Up to 256 pairs over up to 64 experts are routed inside the first product's planes' launch, more ahead of it: against the oracle at
+    either side of both lines, and with entries that name no expert, the same bits as with them replaced."""
+    import ctypes as C
+    from devbuf import DevBuf
+    from peregrine_amd import _ffi, mxfp4
+    from test_oracle_formats_pins import _mx_expert
+    hidden, inter = 96, 64
+    test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, hidden, inter, E, top_k, T)
+    say(f"mxfp4 moe odd entries beside the planes E={E} top_k={top_k} T={T}")
+    rng = np.random.default_rng(T + E)
+    some = [mxfp4.Mxfp4Expert(hidden, inter, 1.702, 7.0, *_mx_expert(rng, hidden, inter), ctx=ctx) for _ in range(3)]
+    tab = (C.c_void_p * E)(*[some[e % 3]._h.value for e in range(E)])
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    idx = np.stack([rng.permutation(E)[:top_k] for _ in range(T)]).astype(np.int32)
+    w = rng.uniform(0.2, 1.0, (T, top_k)).astype(np.float32)
+    idx[rng.integers(0, T, 5), rng.integers(0, top_k, 5)] = [-1, E, 2 ** 31 - 1, -2 ** 31, idx[0, 0]]
+    idx[T - 1, top_k - 1] = idx[T - 1, 0] if top_k > 1 else E
+    fixed, fw = idx.copy(), w.copy()
+    for t in range(T):
+        taken = set()
+        for k in range(top_k):
+            e = int(fixed[t, k])
+            if e < 0 or e >= E or e in taken:
+                fixed[t, k] = e = min(set(range(E)) - taken)
+                fw[t, k] = 0.0
+            taken.add(e)
+    assert (fixed != idx).any()
+
+    def rows(idx, w):
+        dx, di, dw, dout = DevBuf(ctx, host=x), DevBuf(ctx, host=idx), DevBuf(ctx, host=w), DevBuf(ctx, T * hidden * 4)
+        _ffi.check(_ffi.lib.pg_mxfp4_moe_ffn_routed_dev(ctx.handle, dx.ptr, T, di.ptr, dw.ptr, top_k, C.cast(tab, C.POINTER(C.c_void_p)), E, dout.ptr))
+        ctx.sync()
+        return dout.to_host(np.float32)
+    ctx.profile_begin()
+    got = rows(idx, w)
+    assert ("mxfp4_planes_route" in ctx.profile_end()) == (T * top_k <= 256 and E <= 64)
+    np.testing.assert_array_equal(got, rows(fixed, fw))
+    for ex in some:
+        ex.free()
+
+
 @pytest.mark.parametrize("hidden,inter,E,top_k,T", [(64, 96, 6, 6, 3), (512, 512, 200, 64, 1), (512, 96, 70, 12, 5), (64, 512, 2, 1, 9), (64, 96, 9, 4, 6), (96, 64, 5, 3, 8),
                                                    (64, 96, 8, 5, 4), (96, 64, 4, 2, 7)])
 def test_mxfp4_moe_pairs_with_entries_that_name_no_expert(ctx, hidden, inter, E, top_k, T):
