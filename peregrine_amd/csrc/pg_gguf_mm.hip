@@ -143,17 +143,22 @@ __global__ __launch_bounds__(256) void q41_offset_kernel(const uint16_t *__restr
 }
 
 // From 65 tokens on it is a product like any other, over K = the blocks: v_mfma_f32_32x32x2_f32 (the vector form was
-// bound by its own FMAs and LDS reads: 140 of 374 us at 1000 x 4096 -> 14336).  Workgroup = 4 wavefronts of 32 weight rows
+// bound by its own FMAs and LDS reads: 140 of 374 us at 1000 x 4096 -> 14336).  A wavefront takes 32 weight rows
 // x 64 tokens.  The order in which blocks meet the instruction's k-slots is free, so lane half h takes blocks
 // 8 i + 4 h .. + 3 for four instructions: one 128-bit load of a token's sums, and of a weight row's scales one 64-byte run
 // per 8 rows.  Result lane = weight row: the read-modify-write of y goes in 128-byte runs.
+//
+// A step waits for memory and multiplies little, so where few tiles leave the chip idle the chain of steps is what counts.
+// RUNS: a workgroup's four wavefronts share ONE tile, a quarter of the blocks each, and add their sums up through LDS in order
+// of the blocks; else they take four tiles side by side, whose tokens' sums they read in common.
 typedef float v16f __attribute__((ext_vector_type(16)));
+template <bool RUNS>
 __global__ __launch_bounds__(256) void q41_offset_mfma_kernel(const uint16_t *__restrict__ d, const uint16_t *__restrict__ m, int n_out,
                                                               int nb, const float *__restrict__ xsum, int nbp, int rows,
                                                               const float *__restrict__ part, int ks, size_t stride, float *y) {
-    const int lane = threadIdx.x & 63, l31 = lane & 31, h = lane >> 5;
-    const int n = blockIdx.x * 128 + (threadIdx.x >> 6) * 32 + l31, t0 = blockIdx.y * 64;
-    if (n - l31 >= n_out) return;
+    const int lane = threadIdx.x & 63, l31 = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = (RUNS ? blockIdx.x : blockIdx.x * 4 + wave) * 32 + l31, t0 = blockIdx.y * 64;
+    if (n - l31 >= n_out) return;  // (with RUNS: none)
     const int nc = n < n_out ? n : n_out - 1;
     const size_t tile = (size_t)(nc >> 3) * nb * 8 + (nc & 7);
     const float *xt[2];
@@ -201,13 +206,44 @@ __global__ __launch_bounds__(256) void q41_offset_mfma_kernel(const uint16_t *__
             }
         }
     };
-    const int steps = (nb + 7) / 8;
-    load(0, 0);
-    for (int i = 0; i < steps; i += 2) {
+    const int all = (nb + 7) / 8, per = RUNS ? (all + 3) / 4 : all;
+    const int begin = RUNS ? per * wave : 0, steps = RUNS ? min(all, begin + per) : all;
+    if (begin < steps) load(0, begin);
+    for (int i = begin; i < steps; i += 2) {
         if (i + 1 < steps) load(1, i + 1);
         multiply(0);
         if (i + 2 < steps) load(0, i + 2);
         if (i + 1 < steps) multiply(1);
+    }
+    if constexpr (RUNS) {  // register 16 j + r of all four runs is added up and stored by wavefront (16 j + r) / 8
+        __shared__ float sums[4][32][64];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sums[wave][16 * j + r][lane] = acc[j][r];
+        __syncthreads();
+        if (n >= n_out) return;
+        const int j = wave >> 1;
+        auto at = [&](int u) { const int r = 8 * (wave & 1) + u; return 32 * j + 8 * (r >> 2) + 4 * h + (r & 3); };
+        float first[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) first[u] = 0.0f;
+        for (int s = 0; s < (ks > 1 ? ks : 1); ++s) {
+            const float *p = (ks > 1 ? part + (size_t)s * stride : y) + (size_t)t0 * n_out + n;
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = t0 + at(u) < rows ? p[(size_t)at(u) * n_out] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) first[u] += v[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            float sum = sums[0][8 * wave + u][lane];
+#pragma unroll
+            for (int q = 1; q < 4; ++q) sum += sums[q][8 * wave + u][lane];
+            if (t0 + at(u) < rows) y[(size_t)(t0 + at(u)) * n_out + n] = first[u] + sum;
+        }
+        return;
     }
     if (n >= n_out) return;
 #pragma unroll
@@ -1194,7 +1230,13 @@ pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mm
     const size_t stride = rows * w->n_out;
     if (rows > 64) {
         if ((rows + 63) / 64 > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_matmul: too many activation rows");
-        return pg_launch(ctx, "gguf_q4_1_offsets", q41_offset_mfma_kernel, dim3(grid_for(w->n_out, 128), (unsigned)((rows + 63) / 64)), dim3(256), 0,
+        // Few tiles and steps enough to share out: us of the whole product, side by side : RUNS, 70 x 9760 -> 2282 (36 workgroups, 39 steps)
+        // 61.8 : 38.5, 129 x 14336 -> 4096 (96, 56) 100.5 : 78.8, 514 x 7040 -> 1330 (99, 28) 73.3 : 62.2, 256 x 4096 -> 4096 (128, 16) 47.4 : 41.1,
+        // 1008 x 1216 -> 972 (128, 5) 28.3 : 27.0, 1024 x 14336 -> 3072 (384, 56) 293 : 286; but 512 x 4096 -> 8192 (512, 16) 118.7 : 119.8,
+        // 1000 x 4096 -> 14336 (1792, 16) 297 : 304, and of two steps 200 x 512 -> 14336 (448) 25.8 : 29.4.
+        const bool runs = nb > 24 && (size_t)grid_for(w->n_out, 128) * ((rows + 63) / 64) * 2 <= 3 * (size_t)ctx->num_cu;
+        return pg_launch(ctx, "gguf_q4_1_offsets", runs ? q41_offset_mfma_kernel<true> : q41_offset_mfma_kernel<false>,
+                         dim3(grid_for(w->n_out, runs ? 32 : 128), (unsigned)((rows + 63) / 64)), dim3(256), 0,
                          (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, (const float *)md.xsum, nbp, (int)rows, part, ks, stride, y);
     }
     const size_t lds = ((size_t)nb * Q41_TT + 256 * (Q41_TT + 1)) * sizeof(float);

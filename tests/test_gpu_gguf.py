@@ -448,6 +448,35 @@ def test_gguf_q4_1_few_rows(ctx, orc, n_out, k_in, m):
     gw.free()
 
 
+@pytest.mark.parametrize("n_out,k_in,m,runs", [
+    (33, 832, 65, True), (31, 1088, 129, True), (160, 1600, 66, True), (1100, 2112, 64 * 3 + 1, True), (6144, 896, 512, True),  # the last: 384 tiles
+    (95, 768, 65, False), (6144, 832, 513, False),                                                                              # few steps, many tiles
+])
+def test_gguf_q4_1_offsets_on_the_matrix_cores(ctx, orc, n_out, k_in, m, runs):
+    """The offsets of 65 rows and more: a tile's blocks in four runs (quarters of 4, 5, 7 and 9 steps, some of them empty or short)
+    where tiles are few, else four tiles a workgroup.  The grid tells which (256 CUs)."""
+    from peregrine_amd import gguf, _ffi
+    say(f"gguf_matmul Q4_1 offsets n_out={n_out} k_in={k_in} m={m}")
+    raw = H.pack_q4_1(orc.rng_normal(41 + n_out, n_out * k_in, 0.0, 0.02) + np.float32(0.03))
+    x = orc.rng_normal(43 + m, m * k_in)
+    x.reshape(m, k_in)[:, :: max(1, k_in // 40)] *= 20
+    gw = gguf.GgufWeight(raw, 3, n_out, k_in, ctx)
+    _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 1))
+    try:
+        ctx.profile_begin()
+        got = gw.matmul(x, m).reshape(m, n_out)
+        ctx.profile_end()
+        grids = ctx.profile_grids()
+    finally:
+        _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 0))
+    tiles = ((m + 63) // 64) * ((n_out + 31) // 32 if runs else (n_out + 127) // 128)
+    assert list(grids["gguf_q4_1_offsets"]) == [256 * tiles], grids
+    for r in sorted({0, 1, 31, 32, 63, 64, m // 2, m - 1}):
+        want = orc.gguf_matmul(x.reshape(m, k_in)[r], 1, raw, 3, n_out, k_in)
+        H.assert_close_rel(got[r], want, RTOL_ACHIEVED[3], f"row {r}")
+    gw.free()
+
+
 @pytest.mark.parametrize("typ", [2, 8, 3])
 @pytest.mark.parametrize("n_out,k_in,m", [
     (31, 256, 8), (33, 288, 9), (127, 320, 16), (129, 1024, 17), (257, 1056, 24), (1000, 4096, 32), (64, 8224, 33),   # tokens in eights and sixteens
