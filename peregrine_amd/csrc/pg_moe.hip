@@ -55,9 +55,13 @@ __global__ void route_topk_kernel(const float *__restrict__ logits, int T, int E
 // own the digits' took 4.6 us (a layer of 26 tokens, 2 of 4 experts of 1568 x 1696, Q8_0: 31.9 -> 29.5 us; 4, 2 of 8 of 2048 x 4096: 35.4 -> 33.3).
 constexpr size_t MAX_ROUTE_LDS = 48u << 10;
 __host__ __device__ inline size_t route_row(size_t E) { return E | 1; }
-inline bool route_in_one(size_t T, size_t E, size_t top_k) {
+inline size_t route_lds(size_t T, size_t E, size_t top_k, bool logits) { return pg_round_up((logits ? T * route_row(E) * sizeof(float) : 0) + T * top_k, 4); }  // (read four bytes at a time)
+// (The caller's own routing holds no logits.  Where a table of them would not fit it took the three launches as well, 18.5 us and two gaps for
+// 422 tokens over 32 experts, top 4: layers of 422 tokens of 800 x 2752 117.0 : 108.5 us, 380 of 1024 x 1024 67.1 : 59.8, 512 of 2880 x 2880
+// 259.7 : 250.4, 400 of 512 x 640, top 2 47.0 : 41.5.)
+inline bool route_in_one(size_t T, size_t E, size_t top_k, bool logits) {
     // (lists: a wavefront of the 16 takes every 16th expert and looks at 64 pairs at a time: 128 such steps, 4 us, at most)
-    return T * top_k * E <= (1u << 17) && T * route_row(E) * sizeof(float) + T * top_k <= MAX_ROUTE_LDS;
+    return T * top_k * E <= (1u << 17) && route_lds(T, E, top_k, logits) <= MAX_ROUTE_LDS;
 }
 struct route_digits {
     const float *x;
@@ -384,8 +388,8 @@ pg_status pg_moe_cached_table(pg_ctx *ctx, const void *const *host_tab, size_t n
 pg_status pg_launch_moe_routing(pg_ctx *ctx, const float *router_logits_dev, const int *idx_dev, const float *weight_dev, size_t T,
                                 size_t E, size_t top_k, int *topk_idx, float *topk_p, int *lists, int *counts, int *goff, int tile,
                                 const pg_moe_digits *dig) {
-    if (route_in_one(T, E, top_k)) {
-        const size_t lds = pg_round_up((router_logits_dev ? T * route_row(E) * sizeof(float) : 0) + T * top_k, 4);  // (read four bytes at a time)
+    if (route_in_one(T, E, top_k, router_logits_dev != nullptr)) {
+        const size_t lds = route_lds(T, E, top_k, router_logits_dev != nullptr);
         route_digits rd = {};
         if (dig) {
             const int nb = (int)(dig->k / 32);

@@ -362,6 +362,18 @@ def test_mxfp4_moe_finds_the_expert_of_a_tile(ctx, orc, E, T):
     test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, 64, 96, E, 3, T)
 
 
+@pytest.mark.parametrize("E,top_k,T,one", [(32, 4, 373, True), (32, 2, 422, True), (64, 6, 190, True), (64, 4, 512, True), (64, 4, 513, False), (256, 2, 256, True)])
+def test_mxfp4_moe_routing_in_one_launch(ctx, orc, E, top_k, T, one):
+    """A routing whose table of logits would be more than the 48 KB that one launch takes, but which brings none: one launch up to
+    2^17 looks at a pair, three beyond."""
+    ctx.profile_begin()
+    try:
+        test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, 96, 64, E, top_k, T)
+    finally:
+        prof = ctx.profile_end()
+    assert ("moe_route_lists" in prof) == one and ("moe_copy_routing" in prof) != one, sorted(prof)
+
+
 @pytest.mark.parametrize("E,top_k,T", [(8, 3, 85), (8, 3, 86), (8, 4, 64), (9, 4, 65), (64, 4, 64), (65, 4, 40), (3, 3, 85), (5, 2, 120), (40, 8, 32)])
 def test_mxfp4_moe_routing_beside_the_planes(ctx, orc, E, top_k, T):
     """Up to 256 pairs over up to 64 experts are routed inside the first product's planes' launch, more ahead of it: against the oracle at
