@@ -1074,12 +1074,17 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
         return pg_gguf_hmm_rows(ctx, x_dev, m, &w, &y_dev, 1, hks);
     if (apart && q41 && w->k_in <= 32768 && pg_gguf_hmm_takes(ctx, PG_GGML_Q4_0, m, w->n_out, w->k_in, &hks)) {
         // Q4_1 at that size: the first term d sum (q - 8) x as the Q4_0 product on the f16 matrix cores, then the
-        // offsets times the rows' block sums (which the digit launch writes beside its planes)
-        PG_TRY(pg_gguf_hmm_rows(ctx, x_dev, m, &w, &y_dev, 1, hks));
-        PG_TRY(pg_workspace(ctx, pg_mmdigits_bytes(m, w->k_in), &ws));   // (the product is done with the arena)
-        const pg_mmdigits md = pg_mmdigits_carve(ws, m, w->k_in);
-        PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, m, w->k_in, w->ggml_type, md));
-        return pg_launch_q41_offset(ctx, w, md, m, nullptr, 1, y_dev);
+        // offsets times the rows' block sums (in the place of the rows' planes, with which the product is done), which add up
+        // the K chunks' planes too.  us, with a launch that adds them up, and the sums beside digits that nothing reads : now:
+        // 300 x 4096 -> 8192 88 : 78, 777 x 4096 -> 4096 104 : 92.5, 1024 x 14336 -> 3072 274 : 253, of one chunk 1000 x 4096 -> 14336 277 : 273.
+        const size_t sz_p = pg_hmm_planes_bytes(m, w->k_in), sz_part = pg_round_up(pg_gguf_hmm_part_floats(m, w->n_out, hks) * sizeof(float), 256);
+        PG_TRY(pg_workspace(ctx, sz_p + sz_part, &ws));
+        float *part = hks > 1 ? reinterpret_cast<float *>(static_cast<char *>(ws) + sz_p) : nullptr, *first = part ? part : y_dev;
+        const pg_hmm_planes planes = pg_hmm_planes_carve(ws, m, w->k_in);
+        PG_TRY(pg_launch_rows_to_f16_planes(ctx, x_dev, m, w->k_in, planes));
+        PG_TRY(pg_launch_gguf_hmm_group(ctx, w->k_in, &w, &first, 1, m, planes, hks, nullptr, true));
+        PG_TRY(pg_launch_block_sums(ctx, x_dev, m, w->k_in, static_cast<float *>(ws)));
+        return pg_launch_q41_offset(ctx, w, static_cast<const float *>(ws), m, part, hks, y_dev);
     }
     const int ks = pg_gguf_mm_splitk(ctx, w->n_out, w->k_in, (m + 31) / 32, m, false, nullptr);
     const size_t sz_d = pg_mmdigits_bytes(m, w->k_in);
@@ -1093,7 +1098,7 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
     grp.tiled = 1;
     // Q4_1: the Q4_0 product on the same nibbles and scales, then the blocks' offsets times the rows' block sums
     PG_TRY(pg_launch_gguf_mm(ctx, q41 ? PG_GGML_Q4_0 : w->ggml_type, w->n_out, w->k_in, w->qs_tiled, w->d, grp, m, md, y_dev, part, q41));
-    return q41 ? pg_launch_q41_offset(ctx, w, md, m, part, ks, y_dev) : PG_OK;
+    return q41 ? pg_launch_q41_offset(ctx, w, md.xsum, m, part, ks, y_dev) : PG_OK;
 }
 
 // Several products over the same activation rows (q/k/v, gate/up): the rows are rewritten

@@ -72,6 +72,17 @@ __global__ __launch_bounds__(256) void x_to_mm_digits_kernel(const float *__rest
     pg_emit_mm_digits<NIB>(f, row, b, sub, nb, nbp, digits, xs, xsum);
 }
 
+// The rows' block sums alone (where the first term of Q4_1 runs on the f16 matrix cores).
+__global__ __launch_bounds__(256) void block_sums_kernel(const float *__restrict__ x, int nb, int nbp, float *__restrict__ xsum) {
+    const size_t row = blockIdx.y;
+    const int b = blockIdx.x * 32 + (threadIdx.x >> 3), sub = threadIdx.x & 7;
+    if (b >= nb) return;  // whole 8-thread groups leave together
+    const float4 v = reinterpret_cast<const float4 *>(x + (row * nb + b) * 32)[sub];
+    const float f[4] = {v.x, v.y, v.z, v.w};
+    const float t = pg_block_sum(f);
+    if (sub == 0) xsum[row * nbp + b] = t;
+}
+
 // Q4_1's second term on many rows: y[t][n] = first term + sum_b (8 d[n][b] + m[n][b]) * xsum[t][b]; the first,
 // d sum (q - 8) x, is the Q4_0 product on the same nibbles, in y or (ks > 1) in the planes of its K chunks at part.
 //
@@ -1225,7 +1236,14 @@ pg_status pg_launch_x_to_mm_digits(pg_ctx *ctx, const float *x_dev, size_t rows,
                      (float *)nullptr);
 }
 
-pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mmdigits &md, size_t rows, const float *part, int ks, float *y) {
+pg_status pg_launch_block_sums(pg_ctx *ctx, const float *x_dev, size_t rows, size_t k, float *xsum) {
+    if (rows > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_matmul: too many activation rows");
+    const int nb = (int)(k / 32);
+    return pg_launch(ctx, "gguf_block_sums", block_sums_kernel, dim3((unsigned)((nb + 31) / 32), (unsigned)rows), dim3(256), 0, x_dev, nb,
+                     (int)pg_round_up(nb, 4), xsum);
+}
+
+pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const float *xsum, size_t rows, const float *part, int ks, float *y) {
     const int nb = (int)(w->k_in / 32), nbp = (int)pg_round_up(nb, 4);
     const size_t stride = rows * w->n_out;
     if (rows > 64) {
@@ -1237,13 +1255,13 @@ pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mm
         const bool runs = nb > 24 && (size_t)grid_for(w->n_out, 128) * ((rows + 63) / 64) * 2 <= 3 * (size_t)ctx->num_cu;
         return pg_launch(ctx, "gguf_q4_1_offsets", runs ? q41_offset_mfma_kernel<true> : q41_offset_mfma_kernel<false>,
                          dim3(grid_for(w->n_out, runs ? 32 : 128), (unsigned)((rows + 63) / 64)), dim3(256), 0,
-                         (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, (const float *)md.xsum, nbp, (int)rows, part, ks, stride, y);
+                         (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, xsum, nbp, (int)rows, part, ks, stride, y);
     }
     const size_t lds = ((size_t)nb * Q41_TT + 256 * (Q41_TT + 1)) * sizeof(float);
     if (lds > 128 * 1024) return pg_fail(PG_EUNSUPPORTED, "gguf_matmul: Q4_1 rows of %zu on the matrix-core route", w->k_in);
     PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)q41_offset_kernel, 128 * 1024));
     return pg_launch(ctx, "gguf_q4_1_offsets", q41_offset_kernel, dim3(grid_for(w->n_out, 256 / Q41_NQ), (unsigned)((rows + Q41_TT - 1) / Q41_TT)), dim3(256), lds,
-                     (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, (const float *)md.xsum, nbp, (int)rows, part, ks, stride, y);
+                     (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, xsum, nbp, (int)rows, part, ks, stride, y);
 }
 
 // Digits of `act_rows` activation rows that no XCD's L2 (4 MiB) can keep while every workgroup

@@ -396,10 +396,11 @@ pg_status pg_launch_gguf_one_launch(pg_ctx *ctx, int ggml_type, size_t k_in, con
 pg_status pg_launch_x_to_mm_digits(pg_ctx *ctx, const float *x_dev, size_t rows, size_t k, int ggml_type,
                                    const pg_mmdigits &md);
 // Q4_1 on the matrix-core route: the product is the Q4_0 product on the same nibbles and scales plus
-// y[t][n] += sum_b (8 d + m)[n][b] * (sum of x over block b of row t); this adds the second term (md.xsum
-// as pg_launch_x_to_mm_digits leaves it for PG_GGML_Q4_1).  k_in up to 32768.
+// y[t][n] += sum_b (8 d + m)[n][b] * (sum of x over block b of row t); this adds the second term (xsum
+// as pg_launch_x_to_mm_digits leaves it for PG_GGML_Q4_1, or pg_launch_block_sums).  k_in up to 32768.
 // With ks > 1 the first term is still the ks planes at `part` (rows * n_out floats each), added up on the way.
-pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const pg_mmdigits &md, size_t rows, const float *part, int ks, float *y);
+pg_status pg_launch_block_sums(pg_ctx *ctx, const float *x_dev, size_t rows, size_t k, float *xsum);
+pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const float *xsum, size_t rows, const float *part, int ks, float *y);
 // Which activation rows multiply which weights.  Without `counts`: one weight tensor and pairs
 // 0 .. max_count-1.  With `counts`: expert e owns counts[e] pairs, listed (in ascending order) in
 // lists[e * list_stride ..]; its weights are qs_table[e] / d_table[e].  Pair p reads activation
