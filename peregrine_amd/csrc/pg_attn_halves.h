@@ -374,46 +374,86 @@ void gqa_attention_halves_kernel(const char *__restrict__ planes, int n_blocks, 
     }
 }
 
-// The runs' records of every row that has more than one: HD / 4 lanes to a row.
-constexpr int HALVES_RUNS_MAX = 16;
-template <int HD>
-__global__ __launch_bounds__(256) void attn_halves_combine_kernel(attn_args aa) {
+// The runs' records of every row that has more than one, HD / 4 lanes to a row; and what the next product reads instead of f32:
+// AS = 3 / 4 byte digits for Q4_0 / Q8_0 (pg_emit_mm_digits), 5 f16 planes, a token to a workgroup of 1024 (nqh * HD <= 4096).  Rows of one run
+// are then read from where the kernel above left them.  As a launch of its own behind this one the next product's input took 4 to 7 us: blocks of 711 tokens of
+// d 1024 (Q8_0) 126 : 121.5 us, 679 of 2048 256.5 : 251, 602 behind 1841 270 : 264.5, Q4_0 450 of 2048 214 : 208.5, 350 164.5 : 160.5; as f16 planes
+// 777 behind 100 of 4096 859 : 848 (the merge 9.8 + 6.2 : 10.9).
+// MOST: runs at the most; four take half the registers of sixteen, so that twice the wavefronts wait for memory at a time (the f16 planes 15 : 10.9).
+constexpr int HALVES_RUNS_MAX = 16, HALVES_RUNS_FEW = 4;
+struct halves_next {
+    int8_t *digits;
+    float *xs;
+    _Float16 *hi, *lo;
+    float *inv;
+};
+template <int HD, int AS, int MOST>
+__global__ __launch_bounds__(AS == 5 ? 1024 : 256) void attn_halves_combine_kernel(attn_args aa, halves_next next) {
     constexpr int LPR = HD / 4;
     const int G = aa.group, nrows = G * aa.seq_q, rows = aa.nqh * aa.seq_q;
-    const int r_out = blockIdx.x * (256 / LPR) + (int)threadIdx.x / LPR, d = (threadIdx.x % LPR) * 4;
-    if (r_out >= rows) return;
-    const int qt = r_out / aa.nqh, row = qt * G + (r_out % aa.nqh) % G;
-    const int tiles = halves_tiles(aa, row / HALVES_ROWS, nrows), runs = (tiles + aa.chunk - 1) / aa.chunk;
-    if (runs < 2) return;
-    const float *rec = aa.part + (size_t)r_out * aa.splits * (HD + 4);
-    float2 ml[HALVES_RUNS_MAX];
-    float4 v[HALVES_RUNS_MAX];
-#pragma unroll
-    for (int i = 0; i < HALVES_RUNS_MAX; ++i)
-        if (i < aa.splits) {
-            const float *p = rec + (size_t)min(i, runs - 1) * (HD + 4);
-            ml[i] = *reinterpret_cast<const float2 *>(p);
-            v[i] = *reinterpret_cast<const float4 *>(p + 4 + d);
-        }
-    float m = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < HALVES_RUNS_MAX; ++i)
-        if (i < runs) m = fmaxf(m, ml[i].x);
-    float l = 0.f;
-    float4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < HALVES_RUNS_MAX; ++i)
-        if (i < runs) {
-            const float w = ml[i].x == -INFINITY ? 0.f : expf(ml[i].x - m);
-            l = fmaf(ml[i].y, w, l);
-            o.x = fmaf(v[i].x, w, o.x); o.y = fmaf(v[i].y, w, o.y); o.z = fmaf(v[i].z, w, o.z); o.w = fmaf(v[i].w, w, o.w);
-        }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const int r_out = AS == 5 ? (int)blockIdx.x * aa.nqh + (int)threadIdx.x / LPR : (int)blockIdx.x * (256 / LPR) + (int)threadIdx.x / LPR;
+    const int d = (threadIdx.x % LPR) * 4;
+    const bool live = AS == 5 ? (int)threadIdx.x < aa.nqh * LPR : r_out < rows;
+    if (AS != 5 && !live) return;
+    const int qt = AS == 5 ? (int)blockIdx.x : r_out / aa.nqh, head = r_out - qt * aa.nqh, row = qt * G + head % G;
+    const int tiles = halves_tiles(aa, row / HALVES_ROWS, nrows), runs = live ? (tiles + aa.chunk - 1) / aa.chunk : 0;
+    if (AS == 0 && runs < 2) return;
     float4 *at = reinterpret_cast<float4 *>(aa.out + (size_t)r_out * HD + d);
-    float4 w = {o.x * inv, o.y * inv, o.z * inv, o.w * inv};
-    if (aa.accumulate) {
-        const float4 old = *at;
-        w.x += old.x; w.y += old.y; w.z += old.z; w.w += old.w;
+    float4 w = {0.f, 0.f, 0.f, 0.f};
+    if (runs >= 2) {
+        const float *rec = aa.part + (size_t)r_out * aa.splits * (HD + 4);
+        float2 ml[MOST];
+        float4 v[MOST];
+#pragma unroll
+        for (int i = 0; i < MOST; ++i)
+            if (i < aa.splits) {
+                const float *p = rec + (size_t)min(i, runs - 1) * (HD + 4);
+                ml[i] = *reinterpret_cast<const float2 *>(p);
+                v[i] = *reinterpret_cast<const float4 *>(p + 4 + d);
+            }
+        float m = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < MOST; ++i)
+            if (i < runs) m = fmaxf(m, ml[i].x);
+        float l = 0.f;
+        float4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < MOST; ++i)
+            if (i < runs) {
+                const float e = ml[i].x == -INFINITY ? 0.f : expf(ml[i].x - m);
+                l = fmaf(ml[i].y, e, l);
+                o.x = fmaf(v[i].x, e, o.x); o.y = fmaf(v[i].y, e, o.y); o.z = fmaf(v[i].z, e, o.z); o.w = fmaf(v[i].w, e, o.w);
+            }
+        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        w = float4{o.x * inv, o.y * inv, o.z * inv, o.w * inv};
+    } else if (runs == 1) {
+        w = *at;
     }
-    *at = w;
+    if constexpr (AS == 0) {
+        if (aa.accumulate) {
+            const float4 old = *at;
+            w.x += old.x; w.y += old.y; w.z += old.z; w.w += old.w;
+        }
+        *at = w;
+    } else {
+        const float f[4] = {w.x, w.y, w.z, w.w};
+        if constexpr (AS == 5) {
+            __shared__ float red[16];
+            float amax = fmaxf(fmaxf(pg_f16_mag(f[0]), pg_f16_mag(f[1])), fmaxf(pg_f16_mag(f[2]), pg_f16_mag(f[3])));
+            for (int o = 32; o; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+            if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+            __syncthreads();
+            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, red[i]);
+            const pg_f16_row_scale sc = pg_f16_row_scale_of(amax);
+            if (threadIdx.x == 0) {
+                next.inv[2 * qt] = sc.i1;
+                next.inv[2 * qt + 1] = sc.i2;
+            }
+            const size_t k = (size_t)r_out * HD + d;
+            if (live) pg_f16_split4(f, sc, reinterpret_cast<uint2 *>(next.hi + k), reinterpret_cast<uint2 *>(next.lo + k));
+        } else {
+            const int nb = aa.nqh * (HD / 32);
+            pg_emit_mm_digits<AS == 3>(f, (size_t)qt, head * (HD / 32) + d / 32, threadIdx.x & 7, nb, (nb + 3) / 4 * 4, next.digits, next.xs);
+        }
+    }
 }

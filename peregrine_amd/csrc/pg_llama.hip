@@ -1560,7 +1560,8 @@ bool plan_halves(pg_ctx *ctx, size_t group, size_t seq_q, size_t nkv, size_t hd,
     if (chunk > (size_t)HALVES_CHUNK_MAX || p->runs > (size_t)HALVES_RUNS_MAX) return false;
     p->part_bytes = p->runs > 1 ? pg_round_up(rows * nkv * p->runs * (hd + 4) * sizeof(float), 256) : 0;
     // both sides in us: a tile of 32 keys takes a wavefront 5 to 6 with f32 matrix instructions, one on each of 1024 SIMDs, and here
-    // 1.6, or 1.3 of a workgroup's chain where they do not fill the chip; the planes are written at 2.2 TB/s
+    // 1.6, or 1.3 of a workgroup's chain where they do not fill the chip; the planes are written at 2.2 TB/s.  (`digits`: a launch of their own, which a
+    // merge of runs now saves; the line stays where it was, so that no call changes its kernel.)
     const double size = hd / 128.0, work = 4.0 * sum * nkv / (4.0 * cus), waves = 4.0 * p->blocks * nkv;
     size_t c = 0, r = 0;
     const double f32 = split_mfma_tiles(ctx, group, seq_q, nkv, mask_kind, offset, len, &c, &r)
@@ -1579,11 +1580,13 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
                            size_t seq_q, float scale, int mask_kind, size_t offset, size_t window, size_t sink,
                            float logit_cap, float *out, int accumulate, const pg_xdigits *xd = nullptr, int digit_kind = 0,
                            const size_t *global_positions = nullptr, size_t num_global = 0,
-                           const attn_args *rope_fusion = nullptr, const pg_mmdigits *md = nullptr, bool *md_written = nullptr) {
+                           const attn_args *rope_fusion = nullptr, const pg_mmdigits *md = nullptr, bool *md_written = nullptr,
+                           const pg_hmm_planes *hp = nullptr) {
     kc->touch(ctx);
     vc->touch(ctx);
     // With `md` (digit_kind names the tensor type) a merge of key runs writes the rows as the matrix-core
     // product's digit planes instead of f32 and sets *md_written; a kernel that needs no merge writes `out`.
+    // With `hp` the same for the f16 planes (the merge of the f16 matrix-core kernel alone).
     // With `xd` (one-token step, accumulate == 0, head_dim % 32 == 0) the rows also, or only,
     // leave as GEMV digits of kind `digit_kind`; `out` must still be a valid buffer.
     const size_t len = kc->len, hd = kc->head_dim;
@@ -1718,9 +1721,19 @@ pg_status launch_attention(pg_ctx *ctx, const float *q, const pg_kv_cache *kc, c
         PG_TRY(pg_allow_dynamic_lds(ctx, (const void *)kern, lds_bytes));
         PG_TRY(pg_launch(ctx, "gqa_attention_halves", kern, dim3((unsigned)(lp.blocks * nkv * lp.runs)), dim3(256), lds_bytes, (const char *)halves_planes,
                          (int)lp.blocks, aa, (int)nkv, (int)lp.tiles));
-        if (lp.runs > 1)
-            PG_TRY(pg_launch(ctx, "gqa_attention_halves_combine", hd == 64 ? attn_halves_combine_kernel<64> : attn_halves_combine_kernel<128>,
-                             dim3((unsigned)((rows * (hd / 4) + 255) / 256)), dim3(256), 0, aa));
+        if (lp.runs > 1) {
+            const int as = accumulate || xd ? 0 : hp && nqh * hd <= 4096 ? 5 : md ? (digit_kind == PG_GGML_Q4_0 ? 3 : 4) : 0;
+            const halves_next next = {md ? md->digits : nullptr, md ? md->xs : nullptr, hp ? (_Float16 *)hp->hi : nullptr, hp ? (_Float16 *)hp->lo : nullptr,
+                                      hp ? hp->inv : nullptr};
+#define PG_HALVES_COMBINE(AS_)                                                                                                         \
+    (lp.runs <= (size_t)HALVES_RUNS_FEW ? (hd == 64 ? attn_halves_combine_kernel<64, AS_, HALVES_RUNS_FEW> : attn_halves_combine_kernel<128, AS_, HALVES_RUNS_FEW>)  \
+                                        : (hd == 64 ? attn_halves_combine_kernel<64, AS_, HALVES_RUNS_MAX> : attn_halves_combine_kernel<128, AS_, HALVES_RUNS_MAX>))
+            auto *merge = as == 0 ? PG_HALVES_COMBINE(0) : as == 3 ? PG_HALVES_COMBINE(3) : as == 4 ? PG_HALVES_COMBINE(4) : PG_HALVES_COMBINE(5);
+#undef PG_HALVES_COMBINE
+            PG_TRY(pg_launch(ctx, as == 0 ? "gqa_attention_halves_combine" : as == 5 ? "gqa_attention_halves_combine_f16_planes" : "gqa_attention_halves_combine_mm_digits",
+                             merge, dim3((unsigned)(as == 5 ? seq_q : (rows * (hd / 4) + 255) / 256)), dim3(as == 5 ? 1024 : 256), 0, aa, next));
+            if (as && md_written) *md_written = true;
+        }
     } else if (tiled_kernel && (hd == 64 || hd == 128)) {
         // matrix-core kernel: one workgroup per kv head and pair of 32-row items (first with last, ...);
         // the kv head varies fastest, so with eight kv heads each XCD's L2 keeps one head's keys and values
@@ -2459,10 +2472,10 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
     ra.cos_t = b->rope->cos_t; ra.sin_t = b->rope->sin_t; ra.hd = (int)hd; ra.pos0 = (int)offset; ra.nseg = 3;
     PG_TRY(launch_rope(ctx, ra, seq, b->nqh + 2 * b->nkvh));
     cache->len = offset + seq;
-    bool md_written = false;  // (a merge of key runs writes the o-projection's digit planes itself)
+    bool md_written = false;  // (a merge of key runs writes the o-projection's digit or f16 planes itself)
     PG_TRY(launch_attention(ctx, q_rope, cache, cache, b->nqh, seq, 1.0f / sqrtf((float)hd), PG_MASK_CAUSAL, offset, 0, 0,
-                            0.0f, attn, 0, nullptr, type, nullptr, 0, nullptr, hd % 32 == 0 && !hm[3] ? &md_q : nullptr, &md_written));
-    if (hm[3]) PG_TRY(pg_launch_rows_to_f16_planes(ctx, attn, seq, q_dim, pl_q));
+                            0.0f, attn, 0, nullptr, type, nullptr, 0, nullptr, hd % 32 == 0 && !hm[3] ? &md_q : nullptr, &md_written, hm[3] ? &pl_q : nullptr));
+    if (hm[3] && !md_written) PG_TRY(pg_launch_rows_to_f16_planes(ctx, attn, seq, q_dim, pl_q));
     else if (!md_written) PG_TRY(pg_launch_x_to_mm_digits(ctx, attn, seq, q_dim, type, md_q));
     PG_TRY(product(3, md_q));
     PG_TRY(norm_digits(h_dev, 3, h1, b->ffn_norm_w, hm[4]));  // h1 = h + attn . Wo, and its norm as digits

@@ -430,6 +430,28 @@ def test_llama_block_many_token_steps_on_the_f16_matrix_cores(ctx, orc, shape, t
         assert name in prof, (name, sorted(prof))
 
 
+@pytest.mark.parametrize("typ,force,shape,steps,name", [
+    (2, 2, (256, 32, 8, 64, 512), (450,), "gqa_attention_halves_combine_mm_digits"), (8, 2, (256, 32, 8, 128, 544), (331,), "gqa_attention_halves_combine_mm_digits"),
+    (2, 1, (512, 16, 4, 64, 512), (450,), "gqa_attention_halves_combine_f16_planes"), (8, 1, (256, 32, 8, 128, 512), (260,), "gqa_attention_halves_combine_f16_planes"),
+    (8, 1, (256, 30, 6, 128, 512), (300,), "gqa_attention_halves_combine_f16_planes"),       # a token's row that leaves wavefronts of its workgroup idle
+    (2, 1, (256, 66, 2, 64, 512), (420,), "gqa_attention_halves_combine"),                   # a row too wide for one workgroup: f32, converted by a launch of its own
+])
+def test_llama_block_merge_of_runs_writes_the_next_products_rows(ctx, orc, typ, force, shape, steps, name):
+    """The merge of the f16 attention's key runs writes the o-projection's digits or f16 planes; among the rows are some of one run, which the
+    attention has finished itself."""
+    from peregrine_amd import _ffi
+    d, nqh, nkvh, hd, ffn = shape
+    _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, force))
+    try:
+        ctx.profile_begin()
+        _block_case(ctx, orc, d, nqh, nkvh, hd, ffn, typ, steps, max_seq=512, seed=83)
+        prof = ctx.profile_end()
+    finally:
+        _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 0))
+    assert name in prof and ("rows_to_f16_planes" in prof) == (force == 1 and not name.endswith("planes")), sorted(prof)
+    assert "x_to_mm_digits" not in prof, sorted(prof)
+
+
 @pytest.mark.parametrize("ffn", [4096, 4160, 8192, 8256, 16384, 16448, 32768])
 def test_llama_block_silu_up_rows_at_the_edges_of_their_registers(ctx, orc, ffn):
     """SiLU.up as f16 planes: a row is held by 512 threads of 2, 4, 8 or 16 float4s; the longest row of each instance and
