@@ -204,7 +204,7 @@ class Bench:
                 "gemm_tile_k_loop_us": round(loop_us.value, 2),
                 "int8_peak_at_gemm_clock_tops": round(256 * 8192 * g_ghz.value / 1e3, 1),
                 "note": "measured in this run by pg_probe_*: 8 wavefronts per CU issuing only v_mfma_i32_32x32x32_i8 on "
-                        "pseudo-random registers; 128-bit non-temporal reads over 3 x 256 MiB; shader cycles / wall clock "
+                        "pseudo-random registers (the product's own 16x16x64 holds up to 4.0 POP/s so); 128-bit non-temporal reads over 3 x 256 MiB; shader cycles / wall clock "
                         "inside the K loop of the 256x256 tile of a [2048x4096]x[4096x14336] product"}
 
 
@@ -291,7 +291,7 @@ def main():
     gemm_tops = (LAYER_OPS / gemm_lps) / (gemm_avg_ms * 1e-3) / 1e12
     quant_ks = (4096, 4096, 4096, 14336)  # one quantisation per call of the step
     quant_bytes = sum(M_PREFILL * k * 4 + M_PREFILL * k + M_PREFILL * 4 for k in quant_ks)
-    roofline = {"kernel": "gemm_w8a8_kernel (i8 MFMA 32x32x32; the 7 products as 5 launches: q|k|v, o, gate, up, down)", "bound": "mfma",
+    roofline = {"kernel": "gemm_w8a8_kernel (i8 MFMA 16x16x64; the 7 products as 5 launches: q|k|v, o, gate, up, down)", "bound": "mfma",
                 "achieved": round(gemm_tops, 1), "peak": PEAK_INT8_TOPS, "unit": "TOP/s",
                 "frac": round(gemm_tops / PEAK_INT8_TOPS, 4), "traffic": B.traffic_for("gemm_w8a8", grids),
                 "ops_per_launch": int(LAYER_OPS / gemm_lps), "launches_per_step": gemm_lps, "avg_launch_ms": round(gemm_avg_ms, 4),
