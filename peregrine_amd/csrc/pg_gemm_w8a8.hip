@@ -12,8 +12,8 @@
 // fragments read from LDS are as many.  us, 32x32x32 : 16x16x64, weights from HBM: W8A8 2048 x 4096 -> 14336 134 : 124, 2048 x
 // 14336 -> 4096 158 : 149, 2048 x 4096 -> 6144 63 : 58, 1760 x 12387 -> 15665 356 : 327, 960 x 4001 -> 710 18.8 : 17.5 (120 drawn products of 33
 // rows and more 0.98, 40 drawn layers 0.965 of the time); W8A32 2048 x 4096 -> 14336 416 : 395, 888 x 11222 -> 4096 154 : 134, 356 x 4096 -> 14336
-// 92 : 85, 197 x 1024 -> 4096 10.9 : 10.4 (100 drawn 0.98; four wavefronts a workgroup alone on their CU, which issue it every 18
-// cycles instead of 16, up to 2 % longer: 202 x 5949 -> 1265 25.4 : 26.0).
+// 92 : 85, 197 x 1024 -> 4096 10.9 : 10.4 (100 drawn 0.98; but four wavefronts alone on their CU
+// issue it every 18 cycles instead of 16, so that W8A32's 64x64 has eight: pick_w8a32).
 //
 // Workgroup = NWM x NWN wavefronts over a BM x BN output tile; each wavefront
 // holds (BM/NWM/16) x (BN/NWN/16) accumulator tiles of 16x16.  K is consumed in
@@ -836,7 +836,7 @@ int pick_tile(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m
 pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,
                         const pg_qtensor *const *w, float *const *out, int count, size_t m, int32_t *acc,
                         int pick = -1, const int32_t *comb = nullptr, size_t comb_plane = 0) {
-    if (comb) {  // (for products that fill the part with 256x256 tiles: w8a32_large; the first five codes for tests)
+    if (comb) {  // (what one W8A32 launch does not reach; the first five codes for tests)
 #define PG_COMB(CODE, ...) \
     if (code == CODE) return launch_group<__VA_ARGS__, true>(ctx, a_i8, a_stride, a_scales, w, out, count, m, acc, 1, 0, comb, comb_plane);
         const int code = ctx->gemm_force_tile >= 1 && ctx->gemm_force_tile <= 5 ? ctx->gemm_force_tile : 2;
@@ -1156,46 +1156,42 @@ pg_status pg_launch_gemm_w8a8(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride,
     return gemm_dispatch(ctx, a_i8, a_stride, a_scales, &w, &out, 1, m, acc, pick);
 }
 
-// The W8A32 product over three digit planes in one launch, where it is the better route: up to 32 rows the few-row kernel
-// (three or six tiles of planes), beyond that what pick_w8a32 says, unless tiles of 256x256 fill the part and are
-// mostly rows (three quarters; then the two low planes stacked and the combining pass below; `takes` says which).  Tiles
-// filled up by a vocabulary's columns are no reason: the padding rows are multiplied too, and two planes of accumulators of
-// m_pad x n written and read.  us, one launch : stacked: 1 x 4096 -> 50257 62 : 161, 32 x 4096 -> 128256 240 : 423,
-// 191 x 4096 -> 50257 144 : 249, 300 x 1024 -> 32000 54 : 93, 2048 x 14336 -> 32000 2890 : 2570.  (With short K the one
-// launch is also the faster one on tiles that are all rows: 512 x 1024 -> 50257 121 : 348, 2048 x 4096 -> 32000 855 : 859.)
-static bool w8a32_large(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
-    const size_t cus = (size_t)ctx->num_cu, m_pad = pg_round_up(m, 256), t256 = m_pad / 256 * ((w->cols + 255) / 256);
-    return 4 * m >= 3 * m_pad && (t256 * 2 >= 3 * cus || (t256 <= cus && t256 * 10 >= 7 * cus));
-}
+// The W8A32 product over three digit planes in one launch: up to 32 rows the few-row kernel (three or six tiles of planes), beyond
+// that what pick_w8a32 says.  What its 32-bit offsets do not reach takes three launches: the two low planes stacked as one
+// product, and the third plane's with the combining pass below.  That was the route of large products too, as long as one launch had
+// no 64x256 tiles: of 976 products of 5e10 multiply-adds and more the three launches are 2 % faster at the best, 1.35 times as long in the
+// middle and 4 times with short K.  us, three launches : one: 15576 x 15659 -> 1990 1577 : 1609, 2048 x 14336 -> 32000 2236 : 2227, 2048 x 4096 -> 14336
+// 382 : 293, 1000 x 4096 -> 4096 115 : 51, 192 x 256 -> 46080 69 : 22.
 bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
-    return ctx->gemm_force_tile == 0 && !w8a32_large(ctx, w, m) && w->k_pad < (1ull << 22) && w->cols < (1ull << 30) &&
+    return ctx->gemm_force_tile == 0 && w->k_pad < (1ull << 22) && w->cols < (1ull << 30) &&
            2 * pg_round_up(m, PG_MPAD) * w->k_pad + 128 * w->k_pad < (1ull << 31);
 }
-// From 33 rows on: the tiles of 64x64 to 128x128 by rounds of workgroups, one a CU, times what a round takes (18, 24 and 40: us at K =
-// 4096; drawn from 180 shapes to 2500 rows and 130000 columns, 0.1 % over the best of the three), unless other tiles, or up to 512 rows groups
-// of 16 or 32 of them in the few-row kernel (whose wavefronts cut K), are estimated to take less than 0.93 of that, past 700 rows 0.9 (they err
-// more there: at 0.92 one of 85 took 5 % longer).  The estimates as in
-// pick_tile, a group's workgroups counted by XCD as in the few-row route (by the part, 467 x 8337 -> 534 went to groups of 32 rows, 58.6 us where
-// 64x64 takes 39 and 32x64 34), fitted to 480 products of 33 .. 2048 rows, K to 16384 and n to 131072 (weights from HBM and from the Infinity
-// Cache, each kernel timed on each): of those none takes over 2 % longer than with the three tiles alone; 33 to 64 rows 0.77 of the time, 65 to
-// 256 0.83, 257 to 700 0.93, beyond 0.99 (without the margins 0.77, 0.83, 0.92 and 0.97, and now and then 5 % more).  us, those : these: 54 x 2150 -> 488
-// 14.9 : 9.4, 163 x 2016 -> 1010 15.0 : 11.8, 849 x 6977 -> 322 38 : 34, 710 x 5963 -> 1659 48.4 : 45.6.  (Fitted while the tiles ran on
-// 32x32x32 matrix instructions and 128x128 on sixteen wavefronts.  It is eight of 32 x 64 now: ten fragment reads a k-step for 24 instructions
-// where it was eight for twelve; us, then : now: 1000 x 4096 -> 4096 64 : 58, 888 x 11222 -> 4096 154 : 134, 2317 x 3643 -> 2853 114 : 107.)
+// From 33 rows on the kernel of least estimated time: tiles of 32x64 to 128x128, or up to 512 rows groups of 16 or 32 of them in the
+// few-row kernel (whose wavefronts cut K).  The estimates as in pick_tile, a group's workgroups counted by XCD as in the few-row route (by
+// the part, 467 x 8337 -> 534 went to groups of 32 rows, 58.6 us where 64x64 takes 39 and 32x64 34).  Fitted to two thirds of 5760 products of 33 ..
+// 16384 rows, K 64 .. 16384 and n 64 .. 131072 (weights from HBM, each kernel timed on each): on the others the choice takes 0.4 % more than the best
+// kernel up to 64 rows, 0.5 % to 256, 0.65 % beyond (4 to 5 % at the 95th percentile).  Fitted to the kernels as they were on 32x32x32, with a margin
+// for the tiles of 64x64, 64x128 and 128x128, it took 2, 4.4 and 11 % more, and past 700 rows 46, most of it by the three launches
+// above.
+// What the shapes are: 64x64 on four wavefronts, alone on their CU, issues a matrix instruction every 18 cycles, on eight every 16: 0.92 of the time in
+// the middle of those products, 0.83 to 0.98 for nine in ten (197 x 1024 -> 4096 11.1 : 10.3 us, 202 x 5949 -> 1265 34.1 : 31.9).  128x128 has sixteen: on
+// eight of 32 x 64 it is the shorter one over a long K, where 64x256 is shorter still, and up to 1.6 times as long over a short one, where what
+// counts is how many wavefronts store.  us, eight : sixteen : 64x256: 1000 x 4096 -> 4096 52.9 : 58.4 : 51.1, 888 x 11222 -> 4096 124 : 147 : 123, 334 x 104 ->
+// 42211 42.0 : 28.7 : 40.7, 120 x 111 -> 62971 24.7 : 17.4 : 24.0.
 struct w8a32_kernel {
     unsigned bm, bn, resident, runs;  // rows, columns, workgroups a CU holds, parts of K within a workgroup (more than one: groups of rows)
-    double step[2], round, fixed, l2, weights, output, ragged, idle;
+    double step[2], round, fixed, l2, weights, output, ragged, idle, past;
 };
-constexpr w8a32_kernel W8A32[] = {{32, 64, 2, 1, {0.355, 0.394}, 1.94, 2.37, 0.0567, 0.126, 0.500, 0.0, 0.020},
-                                  {32, 128, 1, 1, {0.486}, 2.93, 1.45, 0.0318, 0.230, 0.500, 0.0, 0.214},
-                                  {32, 128, 2, 1, {0.768, 0.757}, 1.46, 2.19, 0.0530, 0.100, 1.149, 0.048, 0.270},
-                                  {64, 128, 1, 1, {0.740}, 2.73, 1.43, 0.0475, 0.100, 1.285, 0.0, 0.170},
-                                  {128, 128, 1, 1, {1.301}, 3.29, 0.42, 0.0726, 0.100, 1.219, 0.536, 0.060},
-                                  {64, 256, 1, 1, {1.152}, 5.35, 0.0, 0.0723, 0.125, 1.154, 1.556, 0.090},
-                                  {16, 32, 1, 4, {0.748}, 0.93, 1.90, 0.0, 0.100, 0.500, 0.0, 0.193},
-                                  {16, 16, 1, 8, {1.127}, 0.0, 2.33, 0.0376, 0.100, 14.382, 0.999, 0.122},
-                                  {32, 32, 1, 4, {1.189}, 1.26, 1.98, 0.0, 0.100, 0.500, 0.0, 0.116},
-                                  {64, 64, 1, 1, {0.568}, 2.20, 1.93, 0.0, 0.226, 3.431, 0.0, 0.231}};
+constexpr w8a32_kernel W8A32[] = {{32, 64, 2, 1, {0.344, 0.385}, 1.507, 2.861, 0.049, 0.178, 0.530, 0.010, 0.018, 0.097},
+                                  {32, 128, 1, 1, {0.475}, 1.791, 2.658, 0.019, 0.214, 2.096, 0.010, 0.088, 0.100},
+                                  {32, 128, 2, 1, {0.759, 0.809}, 1.085, 2.877, 0.027, 0.199, 1.303, 0.073, 0.187, 0.100},
+                                  {64, 128, 1, 1, {0.665}, 2.633, 1.763, 0.021, 0.180, 0.776, 0.011, 0.092, 0.102},
+                                  {128, 128, 1, 1, {1.459}, 2.997, 2.415, 0.019, 0.290, 0.907, 0.213, 0.108, 0.120},
+                                  {64, 256, 1, 1, {1.130}, 3.679, 1.344, 0.043, 0.168, 0.446, 1.601, 0.022, 0.064},
+                                  {16, 32, 1, 4, {0.658}, 1.141, 1.793, 0.010, 0.096, 0.499, 0.010, 0.087, 0.100},
+                                  {16, 16, 1, 8, {1.068}, 0.011, 2.205, 0.036, 0.075, 20.211, 0.921, 0.087, 0.100},
+                                  {32, 32, 1, 4, {1.136}, 1.641, 1.820, 0.010, 0.098, 0.500, 0.010, 0.102, 0.100},
+                                  {64, 64, 1, 1, {0.465}, 1.608, 1.892, 0.017, 0.329, 1.600, 0.010, 0.040, 0.092}};
 // Up to 32 rows: the kernels of 16 and 32 rows a group (-1: the one that takes all rows in a workgroup, up to four wavefronts) from the K on
 // where eight runs of it, or 32 columns a workgroup, are the shorter walk; 110 products of 2 .. 32 rows.  us, before : now: 17 x 6011 -> 420
 // 17.2 : 10.9, 31 x 7127 -> 2249 20.0 : 16.3, 27 x 3326 -> 6259 19.2 : 15.5, 3 x 4650 -> 6594 17.5 : 12.9, 2 x 6124 -> 287 12.0 : 10.3;
@@ -1208,7 +1204,7 @@ static int pick_w8a32_few(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
 }
 static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w->k_pad / 128);
-    const double output = 1e-6 * (double)(m * w->cols), digits = 3.0 + 1.3e-6 * (double)(m * w->k_pad);  // (the launch before, in the margin's us)
+    const double output = 1e-6 * (double)(m * w->cols), past = std::max(0.0, output - 20.0);
     const double weights = 1e-6 * (double)(w->rows * w->cols), ragged = w->cols % 32 ? output : 0.0;
     auto estimate = [&](int i) {
         const w8a32_kernel &t = W8A32[i];
@@ -1216,18 +1212,16 @@ static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
         if (t.runs > 1) columns = (columns + 7) / 8 * 8;
         const size_t wgs = (m + t.bm - 1) / t.bm * columns;
         const double cu = fullest_cu(wgs, cus, t.resident, t.step, (kt + t.runs - 1) / t.runs, t.round, t.idle);
-        const double all = 128e-6 * (double)(wgs * kt) * (3 * t.bm + t.bn) * t.l2 + weights * t.weights + output * t.output + ragged * t.ragged;
+        const double all = 128e-6 * (double)(wgs * kt) * (3 * t.bm + t.bn) * t.l2 + weights * t.weights + output * t.output + ragged * t.ragged + past * t.past;
         const double c2 = cu * cu, a2 = all * all;
-        return digits + t.fixed + sqrt(sqrt(c2 * c2 + a2 * a2));
+        return t.fixed + sqrt(sqrt(c2 * c2 + a2 * a2));
     };
-    auto rounds = [&](size_t bm, size_t bn, size_t us) { return (((m + bm - 1) / bm) * ((w->cols + bn - 1) / bn) + cus - 1) / cus * us; };
-    const size_t c0 = rounds(64, 64, 18), c1 = rounds(64, 128, 24), c2 = rounds(128, 128, 40);
-    int best = c2 < c0 && c2 < c1 ? 4 : c1 < c0 ? 3 : 9;
-    double best_us = (m <= 700 ? 0.93 : 0.9) * estimate(best);
+    int best = -1;
+    double best_us = 0.0;
     for (int i = 0; i < (int)(sizeof(W8A32) / sizeof(W8A32[0])); ++i) {
         if (W8A32[i].runs > 1 && m > 512) continue;
         const double us = estimate(i);
-        if (us < best_us) {
+        if (best < 0 || us < best_us) {
             best = i;
             best_us = us;
         }
@@ -1282,12 +1276,12 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
         case 1: return tiles(launch_group<32, 128, 128, 3, 1, 4, 1, false, 3>);
         case 2: return tiles(launch_group<32, 128, 128, 2, 1, 4, 2, false, 3>);
         case 3: return tiles(launch_group<64, 128, 128, 3, 2, 4, 2, false, 3>);
-        case 4: return tiles(launch_group<128, 128, 128, 2, 4, 2, 2, false, 3>);
+        case 4: return tiles(launch_group<128, 128, 128, 2, 4, 4, 4, false, 3>);
         case 5: return tiles(launch_group<64, 256, 128, 2, 2, 4, 2, false, 3>);
         case 6: return groups(gemm_w8a8_skinny_kernel<3, 2, 4, 3, true, true>, 1, 2, 4, 3);
         case 7: return groups(gemm_w8a8_skinny_kernel<3, 1, 8, 2, true, true>, 1, 1, 8, 2);
         case 8: return groups(gemm_w8a8_skinny_kernel<6, 2, 4, 2, true, true>, 2, 2, 4, 2);
-        default: return tiles(launch_group<64, 64, 128, 3, 2, 2, 1, false, 3>);
+        default: return tiles(launch_group<64, 64, 128, 3, 4, 2, 2, false, 3>);
     }
 }
 

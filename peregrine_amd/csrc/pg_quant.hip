@@ -751,7 +751,7 @@ PG_API pg_status pg_gemv_w8a8_force_shape(pg_ctx *ctx, int wavefronts, int rows_
 // The reference's GPU numerics for the same call: f32 activations times dequantised weights,
 // f32 accumulate (matmul_dequant_i8, src/metal/shaders.rs:2329-2375).  Here the activations
 // become 23/24-bit fixed point per row (power-of-two scale), three byte-digit planes, and every weight fragment meets the
-// three of them on the int8 matrix cores (one launch; a large product two), exact in integers; the only roundings are the
+// three of them on the int8 matrix cores (one launch; beyond its 32-bit offsets two), exact in integers; the only roundings are the
 // activation step (at most 2^-23 of the row's absmax, none for values that are multiples of the scale) and the final f64 -> f32.
 PG_API pg_status pg_matmul_dequant_i8_dev(pg_ctx *ctx, const float *a_dev, size_t m, size_t k,
                                           const pg_qtensor *w, float *out_dev) {
@@ -764,7 +764,7 @@ PG_API pg_status pg_matmul_dequant_i8_dev(pg_ctx *ctx, const float *a_dev, size_
     // a digit plane holds -128 .. 127 (the carry-free split yields -128), a weight -127 .. 127: 128 * 127 * k < 2^31
     PG_CHECK_ARG(k <= 132104, "pg_matmul_dequant_i8: k = %zu would overflow the i32 digit sums", k);
     const size_t m_pad = pg_round_up(m, PG_MPAD), n = w->cols;
-    // One launch over the three digit planes, or, for large products (and under a tile override): the two
+    // One launch over the three digit planes, or, beyond its offsets (and under a tile override): the two
     // low planes as ONE product over the planes stacked row-wise (they lie back to back in the scratch, each m_pad rows;
     // the accumulator planes are then m_pad rows apart), and the third plane's product finishes the sum in its epilogue.
     const bool one = pg_gemm_w8a32_takes(ctx, w, m);

@@ -137,7 +137,8 @@ INT8_ROUTES = [
 ]
 INT8_SPLIT = {(36, 12871, 303), (34, 9736, 451), (71, 12547, 2629)}
 W8A32_ROUTES = [
-    (201, 2071, 1346, _tile(32, 64, 3)), (527, 1156, 1895, _tile(32, 128, 3)), (168, 84, 4949, _tile(32, 128, 2)), (305, 70, 3790, _tile(64, 128, 3)),
-    (539, 77, 3716, _tile(128, 128, 2)), (52, 70, 38752, _tile(64, 256, 2)), (162, 81, 39168, _tile(64, 256, 2)), (289, 216, 2022, _tile(64, 64, 3)),
-    (45, 834, 20, _rows(3, 1, 8, 2, 1)), (47, 70, 18, _rows(3, 2, 4, 3, 1)), (43, 390, 2670, _rows(6, 2, 4, 2, 1)),
+    (201, 2071, 1346, _tile(32, 64, 3)), (527, 1156, 1895, _tile(32, 128, 3)), (168, 84, 4949, _tile(64, 64, 3)), (305, 70, 3790, _tile(64, 128, 3)),
+    (539, 77, 3716, _tile(32, 128, 2)), (52, 70, 38752, _tile(64, 256, 2)), (162, 81, 39168, _tile(64, 256, 2)), (289, 216, 2022, _tile(64, 64, 3)),
+    (45, 834, 20, _rows(3, 1, 8, 2, 1)), (47, 70, 18, _rows(3, 1, 8, 2, 1)), (43, 390, 2670, _rows(6, 2, 4, 2, 1)),
+    (68, 71, 34073, _tile(32, 128, 2)), (248, 67, 11625, _tile(128, 128, 2)), (36, 2199, 1583, _rows(3, 2, 4, 3, 1)),
 ]

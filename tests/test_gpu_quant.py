@@ -566,7 +566,6 @@ def test_wire_record_straight_to_device(ctx, orc):
 
 
 W8A32_SHAPES = [(32, 128, 64), (1, 4096, 1024), (3, 200, 77), (70, 4096, 300), (191, 256, 130),
-                # from 192 rows the three digit planes run as one product over the stacked planes
                 (192, 512, 300), (256, 384, 256), (300, 1000, 520), (700, 256, 1000)]
 
 
@@ -595,13 +594,13 @@ def test_matmul_dequant_i8_vs_oracle(ctx, orc, m, k, n):
 
 
 def test_matmul_dequant_i8_combining_epilogue_on_every_tile(ctx, orc):
-    """From 192 rows the product of the plane of weight 65536 finishes the sum in its epilogue (it reads the other
-    two planes' accumulators).  Every tile shape of the matrix-core kernel in turn, on a ragged shape (the
-    bounds-checked epilogue at the edges, the straight-line one inside), and two shapes that the dispatcher
-    itself gives 256x256 tiles (whole tiles only, and ragged): exact small integers in, exact integers out, and
+    """Where the planes are stacked (beyond one launch's offsets; under a tile override) the product of the plane of weight
+    65536 finishes the sum in its epilogue (it reads the other two planes' accumulators).  Every tile shape of the matrix-core
+    kernel in turn, on a ragged shape (the bounds-checked epilogue at the edges, the straight-line one inside), and two
+    shapes of many 256x256 tiles (whole tiles only, and ragged): exact small integers in, exact integers out, and
     the float64 product as the bar for random data."""
     from peregrine_amd import quant, _ffi
-    for m, k, n, force in [(300, 256, 520, c) for c in TILES] + [(2048, 128, 5888, 0), (2050, 128, 5900, 0)]:
+    for m, k, n, force in [(300, 256, 520, c) for c in TILES] + [(2048, 128, 5888, 2), (2050, 128, 5900, 2)]:
         say(f"matmul_dequant_i8 m={m} k={k} n={n} tile override {force}")
         a = orc.rng_normal(21 + m, m * k)
         a.reshape(m, k)[:, :: max(1, k // 37)] *= 20
@@ -614,10 +613,7 @@ def test_matmul_dequant_i8_combining_epilogue_on_every_tile(ctx, orc):
         try:
             _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, force))
             got = quant.matmul_dequant_i8(a, m, k, qt, ctx).reshape(m, n)
-            if force:
-                assert last_tile(ctx)[:2] == TILES[force]
-            else:
-                assert last_tile(ctx)[:2] == (256, 256)
+            assert last_tile(ctx)[:2] == TILES[force]
             got_int = quant.matmul_dequant_i8(ai, m, k, qt_int, ctx).reshape(m, n)
         finally:
             _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, 0))
@@ -732,7 +728,7 @@ def test_matmul_dequant_i8_on_every_kernel(ctx, orc, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 256, 50257), (32, 384, 65536), (33, 130, 128256), (191, 256, 50257), (383, 128, 45825),
-                                   (192, 256, 50257)])   # (the last one: the low planes stacked)
+                                   (192, 256, 50257)])
 def test_matmul_dequant_i8_wide_weights(ctx, m, k, n):
     """W8A32 over a vocabulary's columns: exact small integers in, exact integers out, on rows and columns of every tile's
     beginning and end; and the float64 product there for random data."""

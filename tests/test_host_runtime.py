@@ -289,12 +289,19 @@ def test_w8a32_over_wide_weights_is_one_launch_in_the_planes_scratch(host, m, n)
     assert taken <= 1.25 * 3 * (m_pad * k + 4 * m_pad) + (2 << 20), taken
 
 
-@pytest.mark.parametrize("m,n,large", [(192, 46080, True), (191, 46080, False), (384, 23040, True), (383, 23040, False), (2048, 5888, True),
-                                       (2048, 5632, False), (192, 65537, False), (192, 98048, False), (192, 98049, True)])
-def test_w8a32_large_products_stack_their_low_planes(host, m, n, large):
-    """Both sides of each condition of the stacked form: 256x256 tiles that fill the part and are mostly rows."""
-    names, _ = dequant_i8_call(host, m, 256, n)
-    assert len(names) == (3 if large else 2), names
+@pytest.mark.parametrize("m,k,n", [(192, 256, 46080), (191, 256, 46080), (384, 256, 23040), (2048, 256, 5888), (192, 256, 98049), (1000, 4096, 4096), (2048, 4096, 14336)])
+def test_w8a32_large_products_are_one_launch(host, m, k, n):
+    """Products that fill the part with 256x256 tiles that are mostly rows: as three launches over stacked planes 69 us where one takes 22
+    (192 x 256 -> 46080), 382 : 293 (2048 x 4096 -> 14336), 115 : 51 (1000 x 4096 -> 4096)."""
+    names, _ = dequant_i8_call(host, m, k, n)
+    assert len(names) == 2, names
+
+
+@pytest.mark.parametrize("m,k,stacked", [(8192, 130048, False), (8192, 130049, True), (7936, 132104, False), (8193, 130048, True)])
+def test_w8a32_products_beyond_one_launchs_offsets_stack_their_low_planes(host, m, k, stacked):
+    """Both sides of the line: two planes of the padded rows and 128 rows of weights within 2^31 bytes."""
+    names, _ = dequant_i8_call(host, m, k, 64)
+    assert len(names) == (3 if stacked else 2), names
 
 
 def test_memory_running_out_empties_the_pool_for_every_allocation(host):
@@ -367,12 +374,21 @@ def test_memory_another_context_has_used_is_not_pooled(host, users):
     host.lib.pg_ctx_destroy(other)
 
 
-@pytest.mark.parametrize("m,k,n,tile", [(197, 1024, 4096, (64, 64)), (356, 4096, 14336, (64, 128)), (1000, 4096, 4096, (128, 128)), (311, 2048, 32000, (64, 128)),
-                                        (155, 1024, 103918, (64, 128)), (888, 11222, 4096, (128, 128))])
-def test_w8a32_tile_is_the_one_that_took_least(host, m, k, n, tile):
-    """Of 64x64, 64x128 and 128x128; another kernel has to be estimated below 0.93 of it (past 700 rows 0.9)."""
+@pytest.mark.parametrize("m,k,n,tiles", [
+    (197, 1024, 4096, ["64ELi64ELi128ELi3ELi4ELi2E"]),                             # 10.3 us on eight wavefronts; on four 11.1, 32x128 10.8
+    (356, 4096, 14336, ["64ELi128E"]),                                             # 78; 64x256 87
+    (1000, 4096, 4096, ["64ELi256E"]),                                             # 51; 64x128 59, 128x128 58
+    (311, 2048, 32000, ["64ELi128E", "64ELi256E"]),                                # 75 and 74; 32x128 86
+    (155, 1024, 103918, ["64ELi128E", "32ELi128ELi128ELi2E", "64ELi256E"]),        # 89, 89 and 90; the next 107
+    (888, 11222, 4096, ["64ELi256E"]),                                             # 123; 64x128 132
+    (334, 104, 42211, ["128ELi128ELi128ELi2ELi4ELi4E"]),                           # 28.7 on sixteen wavefronts; on eight 42.0, 64x128 33.4
+    (120, 111, 62971, ["128ELi128ELi128ELi2ELi4ELi4E"]),                           # 17.4; 24.7, 20.4
+    (467, 8337, 534, ["32ELi64E"]),                                                # 37.2; 64x64 42.2
+])
+def test_w8a32_tile_is_the_one_that_took_least(host, m, k, n, tiles):
+    """Or one within 2 % of it (us, beside each)."""
     names, _ = dequant_i8_call(host, m, k, n)
-    assert len(names) == 2 and "gemm_w8a8_kernelILi%dELi%dE" % tile in names[1], names
+    assert len(names) == 2 and any("gemm_w8a8_kernelILi" + t in names[1] for t in tiles), names
 
 
 def int8_call(host, m, k, ns):
@@ -439,7 +455,7 @@ def test_the_tested_int8_kernels_are_all_there_are():
     assert len({r[3] for r in H.INT8_ROUTES}) == 8 + 9 and len({r[3] for r in H.W8A32_ROUTES}) == 10   # (256x256: the prefill shapes)
 
 
-@pytest.mark.parametrize("code,bm,bn", [(0, 256, 256), (1, 64, 64), (2, 256, 256), (3, 128, 256), (4, 128, 64), (5, 128, 128), (6, 256, 256), (7, 256, 256), (8, 256, 256)])
+@pytest.mark.parametrize("code,bm,bn", [(1, 64, 64), (2, 256, 256), (3, 128, 256), (4, 128, 64), (5, 128, 128), (6, 256, 256), (7, 256, 256), (8, 256, 256)])
 def test_w8a32_last_pass_by_tile_override(host, code, bm, bn):
     host.ok("pg_gemm_w8a8_force_tile", host.ctx, code)
     names, _ = dequant_i8_call(host, 2048, 128, 5888)
