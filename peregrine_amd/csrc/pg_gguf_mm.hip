@@ -1248,11 +1248,16 @@ pg_status pg_launch_q41_offset(pg_ctx *ctx, const pg_gguf_tensor *w, const float
     const size_t stride = rows * w->n_out;
     if (rows > 64) {
         if ((rows + 63) / 64 > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_matmul: too many activation rows");
-        // Few tiles and steps enough to share out: us of the whole product, side by side : RUNS, 70 x 9760 -> 2282 (36 workgroups, 39 steps)
+        // Few tiles and steps enough to share out; the more tiles there are, the more steps it takes, since what four runs of a tile add is
+        // their sums' way through LDS and four times the reads of the rows' sums.  Both timed on 2900 products: to 128 workgroups (half
+        // the CUs) from 4 steps on 0.95 of the time and less, to 192 from 5 on none longer (4: 1.04), beyond, at 4 to 6 steps 1.07 to 1.12, at 9 to 16 about
+        // even, from 17 on 0.97 and less, past 384 no rule.  us of the whole product, side by side : RUNS, 70 x 9760 -> 2282 (36 workgroups, 39 steps)
         // 61.8 : 38.5, 129 x 14336 -> 4096 (96, 56) 100.5 : 78.8, 514 x 7040 -> 1330 (99, 28) 73.3 : 62.2, 256 x 4096 -> 4096 (128, 16) 47.4 : 41.1,
-        // 1008 x 1216 -> 972 (128, 5) 28.3 : 27.0, 1024 x 14336 -> 3072 (384, 56) 293 : 286; but 512 x 4096 -> 8192 (512, 16) 118.7 : 119.8,
-        // 1000 x 4096 -> 14336 (1792, 16) 297 : 304, and of two steps 200 x 512 -> 14336 (448) 25.8 : 29.4.
-        const bool runs = nb > 24 && (size_t)grid_for(w->n_out, 128) * ((rows + 63) / 64) * 2 <= 3 * (size_t)ctx->num_cu;
+        // 1008 x 1216 -> 972 (128, 5) 28.3 : 27.0, 1024 x 14336 -> 3072 (384, 56) 293 : 286; but 171 x 960 -> 13241 (312, 4) 37.0 : 41.3, 413 x 1184 ->
+        // 5268 (294, 5) 37.0 : 40.0, 512 x 4096 -> 8192 (512, 16) 118.7 : 119.8, 1000 x 4096 -> 14336 (1792, 16) 297 : 304, and of two steps 200 x 512 ->
+        // 14336 (448) 25.8 : 29.4.
+        const size_t wgs = (size_t)grid_for(w->n_out, 128) * ((rows + 63) / 64), cus = (size_t)ctx->num_cu;
+        const bool runs = 2 * wgs <= cus ? nb > 24 : 4 * wgs <= 3 * cus ? nb > 32 : 2 * wgs <= 3 * cus && nb > 128;
         return pg_launch(ctx, "gguf_q4_1_offsets", runs ? q41_offset_mfma_kernel<true> : q41_offset_mfma_kernel<false>,
                          dim3(grid_for(w->n_out, runs ? 32 : 128), (unsigned)((rows + 63) / 64)), dim3(256), 0,
                          (const uint16_t *)w->d, (const uint16_t *)w->m, (int)w->n_out, nb, xsum, nbp, (int)rows, part, ks, stride, y);

@@ -449,8 +449,10 @@ def test_gguf_q4_1_few_rows(ctx, orc, n_out, k_in, m):
 
 
 @pytest.mark.parametrize("n_out,k_in,m,runs", [
-    (33, 832, 65, True), (31, 1088, 129, True), (160, 1600, 66, True), (1100, 2112, 64 * 3 + 1, True), (6144, 896, 512, True),  # the last: 384 tiles
-    (95, 768, 65, False), (6144, 832, 513, False),                                                                              # few steps, many tiles
+    (33, 832, 65, True), (31, 1088, 129, True), (160, 1600, 66, True), (1100, 2112, 64 * 3 + 1, True),
+    (2048, 832, 512, True), (3072, 1088, 512, True), (6144, 4160, 512, True),                       # 128, 192 and 384 tiles, the least steps
+    (2049, 1024, 512, False), (3073, 1088, 512, False), (6144, 896, 512, False), (6144, 4096, 512, False), (6144, 4160, 513, False),   # one step or one tile too many
+    (95, 768, 65, False), (6144, 832, 513, False),                                                  # few steps, many tiles
 ])
 def test_gguf_q4_1_offsets_on_the_matrix_cores(ctx, orc, n_out, k_in, m, runs):
     """The offsets of 65 rows and more: a tile's blocks in four runs (quarters of 4, 5, 7 and 9 steps, some of them empty or short)

@@ -471,6 +471,27 @@ def test_w8a32_groups_of_rows_are_counted_by_xcd(host, m, k, n, kernel):
     assert kernel in names[1], names
 
 
+@pytest.mark.parametrize("n,k,m,runs", [
+    (70, 832, 65, True), (972, 1216, 1008, True), (2048, 832, 512, True), (2282, 9760, 70, True), (3072, 1088, 512, True), (3072, 14336, 1024, True),
+    (70, 768, 65, False), (2049, 1024, 512, False), (3073, 1088, 512, False), (13241, 960, 171, False), (5268, 1184, 413, False), (2895, 864, 738, False),
+    (6144, 4096, 512, False), (6144, 4160, 513, False), (14336, 512, 200, False),
+])
+def test_q4_1_offsets_in_runs_where_that_is_shorter(host, n, k, m, runs):
+    """Both sides of each line between four runs of a tile's blocks and four tiles side by side.  171 x 960 -> 13241 takes 37.0 us side by side and
+    41.3 in runs, 413 x 1184 -> 5268 37.0 and 40.0, 738 x 864 -> 2895 37.5 and 41.4."""
+    w = host.new("pg_gguf_upload", host.ctx, bytes(H.pack_q4_1(np.zeros(n * k, np.float32))), 3, n, k)
+    x, y = host.alloc(m * k), host.alloc(m * n)
+    host.ok("pg_gguf_hmm_force", host.ctx, 1)
+    host.lib.pghost_clear_launches()
+    host.ok("pg_gguf_matmul_dev", host.ctx, x, m, w, y)
+    names = [name for name, _ in host.launches() if "q41_offset" in name]
+    assert len(names) == 1 and ("q41_offset_mfma_kernelILb%dE" % runs) in names[0], names
+    host.ok("pg_gguf_hmm_force", host.ctx, 0)
+    for p in (x, y):
+        host.ok("pg_dev_free", host.ctx, p)
+    host.lib.pg_gguf_free(host.ctx, w)
+
+
 def same_call_captured(host, name, *args):
     """A call that has run once at its shape is captured whole, as launches alone."""
     host.ok(name, host.ctx, *args)
