@@ -180,6 +180,7 @@ extern "C" {
     pub fn pg_probe_gemm_clock(ctx: *mut pg_ctx, m: usize, k: usize, n: usize, clock_ghz: *mut f64, loop_us: *mut f64) -> pg_status;
     pub fn pg_gemm_w8a8_last_tile(ctx: *const pg_ctx, bm: *mut c_int, bn: *mut c_int, k_splits: *mut c_int) -> pg_status;
     pub fn pg_gemm_w8a8_force_tile(ctx: *mut pg_ctx, tile: c_int) -> pg_status;
+    pub fn pg_gemm_w8a8_last_order(ctx: *const pg_ctx, row_tiles: *mut c_int, strip: *mut c_int) -> pg_status;
     pub fn pg_gemv_w8a8_force_shape(ctx: *mut pg_ctx, wavefronts: c_int, rows_per_wavefront: c_int) -> pg_status;
     pub fn pg_gguf_hmm_force(ctx: *mut pg_ctx, mode: c_int) -> pg_status;
     pub fn pg_audit_gemv_w8a8_m1(k: usize, n: usize, nch: c_int, rows_per_wavefront: c_int, wavefronts: c_int, f32_row: c_int, w_end: *mut usize, w_bytes: *mut usize, x_end: *mut usize, x_bytes: *mut usize) -> pg_status;

@@ -598,6 +598,8 @@ pg_status pg_probe_gemm_clock(pg_ctx *ctx, size_t m, size_t k, size_t n, double 
  * bits (the W8A32 product's last pass has the first five, 256x256 for the others); tests use the pair to prove each kernel instantiation ran. */
 pg_status pg_gemm_w8a8_last_tile(const pg_ctx *ctx, int *bm, int *bn, int *k_splits);
 pg_status pg_gemm_w8a8_force_tile(pg_ctx *ctx, int tile);
+/* The order of that launch's tiles: its row tiles, and how many of them a strip holds (the last strip what is left). */
+pg_status pg_gemm_w8a8_last_order(const pg_ctx *ctx, int *row_tiles, int *strip);
 /* The one-row product that takes the activation row in f32: the workgroup shape (wavefronts per workgroup 4, 8 or
  * 16; weight rows per wavefront 1 or 2, not 16 x 2) instead of the dispatcher's choice by row length; 0, 0 =
  * automatic.  Every shape gives the same bits. */

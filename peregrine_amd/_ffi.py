@@ -66,6 +66,7 @@ SIGNATURES = {
     "pg_matmul_quantized_fixed_scratch_dev": [_vp, _vp, _sz, _sz, _vp, _vp],
     "pg_fixed_scratch_bytes": [],
     "pg_gemm_w8a8_last_tile": [_vp, C.POINTER(_int), C.POINTER(_int), C.POINTER(_int)],
+    "pg_gemm_w8a8_last_order": [_vp, C.POINTER(_int), C.POINTER(_int)],
     "pg_audit_gemv_w8a8_m1": [_sz, _sz, _int, _int, _int, _int, C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)],
     "pg_audit_gemm_w8a8_skinny": [_sz, _sz, _sz, _int, _int, _int, C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)],
     "pg_audit_gguf_gemv": [_sz, _sz, _int, _int, _int, _int, C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)],

@@ -428,6 +428,8 @@ pg_status launch_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const f
     ctx->gemm_last_bm = BM;
     ctx->gemm_last_bn = BN;
     ctx->gemm_last_splits = splits;
+    ctx->gemm_last_row_tiles = tiles_m;
+    ctx->gemm_last_strip = order.strip;
     PG_TRY(pg_launch(ctx, NP == 3 ? "gemm_w8a32" : "gemm_w8a8", kern, dim3(grid, (unsigned)splits), dim3(64 * NWM * NWN), lds, a_i8, (int)a_stride, order, grp,
                      (int)k_pad, a_scales, acc, (int)m, (int)k_pad, kt_per_split, (long long *)nullptr));
     return pg_launch_check("gemm_w8a8");

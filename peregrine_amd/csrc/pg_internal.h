@@ -92,9 +92,9 @@ struct pg_ctx {
     std::vector<moe_table> moe_tabs;
     // Kernels whose dynamic LDS limit was raised on this context's device (pg_allow_dynamic_lds).
     std::vector<std::pair<const void *, size_t>> lds_raised;  // kernels whose dynamic-LDS limit was raised, and to what
-    // W8A8 GEMM dispatch: the tile of the most recent launch (pg_gemm_w8a8_last_tile) and an
+    // W8A8 GEMM dispatch: the tile and the order of the most recent launch (pg_gemm_w8a8_last_tile, _last_order) and an
     // optional override of the dispatcher's choice (pg_gemm_w8a8_force_tile; 0 = automatic).
-    int gemm_last_bm = 0, gemm_last_bn = 0, gemm_last_splits = 0;
+    int gemm_last_bm = 0, gemm_last_bn = 0, gemm_last_splits = 0, gemm_last_row_tiles = 0, gemm_last_strip = 0;
     int gemm_force_tile = 0;
     int gemv_force_nw = 0, gemv_force_rpw = 0;  // pg_gemv_w8a8_force_shape (0 = the dispatcher chooses)
     int hmm_mode = 0;  // pg_gguf_hmm_force: 0 = the dispatcher chooses, 1 = the f16 matrix-core product wherever it can run, 2 = never

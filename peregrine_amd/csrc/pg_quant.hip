@@ -730,6 +730,13 @@ PG_API pg_status pg_gemm_w8a8_last_tile(const pg_ctx *ctx, int *bm, int *bn, int
     return PG_OK;
 }
 
+PG_API pg_status pg_gemm_w8a8_last_order(const pg_ctx *ctx, int *row_tiles, int *strip) {
+    PG_CHECK_ARG(ctx != nullptr, "null context");
+    if (row_tiles) *row_tiles = ctx->gemm_last_row_tiles;
+    if (strip) *strip = ctx->gemm_last_strip;
+    return PG_OK;
+}
+
 PG_API pg_status pg_gemm_w8a8_force_tile(pg_ctx *ctx, int tile) {
     PG_CHECK_ARG(ctx != nullptr, "null context");
     PG_CHECK_ARG(tile >= 0 && tile <= 8, "pg_gemm_w8a8_force_tile: tile %d (0 .. 8)", tile);

@@ -467,10 +467,10 @@ def test_int8_tiles_store_whole_and_cut_tiles(ctx, orc, semantics, m, k, n):
 
 
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7, 8, "w8a32"])
-@pytest.mark.parametrize("m,n", [(4300, 2690), (1030, 5000)])
+@pytest.mark.parametrize("m,n", [(4300, 2690), (1030, 5000), (3221, 300)])
 def test_int8_tiles_in_strips(ctx, tile, m, n):
-    """Every tile shape over more row tiles than a strip holds, the last strip shorter: each tile is made once, where it belongs.  Small
-    integers: every result is exact."""
+    """Every tile shape over more row tiles than a strip holds, the last strip shorter (1030 rows: with and without strips): each tile is made
+    once, where it belongs.  Small integers: every result is exact."""
     from peregrine_amd import quant, _ffi
     say(f"int8 tiles in strips {tile} m={m} n={n}")
     k = 70
@@ -489,6 +489,10 @@ def test_int8_tiles_in_strips(ctx, tile, m, n):
         finally:
             _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, 0))
     assert (dout.to_host(np.float32).reshape(m, n) == a @ qi.astype(np.float32)).all()   # |sums| < 2^24: exact in any order
+    row_tiles, strip = C.c_int(), C.c_int()
+    _ffi.check(_ffi.lib.pg_gemm_w8a8_last_order(ctx.handle, C.byref(row_tiles), C.byref(strip)))
+    if m > 1030:
+        assert strip.value < row_tiles.value and (tile == "w8a32" or row_tiles.value % strip.value), (row_tiles.value, strip.value)
     qt.free_gpu()
 
 
