@@ -171,8 +171,8 @@ class Bench:
     def traffic_for(kernel, grids):
         """HBM bytes per launch of a kernel family: the committed rocprofv3 --pmc figures per launch
         size, weighted by the launches this run made of each size -- but only while those sizes are
-        exactly the ones the counters were taken on; otherwise None (the kernel or its dispatch
-        changed since: the summary is stale)."""
+        exactly the ones the counters were taken on; otherwise None (the dispatch changed since).  A kernel
+        that changes at the same sizes asks for its counters again: nothing here sees that."""
         got = grids.get(kernel, {})
         LAUNCHES_SEEN[kernel] = sorted(got)
         have = TRAFFIC.get(kernel)
@@ -203,8 +203,8 @@ class Bench:
                 "hbm_read_stream_gbs": round(gbs.value, 1), "gemm_tile_shader_clock_ghz": round(g_ghz.value, 3),
                 "gemm_tile_k_loop_us": round(loop_us.value, 2),
                 "int8_peak_at_gemm_clock_tops": round(256 * 8192 * g_ghz.value / 1e3, 1),
-                "note": "measured in this run by pg_probe_*: 8 wavefronts per CU issuing only v_mfma_i32_32x32x32_i8 on "
-                        "pseudo-random registers (the product's own 16x16x64 holds up to 4.0 POP/s so); 128-bit non-temporal reads over 3 x 256 MiB; shader cycles / wall clock "
+                "note": "measured in this run by pg_probe_*: 8 wavefronts per CU issuing only v_mfma_i32_16x16x64_i8 on "
+                        "pseudo-random registers; 128-bit non-temporal reads over 3 x 256 MiB; shader cycles / wall clock "
                         "inside the K loop of the 256x256 tile of a [2048x4096]x[4096x14336] product"}
 
 

@@ -573,8 +573,8 @@ pg_status pg_profile_get_grids(pg_ctx *ctx, size_t i, size_t *work_items, size_t
 /* Ceilings of the part, measured (no counterpart in the reference; a benchmark reports them
  * beside the published peaks):
  *   pg_probe_mfma_i8    int8 matrix-core rate with every operand in registers, in TOP/s (2 ops
- *                       per multiply-add), one workgroup of 8 wavefronts per CU for `iters` x 8
- *                       MFMAs per wavefront, and the shader clock the loop ran at;
+ *                       per multiply-add), one workgroup of 8 wavefronts per CU for `iters` x 32
+ *                       MFMAs (16x16x64) per wavefront, and the shader clock the loop ran at;
  *   pg_probe_hbm_read   a pure 128-bit read stream: `passes` kernels, each reading
  *                       bytes_per_pass from one of `buffers` distinct buffers in turn (make
  *                       buffers x bytes_per_pass exceed the 256 MB last-level cache), in GB/s;

@@ -10,40 +10,41 @@
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 
-// 8 wavefronts per workgroup, 2 x 4 accumulator tiles of 32x32 per wavefront: the register
+// 8 wavefronts per workgroup, 8 x 4 accumulator tiles of 16x16 per wavefront: the instruction and the register
 // shape of the 256x256 GEMM tile.  clk_out[2 * wg] = shader cycles, [2 * wg + 1] = wall ticks.
+constexpr int PROBE_TM = 8, PROBE_TN = 4;
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void probe_mfma_i8_kernel(int iters, const v4i *__restrict__ in, int *__restrict__ out, long long *__restrict__ clk_out) {
-    v4i a[2], b[4];
+    v4i a[PROBE_TM], b[PROBE_TN];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = in[threadIdx.x + i * 512];
+    for (int i = 0; i < PROBE_TM; ++i) a[i] = in[threadIdx.x + i * 512];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) b[j] = in[threadIdx.x + (2 + j) * 512];
-    v16i acc[2][4];
+    for (int j = 0; j < PROBE_TN; ++j) b[j] = in[threadIdx.x + (PROBE_TM + j) * 512];
+    v4i acc[PROBE_TM][PROBE_TN];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < PROBE_TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+        for (int j = 0; j < PROBE_TN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
     const long long c0 = clock64(), w0 = wall_clock64();
     for (int it = 0; it < iters; ++it) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < PROBE_TM; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], b[j], acc[i][j], 0, 0, 0);
-        asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));  // keep the loop
+            for (int j = 0; j < PROBE_TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i], b[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < PROBE_TM; ++i) asm volatile("" : "+v"(a[i]));  // keep the loop
+#pragma unroll
+        for (int j = 0; j < PROBE_TN; ++j) asm volatile("" : "+v"(b[j]));
     }
     const long long c1 = clock64(), w1 = wall_clock64();
     int s = 0;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < PROBE_TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < PROBE_TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s += acc[i][j][r];
+            for (int r = 0; r < 4; ++r) s += acc[i][j][r];
     out[blockIdx.x * 512 + threadIdx.x] = s;
     if (threadIdx.x == 0) {
         clk_out[2 * blockIdx.x] = c1 - c0;
@@ -99,10 +100,10 @@ PG_API pg_status pg_probe_mfma_i8(pg_ctx *ctx, int iters, double *tops, double *
     PG_CHECK_ARG(iters >= 1 && iters <= (1 << 20), "pg_probe_mfma_i8: iters %d", iters);
     const int wgs = ctx->num_cu;  // one workgroup of 8 wavefronts per CU: two per SIMD
     pg_tmp in, out, clk;
-    PG_TRY(in.alloc(ctx, 6 * 512 * sizeof(v4i)));
+    PG_TRY(in.alloc(ctx, (PROBE_TM + PROBE_TN) * 512 * sizeof(v4i)));
     PG_TRY(out.alloc(ctx, (size_t)wgs * 512 * sizeof(int)));
     PG_TRY(clk.alloc(ctx, (size_t)wgs * 2 * sizeof(long long)));
-    PG_TRY(pg_probe_fill_random(ctx, in.p, 6 * 512 * sizeof(v4i)));
+    PG_TRY(pg_probe_fill_random(ctx, in.p, (PROBE_TM + PROBE_TN) * 512 * sizeof(v4i)));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     PG_HIP(hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) { (void)hipEventDestroy(e0); return pg_fail(PG_EDEVICE, "hipEventCreate failed"); }
@@ -128,8 +129,8 @@ PG_API pg_status pg_probe_mfma_i8(pg_ctx *ctx, int iters, double *tops, double *
     PG_HIP(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, ctx->device));
     double cyc = 0.0, wall = 0.0;
     for (int i = 0; i < wgs; ++i) { cyc += (double)h[2 * i]; wall += (double)h[2 * i + 1]; }
-    // 8 wavefronts x 8 MFMAs x 32*32*32 multiply-adds x 2 ops per workgroup and iteration
-    if (tops) *tops = (double)wgs * 8.0 * 8.0 * 65536.0 * iters / (ms * 1e-3) / 1e12;
+    // 8 wavefronts x the MFMAs x 16*16*64 multiply-adds x 2 ops per workgroup and iteration
+    if (tops) *tops = (double)wgs * 8.0 * (PROBE_TM * PROBE_TN) * 32768.0 * iters / (ms * 1e-3) / 1e12;
     if (clock_ghz) *clock_ghz = wall > 0.0 && wall_khz > 0 ? cyc / (wall / (wall_khz * 1e3)) / 1e9 : 0.0;
     return PG_OK;
 }
