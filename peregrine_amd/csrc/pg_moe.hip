@@ -60,7 +60,11 @@ inline size_t route_lds(size_t T, size_t E, size_t top_k, bool logits) { return 
 // 422 tokens over 32 experts, top 4: layers of 422 tokens of 800 x 2752 117.0 : 108.5 us, 380 of 1024 x 1024 67.1 : 59.8, 512 of 2880 x 2880
 // 259.7 : 250.4, 400 of 512 x 640, top 2 47.0 : 41.5.)
 inline bool route_in_one(size_t T, size_t E, size_t top_k, bool logits) {
-    // (lists: a wavefront of the 16 takes every 16th expert and looks at 64 pairs at a time: 128 such steps, 4 us, at most)
+    // (Lists: a wavefront of the 16 takes every 16th expert and looks at 256 pairs at a time.  From 16 experts on that is 32 looks at the most; with fewer
+    // some wavefronts stand idle and the tokens count instead, up to 48 K entries read by one workgroup.  The three launches read them by as many
+    // wavefronts as tokens / 64, but their lists look at 64 pairs at a time, from memory.  us, three launches : one, over every T and k that the rule
+    // takes: 1 expert 12442 tokens 59 : 18, 2 of 2 117 : 39, 2 of 4 119 : 40, 1 of 8 62 : 21, 4 of 8 of 3687 74 : 30, 2 of 16 40 : 18, few tokens 8.9 : 6.5;
+    // past it 32 experts 0.7 to 1.0 of their time, 64 0.95 to 1.7, more 0.86 to 4.9.)
     return T * top_k * E <= (1u << 17) && route_lds(T, E, top_k, logits) <= MAX_ROUTE_LDS;
 }
 struct route_digits {

@@ -362,7 +362,8 @@ def test_mxfp4_moe_finds_the_expert_of_a_tile(ctx, orc, E, T):
     test_mxfp4_moe_routed_follows_the_oracle(ctx, orc, 64, 96, E, 3, T)
 
 
-@pytest.mark.parametrize("E,top_k,T,one", [(32, 4, 373, True), (32, 2, 422, True), (64, 6, 190, True), (64, 4, 512, True), (64, 4, 513, False), (256, 2, 256, True)])
+@pytest.mark.parametrize("E,top_k,T,one", [(32, 4, 373, True), (32, 2, 422, True), (64, 6, 190, True), (64, 4, 512, True), (64, 4, 513, False), (256, 2, 256, True),
+                                             (4, 2, 16384, True), (4, 2, 16385, False), (2, 2, 24576, True), (2, 2, 24577, False)])
 def test_mxfp4_moe_routing_in_one_launch(ctx, orc, E, top_k, T, one):
     """A routing whose table of logits would be more than the 48 KB that one launch takes, but which brings none: one launch up to
     2^17 looks at a pair, three beyond."""
