@@ -379,7 +379,7 @@ void gqa_attention_halves_kernel(const char *__restrict__ planes, int n_blocks, 
 // are then read from where the kernel above left them.  As a launch of its own behind this one the next product's input took 4 to 7 us: blocks of 711 tokens of
 // d 1024 (Q8_0) 126 : 121.5 us, 679 of 2048 256.5 : 251, 602 behind 1841 270 : 264.5, Q4_0 450 of 2048 214 : 208.5, 350 164.5 : 160.5; as f16 planes
 // 777 behind 100 of 4096 859 : 848 (the merge 9.8 + 6.2 : 10.9).
-// MOST: runs at the most; four take half the registers of sixteen, so that twice the wavefronts wait for memory at a time (the f16 planes 15 : 10.9).
+// MOST: runs at the most; four take a third of the registers of sixteen (34 : 106), so that twice the wavefronts wait for memory at a time (the f16 planes 15 : 10.9).
 constexpr int HALVES_RUNS_MAX = 16, HALVES_RUNS_FEW = 4;
 struct halves_next {
     int8_t *digits;

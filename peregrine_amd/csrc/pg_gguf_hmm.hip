@@ -383,7 +383,8 @@ pg_status pg_launch_rows_to_f16_planes(pg_ctx *ctx, const float *x_dev, size_t r
 // and 0.25 us per row tile; 3 us and 0.48 us per row tile go to the first loads and the results.  The conversion of
 // the rows (1.2 us per million values) and the pass over the chunks' planes (1.5 us per million values of each and of
 // their sum) come on top.  Fitted to 13 shapes (1024 to 14336 -> 1000 to 28672) at 48 to 1024 rows and every (mt, ks): 5 %
-// mean error, and the pair it picks takes 1 % longer than the best on average.
+// mean error, and the pair it picks takes 1 % longer than the best on average.  (Q4_1's chunks are read by its offsets' launch and no pass
+// over them follows: counted as the others' all the same, so its chunks are as many as a Q4_0 product's.)
 struct hmm_plan { int mt, ks; double us; };
 static hmm_plan hmm_plan_for(const pg_ctx *ctx, size_t m, size_t n_total, size_t k_in, int ks_fixed) {
     hmm_plan best = {8, 1, 1e300};

@@ -1476,7 +1476,9 @@ pg_status moe_product(pg_ctx *ctx, const float *src, size_t k_in, size_t n_out, 
 // 33.1 / 33.8, 10 tokens 37.3 / 32.2; of 2880, top 2, 10 tokens 60.1 / 47.3.  Both timed on 351 shapes, 4 to 30 experts,
 // hidden and inter 256 to 5760: 0.6 % over the faster one on average.  Where it errs: few output columns under a long K, which
 // the decode kernel streams at less than half that rate -- hidden 512, inter 3360 to 4096, 36 to 40 pairs 43-47 / 35 -- and
-// narrow experts of 2048 x 512, which would gain 15 % as pairs.  Such calls keep the finer digits they have.)
+// narrow experts of 2048 x 512, which would gain 15 % as pairs.  Such calls keep the finer digits they have.  The tiles' 27 and 20 us
+// hold a routing launch that up to 64 experts no longer have: 4 us less would move calls from the pairs' exact activations to the tiles'
+// digits, so the line stays where it was.)
 bool pairs_faster(size_t T, size_t E, size_t top_k, size_t hidden, size_t inter) {
     const double us_per_expert = 3.0 * (double)hidden * (double)inter * (17.0 / 32.0) / 1e6;  // at 1 TB/s
     const double hit = (double)E * (1.0 - pow(1.0 - (double)top_k / (double)E, (double)T));
