@@ -756,14 +756,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_f32_rows_kernel(const float
 }
 
 // From 33 rows on W8A8 has three routes, and each kernel of each an estimate of what the product takes with the quantisation before it, us;
-// the least is taken (pg_gemm_w8a8_route).  All were fitted together to 1150 single products (m 33 .. 4200, K 64 .. 16384, n 64 .. 131072, every
-// kernel of every route timed on each, the weights from HBM), least squares on the relative error, the more the nearer a kernel is to the
-// best, and in full where it would be taken wrongly.  The choice takes 0.9 % more than the best kernel on average to 64 rows, 1.7 % to 256, 1.2 % to
-// 700, 0.9 % beyond (4, 9, 6 and 5 % at the 95th percentile; a third of them against a fit to the others: 1.2, 2.0, 1.6, 0.8 % on average), and
-// 1 % on 197 groups of two and three weights that are in none of the fits.  A change to a kernel asks for all of it again.  Against the lines
-// and estimates that they replace (fitted to no more than 24000 columns, a CU's workgroups counted over the part): of 820 products over 8 us,
-// 137 more than 5 % faster, 18 that much slower.  us, those : these: 200 x 10240 -> 50257 197 : 165, 225 x 4026 -> 1099 17.4 : 12.5,
-// 64 x 1024 -> 50257 32 : 19, 62 x 5302 -> 14499 28.4 : 22.7, 111 x 7102 -> 49915 123 : 87; but 65 x 444 -> 92928 25.8 : 29.6.
+// the least is taken (pg_gemm_w8a8_route).  All were fitted together to two thirds of 9413 single products (m 33 .. 4200, K 64 .. 16384, n 64 ..
+// 131072, every kernel of every route timed on each, the weights from HBM): least squares on the relative error, the more the nearer a kernel is
+// to the best, then small changes of all numbers as long as the kernels taken are the shorter ones.  On the others the choice takes 1.3 % more than the
+// best kernel on average to 64 rows, 0.9 % to 256, 0.65 % to 700, 0.95 % beyond (5.9, 5.5, 4.1 and 6.0 % at the 95th percentile; of those over 8 us 0.8,
+// 0.55, 0.5 and 0.9 %).  With the numbers fitted to the same tiles on 32x32x32, all row tiles of a panel first, it was 2.0, 2.4, 2.2 and 2.3 % (11 to 12 % at the
+// 95th percentile).  11281 products drawn after the fit, both choices in turn: those over 8 us 0.986 of the time, 1025 of 7475 more than 5 % faster, 115
+// that much slower; shorter ones the same.  A change to a kernel asks for all of it again.  us, those numbers : these: 288 x 117 -> 97561 47.4 : 32.5, 544 x 71 ->
+// 49642 43.1 : 31.1, 530 x 631 -> 65280 89 : 72, 1779 x 512 -> 6406 26.0 : 20.5, 184 x 11725 -> 6400 59 : 46, 99 x 9010 -> 1029 20.8 : 15.9; but 4080 x 128 -> 31781
+// 146 : 175, 34 x 88 -> 118016 15.6 : 18.5, 34 x 10342 -> 4044 17.6 : 20.5.
 //
 // The tiles: the longer of what the fullest CU does (its tiles one after another, as many as its LDS holds at a time: a step of 128 of
 // K by how many are resident, and a round's ends; less of it in proportion to the places that the rounds leave empty, which the
@@ -780,15 +781,15 @@ struct tile_kernel {
     unsigned bm, bn, resident;  // (workgroups a CU holds)
     double step[3], round, fixed, l2, weights, output, ragged, idle, past;  // per MB through L2, M weights, M outputs, M of them off the lines, past 20 M
 };
-constexpr tile_kernel TILES[] = {{1, 64, 64, 3, {0.309, 0.425, 0.380}, 0.960, 3.04, 0.0485, 0.139, 0.500, 0.037, 0.290, 0.744},  // three stages
-                                 {2, 256, 256, 1, {1.587}, 8.972, 4.36, 0.0543, 0.146, 0.548, 0.287, 0.308, 0.100},
-                                 {3, 128, 256, 1, {0.928}, 4.625, 3.29, 0.0432, 0.152, 0.636, 0.313, 0.175, 0.011},
-                                 {4, 128, 64, 2, {0.436, 0.710}, 1.607, 2.49, 0.0314, 0.191, 0.566, 0.174, 0.309, 0.667},
-                                 {5, 128, 128, 1, {0.589}, 2.936, 2.22, 0.0289, 0.194, 0.647, 0.362, 0.240, 0.030},
-                                 {6, 128, 192, 1, {0.759}, 3.683, 3.16, 0.0338, 0.197, 0.698, 0.345, 0.214, 0.006},
-                                 {7, 256, 128, 1, {1.010}, 4.271, 1.76, 0.0487, 0.140, 0.562, 0.225, 0.312, 0.108},
-                                 {8, 256, 192, 1, {1.226}, 7.611, 3.84, 0.0523, 0.200, 0.500, 0.361, 0.232, 0.132},
-                                 {1, 64, 64, 2, {0.291, 0.419}, 1.251, 2.36, 0.0389, 0.149, 0.500, 0.242, 0.239, 0.778}};  // four stages
+constexpr tile_kernel TILES[] = {{1, 64, 64, 3, {0.340, 0.592, 0.557}, 1.197, 2.691, 0.040, 0.138, 0.611, 0.164, 0.141, 0.183},  // three stages
+                                 {2, 256, 256, 1, {1.429}, 7.369, 3.296, 0.052, 0.104, 0.678, 0.119, 0.009, 0.044},
+                                 {3, 128, 256, 1, {0.926}, 4.890, 2.368, 0.026, 0.168, 0.678, 0.174, 0.137, 0.083},
+                                 {4, 128, 64, 2, {0.451, 0.749}, 2.043, 2.399, 0.006, 0.202, 0.706, 0.306, 0.098, 0.006},
+                                 {5, 128, 128, 1, {0.552}, 3.716, 2.376, 0.014, 0.173, 0.814, 0.319, 0.157, 0.018},
+                                 {6, 128, 192, 1, {0.750}, 4.252, 2.324, 0.022, 0.162, 0.628, 0.346, 0.194, 0.0},
+                                 {7, 256, 128, 1, {0.950}, 4.112, 2.229, 0.031, 0.134, 0.696, 0.156, 0.198, 0.004},
+                                 {8, 256, 192, 1, {1.306}, 6.499, 3.026, 0.036, 0.152, 0.530, 0.234, 0.133, 0.190},
+                                 {1, 64, 64, 2, {0.342, 0.478}, 0.960, 2.630, 0.023, 0.160, 0.941, 0.227, 0.152, 0.196}};  // four stages
 constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
 double quantise_us(const pg_qtensor *w, size_t m) { return 3.0 + 0.8e-6 * (double)(m * w->rows); }
 // What the fullest CU takes for its share of `wgs` workgroups of `steps` steps, `resident` of them at a time.
@@ -871,7 +872,7 @@ pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const 
 
 // Some dozens of rows over few columns or a long K (33 .. 256): one or two tiles of activations against every weight row is far too few
 // workgroups to stream the weights (64 on 256 CUs at N = 4096), so K is split until every place of a CU is taken, not one more
-// (a workgroup too many is a round); the partial i32 sums go to `part` ([splits][m][n]) and a second launch adds them and applies the
+// (a workgroup too many is a round: 82 tiles in three runs are 33 workgroups for an XCD's 32 CUs, and 157 x 9208 -> 5214 took 42.7 us so); the partial i32 sums go to `part` ([splits][m][n]) and a second launch adds them and applies the
 // scales.  128x128 tiles with eight wavefronts, one a CU, or 64x64 of four stages, two a CU: over 36 products (K 9300 .. 14300) 0.87 of the time of
 // 64x128 and 128x128 tiles of four wavefronts, split beyond the places.  us, those : these: 135 x 10836 -> 628 21.4 : 18.5, 213 x
 // 13535 -> 1432 34.0 : 25.8, 96 x 12787 -> 2221 31.6 : 22.8, 87 x 12661 -> 4291 45.4 : 32.4, 46 x 13300 -> 9512 44.1 : 39.7.
@@ -881,12 +882,12 @@ struct split_kernel {
     unsigned tile, resident;
     double step[2], round, fixed, l2, weights, parts, idle;  // parts: per M of partial sums
 };
-constexpr split_kernel SPLITS[] = {{128, 1, {0.646}, 0.0, 6.60, 0.0, 0.185, 2.356, 0.0}, {64, 2, {0.775, 0.426}, 1.375, 3.67, 0.0508, 0.129, 2.403, 0.0}};
+constexpr split_kernel SPLITS[] = {{128, 1, {0.567}, 0.0, 8.919, 0.002, 0.198, 1.218, 0.161}, {64, 2, {0.649, 0.619}, 1.467, 4.862, 0.021, 0.175, 1.602, 0.074}};
 // The runs of K, none of them empty, and the k-tiles of one.
 unsigned split_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, const split_kernel &s, unsigned *per) {
     const size_t tiles = ((m + s.tile - 1) / s.tile) * ((w->cols + s.tile - 1) / s.tile), kt = w->k_pad / 128;
-    // (at least two k-tiles a run)
-    const size_t runs = std::max<size_t>(1, std::min<size_t>({s.resident * (size_t)ctx->num_cu / tiles, kt / 2, 16}));
+    // (the places of an XCD, which has all runs of its tiles; at least two k-tiles a run)
+    const size_t runs = std::max<size_t>(1, std::min<size_t>({s.resident * (size_t)(ctx->num_cu / 8) / ((tiles + 7) / 8), kt / 2, 16}));
     *per = (unsigned)((kt + runs - 1) / runs);
     return (unsigned)((kt + *per - 1) / *per);
 }
@@ -921,15 +922,14 @@ struct few_rows_shape {
     int mb, nb, nst, nw;
     double fixed, rows, round, run, loads, output, weights;
 };
-constexpr few_rows_shape FEW_ROWS_SHAPES[] = {{2, 1, 2, 2, 4.432, 0.831, 1.238, 0.528, 9.694, 2.673, 0.122},
-                                              {2, 1, 3, 4, 4.793, 1.442, 1.463, 0.080, 13.909, 0.837, 0.094},
-                                              {2, 1, 3, 8, 4.937, 1.323, 1.189, 0.0, 14.333, 3.440, 0.117},
-                                              {2, 2, 2, 4, 4.587, 1.174, 1.253, 0.590, 9.910, 3.003, 0.120},
-                                              {2, 2, 2, 8, 4.630, 1.283, 1.316, 0.324, 14.129, 3.255, 0.082},
-                                              {3, 1, 2, 8, 4.754, 1.333, 1.235, 0.317, 12.997, 4.109, 0.082},
-                                              {3, 2, 2, 4, 4.815, 1.023, 1.662, 0.593, 12.034, 3.146, 0.071},
-                                              {3, 2, 2, 8, 4.739, 1.238, 1.548, 0.353, 14.674, 3.660, 0.059},
-                                              {4, 2, 3, 4, 4.903, 1.548, 2.224, 0.303, 12.576, 4.001, 0.056}};
+constexpr few_rows_shape FEW_ROWS_SHAPES[] = {{2, 1, 2, 2, 4.600, 1.442, 1.091, 0.492, 8.976, 2.591, 0.155},
+                                              {2, 1, 3, 4, 4.637, 1.471, 1.497, 0.070, 14.408, 0.802, 0.089},
+                                              {2, 1, 3, 8, 4.879, 1.481, 1.061, 0.105, 14.198, 0.612, 0.100},
+                                              {2, 2, 2, 4, 4.503, 1.492, 1.339, 0.569, 9.513, 2.846, 0.151},
+                                              {2, 2, 2, 8, 4.514, 1.504, 1.448, 0.204, 14.012, 3.082, 0.110},
+                                              {3, 1, 2, 8, 4.573, 1.330, 1.483, 0.254, 12.679, 2.967, 0.128},
+                                              {3, 2, 2, 8, 4.803, 1.511, 1.697, 0.466, 13.553, 3.098, 0.081},
+                                              {4, 2, 3, 4, 4.685, 1.642, 2.404, 0.373, 11.769, 3.638, 0.085}};
 }  // namespace
 
 // The route of a product of m rows over `count` weights side by side: 2 to 32 rows the few-row kernel, all rows in a workgroup
@@ -977,7 +977,7 @@ pg_w8a8_route pg_gemm_w8a8_route(const pg_ctx *ctx, const pg_qtensor *const *w, 
             const unsigned runs = split_runs(ctx, w[0], m, s, &per);
             if (runs < 2) continue;
             const size_t tiles = ((m + s.tile - 1) / s.tile) * ((cols + s.tile - 1) / s.tile);
-            const double cu = fullest_cu(tiles * runs, (unsigned)ctx->num_cu, s.resident, s.step, per, s.round, s.idle);
+            const double cu = fullest_cu((tiles + 7) / 8 * 8 * runs, (unsigned)ctx->num_cu, s.resident, s.step, per, s.round, s.idle);
             const double all = 128e-6 * (double)(tiles * (k_pad / 128)) * (2 * s.tile) * s.l2 + weights * s.weights;
             const double c2 = cu * cu, a2 = all * all;
             better(quantise_us(w[0], m) + s.fixed + sqrt(sqrt(c2 * c2 + a2 * a2)) + 1e-6 * (double)(m * cols * runs) * s.parts, PG_W8A8_SPLIT, i);
@@ -1075,7 +1075,7 @@ pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size
         const dim3 grid((unsigned)((wgs + 7) / 8 * 8 * groups));
 #define PG_GROUPS(MBB, NBB, NSTT, NWW) PG_SKINNY(MBB, NBB, NSTT, NWW, false, true)
         PG_GROUPS(2, 1, 2, 2) PG_GROUPS(2, 1, 3, 4) PG_GROUPS(2, 1, 3, 8) PG_GROUPS(2, 2, 2, 4) PG_GROUPS(2, 2, 2, 8)
-        PG_GROUPS(3, 1, 2, 8) PG_GROUPS(3, 2, 2, 4) PG_GROUPS(3, 2, 2, 8) PG_GROUPS(4, 2, 3, 4)
+        PG_GROUPS(3, 1, 2, 8) PG_GROUPS(3, 2, 2, 8) PG_GROUPS(4, 2, 3, 4)
 #undef PG_GROUPS
         return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8 (groups of rows in one launch): no kernel of %d tiles, %d stages, %d wavefronts", sh.nb, sh.nst, sh.nw);
     }

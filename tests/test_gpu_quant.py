@@ -280,7 +280,8 @@ PREFILL_SHAPES = [
     ("k/v_proj", 2048, 4096, 1024, (128, 64)),
     ("gate/up_proj", 2048, 4096, 14336, (256, 256)),
     ("down_proj", 2048, 14336, 4096, (128, 256)),
-    ("unsplit 128x128", 1024, 256, 4096, (128, 128)),
+    ("unsplit 128x128", 1024, 1024, 4096, (128, 128)),
+    ("two steps of K", 1024, 256, 4096, (128, 64)),
 ]
 
 

@@ -431,11 +431,26 @@ def rows_in_groups(mb, nb, nw, nst):
     (62, 5302, [14499], tile(64, 64), False),                         # 22.7; 28.4
     (163, 12022, [6319], tile(128, 128), True),                       # 43.1; 58.2 on 64x64
     (132, 9671, [2828, 7938], tile(64, 64), False),                   # 50; 70 with one apart
+    (288, 117, [97561], tile(256, 256), False),                       # 32.5; 47.4 on 64x64
+    (544, 71, [49642], tile(128, 256), False),                        # 31.1; 43.1 on 64x64
+    (530, 631, [65280], tile(256, 256), False),                       # 71.7; 89.4 on 128x256
+    (1779, 512, [6406], tile(256, 192), False),                       # 20.5; 26.0 on 256x128
+    (184, 11725, [6400], tile(128, 128), True),                       # 45.7; 59.0 on 64x64
+    (99, 9010, [1029], rows_in_groups(3, 1, 8, 2), False),            # 15.9; 20.8 on 64x64, K split
 ])
 def test_int8_product_of_some_rows_takes_a_kernel_that_was_clearly_faster(host, m, k, ns, kernel, finish):
     """Products of which another kernel took at least a tenth longer than this one (us, both sides beside them)."""
     names = int8_call(host, m, k, ns)
     assert kernel in names[1] and len(names) == 2 + finish and ("splitk_finish" in names[-1]) == finish, names
+
+
+@pytest.mark.parametrize("m,k,n,resident", [(195, 15812, 3090, 1), (200, 15888, 3081, 1), (33, 13376, 2060, 2), (34, 13823, 2079, 2), (65, 11004, 8720, 1)])
+def test_int8_runs_of_k_are_as_many_as_an_xcd_has_places(host, m, k, n, resident):
+    """An XCD has all runs of every eighth tile; counted over the part, 50 tiles in five runs are 35 workgroups for its 32 CUs."""
+    names = int8_call(host, m, k, [n])
+    assert len(names) == 3 and "splitk_finish" in names[2], names
+    tiles, runs = host.launches()[1][1][:2]
+    assert tiles % 8 == 0 and 2 <= runs and tiles // 8 * runs <= 32 * resident, (tiles, runs)
 
 
 @pytest.mark.parametrize("m,k,n,kernel", H.INT8_ROUTES)
@@ -452,7 +467,7 @@ def test_w8a32_products_run_on_the_kernels_that_they_are_tested_on(host, m, k, n
 
 
 def test_the_tested_int8_kernels_are_all_there_are():
-    assert len({r[3] for r in H.INT8_ROUTES}) == 8 + 9 and len({r[3] for r in H.W8A32_ROUTES}) == 10   # (256x256: the prefill shapes)
+    assert len({r[3] for r in H.INT8_ROUTES}) == 8 + 8 and len({r[3] for r in H.W8A32_ROUTES}) == 10   # (256x256: the prefill shapes)
 
 
 @pytest.mark.parametrize("code,bm,bn", [(1, 64, 64), (2, 256, 256), (3, 128, 256), (4, 128, 64), (5, 128, 128), (6, 256, 256), (7, 256, 256), (8, 256, 256)])
