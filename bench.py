@@ -394,7 +394,7 @@ def main():
         t32 = B.timed(w8a32_step, args.steps, args.warmup)
         prof32, _ = B.profiled(w8a32_step, args.steps)
         line["w8a32_gate"] = {"workload": "W8A32 product [2048x4096] x [4096x14336] (f32 activations, dequantised i8 weights, f32 accumulate): "
-                                          "three int8 digit planes of 24-bit fixed-point activations: the two low planes as one matrix-core launch, the high plane's launch finishes the sum in its epilogue",
+                                          "three int8 digit planes of 24-bit fixed-point activations, which every weight fragment meets in one matrix-core launch",
                               "value": round(2 * M_PREFILL * 4096 * 14336 / (t32["ms_per_step"] * 1e-3) / 1e12, 1), "unit": "TFLOP/s",
                               **B.stats(t32, 4), "kernels_ms": {k: round(v[0], 5) for k, v in prof32.items()}}
     for ws in weight_sets:
