@@ -8,7 +8,7 @@
 // used for A and B, so the sum is over matching k.
 //
 // Why 16x16x64 and not 32x32x32: on a full chip the power limit sets the rate, and for the same multiply-adds it writes
-// half the accumulators.  On random bytes in registers it holds 3.9 to 4.0 POP/s, 32x32x32 3.5 (5.0 both on zeros); the
+// half the accumulators.  On random bytes in registers it holds 3.9 to 4.1 POP/s (pg_probe_mfma_i8), 32x32x32 3.5 (5.0 both on zeros); the
 // fragments read from LDS are as many.  us, 32x32x32 : 16x16x64, weights from HBM: W8A8 2048 x 4096 -> 14336 134 : 124, 2048 x
 // 14336 -> 4096 158 : 149, 2048 x 4096 -> 6144 63 : 58, 1760 x 12387 -> 15665 356 : 327, 960 x 4001 -> 710 18.8 : 17.5 (120 drawn products of 33
 // rows and more 0.98, 40 drawn layers 0.965 of the time); W8A32 2048 x 4096 -> 14336 416 : 395, 888 x 11222 -> 4096 154 : 134, 356 x 4096 -> 14336
