@@ -706,11 +706,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_f32_rows_kernel(const float
 #pragma unroll
         for (int i = 0; i < VK; ++i) {
             const int idx = lane + 64 * i;
-            if (idx < nvec) {
-                const int b0 = pg_quant_to_i8(v[i].x * inv) & 0xFF, b1 = pg_quant_to_i8(v[i].y * inv) & 0xFF;
-                const int b2 = pg_quant_to_i8(v[i].z * inv) & 0xFF, b3 = pg_quant_to_i8(v[i].w * inv) & 0xFF;
-                reinterpret_cast<int *>(q)[idx] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
-            }
+            if (idx < nvec) reinterpret_cast<int *>(q)[idx] = pg_quant4_to_i8(v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv);
         }
         if (tail && lane < 4) q[4 * nvec + lane] = (int8_t)(lane < tail ? pg_quant_to_i8(tv * inv) : 0);
         for (int idx = nvec + (tail != 0) + lane; idx < k_pad / 4; idx += 64) reinterpret_cast<int *>(q)[idx] = 0;

@@ -203,11 +203,8 @@ __global__ __launch_bounds__(64 * NW) void gemv_w8a8_m1_f32x_kernel(
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int idx = threadIdx.x + NT * i;
-        const int b0 = pg_quant_to_i8(v[i].x * inv_scale) & 0xFF;
-        const int b1 = pg_quant_to_i8(v[i].y * inv_scale) & 0xFF;
-        const int b2 = pg_quant_to_i8(v[i].z * inv_scale) & 0xFF;
-        const int b3 = pg_quant_to_i8(v[i].w * inv_scale) & 0xFF;
-        if (NV * NT == NCH * 256 || idx < NCH * 256) xq[idx] = idx < nvec ? (b0 | (b1 << 8) | (b2 << 16) | (b3 << 24)) : 0;
+        const int q = pg_quant4_to_i8(v[i].x * inv_scale, v[i].y * inv_scale, v[i].z * inv_scale, v[i].w * inv_scale);
+        if (NV * NT == NCH * 256 || idx < NCH * 256) xq[idx] = idx < nvec ? q : 0;
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");
     int acc[RPW];

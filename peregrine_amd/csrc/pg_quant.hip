@@ -120,13 +120,7 @@ __global__ __launch_bounds__(T) void quantize_rows_vec4_kernel(
 #pragma unroll
         for (int i = 0; i < MAXV; ++i) {
             const int idx = threadIdx.x + i * T;
-            if (idx < nvec) {
-                const int b0 = quant_to_i8(v[i].x * inv_scale) & 0xFF;
-                const int b1 = quant_to_i8(v[i].y * inv_scale) & 0xFF;
-                const int b2 = quant_to_i8(v[i].z * inv_scale) & 0xFF;
-                const int b3 = quant_to_i8(v[i].w * inv_scale) & 0xFF;
-                reinterpret_cast<int *>(qr)[idx] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
-            }
+            if (idx < nvec) reinterpret_cast<int *>(qr)[idx] = pg_quant4_to_i8(v[i].x * inv_scale, v[i].y * inv_scale, v[i].z * inv_scale, v[i].w * inv_scale);
         }
         if (TAIL && tail && threadIdx.x < 4) qr[4 * nvec + threadIdx.x] = (int8_t)((int)threadIdx.x < tail ? quant_to_i8(tv * inv_scale) : 0);
         for (int idx = nvec + (tail != 0) + threadIdx.x; idx < npad; idx += T) reinterpret_cast<int *>(qr)[idx] = 0;

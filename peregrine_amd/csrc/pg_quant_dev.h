@@ -2,18 +2,41 @@
 // one-row product that quantises its own activations (pg_gemv_w8a8.hip).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <type_traits>
 
 // round -> clamp(-127,127) -> `as i8` (NaN -> 0), returned as int.   src/quant.rs:101-106
+// Half away from zero is truncation after adding the float just under a half with the value's sign: with a half itself 0.49999997 would
+// reach 1, and every k + 0.5 still does (the sum lies a quarter of an ulp or less below it and rounds up).  Checked against roundf for every
+// float to 144.  The conversion truncates, takes NaN to 0 and saturates (asm: in C++ that would be undefined).  Five vector instructions with
+// the caller's product, where roundf, two clamps and two tests for NaN were fourteen.  With the maximum below, us, before : now: the
+// products of a layer for one row 42.7 : 41.4, 27 rows of a smaller one 34.4 : 33.5, 2048 rows 469 : 466.
 __device__ __forceinline__ int pg_quant_to_i8(float v) {
-    float r = roundf(v);
-    r = fminf(fmaxf(r, -127.0f), 127.0f);
-    return (r != r || v != v) ? 0 : (int)r;
+    int i;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(v + copysignf(0x1.fffffep-2f, v)));
+    return min(max(i, -127), 127);
 }
 
+// Four of them as the bytes of a dword.
+__device__ __forceinline__ int pg_quant4_to_i8(float x, float y, float z, float w) {
+    const unsigned lo = __builtin_amdgcn_perm((unsigned)pg_quant_to_i8(y), (unsigned)pg_quant_to_i8(x), 0x0C0C0400u);
+    const unsigned hi = __builtin_amdgcn_perm((unsigned)pg_quant_to_i8(w), (unsigned)pg_quant_to_i8(z), 0x04000C0Cu);
+    return (int)(lo | hi);
+}
+
+// Maximum over the 64 lanes of a wavefront, all of them active and none negative, in every lane: DPP moves within rows of 16 lanes, then the four rows' through scalar
+// registers (six exchanges through LDS were a chain of 0.2 us).
 __device__ __forceinline__ float pg_wave_max_f32(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
+    auto step = [](float x, auto ctrl) {
+        const int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, false);
+        return fmaxf(x, __int_as_float(y));
+    };
+    v = step(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+    v = step(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+    v = step(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
+    v = step(v, std::integral_constant<int, 0x140>{});  // row_mirror
+    const int b = __float_as_int(v);
+    return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(b, 0)), __int_as_float(__builtin_amdgcn_readlane(b, 16))),
+                 fmaxf(__int_as_float(__builtin_amdgcn_readlane(b, 32)), __int_as_float(__builtin_amdgcn_readlane(b, 48))));
 }
 
 // Maximum over a 256-thread workgroup; `red` = 4 floats of LDS.  Ends with every thread past a barrier.

@@ -71,6 +71,20 @@ def test_quantize_activations_edge_rows_and_empty(ctx, orc):
         quant.quantize_activations(np.zeros(5, np.float32), 2, 3, ctx)
 
 
+@pytest.mark.parametrize("cols", [64, 1028, 1531, 5000])  # less than a wavefront's vectors, a tail of its own, and a workgroup of 1024
+def test_quantize_activations_around_every_half(ctx, orc, cols):
+    """Half away from zero, at a scale of one: every k + 0.5 of either sign with the floats next to it, where the rounding has its edges."""
+    from peregrine_amd import quant
+    half = np.arange(-127, 127, dtype=np.float32) + np.float32(0.5)
+    v = np.concatenate([np.nextafter(half, np.float32(-np.inf)), half, np.nextafter(half, np.float32(np.inf))]).astype(np.float32)
+    a = np.resize(v, (-(-v.size // (cols - 1)), cols - 1))
+    a = np.concatenate([np.full((a.shape[0], 1), 127.0, np.float32), a], 1)
+    qg, sg = quant.quantize_activations(a, a.shape[0], cols, ctx)
+    qc, sc = orc.quantize_activations(a, a.shape[0], cols)
+    assert (np.asarray(sg) == 1.0).all() and (np.asarray(sc) == 1.0).all()
+    assert (np.asarray(qg).reshape(-1) == np.asarray(qc).reshape(-1)).all()
+
+
 @pytest.mark.parametrize("rows,cols", [(128, 96), (100, 70), (4096, 64), (64, 1000), (1, 5), (300, 1)])
 def test_quantize_weights_bit_exact(ctx, orc, rows, cols):
     from peregrine_amd import quant
