@@ -560,6 +560,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
             for (int j = 0; j < 2; ++j)
                 __builtin_amdgcn_global_load_lds((gptr_t)(src[q][j] + kb), (lptr_t)(base + q * TILE + j * 1024), 16, 0, 0);
     };
+    // The scales of the outputs that this thread will store, ahead of the loop: behind it they were a round trip to memory of their own (a layer's
+    // products for 27 rows 33.5 : 33.0 us, 24 x 4096 -> 4096 8.67 : 8.32).
+    constexpr int QUADS = NB * MT * 4, STORES = (QUADS + NW - 1) / NW;  // 64 outputs each: tile pair q / 4, register q % 4
+    float as[STORES], wsc[STORES];
+#pragma unroll
+    for (int t = 0; t < STORES; ++t) {
+        const int q = min(wave + NW * t, QUADS - 1), c = (q >> 2) / MT, b = (q >> 2) - c * MT;
+        as[t] = a_scales[min(r0 + 16 * b + 4 * (lane >> 4) + (q & 3), m - 1)];
+        wsc[t] = w_scales[min(n0 + 16 * c + (lane & 15), n - 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
     v4i acc[NB][MB];
 #pragma unroll
     for (int c = 0; c < NB; ++c)
@@ -610,32 +621,25 @@ __global__ __launch_bounds__(64 * NW) void gemm_w8a8_skinny_kernel(const int8_t 
 #pragma unroll
             for (int i = 0; i < 4; ++i) red[((wave * NB * MB + c * MB + b) * 4 + i) * 64 + lane] = acc[c][b][i];
     __syncthreads();
-    if constexpr (TRI) {
-        for (int e = threadIdx.x; e < NB * MT * 4 * 64; e += 64 * NW) {
-            const int l = e & 63, i = (e >> 6) & 3, cb = e >> 8, c = cb / MT, b = cb - c * MT;
-            int sum[3] = {0, 0, 0};
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
+    for (int t = 0; t < STORES; ++t) {
+        const int q = wave + NW * t;
+        if (q >= QUADS) break;
+        const int c = (q >> 2) / MT, b = (q >> 2) - c * MT, i = q & 3;
+        int sum[MB / MT] = {};
 #pragma unroll
-                for (int w = 0; w < NW; ++w) sum[p] += red[((w * NB * MB + c * MB + p * MT + b) * 4 + i) * 64 + l];
-            const int row = r0 + b * 16 + 4 * (l >> 4) + i, col = n0 + 16 * c + (l & 15);
-            if (row < m && col < n) {
-                const double v = 65536.0 * (double)sum[2] + 256.0 * (double)sum[1] + (double)sum[0];
-                out[(size_t)row * n + col] = (float)(v * (double)a_scales[row] * (double)w_scales[col]);
-            }
-        }
-        return;
-    }
-    for (int e = threadIdx.x; e < NB * MB * 4 * 64; e += 64 * NW) {
-        const int l = e & 63, i = (e >> 6) & 3, cb = e >> 8, c = cb / MB, b = cb - c * MB;
-        int sum = 0;
+        for (int p = 0; p < MB / MT; ++p)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) sum += red[((w * NB * MB + cb) * 4 + i) * 64 + l];
-        const int row = r0 + b * 16 + 4 * (l >> 4) + i, col = n0 + 16 * c + (l & 15);
+            for (int w = 0; w < NW; ++w) sum[p] += red[((w * NB * MB + c * MB + p * MT + b) * 4 + i) * 64 + lane];
+        const int row = r0 + 16 * b + 4 * (lane >> 4) + i, col = n0 + 16 * c + (lane & 15);
         if (row < m && col < n) {
             const size_t o = (size_t)row * n + col;
-            if (out) out[o] = (float)sum * a_scales[row] * w_scales[col];
-            if (acc_out) acc_out[o] = sum;
+            if constexpr (TRI) {
+                out[o] = (float)((65536.0 * (double)sum[2] + 256.0 * (double)sum[1] + (double)sum[0]) * (double)as[t] * (double)wsc[t]);
+            } else {
+                if (out) out[o] = (float)sum[0] * as[t] * wsc[t];
+                if (acc_out) acc_out[o] = sum[0];
+            }
         }
     }
 }
