@@ -375,6 +375,26 @@ def test_gguf_matmul_f16_route_special_rows(ctx, orc):
     gw.free()
 
 
+@pytest.mark.parametrize("k_in", [256, 1024, 1088, 2048, 2112, 4096, 4160, 8192, 8256, 16384, 16448, 32768, 32832])
+def test_gguf_matmul_f16_route_rows_of_every_length(ctx, orc, k_in):
+    """The rows' planes around the lengths where a row takes more registers, more threads, or is read twice; the row's largest value last."""
+    from peregrine_amd import gguf, _ffi
+    n_out, m = 40, 3
+    raw = H.pack_q8_0(orc.rng_normal(61, n_out * k_in, 0.0, 0.02))
+    x = orc.rng_normal(62 + k_in, m * k_in).reshape(m, k_in)
+    x[1, -1] = 300.0
+    x[2, :] *= np.float32(1e-20)
+    gw = gguf.GgufWeight(raw, 8, n_out, k_in, ctx)
+    _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 1))
+    try:
+        got = gw.matmul(x.reshape(-1), m).reshape(m, n_out)
+    finally:
+        _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 0))
+    for r in range(m):
+        H.assert_close_rel(got[r], orc.gguf_matmul(x[r], 1, raw, 8, n_out, k_in), RTOL_F16_ROUTE, f"row {r}")
+    gw.free()
+
+
 @pytest.mark.parametrize("n_out,k_in,m", [(515, 4160, 300), (1100, 2048, 100), (256, 256, 129)])
 def test_gguf_matmul_f16_route_q4_1(ctx, orc, n_out, k_in, m):
     """Q4_1 at prefill sizes: the first term as the Q4_0 product on the f16 matrix cores (same nibbles and scales),
