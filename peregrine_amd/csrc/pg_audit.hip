@@ -148,8 +148,8 @@ PG_API pg_status pg_audit_gguf_skinny(size_t n_out, size_t k_in, int q8, int nw,
     return PG_OK;
 }
 
-// Many rows on the f16 matrix cores (gguf_hmm_kernel<QT, MT>): its largest tile, 128 x 512 (wide = 1: the smaller tiles' rows are clamped
-// alike), or one of 256 x 256 (wide = 0),
+// Many rows on the f16 matrix cores (gguf_hmm_kernel<QT, MT, S>): its largest tile, 128 x 512 (wide = 1: the lower and the narrower tiles' rows are
+// clamped alike), or one of 256 x 256 (wide = 0),
 // K in `ks` chunks of whole stages of 64; the planes are [m][k_in] f16, the payload [n_out][k_in / 32][16 B] (Q8_0: [n_out][2][k_in / 32][16 B]).
 // (Every offset is linear in the stage: the first and the last stage of a chunk bound the rest.)
 PG_API pg_status pg_audit_gguf_hmm(size_t m, size_t n_out, size_t k_in, int q8, int wide, int ks, size_t *plane_end, size_t *plane_bytes,

@@ -1072,7 +1072,7 @@ pg_status pg_gguf_matmul_rows(pg_ctx *ctx, const float *x_dev, size_t m, const p
     }
     if (pg_gguf_hmm_takes(ctx, w->ggml_type, m, w->n_out, w->k_in, &hks))  // many rows of Q4_0 / Q8_0: the f16 matrix cores
         return pg_gguf_hmm_rows(ctx, x_dev, m, &w, &y_dev, 1, hks);
-    if (apart && q41 && w->k_in <= 32768 && pg_gguf_hmm_takes(ctx, PG_GGML_Q4_0, m, w->n_out, w->k_in, &hks)) {
+    if (apart && q41 && w->k_in <= 32768 && pg_gguf_hmm_takes(ctx, PG_GGML_Q4_0, m, w->n_out, w->k_in, &hks, true, 5.0)) {  // (a launch for the sums)
         // Q4_1 at that size: the first term d sum (q - 8) x as the Q4_0 product on the f16 matrix cores, then the
         // offsets times the rows' block sums (in the place of the rows' planes, with which the product is done), which add up
         // the K chunks' planes too.  us, with a launch that adds them up, and the sums beside digits that nothing reads : now:
@@ -1142,8 +1142,9 @@ pg_status pg_gguf_matmul_rows_multi(pg_ctx *ctx, const float *x_dev, size_t m, c
             n_total += w[i]->n_out;
         }
         int hks = 1;
-        if (one_type && pg_gguf_hmm_takes(ctx, w[0]->ggml_type, m, n_total, k_in, &hks)) return pg_gguf_hmm_rows(ctx, x_dev, m, w, y_dev, count, hks);
-        if (one_type && count <= 3 && pg_gguf_one_launch_takes(ctx, w[0]->ggml_type, m, n_total, k_in)) {
+        const bool one_launch = one_type && count <= 3 && !pg_gguf_hmm_holds(ctx, w[0]->ggml_type, m, n_total, k_in) && pg_gguf_one_launch_takes(ctx, w[0]->ggml_type, m, n_total, k_in);
+        if (one_type && !one_launch && pg_gguf_hmm_takes(ctx, w[0]->ggml_type, m, n_total, k_in, &hks)) return pg_gguf_hmm_rows(ctx, x_dev, m, w, y_dev, count, hks);
+        if (one_launch) {
             PG_TRY(pg_workspace(ctx, pg_mmdigits_bytes(m, k_in), &ws));
             const pg_mmdigits md = pg_mmdigits_carve(ws, m, k_in);
             PG_TRY(pg_launch_x_to_mm_digits(ctx, x_dev, m, k_in, w[0]->ggml_type, md));

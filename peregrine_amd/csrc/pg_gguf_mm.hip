@@ -1328,7 +1328,8 @@ static bool skinny_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_ou
 // under many columns, over more than two row tiles (71 x 4896 -> 2614 24 : 31, 67 x 512 -> 13720 11.5 : 17).  Q4_1 up to 64 rows: the offsets' launch goes too (0.6 to 0.9 up to 5 G).  us, before : now:
 // 35 x 1088 -> 465 (Q8_0) 12.4 : 7.6, 12 x 4096 -> 4096 (Q4_1) 9.9 : 8.0, 11 x 1056 -> 2116 (Q8_0) 11.5 : 7.6, 32 x 4096 -> 1024
 // (Q4_0) 13.7 : 9.2, 64 x 4096 -> 4096 (Q4_1) 28.5 : 22.
-// What runs on the f16 matrix cores stays there, and Q4_1 below eight rows with the streaming kernel: both have finer digits.
+// What the f16 matrix cores hold stays there, and Q4_1 below eight rows with the streaming kernel: both have finer digits.  (What they would take by their time
+// alone does not: of 101 products within these lines none is faster there by more than 3 %.)
 static bool ktile_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out, size_t k_in, bool planes) {
     const bool q41 = ggml_type == PG_GGML_Q4_1;
     if (!(ggml_type == PG_GGML_Q4_0 || ggml_type == PG_GGML_Q8_0 || q41) || m < (q41 ? 8 : 2) || k_in % 32 != 0 || k_in > 32768 || n_out < 1 || n_out >= (1u << 24))
@@ -1341,7 +1342,7 @@ static bool ktile_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_out
     if (k_in < 512 && n_out > 8192) return false;                                        // (all columns, hardly any K to split)
     if (m > 64 && (k_in >= (q41 ? 8192 : 6144) || (k_in < 1024 && m * n_out > 500000))) return false;
     if (g > (q41 ? (m <= 64 ? 5.0 : m <= 700 ? 1.8 : 1.0) : m <= 64 ? 1.4 : m <= 128 ? 0.9 : 0.7)) return false;
-    return m <= 16 || !pg_gguf_hmm_takes(ctx, q41 ? PG_GGML_Q4_0 : ggml_type, m, n_out, k_in, nullptr);
+    return m <= 16 || !pg_gguf_hmm_holds(ctx, q41 ? PG_GGML_Q4_0 : ggml_type, m, n_out, k_in);
 }
 
 // Whether a product runs as one launch after the digits.  `planes`: the caller takes the K chunks of the other route unsummed, so that

@@ -489,8 +489,11 @@ size_t pg_hmm_planes_bytes(size_t rows, size_t k);
 pg_hmm_planes pg_hmm_planes_carve(void *base, size_t rows, size_t k);
 pg_status pg_launch_rows_to_f16_planes(pg_ctx *ctx, const float *x_dev, size_t rows, size_t k, const pg_hmm_planes &p);
 // Whether a product of m rows with n_total weight rows (all the tensors of the launch) runs there, and in how many
-// K chunks (*ks_out; their planes need pg_gguf_hmm_part_floats floats).
-bool pg_gguf_hmm_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_total, size_t k_in, int *ks_out);
+// K chunks (*ks_out; their planes need pg_gguf_hmm_part_floats floats).  keep: the chunks' planes are left to their reader (keep_parts of the launch, which
+// has to be given the same); extra_us: what else the caller does on this route and not on the other.
+bool pg_gguf_hmm_takes(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_total, size_t k_in, int *ks_out, bool keep = false, double extra_us = 0.0);
+// Whether it runs there whatever the estimates say.
+bool pg_gguf_hmm_holds(const pg_ctx *ctx, int ggml_type, size_t m, size_t n_total, size_t k_in);
 size_t pg_gguf_hmm_part_floats(size_t m, size_t n_total, int ks);
 pg_status pg_launch_gguf_hmm_group(pg_ctx *ctx, size_t k_in, const pg_gguf_tensor *const *w, float *const *y, int count, size_t m,
                                    const pg_hmm_planes &planes, int ks, float *part, bool keep_parts = false);

@@ -2384,6 +2384,14 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
     int ks[7];
     size_t part_off[7], floats = 0;
     for (int i = 0; i < 7; ++i) {
+        if (i != first_of[i]) {  // (of one launch)
+            few[i] = few[first_of[i]];
+            hm[i] = hm[first_of[i]];
+            ks[i] = ks[first_of[i]];
+            part_off[i] = floats;
+            floats += pg_round_up((size_t)ks[i] * seq * n_of[i], 64);
+            continue;
+        }
         size_t groups = 0, rows = 0;
         for (int j = first_of[i]; j < first_of[i] + count_of[i]; ++j) {
             groups += (n_of[j] + 127) / 128;
@@ -2395,7 +2403,7 @@ static pg_status block_forward_chained(pg_ctx *ctx, pg_llama_block *b, const flo
         // planes, not as digit planes; the down projection's producer holds a row of the FFN width in registers).
         int hks = 1;
         hm[i] = !few[i] && (i != 6 || ffn <= 32768) && count_of[i] <= PG_HMM_MAX_GROUP &&
-                pg_gguf_hmm_takes(ctx, type, seq, rows, k_of[i], &hks);
+                pg_gguf_hmm_takes(ctx, type, seq, rows, k_of[i], &hks, true, 2.0);  // (what its f16 planes take longer than digits)
         if (hm[i]) ks[i] = hks;
         if (ks[i] > PG_MAX_PLANES) return pg_fail(PG_EUNSUPPORTED, "llama block: a product in %d K chunks", ks[i]);
         part_off[i] = floats;

@@ -313,6 +313,40 @@ def test_gguf_matmul_f16_route_every_tile_height(ctx, orc, typ, m, row_tiles):
     gw.free()
 
 
+@pytest.mark.parametrize("typ", [2, 8])
+@pytest.mark.parametrize("n_out,k_in,m,row_tiles,chunks", [
+    (3000, 4160, 100, 4, 8),   # K chunks of 9 stages, the last of 2
+    (3000, 4160, 300, 5, 5),   # of 13
+    (3000, 4160, 600, 6, 3),   # of 22 and 21
+    (3000, 4160, 690, 7, 3),
+    (4313, 4736, 583, 8, 3),   # of 25 and 24
+])
+def test_gguf_matmul_f16_route_stages_shared_by_two_groups(ctx, orc, typ, n_out, k_in, m, row_tiles, chunks):
+    """Tiles of 256 weight rows whose wavefronts take one block of a stage each, in every height, with odd and even numbers of stages
+    (the grid tells the tile): rows at the edges of its row tiles, and the last ones."""
+    from peregrine_amd import gguf, _ffi
+    say(f"gguf_matmul f16 route type={typ} n_out={n_out} k_in={k_in} m={m} row_tiles={row_tiles}")
+    raw = (H.pack_q4_0 if typ == 2 else H.pack_q8_0)(orc.rng_normal(3900 + m, n_out * k_in, 0.0, 0.02))
+    x = orc.rng_normal(317 + m, m * k_in)
+    x.reshape(m, k_in)[:, :: k_in // 40] *= 20
+    gw = gguf.GgufWeight(raw, typ, n_out, k_in, ctx)
+    _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 1))
+    try:
+        ctx.profile_begin()
+        got = gw.matmul(x, m).reshape(m, n_out)
+        ctx.profile_end()
+        grids = ctx.profile_grids()
+    finally:
+        _ffi.check(_ffi.lib.pg_gguf_hmm_force(ctx.handle, 0))
+    bm = 16 * row_tiles
+    tiles = -(-m // bm) * -(-n_out // 256) * chunks
+    assert list(grids["gguf_hmm_q4_0" if typ == 2 else "gguf_hmm_q8_0"]) == [512 * (-(-tiles // 8) * 8)], grids
+    for r in sorted({0, 15, 16, bm - 1, min(bm, m - 1), m // 2, m // bm * bm - 1, m - 2, m - 1} - {-1}):
+        want = orc.gguf_matmul(x.reshape(m, k_in)[r], 1, raw, typ, n_out, k_in)
+        H.assert_close_rel(got[r], want, RTOL_F16_ROUTE, f"row {r}")
+    gw.free()
+
+
 def test_gguf_matmul_f16_route_prefill_size_is_the_dispatchers_choice(ctx, orc):
     """1024 rows over [4096] -> [14336] (a prefill's gate projection): the dispatcher takes the f16 route by itself;
     rows spot-checked against the oracle, and the int8 block route on the same input agrees within its own bar."""

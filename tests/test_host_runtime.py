@@ -261,6 +261,16 @@ def test_products_of_the_f16_route_stay_there(host, typ):
                 assert f16_route(host, typ, m, n, k), (typ, m, n, k)
 
 
+@pytest.mark.parametrize("typ,m,k,n,f16", [
+    (2, 60, 14336, 14336, True), (2, 640, 6656, 2570, True), (8, 583, 4736, 4313, True), (8, 130, 5632, 9000, True), (3, 120, 8192, 6000, True),   # by their time
+    (2, 48, 14336, 14336, False), (2, 72, 2048, 16384, False), (2, 200, 2048, 16384, False), (8, 150, 2048, 8192, False), (3, 200, 4096, 4096, False),
+    (8, 278, 4096, 14438, True), (2, 169, 7616, 11455, True), (2, 140, 6144, 13965, True), (8, 267, 5184, 11881, True), (8, 886, 3904, 4478, True),  # held
+])
+def test_which_products_run_on_the_f16_matrix_cores(host, typ, m, k, n, f16):
+    """Both sides of the line between the routes, and products that keep their finer activations though the int8 route is estimated to be as fast."""
+    assert f16_route(host, typ, m, n, k) == f16
+
+
 def dequant_i8_call(host, m, k, n):
     """The kernels of one W8A32 product and the scratch it made the context take."""
     w = host.alloc(k * n)
