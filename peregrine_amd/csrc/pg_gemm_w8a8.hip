@@ -444,24 +444,41 @@ pg_status launch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *
 
 // out[m, n] = (float)(sum over the K splits of part[s][m, n]) * a_scale[m] * w_scale[n]: the integer sum is
 // exact and order-free, the f32 epilogue is the one of the unsplit product (src/quant.rs:163).
-__global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__restrict__ part, int splits, size_t plane,
-                                                             const float *__restrict__ a_scales,
-                                                             const float *__restrict__ w_scales, int n,
-                                                             float *__restrict__ out, int32_t *__restrict__ acc_out) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+// A pass over memory: V = 4 columns a thread where they come in fours and the arrays allow it, up to eight planes requested together, and the
+// row by a 32-bit division (plane, n and i count vectors; a 64-bit one for every column was most of the launch).  The whole product, us, so :
+// now: 200 x 9216 -> 4096 24.4 : 23.0, 240 x 10384 -> 3136 26.4 : 24.8, by single columns 180 x 6000 -> 3001 21.5 : 19.3.
+template <int V>
+__global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__restrict__ part, int splits, unsigned plane, const float *__restrict__ a_scales,
+                                                            const float *__restrict__ w_scales, unsigned n, float *__restrict__ out, int32_t *__restrict__ acc_out) {
+    typedef int vi __attribute__((ext_vector_type(V)));
+    typedef float vf __attribute__((ext_vector_type(V)));
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
     if (i >= plane) return;
-    int acc = 0, s = 0;
-    for (; s + 8 <= splits; s += 8) {  // eight independent loads in flight
-        int v[8];
+    const unsigned r = i / n, c = i - r * n;
+    const vi *p = reinterpret_cast<const vi *>(part) + i;
+    vi v[8], acc = 0;
+    int s = 0;
+    for (; s + 8 <= splits; s += 8) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = __builtin_nontemporal_load(part + (size_t)(s + u) * plane + i);
+        for (int u = 0; u < 8; ++u) v[u] = __builtin_nontemporal_load(p + (size_t)(s + u) * plane);
 #pragma unroll
         for (int u = 0; u < 8; ++u) acc += v[u];
     }
-    for (; s < splits; ++s) acc += __builtin_nontemporal_load(part + (size_t)s * plane + i);
-    const size_t r = i / n, c = i - r * n;
-    if (out) out[i] = (float)acc * a_scales[r] * w_scales[c];
-    if (acc_out) acc_out[i] = acc;
+    const float a = a_scales[r];
+    const vf ws = reinterpret_cast<const vf *>(w_scales)[c];
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+        if (s + u < splits) v[u] = __builtin_nontemporal_load(p + (size_t)(s + u) * plane);
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+        if (s + u < splits) acc += v[u];
+    if (out) {
+        vf o;
+#pragma unroll
+        for (int k = 0; k < V; ++k) o[k] = (float)acc[k] * a * ws[k];
+        reinterpret_cast<vf *>(out)[i] = o;
+    }
+    if (acc_out) reinterpret_cast<vi *>(acc_out)[i] = acc;
 }
 
 // ---- 2 .. 64 activation rows, or groups of up to 64: one pass over the weights a group, no K split between workgroups ----
@@ -870,19 +887,28 @@ pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const 
 
 }  // namespace
 
-// Some dozens of rows over few columns or a long K (33 .. 256): one or two tiles of activations against every weight row is far too few
+// Some dozens or hundreds of rows over few columns or a long K (33 .. 700): one or two tiles of activations against every weight row is far too few
 // workgroups to stream the weights (64 on 256 CUs at N = 4096), so K is split until every place of a CU is taken, not one more
 // (a workgroup too many is a round: 82 tiles in three runs are 33 workgroups for an XCD's 32 CUs, and 157 x 9208 -> 5214 took 42.7 us so); the partial i32 sums go to `part` ([splits][m][n]) and a second launch adds them and applies the
 // scales.  128x128 tiles with eight wavefronts, one a CU, or 64x64 of four stages, two a CU: over 36 products (K 9300 .. 14300) 0.87 of the time of
 // 64x128 and 128x128 tiles of four wavefronts, split beyond the places.  us, those : these: 135 x 10836 -> 628 21.4 : 18.5, 213 x
 // 13535 -> 1432 34.0 : 25.8, 96 x 12787 -> 2221 31.6 : 22.8, 87 x 12661 -> 4291 45.4 : 32.4, 46 x 13300 -> 9512 44.1 : 39.7.
-// Estimated as the tiles are, with what the last launch reads.
+// Estimated as the tiles are, with what the last launch reads and writes: fitted to two thirds of 300 products of 33 .. 1024 rows (K 1000 ..
+// 14336, n 200 .. 8000) in the measure of the other routes' estimates, 3.3 % mean error.
+// Those err by 9 % on these and are the longer estimates where K is long, so the line leaves them a margin: 3 % up to 32 tiles of 128x128, 8 % up to
+// 40, 21 % beyond (two or three runs gain little: 188 x 7917 -> 4379 21.0 whole : 23.6 split); past 256 rows products of more than 40 stay whole
+// (341 x 6552 -> 3421 24.3 : 28.3), and those of up to 32 tiles of 64x64 too, which keep the few-row kernel's groups of 48 rows that they are tested on
+// (346 x 12805 -> 289 23.9 : 18.6 split).  Of 324 products, 32 are more than 5 % faster than with the numbers of the last launch as it was
+// and whole products from 257 rows on, two more than 3 % slower (109 x 5416 -> 4100 15.9 : 16.6).  us, those : these: 297 x 12683 -> 1210
+// 32.5 : 22.2, 699 x 10156 -> 256 26.8 : 18.3, 488 x 10516 -> 643 28.6 : 20.8, 645 x 7660 -> 385 22.8 : 18.5.
 namespace {
 struct split_kernel {
     unsigned tile, resident;
-    double step[2], round, fixed, l2, weights, parts, idle;  // parts: per M of partial sums
+    double step[2], round, fixed, l2, weights, parts, idle, output;  // parts: per M of partial sums
 };
-constexpr split_kernel SPLITS[] = {{128, 1, {0.567}, 0.0, 8.919, 0.002, 0.198, 1.218, 0.161}, {64, 2, {0.649, 0.619}, 1.467, 4.862, 0.021, 0.175, 1.602, 0.074}};
+constexpr split_kernel SPLITS[] = {{128, 1, {0.515}, 0.100, 8.446, 0.001, 0.105, 1.906, 0.081, -1.719}, {64, 2, {0.487, 0.356}, 0.734, 6.675, 0.011, 0.120, 2.157, 0.037, -2.542}};
+constexpr size_t SPLIT_ROWS = 700, SPLIT_TILES = 40, SPLIT_TILES64 = 33;
+constexpr double split_margin(size_t tiles128) { return tiles128 <= 32 ? 0.97 : tiles128 <= SPLIT_TILES ? 0.92 : 0.79; }
 // The runs of K, none of them empty, and the k-tiles of one.
 unsigned split_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, const split_kernel &s, unsigned *per) {
     const size_t tiles = ((m + s.tile - 1) / s.tile) * ((w->cols + s.tile - 1) / s.tile), kt = w->k_pad / 128;
@@ -904,8 +930,13 @@ pg_status pg_launch_gemm_w8a8_split(pg_ctx *ctx, const int8_t *a_i8, size_t a_st
     if (index == 0) PG_TRY((launch<128, 128, 128, 4, 2, 4, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)runs, (int)per)));
     else PG_TRY((launch<64, 64, 128, 4, 2, 2, 2>(ctx, a_i8, a_stride, a_scales, w, m, nullptr, part, (int)runs, (int)per)));
     const size_t n = w->cols, plane = m * n;
-    return pg_launch(ctx, "gemm_w8a8_finish", splitk_finish_kernel, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0,
-                     (const int32_t *)part, (int)runs, plane, a_scales, (const float *)w->scales, (int)n, out, acc);
+    if (plane > UINT_MAX) return pg_fail(PG_EUNSUPPORTED, "gemm_w8a8: %zu x %zu split over K", m, n);  // (the route splits few tiles only)
+    auto finish = [&](auto kern, unsigned v) {
+        return pg_launch(ctx, "gemm_w8a8_finish", kern, dim3((unsigned)((plane / v + 255) / 256)), dim3(256), 0, (const int32_t *)part, (int)runs,
+                         (unsigned)(plane / v), a_scales, (const float *)w->scales, (unsigned)(n / v), out, acc);
+    };
+    const bool fours = n % 4 == 0 && ((uintptr_t)out | (uintptr_t)acc | (uintptr_t)part | (uintptr_t)w->scales) % 16 == 0;
+    return fours ? finish(splitk_finish_kernel<4>, 4) : finish(splitk_finish_kernel<1>, 1);
 }
 
 // 33 .. 512 rows in one launch of the few-row kernel: groups of 32, 48 or 64 rows, each reading every weight once more (the
@@ -970,7 +1001,8 @@ pg_w8a8_route pg_gemm_w8a8_route(const pg_ctx *ctx, const pg_qtensor *const *w, 
             better(s.fixed + s.rows * digits + sqrt(walk * walk + loads * loads), PG_W8A8_ROWS, i);
         }
     }
-    if (m <= 256 && count == 1)
+    const size_t tiles128 = (m + 127) / 128 * ((cols + 127) / 128), tiles64 = (m + 63) / 64 * ((cols + 63) / 64);
+    if (count == 1 && m <= SPLIT_ROWS && (m <= 256 || (tiles128 <= SPLIT_TILES && tiles64 >= SPLIT_TILES64)))
         for (size_t i = 0; i < sizeof(SPLITS) / sizeof(SPLITS[0]); ++i) {
             const split_kernel &s = SPLITS[i];
             unsigned per;
@@ -979,8 +1011,8 @@ pg_w8a8_route pg_gemm_w8a8_route(const pg_ctx *ctx, const pg_qtensor *const *w, 
             const size_t tiles = ((m + s.tile - 1) / s.tile) * ((cols + s.tile - 1) / s.tile);
             const double cu = fullest_cu((tiles + 7) / 8 * 8 * runs, (unsigned)ctx->num_cu, s.resident, s.step, per, s.round, s.idle);
             const double all = 128e-6 * (double)(tiles * (k_pad / 128)) * (2 * s.tile) * s.l2 + weights * s.weights;
-            const double c2 = cu * cu, a2 = all * all;
-            better(quantise_us(w[0], m) + s.fixed + sqrt(sqrt(c2 * c2 + a2 * a2)) + 1e-6 * (double)(m * cols * runs) * s.parts, PG_W8A8_SPLIT, i);
+            const double c2 = cu * cu, a2 = all * all, planes = 1e-6 * (double)(m * cols) * (runs * s.parts + s.output);
+            better((quantise_us(w[0], m) + s.fixed + sqrt(sqrt(c2 * c2 + a2 * a2)) + planes) / split_margin(tiles128), PG_W8A8_SPLIT, i);
         }
     return best;
 }

@@ -261,7 +261,7 @@ pg_status pg_launch_gemm_w8a8_combine(pg_ctx *ctx, const int8_t *a_i8, size_t a_
 // The W8A32 product over three digit planes (plane_bytes apart) in one launch, where it takes it.
 bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
 pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out);
-// How W8A8 products of two rows and more run: tiles, the few-row kernel (2 .. 512 rows), or tiles with K split over workgroups (33 .. 256 rows
+// How W8A8 products of two rows and more run: tiles, the few-row kernel (2 .. 512 rows), or tiles with K split over workgroups (33 .. 700 rows
 // over one weight: i32 partial sums in `part`, pg_gemm_w8a8_split_bytes of them, and a finishing launch); `index` names the kernel.
 enum pg_w8a8_kind { PG_W8A8_TILES, PG_W8A8_ROWS, PG_W8A8_SPLIT };
 struct pg_w8a8_route { pg_w8a8_kind kind; int index; };

@@ -286,6 +286,27 @@ def np_epilogue(acc, a_s, w_s):
     return (acc.astype(np.float32) * a_s.astype(np.float32)[:, None]) * w_s.astype(np.float32)[None, :]
 
 
+@pytest.mark.parametrize("m,k,n", [(700, 8200, 260), (412, 9001, 333), (300, 12000, 662), (257, 13990, 1031), (200, 9216, 402), (64, 13000, 300)])
+def test_products_split_over_k_at_every_remainder_of_four_columns(ctx, orc, m, k, n):
+    """K split over workgroups, up to 700 rows: the finishing launch by fours (with the accumulators and without), by single columns,
+    and where the result lies one float off a multiple of four."""
+    from peregrine_amd import quant, _ffi
+    say(f"split over K m={m} k={k} n={n}")
+    a = orc.rng_normal(4321 + m, m * k)
+    qt = quant.quantize_weights(orc.rng_normal(8765 + n, k * n, 0.0, 0.02), k, n, ctx)
+    got, got_acc = run_matmul_dev(ctx, a, m, k, qt)
+    assert last_tile(ctx)[2] > 1
+    rows = sorted({0, 63, m // 2, m - 2, m - 1})
+    want, want_acc = orc.matmul_quantized(a.reshape(m, k)[rows].reshape(-1), len(rows), k, qt.data_i8_t, qt.scales, n)
+    assert (got_acc.reshape(m, n)[rows].reshape(-1) == want_acc.reshape(-1)).all()
+    assert (bits(got.reshape(m, n)[rows]).reshape(-1) == bits(want).reshape(-1)).all()
+    x, y = DevBuf(ctx, host=a), DevBuf(ctx, (m * n + 1) * 4)
+    for at in (0, 1):
+        _ffi.check(_ffi.lib.pg_matmul_quantized_dev(ctx.handle, x.ptr, m, k, qt._gpu, C.c_void_p(y.ptr.value + 4 * at), None))
+        ctx.sync()
+        assert (bits(y.to_host(np.float32)[at:at + m * n]) == bits(got.reshape(-1))).all()
+
+
 # benchmark configuration 3: the seven products of one Llama-3-8B layer at M = 2048 are these four shapes;
 # the last column is the output tile the dispatcher must pick (so a dispatcher change cannot
 # silently leave a tile shape without a test)
