@@ -168,7 +168,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const tile_order or
     const int kt0_split = blockIdx.y * kt_per_split;
     const int8_t *a_base = A + (size_t)m0 * lda + (size_t)kt0_split * BK;
     const int8_t *b_base = Bw + (size_t)n0 * ldb + (size_t)kt0_split * BK;
-    if (acc_out) acc_out += (size_t)blockIdx.y * M * N;
+    if (acc_out) acc_out += (size_t)blockIdx.y * M * N * (NP == 3 ? 2 : 1);  // (W8A32: the digits' joined sums, in f64)
 
     // ---- LDS fragment offsets (bytes) for each k-step of a stage.
     const int l31 = lane & 31, half = lane >> 5;
@@ -302,7 +302,7 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const tile_order or
     // every store cost a layer of 2048 rows 3 %.  The one-launch W8A32 product keeps the hint: its tiles take longer than their stores
     // either way.)
     static_assert(TN % 2 == 0, "pairs of column tiles");
-    enum { F32, I32, BOTH };
+    enum { F32, I32, BOTH, F64 };
     auto store = [&](auto hint, auto inside, auto what) {
         constexpr int WHAT = decltype(what)::value;
         auto put = [](auto v, auto *dst) {
@@ -346,6 +346,10 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const tile_order or
                 for (int k = 0; k < 8; ++k) {
                     if (!stored(k)) continue;
                     const size_t o = at + (size_t)k * N;
+                    if constexpr (WHAT == F64) {
+                        put(65536.0 * (double)a[2][k] + 256.0 * (double)a[1][k] + (double)a[0][k], reinterpret_cast<double *>(acc_out) + o);
+                        continue;
+                    }
                     float f;
                     if constexpr (NP == 3) f = (float)((65536.0 * (double)a[2][k] + 256.0 * (double)a[1][k] + (double)a[0][k]) * (double)as[k] * (double)ws);
                     else if constexpr (COMB) f = (float)((65536.0 * (double)a[0][k] + 256.0 * (double)c1[k] + (double)c0[k]) * (double)as[k] * (double)ws);
@@ -366,6 +370,12 @@ void gemm_w8a8_kernel(const int8_t *__restrict__ A, int lda, const tile_order or
     using f32 = std::integral_constant<int, F32>;
     const bool whole = m0 + BM <= M && n0 + BN <= N;
     if constexpr (NP == 3) {
+        if (acc_out) {
+            using f64 = std::integral_constant<int, F64>;
+            if (whole) store(yes{}, yes{}, f64{});
+            else store(yes{}, no{}, f64{});
+            return;
+        }
         if (whole) store(yes{}, yes{}, f32{});
         else store(yes{}, no{}, f32{});
         return;
@@ -479,6 +489,33 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__res
         reinterpret_cast<vf *>(out)[i] = o;
     }
     if (acc_out) reinterpret_cast<vi *>(acc_out)[i] = acc;
+}
+
+// The W8A32 product's: a plane holds the joined sums of the three digits, whole numbers below 2^53 in f64, so their sum is exact and the one rounding
+// that of the unsplit product.
+constexpr int W8A32_RUNS = 8;  // of K, at the most
+template <int V>
+__global__ __launch_bounds__(256) void splitk_finish_w8a32_kernel(const double *__restrict__ part, int splits, unsigned plane, const float *__restrict__ a_scales,
+                                                                  const float *__restrict__ w_scales, unsigned n, float *__restrict__ out) {
+    typedef double vd __attribute__((ext_vector_type(V)));
+    typedef float vf __attribute__((ext_vector_type(V)));
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= plane) return;
+    const unsigned r = i / n, c = i - r * n;
+    const vd *p = reinterpret_cast<const vd *>(part) + i;
+    vd v[W8A32_RUNS], sum = 0;
+#pragma unroll
+    for (int u = 0; u < W8A32_RUNS; ++u)
+        if (u < splits) v[u] = __builtin_nontemporal_load(p + (size_t)u * plane);
+    const float a = a_scales[r];
+    const vf ws = reinterpret_cast<const vf *>(w_scales)[c];
+#pragma unroll
+    for (int u = 0; u < W8A32_RUNS; ++u)
+        if (u < splits) sum += v[u];
+    vf o;
+#pragma unroll
+    for (int k = 0; k < V; ++k) o[k] = (float)(sum[k] * (double)a * (double)ws[k]);
+    reinterpret_cast<vf *>(out)[i] = o;
 }
 
 // ---- 2 .. 64 activation rows, or groups of up to 64: one pass over the weights a group, no K split between workgroups ----
@@ -1236,7 +1273,7 @@ static int pick_w8a32_few(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     if (m <= 16) return n > 16 * cus ? (k >= 1536 ? 6 : -1) : m <= 8 && k >= 3072 ? 7 : -1;
     return n <= 8 * cus ? (k >= 1536 ? 7 : -1) : n <= 16 * cus ? (k >= 1536 ? 6 : -1) : k >= 2560 ? 8 : -1;
 }
-static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m, double *us = nullptr) {
     const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w->k_pad / 128);
     const double output = 1e-6 * (double)(m * w->cols), past = std::max(0.0, output - 20.0);
     const double weights = 1e-6 * (double)(w->rows * w->cols), ragged = w->cols % 32 ? output : 0.0;
@@ -1254,17 +1291,56 @@ static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     double best_us = 0.0;
     for (int i = 0; i < (int)(sizeof(W8A32) / sizeof(W8A32[0])); ++i) {
         if (W8A32[i].runs > 1 && m > 512) continue;
-        const double us = estimate(i);
-        if (best < 0 || us < best_us) {
+        const double t = estimate(i);
+        if (best < 0 || t < best_us) {
             best = i;
-            best_us = us;
+            best_us = t;
         }
     }
+    if (us) *us = best_us;
     return best;
 }
-pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out) {
+// Hundreds of rows over few columns or a long K are few tiles, each of which walks all of K: of those, 64x64 tiles with K in runs, as many as an XCD has
+// CUs for (two stages a run at least), and a launch that adds the runs up.  Estimated as above, fitted to two thirds of 180 products of 33 .. 1024 rows, K
+// 700 .. 14336 and n 64 .. 6000 on that kernel in the measure of the estimates above, 5 % mean error, which leave it 5 %: 48 of them are split then,
+// 0.8 of the time on average, none of them slower.  The line is drawn at 71 tiles: from 72 on three runs or two give 0.85 of the time where they are taken (up to
+// there 0.77), and products there are tested on tiles that walk K whole (467 x 8337 -> 534, 72 tiles).  (Tiles of 32x64 and 32x128 split take 0.5 to 1 % more over all, 64x128, 128x128 and 64x256 5 to 30.)
+// us, whole : split: 286 x 7055 -> 832 30.4 : 22.7, 156 x 11538 -> 829 37.0 : 23.6, 768 x 8136 -> 111 36.5 : 24.4, 62 x 8043 -> 3726 25.0 : 20.1;
+// it stays: 64 x 8192 -> 512 12.3 : 17.4, 150 x 3000 -> 1500 12.8 : 15.4.
+static unsigned w8a32_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, unsigned *per) {
+    *per = (unsigned)(w->k_pad / 128);
+    if (m <= 32 || *per < 4) return 1;
+    const size_t kt = *per, tiles = (m + 63) / 64 * ((w->cols + 63) / 64), cus = (size_t)ctx->num_cu;
+    const size_t most = tiles < 72 ? std::min<size_t>({cus / 8 / ((tiles + 7) / 8), kt / 2, (size_t)W8A32_RUNS}) : 1;
+    if (most < 2) return 1;
+    const unsigned each = (unsigned)((kt + most - 1) / most), runs = (unsigned)((kt + each - 1) / each);
+    const double output = 1e-6 * (double)(m * w->cols), cu = 0.370 * each;
+    const double all = 128e-6 * (double)(tiles * kt) * 256 * 0.014 + 0.105e-6 * (double)(w->rows * w->cols);
+    const double c2 = cu * cu, a2 = all * all;
+    double whole;
+    pick_w8a32(ctx, w, m, &whole);
+    if ((10.414 + sqrt(sqrt(c2 * c2 + a2 * a2)) + output * (1.115 * runs - 3.0)) / 0.95 >= whole) return 1;
+    *per = each;
+    return runs;
+}
+size_t pg_gemm_w8a32_part_bytes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+    unsigned per;
+    const unsigned runs = w8a32_runs(ctx, w, m, &per);
+    return runs > 1 ? (size_t)runs * m * w->cols * sizeof(double) : 0;
+}
+pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part) {
     if (!pg_gemm_w8a32_takes(ctx, w, m)) return pg_fail(PG_EINVAL, "gemm_w8a32: m = %zu", m);
     const size_t k_pad = w->k_pad, n = w->cols;
+    unsigned per;
+    if (const unsigned runs = part ? w8a32_runs(ctx, w, m, &per) : 1; runs > 1) {
+        PG_TRY((launch_group<64, 64, 128, 3, 4, 2, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, static_cast<int32_t *>(part), (int)runs, (int)per, nullptr, 0, plane_bytes)));
+        auto finish = [&](auto kern, size_t v) {
+            return pg_launch(ctx, "gemm_w8a32_finish", kern, dim3((unsigned)((m * n / v + 255) / 256)), dim3(256), 0, (const double *)part, (int)runs,
+                             (unsigned)(m * n / v), a_scales, (const float *)w->scales, (unsigned)(n / v), out);
+        };
+        const bool twos = n % 2 == 0 && (uintptr_t)part % 16 == 0 && ((uintptr_t)out | (uintptr_t)w->scales) % 8 == 0;
+        return twos ? finish(splitk_finish_w8a32_kernel<2>, 2) : finish(splitk_finish_w8a32_kernel<1>, 1);
+    }
     auto one_weight = [&](skinny_wgroup &grp) {
         for (int i = 0; i < PG_GEMM_MAX_GROUP; ++i) {
             grp.w[i] = i ? nullptr : w->w_t;

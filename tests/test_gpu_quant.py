@@ -633,6 +633,30 @@ def test_matmul_dequant_i8_vs_oracle(ctx, orc, m, k, n):
     qt.free_gpu()
 
 
+@pytest.mark.parametrize("m,k,n,runs", [(286, 7055, 832, 3), (768, 8136, 111, 8), (57, 10391, 3087, 4), (485, 7086, 294, 6), (164, 9108, 1114, 4), (330, 12000, 130, 8), (33, 132000, 7, 8)])
+def test_matmul_dequant_i8_split_over_k(ctx, orc, m, k, n, runs):
+    """K in runs over workgroups: whole numbers as activations and powers of two as scales make the product exact, in even and odd
+    numbers of columns, and where the result lies one float off a multiple of two."""
+    from peregrine_amd import quant, _ffi
+    say(f"matmul_dequant_i8 split over K m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + n)
+    a = rng.integers(-100, 101, size=(m, k)).astype(np.float32)
+    q = rng.integers(-127, 128, size=(k, n), dtype=np.int8)
+    s = (2.0 ** rng.integers(-12, -4, size=n)).astype(np.float32)
+    qt = quant.QuantizedTensor(q.reshape(-1), np.ascontiguousarray(q.T).reshape(-1), s, k, n)
+    qt.to_gpu(ctx)
+    rows = sorted({0, 63, 64, m // 2, m - 1} & set(range(m)))
+    want = ((a[rows].astype(np.int64) @ q.astype(np.int64)).astype(np.float64) * s).astype(np.float32)
+    x, y = DevBuf(ctx, host=a), DevBuf(ctx, (m * n + 1) * 4)
+    for at in (0, 1):
+        _ffi.check(_ffi.lib.pg_matmul_dequant_i8_dev(ctx.handle, x.ptr, m, k, qt._gpu, C.c_void_p(y.ptr.value + 4 * at)))
+        ctx.sync()
+        assert last_tile(ctx) == (64, 64, runs)
+        got = y.to_host(np.float32)[at:at + m * n].reshape(m, n)[rows]
+        assert (got == want).all()
+    qt.free_gpu()
+
+
 def test_matmul_dequant_i8_combining_epilogue_on_every_tile(ctx, orc):
     """Where the planes are stacked (beyond one launch's offsets; under a tile override) the product of the plane of weight
     65536 finishes the sum in its epilogue (it reads the other two planes' accumulators).  Every tile shape of the matrix-core
