@@ -21,6 +21,7 @@
 #include "pg_internal.h"
 #include "pg_stream_addr.h"
 #include "pg_digits.h"
+#include "pg_act_dev.h"
 
 namespace {
 
@@ -231,7 +232,9 @@ struct RowLoads {
 //      src/nn.rs:560-652) with the block's sum of y^2 in ss_out[block]: the normalisation factor is a
 //      scalar, which the next product applies to its result (POST);
 //   2  the workgroup multiplies by two tensors (gate, then up = epi.qs1 / d1) and leaves only the digits
-//      of silu(gate) * up (src/models/llama/decoder.rs:143-150).
+//      of silu(gate) * up (src/models/llama/decoder.rs:143-150);
+//   3  the same for pairs of a token and an expert: item i's two tensors from the tables, its digits as row i, the activation
+//      epi.act.  One launch where gate, up, their product and its digits were four of 2 to 4 us each (moe_ffn_core has both sides).
 // POST: the product is multiplied by 1 / sqrt(sum(ss_in[0 .. ss_n)) * ss_inv_dim + eps) before anything else.
 template <int QT, int BPL, int RW, int R, bool Q41 = false, int XM = 0, int NW = 1, int EPI = 0, bool POST = false, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void gguf_gemv_kernel(
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(64 * NW) void gguf_gemv_kernel(
     const float *__restrict__ xsum_base, const float *__restrict__ x_f32, pg_gemv_epi epi) {
     constexpr int SEG = 64 * BPL;  // blocks per K segment
     constexpr bool XF32 = XM == 1, LDSX = XM == 2;
-    constexpr int NT = EPI == 2 ? 2 : 1;  // tensors per workgroup
+    constexpr int NT = EPI >= 2 ? 2 : 1;  // tensors per workgroup
     constexpr int NG = RW / R, NGT = NG * NT;
     static_assert(EPI == 0 || (XM == 0 && !Q41 && NW * RW == 32), "an output block of 32 rows per workgroup");
     static_assert(EPI != 0 || XM != 0 || NW == 1, "several wavefronts per workgroup only where they share something");
@@ -251,17 +254,21 @@ __global__ __launch_bounds__(64 * NW) void gguf_gemv_kernel(
     static_assert(!NORM || (XM == 1 && !POST), "the norm is folded in where the row arrives in f32");
     extern __shared__ __attribute__((aligned(16))) char lds_digits[];  // XM 1, 2: [6 planes][nb][16 B], then nb scales
     const int item = blockIdx.y;
-    const uint8_t *qs_any = qs0;
-    const uint16_t *d_any = d0;
+    const uint8_t *qs_any = qs0, *qs1_any = epi.qs1;
+    const uint16_t *d_any = d0, *d1_any = epi.d1;
     if (batch.qs_table) {
         const int e = batch.expert_of[item];
         qs_any = batch.qs_table[e];
         d_any = batch.d_table[e];
+        if constexpr (EPI == 3) {
+            qs1_any = epi.qs1_table[e];
+            d1_any = epi.d1_table[e];
+        }
     }
     const gv4i_ptr qs = (gv4i_ptr)(uintptr_t)qs_any;
     const gv4i_ptr dsc = (gv4i_ptr)(uintptr_t)d_any;
-    const gv4i_ptr qs_t[2] = {qs, (gv4i_ptr)(uintptr_t)epi.qs1};
-    const gv4i_ptr dsc_t[2] = {dsc, (gv4i_ptr)(uintptr_t)epi.d1};
+    const gv4i_ptr qs_t[2] = {qs, (gv4i_ptr)(uintptr_t)qs1_any};
+    const gv4i_ptr dsc_t[2] = {dsc, (gv4i_ptr)(uintptr_t)d1_any};
     const size_t xrow = (size_t)(item / batch.x_row_div);
     const gv4i_ptr digits = (gv4i_ptr)(uintptr_t)(digits_base + xrow * (size_t)nb * 96);
     const float *__restrict__ xs = xs_base + xrow * (size_t)nb;
@@ -476,7 +483,7 @@ __global__ __launch_bounds__(64 * NW) void gguf_gemv_kernel(
             float v = wave_sum_f32(acc[g][r]);
             if constexpr (POST || NORM) v *= post;
             const int row = row0 + (g % NG) * R + r;
-            if constexpr (EPI != 2) {
+            if constexpr (EPI < 2) {
                 if (lane == 0 && row < n_out) {
                     if (residual_base) v = residual_base[(size_t)item * n_out + row] + v;
                     y[row] = v;
@@ -503,10 +510,11 @@ __global__ __launch_bounds__(64 * NW) void gguf_gemv_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float gv = res[0][e0 + e];
-                    f[e] = gv / (1.0f + expf(-gv)) * res[NT - 1][e0 + e];
+                    if constexpr (EPI == 3) f[e] = pg_act(epi.act, gv) * res[NT - 1][e0 + e];
+                    else f[e] = gv / (1.0f + expf(-gv)) * res[NT - 1][e0 + e];
                 }
             }
-            pg_emit_digits<QT == 4>(f, 0, blockIdx.x, sub, n_out / 32, epi.out_digits, epi.out_xs);
+            pg_emit_digits<QT == 4>(f, EPI == 3 ? item : 0, blockIdx.x, sub, n_out / 32, epi.out_digits, epi.out_xs);
         }
     }
 }
@@ -671,18 +679,18 @@ pg_status launch_gemv_bpl(pg_ctx *ctx, size_t n_out, size_t k_in, const uint8_t 
 // 32 output rows as 32 / RW wavefronts.
 template <int QT, int BPL, int EPI, bool POST>
 pg_status launch_gemv_epi_bpl(pg_ctx *ctx, size_t n_out, size_t k_in, const uint8_t *qs, const uint16_t *d, const pg_xdigits &xd,
-                              float *y, const float *residual, const pg_gemv_epi &epi) {
+                              float *y, const float *residual, const pg_gemv_epi &epi, const pg_gemv_batch &batch) {
     const int nb = (int)(k_in / 32);
-    const pg_gemv_batch one = {1, nullptr, nullptr, nullptr, 1};
     constexpr int NH = QT == 8 ? 2 : 1;
     constexpr int R8 = BPL * NH <= 2 ? 8 : (BPL * NH <= 4 ? 4 : 2);
     const size_t want = (size_t)ctx->num_cu * 6;  // wavefronts wanted in the grid
-    const size_t rows = n_out * (EPI == 2 ? 2 : 1);
+    const size_t rows = n_out * (EPI >= 2 ? 2 : 1) * (size_t)batch.count;
 #define PG_GGUF_GEMV_E_LAUNCH(RWW, RR)                                                                                            \
-    PG_TRY(pg_launch(ctx, EPI == 1 ? (QT == 4 ? "gguf_gemv_q4_0_norm_digits" : "gguf_gemv_q8_0_norm_digits")                      \
-                              : (QT == 4 ? "gguf_gemv_q4_0_swiglu_digits" : "gguf_gemv_q8_0_swiglu_digits"),                      \
-                     gguf_gemv_kernel<QT, BPL, RWW, RR, false, 0, 32 / RWW, EPI, POST>, dim3((unsigned)(n_out / 32)),             \
-                     dim3(64 * (32 / RWW)), 0, qs, d, one, (int)n_out, nb, xd.digits, xd.xs, y, residual, (const uint16_t *)nullptr, \
+    PG_TRY(pg_launch(ctx, EPI == 1   ? (QT == 4 ? "gguf_gemv_q4_0_norm_digits" : "gguf_gemv_q8_0_norm_digits")                    \
+                          : EPI == 2 ? (QT == 4 ? "gguf_gemv_q4_0_swiglu_digits" : "gguf_gemv_q8_0_swiglu_digits")                \
+                                     : (QT == 4 ? "gguf_gemv_q4_0_act_digits" : "gguf_gemv_q8_0_act_digits"),                     \
+                     gguf_gemv_kernel<QT, BPL, RWW, RR, false, 0, 32 / RWW, EPI, POST>, dim3((unsigned)(n_out / 32), (unsigned)batch.count), \
+                     dim3(64 * (32 / RWW)), 0, qs, d, batch, (int)n_out, nb, xd.digits, xd.xs, y, residual, (const uint16_t *)nullptr, \
                      (const float *)nullptr, (const float *)nullptr, epi))
     if constexpr (BPL * NH > 2) {  // (8 or 16 wavefronts would leave too few registers each for rows this long)
         PG_GGUF_GEMV_E_LAUNCH(8, R8);
@@ -697,21 +705,21 @@ pg_status launch_gemv_epi_bpl(pg_ctx *ctx, size_t n_out, size_t k_in, const uint
 
 template <int EPI, bool POST>
 pg_status launch_gemv_epi(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const uint8_t *qs, const uint16_t *d, const pg_xdigits &xd,
-                          float *y, const float *residual, const pg_gemv_epi &epi) {
+                          float *y, const float *residual, const pg_gemv_epi &epi, const pg_gemv_batch &batch = {1, nullptr, nullptr, nullptr, 1}) {
     size_t bpl = (k_in / 32 + 63) / 64;
     if (bpl > 4) bpl = 4;
     if (ggml_type != PG_GGML_Q4_0 && ggml_type != PG_GGML_Q8_0)
         return pg_fail(PG_EUNSUPPORTED, "gguf_gemv: only Q4_0 and Q8_0 products leave their output as digits");
     const bool q4 = ggml_type == PG_GGML_Q4_0;
     switch (bpl) {
-        case 1: return q4 ? launch_gemv_epi_bpl<4, 1, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi)
-                          : launch_gemv_epi_bpl<8, 1, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi);
-        case 2: return q4 ? launch_gemv_epi_bpl<4, 2, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi)
-                          : launch_gemv_epi_bpl<8, 2, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi);
-        case 3: return q4 ? launch_gemv_epi_bpl<4, 3, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi)
-                          : launch_gemv_epi_bpl<8, 3, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi);
-        default: return q4 ? launch_gemv_epi_bpl<4, 4, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi)
-                           : launch_gemv_epi_bpl<8, 4, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi);
+        case 1: return q4 ? launch_gemv_epi_bpl<4, 1, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch)
+                          : launch_gemv_epi_bpl<8, 1, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch);
+        case 2: return q4 ? launch_gemv_epi_bpl<4, 2, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch)
+                          : launch_gemv_epi_bpl<8, 2, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch);
+        case 3: return q4 ? launch_gemv_epi_bpl<4, 3, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch)
+                          : launch_gemv_epi_bpl<8, 3, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch);
+        default: return q4 ? launch_gemv_epi_bpl<4, 4, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch)
+                           : launch_gemv_epi_bpl<8, 4, EPI, POST>(ctx, n_out, k_in, qs, d, xd, y, residual, epi, batch);
     }
 }
 
@@ -899,6 +907,17 @@ pg_status pg_launch_gguf_gemv_swiglu_digits(pg_ctx *ctx, int ggml_type, size_t n
     if (ss_n > 256) return pg_fail(PG_EUNSUPPORTED, "gguf_gemv (digits of SiLU(gate) * up): more than 256 partial sums");
     epi.ss_in = ss_in; epi.ss_n = (int)ss_n; epi.ss_inv_dim = 1.0f / (float)ss_dim; epi.eps = eps;
     return launch_gemv_epi<2, true>(ctx, ggml_type, n_out, k_in, qs_gate, d_gate, xd, nullptr, nullptr, epi);
+}
+
+pg_status pg_launch_gguf_gemv_act_digits(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const pg_gemv_batch &gate, const uint8_t *const *qs_up,
+                                         const uint16_t *const *d_up, int act, const pg_xdigits &xd, const pg_xdigits &out) {
+    if (gate.count == 0) return PG_OK;
+    if (gate.count > 65535) return pg_fail(PG_EUNSUPPORTED, "gguf_gemv: more than 65535 batch items");
+    if (n_out % 32 != 0 || k_in % 32 != 0 || !gate.qs_table || !qs_up || !d_up)
+        return pg_fail(PG_EINVAL, "gguf_gemv (digits of act(gate) * up): [%zu, %zu] or a table is missing", n_out, k_in);
+    pg_gemv_epi epi = {};
+    epi.qs1_table = qs_up; epi.d1_table = d_up; epi.act = act; epi.out_digits = out.digits; epi.out_xs = out.xs;
+    return launch_gemv_epi<3, false>(ctx, ggml_type, n_out, k_in, nullptr, nullptr, xd, nullptr, nullptr, epi, gate);
 }
 
 pg_status pg_launch_gguf_gemv(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in,

@@ -347,7 +347,13 @@ struct pg_gemv_epi {
     float ss_inv_dim, eps;
     const uint8_t *qs1;      // the second tensor (up) of the SiLU(gate) * up form
     const uint16_t *d1;
+    const uint8_t *const *qs1_table;  // or, for pairs, every expert's
+    const uint16_t *const *d1_table;
+    int act;
 };
+// act(gate . x) * up . x of every item (a token and an expert) as row `item` of the next product's digits, one launch.
+pg_status pg_launch_gguf_gemv_act_digits(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in, const pg_gemv_batch &gate, const uint8_t *const *qs_up,
+                                         const uint16_t *const *d_up, int act, const pg_xdigits &xd, const pg_xdigits &out);
 // y[item][row] = product (+ residual[item][row] when `residual` is given).
 pg_status pg_launch_gguf_gemv(pg_ctx *ctx, int ggml_type, size_t n_out, size_t k_in,
                               const uint8_t *qs, const uint16_t *d, const pg_gemv_batch &batch,

@@ -9,6 +9,7 @@
 //      (examples/grok1/moe.rs:99-104), raw softmax probabilities.
 #include "pg_internal.h"
 #include "pg_digits.h"
+#include "pg_act_dev.h"
 #include <algorithm>
 
 namespace {
@@ -241,16 +242,6 @@ __global__ __launch_bounds__(64) void tile_offsets_kernel(const int *__restrict_
     goff[experts] = run;
 }
 
-__device__ __forceinline__ float act_silu(float x) {
-    const float sig = 1.0f / (1.0f + expf(-x));
-    return x * sig;
-}
-__device__ __forceinline__ float act_gelu_tanh(float x) {
-    const float c = sqrtf(2.0f / 3.14159265358979323846f);
-    const float inner = c * (x + 0.044715f * x * x * x);
-    return 0.5f * x * (1.0f + tanhf(inner));
-}
-
 // act(g) * u of every pair as the digit planes of the matrix-core product; g and u as the sums of `planes` planes, `stride`
 // floats apart, in ascending order.  (As two launches, with the products through memory: 10.5 us for 128 pairs of 8192, 5.6 here.)
 template <bool NIB>
@@ -277,16 +268,21 @@ __global__ __launch_bounds__(256) void act_mm_digits_kernel(const float *__restr
     const float gf[4] = {gv.x, gv.y, gv.z, gv.w}, uf[4] = {uv.x, uv.y, uv.z, uv.w};
     float o[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = (act == PG_ACT_GELU_TANH ? act_gelu_tanh(gf[i]) : act_silu(gf[i])) * uf[i];
+    for (int i = 0; i < 4; ++i) o[i] = pg_act(act, gf[i]) * uf[i];
     pg_emit_mm_digits<NIB>(o, row, b, sub, nb, nbp, digits, xs);
 }
 
-__global__ void act_mul_kernel(const float *__restrict__ g, const float *__restrict__ u, size_t n,
-                               int act, float *__restrict__ h) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float a = (act == PG_ACT_GELU_TANH) ? act_gelu_tanh(g[i]) : act_silu(g[i]);
-    h[i] = a * u[i];
+// The same as rows of the streaming kernel's digits.
+template <bool NIB>
+__global__ __launch_bounds__(256) void act_digits_kernel(const float *__restrict__ g, const float *__restrict__ u, int act, int nb, int8_t *__restrict__ digits,
+                                                         float *__restrict__ xs) {
+    const size_t row = blockIdx.y;
+    const int b = blockIdx.x * 32 + (threadIdx.x >> 3), sub = threadIdx.x & 7;
+    if (b >= nb) return;  // whole 8-thread groups leave together
+    const size_t at = ((row * nb + b) * 8 + sub) * 4;
+    const float4 gv = *reinterpret_cast<const float4 *>(g + at), uv = *reinterpret_cast<const float4 *>(u + at);
+    const float o[4] = {pg_act(act, gv.x) * uv.x, pg_act(act, gv.y) * uv.y, pg_act(act, gv.z) * uv.z, pg_act(act, gv.w) * uv.w};
+    pg_emit_digits<NIB>(o, row, b, sub, nb, digits, xs);
 }
 
 // yb: the down product's outputs, the sums of `planes` planes (its K chunks) in ascending order.
@@ -469,6 +465,11 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     //    from two tokens on pairs share experts and the matrix-core kernel, which reads an expert once, wins)
     const bool one_token = T == 1;
     const bool down_stream = narrow || one_token || ffn / 32 < PG_MM_MIN_BLOCKS, up_stream = down_stream || d / 32 < PG_MM_MIN_BLOCKS;
+    // Their gate, up and act(gate) * up are then one launch, up to 150 MB of gate weights; beyond, three: workgroups of one wavefront stream more
+    // evenly than the four whose block of 32 outputs becomes digits.  us, four launches : one, the layer: one token, 16 experts of 2304 x
+    // 1376 (Q8_0) 26.2 : 18.0, 8 of 1024 x 2816, top 2 29.0 : 15.8, 8 of 4096 x 14336 (Q4_0) 52.9 : 47.1, Q8_0 (125 MB) 79.1 : 77.7; but 800 pairs
+    // of 1024 x 256 (223 MB) 163 : 166, one token through 2 of 6144 x 32768 (428 MB) 211 : 218, 400 pairs of 2048 x 480 (418 MB) 198 : 225.
+    const bool one_launch = down_stream && (double)P * (double)ffn * (double)d * (type == PG_GGML_Q4_0 ? 0.5625 : 1.0625) <= 1.5e8;
     PG_CHECK_ARG(!(up_stream || down_stream) || P <= 65535, "pg_moe_ffn: too many pairs for experts this small");
 
     // Arena layout.
@@ -481,12 +482,11 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     const size_t sz_idx = pg_round_up(P * sizeof(int), 256);
     const size_t sz_p = pg_round_up(P * sizeof(float), 256);
     const size_t sz_lists = pg_round_up(E * T * sizeof(int), 256), sz_counts = pg_round_up(E * sizeof(int), 256);
-    const size_t sz_act = pg_round_up(P * ffn * sizeof(float), 256), sz_gu = pg_round_up((size_t)ks_up * P * ffn * sizeof(float), 256);
-    const size_t sz_h = down_stream ? sz_act : 0, sz_y = pg_round_up((size_t)ks_down * P * d * sizeof(float), 256);
+    const size_t sz_gu = one_launch ? 0 : pg_round_up((size_t)ks_up * P * ffn * sizeof(float), 256), sz_y = pg_round_up((size_t)ks_down * P * d * sizeof(float), 256);
     const size_t sz_xd = up_stream ? pg_xdigits_bytes(T, d) : pg_mmdigits_bytes(T, d);
     const size_t sz_hd = down_stream ? pg_xdigits_bytes(P, ffn) : pg_mmdigits_bytes(P, ffn);
     void *ws = nullptr;
-    PG_TRY(pg_workspace(ctx, sz_idx + sz_p + sz_lists + sz_counts + 2 * sz_gu + sz_h + sz_y + sz_xd + sz_hd, &ws));
+    PG_TRY(pg_workspace(ctx, sz_idx + sz_p + sz_lists + sz_counts + 2 * sz_gu + sz_y + sz_xd + sz_hd, &ws));
     char *p = static_cast<char *>(ws);
     int *topk_idx = reinterpret_cast<int *>(p); p += sz_idx;
     float *topk_p = reinterpret_cast<float *>(p); p += sz_p;
@@ -494,7 +494,6 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     int *counts = reinterpret_cast<int *>(p); p += sz_counts;
     float *g = reinterpret_cast<float *>(p); p += sz_gu;
     float *u = reinterpret_cast<float *>(p); p += sz_gu;
-    float *h = reinterpret_cast<float *>(p); p += sz_h;
     float *yb = reinterpret_cast<float *>(p); p += sz_y;
     char *xd_base = p; p += sz_xd;
     char *hd_base = p;
@@ -526,8 +525,10 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
     auto dtable = [&](int which) { return reinterpret_cast<const uint16_t *const *>(tab + which * E); };
     // Each token reaches an expert at most once, so an expert owns at most T pairs.
     const int tiles = (int)((T + 31) / 32);
-    if (up_stream) {  // pair p: activation row p / top_k against expert topk_idx[p]
-        const pg_gemv_batch bg = {(int)P, table(0), dtable(1), topk_idx, (int)top_k};
+    const pg_gemv_batch bg = {(int)P, table(0), dtable(1), topk_idx, (int)top_k};  // pair p: activation row p / top_k against expert topk_idx[p]
+    if (one_launch) {
+        PG_TRY(pg_launch_gguf_gemv_act_digits(ctx, type, ffn, d, bg, table(2), dtable(3), act, xd, pg_xdigits_carve(hd_base, P, ffn)));
+    } else if (up_stream) {
         PG_TRY(pg_launch_gguf_gemv(ctx, type, ffn, d, nullptr, nullptr, bg, xd, g));
         const pg_gemv_batch bu = {(int)P, table(2), dtable(3), topk_idx, (int)top_k};
         PG_TRY(pg_launch_gguf_gemv(ctx, type, ffn, d, nullptr, nullptr, bu, xd, u));
@@ -540,18 +541,21 @@ static pg_status moe_ffn_core(pg_ctx *ctx, const float *x_dev, size_t T, const f
         PG_TRY(as_tiles ? pg_launch_gguf_experts_tiles(ctx, type, ffn, d, gg, P, mt, nw, xm, g)
                         : pg_launch_gguf_mm(ctx, type, ffn, d, nullptr, nullptr, gg, P, xm, g, g, true));
     }
+    const int nb = (int)(ffn / 32);
+    const dim3 blocks(grid_for(nb, 32), (unsigned)P);
+    const bool nib = type == PG_GGML_Q4_0;
     if (down_stream) {
-        PG_TRY(pg_launch(ctx, "moe_act_mul", act_mul_kernel, dim3(grid_for(P * ffn, 256)), dim3(256), 0, g, u, P * ffn, act, h));
         const pg_xdigits hd = pg_xdigits_carve(hd_base, P, ffn);
-        PG_TRY(pg_launch_x_to_digits(ctx, h, P, ffn, type, hd));
+        if (!one_launch)
+            PG_TRY(pg_launch(ctx, "moe_act_digits", nib ? act_digits_kernel<true> : act_digits_kernel<false>, blocks, dim3(256), 0, (const float *)g,
+                             (const float *)u, act, nb, hd.digits, hd.xs));
         const pg_gemv_batch bd = {(int)P, table(4), dtable(5), topk_idx, 1};
         PG_TRY(pg_launch_gguf_gemv(ctx, type, d, ffn, nullptr, nullptr, bd, hd, yb));
     } else {
         const pg_mmdigits hd = pg_mmdigits_carve(hd_base, P, ffn);
-        const int nb = (int)(ffn / 32);
-        auto *kern = type == PG_GGML_Q4_0 ? act_mm_digits_kernel<true> : act_mm_digits_kernel<false>;
+        auto *kern = nib ? act_mm_digits_kernel<true> : act_mm_digits_kernel<false>;
         if (P > 65535) return pg_fail(PG_EUNSUPPORTED, "pg_moe_ffn: more than 65535 pairs");
-        PG_TRY(pg_launch(ctx, "moe_act_mm_digits", kern, dim3(grid_for(nb, 32), (unsigned)P), dim3(256), 0, (const float *)g, (const float *)u,
+        PG_TRY(pg_launch(ctx, "moe_act_mm_digits", kern, blocks, dim3(256), 0, (const float *)g, (const float *)u,
                          ks_up, P * ffn, act, nb, (int)pg_round_up(nb, 4), hd.digits, hd.xs));
         const pg_mm_group gd = {(int)E, table(4), dtable(5), lists, counts, (int)T, tiles, (int)T, 1, 0, 0, 1};
         PG_TRY(as_tiles ? pg_launch_gguf_experts_tiles(ctx, type, d, ffn, gd, P, mt, nw, hd, yb)

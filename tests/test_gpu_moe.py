@@ -68,6 +68,31 @@ def test_moe_one_token_streams_its_experts(ctx, orc, typ):
     H.assert_close_rel(got3[0], got1, MOE_RTOL, "the same token in a batch")
 
 
+@pytest.mark.parametrize("T,d,ffn,E,top_k,act,one", [
+    (1, 160, 32, 3, 3, 1, True), (1, 2080, 96, 2, 1, 0, True), (1, 4128, 480, 2, 2, 1, True), (1, 8224, 64, 2, 1, 0, True),  # 1, 2 and 3 .. 4 blocks a lane, two runs of K
+    (1, 96, 1376, 4, 4, 0, True), (5, 512, 480, 4, 2, 1, True), (33, 64, 224, 3, 2, 0, True),                                # narrow experts of more tokens
+    (40, 7168, 480, 2, 2, 0, False),                                                                                          # beyond the line: a launch for each
+])
+@pytest.mark.parametrize("typ", [8, 2])
+def test_moe_streamed_pairs_in_one_launch(ctx, orc, typ, T, d, ffn, E, top_k, act, one):
+    """Gate, up, act(gate) * up and its digits of streamed pairs in one launch: every number of blocks a lane, the smallest experts, and
+    both sides of the line; the launches tell which."""
+    from peregrine_amd import gguf, moe
+    say(f"moe streamed pairs typ={typ} T={T} d={d} ffn={ffn} E={E} top_k={top_k} act={act}")
+    raws = build(orc, 190 + d + ffn, d, ffn, E, typ)
+    x = orc.rng_normal(15 + T, T * d)
+    logits = orc.rng_normal(16 + T, T * E).reshape(T, E)
+    mk = lambda rs, n_out, k_in: [gguf.GgufWeight(r, typ, n_out, k_in, ctx) for r in rs]
+    ex = moe.MoEExperts(mk(raws[0], ffn, d), mk(raws[1], ffn, d), mk(raws[2], d, ffn), top_k, act, ctx)
+    ctx.profile_begin()
+    got = ex.forward(x, logits).reshape(T, d)
+    prof = ctx.profile_end()
+    assert any(k.endswith("_act_digits") and k.startswith("gguf_gemv") for k in prof) == one and ("moe_act_digits" in prof) != one, prof
+    want, _, _ = orc.moe_ffn(x, T, d, ffn, E, top_k, logits, raws[0], raws[1], raws[2], typ, act)
+    for t in range(T):
+        H.assert_close_rel(got[t], want.reshape(T, d)[t], MOE_RTOL, f"token {t}")
+
+
 def test_moe_grok_shaped_reduced(ctx, orc):
     """benchmark configuration 5's structure (8 experts, top-2, 64 tokens, Q8_0, SiLU) at reduced
     width (d 512, ffn 1024) so the oracle finishes in seconds."""
