@@ -65,7 +65,7 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 }
 
 __device__ __forceinline__ float block_max(float v, float *red) {
-    for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
+    v = pg_wave_max_f32(v);
     const int wave = threadIdx.x >> 6;
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[wave] = v;
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(attn_args aa) {
                     if (d0 + j < hd) dot += q4[j] * kr[j];
             }
         }
-        for (int m = 1; m < L; m <<= 1) dot += __shfl_xor(dot, m);
+        dot = pg_group_sum_f32(dot, L);
         if (kt < n) {
             float s = -INFINITY;
             if (live) {
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(256) void gqa_attention_short_kernel(attn_args aa) 
 #pragma unroll
     for (int u = 0; u < ATT_SHORT_ROUNDS; ++u) {
         float dot = q4.x * kv[u].x + q4.y * kv[u].y + q4.z * kv[u].z + q4.w * kv[u].w;
-        for (int m = 1; m < L; m <<= 1) dot += __shfl_xor(dot, m);
+        dot = pg_group_sum_f32(dot, L);
         s[u] = -INFINITY;
         if (live[u]) {
             s[u] = dot * aa.scale;

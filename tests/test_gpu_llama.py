@@ -141,6 +141,15 @@ def test_gqa_attention_unmasked(ctx, orc, nqh, nkvh, hd, seq_q, length):
                     appends=(1, length - 1) if length > 1 else None)
 
 
+@pytest.mark.parametrize("hd", [2, 4, 8, 16, 32, 64, 96, 128, 192, 256])
+@pytest.mark.parametrize("seq_q,length", [(3, 37), (70, 150)])
+def test_gqa_attention_every_number_of_lanes_a_key(ctx, orc, hd, seq_q, length):
+    """1 to 64 lanes sum a key's score: few rows (the short kernel) and, where no matrix-core kernel has the head size, many."""
+    from peregrine_amd import llama
+    say(f"attention hd={hd} seq_q={seq_q} len={length}")
+    _attention_case(ctx, orc, 4, 2, hd, seq_q, length, llama.AttentionMask.causal(length - seq_q), None, 300 + hd)
+
+
 def test_gqa_attention_masks_and_logit_cap(ctx, orc):
     from peregrine_amd import llama
     M = llama.AttentionMask
