@@ -10,6 +10,7 @@
 #include "pg_internal.h"
 #include "pg_digits.h"
 #include "pg_act_dev.h"
+#include "pg_quant_dev.h"
 #include <algorithm>
 
 namespace {
@@ -68,6 +69,36 @@ inline bool route_in_one(size_t T, size_t E, size_t top_k, bool logits) {
     // past it 32 experts 0.7 to 1.0 of their time, 64 0.95 to 1.7, more 0.86 to 4.9.)
     return T * top_k * E <= (1u << 17) && route_lds(T, E, top_k, logits) <= MAX_ROUTE_LDS;
 }
+// A token's softmax and top-k on one wavefront, a lane an expert (up to 64): the steps of the thread's loops in route_lists_kernel, whose every look at an
+// expert waits for LDS -- E (3 + k) of them one behind the other, some 130 cycles each, are 6 us for 16 experts and 4 choices.  The sum
+// of the exponentials is added up in the same order; a NaN anywhere makes the sum and with it every probability NaN, and the lowest experts
+// not taken are the choice.
+__device__ __forceinline__ void route_token(const float *x, int E, int top_k, uint8_t *mine, int *idx, float *p_out) {
+    const int lane = threadIdx.x & 63;
+    const bool in = lane < E;
+    const float v = in ? x[lane] : -INFINITY, mx = pg_wave_max_f32(v);
+    const float ex = expf(v - mx);
+    float sum = 0.0f;
+    for (int e = 0; e < E; ++e) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ex), e));
+    const float p = ex / sum;
+    bool free = in;
+    for (int k = 0; k < top_k; ++k) {
+        const float best = pg_wave_max_f32(free ? p : -1.0f);
+        const unsigned long long at = __ballot(free && (p == best || p != p));
+        const int e = __ffsll(at) - 1;
+        if (lane == e) {
+            free = false;
+            mine[k] = (uint8_t)e;
+            idx[k] = e;
+            p_out[k] = p;
+        }
+    }
+}
+// Up to 16 tokens, a wavefront each; a second round of them is as long as the first (1.3 us, 16 experts and 4 choices), where all threads' walks are one.  us, a
+// layer, a thread a token : a wavefront: one token, 4 of 16 experts of 2400 x 2080 (Q4_0) 26.6 : 22.4, 8 of 32 of 2048 x 768 35.1 : 18.9, 2 of 8 of 1024 x 2816 (Q8_0)
+// 16.1 : 14.9, 10 tokens, 4 of 8 of 896 x 7936 55.4 : 54.1; but 45, 2 of 16 of 608 x 2656 36.9 : 37.8, 64, 4 of 16 of 2048 x 2048 61.9 : 64.3.
+__device__ __forceinline__ bool route_by_wave(int T, int E) { return T <= 16 && E <= 64; }
+
 struct route_digits {
     const float *x;
     int nb, nbp, blocks;  // blocks of 32 a row, the same rounded up to 4, blocks of all rows
@@ -98,7 +129,12 @@ __global__ __launch_bounds__(1024) void route_lists_kernel(const float *__restri
         for (int i = threadIdx.x; i < T * E; i += 1024) prob[i / E * row + i % E] = logits[i];
         __syncthreads();
     }
-    for (int t = threadIdx.x; t < T; t += 1024) {
+    const bool by_wave = LOGITS && route_by_wave(T, E);
+    if (by_wave) {
+        const int t = threadIdx.x >> 6;
+        if (t < T) route_token(prob + t * row, E, top_k, chosen + t * top_k, topk_idx + t * top_k, topk_p + t * top_k);
+    }
+    for (int t = threadIdx.x; !by_wave && t < T; t += 1024) {
         uint8_t *mine = chosen + t * top_k;
         if (LOGITS) {
             float *x = prob + t * row;

@@ -377,6 +377,15 @@ def test_moe_routing_in_one_launch_and_split_products(ctx, orc, T, E, top_k, d, 
 
 
 @pytest.mark.parametrize("T,E,top_k,d,ffn,typ", [
+    (5, 16, 16, 160, 512, 8), (16, 2, 1, 160, 512, 2), (11, 64, 8, 160, 512, 8), (11, 65, 8, 160, 512, 8),  # 64 experts are a wavefront's lanes
+    (16, 8, 2, 160, 512, 8), (17, 8, 2, 160, 512, 8), (16, 1, 1, 160, 512, 8), (17, 64, 4, 160, 512, 2),       # both sides of the line
+])
+def test_moe_routing_of_a_token_on_a_wavefront(ctx, orc, T, E, top_k, d, ffn, typ):
+    """The same choices and probabilities by a lane an expert: all experts chosen, ties, infinite and NaN logits."""
+    test_moe_routing_in_one_launch_and_split_products(ctx, orc, T, E, top_k, d, ffn, typ)
+
+
+@pytest.mark.parametrize("T,E,top_k,d,ffn,typ", [
     (2, 4, 1, 512, 512, 8), (8, 2, 2, 544, 1056, 2), (9, 2, 2, 544, 1056, 8), (17, 3, 2, 608, 992, 2),   # tiles of 8 and 16 pairs and past them
     (33, 5, 2, 1024, 544, 8), (64, 1, 1, 512, 1024, 8), (65, 70, 2, 512, 544, 2), (130, 130, 1, 512, 512, 8),  # past 64 and 128 experts
 ])
