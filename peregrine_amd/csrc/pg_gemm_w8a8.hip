@@ -946,11 +946,22 @@ struct split_kernel {
 constexpr split_kernel SPLITS[] = {{128, 1, {0.515}, 0.100, 8.446, 0.001, 0.105, 1.906, 0.081, -1.719}, {64, 2, {0.487, 0.356}, 0.734, 6.675, 0.011, 0.120, 2.157, 0.037, -2.542}};
 constexpr size_t SPLIT_ROWS = 700, SPLIT_TILES = 40, SPLIT_TILES64 = 33;
 constexpr double split_margin(size_t tiles128) { return tiles128 <= 32 ? 0.97 : tiles128 <= SPLIT_TILES ? 0.92 : 0.79; }
+constexpr size_t SPLIT_RUNS = 16;  // of K, at the most
+// The most partial sums that a product of up to m rows leaves where an XCD's `places` hold all runs of its tiles.  More rows are more tiles and then
+// fewer runs, so a product may leave more than a larger one does; the scratch is taken for the most, so that a program that has run
+// its largest batch finds it large enough for every other one, also under a capture, and no graph's scratch is freed (8192 -> 643 took 13.6 MB at 488 rows
+// and 11.5 at 1024).  r runs are for up to places / r tiles an XCD.
+size_t most_partial_sums(size_t m, size_t n, size_t tile, size_t places, size_t most_runs) {
+    const size_t columns = (n + tile - 1) / tile;
+    size_t most = 0;
+    for (size_t r = 2; r <= most_runs && r <= places; ++r) most = std::max(most, r * n * std::min(m, 8 * (places / r) / columns * tile));
+    return most;
+}
 // The runs of K, none of them empty, and the k-tiles of one.
 unsigned split_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, const split_kernel &s, unsigned *per) {
     const size_t tiles = ((m + s.tile - 1) / s.tile) * ((w->cols + s.tile - 1) / s.tile), kt = w->k_pad / 128;
     // (the places of an XCD, which has all runs of its tiles; at least two k-tiles a run)
-    const size_t runs = std::max<size_t>(1, std::min<size_t>({s.resident * (size_t)(ctx->num_cu / 8) / ((tiles + 7) / 8), kt / 2, 16}));
+    const size_t runs = std::max<size_t>(1, std::min<size_t>({s.resident * (size_t)(ctx->num_cu / 8) / ((tiles + 7) / 8), kt / 2, SPLIT_RUNS}));
     *per = (unsigned)((kt + runs - 1) / runs);
     return (unsigned)((kt + *per - 1) / *per);
 }
@@ -958,6 +969,12 @@ unsigned split_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, const spli
 size_t pg_gemm_w8a8_split_bytes(const pg_ctx *ctx, const pg_qtensor *w, size_t m, int index) {
     unsigned per;
     return (size_t)split_runs(ctx, w, m, SPLITS[index], &per) * m * w->cols * sizeof(int32_t);
+}
+size_t pg_gemm_w8a8_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+    size_t values = 0;
+    for (const split_kernel &s : SPLITS)
+        if (m >= 33) values = std::max(values, most_partial_sums(std::min(m, SPLIT_ROWS), w->cols, s.tile, s.resident * (size_t)(ctx->num_cu / 8), std::min<size_t>(w->k_pad / 256, SPLIT_RUNS)));
+    return values * sizeof(int32_t);
 }
 pg_status pg_launch_gemm_w8a8_split(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales, const pg_qtensor *w, size_t m,
                                     float *out, int32_t *acc, int32_t *part, int index) {
@@ -1323,16 +1340,14 @@ static unsigned w8a32_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, uns
     *per = each;
     return runs;
 }
-size_t pg_gemm_w8a32_part_bytes(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
-    unsigned per;
-    const unsigned runs = w8a32_runs(ctx, w, m, &per);
-    return runs > 1 ? (size_t)runs * m * w->cols * sizeof(double) : 0;
+size_t pg_gemm_w8a32_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
+    return m <= 32 ? 0 : most_partial_sums(m, w->cols, 64, (size_t)ctx->num_cu / 8, std::min<size_t>(w->k_pad / 256, W8A32_RUNS)) * sizeof(double);
 }
 pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part) {
     if (!pg_gemm_w8a32_takes(ctx, w, m)) return pg_fail(PG_EINVAL, "gemm_w8a32: m = %zu", m);
     const size_t k_pad = w->k_pad, n = w->cols;
     unsigned per;
-    if (const unsigned runs = part ? w8a32_runs(ctx, w, m, &per) : 1; runs > 1) {
+    if (const unsigned runs = w8a32_runs(ctx, w, m, &per); runs > 1) {
         PG_TRY((launch_group<64, 64, 128, 3, 4, 2, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, static_cast<int32_t *>(part), (int)runs, (int)per, nullptr, 0, plane_bytes)));
         auto finish = [&](auto kern, size_t v) {
             return pg_launch(ctx, "gemm_w8a32_finish", kern, dim3((unsigned)((m * n / v + 255) / 256)), dim3(256), 0, (const double *)part, (int)runs,

@@ -260,8 +260,8 @@ pg_status pg_launch_gemm_w8a8_combine(pg_ctx *ctx, const int8_t *a_i8, size_t a_
                                       const pg_qtensor *w, size_t m, float *out, const int32_t *comb, size_t comb_plane);
 // The W8A32 product over three digit planes (plane_bytes apart) in one launch, where it takes it.
 bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
-// `part`: pg_gemm_w8a32_part_bytes of scratch where it splits K over workgroups, else null.
-size_t pg_gemm_w8a32_part_bytes(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
+// `part`: pg_gemm_w8a32_split_room of scratch, for the partial sums where K is split over workgroups.
+size_t pg_gemm_w8a32_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
 pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part);
 // How W8A8 products of two rows and more run: tiles, the few-row kernel (2 .. 512 rows), or tiles with K split over workgroups (33 .. 700 rows
 // over one weight: i32 partial sums in `part`, pg_gemm_w8a8_split_bytes of them, and a finishing launch); `index` names the kernel.
@@ -269,6 +269,7 @@ enum pg_w8a8_kind { PG_W8A8_TILES, PG_W8A8_ROWS, PG_W8A8_SPLIT };
 struct pg_w8a8_route { pg_w8a8_kind kind; int index; };
 pg_w8a8_route pg_gemm_w8a8_route(const pg_ctx *ctx, const pg_qtensor *const *w, int count, size_t m);
 size_t pg_gemm_w8a8_split_bytes(const pg_ctx *ctx, const pg_qtensor *w, size_t m, int index);
+size_t pg_gemm_w8a8_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m);  // the most that products of up to m rows need
 pg_status pg_launch_gemm_w8a8_split(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales, const pg_qtensor *w, size_t m,
                                     float *out, int32_t *acc, int32_t *part, int index);
 pg_status pg_launch_gemm_w8a8_skinny_group(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const float *a_scales,

@@ -546,6 +546,31 @@ def test_int8_products_are_captured_after_one_eager_call(host, n, k):
         same_call_captured(host, "pg_matmul_dequant_i8_dev", x, m, k, q, y)
 
 
+@pytest.mark.parametrize("call", ["pg_matmul_quantized_dev", "pg_matmul_dequant_i8_dev"])
+@pytest.mark.parametrize("n,k", [(643, 8192), (832, 7055), (756, 5127), (134, 8143), (4096, 14336), (2373, 6563), (289, 12805), (534, 8337), (50257, 256)])
+def test_int8_products_of_fewer_rows_need_no_more_scratch(host, call, n, k):
+    """A program that has run its largest batch captures any smaller one: K is split over workgroups, with partial sums in the scratch, for some
+    numbers of rows only (8192 -> 643: 488, but not 1024), and the workspace does not grow for them.  Nor does it grow eagerly, which would free
+    the one that an earlier graph writes."""
+    w = host.alloc(n * k)
+    q = host.new("pg_qtensor_from_f32_dev", host.ctx, w, k, n)
+    rows = sorted({1, 5, 33, 48, 62, 64, 65, 97, 129, 200, 257, 286, 320, 321, 385, 467, 488, 513, 645, 700, 701, 900, 1024, 2048}, reverse=True)
+    x, y = host.alloc(rows[0] * k), host.alloc(rows[0] * n)
+    args = lambda m: (x, m, k, q, y) + ((None,) if call == "pg_matmul_quantized_dev" else ())
+    for i, largest in enumerate(rows):
+        ctx = host.new("pg_ctx_create", 0, None)
+        host.ok(call, ctx, *args(largest))
+        used = host.lib.pghost_used()
+        for m in rows[i + 1:]:
+            host.lib.pghost_begin_capture(host.stream(ctx))
+            st = getattr(host.lib, call)(ctx, *args(m))
+            assert host.lib.pghost_end_capture(host.stream(ctx)) and st == 0, (largest, m, host.lib.pg_last_error())
+            host.ok(call, ctx, *args(m))
+            assert host.lib.pghost_used() == used, (largest, m)
+        host.lib.pg_ctx_destroy(ctx)
+    host.lib.pg_qtensor_free(host.ctx, q)
+
+
 def test_expert_layers_are_captured_after_one_eager_call(host):
     d, ffn, E, k = 256, 512, 8, 2
     tab = lambda n_out, k_in: (C.c_void_p * E)(*[host.new("pg_gguf_upload", host.ctx, bytes(n_out * k_in // 32 * 34), 8, n_out, k_in).value for _ in range(E)])
