@@ -148,17 +148,17 @@ PG_API pg_status pg_audit_gguf_skinny(size_t n_out, size_t k_in, int q8, int nw,
     return PG_OK;
 }
 
-// Many rows on the f16 matrix cores (gguf_hmm_kernel<QT, MT, S>): its largest tile, 128 x 512 (wide = 1: the lower and the narrower tiles' rows are
-// clamped alike), or one of 256 x 256 (wide = 0),
-// K in `ks` chunks of whole stages of 64; the planes are [m][k_in] f16, the payload [n_out][k_in / 32][16 B] (Q8_0: [n_out][2][k_in / 32][16 B]).
-// (Every offset is linear in the stage: the first and the last stage of a chunk bound the rest.)
+// Many rows on the f16 matrix cores (gguf_hmm_kernel<QT, MT, S>): its tallest tiles, 128 rows (the lower ones' are clamped alike) x 512 weight rows (wide = 1,
+// S = 1) or 256 (wide = 0, S = 2), K in `ks` chunks of whole stages of 64 (those that S = 2 does not take run as S = 1); the planes are
+// [m][k_in] f16, the payload [n_out][k_in / 32][16 B] (Q8_0: [n_out][2][k_in / 32][16 B]).
+// (Every offset is linear in the stage: the first and the last stage of a chunk bound the rest.  S = 2 asks for a chunk's first two whatever it has.)
 PG_API pg_status pg_audit_gguf_hmm(size_t m, size_t n_out, size_t k_in, int q8, int wide, int ks, size_t *plane_end, size_t *plane_bytes,
                                    size_t *qs_end, size_t *qs_bytes, size_t *d_end, size_t *d_bytes) {
     PG_CHECK_ARG(m > 0 && n_out >= 2 && k_in >= 64 && k_in % 64 == 0 && ks >= 1, "pg_audit_gguf_hmm: bad arguments");
     const int nb = (int)(k_in / 32), K = (int)k_in, M = (int)m, N = (int)n_out;
-    PG_CHECK_ARG(!q8 || wide, "pg_audit_gguf_hmm: Q8_0 runs the 128 x 512 tiles only");
-    const int nwn = wide ? 8 : 4, bm = wide ? 128 : 256, bn = 64 * nwn, lx = bm / 64, lw = (bn * (q8 ? 64 : 32) / 1024 + 7) / 8;
     const int stages = nb / 2, kt_per = (stages + ks - 1) / ks;
+    const int s = wide || !pg_hmm_chunk((unsigned)stages, (unsigned)ks, 2) ? 1 : 2;
+    const int nwn = 8 / s, bm = 128, bn = 64 * nwn, lx = bm / 64, lw = (bn * (q8 ? 64 : 32) / 1024 + 7) / 8;
     const int tiles_m = (M + bm - 1) / bm, panels = (N + bn - 1) / bn;
     auto swz128 = [](int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); };
     span_check pl, qs, d;
@@ -169,7 +169,7 @@ PG_API pg_status pg_audit_gguf_hmm(size_t m, size_t n_out, size_t k_in, int q8, 
                 const int m0 = tm * bm, n0 = np * bn;
                 for (int wave = 0; wave < 8; ++wave)
                     for (int lane = 0; lane < 64; ++lane)
-                        for (int st : {kt0, kt0 + kt_n - 1}) {
+                        for (int st : {kt0, kt0 + s - 1, kt0 + kt_n - 1}) {
                             for (int i = 0; i < lx; ++i) {
                                 const int row = 8 * (wave + 8 * i) + (lane >> 3);
                                 pl.touch(pg_hmm_plane_offset(pg_hmm_clamp_row(m0 + row, M), K, st, (lane & 7) ^ swz128(row)), 16);

@@ -592,11 +592,6 @@ pg_status pg_launch_rows_to_f16_planes(pg_ctx *ctx, const float *x_dev, size_t r
 // best (mt, s, ks) of an earlier fit and four others timed on each): on the others 4.5 % mean error with s = 1 and 3.8 with s = 2, and what is picked
 // takes 0.5 % longer than the best on average; the best with s = 1 alone takes 7 % more, with s = 2 alone 1.  (Q4_1's chunks are read by its offsets' launch.)
 struct hmm_plan { int mt, s, ks; double us; };
-// The stages of a K chunk (all but the last), 0: one would be empty, or (s = 2: the kernel's first two are requested together) of a single stage.
-static unsigned hmm_chunk(unsigned stages, unsigned ks, int s) {
-    const unsigned per = ks == 1 ? stages : (stages + ks - 1) / ks;
-    return (ks - 1) * per + (unsigned)s <= stages ? per : 0;
-}
 static hmm_plan hmm_plan_for(const pg_ctx *ctx, bool q8, size_t m_, size_t n_total, size_t k_in, int ks_fixed, bool keep) {
     // (a call waits for this: 32-bit divisions, and no more chunks once there are three rounds)
     hmm_plan best = {8, 1, 1, 1e300};
@@ -609,7 +604,7 @@ static hmm_plan hmm_plan_for(const pg_ctx *ctx, bool q8, size_t m_, size_t n_tot
             for (unsigned ks = ks_fixed > 0 ? (unsigned)ks_fixed : 1; ks <= (ks_fixed > 0 ? (unsigned)ks_fixed : 8u); ++ks) {
                 const unsigned rounds = ((tiles * ks + 7) / 8 + cus_per_xcd - 1) / cus_per_xcd;
                 if (ks_fixed <= 0 && ks > 1 && rounds > 3) break;
-                const unsigned per = hmm_chunk(stages, ks, s);
+                const unsigned per = pg_hmm_chunk(stages, ks, s);
                 if (!per || (ks_fixed <= 0 && ks > 1 && per < 8)) continue;
                 const double idle = 1.0 - (double)(tiles * ks) / (double)(rounds * cus_per_xcd * 8);
                 double us = s == 1 ? rounds * (per * (0.752 + 0.293 * mt + 0.241 * x) + 3.07 + 0.874 * mt) * (1.0 - 0.138 * idle)
@@ -718,7 +713,7 @@ pg_status pg_launch_gguf_hmm_group(pg_ctx *ctx, size_t k_in, const pg_gguf_tenso
         }
     }
     const int tiles_m = (int)((m + bm - 1) / bm), ntiles = tiles_m * panels;
-    const int kt_per = (int)hmm_chunk((unsigned)(k_in / 64), (unsigned)ks, plan.s);
+    const int kt_per = (int)pg_hmm_chunk((unsigned)(k_in / 64), (unsigned)ks, plan.s);
     if (kt_per == 0) return pg_fail(PG_EINVAL, "gguf (f16 matrix cores): %d K chunks of %zu stages leave one empty", ks, k_in / 64);
     const dim3 grid((unsigned)(((size_t)ntiles * ks + 7) / 8 * 8));
     const int nb = (int)(k_in / 32);

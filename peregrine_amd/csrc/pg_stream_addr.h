@@ -107,6 +107,11 @@ PG_HD size_t pg_mt_scale_store(size_t tg, int ncp, int b, int col) {
 
 // ---- many rows on the f16 matrix cores (gguf_hmm_kernel): per stage of two blocks a wavefront fills its share
 // of the two activation planes, of the packed weights and of their scales
+// The stages of a K chunk (all but the last), 0: one would be empty, or (s = 2: the kernel's first two are requested together) of a single stage.
+PG_HD unsigned pg_hmm_chunk(unsigned stages, unsigned ks, int s) {
+    const unsigned per = ks == 1 ? stages : (stages + ks - 1) / ks;
+    return (ks - 1) * per + (unsigned)s <= stages ? per : 0;
+}
 // activation or weight row a fill lane fetches: rows past the end repeat the last (their outputs are never stored)
 PG_HD int pg_hmm_clamp_row(int row, int rows) { return row < rows ? row : rows - 1; }
 // byte offset in an f16 plane [rows][k]: row, stage (64 k = 128 bytes), 16-byte chunk of the stage's run

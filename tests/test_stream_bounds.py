@@ -130,6 +130,19 @@ def test_f16_matrix_core_fills_stay_inside_planes_payload_and_scales():
                 assert de <= db, (what, de, db)
 
 
+@pytest.mark.parametrize("q8", [0, 1])
+def test_f16_matrix_core_fills_of_the_half_wide_tiles_stay_inside(q8):
+    """gguf_hmm_kernel<QT, MT, 2>: 256 weight rows a workgroup, a chunk's first two stages asked for before the first is looked at (an odd
+    number of stages, and chunks of two)."""
+    for m, n, k in itertools.product([2, 49, 127, 128, 129, 300], [2, 77, 255, 256, 257, 515, 1100], [256, 320, 576, 1088, 4096]):
+        for ks in range(1, 9):
+            v = [C.c_size_t() for _ in range(6)]
+            check(lib.pg_audit_gguf_hmm(m, n, k, q8, 0, ks, *[C.byref(x) for x in v]))
+            pe, pb, qe, qb, de, db = (x.value for x in v)
+            what = f"gguf_hmm m={m} n={n} k={k} q8={q8} ks={ks}"
+            assert pe == pb and qe == qb and de <= db, (what, pe, pb, qe, qb, de, db)
+
+
 def test_mxfp4_rows_loads_stay_inside_the_fragment_planes():
     for k, n in itertools.product([32, 64, 512, 2880, 4096, 28160], [1, 15, 16, 17, 100, 2880]):
         for rg, nw in ((1, 16), (1, 8), (2, 8), (4, 8), (8, 8), (1, 4), (2, 4), (4, 4)):
