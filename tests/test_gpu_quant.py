@@ -633,6 +633,21 @@ def test_matmul_dequant_i8_vs_oracle(ctx, orc, m, k, n):
     qt.free_gpu()
 
 
+@pytest.mark.parametrize("m,k,n,runs", [(587, 4137, 316, 9), (670, 8232, 281, 9)])
+def test_products_split_over_k_whose_last_run_is_one_tile_of_k(ctx, orc, m, k, n, runs):
+    """33 k-tiles in runs of four, 65 in runs of eight."""
+    from peregrine_amd import quant
+    say(f"split over K, a last run of one k-tile, m={m} k={k} n={n}")
+    a = orc.rng_normal(99 + m, m * k)
+    qt = quant.quantize_weights(orc.rng_normal(98 + n, k * n, 0.0, 0.02), k, n, ctx)
+    got, got_acc = run_matmul_dev(ctx, a, m, k, qt)
+    assert last_tile(ctx) == (64, 64, runs)
+    rows = sorted({0, 63, m // 2, m - 1})
+    want, want_acc = orc.matmul_quantized(a.reshape(m, k)[rows].reshape(-1), len(rows), k, qt.data_i8_t, qt.scales, n)
+    assert (got_acc.reshape(m, n)[rows].reshape(-1) == want_acc.reshape(-1)).all()
+    assert (bits(got.reshape(m, n)[rows]).reshape(-1) == bits(want).reshape(-1)).all()
+
+
 @pytest.mark.parametrize("m,k,n,runs", [(286, 7055, 832, 3), (768, 8136, 111, 8), (57, 10391, 3087, 4), (485, 7086, 294, 6), (164, 9108, 1114, 4), (330, 12000, 130, 8), (33, 132000, 7, 8)])
 def test_matmul_dequant_i8_split_over_k(ctx, orc, m, k, n, runs):
     """K in runs over workgroups: whole numbers as activations and powers of two as scales make the product exact, in even and odd
@@ -654,6 +669,40 @@ def test_matmul_dequant_i8_split_over_k(ctx, orc, m, k, n, runs):
         assert last_tile(ctx) == (64, 64, runs)
         got = y.to_host(np.float32)[at:at + m * n].reshape(m, n)[rows]
         assert (got == want).all()
+    qt.free_gpu()
+
+
+@pytest.mark.parametrize("m,k,n,runs", [(286, 7055, 832, 3), (768, 7200, 111, 8), (57, 10391, 3087, 4), (164, 9108, 1114, 4), (33, 20000, 7, 8)])
+def test_matmul_dequant_i8_split_over_k_rounds_once(ctx, orc, m, k, n, runs):
+    """Ordinary rows, of a small and of a large scale, of infinities and of NaN: K in runs (the last of 768 x 7200 a single k-tile) gives the bits of the whole
+    product, which a tile override makes in another way."""
+    from peregrine_amd import quant, _ffi
+    say(f"matmul_dequant_i8 split against whole m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, ::53] *= 20.0
+    a[1] *= np.float32(1e-30)
+    a[2] *= np.float32(1e30)
+    a[3, k // 2], a[4, 0] = np.inf, np.nan
+    qt = quant.quantize_weights(orc.rng_normal(77 + n, k * n, 0.0, 0.02), k, n, ctx)
+    qt.to_gpu(ctx)
+    x, y = DevBuf(ctx, host=a), DevBuf(ctx, m * n * 4)
+    got = []
+    for tile in (0, 1):
+        _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, tile))
+        try:
+            _ffi.check(_ffi.lib.pg_matmul_dequant_i8_dev(ctx.handle, x.ptr, m, k, qt._gpu, y.ptr))
+            ctx.sync()
+        finally:
+            _ffi.check(_ffi.lib.pg_gemm_w8a8_force_tile(ctx.handle, 0))
+        assert last_tile(ctx)[2] == (1 if tile else runs)
+        got.append(y.to_host(np.float32).copy().reshape(m, n))
+    same = (bits(got[0]) == bits(got[1])).reshape(m, n) | (np.isnan(got[0]) & np.isnan(got[1]))
+    assert same.all(), np.argwhere(~same)[:5]
+    assert np.isfinite(got[0][5:]).all() and (np.abs(got[0][5:]).max(axis=1) > 0).all()
+    exact = a[5:].astype(np.float64) @ orc.dequantize(qt.data_i8, qt.scales, k, n).reshape(k, n).astype(np.float64)
+    for r in (0, m // 2, m - 6):
+        H.assert_close_rel(got[0][5 + r], exact[r], 1e-5, f"row {5 + r} vs exact")
     qt.free_gpu()
 
 
