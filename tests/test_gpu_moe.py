@@ -376,6 +376,31 @@ def test_moe_routing_in_one_launch_and_split_products(ctx, orc, T, E, top_k, d, 
         H.assert_close_rel(again[t], got[keep][t], 1e-4, f"the routing handed in, row {t}")
 
 
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("typ,T,d,ffn,E,top_k", [(2, 40, 7168, 480, 2, 2), (8, 25, 7168, 480, 2, 2), (8, 50, 9216, 192, 3, 2), (2, 150, 4160, 448, 4, 2)])
+def test_moe_streamed_pairs_in_one_launch_are_the_bits_of_three(ctx, orc, typ, T, d, ffn, E, top_k, act):
+    """The rows of a call beyond the line, which takes a launch each for gate, up and the activation's digits, are those of calls of
+    a few of its tokens, and of one, which take one launch (and whose routing is a wavefront a token)."""
+    from peregrine_amd import gguf, moe
+    say(f"moe one launch against three typ={typ} T={T} d={d} ffn={ffn} E={E} top_k={top_k} act={act}")
+    raws = build(orc, 190 + d + ffn, d, ffn, E, typ)
+    x = orc.rng_normal(15 + T, T * d).reshape(T, d)
+    logits = orc.rng_normal(16 + T, T * E).reshape(T, E)
+    mk = lambda rs, n_out, k_in: [gguf.GgufWeight(r, typ, n_out, k_in, ctx) for r in rs]
+    ex = moe.MoEExperts(mk(raws[0], ffn, d), mk(raws[1], ffn, d), mk(raws[2], d, ffn), top_k, act, ctx)
+
+    def rows(of, one):
+        ctx.profile_begin()
+        got = np.asarray(ex.forward(np.ascontiguousarray(x[of]), np.ascontiguousarray(logits[of])), np.float32).reshape(-1, d)
+        prof = ctx.profile_end()
+        assert any(k.startswith("gguf_gemv") and k.endswith("_act_digits") for k in prof) == one and ("moe_act_digits" in prof) != one, prof
+        return got.view(np.uint32)
+
+    whole = rows(slice(0, T), False)
+    for of in (slice(0, 7), slice(T - 16, T), slice(3, 4), slice(T - 1, T)):
+        assert (rows(of, True) == whole[of]).all(), of
+
+
 @pytest.mark.parametrize("T,E,top_k,d,ffn,typ", [
     (5, 16, 16, 160, 512, 8), (16, 2, 1, 160, 512, 2), (11, 64, 8, 160, 512, 8), (11, 65, 8, 160, 512, 8),  # 64 experts are a wavefront's lanes
     (16, 8, 2, 160, 512, 8), (17, 8, 2, 160, 512, 8), (16, 1, 1, 160, 512, 8), (17, 64, 4, 160, 512, 2),       # both sides of the line
