@@ -142,12 +142,65 @@ def test_gqa_attention_unmasked(ctx, orc, nqh, nkvh, hd, seq_q, length):
 
 
 @pytest.mark.parametrize("hd", [2, 4, 8, 16, 32, 64, 96, 128, 192, 256])
-@pytest.mark.parametrize("seq_q,length", [(3, 37), (70, 150)])
+@pytest.mark.parametrize("seq_q,length", [(3, 37), (70, 150), (130, 150)])  # (12 and 280 rows of 4 heads; 520 are many)
 def test_gqa_attention_every_number_of_lanes_a_key(ctx, orc, hd, seq_q, length):
     """1 to 64 lanes sum a key's score: few rows (the short kernel) and, where no matrix-core kernel has the head size, many."""
     from peregrine_amd import llama
     say(f"attention hd={hd} seq_q={seq_q} len={length}")
     _attention_case(ctx, orc, 4, 2, hd, seq_q, length, llama.AttentionMask.causal(length - seq_q), None, 300 + hd)
+
+
+def _tree_sum(p, steps):
+    """f32 sum over the last axis: at every step what position ^ step holds is added."""
+    p = p.astype(np.float32)
+    for m in steps:
+        p = p + p[..., np.arange(p.shape[-1]) ^ m]
+    return p[..., 0]
+
+
+@pytest.mark.parametrize("hd,seq_q,length,kernel", [
+    (16, 3, 40, "gqa_attention_short"), (32, 3, 40, "gqa_attention_short"), (64, 3, 40, "gqa_attention_short"), (100, 3, 40, "gqa_attention_short"),
+    (128, 3, 40, "gqa_attention_short"), (256, 3, 40, "gqa_attention_short"),
+    (16, 70, 200, "gqa_attention"), (32, 70, 200, "gqa_attention"), (48, 70, 200, "gqa_attention"), (96, 70, 200, "gqa_attention"), (192, 70, 200, "gqa_attention"),
+])
+def test_gqa_attention_sums_a_keys_score_in_one_order(ctx, hd, seq_q, length, kernel):
+    """A key's lanes add what the lane ^ 1, ^ 2, ^ 4 .. beside them holds, in f32 and in this order.  Parts of 2^24 that cancel and whole numbers of a few
+    units: in this order a score loses other units than in the opposite one or one after the other, which the outputs show."""
+    from peregrine_amd import llama
+    rng = np.random.default_rng(hd)
+    lanes = 1 << max(0, (-(-hd // 4) - 1).bit_length())
+    say(f"attention order hd={hd} seq_q={seq_q} len={length} lanes={lanes}")
+    used = -(-hd // 4)
+    p = np.zeros((length, lanes), np.float64)
+    p[:, :used] = rng.integers(-3, 4, (length, used))
+    for t in range(length):
+        at = rng.permutation(used)[: used // 2 * 2].reshape(2, -1)
+        p[t, at[0]] += 2.0 ** 24
+        p[t, at[1]] -= 2.0 ** 24
+    k = rng.standard_normal((1, length, hd)).astype(np.float32)
+    k[0, :, ::4] = p[:, :used]
+    heads = 8                                                          # (560 rows of 70 tokens: past the short kernel's)
+    q = np.zeros((heads, seq_q, hd), np.float32)
+    q[:, :, ::4] = 1.0
+    v = rng.standard_normal((1, length, hd)).astype(np.float32)
+    cache = llama.StandardKVCache(1, hd, ctx)
+    cache.append(k, v, length)
+    got = np.zeros(seq_q * heads * hd, np.float32)
+    ctx.profile_begin()
+    llama.gqa_attention(q, cache, cache, heads, 1, seq_q, hd, 0.125, llama.AttentionMask.none(), None, got, ctx)
+    prof = ctx.profile_end()
+    assert kernel in prof, prof
+
+    def output(score):
+        e = np.exp(score * 0.125 - (score * 0.125).max())
+        return (e / e.sum()) @ v[0].astype(np.float64)
+
+    steps = [1 << i for i in range(lanes.bit_length() - 1)]
+    want = output(_tree_sum(p, steps).astype(np.float64))
+    for other in (_tree_sum(p, steps[::-1]).astype(np.float64), np.cumsum(p.astype(np.float32), 1, dtype=np.float32)[:, -1].astype(np.float64)):
+        assert np.abs(output(other) - want).max() > 1e-3               # (the test would see another order)
+    for row in got.reshape(-1, hd):
+        H.assert_close_rel(row, want, RTOL_F32 * 4, "gqa_attention")
 
 
 def test_gqa_attention_masks_and_logit_cap(ctx, orc):
