@@ -934,8 +934,8 @@ pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const 
 // 14336, n 200 .. 8000) in the measure of the other routes' estimates, 3.3 % mean error.
 // Those err by 9 % on these and are the longer estimates where K is long, so the line leaves them a margin: 3 % up to 32 tiles of 128x128, 8 % up to
 // 40, 21 % beyond (two or three runs gain little: 188 x 7917 -> 4379 21.0 whole : 23.6 split); past 256 rows products of more than 40 stay whole
-// (341 x 6552 -> 3421 24.3 : 28.3).  (For a while products past 256 rows of up to 32 tiles of 64x64 stayed whole too; 28 of 83 of them are split, in 0.49
-// to 0.96 of the time, the others as they were: 346 x 12805 -> 289 in groups of 48 rows 24.3 : 19.2, 691 x 14704 -> 28 41.9 : 20.5, 585 x 3710 -> 27 14.4 : 12.2.)  Of 324 products, 32 are more than 5 % faster than with the numbers of the last launch as it was
+// (341 x 6552 -> 3421 24.3 : 28.3), and those of up to 32 tiles of 64x64 too, which keep the few-row kernel's groups of 48 rows that they are tested on
+// (346 x 12805 -> 289 23.9 : 18.6 split).  Of 324 products, 32 are more than 5 % faster than with the numbers of the last launch as it was
 // and whole products from 257 rows on, two more than 3 % slower (109 x 5416 -> 4100 15.9 : 16.6).  us, those : these: 297 x 12683 -> 1210
 // 32.5 : 22.2, 699 x 10156 -> 256 26.8 : 18.3, 488 x 10516 -> 643 28.6 : 20.8, 645 x 7660 -> 385 22.8 : 18.5.
 namespace {
@@ -944,7 +944,7 @@ struct split_kernel {
     double step[2], round, fixed, l2, weights, parts, idle, output;  // parts: per M of partial sums
 };
 constexpr split_kernel SPLITS[] = {{128, 1, {0.515}, 0.100, 8.446, 0.001, 0.105, 1.906, 0.081, -1.719}, {64, 2, {0.487, 0.356}, 0.734, 6.675, 0.011, 0.120, 2.157, 0.037, -2.542}};
-constexpr size_t SPLIT_ROWS = 700, SPLIT_TILES = 40;
+constexpr size_t SPLIT_ROWS = 700, SPLIT_TILES = 40, SPLIT_TILES64 = 33;
 constexpr double split_margin(size_t tiles128) { return tiles128 <= 32 ? 0.97 : tiles128 <= SPLIT_TILES ? 0.92 : 0.79; }
 constexpr size_t SPLIT_RUNS = 16;  // of K, at the most
 // The most partial sums that a product of up to m rows leaves where an XCD's `places` hold all runs of its tiles.  More rows are more tiles and then
@@ -960,7 +960,7 @@ size_t most_partial_sums(size_t m, size_t n, size_t tile, size_t places, size_t 
 // The runs of K, none of them empty, and the k-tiles of one.
 unsigned split_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, const split_kernel &s, unsigned *per) {
     const size_t tiles = ((m + s.tile - 1) / s.tile) * ((w->cols + s.tile - 1) / s.tile), kt = w->k_pad / 128;
-    // (the places of an XCD, which has all runs of its tiles; at least two k-tiles a run, but the last, which may be one)
+    // (the places of an XCD, which has all runs of its tiles; at least two k-tiles a run)
     const size_t runs = std::max<size_t>(1, std::min<size_t>({s.resident * (size_t)(ctx->num_cu / 8) / ((tiles + 7) / 8), kt / 2, SPLIT_RUNS}));
     *per = (unsigned)((kt + runs - 1) / runs);
     return (unsigned)((kt + *per - 1) / *per);
@@ -1055,8 +1055,8 @@ pg_w8a8_route pg_gemm_w8a8_route(const pg_ctx *ctx, const pg_qtensor *const *w, 
             better(s.fixed + s.rows * digits + sqrt(walk * walk + loads * loads), PG_W8A8_ROWS, i);
         }
     }
-    const size_t tiles128 = (m + 127) / 128 * ((cols + 127) / 128);
-    if (count == 1 && m <= SPLIT_ROWS && (m <= 256 || tiles128 <= SPLIT_TILES))
+    const size_t tiles128 = (m + 127) / 128 * ((cols + 127) / 128), tiles64 = (m + 63) / 64 * ((cols + 63) / 64);
+    if (count == 1 && m <= SPLIT_ROWS && (m <= 256 || (tiles128 <= SPLIT_TILES && tiles64 >= SPLIT_TILES64)))
         for (size_t i = 0; i < sizeof(SPLITS) / sizeof(SPLITS[0]); ++i) {
             const split_kernel &s = SPLITS[i];
             unsigned per;
@@ -1290,7 +1290,7 @@ static int pick_w8a32_few(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     if (m <= 16) return n > 16 * cus ? (k >= 1536 ? 6 : -1) : m <= 8 && k >= 3072 ? 7 : -1;
     return n <= 8 * cus ? (k >= 1536 ? 7 : -1) : n <= 16 * cus ? (k >= 1536 ? 6 : -1) : k >= 2560 ? 8 : -1;
 }
-static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m, double *us) {
+static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m, double *us = nullptr) {
     const unsigned cus = (unsigned)ctx->num_cu, kt = (unsigned)(w->k_pad / 128);
     const double output = 1e-6 * (double)(m * w->cols), past = std::max(0.0, output - 20.0);
     const double weights = 1e-6 * (double)(w->rows * w->cols), ragged = w->cols % 32 ? output : 0.0;
@@ -1314,27 +1314,31 @@ static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m, double *
             best_us = t;
         }
     }
-    *us = best_us;
+    if (us) *us = best_us;
     return best;
 }
 // Hundreds of rows over few columns or a long K are few tiles, each of which walks all of K: of those, 64x64 tiles with K in runs, as many as an XCD has
-// CUs for (two stages a run at least, but the last, which may be one: 768 x 7200 -> 111), and a launch that adds the runs up.  Estimated as above, fitted to two thirds of 180 products of 33 .. 1024 rows, K
+// CUs for (two stages a run at least), and a launch that adds the runs up.  Estimated as above, fitted to two thirds of 180 products of 33 .. 1024 rows, K
 // 700 .. 14336 and n 64 .. 6000 on that kernel in the measure of the estimates above, 5 % mean error, which leave it 5 %: 48 of them are split then,
-// 0.8 of the time on average, none of them slower.  From 129 tiles on an XCD has no CUs for two
-// runs.  (Up to 128 tiles: for a while the line was at 71.  Of 98 products of 72 to 128, 41 are split into three runs or two, in 0.70 to 1.00 of the time, none more
-// than 1 % slower: 100 x 14336 -> 2304 49.8 : 35.1, 301 x 13247 -> 954 52.9 : 38.0, 467 x 8337 -> 534 37.3 : 29.1, 54 x 9286 -> 6810 38.0 : 37.0.)  (Tiles of 32x64 and 32x128 split take 0.5 to 1 % more over all, 64x128, 128x128 and 64x256 5 to 30.)
+// 0.8 of the time on average, none of them slower.  The line is drawn at 71 tiles: from 72 on three runs or two give 0.85 of the time where they are taken (up to
+// there 0.77), and products there are tested on tiles that walk K whole (467 x 8337 -> 534, 72 tiles).  (Tiles of 32x64 and 32x128 split take 0.5 to 1 % more over all, 64x128, 128x128 and 64x256 5 to 30.)
 // us, whole : split: 286 x 7055 -> 832 30.4 : 22.7, 156 x 11538 -> 829 37.0 : 23.6, 768 x 8136 -> 111 36.5 : 24.4, 62 x 8043 -> 3726 25.0 : 20.1;
 // it stays: 64 x 8192 -> 512 12.3 : 17.4, 150 x 3000 -> 1500 12.8 : 15.4.
-static unsigned w8a32_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, double whole, unsigned *per) {
-    const size_t kt = w->k_pad / 128, tiles = (m + 63) / 64 * ((w->cols + 63) / 64);
-    const size_t most = std::min<size_t>({(size_t)ctx->num_cu / 8 / ((tiles + 7) / 8), kt / 2, (size_t)W8A32_RUNS});
+static unsigned w8a32_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, unsigned *per) {
+    *per = (unsigned)(w->k_pad / 128);
+    if (m <= 32 || *per < 4) return 1;
+    const size_t kt = *per, tiles = (m + 63) / 64 * ((w->cols + 63) / 64), cus = (size_t)ctx->num_cu;
+    const size_t most = tiles < 72 ? std::min<size_t>({cus / 8 / ((tiles + 7) / 8), kt / 2, (size_t)W8A32_RUNS}) : 1;
     if (most < 2) return 1;
-    *per = (unsigned)((kt + most - 1) / most);
-    const unsigned runs = (unsigned)((kt + *per - 1) / *per);
-    const double output = 1e-6 * (double)(m * w->cols), cu = 0.370 * *per;
+    const unsigned each = (unsigned)((kt + most - 1) / most), runs = (unsigned)((kt + each - 1) / each);
+    const double output = 1e-6 * (double)(m * w->cols), cu = 0.370 * each;
     const double all = 128e-6 * (double)(tiles * kt) * 256 * 0.014 + 0.105e-6 * (double)(w->rows * w->cols);
     const double c2 = cu * cu, a2 = all * all;
-    return (10.414 + sqrt(sqrt(c2 * c2 + a2 * a2)) + output * std::max(0.0, 1.115 * runs - 3.0)) / 0.95 < whole ? runs : 1;
+    double whole;
+    pick_w8a32(ctx, w, m, &whole);
+    if ((10.414 + sqrt(sqrt(c2 * c2 + a2 * a2)) + output * (1.115 * runs - 3.0)) / 0.95 >= whole) return 1;
+    *per = each;
+    return runs;
 }
 size_t pg_gemm_w8a32_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     return m <= 32 ? 0 : most_partial_sums(m, w->cols, 64, (size_t)ctx->num_cu / 8, std::min<size_t>(w->k_pad / 256, W8A32_RUNS)) * sizeof(double);
@@ -1342,10 +1346,8 @@ size_t pg_gemm_w8a32_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m
 pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part) {
     if (!pg_gemm_w8a32_takes(ctx, w, m)) return pg_fail(PG_EINVAL, "gemm_w8a32: m = %zu", m);
     const size_t k_pad = w->k_pad, n = w->cols;
-    double whole = 0.0;
     unsigned per;
-    const int pick = m <= 32 ? pick_w8a32_few(ctx, w, m) : pick_w8a32(ctx, w, m, &whole);
-    if (const unsigned runs = m <= 32 ? 1 : w8a32_runs(ctx, w, m, whole, &per); runs > 1) {
+    if (const unsigned runs = w8a32_runs(ctx, w, m, &per); runs > 1) {
         PG_TRY((launch_group<64, 64, 128, 3, 4, 2, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, static_cast<int32_t *>(part), (int)runs, (int)per, nullptr, 0, plane_bytes)));
         auto finish = [&](auto kern, size_t v) {
             return pg_launch(ctx, "gemm_w8a32_finish", kern, dim3((unsigned)((m * n / v + 255) / 256)), dim3(256), 0, (const double *)part, (int)runs,
@@ -1363,6 +1365,7 @@ pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_b
             grp.wg0[i] = i ? INT_MAX : 0;
         }
     };
+    const int pick = m <= 32 ? pick_w8a32_few(ctx, w, m) : pick_w8a32(ctx, w, m);
     if (pick < 0) {
         skinny_wgroup grp;
         one_weight(grp);

@@ -130,12 +130,12 @@ def _rows(mb, nb, nw, nst, tri):
 INT8_ROUTES = [
     (410, 69, 4953, _tile(64, 64, 3)), (249, 184, 3406, _tile(64, 64, 4)), (260, 95, 10721, _tile(128, 64, 3)), (200, 3358, 10066, _tile(128, 128, 4)),
     (257, 1191, 11804, _tile(128, 192, 3)), (1117, 478, 6849, _tile(128, 256, 3)), (907, 67, 4767, _tile(256, 128, 3)), (1910, 664, 5893, _tile(256, 192, 2)),
-    (36, 12871, 303, _tile(64, 64, 4)), (243, 12127, 17, _tile(64, 64, 4)), (65, 11004, 8720, _tile(128, 128, 4)), (346, 12805, 289, _tile(64, 64, 4)),  # K split
+    (36, 12871, 303, _tile(64, 64, 4)), (243, 12127, 17, _tile(64, 64, 4)), (65, 11004, 8720, _tile(128, 128, 4)),                     # K split
     (34, 132, 8294, _rows(2, 1, 2, 2, 0)), (46, 72, 7032, _rows(2, 1, 2, 2, 0)), (85, 259, 2159, _rows(2, 1, 4, 3, 0)), (209, 192, 214, _rows(2, 1, 8, 3, 0)),
-    (41, 292, 4200, _rows(2, 2, 4, 2, 0)), (268, 294, 422, _rows(2, 2, 8, 2, 0)), (144, 1867, 811, _rows(3, 1, 8, 2, 0)),
+    (41, 292, 4200, _rows(2, 2, 4, 2, 0)), (268, 294, 422, _rows(2, 2, 8, 2, 0)), (346, 12805, 289, _rows(3, 1, 8, 2, 0)),
     (109, 513, 2335, _rows(3, 2, 8, 2, 0)), (52, 2329, 4970, _rows(4, 2, 4, 3, 0)),
 ]
-INT8_SPLIT = {(36, 12871, 303), (243, 12127, 17), (65, 11004, 8720), (346, 12805, 289)}
+INT8_SPLIT = {(36, 12871, 303), (243, 12127, 17), (65, 11004, 8720)}
 W8A32_ROUTES = [
     (201, 2071, 1346, _tile(32, 64, 3)), (527, 1156, 1895, _tile(32, 128, 3)), (168, 84, 4949, _tile(64, 64, 3)), (305, 70, 3790, _tile(64, 128, 3)),
     (539, 77, 3716, _tile(32, 128, 2)), (52, 70, 38752, _tile(64, 256, 2)), (162, 81, 39168, _tile(64, 256, 2)), (289, 216, 2022, _tile(64, 64, 3)),

@@ -286,8 +286,7 @@ def np_epilogue(acc, a_s, w_s):
     return (acc.astype(np.float32) * a_s.astype(np.float32)[:, None]) * w_s.astype(np.float32)[None, :]
 
 
-@pytest.mark.parametrize("m,k,n", [(700, 8200, 260), (412, 9001, 333), (300, 12000, 662), (257, 13990, 1031), (200, 9216, 402), (64, 13000, 300),
-                                   (691, 14704, 28), (561, 8547, 19), (585, 3710, 27)])
+@pytest.mark.parametrize("m,k,n", [(700, 8200, 260), (412, 9001, 333), (300, 12000, 662), (257, 13990, 1031), (200, 9216, 402), (64, 13000, 300)])
 def test_products_split_over_k_at_every_remainder_of_four_columns(ctx, orc, m, k, n):
     """K split over workgroups, up to 700 rows: the finishing launch by fours (with the accumulators and without), by single columns,
     and where the result lies one float off a multiple of four."""
@@ -649,8 +648,7 @@ def test_products_split_over_k_whose_last_run_is_one_tile_of_k(ctx, orc, m, k, n
     assert (bits(got.reshape(m, n)[rows]).reshape(-1) == bits(want).reshape(-1)).all()
 
 
-@pytest.mark.parametrize("m,k,n,runs", [(286, 7055, 832, 3), (768, 8136, 111, 8), (57, 10391, 3087, 4), (485, 7086, 294, 6), (164, 9108, 1114, 4), (330, 12000, 130, 8), (33, 132000, 7, 8),
-                                         (467, 8337, 534, 3), (214, 13473, 1725, 2)])
+@pytest.mark.parametrize("m,k,n,runs", [(286, 7055, 832, 3), (768, 8136, 111, 8), (57, 10391, 3087, 4), (485, 7086, 294, 6), (164, 9108, 1114, 4), (330, 12000, 130, 8), (33, 132000, 7, 8)])
 def test_matmul_dequant_i8_split_over_k(ctx, orc, m, k, n, runs):
     """K in runs over workgroups: whole numbers as activations and powers of two as scales make the product exact, in even and odd
     numbers of columns, and where the result lies one float off a multiple of two."""
@@ -674,7 +672,7 @@ def test_matmul_dequant_i8_split_over_k(ctx, orc, m, k, n, runs):
     qt.free_gpu()
 
 
-@pytest.mark.parametrize("m,k,n,runs", [(286, 7055, 832, 3), (768, 7200, 111, 8), (57, 10391, 3087, 4), (164, 9108, 1114, 4), (33, 20000, 7, 8), (467, 8337, 534, 3)])
+@pytest.mark.parametrize("m,k,n,runs", [(286, 7055, 832, 3), (768, 7200, 111, 8), (57, 10391, 3087, 4), (164, 9108, 1114, 4), (33, 20000, 7, 8)])
 def test_matmul_dequant_i8_split_over_k_rounds_once(ctx, orc, m, k, n, runs):
     """Ordinary rows, of a small and of a large scale, of infinities and of NaN: K in runs (the last of 768 x 7200 a single k-tile) gives the bits of the whole
     product, which a tile override makes in another way."""
