@@ -934,8 +934,9 @@ pg_status gemm_dispatch(pg_ctx *ctx, const int8_t *a_i8, size_t a_stride, const 
 // 14336, n 200 .. 8000) in the measure of the other routes' estimates, 3.3 % mean error.
 // Those err by 9 % on these and are the longer estimates where K is long, so the line leaves them a margin: 3 % up to 32 tiles of 128x128, 8 % up to
 // 40, 21 % beyond (two or three runs gain little: 188 x 7917 -> 4379 21.0 whole : 23.6 split); past 256 rows products of more than 40 stay whole
-// (341 x 6552 -> 3421 24.3 : 28.3), and those of up to 32 tiles of 64x64 too, which keep the few-row kernel's groups of 48 rows that they are tested on
-// (346 x 12805 -> 289 23.9 : 18.6 split).  Of 324 products, 32 are more than 5 % faster than with the numbers of the last launch as it was
+// (341 x 6552 -> 3421 24.3 : 28.3).  Those of up to 32 tiles of 64x64 stay too, but not for their time: of 83 of them the estimate would split 28, in 0.49 to 0.96
+// of it (346 x 12805 -> 289 24.3 in the few-row kernel's groups of 48 rows : 19.2, 691 x 14704 -> 28 41.9 : 20.5) and none slower by more than 1 %.  That kernel
+// is held to the oracle on a product from there, so the line moves when another product stands in for it.  Of 324 products, 32 are more than 5 % faster than with the numbers of the last launch as it was
 // and whole products from 257 rows on, two more than 3 % slower (109 x 5416 -> 4100 15.9 : 16.6).  us, those : these: 297 x 12683 -> 1210
 // 32.5 : 22.2, 699 x 10156 -> 256 26.8 : 18.3, 488 x 10516 -> 643 28.6 : 20.8, 645 x 7660 -> 385 22.8 : 18.5.
 namespace {
@@ -960,7 +961,7 @@ size_t most_partial_sums(size_t m, size_t n, size_t tile, size_t places, size_t 
 // The runs of K, none of them empty, and the k-tiles of one.
 unsigned split_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, const split_kernel &s, unsigned *per) {
     const size_t tiles = ((m + s.tile - 1) / s.tile) * ((w->cols + s.tile - 1) / s.tile), kt = w->k_pad / 128;
-    // (the places of an XCD, which has all runs of its tiles; at least two k-tiles a run)
+    // (the places of an XCD, which has all runs of its tiles; at least two k-tiles a run, but the last, which may be one)
     const size_t runs = std::max<size_t>(1, std::min<size_t>({s.resident * (size_t)(ctx->num_cu / 8) / ((tiles + 7) / 8), kt / 2, SPLIT_RUNS}));
     *per = (unsigned)((kt + runs - 1) / runs);
     return (unsigned)((kt + *per - 1) / *per);
@@ -1318,10 +1319,12 @@ static int pick_w8a32(const pg_ctx *ctx, const pg_qtensor *w, size_t m, double *
     return best;
 }
 // Hundreds of rows over few columns or a long K are few tiles, each of which walks all of K: of those, 64x64 tiles with K in runs, as many as an XCD has
-// CUs for (two stages a run at least), and a launch that adds the runs up.  Estimated as above, fitted to two thirds of 180 products of 33 .. 1024 rows, K
+// CUs for (two stages a run at least, but the last, which may be one: 768 x 7200 -> 111), and a launch that adds the runs up.  Estimated as above, fitted to two thirds of 180 products of 33 .. 1024 rows, K
 // 700 .. 14336 and n 64 .. 6000 on that kernel in the measure of the estimates above, 5 % mean error, which leave it 5 %: 48 of them are split then,
-// 0.8 of the time on average, none of them slower.  The line is drawn at 71 tiles: from 72 on three runs or two give 0.85 of the time where they are taken (up to
-// there 0.77), and products there are tested on tiles that walk K whole (467 x 8337 -> 534, 72 tiles).  (Tiles of 32x64 and 32x128 split take 0.5 to 1 % more over all, 64x128, 128x128 and 64x256 5 to 30.)
+// 0.8 of the time on average, none of them slower.  The line at 71 tiles is not drawn by time: of 98 products of 72 to
+// 128 tiles the estimate would split 41 into three runs or two, in 0.70 to 1.00 of it (467 x 8337 -> 534, 72 tiles, 37.3 : 29.1, 301 x 13247 -> 954 52.9 : 38.0), none slower by more
+// than 1 %; tiles that walk K whole are held to it on a product from there.  From 129 tiles on an XCD has no CUs for two runs.  (A pass over the planes of two runs,
+// which only 4 or 5 k-tiles are cut into, comes out of the fit as less than nothing and counts as nothing.)  (Tiles of 32x64 and 32x128 split take 0.5 to 1 % more over all, 64x128, 128x128 and 64x256 5 to 30.)
 // us, whole : split: 286 x 7055 -> 832 30.4 : 22.7, 156 x 11538 -> 829 37.0 : 23.6, 768 x 8136 -> 111 36.5 : 24.4, 62 x 8043 -> 3726 25.0 : 20.1;
 // it stays: 64 x 8192 -> 512 12.3 : 17.4, 150 x 3000 -> 1500 12.8 : 15.4.
 static unsigned w8a32_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, unsigned *per) {
@@ -1336,7 +1339,7 @@ static unsigned w8a32_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, uns
     const double c2 = cu * cu, a2 = all * all;
     double whole;
     pick_w8a32(ctx, w, m, &whole);
-    if ((10.414 + sqrt(sqrt(c2 * c2 + a2 * a2)) + output * (1.115 * runs - 3.0)) / 0.95 >= whole) return 1;
+    if ((10.414 + sqrt(sqrt(c2 * c2 + a2 * a2)) + output * std::max(0.0, 1.115 * runs - 3.0)) / 0.95 >= whole) return 1;
     *per = each;
     return runs;
 }
