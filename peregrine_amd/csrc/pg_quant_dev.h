@@ -6,10 +6,12 @@
 
 // round -> clamp(-127,127) -> `as i8` (NaN -> 0), returned as int.   src/quant.rs:101-106
 // Half away from zero is truncation after adding the float just under a half with the value's sign: with a half itself 0.49999997 would
-// reach 1, and every k + 0.5 still does (the sum lies a quarter of an ulp or less below it and rounds up).  Checked against roundf for every
+// reach 1, and every k + 0.5 still does (the exact sum lies a quarter of an ulp or less below k + 1 and rounds up to it; from 0.5 it lies half an ulp below 1, a
+// tie, which goes to the even 1).  Checked against roundf for every
 // float to 144.  The conversion truncates, takes NaN to 0 and saturates (asm: in C++ that would be undefined).  Five vector instructions with
 // the caller's product, where roundf, two clamps and two tests for NaN were fourteen.  With the maximum below, us, before : now: the
-// products of a layer for one row 42.7 : 41.4, 27 rows of a smaller one 34.4 : 33.5, 2048 rows 469 : 466.
+// products of a layer for one row 42.7 : 41.4, 27 rows of a smaller one 34.4 : 33.5; a single small product and layers of
+// 2048 rows (468 : 464) within what runs differ.
 __device__ __forceinline__ int pg_quant_to_i8(float v) {
     int i;
     asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(v + copysignf(0x1.fffffep-2f, v)));
@@ -23,7 +25,7 @@ __device__ __forceinline__ int pg_quant4_to_i8(float x, float y, float z, float 
     return (int)(lo | hi);
 }
 
-// Maximum over the 64 lanes of a wavefront, all of them active and none negative, in every lane: DPP moves within rows of 16 lanes, then the four rows' through scalar
+// Maximum over the 64 lanes of a wavefront, all of them active, in every lane; values of either sign and -inf (scores, logits), NaN passed over as by fmaxf: DPP moves within rows of 16 lanes, then the four rows' through scalar
 // registers (six exchanges through LDS were a chain of 0.2 us).
 __device__ __forceinline__ float pg_wave_max_f32(float v) {
     auto step = [](float x, auto ctrl) {

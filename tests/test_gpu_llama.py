@@ -203,6 +203,35 @@ def test_gqa_attention_sums_a_keys_score_in_one_order(ctx, hd, seq_q, length, ke
         H.assert_close_rel(row, want, RTOL_F32 * 4, "gqa_attention")
 
 
+@pytest.mark.parametrize("hd,seq_q,length,kernel", [
+    (64, 3, 40, "gqa_attention_short"), (64, 3, 900, "gqa_combine"), (48, 70, 200, "gqa_attention"), (128, 1, 3000, "gqa_combine"), (128, 130, 200, None),
+])
+def test_gqa_attention_of_scores_that_are_all_far_below_zero(ctx, hd, seq_q, length, kernel):
+    """The largest score is -600 and a row has no weight above zero for a maximum that is taken as zero (exp(-600) is none in f32).  The scores
+    are whole numbers, exact in f32."""
+    from peregrine_amd import llama
+    say(f"attention scores below zero hd={hd} seq_q={seq_q} len={length}")
+    rng = np.random.default_rng(hd + length)
+    heads = 8
+    k = rng.standard_normal((1, length, hd)).astype(np.float32)
+    k[0, :, 0] = 600 + rng.integers(0, 5, length)
+    k[0, rng.integers(length), 0] = 600
+    q = np.zeros((heads, seq_q, hd), np.float32)
+    q[:, :, 0] = -1.0
+    v = rng.standard_normal((1, length, hd)).astype(np.float32)
+    cache = llama.StandardKVCache(1, hd, ctx)
+    cache.append(k, v, length)
+    got = np.zeros(seq_q * heads * hd, np.float32)
+    ctx.profile_begin()
+    llama.gqa_attention(q, cache, cache, heads, 1, seq_q, hd, 1.0, llama.AttentionMask.none(), None, got, ctx)
+    prof = ctx.profile_end()
+    assert kernel is None or kernel in prof, prof
+    e = np.exp(600.0 - k[0, :, 0].astype(np.float64))
+    want = (e / e.sum()) @ v[0].astype(np.float64)
+    for row in got.reshape(-1, hd):
+        H.assert_close_rel(row, want, RTOL_F32 * 4, "gqa_attention")
+
+
 def test_gqa_attention_masks_and_logit_cap(ctx, orc):
     from peregrine_amd import llama
     M = llama.AttentionMask

@@ -410,6 +410,25 @@ def test_moe_routing_of_a_token_on_a_wavefront(ctx, orc, T, E, top_k, d, ffn, ty
     test_moe_routing_in_one_launch_and_split_products(ctx, orc, T, E, top_k, d, ffn, typ)
 
 
+@pytest.mark.parametrize("T,E,top_k", [(1, 2, 1), (3, 16, 4), (16, 64, 8), (17, 16, 4)])
+def test_moe_routing_of_logits_that_are_all_far_below_zero(ctx, orc, T, E, top_k):
+    """The largest logit of a token is -600: with a maximum taken as zero every probability would be 0 / 0.  A wavefront's lanes beyond the experts
+    and the experts chosen before take no part."""
+    from peregrine_amd import gguf, moe
+    say(f"moe logits below zero T={T} E={E} top_k={top_k}")
+    d, ffn, distinct = 160, 512, min(E, 3)
+    raws = build(orc, 60 + E, d, ffn, distinct, 8)
+    x = orc.rng_normal(T + 70, T * d).reshape(T, d)
+    logits = (-600.0 - np.abs(orc.rng_normal(T + 71, T * E)).reshape(T, E)).astype(np.float32)
+    logits[0, 0] = -600.0
+    mk = lambda rs, n_out, k_in: (lambda ws: [ws[e % distinct] for e in range(E)])([gguf.GgufWeight(r, 8, n_out, k_in, ctx) for r in rs])
+    ex = moe.MoEExperts(mk(raws[0], ffn, d), mk(raws[1], ffn, d), mk(raws[2], d, ffn), top_k, moe.SILU, ctx)
+    got = ex.forward(x, logits).reshape(T, d)
+    want, _, _ = orc.moe_ffn(x.reshape(-1), T, d, ffn, E, top_k, logits, *[[r[e % distinct] for e in range(E)] for r in raws], 8, moe.SILU)
+    for t in range(T):
+        H.assert_close_rel(got[t], want[t], MOE_RTOL, f"token {t}")
+
+
 @pytest.mark.parametrize("T,E,top_k,d,ffn,typ", [
     (2, 4, 1, 512, 512, 8), (8, 2, 2, 544, 1056, 2), (9, 2, 2, 544, 1056, 8), (17, 3, 2, 608, 992, 2),   # tiles of 8 and 16 pairs and past them
     (33, 5, 2, 1024, 544, 8), (64, 1, 1, 512, 1024, 8), (65, 70, 2, 512, 544, 2), (130, 130, 1, 512, 512, 8),  # past 64 and 128 experts
