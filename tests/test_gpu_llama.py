@@ -142,12 +142,18 @@ def test_gqa_attention_unmasked(ctx, orc, nqh, nkvh, hd, seq_q, length):
 
 
 @pytest.mark.parametrize("hd", [2, 4, 8, 16, 32, 64, 96, 128, 192, 256])
-@pytest.mark.parametrize("seq_q,length", [(3, 37), (70, 150), (130, 150)])  # (12 and 280 rows of 4 heads; 520 are many)
+@pytest.mark.parametrize("seq_q,length", [(3, 37), (70, 150)])
 def test_gqa_attention_every_number_of_lanes_a_key(ctx, orc, hd, seq_q, length):
     """1 to 64 lanes sum a key's score: few rows (the short kernel) and, where no matrix-core kernel has the head size, many."""
     from peregrine_amd import llama
     say(f"attention hd={hd} seq_q={seq_q} len={length}")
     _attention_case(ctx, orc, 4, 2, hd, seq_q, length, llama.AttentionMask.causal(length - seq_q), None, 300 + hd)
+
+
+@pytest.mark.parametrize("hd", [2, 4, 8, 16, 32, 64, 96, 128, 192, 256])
+def test_gqa_attention_every_number_of_lanes_a_key_of_many_rows(ctx, orc, hd):
+    """The same where the rows are many (130 tokens of 4 heads; the 280 rows above are still few)."""
+    test_gqa_attention_every_number_of_lanes_a_key(ctx, orc, hd, 130, 150)
 
 
 def _tree_sum(p, steps):
