@@ -27,11 +27,12 @@
 // tiles are few K is cut into half as many chunks between workgroups, or none, and that many planes fewer go through
 // memory; it brings the activations to LDS twice as often, which is why some wide launches keep S = 1.  us, S = 1 : S = 2,
 // the kernel + the sum of its chunks: 100 x 4096 -> 28672 (Q4_0) 61.3 + 13.7 : 58.5 + 7.9, 250 x 2048 -> 16384 (Q8_0)
-// 48.6 + 11.3 : 44.5, 500 x 2048 -> 11264 59.3 + 14.3 : 57.7, 777 x 14336 -> 4096 178 : 189.
+// 48.6 + 11.3 : 44.5, 500 x 2048 -> 11264 59.3 + 14.3 : 57.7, as long either way 777 x 14336 -> 4096 (Q8_0) 176 + 15.9 : 184 + 8.7 (S = 2 is
+// taken); S = 1 is kept by 777 x 4096 -> 28672 (Q8_0) 367 : 401, 1024 x 4096 -> 28672 (Q4_0) 418 : 458, 300 x 4096 -> 28672 (Q4_0) 143 : 165.
 //
 // What bounds it: 1024 rows of 4096 -> 28672 (Q8_0) are 481 G f16 operations over the two planes and take 425 to 495 us
 // (short and sustained runs), 0.97 to 1.13 PFLOP/s where a library's dense bf16 product holds 1.34: the chip's power limit
-// first, the instruction mix of the step after it.  The tile's rows follow the launch (hmm_plan_for): 777 rows are 9 tiles
+// first (1.85 to 2.1 of 2.4 GHz, either form, the matrix pipe busy 51 to 59 % of those cycles, 43 to 48 over short walks), the instruction mix of the step after it.  The tile's rows follow the launch (hmm_plan_for): 777 rows are 9 tiles
 // of 96 (504 workgroups, two full rounds of the CUs: 366 us) and not 7 of 128 (392: 15 % of the rows padding, the second
 // round half empty: 478 us).  Spreading the loads over the steps instead of issuing them together took 9 % (MT = 8) to
 // 20 % (MT = 4) off a stage, asking for all rows' scales before the first store 8 to 25 us off every launch.
