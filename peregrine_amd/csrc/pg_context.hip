@@ -33,10 +33,14 @@ pg_status pg_use(pg_ctx *ctx) {
     return PG_OK;
 }
 
-pg_status pg_refuse_capture(pg_ctx *ctx, const char *what) {
+static bool capturing(pg_ctx *ctx) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) (void)hipGetLastError();
-    if (st != hipStreamCaptureStatusNone) return pg_fail(PG_EDEVICE, "%s: not permitted while the stream is capturing", what);
+    return st != hipStreamCaptureStatusNone;
+}
+
+pg_status pg_refuse_capture(pg_ctx *ctx, const char *what) {
+    if (capturing(ctx)) return pg_fail(PG_EDEVICE, "%s: not permitted while the stream is capturing", what);
     return PG_OK;
 }
 
@@ -73,6 +77,20 @@ pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out) {
         ctx->ws_bytes = want;
     }
     *out = ctx->ws;
+    return PG_OK;
+}
+
+pg_status pg_workspace_with_room(pg_ctx *ctx, size_t bytes, size_t room, void **out, size_t *got) {
+    if (bytes + room > ctx->ws_bytes) {
+        if (capturing(ctx)) {
+            if (bytes <= ctx->ws_bytes) room = ctx->ws_bytes - bytes;
+        } else if (room && pg_workspace(ctx, bytes + room, out) != PG_OK) {
+            (void)hipGetLastError();
+            room = 0;
+        }
+    }
+    PG_TRY(pg_workspace(ctx, bytes + room, out));
+    *got = ctx->ws_bytes - bytes;
     return PG_OK;
 }
 

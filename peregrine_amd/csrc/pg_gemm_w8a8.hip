@@ -1346,11 +1346,11 @@ static unsigned w8a32_runs(const pg_ctx *ctx, const pg_qtensor *w, size_t m, uns
 size_t pg_gemm_w8a32_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m) {
     return m <= 32 ? 0 : most_partial_sums(m, w->cols, 64, (size_t)ctx->num_cu / 8, std::min<size_t>(w->k_pad / 256, W8A32_RUNS)) * sizeof(double);
 }
-pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part) {
+pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part, size_t part_bytes) {
     if (!pg_gemm_w8a32_takes(ctx, w, m)) return pg_fail(PG_EINVAL, "gemm_w8a32: m = %zu", m);
     const size_t k_pad = w->k_pad, n = w->cols;
     unsigned per;
-    if (const unsigned runs = w8a32_runs(ctx, w, m, &per); runs > 1) {
+    if (const unsigned runs = w8a32_runs(ctx, w, m, &per); runs > 1 && runs * m * n * sizeof(double) <= part_bytes) {
         PG_TRY((launch_group<64, 64, 128, 3, 4, 2, 2, false, 3>(ctx, planes, k_pad, a_scales, &w, &out, 1, m, static_cast<int32_t *>(part), (int)runs, (int)per, nullptr, 0, plane_bytes)));
         auto finish = [&](auto kern, size_t v) {
             return pg_launch(ctx, "gemm_w8a32_finish", kern, dim3((unsigned)((m * n / v + 255) / 256)), dim3(256), 0, (const double *)part, (int)runs,

@@ -186,6 +186,9 @@ pg_status pg_refuse_capture(pg_ctx *ctx, const char *what);
 hipError_t pg_dev_malloc(pg_ctx *ctx, void **p, size_t bytes);
 // Scratch arena of at least `bytes` (256-byte aligned); contents undefined.
 pg_status pg_workspace(pg_ctx *ctx, size_t bytes, void **out);
+// The same with `room` bytes behind them that the caller can do without: a capture takes the arena as it is, and where memory has run out
+// there are the bytes alone.  *got: what lies behind them.
+pg_status pg_workspace_with_room(pg_ctx *ctx, size_t bytes, size_t room, void **out, size_t *got);
 // Pinned host memory of at least `bytes` (the context's one block; contents undefined).  The caller has waited for
 // every launch or copy that used it before.
 pg_status pg_pinned(pg_ctx *ctx, size_t bytes, void **out);
@@ -260,9 +263,9 @@ pg_status pg_launch_gemm_w8a8_combine(pg_ctx *ctx, const int8_t *a_i8, size_t a_
                                       const pg_qtensor *w, size_t m, float *out, const int32_t *comb, size_t comb_plane);
 // The W8A32 product over three digit planes (plane_bytes apart) in one launch, where it takes it.
 bool pg_gemm_w8a32_takes(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
-// `part`: pg_gemm_w8a32_split_room of scratch, for the partial sums where K is split over workgroups.
+// `part`, part_bytes: scratch for the partial sums where K is split over workgroups, as it is where they find room (pg_gemm_w8a32_split_room always does).
 size_t pg_gemm_w8a32_split_room(const pg_ctx *ctx, const pg_qtensor *w, size_t m);
-pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part);
+pg_status pg_launch_gemm_w8a32(pg_ctx *ctx, const int8_t *planes, size_t plane_bytes, const float *a_scales, const pg_qtensor *w, size_t m, float *out, void *part, size_t part_bytes);
 // How W8A8 products of two rows and more run: tiles, the few-row kernel (2 .. 512 rows), or tiles with K split over workgroups (33 .. 700 rows
 // over one weight: i32 partial sums in `part`, pg_gemm_w8a8_split_bytes of them, and a finishing launch); `index` names the kernel.
 enum pg_w8a8_kind { PG_W8A8_TILES, PG_W8A8_ROWS, PG_W8A8_SPLIT };

@@ -563,20 +563,19 @@ static pg_status matmul_quantized_on(pg_ctx *ctx, const float *a_dev, size_t m, 
     const size_t a_bytes = m_pad * w->k_pad;
     const size_t sz_scales = pg_round_up(m_pad * sizeof(float), 256);
     pg_w8a8_route route = pg_gemm_w8a8_route(ctx, &w, 1, m);
-    size_t part_bytes = route.kind == PG_W8A8_SPLIT ? pg_gemm_w8a8_split_bytes(ctx, w, m, route.index) : 0;
-    if (part_bytes && fixed && a_bytes + sz_scales + part_bytes > fixed_cap) {  // (the partial planes are no reason to refuse)
-        route = {PG_W8A8_TILES, -1};
-        part_bytes = 0;
-    }
-    const size_t need = a_bytes + sz_scales + part_bytes;
+    const size_t part_bytes = route.kind == PG_W8A8_SPLIT ? pg_gemm_w8a8_split_bytes(ctx, w, m, route.index) : 0;
+    const size_t need = a_bytes + sz_scales;
     void *ws = fixed;
+    size_t room = 0;
     if (fixed) {
         if (need > fixed_cap)
             return pg_fail(PG_EINVAL, "this product needs %zu bytes of scratch (m = %zu, k = %zu, n = %zu); the fixed scratch holds %zu",
                            need, m, k, w->cols, fixed_cap);
+        room = fixed_cap - need;
     } else {
-        PG_TRY(pg_workspace(ctx, a_bytes + sz_scales + pg_gemm_w8a8_split_room(ctx, w, m), &ws));
+        PG_TRY(pg_workspace_with_room(ctx, need, pg_gemm_w8a8_split_room(ctx, w, m), &ws, &room));
     }
+    if (part_bytes > room) route = {PG_W8A8_TILES, -1};  // (the partial planes are no reason to refuse; the sums are whole numbers either way)
     int8_t *a_i8 = static_cast<int8_t *>(ws);
     float *a_scales = reinterpret_cast<float *>(a_i8 + a_bytes);
     PG_TRY(pg_launch_quantize_activations(ctx, a_dev, m, k, a_i8, w->k_pad, a_scales));
@@ -772,14 +771,15 @@ PG_API pg_status pg_matmul_dequant_i8_dev(pg_ctx *ctx, const float *a_dev, size_
     const size_t plane_bytes = m_pad * w->k_pad, plane_elems = m_pad * n;
     // (the product's prologue reads a scale per stacked row, whether or not it writes f32: three planes' worth)
     const size_t sz_planes = pg_round_up(3 * plane_bytes, 256), sz_scales = pg_round_up(3 * m_pad * sizeof(float), 256);
-    const size_t sz_part = std::max(pg_gemm_w8a32_split_room(ctx, w, m), one ? 0 : 2 * plane_elems * sizeof(int32_t));
+    const size_t sz_acc = one ? 0 : 2 * plane_elems * sizeof(int32_t), split_room = pg_gemm_w8a32_split_room(ctx, w, m);
     void *ws = nullptr;
-    PG_TRY(pg_workspace(ctx, sz_planes + sz_scales + sz_part, &ws));
+    size_t room = 0;
+    PG_TRY(pg_workspace_with_room(ctx, sz_planes + sz_scales + sz_acc, split_room > sz_acc ? split_room - sz_acc : 0, &ws, &room));
     int8_t *planes = static_cast<int8_t *>(ws);
     float *row_scales = reinterpret_cast<float *>(planes + sz_planes);
     int32_t *acc = reinterpret_cast<int32_t *>(planes + sz_planes + sz_scales);
     PG_TRY(launch_quantize_rows<true>(ctx, "rows_to_digits3", a_dev, m, k, planes, w->k_pad, row_scales, plane_bytes));
-    if (one) return pg_launch_gemm_w8a32(ctx, planes, plane_bytes, row_scales, w, m, out_dev, acc);
+    if (one) return pg_launch_gemm_w8a32(ctx, planes, plane_bytes, row_scales, w, m, out_dev, acc, room);
     PG_TRY(pg_launch_gemm_w8a8(ctx, planes, w->k_pad, row_scales, w, m_pad + m, nullptr, acc));
     return pg_launch_gemm_w8a8_combine(ctx, planes + 2 * plane_bytes, w->k_pad, row_scales, w, m, out_dev, acc, plane_elems);
 }

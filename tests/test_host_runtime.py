@@ -571,6 +571,61 @@ def test_int8_products_of_fewer_rows_need_no_more_scratch(host, call, n, k):
     host.lib.pg_qtensor_free(host.ctx, q)
 
 
+SPLIT_CALLS = [("pg_matmul_quantized_dev", 488, 643, 8192, "splitk_finish_kernel"), ("pg_matmul_dequant_i8_dev", 286, 832, 7055, "splitk_finish_w8a32")]
+
+
+@pytest.mark.parametrize("call,m,n,k,finish", SPLIT_CALLS)
+def test_int8_products_are_captured_whole_where_the_scratch_has_no_room_to_split_k(host, call, m, n, k, finish):
+    """The partial sums are no reason to refuse a capture: whatever eager call has left room for the rows, K is split where its planes find
+    room behind them and walked whole where they do not (integer sums: the same bits).  Only rows without room are refused."""
+    w = host.alloc(n * k)
+    q = host.new("pg_qtensor_from_f32_dev", host.ctx, w, k, n)
+    few = host.new("pg_qtensor_from_f32_dev", host.ctx, host.alloc(8 * 4096), 4096, 8)
+    x, y = host.alloc(2048 * 4096), host.alloc(2048 * n)
+    tail = (None,) if call == "pg_matmul_quantized_dev" else ()
+    seen = []
+    for rows in range(0, 2049, 256):     # of another weight, whose rows alone size the scratch
+        ctx = host.new("pg_ctx_create", 0, None)
+        before = host.lib.pghost_used()
+        if rows:
+            host.ok("pg_matmul_dequant_i8_dev", ctx, x, rows, 4096, few, y)
+        arena = host.lib.pghost_used() - before
+        host.lib.pghost_clear_launches()
+        host.lib.pghost_begin_capture(host.stream(ctx))
+        st = getattr(host.lib, call)(ctx, x, m, k, q, y, *tail)
+        assert host.lib.pghost_end_capture(host.stream(ctx)) == (st == 0)
+        names = [name for name, _ in host.launches()]
+        seen.append("refused" if st else "split" if finish in names[-1] else "whole")
+        assert host.lib.pghost_used() - before == arena
+        host.lib.pg_ctx_destroy(ctx)
+    assert seen[0] == "refused" and seen[-1] == "split" and "whole" in seen, seen
+    assert seen == sorted(seen, key=["refused", "whole", "split"].index), seen
+    for t in (q, few):
+        host.lib.pg_qtensor_free(host.ctx, t)
+
+
+@pytest.mark.parametrize("call,m,n,k,finish", SPLIT_CALLS)
+def test_int8_products_do_without_the_room_to_split_k_where_memory_has_run_out(host, call, m, n, k, finish):
+    w = host.alloc(n * k)
+    q = host.new("pg_qtensor_from_f32_dev", host.ctx, w, k, n)
+    x, y = host.alloc(m * k), host.alloc(m * n)
+    tail = (None,) if call == "pg_matmul_quantized_dev" else ()
+    k_pad, m_pad = (k + 127) // 128 * 128, (m + 255) // 256 * 256
+    rows = m_pad * k_pad * (1 if tail else 3)
+    used, seen = host.lib.pghost_used(), []
+    for free in (rows // 2, rows * 5 // 4 + (2 << 20), rows * 5 // 4 + (80 << 20)):
+        ctx = host.new("pg_ctx_create", 0, None)
+        host.lib.pghost_limit(used + free)
+        host.lib.pghost_clear_launches()
+        st = getattr(host.lib, call)(ctx, x, m, k, q, y, *tail)
+        host.lib.pghost_limit(NO_LIMIT)
+        names = [name for name, _ in host.launches()]
+        seen.append("refused" if st else "split" if finish in names[-1] else "whole")
+        host.lib.pg_ctx_destroy(ctx)
+    assert seen == ["refused", "whole", "split"], seen
+    host.lib.pg_qtensor_free(host.ctx, q)
+
+
 def test_expert_layers_are_captured_after_one_eager_call(host):
     d, ffn, E, k = 256, 512, 8, 2
     tab = lambda n_out, k_in: (C.c_void_p * E)(*[host.new("pg_gguf_upload", host.ctx, bytes(n_out * k_in // 32 * 34), 8, n_out, k_in).value for _ in range(E)])
