@@ -162,6 +162,60 @@ def test_few_row_products_replayed_from_a_graph(ctx, orc):
     gw.free()
 
 
+@pytest.mark.parametrize("call,m,n,k,rows,runs", [("pg_matmul_quantized_dev", 488, 643, 8192, 512, 5), ("pg_matmul_dequant_i8_dev", 286, 832, 7055, 768, 3)])
+def test_split_products_replayed_from_a_graph_whose_arena_has_no_room_to_split(ctx, orc, call, m, n, k, rows, runs):
+    """K is split over workgroups eagerly; a capture in a context whose scratch holds the rows (another product left it so), but not the partial
+    sums, takes the product whole: the same bits at every replay."""
+    import peregrine_amd
+    from peregrine_amd import _ffi, quant
+    hip, lib = Hip(), _ffi.lib
+    tail = (None,) if call == "pg_matmul_quantized_dev" else ()
+    inputs = [orc.rng_normal(60 + i, m * k) for i in range(3)]
+    wf, few = orc.rng_normal(61, k * n, 0.0, 0.02), orc.rng_normal(62, 4096 * 8)
+
+    def last_runs(c):
+        v = [C.c_int() for _ in range(3)]
+        _ffi.check(lib.pg_gemm_w8a8_last_tile(c.handle, *[C.byref(t) for t in v]))
+        return v[2].value
+
+    def product(c, x, w, y):
+        return getattr(lib, call)(c.handle, x.ptr, m, k, w._gpu, y.ptr, *tail)
+
+    qt = quant.quantize_weights(wf, k, n, ctx).to_gpu(ctx)
+    y = DevBuf(ctx, m * n * 4)
+    want = []
+    for v in inputs:
+        x = DevBuf(ctx, host=v)
+        _ffi.check(product(ctx, x, qt, y))
+        ctx.sync()
+        want.append(y.to_host(np.float32).copy())
+    assert last_runs(ctx) == runs
+    c2 = peregrine_amd.Context()
+    q2, f2 = quant.quantize_weights(wf, k, n, ctx).to_gpu(c2), quant.quantize_weights(few, 4096, 8, ctx).to_gpu(c2)
+    nan = np.full(m * n, np.nan, np.float32)
+    x2, y2, xf, yf = DevBuf(c2, host=inputs[0]), DevBuf(c2, m * n * 4), DevBuf(c2, host=np.ones(rows * 4096, np.float32)), DevBuf(c2, rows * 8 * 4)
+    other = lambda: _ffi.check(lib.pg_matmul_dequant_i8_dev(c2.handle, xf.ptr, rows, 4096, f2._gpu, yf.ptr))
+    other()
+    c2.sync()
+    say(f"capturing {call} m={m} k={k} n={n}")
+    graph, ex = hip.capture(c2.stream, lambda: _ffi.check(product(c2, x2, q2, y2)))
+    try:
+        assert last_runs(c2) == 1
+        for i, v in enumerate(inputs):
+            other()                                                       # other work in between, in the same scratch
+            _ffi.check(lib.pg_memcpy_h2d(c2.handle, x2.ptr, C.c_void_p(v.ctypes.data), v.nbytes))
+            _ffi.check(lib.pg_memcpy_h2d(c2.handle, y2.ptr, C.c_void_p(nan.ctypes.data), nan.nbytes))
+            c2.sync()
+            hip.ok(hip.lib.hipGraphLaunch(ex, c2.stream), "hipGraphLaunch")
+            c2.sync()
+            assert (y2.to_host(np.float32).view(np.uint32) == want[i].view(np.uint32)).all(), f"replay {i} differs from the eager, split product"
+    finally:
+        hip.lib.hipGraphExecDestroy(ex)
+        hip.lib.hipGraphDestroy(graph)
+    for w in (qt, q2, f2):
+        w.free_gpu()
+
+
 def test_mxfp4_products_and_moe_replayed_from_a_graph(ctx, orc):
     """MXFP4 over many rows (digit records, tiles over two runs of K, their sum) and the gpt-oss MoE layer over
     MXFP4 experts in both its forms (token tiles of all experts in one launch; pair by pair for a few pairs),
